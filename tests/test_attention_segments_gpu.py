@@ -1,0 +1,54 @@
+"""Decoded rows with four waves a segment: the same bits as the kernels with a wave a segment (plain attention) and as the prompt
+rows' kernel at the same position (capped scores, kept keys, windows, sinks)."""
+import ctypes
+
+import pytest
+import torch
+from test_kernels_gpu import DTYPES, build_cache, kern, rand, run_attention
+
+pytestmark = pytest.mark.gpu
+
+# Keys of a request: one, around a tile of 64, around a segment of 256, a last segment of one tile, and several segments.
+LENGTHS = [1, 5, 63, 64, 65, 128, 191, 193, 255, 256, 257, 320, 513, 700]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,P,window", [(4, 2, 64, 64, 0), (20, 1, 48, 16, 0), (8, 2, 128, 64, 300), (8, 8, 112, 8, 70), (6, 1, 256, 128, 0),
+                                               (4, 1, 208, 32, 64)])
+def test_plain_rows_agree(dtype, nq, nkv, d, P, window):
+    k = kern(dtype)
+    q = [rand((1, nq, d), dtype, 10 + i) for i in range(len(LENGTHS))]
+    keys = [rand((n, nkv, d), dtype, 40 + i) for i, n in enumerate(LENGTHS)]
+    values = [rand((n, nkv, d), dtype, 70 + i) for i, n in enumerate(LENGTHS)]
+    got = {m: run_attention(k, q, keys, values, P, dtype, window=window, poison=float("nan"), seed=m, decode_mode=m, decode_split=m == 7) for m in (3, 7, 1)}
+    assert not torch.isnan(got[7]).any()
+    assert torch.equal(got[7], got[3]) and torch.equal(got[1], got[3])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,P,window,keep,cap", [(4, 2, 64, 64, 0, 0, 20.0), (20, 1, 48, 16, 100, 7, 0.0), (8, 2, 128, 64, 300, 16, 20.0),
+                                                        (8, 8, 112, 8, 64, 70, 5.0), (6, 1, 256, 128, 0, 0, 0.0)])
+def test_capped_rows_agree_with_prompt_rows(dtype, nq, nkv, d, P, window, keep, cap):
+    """The last row of a sequence as a decoded token and as a prompt portion of one row."""
+    k = kern(dtype)
+    p, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    fn = k.lib.vk_paged_attention_capped
+    fn.argtypes = [p] * 5 + [i, p, p, p, i, i, i, p, i, i, i, i, i, i, i, f, f, p, i, p]
+    S = len(LENGTHS)
+    keys = [rand((n, nkv, d), dtype, 40 + j) for j, n in enumerate(LENGTHS)]
+    values = [rand((n, nkv, d), dtype, 70 + j) for j, n in enumerate(LENGTHS)]
+    kc, vc, table = (x.cuda() for x in build_cache(keys, values, P, sum(-(-n // P) for n in LENGTHS) + 3, 3, dtype, float("nan")))
+    q = torch.cat([rand((1, nq, d), dtype, 10 + j) for j in range(S)]).cuda()
+    cu = torch.arange(S + 1, dtype=torch.int32, device="cuda")
+    k_len = torch.tensor(LENGTHS, dtype=torch.int32, device="cuda")
+    items = torch.stack([torch.arange(S), torch.zeros(S)], 1).to(torch.int32).cuda()
+    sinks = torch.linspace(-1, 1, nq, device="cuda")
+    nseg = -(-max(LENGTHS) // 256)
+    scratch = torch.full((k.attn_scratch_floats(S, nq, d, nseg),), float("nan"), device="cuda")
+    out = [torch.zeros_like(q), torch.zeros_like(q)]
+    for mode in (0, 1):
+        assert fn(out[mode].data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], cu.data_ptr(), k_len.data_ptr(),
+                  items.data_ptr(), S, mode, nseg, scratch.data_ptr(), S, nq, nkv, d, P, window, keep, d ** -0.5, cap, sinks.data_ptr(), 1,
+                  torch.cuda.current_stream().cuda_stream) == 0
+    assert not torch.isnan(out[1]).any()
+    assert torch.equal(out[0], out[1])

@@ -33,7 +33,8 @@
 //   attn_decode_seg    decoded tokens: a wave walks the tiles of a segment with the next tile's
 //                      fragments in flight; the segment's (M, L, ACC) goes to a scratch buffer ...
 //   attn_combine       ... which this one folds.
-//   attn_decode_pair   the same with two waves a segment, for steps with few segments.
+//   attn_decode_quad   the same with four waves a segment, one tile's scores each: for steps with few segments, and for
+//                      every step of the variant with capped scores.
 //   attn_decode_plain  the same with a tile's fragments asked for when they are needed: for head and
 //                      element sizes whose fragments of two tiles do not fit a wave's registers.
 //
@@ -211,14 +212,15 @@ constexpr int KSUB = S_PER_LANE / 4;    // 16-key MFMA sub-tiles per tile
 // Key fragments of the whole tile, all in flight together.
 // EXACT (here and below): the head size is the padded one and a page holds a tile or more, known
 // at compile time, so that no branch on either is left in the code.
+// page: the tile's page where the caller has read it from the table already, else -1.
 template <int NQS, bool EXACT>
-__device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[KSUB][NQS]) {
+__device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[KSUB][NQS], int page = -1) {
   const int d = EXACT ? NQS * VK_SLAB : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const bool dfull = EXACT || d % VK_SLAB == 0;    // else the last slab along d is partly outside the head
   const int last_key = c.k_len - 1;
   // With pages of at least a tile, the tile lies in one page: one table lookup for the wave.
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* kpage = c.kbase + (one_page ? (int64_t)c.bt[kb >> lp] * c.page_stride : 0);
+  const elem_t* kpage = c.kbase + (one_page ? (int64_t)(page >= 0 ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int sub = 0; sub < KSUB; ++sub) {
 #ifdef VK_BF16
@@ -241,11 +243,11 @@ __device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[
 }
 
 template <int NDT, bool EXACT>
-__device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf)[NDT][KEY_SLABS]) {
+__device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf)[NDT][KEY_SLABS], int page = -1) {
   const int d = EXACT ? NDT * 16 : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const int last_key = c.k_len - 1;
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* vpage = c.vbase + (one_page ? (int64_t)c.bt[kb >> lp] * c.page_stride : 0);
+  const elem_t* vpage = c.vbase + (one_page ? (int64_t)(page >= 0 ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
     if (dt * 16 < d) {
@@ -991,113 +993,6 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
   }
 }
 
-// The same with two waves a segment, for steps with so few (token, kv head, segment) triples that a wave each
-// leaves most of the chip idle and every wave waits for its four tiles one after the other: the first wave
-// takes the first half of the segment's tiles, the second wave the rest.  The second wave asks for its first
-// tile's keys and values at once and computes that tile's scores, which need no state; when the first wave has
-// left the segment's state in LDS, the second takes it and goes on from there as the one wave would: the same
-// bits, and the loads of both halves in flight together.
-template <int DPAD, bool EXACT>
-__global__ __launch_bounds__(128, 2) void attn_decode_pair_kernel(AttnArgs a) {
-  constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB;
-  __shared__ f32x4 hand_acc[NDT][64];
-  __shared__ float hand_ml[2][64];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
-  const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seg = blockIdx.z;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
-  const int lo = first_visible(a, pos);
-  const int s0 = max(lo / TILE_KEYS, seg * SEG_TILES), s1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
-  if (s0 > s1) return;                                  // the whole workgroup
-  const int n = s1 - s0 + 1, n_first = (n + 1) >> 1;
-  const bool paired = n > 1;                            // the same for both waves
-  const int t0 = wave == 0 ? s0 : s0 + n_first, t1 = wave == 0 ? s0 + n_first - 1 : s1;
-  if (t0 > t1) return;                                  // the second wave of a segment with one tile: no barrier follows for the first either
-
-  RowCtx c;
-  init_ctx(c, a, seq, kvh, k_len);
-  c.r16 = lane & 15;
-  c.g = lane >> 4;
-  c.row_ok = c.r16 < min(16, G - ht * 16);
-  c.pos = pos;
-  c.lo = lo;
-  c.wave_lo = lo;
-  const int head = kvh * G + ht * 16 + c.r16;
-  frag_t qf[NQS];
-  load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
-  frag_t kf[KSUB][NQS];
-  frag_t vf[NDT][KEY_SLABS];
-  load_keys<NQS, EXACT>(c, t0 * TILE_KEYS, kf);
-  load_values<NDT, EXACT>(c, t0 * TILE_KEYS, vf);
-  float M = -INFINITY, L = 0.f;
-  f32x4 ACC[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) ACC[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float sc[S_PER_LANE];
-  // A tile's scores, and its successor's keys asked for.
-  auto front = [&](int t, bool more) {
-    tile_scores<NQS, EXACT>(c, kf, qf, sc);
-    __builtin_amdgcn_sched_barrier(0);
-    if (more) load_keys<NQS, EXACT>(c, (t + 1) * TILE_KEYS, kf);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // The tile onto the state, and its successor's values asked for.
-  auto back = [&](int t, bool more) {
-    const int kb = t * TILE_KEYS;
-    const bool full = kb >= lo && kb + TILE_KEYS - 1 <= pos;
-    frag_t pf[KEY_SLABS];
-    float ca;
-    const bool fresh = !(M > -INFINITY);
-    tile_probs(sc, kb, c.g, c.row_ok, lo, pos, c.scale_log2, full, M, L, ca, pf);
-    scale_state<NDT>(ACC, ca, fresh);
-    tile_pv<NDT, EXACT>(c, kb, vf, pf, ACC);
-    __builtin_amdgcn_sched_barrier(0);
-    if (more) load_values<NDT, EXACT>(c, kb + TILE_KEYS, vf);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // At most two tiles a wave.
-  front(t0, t0 < t1);
-  if (wave == 1) {
-    // The segment's state as the first wave left it (every lane its own part: the same lanes hold the same rows
-    // and columns in both waves).
-    __syncthreads();
-    M = hand_ml[0][lane];
-    L = hand_ml[1][lane];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) ACC[dt] = hand_acc[dt][lane];
-  }
-  back(t0, t0 < t1);
-  if (t0 < t1) {
-    front(t1, false);
-    back(t1, false);
-  }
-  if (wave == 0 && paired) {
-    hand_ml[0][lane] = M;
-    hand_ml[1][lane] = L;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) hand_acc[dt][lane] = ACC[dt];
-    __syncthreads();
-    return;
-  }
-  if (!c.row_ok) return;
-  const int64_t prow = ((int64_t)blockIdx.x * a.nq + head) * a.nseg + seg;
-  if (c.g == 0) {
-    a.part_ml[2 * prow] = M;
-    a.part_ml[2 * prow + 1] = L;
-  }
-  if (M > -INFINITY) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      if (EXACT || dt * 16 < a.d) *reinterpret_cast<f32x4*>(&a.part_acc[prow * a.d + dt * 16 + 4 * c.g]) = ACC[dt];
-  }
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // Capped scores, kept first keys, a sink, and probabilities that are not rounded.
 //
@@ -1204,7 +1099,9 @@ __global__ __launch_bounds__(256) void attn_prefill_ext_kernel(AttnArgs a, int h
   }
 }
 
-// Decoded tokens: attn_decode_plain_kernel with the things above; attn_combine_kernel folds its segments.
+// Decoded tokens: attn_decode_plain_kernel with the things above, for heads whose four tiles no workgroup's registers hold
+// (32-bit, wider than 128); attn_combine_kernel folds its segments.
+#ifndef VK_BF16
 template <int DPAD, bool V_LATE, bool REL>
 __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnArgs a) {
   constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB;
@@ -1255,118 +1152,44 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
       if (dt * 16 < a.d) *reinterpret_cast<f32x4*>(&a.part_acc[prow * a.d + dt * 16 + 4 * c.g]) = ACC[dt];
   }
 }
+#endif
 
-// Decoded tokens of the same variant where a wave's registers hold two tiles' fragments: attn_decode_seg_kernel's walk
-// (the next tile's keys asked for when this tile's scores are done, its values when this tile's product is), over the
-// tiles of the segment that hold kept first keys or keys of the window.
-template <int DPAD, bool EXACT, bool REL>
-__global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_ext_kernel(AttnArgs a) {
-  constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
-  const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seg = blockIdx.z * SEG_WAVES + wave;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
-  const int lo = first_visible(a, pos);
-  const int keep = a.window > 0 ? a.keep : 0;
-  const int keep_tiles = (keep + TILE_KEYS - 1) / TILE_KEYS, tile_lo = lo / TILE_KEYS;
-  // The segment's tiles that hold visible keys, as a mask of SEG_TILES bits.
-  unsigned wanted = 0;
-#pragma unroll
-  for (int j = 0; j < SEG_TILES; ++j) {
-    const int t = seg * SEG_TILES + j;
-    if (t <= pos / TILE_KEYS && (t < keep_tiles || t >= tile_lo)) wanted |= 1u << j;
-  }
-  wanted = __builtin_amdgcn_readfirstlane(wanted);
-  if (wanted == 0) return;   // whole wave; no barrier follows
-
-  RowCtx c;
-  init_ctx(c, a, seq, kvh, k_len);
-  c.r16 = lane & 15;
-  c.g = lane >> 4;
-  c.row_ok = c.r16 < min(16, G - ht * 16);
-  c.pos = pos;
-  c.lo = lo;
-  c.wave_lo = lo;
-  c.keep = keep;
-  const int head = kvh * G + ht * 16 + c.r16;
-  init_rel<REL>(c, a, c.row_ok ? head : kvh * G, pos, pos);
-  frag_t qf[NQS];
-  load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
-  frag_t kf[KSUB][NQS];
-  frag_t vf[NDT][KEY_SLABS];
-  const int first_kb = (seg * SEG_TILES + __builtin_ctz(wanted)) * TILE_KEYS;
-  load_keys<NQS, EXACT>(c, first_kb, kf);
-  load_values<NDT, EXACT>(c, first_kb, vf);
-  float M = -INFINITY, L = 0.f;
-  f32x4 ACC[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) ACC[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < SEG_TILES; ++j) {
-    if ((wanted >> j) & 1u) {
-      const int kb = (seg * SEG_TILES + j) * TILE_KEYS;
-      const unsigned rest = j + 1 < SEG_TILES ? wanted >> (j + 1) : 0u;
-      const bool more = rest != 0;
-      const int next = more ? kb + (1 + __builtin_ctz(rest)) * TILE_KEYS : kb;
-      float sc[S_PER_LANE];
-      tile_scores<NQS, EXACT>(c, kf, qf, sc);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) load_keys<NQS, EXACT>(c, next, kf);
-      __builtin_amdgcn_sched_barrier(0);
-      tile_softmax_pv_ext<NDT, REL>(c, a.scale, a.softcap, sc, kb, vf, M, L, ACC);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) load_values<NDT, EXACT>(c, next, vf);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  if (!c.row_ok) return;
-  const int64_t prow = ((int64_t)blockIdx.x * a.nq + head) * a.nseg + seg;
-  if (c.g == 0) {
-    a.part_ml[2 * prow] = M;
-    a.part_ml[2 * prow + 1] = L;
-  }
-  if (M > -INFINITY) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      if (EXACT || dt * 16 < a.d) *reinterpret_cast<f32x4*>(&a.part_acc[prow * a.d + dt * 16 + 4 * c.g]) = ACC[dt];
-  }
-}
-
-#ifdef VK_BF16
-// Decoded tokens of the same variant with the widest heads, whose fragments of two tiles no wave's registers hold: a
-// workgroup of four waves takes a segment.  Wave j computes the scores of the segment's tile j; the tiles' maxima pass through
-// LDS, so that every wave knows how the rows' reference maximum moves from tile to tile; wave j turns its scores into
-// weights, which pass through LDS too; then every wave adds up a quarter of the output columns over the four tiles, in
-// order.  Keys and values are all asked for at once, at the start.  The operations on a row's sums, and their order, are those
-// of the kernels above.
-template <int DPAD, bool EXACT, bool REL>
-__global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel(AttnArgs a) {
+// Decoded tokens, four waves a segment, for the plain attention and (EXT) the variant.  Wave j computes the scores of the
+// segment's tile j; the tiles' maxima pass through LDS, so that every wave knows how the rows' reference maximum moves from tile to
+// tile; wave j turns its scores into weights, which pass through LDS too; then every wave adds up a quarter of the output columns over
+// the four tiles, in order.  The operations on a row's sums, and their order, are those of the kernels above.
+// What bounds a step of few segments is the chain of dependent loads and of tiles, not bytes: here keys and values of the whole
+// segment are asked for at once, right behind the step's numbers, whose table entries are read together with the sequence's lengths
+// (a page that turns out not to be needed is read and not used), and the four tiles' scores are computed side by side.
+template <int DPAD, bool EXACT, bool EXT, bool REL>
+__global__ __launch_bounds__(64 * SEG_TILES, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a) {
+  static_assert(EXT || !REL, "biases by distance belong to the variant");
   constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB, ND = NDT / SEG_TILES;   // ND: column blocks of a wave
-  __shared__ frag_t probs[SEG_TILES][P_PARTS][KEY_SLABS][64];
+  constexpr int NP = EXT ? P_PARTS : 1;                                        // numbers that a weight is split into
+  __shared__ frag_t probs[SEG_TILES][NP][KEY_SLABS][64];
   __shared__ float tile_max[SEG_TILES][16], tile_sum[SEG_TILES][16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seg = blockIdx.z;
+  const int seg = blockIdx.z, first_tile = seg * SEG_TILES;
   const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
   const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
   const int k_len = a.k_len[seq];
+  const int lp = __builtin_ctz(a.P);
+  int page[SEG_TILES];                  // of the segment's tiles, where a tile lies in one page
+#pragma unroll
+  for (int j = 0; j < SEG_TILES; ++j)
+    page[j] = EXACT || a.P >= TILE_KEYS ? a.block_table[(int64_t)seq * a.bt_stride + min((first_tile + j) * TILE_KEYS >> lp, a.bt_stride - 1)] : -1;
   const int tok = q_begin + q_off;
   const int pos = k_len - q_len + q_off;
   const int lo = first_visible(a, pos);
-  const int keep = a.window > 0 ? a.keep : 0;
+  const int keep = EXT && a.window > 0 ? a.keep : 0;
   const int keep_tiles = (keep + TILE_KEYS - 1) / TILE_KEYS, tile_lo = lo / TILE_KEYS;
-  unsigned wanted = 0;
+  unsigned wanted = 0;                  // the segment's tiles that hold visible keys
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j) {
-    const int t = seg * SEG_TILES + j;
+    const int t = first_tile + j;
     if (t <= pos / TILE_KEYS && (t < keep_tiles || t >= tile_lo)) wanted |= 1u << j;
   }
   wanted = __builtin_amdgcn_readfirstlane(wanted);
@@ -1382,14 +1205,16 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
   c.wave_lo = lo;
   c.keep = keep;
   const int head = kvh * G + ht * 16 + c.r16;
-  init_rel<REL>(c, a, c.row_ok ? head : kvh * G, pos, pos);
-  const int first_tile = seg * SEG_TILES;
+  if constexpr (REL) init_rel<REL>(c, a, c.row_ok ? head : kvh * G, pos, pos);
   const bool mine = (wanted >> wave) & 1u;
   frag_t qf[NQS];
   frag_t kf[KSUB][NQS];
   if (mine) {
     load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
-    load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf);
+    int my_page = page[0];
+#pragma unroll
+    for (int j = 1; j < SEG_TILES; ++j) my_page = wave == j ? page[j] : my_page;
+    load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf, my_page);
   }
   // This wave's columns of every tile's values: a context whose head starts at them.
   RowCtx cv = c;
@@ -1398,19 +1223,20 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
   frag_t vf[SEG_TILES][ND][KEY_SLABS];
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j)
-    if ((wanted >> j) & 1u) load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j]);
+    if ((wanted >> j) & 1u) load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the scores of this wave's tile and their maximum a row ----
+  const float unit = EXT ? LOG2E : a.scale_log2;             // what takes a score to powers of two
   float sc[S_PER_LANE];
   bool vis[S_PER_LANE];
   const int kb = (first_tile + wave) * TILE_KEYS;
   float tmax = -INFINITY;
   if (mine) {
     float rb[REL ? S_PER_LANE : 1];
-    tile_bias<REL>(c, kb, rb);
+    if constexpr (REL) tile_bias<REL>(c, kb, rb);
     tile_scores<NQS, EXACT>(c, kf, qf, sc);
-    natural_scores<REL>(sc, a.scale, a.softcap, rb);
+    if constexpr (EXT) natural_scores<REL>(sc, a.scale, a.softcap, rb);
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
       const int key = kb + (i / VK_VEC) * VK_SLAB + c.g * VK_VEC + (i % VK_VEC);
@@ -1427,7 +1253,7 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
   float M = -INFINITY, my_max = -INFINITY, ca[SEG_TILES];
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j) {
-    const float m = tile_max[j][c.r16] * LOG2E;              // -inf: the row sees no key of the tile
+    const float m = tile_max[j][c.r16] * unit;               // -inf: the row sees no key of the tile
     const float Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
     ca[j] = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
     M = Mn;
@@ -1435,23 +1261,25 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
   }
   if (mine) {
     float psum = 0.f;
-    frag_t pf[P_PARTS][KEY_SLABS];
+    frag_t pf[NP][KEY_SLABS];
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
-      const float p = vis[i] ? fast_exp2(__builtin_fmaf(sc[i], LOG2E, -my_max)) : 0.f;
+      const float p = vis[i] ? fast_exp2(__builtin_fmaf(sc[i], unit, -my_max)) : 0.f;
       psum = psum + p;
-      const __bf16 hi = (__bf16)p;
-      const float r1 = p - (float)hi;
-      const __bf16 mid = (__bf16)r1;
+      const elem_t hi = (elem_t)p;
       pf[0][i / VK_VEC][i % VK_VEC] = hi;
-      pf[1][i / VK_VEC][i % VK_VEC] = mid;
-      pf[2][i / VK_VEC][i % VK_VEC] = (__bf16)(r1 - (float)mid);
+      if constexpr (NP == 3) {
+        const float r1 = p - (float)hi;
+        const elem_t mid = (elem_t)r1;
+        pf[1][i / VK_VEC][i % VK_VEC] = mid;
+        pf[2][i / VK_VEC][i % VK_VEC] = (elem_t)(r1 - (float)mid);
+      }
     }
     psum = psum + lane_xor16(psum);
     psum = psum + lane_xor32(psum);
     if (c.g == 0) tile_sum[wave][c.r16] = psum;
 #pragma unroll
-    for (int part = 0; part < P_PARTS; ++part)
+    for (int part = 0; part < NP; ++part)
 #pragma unroll
       for (int ks = 0; ks < KEY_SLABS; ++ks) probs[wave][part][ks][lane] = pf[part][ks];
   }
@@ -1472,15 +1300,15 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt) zero_unowned(vf[j][dt], kj, c.g, lo, k_len, keep);
       }
-      frag_t pf[P_PARTS][KEY_SLABS];
+      frag_t pf[NP][KEY_SLABS];
 #pragma unroll
-      for (int part = 0; part < P_PARTS; ++part)
+      for (int part = 0; part < NP; ++part)
 #pragma unroll
         for (int ks = 0; ks < KEY_SLABS; ++ks) pf[part][ks] = probs[j][part][ks][lane];
 #pragma unroll
       for (int ks = 0; ks < KEY_SLABS; ++ks)
 #pragma unroll
-        for (int part = 0; part < P_PARTS; ++part)
+        for (int part = 0; part < NP; ++part)
 #pragma unroll
           for (int dt = 0; dt < ND; ++dt)
             if (EXACT || dt * 16 < cv.d) ACC[dt] = mma_slab(vf[j][dt][ks], pf[part][ks], ACC[dt]);
@@ -1498,7 +1326,6 @@ __global__ __launch_bounds__(64 * SEG_TILES, 1) void attn_decode_quad_ext_kernel
       if (EXACT || dt * 16 < cv.d) *reinterpret_cast<f32x4*>(&a.part_acc[prow * a.d + (wave * ND + dt) * 16 + 4 * c.g]) = ACC[dt];
   }
 }
-#endif
 
 // Folds the segment results of one (token, head) in ascending segment order.
 // One wave per row; lane j owns output columns j, j+64, ...
@@ -1598,7 +1425,7 @@ int vk_attn_prefill_shares_tiles(int d, int P) {
 //   the longest sequence; scratch must hold vk_attn_scratch_floats(n_items, ...)) and folded by a
 //   second kernel; the kernel is chosen by shape.  modes 3, 4, 5, 7: the same through a named kernel
 //   (3 and 4: a wave per segment that asks for a tile's fragments when it needs them, the kernel for every
-//   shape; 5: a wave per segment with two tiles' fragments in registers; 7: two waves per segment; tests
+//   shape; 5: a wave per segment with two tiles' fragments in registers; 7: four waves per segment where it has the size; tests
 //   and measurements; the same bits).
 int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const elem_t* vc,
                        const int32_t* block_table, int bt_stride, const int32_t* cu_q, const int32_t* k_len,
@@ -1687,26 +1514,29 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   a.part_acc = scratch + (((int64_t)n_items * nq * nseg * 2 + 3) & ~(int64_t)3);
   const dim3 grid(n_items, nkv * ((G + 15) / 16), nseg);
   VK_REQUIRE(grid.y <= 65535 && nq <= 65535, "attention: too many heads");
-  static_assert(SEG_TILES == 4, "the pair kernel gives a wave two tiles at most");
-  // Two waves a segment while there are no more segments in work than one and a quarter per compute unit
-  // (measured on MI355X, head size 128, 8 kv heads, with the fold of the segments; a wave against two waves a
-  // segment: 1 token of 2,090 keys, 72 segments, 14.7 against 12.6 us; 2 tokens, 144: 14.9, 12.9; 4 tokens, 288:
-  // 15.7, 14.9; 8 tokens of 1,000 keys, 256: 14.0, 13.1; 6 tokens of 2,090, 432: 17.5, 19.2; 8 tokens, 576: 19.8,
-  // 21.4; 1 token of 32,800 keys, 1,032: 60.3, 62.0).
-  const bool pair_fits = seg_fits;
-  if (vk_decode_variant == 4 ||
-      (vk_decode_variant == 0 && pair_fits && 4 * (int64_t)grid.x * grid.y * grid.z <= 5 * (int64_t)attn_device_cus())) {
+  // Four waves a segment while segments are few enough that a step waits for chains of loads and tiles and not for bytes: up to two
+  // and a half of them a compute unit, or six where the other choice is the kernel without a tile in flight (32-bit, more than 64
+  // entries a head).  Measured on MI355X with the fold of the segments, a wave (or before this kernel two) a segment against four,
+  // 16-bit elements, head size 128: 1 token of 23 keys, 8 segments, 12.0 against 8.1 us; 3 tokens of 220 keys, 24: 15.4, 10.5; 8 of
+  // 530, 192: 12.1, 10.4; 8 of 1,030, 320: 14.2, 12.6; 8 of 2,090, 576: 21.0, 19.3; 24 of 2,048, 1,536: 35.8, 36.3; head size 64,
+  // 1,536: 16.7, 18.0; 32-bit, head size 128: 3 tokens of 220 keys 43.5, 17.2; 64 of 530, 1,536: 99.7, 78.6; 64 of 2,060, 4,608:
+  // 258, 276.  (32-bit with wider heads: four tiles' fragments do not fit the registers.)
+  const bool quad_fits = sizeof(elem_t) * vk_dpad(d) <= 512;
+  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = (seg_fits || sizeof(elem_t) == 2 ? 5 : 12) * (int64_t)attn_device_cus() / 2;
+  if (quad_fits && (vk_decode_variant == 4 || (vk_decode_variant == 0 && segments <= quad_most))) {
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
-#define DECODE_PAIR(DP)                                                           \
-  do {                                                                            \
-    if (exact) attn_decode_pair_kernel<DP, true><<<grid, 128, 0, st>>>(a);        \
-    else attn_decode_pair_kernel<DP, false><<<grid, 128, 0, st>>>(a);             \
+#define DECODE_QUAD(DP)                                                                               \
+  do {                                                                                                \
+    if (exact) attn_decode_quad_kernel<DP, true, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);   \
+    else attn_decode_quad_kernel<DP, false, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);        \
   } while (0)
-    if (d <= 64) DECODE_PAIR(64);
-    else if (d <= 128) DECODE_PAIR(128);
-    else DECODE_PAIR(256);
-#undef DECODE_PAIR
-    if (vk_check_launch("attention (decoded rows, two waves per segment)")) return 1;
+    if (d <= 64) DECODE_QUAD(64);
+    else if (d <= 128) DECODE_QUAD(128);
+#ifdef VK_BF16
+    else DECODE_QUAD(256);
+#endif
+#undef DECODE_QUAD
+    if (vk_check_launch("attention (decoded rows, four waves per segment)")) return 1;
     attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
     return vk_check_launch("attention (combine)");
   }
@@ -1817,56 +1647,43 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
   a.part_ml = scratch;
   a.part_acc = scratch + (((int64_t)n_items * nq * nseg * 2 + 3) & ~(int64_t)3);
   VK_REQUIRE(nkv * ((G + 15) / 16) <= 65535 && nq <= 65535, "attention: too many heads");
-  if (sizeof(elem_t) * vk_dpad(d) <= 256) {
-    // A wave's registers hold two tiles' fragments: the walk with the next tile in flight.
+  if (sizeof(elem_t) * vk_dpad(d) <= 512) {
+    // Four waves a segment whatever the number of segments: a tile costs the variant three products a slab and the cap's exponentials,
+    // so that a wave a segment was a chain of arithmetic too.  Measured on MI355X with the fold, windows of 1,024, a wave against four
+    // a segment, 16-bit elements, head size 128, 8 kv heads: 1 token of 500 keys 24.2 against 11.9 us; 8 of 300 19.3, 11.4; 8 of
+    // 2,090 27.8, 15.7; 64 of 2,060 57.4, 53.3; 32-bit: 3 tokens of 220 keys 42.6, 16.8; 64 of 2,060 182, 164.
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
-    const dim3 sgrid(n_items, nkv * ((G + 15) / 16), (nseg + SEG_WAVES - 1) / SEG_WAVES);
-#define DECODE_SEG_EXT_OF(DP, REL)                                                                \
-  do {                                                                                            \
-    if (exact) attn_decode_seg_ext_kernel<DP, true, REL><<<sgrid, 64 * SEG_WAVES, 0, st>>>(a);    \
-    else attn_decode_seg_ext_kernel<DP, false, REL><<<sgrid, 64 * SEG_WAVES, 0, st>>>(a);         \
+    const dim3 qgrid(n_items, nkv * ((G + 15) / 16), nseg);
+#define DECODE_QUAD_EXT_OF(DP, REL)                                                                        \
+  do {                                                                                                     \
+    if (exact) attn_decode_quad_kernel<DP, true, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);          \
+    else attn_decode_quad_kernel<DP, false, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);               \
   } while (0)
-#define DECODE_SEG_EXT(DP) do { if (rel != nullptr) DECODE_SEG_EXT_OF(DP, true); else DECODE_SEG_EXT_OF(DP, false); } while (0)
+#define DECODE_QUAD_EXT(DP) do { if (rel != nullptr) DECODE_QUAD_EXT_OF(DP, true); else DECODE_QUAD_EXT_OF(DP, false); } while (0)
+    if (d <= 64) DECODE_QUAD_EXT(64);
+    else if (d <= 128) DECODE_QUAD_EXT(128);
 #ifdef VK_BF16
-    if (d <= 64) DECODE_SEG_EXT(64);
-    else DECODE_SEG_EXT(128);
-#else
-    DECODE_SEG_EXT(64);
+    else DECODE_QUAD_EXT(256);
 #endif
-#undef DECODE_SEG_EXT
-#undef DECODE_SEG_EXT_OF
-    if (vk_check_launch("attention (decoded rows, capped scores, wave per segment)")) return 1;
+#undef DECODE_QUAD_EXT
+#undef DECODE_QUAD_EXT_OF
+    if (vk_check_launch("attention (decoded rows, capped scores, four waves a segment)")) return 1;
     attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
     return vk_check_launch("attention (combine)");
   }
 #ifdef VK_BF16
-  // (128 < d: the smaller sizes went the way above.)
-  const dim3 qgrid(n_items, nkv * ((G + 15) / 16), nseg);
-  const bool exact = P >= TILE_KEYS && d == 256;
-  if (rel != nullptr) {
-    if (exact) attn_decode_quad_ext_kernel<256, true, true><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);
-    else attn_decode_quad_ext_kernel<256, false, true><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);
-  } else {
-    if (exact) attn_decode_quad_ext_kernel<256, true, false><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);
-    else attn_decode_quad_ext_kernel<256, false, false><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);
-  }
-  if (vk_check_launch("attention (decoded rows, capped scores, four waves a segment)")) return 1;
-  attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
-  return vk_check_launch("attention (combine)");
+  return vk_fail("attention: no kernel for decoded rows of head size %d", d);      // (none is wider than 256)
 #else
   const dim3 grid(n_items, nkv * ((G + 15) / 16), (nseg + PLAIN_WAVES - 1) / PLAIN_WAVES);
   const bool late = (int64_t)grid.x * grid.y * nseg > 1024;
-#define DECODE_EXT_OF(DP, REL)                                                                \
-  do {                                                                                        \
-    if (late) attn_decode_ext_kernel<DP, true, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);    \
-    else attn_decode_ext_kernel<DP, false, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);        \
+#define DECODE_EXT(REL)                                                                        \
+  do {                                                                                         \
+    if (late) attn_decode_ext_kernel<256, true, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);    \
+    else attn_decode_ext_kernel<256, false, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);        \
   } while (0)
-#define DECODE_EXT(DP) do { if (rel != nullptr) DECODE_EXT_OF(DP, true); else DECODE_EXT_OF(DP, false); } while (0)
-  // (d <= 64 went the way above.)
-  if (d <= 128) DECODE_EXT(128);
-  else DECODE_EXT(256);
+  if (rel != nullptr) DECODE_EXT(true);
+  else DECODE_EXT(false);
 #undef DECODE_EXT
-#undef DECODE_EXT_OF
   if (vk_check_launch("attention (decoded rows, capped scores)")) return 1;
   attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
   return vk_check_launch("attention (combine)");
