@@ -1,0 +1,96 @@
+"""The recurrences' kernels for whole vectors (prompts in chunks, steps of single tokens) against the walk that takes every shape, which
+rows of an odd length lead to: the same bits in the read-outs and the states, whatever the lengths; and both against the equations."""
+import ctypes
+
+import pytest
+import torch
+from test_kernels_gpu import DTYPES, kern
+
+pytestmark = pytest.mark.gpu
+
+
+def run(k, kind, d, heads, lengths, fresh, odd, dtype):
+    """One step of sequences of these lengths; odd: rows one element longer, so that they are not whole vectors."""
+    g = torch.Generator().manual_seed(3)
+    T, S, H, dv = sum(lengths), len(lengths), heads, 128
+    G = H // 2 if kind == "delta" else H
+    cols = 2 * G * d + H * dv
+    x = torch.randn(T, cols, generator=g)
+    rows = torch.zeros(T, cols + (1 if odd else 0))
+    rows[:, :cols] = x
+    rows = rows.to(torch.float32 if kind == "delta" else dtype).cuda()
+    decay = (0.9 + 0.1 * torch.rand(T, H, d, generator=g)).cuda()
+    head_decay = (0.9 + 0.1 * torch.rand(H, generator=g)).cuda()
+    beta = torch.randn(T, H, generator=g).to(dtype).cuda()
+    state = torch.randn(S + 1, H * d * dv, generator=g).cuda()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    positions = torch.arange(T, dtype=torch.int32) + (0 if fresh else 7)
+    for s in range(S):
+        positions[cu[s]] = 0 if fresh and s % 2 == 0 else 5
+    cu, positions, slots = i32(cu), positions.cuda(), i32([(s + 1) % (S + 1) for s in range(S)])
+    out = torch.full((T, H, dv), float("nan"), device="cuda")
+    p, i, l, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
+    stream = torch.cuda.current_stream().cuda_stream
+    where = (cu.data_ptr(), positions.data_ptr(), slots.data_ptr(), T, S, H)
+    if kind == "delta":
+        fn = k.lib.vk_delta_rule
+        fn.argtypes = [p, p, l, i, i, i, p, p, l, p, l, p, p, p, i, i, i, i, i, i, p]
+        rc = fn(out.data_ptr(), rows.data_ptr(), rows.shape[1], 0, G * d, 2 * G * d, decay.data_ptr(), beta.data_ptr(), H, state.data_ptr(), state.shape[1],
+                *where, G, d, dv, stream)
+    else:
+        fn = k.lib.vk_gla_rule if kind == "gla" else k.lib.vk_linear_rule
+        fn.argtypes = [p, p, l, i, i, i, p, p, l, p, p, p, i, i, i, i, i, f, p]
+        rc = fn(out.data_ptr(), rows.data_ptr(), rows.shape[1], 0, H * d, 2 * H * d, (decay if kind == "gla" else head_decay).data_ptr(), state.data_ptr(),
+                state.shape[1], *where, d, dv, 0.3, stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    return out.cpu(), state.cpu()
+
+
+def plain(kind, d, heads, n, dtype):
+    """The read-outs of one sequence from a zero state, for run()'s numbers, in 64 bits."""
+    g = torch.Generator().manual_seed(3)
+    H, dv = heads, 128
+    G = H // 2 if kind == "delta" else H
+    x = torch.randn(n, 2 * G * d + H * dv, generator=g).to(torch.float32 if kind == "delta" else dtype).double()
+    decay = (0.9 + 0.1 * torch.rand(n, H, d, generator=g)).double()
+    head_decay = (0.9 + 0.1 * torch.rand(H, generator=g)).double()
+    beta = torch.randn(n, H, generator=g).to(dtype).double().sigmoid()
+    if kind == "linear":
+        decay = head_decay[None, :, None].expand(n, H, d)
+    q, key = (x[:, j * G * d:(j + 1) * G * d].view(n, G, d).repeat_interleave(H // G, 1) for j in (0, 1))
+    v = x[:, 2 * G * d:].view(n, H, dv)
+    S, out = torch.zeros(H, d, dv).double(), []
+    for t in range(n):
+        S = decay[t][:, :, None] * S
+        u = beta[t][:, None] * (v[t] - (S * key[t][:, :, None]).sum(1)) if kind == "delta" else v[t]
+        S = S + key[t][:, :, None] * u[:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1) * (1.0 if kind == "delta" else 0.3))
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d", [8, 16, 40, 64, 100, 128, 200, 300])
+@pytest.mark.parametrize("kind", ["delta", "gla", "linear"])
+def test_the_equations(kind, d, dtype):
+    """Sums over 1 to 64 lanes.  Everything is 32-bit: 45 tokens of a decayed sum of products are good to a few 1e-7 of their size;
+    the delta rule's corrections, which may grow with keys that are no unit vectors, are left to the key sizes where they stay small."""
+    if kind == "delta" and d > 128:
+        pytest.skip("with random keys of this size the corrections overflow")
+    got, want = run(kern(dtype), kind, d, 2, [45], True, False, dtype)[0].double(), plain(kind, d, 2, 45, dtype)
+    assert (got - want).norm() < 5e-6 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kind", ["delta", "gla", "linear"])
+def test_the_same_bits_as_the_walk_for_every_shape(kind, d, dtype):
+    k = kern(dtype)
+    for heads, lengths, fresh in ((4, [1], True), (4, [1, 1, 1], True), (4, [1, 1, 1], False), (4, [16], True), (4, [15, 1, 17], False), (4, [33, 2, 48], True),
+                                  (48, [17, 5, 32], False)):           # the last: so many workgroups that a lane takes two columns
+        got, want = (run(k, kind, d, heads, lengths, fresh, odd, dtype) for odd in (False, True))
+        assert not torch.isnan(got[0]).any()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -72,16 +72,24 @@ __device__ __forceinline__ float lane_xor32(float v) {
 // The sum over the R neighbouring lanes of an aligned group, in every lane of the group: a butterfly whose steps stay
 // in the vector unit (quad permutes, the mirrors of a half row and of a row, the swaps of rows and halves).  The order
 // of the additions is fixed by R.
+// (All lanes of a group are active where these are called, so that no lane keeps an old value and the compiler folds the permute into
+// the addition: one instruction a step instead of four.)
 __device__ __forceinline__ float dpp_f(float v, int ctrl_tag) {
   const int x = __builtin_bit_cast(int, v);
   int y;
   switch (ctrl_tag) {
-    case 0: y = __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false); break;    // quad_perm [1, 0, 3, 2]
-    case 1: y = __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false); break;    // quad_perm [2, 3, 0, 1]
-    case 2: y = __builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false); break;   // row_half_mirror
-    default: y = __builtin_amdgcn_update_dpp(x, x, 0x140, 0xF, 0xF, false); break;  // row_mirror
+    case 0: y = __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true); break;    // quad_perm [1, 0, 3, 2]
+    case 1: y = __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true); break;    // quad_perm [2, 3, 0, 1]
+    case 2: y = __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true); break;   // row_half_mirror
+    default: y = __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, true); break;  // row_mirror
   }
   return __builtin_bit_cast(float, y);
+}
+// The sum of a swap's two results.  (Each is copied first: a bit cast of a vector's element reads the vector's first one.)
+template <typename PAIR>
+__device__ __forceinline__ float pair_sum(const PAIR& r) {
+  const unsigned a = r[0], b = r[1];
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
 template <int R>
 __device__ __forceinline__ float group_sum(float v) {
@@ -89,8 +97,15 @@ __device__ __forceinline__ float group_sum(float v) {
   if (R >= 4) v = v + dpp_f(v, 1);
   if (R >= 8) v = v + dpp_f(v, 2);
   if (R >= 16) v = v + dpp_f(v, 3);
-  if (R >= 32) v = v + lane_xor16(v);
-  if (R >= 64) v = v + lane_xor32(v);
+  // A swap of a number with itself leaves the two rows' (halves') numbers in every lane of both, whichever was its own.
+  if (R >= 32) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    v = pair_sum(__builtin_amdgcn_permlane16_swap(u, u, false, false));
+  }
+  if (R >= 64) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    v = pair_sum(__builtin_amdgcn_permlane32_swap(u, u, false, false));
+  }
   return v;
 }
 

@@ -18,6 +18,23 @@
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 
+// N (4 or 8) neighbouring numbers of a row, in whole vectors.
+template <int N>
+__device__ __forceinline__ void load_row(const float* p, float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; i += 4) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(p + i);
+    v[i] = x.x; v[i + 1] = x.y; v[i + 2] = x.z; v[i + 3] = x.w;
+  }
+}
+template <int N>
+__device__ __forceinline__ void load_row(const __bf16* p, float (&v)[N]) {
+  typedef __attribute__((ext_vector_type(N))) __bf16 vec;
+  const vec x = *reinterpret_cast<const vec*>(p);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = (float)x[i];
+}
+
 // y[t, c] = silu(sum over j of taps[c, j] * x[t - (K - 1) + j, c]): inputs before the step's first token come from the
 // sequence's carried tail (its last K - 1 inputs, oldest first), or are zero when the sequence starts here.
 __global__ __launch_bounds__(256) void delta_conv_kernel(float* __restrict__ y, const elem_t* __restrict__ x, int64_t ldx,
@@ -317,6 +334,279 @@ __global__ __launch_bounds__(RULE_THREADS) void delta_rule_kernel(float* __restr
   }
 }
 
+// The same recurrence for key sizes 64 and 128 (vectors throughout; rule_launch says which calls), a whole chunk of 16 tokens at a
+// time.  What bounds the walk above is instructions: a token's staging goes element by element and its read-out is summed over the
+// lanes on its own.  Here a thread brings in 16-byte vectors, a lane may hold four channels of two columns (q, k and decays read from LDS
+// once for both), v and beta are read four tokens at a time, the inputs of the second next token while this one is computed; and the
+// sums of the read-outs wait until the chunk ends, when 16 tokens' partial sums go through the lanes together: each step of the
+// butterfly leaves a lane half as many sums (16, 8, 4, 2, 1), 45 instructions instead of 16 x 8 a column.  Every sum adds the same
+// numbers in the same order as above: the bits are the same.  A wave alone on its SIMD issues an instruction every eight clocks or so
+// (two waves: every six), which is what a walk of few sequences now waits for.  Measured on MI355X, 2,048 tokens x 32 heads of 128 x
+// 128: delta rule 852 -> 333 us, a decay per channel 698 -> 235, a decay per head 621 -> 192.
+template <int D, int CC_>
+struct WalkShape {
+  static constexpr int LANES = D / 4;                 // lanes that share their columns
+  static constexpr int GROUPS = 64 / LANES;           // such groups a wave
+  static constexpr int CC = CC_;                      // columns of a lane
+  static constexpr int CB = 4 * GROUPS * CC;          // columns of a workgroup
+  static constexpr int TC = 16;                       // tokens a chunk
+  static constexpr int EPT = TC * D / RULE_THREADS;   // elements of q, k and the decays that a thread brings in of a chunk
+  static constexpr int NV = (TC * CB + RULE_THREADS - 1) / RULE_THREADS;   // and of v
+};
+
+// The sums over the lanes of one column's 16 read-outs: lane r of the column ends with token walk_token(r)'s.  Whether a lane goes on
+// with the first or the second of two sums is chosen so that the partner of every later step has gone on with the same ones.
+__device__ __forceinline__ int walk_token(int r) {
+  const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;
+  return (b0 ^ b2) | (b1 ^ b2) << 1 | (b2 ^ b3) << 2 | b3 << 3;
+}
+__device__ __forceinline__ float walk_sums(float (&p)[16], int token) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 0), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 0);
+    p[i] = token & 1 ? b : a;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 1), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 1);
+    p[i] = token & 2 ? b : a;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 2), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 2);
+    p[i] = token & 4 ? b : a;
+  }
+  const float a = p[0] + dpp_f(p[0], 3), b = p[1] + dpp_f(p[1], 3);
+  return token & 8 ? b : a;
+}
+
+template <int D, int CC_, bool DELTA, typename IN, bool HEAD_DECAY>
+__global__ __launch_bounds__(RULE_THREADS, 2) void rule_walk_kernel(float* __restrict__ out, const IN* __restrict__ qkv, int64_t ld, int q_col, int k_col,
+                                                                    int v_col, const float* __restrict__ decay, const elem_t* __restrict__ b, int64_t ldb,
+                                                                    float* state, int64_t state_stride, const int32_t* __restrict__ cu_q,
+                                                                    const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, int H, int G,
+                                                                    int dv, float q_scale) {
+  using W = WalkShape<D, CC_>;
+  constexpr int CC = W::CC, CB = W::CB, TC = W::TC, EPT = W::EPT;
+  constexpr int V_AT = (HEAD_DECAY ? 2 : 3) * TC * D, B_AT = V_AT + CB * TC, BUF = B_AT + TC;    // floats: k, q, decays, v [column][token], beta
+  __shared__ __attribute__((aligned(16))) float smem[2 * BUF];
+  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane % W::LANES, col = (wave * W::GROUPS + lane / W::LANES) * CC;        // the lane's first column in the block
+  const int g = h / (H / G);
+  const int first = cu_q[s], n = cu_q[s + 1] - first;
+  if (n <= 0) return;                                 // the whole workgroup
+  const bool fresh = positions[first] == 0;
+  float* S_mem = state + (int64_t)slots[s] * state_stride + ((int64_t)h * dv + blockIdx.z * CB + col) * D + r * 4;
+  f32x4 S[CC];
+#pragma unroll
+  for (int j = 0; j < CC; ++j) S[j] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(S_mem + (int64_t)j * D);
+
+  // A thread brings in EPT neighbouring channels of one token's q, k and decays, and NV entries of v.  Tokens beyond the last read
+  // the last one again and are not used.
+  const int in_tok = tid / (D / EPT), in_c = (tid % (D / EPT)) * EPT;
+  float pk[EPT], pq[EPT], pg[EPT], pv[W::NV], pb = 0.f;
+  const float head_g = HEAD_DECAY ? decay[h] : 1.f;
+  auto fetch = [&](int t0) {
+    const int64_t t = first + min(t0 + in_tok, n - 1);
+    const IN* row = qkv + t * ld + (int64_t)g * D + in_c;
+    load_row<EPT>(row + k_col, pk);
+    load_row<EPT>(row + q_col, pq);
+    if (!HEAD_DECAY) load_row<EPT>(decay + (t * H + h) * D + in_c, pg);
+#pragma unroll
+    for (int i = 0; i < W::NV; ++i) {
+      const int e = min(tid + i * RULE_THREADS, TC * CB - 1);
+      pv[i] = to_f32(qkv[(int64_t)(first + min(t0 + e / CB, n - 1)) * ld + v_col + (int64_t)h * dv + blockIdx.z * CB + e % CB]);
+    }
+    if (DELTA && tid < TC) pb = sigmoid_f(to_f32(b[(int64_t)(first + min(t0 + tid, n - 1)) * ldb + h]));
+  };
+  auto stage = [&](float* base) {
+    const int at = in_tok * D + in_c;
+#pragma unroll
+    for (int i = 0; i < EPT; i += 4) {
+      *reinterpret_cast<f32x4*>(base + at + i) = f32x4{pk[i], pk[i + 1], pk[i + 2], pk[i + 3]};
+      f32x4 q4 = {pq[i], pq[i + 1], pq[i + 2], pq[i + 3]};
+      if (!DELTA) { q4.x = q4.x * q_scale; q4.y = q4.y * q_scale; q4.z = q4.z * q_scale; q4.w = q4.w * q_scale; }
+      *reinterpret_cast<f32x4*>(base + TC * D + at + i) = q4;
+      if (!HEAD_DECAY) *reinterpret_cast<f32x4*>(base + 2 * TC * D + at + i) = f32x4{pg[i], pg[i + 1], pg[i + 2], pg[i + 3]};
+    }
+#pragma unroll
+    for (int i = 0; i < W::NV; ++i) {
+      const int e = tid + i * RULE_THREADS;
+      if (e < TC * CB) base[V_AT + (e % CB) * TC + e / CB] = pv[i];
+    }
+    if (DELTA && tid < TC) base[B_AT + tid] = pb;
+  };
+  const int token = walk_token(r);
+
+  fetch(0);
+  stage(smem);
+  __syncthreads();
+  for (int t0 = 0, buffer = 0; t0 < n; t0 += TC, buffer ^= 1) {
+    const float* base = smem + buffer * BUF;
+    const float* kr = base + r * 4;
+    if (t0 + TC < n) fetch(t0 + TC);
+    // The tokens' inputs as this lane needs them, asked for AHEAD tokens before they are used: LDS answers four waves' vectors later than
+    // one token's arithmetic takes.
+    constexpr int AHEAD = 2;
+    f32x4 kn[AHEAD], qn[AHEAD], gn[AHEAD];
+    auto read = [&](int tok, int to) {
+      kn[to] = *reinterpret_cast<const f32x4*>(kr + tok * D);
+      qn[to] = *reinterpret_cast<const f32x4*>(kr + TC * D + tok * D);
+      if (!HEAD_DECAY) gn[to] = *reinterpret_cast<const f32x4*>(kr + 2 * TC * D + tok * D);
+      else gn[to] = f32x4{head_g, head_g, head_g, head_g};
+    };
+    // One token onto the states; the lane's part of its read-outs.
+    auto step = [&](const f32x4& k4, const f32x4& q4, const f32x4& g4, const float (&v)[CC], float beta, float (&o)[CC]) {
+      float u[CC];
+#pragma unroll
+      for (int j = 0; j < CC; ++j) {
+        S[j].x = S[j].x * g4.x; S[j].y = S[j].y * g4.y; S[j].z = S[j].z * g4.z; S[j].w = S[j].w * g4.w;
+        u[j] = v[j];
+      }
+      if (DELTA) {
+#pragma unroll
+        for (int j = 0; j < CC; ++j) {
+          float dot = __builtin_fmaf(S[j].x, k4.x, 0.f);
+          dot = __builtin_fmaf(S[j].y, k4.y, dot);
+          dot = __builtin_fmaf(S[j].z, k4.z, dot);
+          u[j] = __builtin_fmaf(S[j].w, k4.w, dot);
+        }
+#pragma unroll
+        for (int j = 0; j < CC; ++j) u[j] = beta * (v[j] - group_sum<W::LANES>(u[j]));
+      }
+#pragma unroll
+      for (int j = 0; j < CC; ++j) {
+        S[j].x = __builtin_fmaf(k4.x, u[j], S[j].x);
+        o[j] = __builtin_fmaf(S[j].x, q4.x, 0.f);
+        S[j].y = __builtin_fmaf(k4.y, u[j], S[j].y);
+        o[j] = __builtin_fmaf(S[j].y, q4.y, o[j]);
+        S[j].z = __builtin_fmaf(k4.z, u[j], S[j].z);
+        o[j] = __builtin_fmaf(S[j].z, q4.z, o[j]);
+        S[j].w = __builtin_fmaf(k4.w, u[j], S[j].w);
+        o[j] = __builtin_fmaf(S[j].w, q4.w, o[j]);
+      }
+    };
+    float* rows = out + ((int64_t)(first + t0) * H + h) * dv + blockIdx.z * CB + col;
+    if (n - t0 >= TC) {
+      float part[CC][TC];
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) read(i, i);
+#pragma unroll
+      for (int t4 = 0; t4 < TC; t4 += 4) {
+        f32x4 v4[CC], b4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < CC; ++j) v4[j] = *reinterpret_cast<const f32x4*>(base + V_AT + (col + j) * TC + t4);
+        if (DELTA) b4 = *reinterpret_cast<const f32x4*>(base + B_AT + t4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int at = (t4 + i) % AHEAD;
+          const f32x4 k4 = kn[at], q4 = qn[at], g4 = gn[at];
+          if (t4 + i + AHEAD < TC) read(t4 + i + AHEAD, at);
+          float v[CC], o[CC];
+#pragma unroll
+          for (int j = 0; j < CC; ++j) v[j] = v4[j][i];
+          step(k4, q4, g4, v, b4[i], o);
+#pragma unroll
+          for (int j = 0; j < CC; ++j) part[j][t4 + i] = o[j];
+        }
+      }
+      // Every lane ends with one token's sums over a row of 16 lanes.  With 32 lanes a column the swap of two rows adds the other
+      // row's: of two columns the first one's sum then is in the even rows and the second's in the odd ones.
+      float sums[CC];
+#pragma unroll
+      for (int j = 0; j < CC; ++j) sums[j] = walk_sums(part[j], token);
+      float* row = rows + (int64_t)token * H * dv;
+      if constexpr (W::LANES == 32) {
+        const unsigned a = __builtin_bit_cast(unsigned, sums[0]), z = __builtin_bit_cast(unsigned, sums[CC - 1]);
+        const float o = pair_sum(__builtin_amdgcn_permlane16_swap(a, z, false, false));
+        if (CC == 2) row[(lane >> 4) & 1] = o;
+        else if ((lane & 16) == 0) row[0] = o;
+      } else {
+#pragma unroll
+        for (int j = 0; j < CC; ++j) row[j] = sums[j];
+      }
+    } else {
+      for (int tok = 0; tok < n - t0; ++tok) {
+        read(tok, 0);
+        float v[CC], o[CC];
+#pragma unroll
+        for (int j = 0; j < CC; ++j) v[j] = base[V_AT + (col + j) * TC + tok];
+        step(kn[0], qn[0], gn[0], v, DELTA ? base[B_AT + tok] : 0.f, o);
+#pragma unroll
+        for (int j = 0; j < CC; ++j) {
+          o[j] = group_sum<W::LANES>(o[j]);
+          if (r == 0) rows[(int64_t)tok * H * dv + j] = o[j];
+        }
+      }
+    }
+    if (t0 + TC < n) stage(smem + (buffer ^ 1) * BUF);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < CC; ++j) *reinterpret_cast<f32x4*>(S_mem + (int64_t)j * D) = S[j];
+}
+
+// The same for a step of single tokens: no LDS, a lane holds four channels of four columns, and states, q, k and decays are asked for
+// together.  What bounds it is the states' way in and out; the walk's workgroups, with LDS for chunks of tokens, did not all fit the
+// device at once.  8 tokens x 32 heads of 128 x 128 (33.5 MB): 18.6 -> 6.2 us.
+template <int D, bool DELTA, typename IN, bool HEAD_DECAY>
+__global__ __launch_bounds__(RULE_THREADS) void rule_token_kernel(float* __restrict__ out, const IN* __restrict__ qkv, int64_t ld, int q_col, int k_col,
+                                                                  int v_col, const float* __restrict__ decay, const elem_t* __restrict__ b, int64_t ldb,
+                                                                  float* state, int64_t state_stride, const int32_t* __restrict__ cu_q,
+                                                                  const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, int H, int G,
+                                                                  int dv, float q_scale) {
+  constexpr int LANES = D / 4, CC = 4, CB = 4 * (64 / LANES) * CC;
+  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane % LANES, col = blockIdx.z * CB + (wave * (64 / LANES) + lane / LANES) * CC;
+  if (col >= dv) return;                            // columns are whole groups of four; no barrier follows
+  const int g = h / (H / G);
+  const int64_t t = cu_q[s];
+  const bool fresh = positions[t] == 0;
+  float* S_mem = state + (int64_t)slots[s] * state_stride + ((int64_t)h * dv + col) * D + r * 4;
+  f32x4 S[CC];
+#pragma unroll
+  for (int j = 0; j < CC; ++j) S[j] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(S_mem + (int64_t)j * D);
+  const IN* row = qkv + t * ld;
+  float k4[4], q4[4], g4[4], v[CC], o[CC];
+  load_row<4>(row + k_col + (int64_t)g * D + r * 4, k4);
+  load_row<4>(row + q_col + (int64_t)g * D + r * 4, q4);
+  if (HEAD_DECAY) {
+    const float head_g = decay[h];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g4[i] = head_g;
+  } else {
+    load_row<4>(decay + (t * H + h) * D + r * 4, g4);
+  }
+#pragma unroll
+  for (int j = 0; j < CC; ++j) v[j] = to_f32(row[v_col + (int64_t)h * dv + col + j]);
+  const float beta = DELTA ? sigmoid_f(to_f32(b[t * ldb + h])) : 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q4[i] = DELTA ? q4[i] : q4[i] * q_scale;
+#pragma unroll
+  for (int j = 0; j < CC; ++j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j][i] = S[j][i] * g4[i];
+    if (DELTA) {
+      float dot = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(S[j][i], k4[i], dot);
+      v[j] = beta * (v[j] - group_sum<LANES>(dot));
+    }
+    o[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      S[j][i] = __builtin_fmaf(k4[i], v[j], S[j][i]);
+      o[j] = __builtin_fmaf(S[j][i], q4[i], o[j]);
+    }
+    *reinterpret_cast<f32x4*>(S_mem + (int64_t)j * D) = S[j];
+    o[j] = group_sum<LANES>(o[j]);
+  }
+  if (r == 0) {
+#pragma unroll
+    for (int j = 0; j < CC; ++j) out[(t * H + h) * dv + col + j] = o[j];
+  }
+}
+
 // y[t, h, :] = o / sqrt(mean(o^2) + eps) * w * sigmoid(gate[t, h, :]) (gate_kind 1: * silu(gate[t, h, :])), stored as elements in rows of length ldy; the
 // columns beyond the heads are set to zero (a projection with padded columns reads them).  One wave per (token, head).
 __global__ __launch_bounds__(64) void delta_out_kernel(elem_t* __restrict__ y, int64_t ldy, const float* __restrict__ o,
@@ -456,19 +746,60 @@ int vk_delta_prep(float* x, int64_t ld, int q_col, int k_col, int T, int G, int 
   return vk_check_launch("delta prep");
 }
 
+static int rule_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    cus = n > 0 ? n : 256;
+  }
+  return cus;
+}
+
 // out [T, H, dv] floats.  qkv: float rows of length ld with q (G heads of d) at q_col, k at k_col, v (H heads of dv) at
 // v_col; decay [T, H, d] floats; b: elements, beta's pre-activation of head h at b[t * ldb + h].  state: per slot,
-// the H states at its start, each [dv][d].
+// the H states at its start, each [dv][d].  T: the step's tokens, at least one a sequence.
 extern "C++" {
 template <bool DELTA, typename IN, bool HEAD_DECAY = false>
 static int rule_launch(float* out, const IN* qkv, int64_t ld, int q_col, int k_col, int v_col, const float* decay, const elem_t* b, int64_t ldb,
-                       float* state, int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int S, int H, int G,
+                       float* state, int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T, int S, int H, int G,
                        int d, int dv, float q_scale, hipStream_t st) {
   VK_REQUIRE(S >= 0 && H > 0 && G > 0 && H % G == 0 && d > 0 && dv > 0, "delta rule: bad sizes H=%d G=%d d=%d dv=%d", H, G, d, dv);
   VK_REQUIRE(decay != nullptr, "delta rule: the decays are missing");
   VK_REQUIRE(d <= 1024, "delta rule: key size %d exceeds 1024", d);
   VK_REQUIRE(state_stride >= (int64_t)H * d * dv, "delta rule: the state is too small");
   if (S == 0) return 0;
+  // Key sizes 64 and 128 whose rows are whole vectors go by the kernels made for them: a step of single tokens, four columns a lane at a
+  // time; prompts in chunks where the value columns fill whole workgroups.  Every other shape keeps the walk for all of them.
+  const auto whole = [](int64_t n, size_t bytes) { return n * (int64_t)bytes % 16 == 0; };
+  const bool vectors = (d == 64 || d == 128) && whole(ld, sizeof(IN)) && whole(q_col, sizeof(IN)) && whole(k_col, sizeof(IN)) &&
+                       whole(state_stride, sizeof(float)) && (((uintptr_t)qkv | (uintptr_t)state | (uintptr_t)out) & 15) == 0 &&
+                       (HEAD_DECAY || ((uintptr_t)decay & 15) == 0);
+#define RULE_ARGS out, qkv, ld, q_col, k_col, v_col, decay, b, ldb, state, state_stride, cu_q, positions, slots, H, G, dv, q_scale
+  if (vectors && T == S && dv % 4 == 0) {
+    const int block = d == 64 ? 64 : 32;              // columns of a workgroup
+    const dim3 tgrid(S, H, (dv + block - 1) / block);
+    VK_REQUIRE(tgrid.y <= 65535 && tgrid.z <= 65535, "delta rule: too many heads or columns");
+    if (d == 64) rule_token_kernel<64, DELTA, IN, HEAD_DECAY><<<tgrid, RULE_THREADS, 0, st>>>(RULE_ARGS);
+    else rule_token_kernel<128, DELTA, IN, HEAD_DECAY><<<tgrid, RULE_THREADS, 0, st>>>(RULE_ARGS);
+    return vk_check_launch("delta rule (single tokens)");
+  }
+  // One column a lane while that is no more than two workgroups a compute unit, two columns beyond: twice the waves, or two thirds of
+  // the instructions a token and column (2,048 tokens of 32 heads, a column each against two: linear 192 and 222 us, delta 333 and 365,
+  // of 8 heads 142 and 194, 272 and 350; three prompts of 1,111, 741 and 370 tokens and 32 heads: 207 and 166, 401 and 311).
+  const int per = 256 / (d / 4);                      // columns of a workgroup with a column a lane
+  const int walk_cols = (int64_t)S * H * ((dv + per - 1) / per) <= 2 * (int64_t)rule_cus() ? per : 2 * per;
+  if (vectors && T > S && dv % walk_cols == 0) {
+    const dim3 wgrid(S, H, dv / walk_cols);
+    VK_REQUIRE(wgrid.y <= 65535 && wgrid.z <= 65535, "delta rule: too many heads or columns");
+#define WALK(DD, CC) rule_walk_kernel<DD, CC, DELTA, IN, HEAD_DECAY><<<wgrid, RULE_THREADS, 0, st>>>(RULE_ARGS)
+    if (d == 64) { if (walk_cols == per) WALK(64, 1); else WALK(64, 2); }
+    else { if (walk_cols == per) WALK(128, 1); else WALK(128, 2); }
+#undef WALK
+    return vk_check_launch("delta rule (chunks)");
+  }
+#undef RULE_ARGS
   const int R = vk_delta_lanes_per_column(d), DR = rule_channels_per_lane(d);
   const int cols = 4 * 64 / R;
   const dim3 grid(S, H, (dv + cols - 1) / cols);
@@ -496,9 +827,9 @@ static int rule_launch(float* out, const IN* qkv, int64_t ld, int q_col, int k_c
 }  // extern "C++"
 
 int vk_delta_rule(float* out, const float* qkv, int64_t ld, int q_col, int k_col, int v_col, const float* decay, const elem_t* b, int64_t ldb,
-                  float* state, int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int S, int H, int G,
+                  float* state, int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T, int S, int H, int G,
                   int d, int dv, hipStream_t st) {
-  return rule_launch<true, float>(out, qkv, ld, q_col, k_col, v_col, decay, b, ldb, state, state_stride, cu_q, positions, slots, S, H, G, d, dv, 1.f,
+  return rule_launch<true, float>(out, qkv, ld, q_col, k_col, v_col, decay, b, ldb, state, state_stride, cu_q, positions, slots, T, S, H, G, d, dv, 1.f,
                                   st);
 }
 
@@ -515,18 +846,18 @@ int vk_gla_decay(float* g, const elem_t* a, int64_t lda, const void* bias, int w
 // The recurrence S <- diag(g) S + k v^T, o = S^T (q * q_scale) per head.  x: element rows of length ld with q (H heads of
 // d) at q_col, k at k_col, v (H heads of dv) at v_col; decay [T, H, d] floats; out [T, H, dv] floats; state as vk_delta_rule's.
 int vk_gla_rule(float* out, const elem_t* x, int64_t ld, int q_col, int k_col, int v_col, const float* decay, float* state, int64_t state_stride,
-                const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int S, int H, int d, int dv, float q_scale, hipStream_t st) {
-  return rule_launch<false, elem_t>(out, x, ld, q_col, k_col, v_col, decay, nullptr, 0, state, state_stride, cu_q, positions, slots, S, H, H, d, dv,
+                const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T, int S, int H, int d, int dv, float q_scale, hipStream_t st) {
+  return rule_launch<false, elem_t>(out, x, ld, q_col, k_col, v_col, decay, nullptr, 0, state, state_stride, cu_q, positions, slots, T, S, H, H, d, dv,
                                     q_scale, st);
 }
 
 // Linear attention with one fixed decay a head: S <- decay[h] S + k v^T, o = S^T (q * q_scale), with q, k (H heads of d) and v
 // (H heads of dv) the elements at the three columns of x.  head_decay [H] floats.
 int vk_linear_rule(float* out, const elem_t* x, int64_t ld, int q_col, int k_col, int v_col, const float* head_decay, float* state,
-                   int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int S, int H, int d, int dv, float q_scale,
+                   int64_t state_stride, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T, int S, int H, int d, int dv, float q_scale,
                    hipStream_t st) {
   VK_REQUIRE(head_decay != nullptr, "linear attention: the heads' decays are missing");
-  return rule_launch<false, elem_t, true>(out, x, ld, q_col, k_col, v_col, head_decay, nullptr, 0, state, state_stride, cu_q, positions, slots, S, H, H, d,
+  return rule_launch<false, elem_t, true>(out, x, ld, q_col, k_col, v_col, head_decay, nullptr, 0, state, state_stride, cu_q, positions, slots, T, S, H, H, d,
                                           dv, q_scale, st);
 }
 

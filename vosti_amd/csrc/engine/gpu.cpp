@@ -111,7 +111,7 @@ struct Kernels::Fn {
   int (*delta_unit)(P, int64_t, int, int, int, int, float, float, hipStream_t);
   int (*delta_decay)(P, CP, CP, CP, int, int, int, int, hipStream_t);
   int (*delta_prep)(P, int64_t, int, int, int, int, int, int, float, float, P, CP, CP, CP, int, hipStream_t);
-  int (*delta_rule)(P, CP, int64_t, int, int, int, CP, CP, int64_t, P, int64_t, CP, CP, CP, int, int, int, int, int, hipStream_t);
+  int (*delta_rule)(P, CP, int64_t, int, int, int, CP, CP, int64_t, P, int64_t, CP, CP, CP, int, int, int, int, int, int, hipStream_t);
   int (*delta_out)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, hipStream_t);
   int (*delta_conv_bias)(P, CP, int64_t, CP, CP, P, int64_t, int64_t, CP, CP, CP, CP, int, int, int, int, hipStream_t);
   int (*paged_attention_blocked)(P, CP, CP, CP, CP, int, CP, CP, CP, int, int, int, P, int, int, int, int, int, int, float, float, CP, int,
@@ -133,7 +133,7 @@ struct Kernels::Fn {
   int (*qkv_post_norm_angles)(CP, int64_t, P, P, P, CP, CP, int, int, float, CP, float, int, CP, CP, int, int, int, int, int, hipStream_t);
   int (*gate_mul)(P, int64_t, CP, int64_t, int, int, int, hipStream_t);
   int (*gla_decay)(P, CP, int64_t, CP, int, int, int, float, hipStream_t);
-  int (*gla_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, float, hipStream_t);
+  int (*gla_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*gated_head_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, int, hipStream_t);
   int (*moe_route_bias)(P, P, P, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*moe_up_plain)(P, int64_t, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
@@ -149,7 +149,7 @@ struct Kernels::Fn {
   int (*gemm_heads)(P, int64_t, int64_t, CP, int64_t, int64_t, CP, int, int, int, int, hipStream_t);
   int (*latent_post)(CP, int64_t, CP, int64_t, int64_t, int, P, P, P, CP, int, float, CP, float, int, CP, CP, int, int, int, int, int, int, hipStream_t);
   int (*qkv_post_norm_angles_paired)(CP, int64_t, P, P, P, CP, CP, int, int, float, CP, float, int, int, CP, CP, int, int, int, int, int, hipStream_t);
-  int (*linear_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, float, hipStream_t);
+  int (*linear_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*side_gate)(P, int64_t, CP, int64_t, CP, int64_t, CP, int, int, int, hipStream_t);
   int (*gated_row_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, float, int, hipStream_t);
   int (*silu_columns)(P, int64_t, int64_t, int, int, hipStream_t);
@@ -712,7 +712,7 @@ Tensor Kernels::delta_rule(const Tensor& qkv, int q_col, int k_col, int v_col, c
   Tensor out = empty({T, H, dv}, DType::F32);
   call(fn_->delta_rule(out.data, qkv.data, qkv.dim(1), q_col, k_col, v_col, decay.data,
                        static_cast<const char*>(b.data) + (size_t)b_col * dtype_bytes(dtype_), b.dim(1), state.data, state.dim(1), cu_q.data,
-                       positions.data, slots.data, (int)S, H, G, d, dv, stream));
+                       positions.data, slots.data, (int)T, (int)S, H, G, d, dv, stream));
   return out;
 }
 
@@ -854,7 +854,7 @@ Tensor Kernels::gla_rule(const Tensor& x, int64_t q_col, int64_t k_col, int64_t 
   expect(slots, "state slots", DType::I32, {S});
   Tensor out = empty({T, H, dv}, DType::F32);
   call(fn_->gla_rule(out.data, x.data, x.dim(1), (int)q_col, (int)k_col, (int)v_col, decay.data, state.data, state.dim(1), cu_q.data, positions.data,
-                     slots.data, (int)S, H, d, dv, q_scale, stream));
+                     slots.data, (int)T, (int)S, H, d, dv, q_scale, stream));
   return out;
 }
 
@@ -1306,7 +1306,7 @@ Tensor Kernels::linear_rule(const Tensor& x, int64_t q_col, int64_t k_col, int64
   expect(slots, "state slots", DType::I32, {S});
   Tensor out = empty({T, H, dv}, DType::F32);
   call(fn_->linear_rule(out.data, x.data, x.dim(1), (int)q_col, (int)k_col, (int)v_col, head_decay.data, state.data, state.dim(1),
-                        cu_q.data, positions.data, slots.data, (int)S, H, d, dv, q_scale, stream));
+                        cu_q.data, positions.data, slots.data, (int)T, (int)S, H, d, dv, q_scale, stream));
   return out;
 }
 
