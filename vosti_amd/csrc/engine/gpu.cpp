@@ -161,7 +161,7 @@ struct Kernels::Fn {
   int (*attention_wide_limit)();
   int (*gemm_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_split_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
-  int (*gemm_grouped_act)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, int, hipStream_t);
+  int (*gemm_grouped_act)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, CP, int, hipStream_t);
   int (*moe_route_corrected)(P, P, P, CP, CP, CP, int, int, int, int, int, int, int, int, float, hipStream_t);
   int (*stream_add_norm)(P, P, CP, int, CP, int, int, int, float, hipStream_t);
   int (*embed_bigram)(P, CP, CP, CP, CP, int, int, int, int64_t, int64_t, int64_t, hipStream_t);
@@ -1361,7 +1361,8 @@ void Kernels::relu_square(Tensor& x) {
 
 bool Kernels::gemm_grouped_takes(int64_t K) const { return K % (dtype_ == DType::BF16 ? 64 : 32) == 0; }
 
-Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation) {
+Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation, const Tensor* row_pair) {
+  if (row_pair) expect(*row_pair, "rows' pairs", DType::I32, {act.dim(0)});
   expect(act, "activation", dtype_);
   expect(w, "weights", dtype_);
   if (act.shape.size() != 2 || w.shape.size() != 3 || act.dim(1) != w.dim(2) || act.dim(0) % 128 || !gemm_grouped_takes(act.dim(1)))
@@ -1369,7 +1370,7 @@ Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& b
   expect(block_weights, "the blocks' matrices", DType::I32, {act.dim(0) / 128});
   Tensor out = empty({act.dim(0), w.dim(1)});
   call(fn_->gemm_grouped_act(out.data, act.data, w.data, (int)act.dim(0), (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), block_weights.data,
-                             w.dim(1) * w.dim(2), activation, stream));
+                             w.dim(1) * w.dim(2), row_pair ? row_pair->data : nullptr, activation, stream));
   return out;
 }
 

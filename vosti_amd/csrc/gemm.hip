@@ -517,17 +517,6 @@ static int launch_tiled(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // computed meanwhile.  One barrier per K tile.  Rows beyond N or M are clamped
 // (their results are dropped).  Same tile shape, swizzle and reduction order as
 // gemm_tiled_kernel<4, 4>.
-__device__ __forceinline__ void wait_vmcnt(int n) {
-  // s_waitcnt with only vmcnt set: vmcnt is bits [3:0] and [15:14]; expcnt and lgkmcnt left at their maxima.
-  switch (n) {
-    case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-    case 8: __builtin_amdgcn_s_waitcnt(0x0F78); break;
-    case 16: __builtin_amdgcn_s_waitcnt(0x4F70); break;
-    case 24: __builtin_amdgcn_s_waitcnt(0x4F78); break;
-    default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-  }
-}
-
 // With SWIGLU the weight holds N gate rows, then N up rows, and the output has N columns: a workgroup
 // takes 64 gate rows and the matching 64 up rows as its 128 weight rows (the waves with wn = 0 the
 // gate, those with wn = 1 the up projection), and at the end the up values pass through LDS to the
@@ -568,14 +557,18 @@ __device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ be
 }
 
 // PFD > 0: every wave touches, PFD tiles ahead, the 64 rows of the workgroup's tiles that are its share.
-template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int PFD = 0>
-__global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act,
+// NWN: waves along the weight rows, two of a workgroup of four waves or four of eight, which takes 64 FNW weight rows.
+template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int PFD = 0, int NWN = 2>
+__global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act,
                                                         const elem_t* __restrict__ w, int M, int N, int K,
                                                         int64_t lda, int64_t ldo, int out_form, int band_w,
-                                                        const int32_t* __restrict__ block_weights, int64_t weights_stride) {
+                                                        const int32_t* __restrict__ block_weights, int64_t weights_stride,
+                                                        const int32_t* __restrict__ row_pair) {
   static_assert(FNW >= 2 && FNW <= 5 && (FNW == 4 || !SWIGLU), "two to five weight fragments per wave; four with SwiGLU");
   static_assert(PFD == 0 || FNW == 2 || FNW == 4, "the touch-ahead wants a wave's 64 rows to be of one kind");
-  constexpr int BN = 32 * FNW;                          // weight rows of the workgroup
+  static_assert(NWN == 2 || (NWN == 4 && !SWIGLU && PFD == 0), "two waves or four along the weight rows");
+  constexpr int BN = 16 * FNW * NWN;                    // weight rows of the workgroup
+  constexpr int NA = 8 / NWN, PER_TILE = FNW + NA;      // loads of activation rows, and all loads, per K tile and wave
   constexpr int W_BYTES = BN * T_ROWB, STAGE_BYTES = W_BYTES + 128 * T_ROWB;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [stage][w tile, act tile]
 
@@ -583,7 +576,7 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
   // then needs no vector registers.
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
-  const int wn = wave & 1, wm = wave >> 1;
+  const int wn = wave % NWN, wm = wave / NWN;
   // Workgroups start in the order of their linear index.  That order walks bands of band_w column
   // blocks: all row blocks of a band before the next band, so that a band's weights are read from HBM
   // once and found in the caches by the other row blocks (a matrix larger than the memory-side cache
@@ -606,6 +599,9 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
   }
   const int n_blk = nb * (SWIGLU ? 64 : BN), m_blk = mb * 128;
   const int ntiles = K / (2 * VK_SLAB);
+  // A wave without rows (the second half of a group's last block of up to 64 rows: rows without a pair come last in a group) helps to
+  // bring the tiles in and leaves the matrix unit to the others.
+  const bool idle = NWN == 4 && row_pair != nullptr && wm == 1 && row_pair[m_blk + 64] < 0;
 
   // A wave-level load moves 8 rows x 128 bytes; lane i fills LDS slot i of the 1 KB block, which is
   // row i/8, physical 16-byte column i%8, i.e. logical column (i%8) ^ (i/8).
@@ -616,7 +612,7 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
   const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (int64_t)min(n_blk, N - 1) * K);
   const unsigned char* ubase = reinterpret_cast<const unsigned char*>(w + (int64_t)(N + min(n_blk, N - 1)) * K);   // SWIGLU: the up rows
   const unsigned char* abase = reinterpret_cast<const unsigned char*>(act + (int64_t)min(m_blk, M - 1) * lda);
-  unsigned offw[FNW], offa[4];
+  unsigned offw[FNW], offa[NA];
 #pragma unroll
   for (int j = 0; j < FNW; ++j) {
     const int row = (wave * FNW + j) * 8 + lr;
@@ -625,12 +621,12 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
     offw[j] = (unsigned)(((int64_t)clamped * K + lc * VK_VEC) * (int64_t)sizeof(elem_t));
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int clamped = min(m_blk + (wave * 4 + j) * 8 + lr, M - 1) - min(m_blk, M - 1);
+  for (int j = 0; j < NA; ++j) {
+    const int clamped = min(m_blk + (wave * NA + j) * 8 + lr, M - 1) - min(m_blk, M - 1);
     offa[j] = (unsigned)(((int64_t)clamped * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
   }
   const unsigned lds0 = lds_offset_of(lds);
-  auto issue = [&](int kt) {                 // FNW + 4 loads per wave
+  auto issue = [&](int kt) {                 // PER_TILE loads per wave
     const unsigned base = lds0 + (kt % S) * STAGE_BYTES;
     const int64_t kb = (int64_t)kt * 2 * VK_SLAB * (int64_t)sizeof(elem_t);
 #pragma unroll
@@ -639,7 +635,7 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
       pipe_load_to_lds16_sv((up ? ubase : wbase) + kb, offw[j], base + (wave * FNW + j) * 8 * T_ROWB);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) pipe_load_to_lds16_sv(abase + kb, offa[j], base + W_BYTES + (wave * 4 + j) * 8 * T_ROWB);
+    for (int j = 0; j < NA; ++j) pipe_load_to_lds16_sv(abase + kb, offa[j], base + W_BYTES + (wave * NA + j) * 8 * T_ROWB);
   };
 
   // The lines a wave touches ahead: row wave * 64 + lane of the workgroup's weight rows followed by its
@@ -672,14 +668,26 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe_kernel(elem_t* __restrict__ 
 #pragma unroll
   for (int p = 0; p < S - 1; ++p)
     if (p < ntiles) issue(p);
+  if (idle) {
+    for (int kt = 0; kt < ntiles; ++kt) {
+      if (S == 2 || kt + 1 == ntiles) wait_vmcnt_n<0>();
+      else if (S == 3 || kt + 2 == ntiles) wait_vmcnt_n<PER_TILE>();
+      else wait_vmcnt_n<2 * PER_TILE>();
+      __syncthreads();
+      if (kt + S - 1 < ntiles) issue(kt + S - 1);
+    }
+    return;
+  }
 
   auto step = [&](int kt) {
-    // Tile kt has landed once at most the loads of the tiles after it are outstanding (FNW + 4 per tile and wave).
+    // Tile kt has landed once at most the loads of the tiles after it are outstanding (PER_TILE per tile and wave).
     if (PFD > 0) {
       if (kt == 0) wait_vmcnt_n<0>(); else wait_vmcnt_n<1>();      // the one touch that was issued behind tile kt's loads may still fly
     } else {
       const int later = min(S - 2, ntiles - 1 - kt);
-      wait_vmcnt((FNW + 4) * later);
+      if (later == 0) wait_vmcnt_n<0>();
+      else if (later == 1) wait_vmcnt_n<PER_TILE>();
+      else wait_vmcnt_n<2 * PER_TILE>();
     }
     __syncthreads();       // every wave's part of tile kt is there; everyone is done with tile kt-1's buffer
     if (kt + S - 1 < ntiles) issue(kt + S - 1);
@@ -794,7 +802,8 @@ static const int pipe_band_blocks = 64;
 
 template <int S, bool SWIGLU = false, int FNW = 4>
 static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
-                       int form, hipStream_t st, const int32_t* block_weights = nullptr, int64_t weights_stride = 0) {
+                       int form, hipStream_t st, const int32_t* block_weights = nullptr, int64_t weights_stride = 0,
+                       const int32_t* row_pair = nullptr) {
   constexpr int BN = SWIGLU ? 64 : 32 * FNW;                         // output columns of a workgroup
   const size_t smem = (size_t)S * (32 * FNW + 128) * T_ROWB;         // also holds the 32 KB that SWIGLU passes between waves
   static bool configured = false;
@@ -805,6 +814,27 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   }
   dim3 grid((N + BN - 1) / BN, (M + 127) / 128);
   VK_REQUIRE(grid.y <= 65535, "gemm: too many rows (%d)", M);
+  if constexpr (S == 2 && !SWIGLU && FNW == 4 && sizeof(elem_t) == 2) {
+    // A grouped product is bound by its weights' way from memory: an expert's matrix serves two or three blocks of rows where a dense
+    // product's serves all of them.  Workgroups of 256 weight rows (eight waves) with three stages have two tiles of 48 KB on their way
+    // a compute unit where two workgroups of 128 with two stages have two of 32, and 16 column blocks of all row blocks before the next
+    // 16 keep the blocks of an expert together in time and on their chip part.  Measured on MI355X, 32 experts, before and after with the
+    // idle waves: 2,048 tokens x 3 choices, 6,144 x 4,096 weights 548 -> 484 us, 4,096 x 3,072 290 -> 241; 2,445 x 4, 6,144 x 4,096 690 ->
+    // 615; 700 x 3 394 -> 339; 1,360 x 3, 4,608 x 4,096 367 -> 327; 1,334 x 4, 2,048 x 1,536 66 -> 68.  (Touching the weights' lines two to
+    // eight tiles ahead instead: 548 -> 586 to 699.)
+    if (block_weights != nullptr && K % KC == 0) {
+      constexpr size_t wide_smem = (size_t)3 * (256 + 128) * T_ROWB;
+      static bool wide = false;
+      if (!wide) {
+        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<3, true, false, 4, 0, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_smem);
+        wide = true;
+      }
+      const dim3 wgrid((N + 255) / 256, grid.y);
+      gemm_pipe_kernel<3, true, false, 4, 0, 4><<<wgrid, 512, wide_smem, st>>>(out, act, w, M, N, K, lda, ldo, form, wgrid.x > 16 ? 16 : (int)wgrid.x, block_weights,
+                                                                              weights_stride, row_pair);
+      return vk_check_launch("gemm_pipe (grouped)");
+    }
+  }
   const int band_w = (pipe_band_blocks > 0 && grid.y > 1 && (int)grid.x > pipe_band_blocks) ? pipe_band_blocks : (int)grid.x;
   if constexpr (S == 2 && (FNW == 2 || FNW == 4)) {
     // No more workgroups than compute units: each waits for its own loads with nothing to run meanwhile, and
@@ -817,12 +847,12 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
         (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         touched = true;
       }
-      gemm_pipe_kernel<S, true, SWIGLU, FNW, 4><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride);
+      gemm_pipe_kernel<S, true, SWIGLU, FNW, 4><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
       return vk_check_launch("gemm_pipe");
     }
   }
-  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride);
-  else gemm_pipe_kernel<S, false, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride);
+  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
+  else gemm_pipe_kernel<S, false, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
   return vk_check_launch("gemm_pipe");
 }
 
@@ -1293,9 +1323,10 @@ static int out_form_of(const elem_t* out, int64_t ldo, int activation) {
 // A grouped product through the tile kernel: rows in blocks of 128, block b multiplied by the weight matrix
 // block_weights[b] of several [N, K] matrices that lie weights_stride elements apart (negative: the block is skipped and
 // its output rows are left as they are).  K in whole pairs of slabs (128 bytes of a row).  The same bits as vk_gemm gives
-// for the same rows and matrix.
+// for the same rows and matrix.  row_pair [M] or null: a block whose row 64 has a negative entry has no rows from there on, and its
+// outputs there are left as they are.
 int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
-                        const int32_t* block_weights, int64_t weights_stride, int activation, hipStream_t st) {
+                        const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, int activation, hipStream_t st) {
   VK_REQUIRE(activation == 0 || activation == 1, "grouped gemm: unknown activation %d", activation);
   VK_REQUIRE(M >= 0 && N > 0 && K > 0 && M % 128 == 0, "grouped gemm: bad sizes M=%d N=%d K=%d (rows in blocks of 128)", M, N, K);
   VK_REQUIRE(K % (2 * VK_SLAB) == 0, "grouped gemm: K=%d must be a multiple of %d", K, 2 * VK_SLAB);
@@ -1303,12 +1334,12 @@ int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, 
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0 && block_weights != nullptr && weights_stride % VK_VEC == 0,
              "grouped gemm: operands must be 16-byte aligned");
   if (M == 0) return 0;
-  return launch_pipe<2>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride);
+  return launch_pipe<2>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair);
 }
 
 int vk_gemm_grouped(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                     const int32_t* block_weights, int64_t weights_stride, hipStream_t st) {
-  return vk_gemm_grouped_act(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, 0, st);
+  return vk_gemm_grouped_act(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, nullptr, 0, st);
 }
 
 // kernel: 0 = choose by size, 1 = skinny (M <= 64), 2 = tiled (pipelined if K allows), 3 = tiled through
