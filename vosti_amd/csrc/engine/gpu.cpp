@@ -126,8 +126,8 @@ struct Kernels::Fn {
   int (*gemm_grouped)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, hipStream_t);
   int (*moe_route)(P, P, P, CP, CP, int, int, int, int, float, hipStream_t);
   int (*moe_plan)(CP, P, P, P, P, P, int, int, int, int, hipStream_t);
-  int (*moe_up)(P, int64_t, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
-  int (*moe_down)(P, CP, int64_t, CP, CP, CP, int, int, int, int, int, hipStream_t);
+  int (*moe_up)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
+  int (*moe_down)(P, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_combine)(P, CP, CP, CP, int, int, int, hipStream_t);
   int (*moe_relu_square)(P, int64_t, hipStream_t);
   int (*qkv_post_norm_angles)(CP, int64_t, P, P, P, CP, CP, int, int, float, CP, float, int, CP, CP, int, int, int, int, int, hipStream_t);
@@ -136,7 +136,7 @@ struct Kernels::Fn {
   int (*gla_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*gated_head_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, int, hipStream_t);
   int (*moe_route_bias)(P, P, P, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
-  int (*moe_up_plain)(P, int64_t, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
+  int (*moe_up_plain)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_glu)(P, CP, int64_t, int, float, float, float, hipStream_t);
   int (*moe_combine_add)(P, CP, CP, CP, CP, int, int, int, hipStream_t);
   int (*stream_norm_add_f32)(P, CP, CP, CP, int, int, int, float, float, float, hipStream_t);
@@ -983,7 +983,7 @@ Tensor Kernels::moe_up(const Tensor& h, const Tensor& w_up, const MoePlan& plan)
     throw EngineError("experts (up): input " + h.describe() + ", weights " + w_up.describe());
   const int64_t T = h.dim(0), N = w_up.dim(1);
   Tensor act = empty({plan.row_pair.dim(0), N});
-  call(fn_->moe_up(act.data, N, h.data, h.dim(1), w_up.data, plan.row_pair.data, plan.row_token.data, plan.tile_expert.data, (int)T, plan.top,
+  call(fn_->moe_up(act.data, N, h.data, h.dim(1), w_up.data, plan.row_pair.data, plan.row_token.data, plan.tile_expert.data, plan.expert_start.data, (int)T, plan.top,
                    plan.experts, (int)N, (int)h.dim(1), stream));
   return act;
 }
@@ -996,7 +996,7 @@ Tensor Kernels::moe_down(const Tensor& act, const Tensor& w_down, const MoePlan&
     throw EngineError("experts (down): activations " + act.describe() + ", weights " + w_down.describe());
   const int64_t W = w_down.dim(1), T = plan.idx.dim(0);
   Tensor y = empty({act.dim(0), W});
-  call(fn_->moe_down(y.data, act.data, act.dim(1), w_down.data, plan.row_pair.data, plan.tile_expert.data, (int)T, plan.top, plan.experts, (int)W,
+  call(fn_->moe_down(y.data, act.data, act.dim(1), w_down.data, plan.row_pair.data, plan.tile_expert.data, plan.expert_start.data, (int)T, plan.top, plan.experts, (int)W,
                      (int)act.dim(1), stream));
   return y;
 }
@@ -1009,7 +1009,7 @@ Tensor Kernels::moe_up_plain(const Tensor& h, const Tensor& w, const MoePlan& pl
     throw EngineError("experts (up): input " + h.describe() + ", weights " + w.describe());
   const int64_t T = h.dim(0), N = w.dim(1);
   Tensor act = empty({plan.row_pair.dim(0), N});
-  call(fn_->moe_up_plain(act.data, N, h.data, h.dim(1), w.data, plan.row_pair.data, plan.row_token.data, plan.tile_expert.data, (int)T, plan.top,
+  call(fn_->moe_up_plain(act.data, N, h.data, h.dim(1), w.data, plan.row_pair.data, plan.row_token.data, plan.tile_expert.data, plan.expert_start.data, (int)T, plan.top,
                          plan.experts, (int)N, (int)h.dim(1), stream));
   return act;
 }

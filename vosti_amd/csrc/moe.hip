@@ -293,6 +293,99 @@ __global__ __launch_bounds__(64 * MOE_WAVES) void moe_gemm_kernel(elem_t* __rest
   }
 }
 
+// The same products (16-bit elements, K in whole slabs, up to MOE_STREAM_CHUNKS chunks), built to keep memory busy where the kernel above
+// is bound by its workgroups' starts: 64 to 128 KB of weights each behind three dependent loads, and idle waves where K has fewer than
+// eight chunks.  Workgroups of a wave a chunk stay for the whole launch and take equal, contiguous shares of the (row tile, 16
+// features) units of all tiles in use, tile by tile; a wave keeps its chunk of the tile's rows in registers and streams the weights
+// through a window of MOE_STREAM_W slabs that runs on across units and tiles; one barrier a unit, and the waves take turns at adding
+// up a unit's chunk sums.  No load is predicated: rows without a pair are read like others and not stored, features beyond N are clamped.
+// WHOLE: K in whole chunks; else the last chunk's missing slabs are read again from its last one and multiplied by zeros.
+// Measured on MI355X, 32 experts, eight tokens: 4 choices, 3,072 x 2,048 weights 62.7 -> 53.4 us, 2,048 x 1,536 36.5 -> 31.6 (a plain
+// read of so many bytes, 260 and 130 MB, is about as long); five tokens of 3 choices, 4,096 x 4,608 75.1 -> 70.8.
+#ifdef VK_BF16
+#define MOE_STREAM_W 8
+#define MOE_STREAM_CHUNKS 16
+template <int MODE, bool WHOLE>
+__global__ __launch_bounds__(64 * MOE_STREAM_CHUNKS) void moe_stream_kernel(elem_t* __restrict__ out, int64_t ldo, const elem_t* __restrict__ x, int64_t ldx,
+                                                                            const elem_t* __restrict__ w, int64_t expert_stride,
+                                                                            const int32_t* __restrict__ row_pair, const int32_t* __restrict__ row_token,
+                                                                            const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ expert_start,
+                                                                            int E, int N, int K, int vec) {
+  constexpr int SL = MOE_KC_SLABS, W = MOE_STREAM_W;
+  extern __shared__ f32x4 part[];                 // [2][waves][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int features = (N + 15) / 16;
+  const int64_t units = (int64_t)(expert_start[E] / MOE_TILE) * features;
+  const int lo = (int)(units * blockIdx.x / gridDim.x), hi = (int)(units * (blockIdx.x + 1) / gridDim.x);
+  if (lo >= hi) return;                           // the whole workgroup
+  const int have = WHOLE ? SL : min(SL, (K - wave * MOE_KC) / VK_SLAB);      // slabs of this wave's chunk
+  const int64_t k0 = (int64_t)wave * MOE_KC + kq * VK_VEC;
+  auto weights = [&](int tile, int f) { return w + (int64_t)tile_expert[tile] * expert_stride + (int64_t)min(f * 16 + r16, N - 1) * K + k0; };
+  auto at = [&](int i) { return (WHOLE ? i : min(i, have - 1)) * VK_SLAB; };
+  frag_t rows[SL], window[W];
+  auto bring = [&](int tile) {
+    const int row = tile * MOE_TILE + r16;
+    const elem_t* xr = x + (int64_t)(MODE != 0 ? row_token[row] : row) * ldx + k0;
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+      rows[i] = *reinterpret_cast<const frag_t*>(xr + at(i));
+      if (!WHOLE && i >= have) rows[i] = zero_frag();
+    }
+  };
+  int tile = lo / features, f = lo - tile * features;
+  const elem_t* here = weights(tile, f);
+#pragma unroll
+  for (int i = 0; i < W; ++i) window[i] = *reinterpret_cast<const frag_t*>(here + at(i));
+  bring(tile);
+  for (int u = lo, parity = 0; u < hi; ++u, parity ^= 1) {
+    const int next_f = f + 1 < features ? f + 1 : 0, next_tile = f + 1 < features ? tile : tile + 1;
+    const bool more = u + 1 < hi;
+    const elem_t* next = more ? weights(next_tile, next_f) : here;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+      const frag_t fw = window[i % W];
+      if (i + W < SL) window[i % W] = *reinterpret_cast<const frag_t*>(here + at(i + W));
+      else if (more) window[i % W] = *reinterpret_cast<const frag_t*>(next + at(i + W - SL));
+      acc = mma_slab(fw, rows[i], acc);
+    }
+    f32x4* sums = part + (size_t)parity * waves * 64;
+    sums[wave * 64 + lane] = acc;
+    __syncthreads();
+    if (wave == u % waves) {
+      f32x4 total = {0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < waves; ++c) {
+        const f32x4 p = sums[c * 64 + lane];
+        total.x = total.x + p.x; total.y = total.y + p.y; total.z = total.z + p.z; total.w = total.w + p.w;
+      }
+      if (MODE == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float rl = fmaxf(round_to_elem(total[i]), 0.f);
+          total[i] = rl * rl;
+        }
+      }
+      const int row = tile * MOE_TILE + r16, first = f * 16 + kq * 4;
+      if (row_pair[row] >= 0) {
+        elem_t* o = out + (int64_t)row * ldo + first;
+        if (vec && first + 3 < N) {
+          store_elems4(o, total);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (first + i < N) o[i] = from_f32<elem_t>(total[i]);
+        }
+      }
+    }
+    if (more && next_tile != tile) bring(next_tile);
+    tile = next_tile;
+    f = next_f;
+    here = next;
+  }
+}
+#endif
+
 // x <- max(x, 0)^2, element by element: the experts' activation on a product that was left as elements.  A thread
 // takes a 16-byte vector (n in whole vectors).
 __global__ __launch_bounds__(256) void moe_relu_square_kernel(elem_t* x, int64_t nvec) {
@@ -457,31 +550,66 @@ int vk_moe_plan(const int32_t* idx, int32_t* row_pair, int32_t* row_token, int32
   return vk_check_launch("expert plan");
 }
 
+static int moe_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    cus = n > 0 ? n : 256;
+  }
+  return cus;
+}
+
+// An expert product of rows in tiles of 16: by the streaming kernel where it takes the sizes, else by the one for every K.
+extern "C++" {
+template <int MODE>
+static int moe_product(elem_t* out, int64_t ldo, const elem_t* x, int64_t ldx, const elem_t* w, const int32_t* row_pair, const int32_t* row_token,
+                       const int32_t* tile_expert, const int32_t* expert_start, int tiles, int E, int N, int K, hipStream_t st, const char* what) {
+#ifdef VK_BF16
+  const int chunks = (K + MOE_KC - 1) / MOE_KC;
+  // Six to eight chunks keep six to eight of the other kernel's eight waves at work in one round, and its many workgroups then bring the
+  // larger matrices in as fast (three tokens, 6,144 x 4,096 weights: 90.0 us there, 91.2 here; 4,096 x 3,072: 52.7, 54.0).
+  if (K % VK_SLAB == 0 && ldx % VK_VEC == 0 && (chunks <= 5 || (chunks > MOE_WAVES && chunks <= MOE_STREAM_CHUNKS))) {
+    // As many workgroups as the device holds at once: 16 waves a compute unit (128 registers).
+    const int64_t units = (int64_t)tiles * ((N + 15) / 16);
+    const int grid = (int)std::min<int64_t>(units, (int64_t)moe_cus() * (16 / chunks));
+    const int vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
+    const size_t smem = (size_t)2 * chunks * 64 * sizeof(f32x4);
+    if (K % MOE_KC == 0)
+      moe_stream_kernel<MODE, true><<<grid, 64 * chunks, smem, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, expert_start, E, N, K, vec);
+    else
+      moe_stream_kernel<MODE, false><<<grid, 64 * chunks, smem, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, expert_start, E, N, K, vec);
+    return vk_check_launch(what);
+  }
+#endif
+  moe_gemm_kernel<MODE><<<dim3((N + 15) / 16, tiles), 64 * MOE_WAVES, 0, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, N, K);
+  return vk_check_launch(what);
+}
+}  // extern "C++"
+
 // act [max_rows, ldo] elements = relu(x[token of row] . w_up[expert of row])^2; w_up [E, N, K].
 int vk_moe_up(elem_t* act, int64_t ldo, const elem_t* x, int64_t ldx, const elem_t* w_up, const int32_t* row_pair, const int32_t* row_token,
-              const int32_t* tile_expert, int T, int top, int E, int N, int K, hipStream_t st) {
+              const int32_t* tile_expert, const int32_t* expert_start, int T, int top, int E, int N, int K, hipStream_t st) {
   VK_REQUIRE(T >= 0 && top > 0 && E > 0 && N > 0 && K > 0 && K % VK_VEC == 0 && ldx % VK_VEC == 0 && ldx >= K && ldo >= N,
              "experts (up): bad sizes N=%d K=%d (K in whole 16-byte vectors)", N, K);
   VK_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w_up % 16) == 0, "experts (up): operands must be 16-byte aligned");
   if (T == 0) return 0;
   const int tiles = vk_moe_max_tiles(T, top, E, MOE_TILE);
   VK_REQUIRE(tiles <= 65535, "experts (up): too many tiles for one launch");
-  moe_gemm_kernel<1><<<dim3((N + 15) / 16, tiles), 64 * MOE_WAVES, 0, st>>>(act, ldo, x, ldx, w_up, (int64_t)N * K, row_pair, row_token, tile_expert,
-                                                                               N, K);
-  return vk_check_launch("experts (up)");
+  return moe_product<1>(act, ldo, x, ldx, w_up, row_pair, row_token, tile_expert, expert_start, tiles, E, N, K, st, "experts (up)");
 }
 
 // act [max_rows, ldo] elements = x[token of row] . w[expert of row], no activation; w [E, N, K].
 int vk_moe_up_plain(elem_t* act, int64_t ldo, const elem_t* x, int64_t ldx, const elem_t* w, const int32_t* row_pair, const int32_t* row_token,
-                    const int32_t* tile_expert, int T, int top, int E, int N, int K, hipStream_t st) {
+                    const int32_t* tile_expert, const int32_t* expert_start, int T, int top, int E, int N, int K, hipStream_t st) {
   VK_REQUIRE(T >= 0 && top > 0 && E > 0 && N > 0 && K > 0 && K % VK_VEC == 0 && ldx % VK_VEC == 0 && ldx >= K && ldo >= N,
              "experts (up): bad sizes N=%d K=%d (K in whole 16-byte vectors)", N, K);
   VK_REQUIRE(((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0, "experts (up): operands must be 16-byte aligned");
   if (T == 0) return 0;
   const int tiles = vk_moe_max_tiles(T, top, E, MOE_TILE);
   VK_REQUIRE(tiles <= 65535, "experts (up): too many tiles for one launch");
-  moe_gemm_kernel<2><<<dim3((N + 15) / 16, tiles), 64 * MOE_WAVES, 0, st>>>(act, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, N, K);
-  return vk_check_launch("experts (up)");
+  return moe_product<2>(act, ldo, x, ldx, w, row_pair, row_token, tile_expert, expert_start, tiles, E, N, K, st, "experts (up)");
 }
 
 // out [rows, F] elements from in [rows, 2 F]: the gated activation with clamped inputs (moe_glu_kernel).
@@ -508,17 +636,15 @@ int vk_moe_glu_weighed(elem_t* out, const elem_t* in, int64_t rows, int F, float
 }
 
 // y [max_rows, N] elements = act[row] . w_down[expert of row]; w_down [E, N, K]; act rows of length lda >= K.
-int vk_moe_down(elem_t* y, const elem_t* act, int64_t lda, const elem_t* w_down, const int32_t* row_pair, const int32_t* tile_expert, int T,
-                int top, int E, int N, int K, hipStream_t st) {
+int vk_moe_down(elem_t* y, const elem_t* act, int64_t lda, const elem_t* w_down, const int32_t* row_pair, const int32_t* tile_expert,
+                const int32_t* expert_start, int T, int top, int E, int N, int K, hipStream_t st) {
   VK_REQUIRE(T >= 0 && top > 0 && E > 0 && N > 0 && K > 0 && K % VK_VEC == 0 && lda % VK_VEC == 0 && lda >= K,
              "experts (down): bad sizes N=%d K=%d (K in whole 16-byte vectors)", N, K);
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w_down % 16) == 0, "experts (down): operands must be 16-byte aligned");
   if (T == 0) return 0;
   const int tiles = vk_moe_max_tiles(T, top, E, MOE_TILE);
   VK_REQUIRE(tiles <= 65535, "experts (down): too many tiles for one launch");
-  moe_gemm_kernel<0><<<dim3((N + 15) / 16, tiles), 64 * MOE_WAVES, 0, st>>>(y, N, act, lda, w_down, (int64_t)N * K, row_pair, nullptr, tile_expert,
-                                                                                N, K);
-  return vk_check_launch("experts (down)");
+  return moe_product<0>(y, N, act, lda, w_down, row_pair, nullptr, tile_expert, expert_start, tiles, E, N, K, st, "experts (down)");
 }
 
 int vk_moe_relu_square(elem_t* x, int64_t n, hipStream_t st) {
