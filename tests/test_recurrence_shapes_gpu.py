@@ -94,3 +94,59 @@ def test_the_same_bits_as_the_walk_for_every_shape(kind, d, dtype):
         got, want = (run(k, kind, d, heads, lengths, fresh, odd, dtype) for odd in (False, True))
         assert not torch.isnan(got[0]).any()
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def run_scan(k, heads, P, lengths, fresh, odd):
+    """The state-space scan with 128 state rows over sequences of these lengths; odd: rows one number longer."""
+    g = torch.Generator().manual_seed(4)
+    T, S, H, N, G = sum(lengths), len(lengths), heads, 128, 2
+    cols = H * P + 2 * G * N
+    rows = torch.zeros(T, cols + (1 if odd else 0))
+    rows[:, :cols] = torch.randn(T, cols, generator=g)
+    dt = torch.randn(T, H, generator=g).to(k.dtype)
+    bias, A_log, D = (torch.rand(H, generator=g) for _ in range(3))
+    state = torch.randn(S + 1, H * P * N, generator=g)
+    cu = [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    positions = torch.arange(T, dtype=torch.int32)
+    for s in range(S):
+        positions[cu[s]] = 0 if fresh and s % 2 == 0 else 5
+    slots = [(s + 1) % (S + 1) for s in range(S)]
+    want = None
+    if lengths == [45]:
+        z = dt.double() + bias.double()
+        step = torch.nn.functional.softplus(z)
+        decay = torch.exp(-torch.exp(A_log.double()) * step)
+        St, want = torch.zeros(H, N, P).double(), []
+        for t in range(T):
+            row = rows[t].double()
+            x, B, C = row[:H * P].view(H, P), row[H * P:H * P + G * N].view(G, N), row[H * P + G * N:H * P + 2 * G * N].view(G, N)
+            B, C = B.repeat_interleave(H // G, 0), C.repeat_interleave(H // G, 0)
+            St = decay[t][:, None, None] * St + step[t][:, None, None] * B[:, :, None] * x[:, None, :]
+            want.append((St * C[:, :, None]).sum(1) + D.double()[:, None] * x)
+        want = torch.stack(want)
+    dev = [v.cuda() for v in (rows, dt, bias, A_log, D, state, torch.tensor(cu, dtype=torch.int32), positions, torch.tensor(slots, dtype=torch.int32))]
+    rows, dt, bias, A_log, D, state, cu, positions, slots = dev
+    y = torch.full((T, H, P), float("nan"), device="cuda")
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    fn = k.lib.vk_ssm_scan
+    fn.argtypes = [p, p, l, i, i, p, l, p, p, p, i, p, l, p, p, p, i, i, i, i, i, i, p]
+    assert fn(y.data_ptr(), rows.data_ptr(), rows.shape[1], H * P, H * P + G * N, dt.data_ptr(), H, bias.data_ptr(), A_log.data_ptr(), D.data_ptr(), 1,
+              state.data_ptr(), state.shape[1], cu.data_ptr(), positions.data_ptr(), slots.data_ptr(), S, T, H, G, N, P,
+              torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    return y.cpu(), state.cpu(), want
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("P", [48, 64])
+def test_the_state_space_scan(P, dtype):
+    k = kern(dtype)
+    for heads, lengths, fresh in ((2, [45], True), (2, [1], True), (4, [1, 1, 1], False), (4, [16], True), (4, [15, 1, 17], False), (4, [33, 2, 48], True),
+                                  (64, [17, 5, 32], False)):           # the last: so many workgroups that a lane takes two columns
+        (y, state, want), (y2, state2, _) = run_scan(k, heads, P, lengths, fresh, False), run_scan(k, heads, P, lengths, fresh, True)
+        assert not torch.isnan(y).any()
+        assert torch.equal(y, y2) and torch.equal(state, state2)
+        if want is not None:                               # 32-bit sums of 128 products and 45 decayed terms
+            assert (y.double() - want).norm() < 5e-6 * want.norm()

@@ -109,6 +109,33 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Sixteen of group_sum<16>'s sums at once (a recurrence's read-outs of 16 tokens): lane r of the 16 ends with the one of token
+// walk_token(r).  Each step of the butterfly leaves a lane half as many; whether it goes on with the first or the second of two is chosen
+// so that the partner of every later step has gone on with the same ones.
+__device__ __forceinline__ int walk_token(int r) {
+  const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;
+  return (b0 ^ b2) | (b1 ^ b2) << 1 | (b2 ^ b3) << 2 | b3 << 3;
+}
+__device__ __forceinline__ float walk_sums(float (&p)[16], int token) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 0), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 0);
+    p[i] = token & 1 ? b : a;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 1), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 1);
+    p[i] = token & 2 ? b : a;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = p[2 * i] + dpp_f(p[2 * i], 2), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 2);
+    p[i] = token & 4 ? b : a;
+  }
+  const float a = p[0] + dpp_f(p[0], 3), b = p[1] + dpp_f(p[1], 3);
+  return token & 8 ? b : a;
+}
+
 __device__ __forceinline__ float wave_max_xor(float v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, VK_WAVE));

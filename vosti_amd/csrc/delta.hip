@@ -354,32 +354,6 @@ struct WalkShape {
   static constexpr int NV = (TC * CB + RULE_THREADS - 1) / RULE_THREADS;   // and of v
 };
 
-// The sums over the lanes of one column's 16 read-outs: lane r of the column ends with token walk_token(r)'s.  Whether a lane goes on
-// with the first or the second of two sums is chosen so that the partner of every later step has gone on with the same ones.
-__device__ __forceinline__ int walk_token(int r) {
-  const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;
-  return (b0 ^ b2) | (b1 ^ b2) << 1 | (b2 ^ b3) << 2 | b3 << 3;
-}
-__device__ __forceinline__ float walk_sums(float (&p)[16], int token) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float a = p[2 * i] + dpp_f(p[2 * i], 0), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 0);
-    p[i] = token & 1 ? b : a;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = p[2 * i] + dpp_f(p[2 * i], 1), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 1);
-    p[i] = token & 2 ? b : a;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float a = p[2 * i] + dpp_f(p[2 * i], 2), b = p[2 * i + 1] + dpp_f(p[2 * i + 1], 2);
-    p[i] = token & 4 ? b : a;
-  }
-  const float a = p[0] + dpp_f(p[0], 3), b = p[1] + dpp_f(p[1], 3);
-  return token & 8 ? b : a;
-}
-
 template <int D, int CC_, bool DELTA, typename IN, bool HEAD_DECAY>
 __global__ __launch_bounds__(RULE_THREADS, 2) void rule_walk_kernel(float* __restrict__ out, const IN* __restrict__ qkv, int64_t ld, int q_col, int k_col,
                                                                     int v_col, const float* __restrict__ decay, const elem_t* __restrict__ b, int64_t ldb,
