@@ -150,3 +150,43 @@ def test_the_state_space_scan(P, dtype):
         assert torch.equal(y, y2) and torch.equal(state, state2)
         if want is not None:                               # 32-bit sums of 128 products and 45 decayed terms
             assert (y.double() - want).norm() < 5e-6 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K,C,with_bias", [(2, 1028, False), (3, 64, True), (4, 260, False), (4, 96, True), (6, 96, False), (1, 40, False)])
+def test_the_short_convolution(K, C, with_bias, dtype):
+    """Groups of 16 tokens within a sequence, across sequences and at the end; single tokens with their tails; against the sums written out
+    with the tails that the step before left."""
+    k = kern(dtype)
+    g = torch.Generator().manual_seed(5)
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    taps = (0.4 * torch.randn(C, K, generator=g)).to(dtype)
+    bias = (0.2 * torch.randn(C, generator=g)).to(dtype)
+    fn = k.lib.vk_delta_conv_bias if with_bias else k.lib.vk_delta_conv
+    fn.argtypes = [p, p, l, p] + ([p] if with_bias else []) + [p, l, l, p, p, p, p, i, i, i, i, p]
+    offset, S = 8, 4
+    state = torch.randn(S, offset + 32 + max(K - 1, 1) * C, generator=g).cuda()
+    fed = [[] for _ in range(S)]
+    for lengths in ([40, 1, 17, 2], [1, 1, 1, 1], [16, 3, 33, 1], [1, 1, 1, 1]):
+        T = sum(lengths)
+        x = torch.randn(T, C + 8, generator=g).to(dtype)
+        cu = [0]
+        for n in lengths:
+            cu.append(cu[-1] + n)
+        positions, seq, want = torch.zeros(T, dtype=torch.int32), torch.zeros(T, dtype=torch.int32), []
+        for s in range(S):
+            positions[cu[s]:cu[s + 1]] = torch.arange(lengths[s], dtype=torch.int32) + len(fed[s])
+            seq[cu[s]:cu[s + 1]] = s
+            for t in range(cu[s], cu[s + 1]):
+                fed[s].append(x[t, :C].double())
+                z = (bias.double() if with_bias else torch.zeros(C).double()) + sum(
+                    taps[:, j].double() * fed[s][len(fed[s]) - K + j] for j in range(K) if len(fed[s]) - K + j >= 0)
+                want.append(z * torch.sigmoid(z))
+        y = torch.full((T, C), float("nan"), device="cuda")
+        xs, tg, bg = x.cuda(), taps.cuda(), bias.cuda()
+        i32 = [v.to(torch.int32).cuda() for v in (seq, torch.tensor(cu), positions, torch.arange(S))]
+        args = (y.data_ptr(), xs.data_ptr(), xs.shape[1], tg.data_ptr()) + ((bg.data_ptr(),) if with_bias else ())
+        assert fn(*args, state.data_ptr(), state.shape[1], offset, *(v.data_ptr() for v in i32), T, S, C, K, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        # 32-bit sums of up to six products and a logistic function.
+        assert (y.cpu().double() - torch.stack(want)).abs().max() < 2e-5
