@@ -46,14 +46,6 @@ template <> __device__ __forceinline__ __bf16 from_f32<__bf16>(float x) { return
 // The value an element-typed store would hold, as a float.
 __device__ __forceinline__ float round_to_elem(float x) { return to_f32(from_f32<elem_t>(x)); }
 
-__device__ __forceinline__ float wave_sum_xor(float v) {
-  // Butterfly: every lane ends with the same value; the order of the additions
-  // is fixed by the lane pattern.
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off, VK_WAVE);
-  return v;
-}
-
 // The values of lanes l ^ 16 and l ^ 32 (what __shfl_xor gives), through the row and half swaps of
 // gfx950, which stay in the vector unit instead of going through LDS.
 __device__ __forceinline__ float lane_xor16(float v) {
@@ -136,10 +128,40 @@ __device__ __forceinline__ float walk_sums(float (&p)[16], int token) {
   return token & 8 ? b : a;
 }
 
+// The value of lane l ^ OFF where the steps 32, 16, 8, 4, 2, 1 of a butterfly over the whole wave are taken in this order, so that at
+// step 4 lanes 8 apart hold the same value and a rotation of their row brings either: all in the vector unit (a shuffle through LDS
+// is several times as long, and a norm of a few rows waits for six of them).  All lanes are active.
+template <int OFF>
+__device__ __forceinline__ float wave_partner(float v) {
+  if (OFF == 32) return lane_xor32(v);
+  if (OFF == 16) return lane_xor16(v);
+  const int x = __builtin_bit_cast(int, v);
+  const int y = OFF == 8   ? __builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true)      // row_ror:8
+                : OFF == 4 ? __builtin_amdgcn_mov_dpp(x, 0x124, 0xF, 0xF, true)      // row_ror:4
+                : OFF == 2 ? __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true)       // quad_perm [2, 3, 0, 1]
+                           : __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true);      // quad_perm [1, 0, 3, 2]
+  return __builtin_bit_cast(float, y);
+}
+
+// Butterflies over a wave: every lane ends with the same value; the order of the additions is fixed by the lane pattern (lanes 32
+// apart first).
+__device__ __forceinline__ float wave_sum_xor(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  v = pair_sum(__builtin_amdgcn_permlane32_swap(u, u, false, false));
+  const unsigned w = __builtin_bit_cast(unsigned, v);
+  v = pair_sum(__builtin_amdgcn_permlane16_swap(w, w, false, false));
+  v = v + wave_partner<8>(v);
+  v = v + wave_partner<4>(v);
+  v = v + wave_partner<2>(v);
+  return v + wave_partner<1>(v);
+}
 __device__ __forceinline__ float wave_max_xor(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, VK_WAVE));
-  return v;
+  v = fmaxf(v, wave_partner<32>(v));
+  v = fmaxf(v, wave_partner<16>(v));
+  v = fmaxf(v, wave_partner<8>(v));
+  v = fmaxf(v, wave_partner<4>(v));
+  v = fmaxf(v, wave_partner<2>(v));
+  return fmaxf(v, wave_partner<1>(v));
 }
 
 // Host side -----------------------------------------------------------------

@@ -76,12 +76,18 @@ __device__ __forceinline__ int wave_argmax(const float* v, int n, int lane, floa
     const float x = v[i];
     if (x > best) { best = x; at = i; }
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const float ov = __shfl_xor(best, off, VK_WAVE);
-    const int oe = __shfl_xor(at, off, VK_WAVE);
+  auto step = [&](float ov, int oe) {
     if (ov > best || (ov == best && oe < at)) { best = ov; at = oe; }
-  }
+  };
+  const auto as_float = [&] { return __builtin_bit_cast(float, at); };
+#define ARGMAX_STEP(OFF) step(wave_partner<OFF>(best), __builtin_bit_cast(int, wave_partner<OFF>(as_float())))
+  ARGMAX_STEP(32);
+  ARGMAX_STEP(16);
+  ARGMAX_STEP(8);
+  ARGMAX_STEP(4);
+  ARGMAX_STEP(2);
+  ARGMAX_STEP(1);
+#undef ARGMAX_STEP
   return min(at, n - 1);        // scores that are no numbers must not become an address
 }
 

@@ -194,8 +194,7 @@ __global__ __launch_bounds__(256) void qkv_post_vec_kernel(QkvPostArgs a, int pe
       float part = 0.f;
 #pragma unroll
       for (int e = 0; e < VK_VEC; ++e) part = part + xv[e] * xv[e];
-#pragma unroll
-      for (int m = 1; m < LPH; m <<= 1) part = part + __shfl_xor(part, m, VK_WAVE);
+      part = group_sum<LPH>(part);
       const float rr = rsqrtf(part / (float)d + a.eps);
       float wv[VK_VEC];
       if (a.w_is_f32) {

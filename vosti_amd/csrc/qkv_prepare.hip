@@ -99,8 +99,7 @@ __global__ __launch_bounds__(PREP_THREADS) void qkv_prepare_kernel(PrepareArgs a
         float part = 0.f;
 #pragma unroll
         for (int e = 0; e < VK_VEC; ++e) part = part + v[e] * v[e];
-#pragma unroll
-        for (int m = 1; m < LPH; m <<= 1) part = part + __shfl_xor(part, m, VK_WAVE);
+        part = group_sum<LPH>(part);
         rr = rsqrtf(part / (float)a.size + a.eps);
       }
       if (live && kind != 2) {
@@ -133,8 +132,7 @@ __global__ __launch_bounds__(PREP_THREADS) void qkv_prepare_kernel(PrepareArgs a
       float part = 0.f;
 #pragma unroll
       for (int e = 0; e < VK_VEC; ++e) part = part + v[e] * v[e];
-#pragma unroll
-      for (int m = 1; m < LPH; m <<= 1) part = part + __shfl_xor(part, m, VK_WAVE);
+      part = group_sum<LPH>(part);
       const float rr = rsqrtf(part / (float)a.size + a.eps);
       if (kind != 2) {
 #pragma unroll
