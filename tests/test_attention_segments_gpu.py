@@ -10,25 +10,29 @@ pytestmark = pytest.mark.gpu
 
 # Keys of a request: one, around a tile of 64, around a segment of 256, a last segment of one tile, and several segments.
 LENGTHS = [1, 5, 63, 64, 65, 128, 191, 193, 255, 256, 257, 320, 513, 700]
+# The same up to two segments, whose launch folds them itself.
+SHORT = [1, 16, 64, 65, 255, 256, 257, 300, 320, 449, 511, 512]
 
 
+@pytest.mark.parametrize("LENGTHS", [LENGTHS, SHORT], ids=["long", "short"])
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,P,window", [(4, 2, 64, 64, 0), (20, 1, 48, 16, 0), (8, 2, 128, 64, 300), (8, 8, 112, 8, 70), (6, 1, 256, 128, 0),
                                                (4, 1, 208, 32, 64)])
-def test_plain_rows_agree(dtype, nq, nkv, d, P, window):
+def test_plain_rows_agree(LENGTHS, dtype, nq, nkv, d, P, window):
     k = kern(dtype)
     q = [rand((1, nq, d), dtype, 10 + i) for i in range(len(LENGTHS))]
     keys = [rand((n, nkv, d), dtype, 40 + i) for i, n in enumerate(LENGTHS)]
     values = [rand((n, nkv, d), dtype, 70 + i) for i, n in enumerate(LENGTHS)]
-    got = {m: run_attention(k, q, keys, values, P, dtype, window=window, poison=float("nan"), seed=m, decode_mode=m, decode_split=m == 7) for m in (3, 7, 1)}
+    got = {m: run_attention(k, q, keys, values, P, dtype, window=window, poison=float("nan"), seed=m, decode_mode=m, decode_split=m == 7 and max(LENGTHS) > 512) for m in (3, 7, 1)}
     assert not torch.isnan(got[7]).any()
     assert torch.equal(got[7], got[3]) and torch.equal(got[1], got[3])
 
 
+@pytest.mark.parametrize("LENGTHS", [LENGTHS, SHORT], ids=["long", "short"])
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nq,nkv,d,P,window,keep,cap", [(4, 2, 64, 64, 0, 0, 20.0), (20, 1, 48, 16, 100, 7, 0.0), (8, 2, 128, 64, 300, 16, 20.0),
                                                         (8, 8, 112, 8, 64, 70, 5.0), (6, 1, 256, 128, 0, 0, 0.0)])
-def test_capped_rows_agree_with_prompt_rows(dtype, nq, nkv, d, P, window, keep, cap):
+def test_capped_rows_agree_with_prompt_rows(LENGTHS, dtype, nq, nkv, d, P, window, keep, cap):
     """The last row of a sequence as a decoded token and as a prompt portion of one row."""
     k = kern(dtype)
     p, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float

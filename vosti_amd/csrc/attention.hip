@@ -1161,18 +1161,24 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 // What bounds a step of few segments is the chain of dependent loads and of tiles, not bytes: here keys and values of the whole
 // segment are asked for at once, right behind the step's numbers, whose table entries are read together with the sequence's lengths
 // (a page that turns out not to be needed is read and not used), and the four tiles' scores are computed side by side.
-template <int DPAD, bool EXACT, bool EXT, bool REL>
-__global__ __launch_bounds__(64 * SEG_TILES, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a) {
+// SEGS 2: a workgroup of eight waves takes both segments of a launch that has no more than two, folds them as attn_combine_kernel
+// does and writes the output: a launch less, where a launch that waits for the one before is a third of the two.
+template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1>
+__global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a) {
+  static_assert(SEGS == 1 || sizeof(elem_t) * DPAD <= 256, "eight waves have 256 registers each");
   static_assert(EXT || !REL, "biases by distance belong to the variant");
   constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB, ND = NDT / SEG_TILES;   // ND: column blocks of a wave
   constexpr int NP = EXT ? P_PARTS : 1;                                        // numbers that a weight is split into
-  __shared__ frag_t probs[SEG_TILES][NP][KEY_SLABS][64];
-  __shared__ float tile_max[SEG_TILES][16], tile_sum[SEG_TILES][16];
+  __shared__ frag_t probs_of[SEGS][SEG_TILES][NP][KEY_SLABS][64];
+  __shared__ float tile_max_of[SEGS][SEG_TILES][16], tile_sum_of[SEGS][SEG_TILES][16];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave8 % SEG_TILES, my_seg = wave8 / SEG_TILES;
+  auto& probs = probs_of[my_seg];
+  auto& tile_max = tile_max_of[my_seg];
+  auto& tile_sum = tile_sum_of[my_seg];
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seg = blockIdx.z, first_tile = seg * SEG_TILES;
+  const int seg = blockIdx.z * SEGS + my_seg, first_tile = seg * SEG_TILES;
   const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
   const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
   const int k_len = a.k_len[seq];
@@ -1193,7 +1199,7 @@ __global__ __launch_bounds__(64 * SEG_TILES, sizeof(elem_t) * DPAD <= 256 ? 2 : 
     if (t <= pos / TILE_KEYS && (t < keep_tiles || t >= tile_lo)) wanted |= 1u << j;
   }
   wanted = __builtin_amdgcn_readfirstlane(wanted);
-  if (wanted == 0) return;   // the whole workgroup
+  if (SEGS == 1 && wanted == 0) return;   // the whole workgroup
 
   RowCtx c;
   init_ctx(c, a, seq, kvh, k_len);
@@ -1313,6 +1319,36 @@ __global__ __launch_bounds__(64 * SEG_TILES, sizeof(elem_t) * DPAD <= 256 ? 2 : 
           for (int dt = 0; dt < ND; ++dt)
             if (EXACT || dt * 16 < cv.d) ACC[dt] = mma_slab(vf[j][dt][ks], pf[part][ks], ACC[dt]);
     }
+  }
+  if constexpr (SEGS == 2) {
+    // The second segment's state to the first one's waves, lane by lane: the same lanes hold the same rows and columns.
+    __syncthreads();                      // the weights have been read
+    f32x4* hand = reinterpret_cast<f32x4*>(&probs_of[0][0][0][0][0]);
+    static_assert((size_t)SEG_TILES * (ND + 1) * 64 * sizeof(f32x4) <= sizeof(probs_of), "the hand-over fits the weights' place");
+    if (my_seg == 1) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) hand[(wave * (ND + 1) + dt) * 64 + lane] = ACC[dt];
+      hand[(wave * (ND + 1) + ND) * 64 + lane] = f32x4{M, L, 0.f, 0.f};
+    }
+    __syncthreads();
+    if (my_seg == 1 || !c.row_ok) return;
+    float Mt = -INFINITY, Lt = 0.f;
+    f32x4 out[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) out[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    fold<ND>(Mt, Lt, out, M, L, ACC);
+    const f32x4 other = hand[(wave * (ND + 1) + ND) * 64 + lane];
+    f32x4 theirs[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) theirs[dt] = hand[(wave * (ND + 1) + dt) * 64 + lane];
+    fold<ND>(Mt, Lt, out, other.x, other.y, theirs);
+    if (a.sinks != nullptr && Mt > -INFINITY) Lt = Lt + sink_term(a, head, Mt);
+    const float inv = (Lt > 0.f ? 1.0f / Lt : 0.f) * out_gate(a, tok, head);
+    elem_t* orow = a.out + ((int64_t)tok * a.nq + head) * a.d + wave * ND * 16 + 4 * c.g;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+      if (EXACT || dt * 16 < cv.d) store_elems4(orow + dt * 16, f32x4{out[dt].x * inv, out[dt].y * inv, out[dt].z * inv, out[dt].w * inv});
+    return;
   }
   if (!c.row_ok) return;
   const int64_t prow = ((int64_t)blockIdx.x * a.nq + head) * a.nseg + seg;
@@ -1530,6 +1566,23 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
     if (exact) attn_decode_quad_kernel<DP, true, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);   \
     else attn_decode_quad_kernel<DP, false, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);        \
   } while (0)
+#define DECODE_BOTH(DP)                                                                                                        \
+  do {                                                                                                                         \
+    if (exact) attn_decode_quad_kernel<DP, true, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);        \
+    else attn_decode_quad_kernel<DP, false, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);             \
+  } while (0)
+    // No more than two segments (512 keys): without the second launch.  A recorded step's launch covers 512 keys whatever it holds, so
+    // that most requests this is for have one segment in work: 1 token of 23 keys 8.1 -> 5.1 us, 3 of 220 keys 10.5 -> 8.3, 8 of 300
+    // 10.2 -> 9.4; with both full a compute unit brings in twice the keys (5 of 400 10.5 -> 11.3, 1 of 500 10.6 -> 12.3).
+    if (nseg <= 2 && sizeof(elem_t) * vk_dpad(d) <= 256) {
+#ifdef VK_BF16
+      if (d > 64) DECODE_BOTH(128);
+      else
+#endif
+        DECODE_BOTH(64);
+      return vk_check_launch("attention (decoded rows, both segments)");
+    }
+#undef DECODE_BOTH
     if (d <= 64) DECODE_QUAD(64);
     else if (d <= 128) DECODE_QUAD(128);
 #ifdef VK_BF16
@@ -1659,6 +1712,22 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     if (exact) attn_decode_quad_kernel<DP, true, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);          \
     else attn_decode_quad_kernel<DP, false, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);               \
   } while (0)
+#define DECODE_BOTH_EXT_OF(DP, REL)                                                                                             \
+  do {                                                                                                                         \
+    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);         \
+    else attn_decode_quad_kernel<DP, false, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);              \
+  } while (0)
+#define DECODE_BOTH_EXT(DP) do { if (rel != nullptr) DECODE_BOTH_EXT_OF(DP, true); else DECODE_BOTH_EXT_OF(DP, false); } while (0)
+    if (nseg <= 2 && sizeof(elem_t) * vk_dpad(d) <= 256) {
+#ifdef VK_BF16
+      if (d > 64) DECODE_BOTH_EXT(128);
+      else
+#endif
+        DECODE_BOTH_EXT(64);
+      return vk_check_launch("attention (decoded rows, capped scores, both segments)");
+    }
+#undef DECODE_BOTH_EXT
+#undef DECODE_BOTH_EXT_OF
 #define DECODE_QUAD_EXT(DP) do { if (rel != nullptr) DECODE_QUAD_EXT_OF(DP, true); else DECODE_QUAD_EXT_OF(DP, false); } while (0)
     if (d <= 64) DECODE_QUAD_EXT(64);
     else if (d <= 128) DECODE_QUAD_EXT(128);
