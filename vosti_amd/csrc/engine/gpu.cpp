@@ -124,8 +124,7 @@ struct Kernels::Fn {
   int (*ssm_gate_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, hipStream_t);
   int (*moe_max_tiles)(int, int, int, int);
   int (*gemm_grouped)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, hipStream_t);
-  int (*moe_route)(P, P, P, CP, CP, int, int, int, int, float, hipStream_t);
-  int (*moe_plan)(CP, P, P, P, P, P, int, int, int, int, hipStream_t);
+  int (*moe_route_plan)(P, P, P, CP, CP, CP, int, CP, int, int, int, int, int, float, int, int, int, int, float, P, P, P, P, P, int, hipStream_t);
   int (*moe_up)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_down)(P, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_combine)(P, CP, CP, CP, int, int, int, hipStream_t);
@@ -135,7 +134,6 @@ struct Kernels::Fn {
   int (*gla_decay)(P, CP, int64_t, CP, int, int, int, float, hipStream_t);
   int (*gla_rule)(P, CP, int64_t, int, int, int, CP, P, int64_t, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*gated_head_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, int, hipStream_t);
-  int (*moe_route_bias)(P, P, P, CP, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*moe_up_plain)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_glu)(P, CP, int64_t, int, float, float, float, hipStream_t);
   int (*moe_combine_add)(P, CP, CP, CP, CP, int, int, int, hipStream_t);
@@ -143,7 +141,6 @@ struct Kernels::Fn {
   int (*cast_from_f32)(P, CP, int64_t, hipStream_t);
   int (*stream_norm_add_rounded)(P, CP, CP, CP, int, int, int, float, float, float, P, hipStream_t);
   int (*stream_norm_add_f32_rounded)(P, CP, CP, CP, int, int, int, float, float, float, P, hipStream_t);
-  int (*moe_route_scored)(P, P, P, CP, CP, CP, int, int, int, int, int, float, int, int, int, float, hipStream_t);
   int (*moe_glu_weighed)(P, CP, int64_t, int, float, float, float, CP, CP, hipStream_t);
   int (*norm_columns)(P, int64_t, CP, int64_t, int, int, CP, int, float, int, hipStream_t);
   int (*gemm_heads)(P, int64_t, int64_t, CP, int64_t, int64_t, CP, int, int, int, int, hipStream_t);
@@ -162,7 +159,6 @@ struct Kernels::Fn {
   int (*gemm_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_split_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
   int (*gemm_grouped_act)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, CP, int, hipStream_t);
-  int (*moe_route_corrected)(P, P, P, CP, CP, CP, int, int, int, int, int, int, int, int, float, hipStream_t);
   int (*stream_add_norm)(P, P, CP, int, CP, int, int, int, float, hipStream_t);
   int (*embed_bigram)(P, CP, CP, CP, CP, int, int, int, int64_t, int64_t, int64_t, hipStream_t);
   int (*qkv_prepare)(CP, int64_t, P, P, P, int, CP, CP, int, int, int, float, CP, int, CP, CP, CP, int64_t, int, int, CP, int, int, int, int, int, int,
@@ -205,20 +201,20 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(delta_out, "vk_delta_out"); VK(delta_conv_bias, "vk_delta_conv_bias"); VK(paged_attention_blocked, "vk_paged_attention_blocked");
   VK(qkv_post_angles, "vk_qkv_post_angles"); VK(embed_scaled, "vk_embed_scaled"); VK(stream_add, "vk_stream_add");
   VK(stream_pair_norm, "vk_stream_pair_norm"); VK(ssm_scan, "vk_ssm_scan"); VK(ssm_gate_norm, "vk_ssm_gate_norm");
-  VK(moe_max_tiles, "vk_moe_max_tiles"); VK(moe_route, "vk_moe_route"); VK(moe_plan, "vk_moe_plan"); VK(moe_up, "vk_moe_up");
+  VK(moe_max_tiles, "vk_moe_max_tiles"); VK(moe_route_plan, "vk_moe_route_plan"); VK(moe_up, "vk_moe_up");
   VK(moe_down, "vk_moe_down"); VK(moe_combine, "vk_moe_combine"); VK(moe_relu_square, "vk_moe_relu_square"); VK(gemm_grouped, "vk_gemm_grouped");
   VK(qkv_post_norm_angles, "vk_qkv_post_norm_angles"); VK(gate_mul, "vk_gate_mul"); VK(gla_decay, "vk_gla_decay"); VK(gla_rule, "vk_gla_rule");
-  VK(gated_head_norm, "vk_gated_head_norm"); VK(moe_route_bias, "vk_moe_route_bias"); VK(moe_up_plain, "vk_moe_up_plain"); VK(moe_glu, "vk_moe_glu");
+  VK(gated_head_norm, "vk_gated_head_norm"); VK(moe_up_plain, "vk_moe_up_plain"); VK(moe_glu, "vk_moe_glu");
   VK(moe_combine_add, "vk_moe_combine_add"); VK(stream_norm_add_f32, "vk_stream_norm_add_f32");
   VK(stream_norm_add_rounded, "vk_stream_norm_add_rounded"); VK(stream_norm_add_f32_rounded, "vk_stream_norm_add_f32_rounded");
-  VK(cast_from_f32, "vk_cast_from_f32"); VK(moe_route_scored, "vk_moe_route_scored"); VK(moe_glu_weighed, "vk_moe_glu_weighed");
+  VK(cast_from_f32, "vk_cast_from_f32"); VK(moe_glu_weighed, "vk_moe_glu_weighed");
   VK(norm_columns, "vk_norm_columns"); VK(gemm_heads, "vk_gemm_heads"); VK(latent_post, "vk_latent_post");
   VK(qkv_post_norm_angles_paired, "vk_qkv_post_norm_angles_paired"); VK(linear_rule, "vk_linear_rule"); VK(side_gate, "vk_side_gate");
   VK(gated_row_norm, "vk_gated_row_norm"); VK(silu_columns, "vk_silu_columns");
   VK(hyper_in_place, "vk_hyper_in_place"); VK(hyper_step, "vk_hyper_step"); VK(hyper_close, "vk_hyper_close"); VK(embed_normed, "vk_embed_normed");
   VK(attention_wide, "vk_attention_wide"); VK(attention_wide_limit, "vk_attention_wide_limit");
   VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_act, "vk_gemm_grouped_act");
-  VK(moe_route_corrected, "vk_moe_route_corrected"); VK(stream_add_norm, "vk_stream_add_norm"); VK(embed_bigram, "vk_embed_bigram");
+  VK(stream_add_norm, "vk_stream_add_norm"); VK(embed_bigram, "vk_embed_bigram");
   VK(qkv_prepare, "vk_qkv_prepare"); VK(paged_attention_biased, "vk_paged_attention_biased"); VK(attn_rel_pad, "vk_attn_rel_pad");
 #undef VK
   segment_keys_ = fn_->attn_segment_keys();
@@ -938,40 +934,28 @@ Kernels::MoePlan Kernels::empty_plan(const Tensor& h, const Tensor& router, int 
   return p;
 }
 
-void Kernels::fill_plan(MoePlan& p) {
-  call(fn_->moe_plan(p.idx.data, p.row_pair.data, p.row_token.data, p.pair_row.data, p.tile_expert.data, p.expert_start.data, (int)p.idx.dim(0), p.top,
-                     p.experts, p.tile_rows, stream));
+// The router's launches and the plan's into p.
+void Kernels::route_and_plan(MoePlan& p, const Tensor& h, const Tensor& router, const Tensor* bias, const Tensor* correction, float weight_eps, int score_kind,
+                             int groups, int keep, int group_score, float scale) {
+  const int64_t T = h.dim(0), E = router.dim(0);
+  const int bf = bias ? norm_weight(*bias, "router bias", E) : 0, cf = correction ? norm_weight(*correction, "router correction", E) : 0;
+  Tensor logits = empty({T, E}, DType::F32);
+  call(fn_->moe_route_plan(p.idx.data, p.wts.data, logits.data, h.data, router.data, bias ? bias->data : nullptr, bf, correction ? correction->data : nullptr, cf,
+                           (int)T, (int)h.dim(1), (int)E, p.top, weight_eps, score_kind, groups, keep, group_score, scale, p.row_pair.data, p.row_token.data,
+                           p.pair_row.data, p.tile_expert.data, p.expert_start.data, p.tile_rows, stream));
 }
 
 Kernels::MoePlan Kernels::moe_route_corrected(const Tensor& h, const Tensor& router, const Tensor& correction, int top, int tile_rows, int groups, int keep,
                                               int group_score, float scale) {
   MoePlan p = empty_plan(h, router, top, tile_rows);
-  const int64_t T = h.dim(0), E = router.dim(0);
-  const int cf = norm_weight(correction, "router correction", E);
-  Tensor logits = empty({T, E}, DType::F32);
-  call(fn_->moe_route_corrected(p.idx.data, p.wts.data, logits.data, h.data, router.data, correction.data, cf, (int)T, (int)h.dim(1), (int)E, top, groups,
-                                keep, group_score, scale, stream));
-  fill_plan(p);
+  route_and_plan(p, h, router, nullptr, &correction, 0.f, 1, groups, keep, group_score, scale);
   return p;
 }
 
 Kernels::MoePlan Kernels::moe_route_scored(const Tensor& h, const Tensor& router, int top, float weight_eps, int tile_rows, const Tensor* bias,
                                            int score_kind, int groups, int keep, float scale) {
   MoePlan p = empty_plan(h, router, top, tile_rows);
-  const int64_t T = h.dim(0), E = router.dim(0);
-  Tensor logits = empty({T, E}, DType::F32);
-  if (score_kind != 0 || groups != 1 || scale != 1.f) {
-    const int bf = bias ? norm_weight(*bias, "router bias", E) : 0;
-    call(fn_->moe_route_scored(p.idx.data, p.wts.data, logits.data, h.data, router.data, bias ? bias->data : nullptr, bf, (int)T, (int)h.dim(1), (int)E,
-                               top, weight_eps, score_kind, groups, keep, scale, stream));
-  } else if (bias) {
-    const int bf = norm_weight(*bias, "router bias", E);
-    call(fn_->moe_route_bias(p.idx.data, p.wts.data, logits.data, h.data, router.data, bias->data, bf, (int)T, (int)h.dim(1), (int)E, top, weight_eps,
-                             stream));
-  } else {
-    call(fn_->moe_route(p.idx.data, p.wts.data, logits.data, h.data, router.data, (int)T, (int)h.dim(1), (int)E, top, weight_eps, stream));
-  }
-  fill_plan(p);
+  route_and_plan(p, h, router, bias, nullptr, weight_eps, score_kind, groups, keep, 0, scale);
   return p;
 }
 

@@ -317,7 +317,8 @@ class Kernels {
   void expect(const Tensor& t, const char* what, DType dtype, std::vector<int64_t> shape = {}) const;
   int norm_weight(const Tensor& w, const char* what, int64_t n) const;   // 1 if the weight is float32
   MoePlan empty_plan(const Tensor& h, const Tensor& router, int top, int tile_rows);   // a plan's arrays, not yet written
-  void fill_plan(MoePlan& p);                                                          // from the choices to the rows' places
+  void route_and_plan(MoePlan& p, const Tensor& h, const Tensor& router, const Tensor* bias, const Tensor* correction, float weight_eps, int score_kind, int groups,
+                      int keep, int group_score, float scale);                                                          // from the choices to the rows' places
   bool split(Tensor& out, const Tensor& act, const Tensor& w, bool swiglu, const Tensor* workspace);
 
   std::string name_;

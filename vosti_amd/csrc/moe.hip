@@ -24,41 +24,54 @@
 // order (fused multiply-adds), a butterfly follows over the lanes and the four waves' sums are added in wave order: the
 // order depends on the width alone.
 // bias: one number an expert that is added to its logit (elements or floats), or null.
+// EX: experts of a workgroup, one after the other on the rows it holds: with one every expert's workgroup reads a group's rows again from
+// the second-level cache, which a prompt's 32 experts wait for (2,048 tokens of 4,096 entries: 37 us, with four 24); few tokens want the workgroups.
+template <int EX>
 __global__ __launch_bounds__(256) void moe_logits_kernel(float* __restrict__ z, const elem_t* __restrict__ h, const elem_t* __restrict__ router,
                                                          int T, int W, int E, const void* __restrict__ bias, int bias_is_f32) {
-  __shared__ float part[4][MOE_ROUTE_TOKENS];
+  __shared__ float part[4][EX][MOE_ROUTE_TOKENS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t0 = blockIdx.x * MOE_ROUTE_TOKENS, e = blockIdx.y;
+  const int t0 = blockIdx.x * MOE_ROUTE_TOKENS, e0 = blockIdx.y * EX;
   if (t0 >= T) return;         // the grid is rounded up: the whole workgroup
-  float acc[MOE_ROUTE_TOKENS];
+  float acc[EX][MOE_ROUTE_TOKENS];
 #pragma unroll
-  for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) acc[i] = 0.f;
-  const elem_t* wr = router + (int64_t)e * W;
-#pragma unroll 2
+  for (int x = 0; x < EX; ++x)
+#pragma unroll
+    for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) acc[x][i] = 0.f;
+  const elem_t* wr = router + (int64_t)e0 * W;
+#pragma unroll EX == 1 ? 2 : 1
   for (int c = threadIdx.x * VK_VEC; c < W; c += 256 * VK_VEC) {
-    float wv[VK_VEC];
-    load_elems(wr + c, wv);
+    float wv[EX][VK_VEC];
+#pragma unroll
+    for (int x = 0; x < EX; ++x) load_elems(wr + (int64_t)x * W + c, wv[x]);
 #pragma unroll
     for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) {
       float hv[VK_VEC];
       load_elems(h + (int64_t)min(t0 + i, T - 1) * W + c, hv);
 #pragma unroll
-      for (int j = 0; j < VK_VEC; ++j) acc[i] = __builtin_fmaf(hv[j], wv[j], acc[i]);
+      for (int x = 0; x < EX; ++x)
+#pragma unroll
+        for (int j = 0; j < VK_VEC; ++j) acc[x][i] = __builtin_fmaf(hv[j], wv[x][j], acc[x][i]);
     }
   }
 #pragma unroll
-  for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) {
-    const float v = wave_sum_xor(acc[i]);
-    if (lane == 0) part[wave][i] = v;
-  }
+  for (int x = 0; x < EX; ++x)
+#pragma unroll
+    for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) {
+      const float v = wave_sum_xor(acc[x][i]);
+      if (lane == 0) part[wave][x][i] = v;
+    }
   __syncthreads();
-  if (threadIdx.x < MOE_ROUTE_TOKENS && t0 + (int)threadIdx.x < T) {
-    float v = part[0][threadIdx.x];
-    v = v + part[1][threadIdx.x];
-    v = v + part[2][threadIdx.x];
-    v = v + part[3][threadIdx.x];
-    if (bias != nullptr) v = v + load_weight(bias, bias_is_f32, e);
-    z[(int64_t)(t0 + threadIdx.x) * E + e] = v;
+  if (threadIdx.x < EX * MOE_ROUTE_TOKENS) {
+    const int x = threadIdx.x / MOE_ROUTE_TOKENS, i = threadIdx.x % MOE_ROUTE_TOKENS;
+    if (t0 + i < T) {
+      float v = part[0][x][i];
+      v = v + part[1][x][i];
+      v = v + part[2][x][i];
+      v = v + part[3][x][i];
+      if (bias != nullptr) v = v + load_weight(bias, bias_is_f32, e0 + x);
+      z[(int64_t)(t0 + i) * E + e0 + x] = v;
+    }
   }
 }
 
@@ -99,15 +112,28 @@ __device__ __forceinline__ int wave_argmax(const float* v, int n, int lane, floa
 // (group_score 0) or the sum of its two largest (1), and only experts of the `keep` best groups can be chosen.
 // correction (score 1 only; [E] elements or floats, or null): a number an expert that joins its score for the choice, of groups
 // and of experts, and not its weight.  Scores so corrected may be negative.
-__global__ __launch_bounds__(256) void moe_choose_kernel(int32_t* __restrict__ idx, float* __restrict__ wts, const float* __restrict__ logits,
-                                                         int T, int E, int top, float weight_eps, int score_kind, int groups, int keep, float scale,
-                                                         int group_score, const void* __restrict__ correction, int correction_is_f32) {
-  extern __shared__ float scores[];      // [4][E], with a correction [4][E] of the scores without it, then [4][groups]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= T) return;
+// scores: LDS of the workgroup, [waves][E], with a correction [waves][E] of the scores without it, then [waves][groups].
+struct MoeChoice {
+  int32_t* idx;
+  float* wts;
+  const float* logits;
+  int T, E, top;
+  float weight_eps;
+  int score_kind, groups, keep;
+  float scale;
+  int group_score;
+  const void* correction;
+  int correction_is_f32;
+};
+__device__ __forceinline__ void moe_choose_token(const MoeChoice& a, float* scores, int t, int wave, int waves, int lane) {
+  int32_t* idx = a.idx;
+  float* wts = a.wts;
+  const float* logits = a.logits;
+  const int E = a.E, top = a.top, score_kind = a.score_kind, groups = a.groups, keep = a.keep, group_score = a.group_score, correction_is_f32 = a.correction_is_f32;
+  const float weight_eps = a.weight_eps, scale = a.scale;
+  const void* correction = a.correction;
   float* z = scores + wave * E;
-  float* raw = correction != nullptr ? z + 4 * E : z;
+  float* raw = correction != nullptr ? z + waves * E : z;
   float mx = -INFINITY;
   for (int e = lane; e < E; e += 64) {
     z[e] = logits[(int64_t)t * E + e];
@@ -124,7 +150,7 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(int32_t* __restrict__ i
   sum = score_kind == 1 ? 1.f : wave_sum_xor(sum);
   if (keep < groups) {
     // A kept group's score is marked with -inf; the experts of the others are then marked as if they had been chosen.
-    float* gs = scores + (correction != nullptr ? 8 : 4) * E + wave * groups;
+    float* gs = scores + (correction != nullptr ? 2 : 1) * waves * E + wave * groups;
     const int size = E / groups;
     wave_lds_fence();
     for (int g = lane; g < groups; g += 64) {
@@ -170,45 +196,91 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(int32_t* __restrict__ i
   for (int k = 64 + lane; k < top; k += 64) wts[(int64_t)t * top + k] = (wts[(int64_t)t * top + k] / denom) * scale;
 }
 
+__global__ __launch_bounds__(256) void moe_choose_kernel(MoeChoice a) {
+  extern __shared__ float scores[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = blockIdx.x * 4 + wave;
+  if (t < a.T) moe_choose_token(a, scores, t, wave, 4, lane);
+}
+
 // The plan, by one workgroup.  counts the pairs of every expert, gives expert e the rows [start_e, start_e + tile_rows *
 // ceil(count_e / tile_rows)) and every pair a row among its expert's (in no fixed order: a row's result does not depend on
 // its place).  row_pair [max_rows]: the pair (token * top + choice) of a row, or -1; row_token [max_rows]: the row's
 // token (0 for a row without a pair); pair_row [pairs]; tile_expert [max_tiles]: the expert of a tile, or -1 beyond the
 // last; expert_start [E + 1]: the first row of every expert, and the rows in use.
-__global__ __launch_bounds__(1024) void moe_plan_kernel(const int32_t* __restrict__ idx, int32_t* __restrict__ row_pair,
-                                                        int32_t* __restrict__ row_token, int32_t* __restrict__ pair_row,
-                                                        int32_t* __restrict__ tile_expert, int32_t* __restrict__ expert_start, int pairs, int top,
-                                                        int E, int max_tiles, int tile_rows) {
-  extern __shared__ int32_t plan[];      // [E] counts, then [E] cursors
+struct MoePlanArgs {
+  const int32_t* idx;
+  int32_t *row_pair, *row_token, *pair_row, *tile_expert, *expert_start;
+  int pairs, top, E, max_tiles, tile_rows;
+};
+// By all threads of a workgroup of 1,024; plan: LDS, [E] counts, then [E] cursors.
+__device__ __forceinline__ void moe_make_plan(const MoePlanArgs& a, int32_t* plan) {
   int32_t* count = plan;
-  int32_t* cursor = plan + E;
-  for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;
-  for (int r = threadIdx.x; r < max_tiles * tile_rows; r += blockDim.x) {
-    row_pair[r] = -1;
-    row_token[r] = 0;
+  int32_t* cursor = plan + a.E;
+  for (int e = threadIdx.x; e < a.E; e += blockDim.x) count[e] = 0;
+  for (int r = threadIdx.x; r < a.max_tiles * a.tile_rows; r += blockDim.x) {
+    a.row_pair[r] = -1;
+    a.row_token[r] = 0;
   }
-  for (int i = threadIdx.x; i < max_tiles; i += blockDim.x) tile_expert[i] = -1;
+  for (int i = threadIdx.x; i < a.max_tiles; i += blockDim.x) a.tile_expert[i] = -1;
   __syncthreads();
-  for (int i = threadIdx.x; i < pairs; i += blockDim.x) atomicAdd(&count[idx[i]], 1);
+  for (int i = threadIdx.x; i < a.pairs; i += blockDim.x) atomicAdd(&count[a.idx[i]], 1);
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (a.E <= 64) {
+    // One wave, an expert a lane: the tiles before an expert's are a running sum over the lanes.
+    if (threadIdx.x < 64) {
+      const int e = threadIdx.x;
+      const int n = e < a.E ? (count[e] + a.tile_rows - 1) / a.tile_rows : 0;
+      int upto = n;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int other = __shfl_up(upto, off, VK_WAVE);
+        if (e >= off) upto += other;
+      }
+      const int tile = upto - n;
+      if (e < a.E) {
+        cursor[e] = tile * a.tile_rows;
+        a.expert_start[e] = tile * a.tile_rows;
+        for (int j = 0; j < n; ++j) a.tile_expert[tile + j] = e;
+        if (e == a.E - 1) a.expert_start[a.E] = upto * a.tile_rows;
+      }
+    }
+  } else if (threadIdx.x == 0) {
     int tile = 0;
-    for (int e = 0; e < E; ++e) {
-      const int n = (count[e] + tile_rows - 1) / tile_rows;
-      cursor[e] = tile * tile_rows;
-      expert_start[e] = tile * tile_rows;
-      for (int j = 0; j < n; ++j) tile_expert[tile + j] = e;
+    for (int e = 0; e < a.E; ++e) {
+      const int n = (count[e] + a.tile_rows - 1) / a.tile_rows;
+      cursor[e] = tile * a.tile_rows;
+      a.expert_start[e] = tile * a.tile_rows;
+      for (int j = 0; j < n; ++j) a.tile_expert[tile + j] = e;
       tile += n;
     }
-    expert_start[E] = tile * tile_rows;
+    a.expert_start[a.E] = tile * a.tile_rows;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
-    const int row = atomicAdd(&cursor[idx[i]], 1);
-    row_pair[row] = i;
-    row_token[row] = i / top;
-    pair_row[i] = row;
+  for (int i = threadIdx.x; i < a.pairs; i += blockDim.x) {
+    const int row = atomicAdd(&cursor[a.idx[i]], 1);
+    a.row_pair[row] = i;
+    a.row_token[row] = i / a.top;
+    a.pair_row[i] = row;
   }
+}
+__global__ __launch_bounds__(1024) void moe_plan_kernel(MoePlanArgs a) {
+  extern __shared__ int32_t plan[];
+  moe_make_plan(a, plan);
+}
+
+// The choice and the plan of a few tokens in one launch, a wave a token after the other: two launches that wait for each other took 11 to
+// 15 us for some hundred numbers.
+#define MOE_FEW_TOKENS 32
+__global__ __launch_bounds__(1024) void moe_choose_plan_kernel(MoeChoice c, MoePlanArgs p) {
+  extern __shared__ float scores[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int t = wave; t < c.T; t += 16) {
+    moe_choose_token(c, scores, t, wave, 16, lane);
+    wave_lds_fence();
+  }
+  __syncthreads();                // every choice is made and, through this compute unit's cache, to be read by all its waves
+  moe_make_plan(p, reinterpret_cast<int32_t*>(scores));
 }
 
 // One tile of 16 rows and 16 output features a workgroup: out[row, f] = sum over k of x[row, k] * w[expert][f, k], in
@@ -495,7 +567,7 @@ int vk_moe_max_tiles(int T, int top, int E, int tile_rows) {
 // logits: scratch [T, E] floats.  bias [E] (elements, or floats with bias_is_f32) or null.
 static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32, int T, int W,
                         int E, int top, float weight_eps, hipStream_t st, int score_kind = 0, int groups = 1, int keep = 1, float scale = 1.f, int group_score = 0,
-                        const void* correction = nullptr, int correction_is_f32 = 0) {
+                        const void* correction = nullptr, int correction_is_f32 = 0, const MoePlanArgs* plan = nullptr) {
   VK_REQUIRE(T >= 0 && W > 0 && W % VK_VEC == 0 && E > 0 && top > 0 && top <= E && E <= 4096,
              "router: bad sizes T=%d W=%d E=%d top=%d (the width in whole 16-byte vectors, at most 4096 experts)", T, W, E, top);
   VK_REQUIRE(((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0, "router: operands must be 16-byte aligned");
@@ -506,54 +578,40 @@ static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h
   // whose cache then holds its rows.
   const int groups_of_tokens = (T + MOE_ROUTE_TOKENS - 1) / MOE_ROUTE_TOKENS;
   const int grid_x = groups_of_tokens > 8 ? (groups_of_tokens + 7) / 8 * 8 : groups_of_tokens;
-  moe_logits_kernel<<<dim3(grid_x, E), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
+  if (E % 4 == 0 && T >= 256) moe_logits_kernel<4><<<dim3(grid_x, E / 4), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
+  else moe_logits_kernel<1><<<dim3(grid_x, E), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
   if (vk_check_launch("router (logits)")) return 1;
-  const size_t lds = (size_t)4 * ((correction != nullptr ? 2 : 1) * E + (keep < groups ? groups : 0)) * sizeof(float);
-  VK_REQUIRE(lds <= 65536, "router: %d experts in %d groups are too many", E, groups);
-  moe_choose_kernel<<<(T + 3) / 4, 256, lds, st>>>(idx, wts, logits, T, E, top, weight_eps, score_kind, groups, keep, scale,
-                                                        group_score, correction, correction_is_f32);
-  return vk_check_launch("router (choice)");
+  const MoeChoice c = {idx, wts, logits, T, E, top, weight_eps, score_kind, groups, keep, scale, group_score, correction, correction_is_f32};
+  const size_t a_wave = ((correction != nullptr ? 2 : 1) * (size_t)E + (keep < groups ? groups : 0)) * sizeof(float);
+  VK_REQUIRE(4 * a_wave <= 65536, "router: %d experts in %d groups are too many", E, groups);
+  if (plan != nullptr && T <= MOE_FEW_TOKENS && 16 * a_wave <= 65536) {
+    moe_choose_plan_kernel<<<1, 1024, std::max(16 * a_wave, (size_t)2 * E * sizeof(int32_t)), st>>>(c, *plan);
+    return vk_check_launch("router (choice and plan)");
+  }
+  moe_choose_kernel<<<(T + 3) / 4, 256, 4 * a_wave, st>>>(c);
+  if (vk_check_launch("router (choice)")) return 1;
+  if (plan == nullptr) return 0;
+  moe_plan_kernel<<<1, 1024, (size_t)2 * E * sizeof(int32_t), st>>>(*plan);
+  return vk_check_launch("expert plan");
 }
 
-int vk_moe_route(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, int T, int W, int E, int top, float weight_eps,
-                 hipStream_t st) {
-  return route_launch(idx, wts, logits, h, router, nullptr, 0, T, W, E, top, weight_eps, st);
-}
-
-// The same with a bias an expert on the logits, which both the choice and the weights see.  With weight_eps 0 the weights
-// are the softmax over the chosen logits alone: exp(z_k) / sum over the chosen exp(z_j), whatever the others are.
-int vk_moe_route_bias(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32, int T, int W,
-                      int E, int top, float weight_eps, hipStream_t st) {
-  VK_REQUIRE(bias != nullptr, "router: the bias is missing");
-  return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st);
-}
-
-// The same with a choice of score: 0 is vk_moe_route (vk_moe_route_bias with a bias), 1 gives every chosen expert the
-// logistic function of its logit as its weight, not divided by anything, 2 the softmax over all experts as it is.  bias may be
-// null.  groups, keep: only experts of the `keep` best of that many equal groups can be chosen (1, 1: all); scale: on every
-// weight.
-int vk_moe_route_scored(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32, int T, int W,
-                        int E, int top, float weight_eps, int score_kind, int groups, int keep, float scale, hipStream_t st) {
-  VK_REQUIRE(score_kind >= 0 && score_kind <= 2, "router: score kind %d", score_kind);
-  return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale);
-}
-
-// vk_moe_route_scored with score 1 (logistic scores as they are) and a correction [E] (elements, or floats with
-// correction_is_f32) that joins the scores for the choice of groups and experts and not for the weights; group_score 0: a group
-// is worth its largest corrected score, 1: the sum of its two largest.
-int vk_moe_route_corrected(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* correction, int correction_is_f32,
-                           int T, int W, int E, int top, int groups, int keep, int group_score, float scale, hipStream_t st) {
-  VK_REQUIRE(correction != nullptr && (group_score == 0 || group_score == 1), "router: the correction is missing, or group score %d", group_score);
-  return route_launch(idx, wts, logits, h, router, nullptr, 0, T, W, E, top, 0.f, st, 1, groups, keep, scale, group_score, correction, correction_is_f32);
-}
-
-int vk_moe_plan(const int32_t* idx, int32_t* row_pair, int32_t* row_token, int32_t* pair_row, int32_t* tile_expert, int32_t* expert_start, int T,
-                int top, int E, int tile_rows, hipStream_t st) {
+// The router and the plan.  bias: an expert's number on its logit, which both the choice and the weights see, or null.  score_kind 0: the
+// softmax over all experts, a chosen one's divided by the sum of the chosen plus weight_eps (with weight_eps 0 the softmax over the
+// chosen logits alone, whatever the others are); 1: the logistic function of a chosen logit as it is; 2: the softmax over all experts as it
+// is.  groups, keep: only experts of the `keep` best of that many equal groups can be chosen (1, 1: all); group_score 0: a group is worth
+// its largest score, 1: the sum of its two largest.  correction (score 1, no bias; [E] elements or floats): joins the scores for the choice
+// of groups and experts and not for the weights.  scale: on every weight.  tile_rows: rows of a tile of the plan (moe_plan_kernel).
+int vk_moe_route_plan(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32,
+                      const void* correction, int correction_is_f32, int T, int W, int E, int top, float weight_eps, int score_kind, int groups, int keep,
+                      int group_score, float scale, int32_t* row_pair, int32_t* row_token, int32_t* pair_row, int32_t* tile_expert, int32_t* expert_start,
+                      int tile_rows, hipStream_t st) {
+  VK_REQUIRE(score_kind >= 0 && score_kind <= 2 && (group_score == 0 || group_score == 1), "router: score kind %d, group score %d", score_kind, group_score);
+  VK_REQUIRE(correction == nullptr || (bias == nullptr && score_kind == 1), "router: a correction goes with logistic scores and without a bias");
   VK_REQUIRE(T >= 0 && top > 0 && E > 0 && E <= 4096 && tile_rows > 0, "expert plan: bad sizes T=%d top=%d E=%d", T, top, E);
   if (T == 0) return 0;
-  moe_plan_kernel<<<1, 1024, (size_t)2 * E * sizeof(int32_t), st>>>(idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E,
-                                                                    vk_moe_max_tiles(T, top, E, tile_rows), tile_rows);
-  return vk_check_launch("expert plan");
+  const MoePlanArgs plan = {idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E, vk_moe_max_tiles(T, top, E, tile_rows), tile_rows};
+  return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale, group_score, correction,
+                      correction_is_f32, &plan);
 }
 
 static int moe_cus() {
