@@ -42,3 +42,35 @@ def test_rows_in_use_get_the_plain_product(N, K, activation, dtype):
                     want = (want.float().clamp(min=0.0) ** 2).to(dtype)
                 assert torch.equal(out[at:at + n], want)
             at += 128 * (-(-n // 128))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K,lda", [(256, 512, 512), (96, 1024, 1088), (1100, 512, 520), (300, 192, 192)])
+def test_named_rows_are_as_their_copy(N, K, lda, dtype):
+    """Rows that a table names out of order, several times and never, against their copy in the product's order; rows further apart than
+    they are long; K of whole chunks and not; few workgroups and many."""
+    k = kern(dtype)
+    g = torch.Generator().manual_seed(3)
+    for experts, T in ((2, 1), (40, 333)):
+        w = rand((experts, N, K), dtype, 5, 0.1).cuda()
+        x = rand((T, lda), dtype, 6).cuda()
+        counts = torch.randint(0, 130, (experts,), generator=g).tolist()
+        blocks = [e for e, n in enumerate(counts) for _ in range(-(-n // 128))] + [-1]
+        M = 128 * len(blocks)
+        pairs, at = torch.full((M,), -1, dtype=torch.int32), 0
+        for n in counts:
+            pairs[at:at + n] = torch.arange(n, dtype=torch.int32)
+            at += 128 * (-(-n // 128))
+        named = torch.randint(0, T, (M,), generator=g, dtype=torch.int32)
+        copy = x[named.long().cuda()].contiguous()
+        which, row_pair, row = (torch.as_tensor(v, dtype=torch.int32).cuda() for v in (blocks, pairs, named))
+        p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+        fn = k.lib.vk_gemm_grouped_rows
+        fn.argtypes = [p, p, p, i, i, i, l, l, p, l, p, p, i, i, p]
+        stream = torch.cuda.current_stream().cuda_stream
+        outs = [torch.zeros(M, N, dtype=dtype, device="cuda") for _ in range(2)]
+        for out, act, rows in ((outs[0], copy, None), (outs[1], x, row.data_ptr())):
+            assert fn(out.data_ptr(), act.data_ptr(), w.data_ptr(), M, N, K, lda, N, which.data_ptr(), N * K, row_pair.data_ptr(), rows, T, 0, stream) == 0
+        assert torch.equal(*outs)
+        # More bytes than the offsets reach are refused.
+        assert fn(outs[0].data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, lda, N, which.data_ptr(), N * K, None, row.data_ptr(), 1 << 30, 0, stream) != 0

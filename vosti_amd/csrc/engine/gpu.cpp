@@ -158,7 +158,7 @@ struct Kernels::Fn {
   int (*attention_wide_limit)();
   int (*gemm_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_split_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
-  int (*gemm_grouped_act)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, CP, int, hipStream_t);
+  int (*gemm_grouped_rows)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, CP, CP, int, int, hipStream_t);
   int (*stream_add_norm)(P, P, CP, int, CP, int, int, int, float, hipStream_t);
   int (*embed_bigram)(P, CP, CP, CP, CP, int, int, int, int64_t, int64_t, int64_t, hipStream_t);
   int (*qkv_prepare)(CP, int64_t, P, P, P, int, CP, CP, int, int, int, float, CP, int, CP, CP, CP, int64_t, int, int, CP, int, int, int, int, int, int,
@@ -213,7 +213,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(gated_row_norm, "vk_gated_row_norm"); VK(silu_columns, "vk_silu_columns");
   VK(hyper_in_place, "vk_hyper_in_place"); VK(hyper_step, "vk_hyper_step"); VK(hyper_close, "vk_hyper_close"); VK(embed_normed, "vk_embed_normed");
   VK(attention_wide, "vk_attention_wide"); VK(attention_wide_limit, "vk_attention_wide_limit");
-  VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_act, "vk_gemm_grouped_act");
+  VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_rows, "vk_gemm_grouped_rows");
   VK(stream_add_norm, "vk_stream_add_norm"); VK(embed_bigram, "vk_embed_bigram");
   VK(qkv_prepare, "vk_qkv_prepare"); VK(paged_attention_biased, "vk_paged_attention_biased"); VK(attn_rel_pad, "vk_attn_rel_pad");
 #undef VK
@@ -1345,16 +1345,21 @@ void Kernels::relu_square(Tensor& x) {
 
 bool Kernels::gemm_grouped_takes(int64_t K) const { return K % (dtype_ == DType::BF16 ? 64 : 32) == 0; }
 
-Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation, const Tensor* row_pair) {
-  if (row_pair) expect(*row_pair, "rows' pairs", DType::I32, {act.dim(0)});
+Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation, const Tensor* row_pair, const Tensor* act_row) {
+  const int64_t rows = act_row ? act_row->numel() : act.dim(0);
+  if (row_pair) expect(*row_pair, "rows' pairs", DType::I32, {rows});
+  if (act_row) expect(*act_row, "the activation's rows", DType::I32, {rows});
   expect(act, "activation", dtype_);
   expect(w, "weights", dtype_);
-  if (act.shape.size() != 2 || w.shape.size() != 3 || act.dim(1) != w.dim(2) || act.dim(0) % 128 || !gemm_grouped_takes(act.dim(1)))
+  if (act.shape.size() != 2 || w.shape.size() != 3 || act.dim(1) != w.dim(2) || rows % 128 || !gemm_grouped_takes(act.dim(1)))
     throw EngineError("grouped gemm: activation " + act.describe() + ", weights " + w.describe());
-  expect(block_weights, "the blocks' matrices", DType::I32, {act.dim(0) / 128});
-  Tensor out = empty({act.dim(0), w.dim(1)});
-  call(fn_->gemm_grouped_act(out.data, act.data, w.data, (int)act.dim(0), (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), block_weights.data,
-                             w.dim(1) * w.dim(2), row_pair ? row_pair->data : nullptr, activation, stream));
+  // The kernel reaches a named row by an offset of 31 bits; rows that lie further apart are copied into the product's order first.
+  if (act_row && act.bytes() >= ((size_t)1 << 31)) return gemm_grouped(gather_rows(act, *act_row), w, block_weights, activation, row_pair);
+  expect(block_weights, "the blocks' matrices", DType::I32, {rows / 128});
+  Tensor out = empty({rows, w.dim(1)});
+  call(fn_->gemm_grouped_rows(out.data, act.data, w.data, (int)rows, (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), block_weights.data,
+                              w.dim(1) * w.dim(2), row_pair ? row_pair->data : nullptr, act_row ? act_row->data : nullptr, (int)act.dim(0), activation,
+                              stream));
   return out;
 }
 

@@ -230,7 +230,9 @@ class Kernels {
   // act [M, K] in blocks of 128 rows, block b times the matrix block_weights[b] of w [matrices, N, K] (negative: the
   // block is skipped); [M, N] elements, the bits gemm gives for the same rows and matrix.  K in whole pairs of slabs.
   // row_pair (a plan's): blocks without rows from their 64th on leave that half of their outputs as it is.
-  Tensor gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation = 0, const Tensor* row_pair = nullptr);
+  // act_row: the row of act that each row of the product is (a plan's row_token).
+  Tensor gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation = 0, const Tensor* row_pair = nullptr,
+                      const Tensor* act_row = nullptr);
   bool gemm_grouped_takes(int64_t K) const;
   // moe_route with a choice of score: 0 as moe_route; 1: a chosen expert's weight is the logistic function of its logit.
   // 2: the softmax over all experts as it is.  groups, keep: only experts of the `keep` best of that many equal groups can be

@@ -558,12 +558,13 @@ __device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ be
 
 // PFD > 0: every wave touches, PFD tiles ahead, the 64 rows of the workgroup's tiles that are its share.
 // NWN: waves along the weight rows, two of a workgroup of four waves or four of eight, which takes 64 FNW weight rows.
-template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int PFD = 0, int NWN = 2>
+// GROUPED: block_weights, row_pair and act_row count.
+template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int PFD = 0, int NWN = 2, bool GROUPED = false>
 __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act,
                                                         const elem_t* __restrict__ w, int M, int N, int K,
                                                         int64_t lda, int64_t ldo, int out_form, int band_w,
                                                         const int32_t* __restrict__ block_weights, int64_t weights_stride,
-                                                        const int32_t* __restrict__ row_pair) {
+                                                        const int32_t* __restrict__ row_pair, const int32_t* __restrict__ act_row) {
   static_assert(FNW >= 2 && FNW <= 5 && (FNW == 4 || !SWIGLU), "two to five weight fragments per wave; four with SwiGLU");
   static_assert(PFD == 0 || FNW == 2 || FNW == 4, "the touch-ahead wants a wave's 64 rows to be of one kind");
   static_assert(NWN == 2 || (NWN == 4 && !SWIGLU && PFD == 0), "two waves or four along the weight rows");
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
   }
   // A grouped product: every block of 128 rows has a weight matrix of its own, block_weights[mb] of several that lie
   // weights_stride elements apart (a negative number: the block is not in use).
-  if (block_weights != nullptr) {
+  if constexpr (GROUPED) {
     const int which = block_weights[mb];
     if (which < 0) return;
     w += (int64_t)which * weights_stride;
@@ -601,7 +602,7 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
   const int ntiles = K / (2 * VK_SLAB);
   // A wave without rows (the second half of a group's last block of up to 64 rows: rows without a pair come last in a group) helps to
   // bring the tiles in and leaves the matrix unit to the others.
-  const bool idle = NWN == 4 && row_pair != nullptr && wm == 1 && row_pair[m_blk + 64] < 0;
+  const bool idle = GROUPED && NWN == 4 && row_pair != nullptr && wm == 1 && row_pair[m_blk + 64] < 0;
 
   // A wave-level load moves 8 rows x 128 bytes; lane i fills LDS slot i of the 1 KB block, which is
   // row i/8, physical 16-byte column i%8, i.e. logical column (i%8) ^ (i/8).
@@ -611,7 +612,14 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
   // 32-bit offset per lane that never changes: no vector arithmetic per load.
   const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (int64_t)min(n_blk, N - 1) * K);
   const unsigned char* ubase = reinterpret_cast<const unsigned char*>(w + (int64_t)(N + min(n_blk, N - 1)) * K);   // SWIGLU: the up rows
-  const unsigned char* abase = reinterpret_cast<const unsigned char*>(act + (int64_t)min(m_blk, M - 1) * lda);
+  // act_row: a row of the product is a row of act that the table names (below 2^31 bytes from act's first: the caller's rule).
+  const bool named = GROUPED && act_row != nullptr;
+  const int first_row = named ? 0 : min(m_blk, M - 1);
+  auto act_off = [&](int r, int col) {         // of entry `col` of the block's row r, in bytes from the base
+    const int row = min(m_blk + r, M - 1);
+    return (unsigned)(((int64_t)((named ? act_row[row] : row) - first_row) * lda + col) * (int64_t)sizeof(elem_t));
+  };
+  const unsigned char* abase = reinterpret_cast<const unsigned char*>(act + (int64_t)first_row * lda);
   unsigned offw[FNW], offa[NA];
 #pragma unroll
   for (int j = 0; j < FNW; ++j) {
@@ -621,10 +629,7 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
     offw[j] = (unsigned)(((int64_t)clamped * K + lc * VK_VEC) * (int64_t)sizeof(elem_t));
   }
 #pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    const int clamped = min(m_blk + (wave * NA + j) * 8 + lr, M - 1) - min(m_blk, M - 1);
-    offa[j] = (unsigned)(((int64_t)clamped * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
-  }
+  for (int j = 0; j < NA; ++j) offa[j] = act_off((wave * NA + j) * 8 + lr, lc * VK_VEC);
   const unsigned lds0 = lds_offset_of(lds);
   auto issue = [&](int kt) {                 // PER_TILE loads per wave
     const unsigned base = lds0 + (kt % S) * STAGE_BYTES;
@@ -652,7 +657,7 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
       pf_off = (unsigned)((int64_t)(min(n_blk + local, N - 1) - min(n_blk, N - 1)) * K * (int64_t)sizeof(elem_t));
     } else {
       pf_base = abase;
-      pf_off = (unsigned)((int64_t)(min(m_blk + min(r - BN, 127), M - 1) - min(m_blk, M - 1)) * lda * (int64_t)sizeof(elem_t));
+      pf_off = act_off(min(r - BN, 127), 0);
     }
   }
 
@@ -800,21 +805,21 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
 // which move a column block from part to part, 780 to 830.
 static const int pipe_band_blocks = 64;
 
-template <int S, bool SWIGLU = false, int FNW = 4>
+template <int S, bool SWIGLU = false, int FNW = 4, bool GROUPED = false>
 static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                        int form, hipStream_t st, const int32_t* block_weights = nullptr, int64_t weights_stride = 0,
-                       const int32_t* row_pair = nullptr) {
+                       const int32_t* row_pair = nullptr, const int32_t* act_row = nullptr) {
   constexpr int BN = SWIGLU ? 64 : 32 * FNW;                         // output columns of a workgroup
   const size_t smem = (size_t)S * (32 * FNW + 128) * T_ROWB;         // also holds the 32 KB that SWIGLU passes between waves
   static bool configured = false;
   if (!configured) {
-    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, false, SWIGLU, FNW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 0, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, false, SWIGLU, FNW, 0, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     configured = true;
   }
   dim3 grid((N + BN - 1) / BN, (M + 127) / 128);
   VK_REQUIRE(grid.y <= 65535, "gemm: too many rows (%d)", M);
-  if constexpr (S == 2 && !SWIGLU && FNW == 4 && sizeof(elem_t) == 2) {
+  if constexpr (GROUPED && sizeof(elem_t) == 2) {
     // A grouped product is bound by its weights' way from memory: an expert's matrix serves two or three blocks of rows where a dense
     // product's serves all of them.  Workgroups of 256 weight rows (eight waves) with three stages have two tiles of 48 KB on their way
     // a compute unit where two workgroups of 128 with two stages have two of 32, and 16 column blocks of all row blocks before the next
@@ -822,16 +827,16 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     // idle waves: 2,048 tokens x 3 choices, 6,144 x 4,096 weights 548 -> 484 us, 4,096 x 3,072 290 -> 241; 2,445 x 4, 6,144 x 4,096 690 ->
     // 615; 700 x 3 394 -> 339; 1,360 x 3, 4,608 x 4,096 367 -> 327; 1,334 x 4, 2,048 x 1,536 66 -> 68.  (Touching the weights' lines two to
     // eight tiles ahead instead: 548 -> 586 to 699.)
-    if (block_weights != nullptr && K % KC == 0) {
+    if (K % KC == 0) {
       constexpr size_t wide_smem = (size_t)3 * (256 + 128) * T_ROWB;
       static bool wide = false;
       if (!wide) {
-        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<3, true, false, 4, 0, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_smem);
+        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<3, true, false, 4, 0, 4, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_smem);
         wide = true;
       }
       const dim3 wgrid((N + 255) / 256, grid.y);
-      gemm_pipe_kernel<3, true, false, 4, 0, 4><<<wgrid, 512, wide_smem, st>>>(out, act, w, M, N, K, lda, ldo, form, wgrid.x > 16 ? 16 : (int)wgrid.x, block_weights,
-                                                                              weights_stride, row_pair);
+      gemm_pipe_kernel<3, true, false, 4, 0, 4, true><<<wgrid, 512, wide_smem, st>>>(out, act, w, M, N, K, lda, ldo, form, wgrid.x > 16 ? 16 : (int)wgrid.x, block_weights,
+                                                                              weights_stride, row_pair, act_row);
       return vk_check_launch("gemm_pipe (grouped)");
     }
   }
@@ -844,15 +849,15 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     if (K % KC == 0 && (int64_t)grid.x * grid.y <= device_cus()) {
       static bool touched = false;
       if (!touched) {
-        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 4, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
         touched = true;
       }
-      gemm_pipe_kernel<S, true, SWIGLU, FNW, 4><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
+      gemm_pipe_kernel<S, true, SWIGLU, FNW, 4, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
       return vk_check_launch("gemm_pipe");
     }
   }
-  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
-  else gemm_pipe_kernel<S, false, SWIGLU, FNW><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair);
+  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW, 0, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
+  else gemm_pipe_kernel<S, false, SWIGLU, FNW, 0, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
   return vk_check_launch("gemm_pipe");
 }
 
@@ -1324,17 +1329,28 @@ static int out_form_of(const elem_t* out, int64_t ldo, int activation) {
 // block_weights[b] of several [N, K] matrices that lie weights_stride elements apart (negative: the block is skipped and
 // its output rows are left as they are).  K in whole pairs of slabs (128 bytes of a row).  The same bits as vk_gemm gives
 // for the same rows and matrix.  row_pair [M] or null: a block whose row 64 has a negative entry has no rows from there on, and its
-// outputs there are left as they are.
-int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
-                        const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, int activation, hipStream_t st) {
+// outputs there are left as they are.  act_row [M] or null: row r of the product is row act_row[r] of act, which has act_rows rows
+// (fewer than 2^31 bytes); all entries must lie in 0 .. act_rows - 1, those of rows without a pair too.
+// This spares the rows' copy in the order of the product: 32 us, of 535 with the product (2,048 tokens x 3 choices, 6,144 x 4,096 weights);
+// the product itself, which then finds a token's row in the caches for each of its experts, 505 -> 472 us.
+int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
+                         const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, const int32_t* act_row, int act_rows,
+                         int activation, hipStream_t st) {
   VK_REQUIRE(activation == 0 || activation == 1, "grouped gemm: unknown activation %d", activation);
   VK_REQUIRE(M >= 0 && N > 0 && K > 0 && M % 128 == 0, "grouped gemm: bad sizes M=%d N=%d K=%d (rows in blocks of 128)", M, N, K);
   VK_REQUIRE(K % (2 * VK_SLAB) == 0, "grouped gemm: K=%d must be a multiple of %d", K, 2 * VK_SLAB);
   VK_REQUIRE(lda >= K && lda % VK_VEC == 0 && ldo >= N, "grouped gemm: bad row strides");
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0 && block_weights != nullptr && weights_stride % VK_VEC == 0,
              "grouped gemm: operands must be 16-byte aligned");
+  VK_REQUIRE(act_row == nullptr || (act_rows > 0 && (int64_t)act_rows * lda * (int64_t)sizeof(elem_t) < ((int64_t)1 << 31)),
+             "grouped gemm: %d rows to choose from", act_rows);
   if (M == 0) return 0;
-  return launch_pipe<2>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair);
+  return launch_pipe<2, false, 4, true>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair, act_row);
+}
+
+int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
+                        const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, int activation, hipStream_t st) {
+  return vk_gemm_grouped_rows(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, row_pair, nullptr, 0, activation, st);
 }
 
 int vk_gemm_grouped(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
