@@ -58,3 +58,49 @@ def test_tiles_get_the_plain_product(N, K, dtype):
             assert torch.equal(outs[0][at], want) and torch.equal(outs[2][at], want)
             assert torch.equal(outs[1][at], (want.float().clamp(min=0.0) ** 2).to(dtype))
     assert torch.isnan(outs[0][pair < 0]).all()           # nothing is stored there
+
+
+def offered_plan(counts, offered, top):
+    """A plan of `counts` rows an expert, in tiles of 16, as long as the launches of `offered` tokens expect it: pair, token, tile, start."""
+    tiles, pairs, start = [], [], [0]
+    for e, n in enumerate(counts):
+        here = -(-n // 16)
+        tiles += [e] * here
+        pairs += list(range(len(pairs), len(pairs) + n)) + [-1] * (16 * here - n)
+        start.append(len(pairs))
+    most = (offered * top + min(len(counts), offered * top) * 15) // 16
+    assert len(tiles) <= most
+    pairs += [-1] * (16 * most - len(pairs))
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    return dev(pairs), dev(tiles + [-1] * (most - len(tiles))), dev(start)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K", [96, 544, 1184, 2304, 4640])
+def test_an_infinite_weight_gives_infinities(K, dtype):
+    """In the last slab of a reduction that ends inside a chunk: the product is infinite with the sign of the row's entry, and no other
+    output notices."""
+    k, N, top, offered = kern(dtype), 40, 4, 16384
+    counts = [5, 16, 2]
+    pair, tile, start = offered_plan(counts, offered, top)
+    w = rand((len(counts), N, K), dtype, 5, 0.1).cuda()
+    x = rand((20, K), dtype, 6).cuda()
+    w[1, 7, K - 3] = float("inf")
+    token = torch.randint(0, len(x), (len(pair),), generator=torch.Generator().manual_seed(2)).to(torch.int32).cuda()
+    rows = x[token.long()].contiguous()
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    up, down = k.lib.vk_moe_up_plain, k.lib.vk_moe_down
+    up.argtypes, down.argtypes = [p, l, p, l, p, p, p, p, p, i, i, i, i, i, p], [p, p, l, p, p, p, p, i, i, i, i, i, p]
+    outs = [torch.full((len(pair), N), float("nan"), dtype=dtype, device="cuda") for _ in range(2)]
+    stream = torch.cuda.current_stream().cuda_stream
+    sizes = (offered, top, len(counts), N, K, stream)
+    assert up(outs[0].data_ptr(), N, x.data_ptr(), K, w.data_ptr(), pair.data_ptr(), token.data_ptr(), tile.data_ptr(), start.data_ptr(), *sizes) == 0
+    assert down(outs[1].data_ptr(), rows.data_ptr(), K, w.data_ptr(), pair.data_ptr(), tile.data_ptr(), start.data_ptr(), *sizes) == 0
+    at = start.tolist()
+    for out in outs:
+        for e, n in enumerate(counts):
+            got = out[at[e]:at[e] + n].double()
+            if e == 1:
+                assert torch.equal(got[:, 7], torch.copysign(torch.full_like(got[:, 7], float("inf")), rows[at[e]:at[e] + n, K - 3].double()))
+                got[:, 7] = 0.0
+            assert torch.isfinite(got).all()

@@ -377,7 +377,8 @@ __global__ __launch_bounds__(64 * MOE_WAVES) void moe_gemm_kernel(elem_t* __rest
 // features) units of all tiles in use, tile by tile; a wave keeps its chunk of the tile's rows in registers and streams the weights
 // through a window of MOE_STREAM_W slabs that runs on across units and tiles; one barrier a unit, and the waves take turns at adding
 // up a unit's chunk sums.  No load is predicated: rows without a pair are read like others and not stored, features beyond N are clamped.
-// WHOLE: K in whole chunks; else the last chunk's missing slabs are read again from its last one and multiplied by zeros.
+// WHOLE: K in whole chunks; else the loads of the last chunk's missing slabs read its last one again, and the products are left out (a
+// product with zeros would make a NaN of an infinite weight).
 // Measured on MI355X, 32 experts, eight tokens: 4 choices, 3,072 x 2,048 weights 62.7 -> 53.4 us, 2,048 x 1,536 36.5 -> 31.6 (a plain
 // read of so many bytes, 260 and 130 MB, is about as long); five tokens of 3 choices, 4,096 x 4,608 75.1 -> 70.8.
 #ifdef VK_BF16
@@ -406,10 +407,7 @@ __global__ __launch_bounds__(64 * MOE_STREAM_CHUNKS) void moe_stream_kernel(elem
     const int row = tile * MOE_TILE + r16;
     const elem_t* xr = x + (int64_t)(MODE != 0 ? row_token[row] : row) * ldx + k0;
 #pragma unroll
-    for (int i = 0; i < SL; ++i) {
-      rows[i] = *reinterpret_cast<const frag_t*>(xr + at(i));
-      if (!WHOLE && i >= have) rows[i] = zero_frag();
-    }
+    for (int i = 0; i < SL; ++i) rows[i] = *reinterpret_cast<const frag_t*>(xr + at(i));
   };
   int tile = lo / features, f = lo - tile * features;
   const elem_t* here = weights(tile, f);
@@ -426,7 +424,7 @@ __global__ __launch_bounds__(64 * MOE_STREAM_CHUNKS) void moe_stream_kernel(elem
       const frag_t fw = window[i % W];
       if (i + W < SL) window[i % W] = *reinterpret_cast<const frag_t*>(here + at(i + W));
       else if (more) window[i % W] = *reinterpret_cast<const frag_t*>(next + at(i + W - SL));
-      acc = mma_slab(fw, rows[i], acc);
+      if (WHOLE || i < have) acc = mma_slab(fw, rows[i], acc);
     }
     f32x4* sums = part + (size_t)parity * waves * 64;
     sums[wave * 64 + lane] = acc;
