@@ -190,3 +190,29 @@ def test_the_short_convolution(K, C, with_bias, dtype):
         torch.cuda.synchronize()
         # 32-bit sums of up to six products and a logistic function.
         assert (y.cpu().double() - torch.stack(want)).abs().max() < 2e-5
+
+
+def test_more_channels_than_a_grid_of_groups():
+    """More than 65,535 groups of 256 channels: as many sequences as tokens, and fewer, against the same channels in two halves."""
+    k, K = kern(torch.bfloat16), 2
+    C = 256 * 65535 + 512
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    fn = k.lib.vk_delta_conv
+    fn.argtypes = [p, p, l, p, p, l, l, p, p, p, p, i, i, i, i, p]
+    g = torch.Generator(device="cuda").manual_seed(7)
+    for T in (1, 3):
+        x, taps = (torch.randn(n, C, device="cuda", generator=g).to(torch.bfloat16) for n in (T, K))
+        taps = taps.T.contiguous()
+        seq, cu, positions, slots = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0] * T, [0, T], [1 + t for t in range(T)], [0]))
+        tail = torch.randn(1, C, device="cuda", generator=g)
+        outs = []
+        for cuts in ((0, C), (0, C // 2, C)):
+            state, y = tail.clone(), torch.full((T, C), float("nan"), device="cuda")
+            for a, b in zip(cuts, cuts[1:]):
+                part, tails = (y if b - a == C else y[:, a:b].contiguous()), state[:, a:b].contiguous()
+                assert fn(part.data_ptr(), x[:, a:].data_ptr(), C, taps[a:b].contiguous().data_ptr(), tails.data_ptr(), b - a, 0, seq.data_ptr(), cu.data_ptr(),
+                          positions.data_ptr(), slots.data_ptr(), T, 1, b - a, K, torch.cuda.current_stream().cuda_stream) == 0
+                y[:, a:b], state[:, a:b] = part, tails
+            outs.append((y, state))
+        assert not torch.isnan(outs[0][0]).any()
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])

@@ -754,7 +754,7 @@ int vk_delta_lanes_per_column(int d) {
 }
 
 // y [T, C] floats from the columns x[:, 0:C] of rows of length ldx; then the tails are moved on.  bias: [C] or null, what
-// every channel's sum starts from.
+// every channel's sum starts from.  T: the step's tokens, at least one a sequence.
 static int conv_launch(float* y, const elem_t* x, int64_t ldx, const elem_t* taps, const elem_t* bias, float* state, int64_t state_stride,
                        int64_t tail_offset, const int32_t* token_seq, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T,
                        int S, int C, int K, hipStream_t st) {
@@ -762,14 +762,15 @@ static int conv_launch(float* y, const elem_t* x, int64_t ldx, const elem_t* tap
              DELTA_MAX_TAPS + 1);
   VK_REQUIRE(ldx >= C && tail_offset >= 0 && state_stride >= tail_offset + (int64_t)(K - 1) * C, "short convolution: the state does not hold the tails");
   if (T == 0 || S == 0) return 0;
-  VK_REQUIRE((C + 255) / 256 <= 65535, "short convolution: too many channels (%d)", C);
-  if (T == S) {                 // every sequence brings one token
-    delta_conv_token_kernel<<<dim3(S, (C + 255) / 256), 256, 0, st>>>(y, x, ldx, taps, state, state_stride, tail_offset, cu_q, positions, slots, C, K, bias);
+  // Groups of channels: more than a grid has room for are left to the kernel for every shape, whose workgroups walk them.
+  const int groups = (C + 255) / 256;
+  if (T == S && groups <= 65535) {                 // every sequence brings one token
+    delta_conv_token_kernel<<<dim3(S, groups), 256, 0, st>>>(y, x, ldx, taps, state, state_stride, tail_offset, cu_q, positions, slots, C, K, bias);
     return vk_check_launch("short convolution (single tokens)");
   }
-  const int by = (C + 255) / 256 < 64 ? (C + 255) / 256 : 64;
+  const int by = groups < 64 ? groups : 64;
   const size_t four = 4 * sizeof(elem_t);
-  if (K >= 2 && K <= 4 && C % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % four == 0 && state_stride % 4 == 0 && tail_offset % 4 == 0 &&
+  if (K >= 2 && K <= 4 && groups <= 4 * 65535 && C % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % four == 0 && state_stride % 4 == 0 && tail_offset % 4 == 0 &&
       (((uintptr_t)y | (uintptr_t)state) & 15) == 0) {
     const dim3 wgrid((T + CONV_TOKENS - 1) / CONV_TOKENS, (C / 4 + 255) / 256);
 #define CONV_WALK(K_) delta_conv_walk_kernel<K_><<<wgrid, 256, 0, st>>>(y, x, ldx, taps, state, state_stride, tail_offset, token_seq, cu_q, positions, slots, T, C, bias)
