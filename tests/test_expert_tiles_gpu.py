@@ -76,7 +76,7 @@ def offered_plan(counts, offered, top):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("K", [96, 544, 1184, 2304, 4640])
+@pytest.mark.parametrize("K", [96, 544, 1184, 1920, 2304, 4640])
 def test_an_infinite_weight_gives_infinities(K, dtype):
     """In the last slab of a reduction that ends inside a chunk: the product is infinite with the sign of the row's entry, and no other
     output notices."""
@@ -104,3 +104,43 @@ def test_an_infinite_weight_gives_infinities(K, dtype):
                 assert torch.equal(got[:, 7], torch.copysign(torch.full_like(got[:, 7], float("inf")), rows[at[e]:at[e] + n, K - 3].double()))
                 got[:, 7] = 0.0
             assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K", [(4104, 512), (2056, 1024), (1048, 1536), (1048, 2048), (1048, 2560), (264, 4608), (264, 8192), (4104, 480), (2056, 992),
+                                 (1048, 1184), (1048, 1920), (1048, 2304)])
+def test_workgroups_that_stay_for_several_units(N, K, dtype):
+    """More (tile, 16 features) units than the device holds workgroups of the streaming kernel, two to three a workgroup: its window goes on from
+    unit to unit, tile to tile and expert to expert, the last features are clamped, and every row in use still gets the plain product."""
+    k, top = kern(dtype), 4
+    counts = [0, 16, 17, 130, 1, 300, 5, 128]
+    used, features = sum(-(-n // 16) for n in counts), -(-N // 16)
+    chunks, cus = -(-K // 512), torch.cuda.get_device_properties(0).multi_processor_count
+    assert used * features > 2 * cus * (16 // chunks)
+    # As many tokens as a launch of this kernel's sizes needs, whichever of its lines applies.
+    offered = -(-max(used, -(-12288 // features)) * 16 // top)
+    pair, tile, start = offered_plan(counts, offered, top)
+    w = torch.randn(len(counts), N, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(5)).mul_(0.1).to(dtype)
+    x = rand((64, K), dtype, 6).cuda()
+    token = torch.randint(0, len(x), (len(pair),), generator=torch.Generator().manual_seed(2)).to(torch.int32).cuda()
+    token[pair < 0] = 0
+    rows = x[token.long()].contiguous()
+    rows[pair < 0] = float("nan")                          # rows without a pair may hold anything
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    up, act, down = k.lib.vk_moe_up_plain, k.lib.vk_moe_up, k.lib.vk_moe_down
+    up.argtypes = act.argtypes = [p, l, p, l, p, p, p, p, p, i, i, i, i, i, p]
+    down.argtypes = [p, p, l, p, p, p, p, i, i, i, i, i, p]
+    stream = torch.cuda.current_stream().cuda_stream
+    sizes = (offered, top, len(counts), N, K, stream)
+    outs = [torch.full((len(pair), N), float("nan"), dtype=dtype, device="cuda") for _ in range(3)]
+    for fn, out in ((up, outs[0]), (act, outs[1])):
+        assert fn(out.data_ptr(), N, x.data_ptr(), K, w.data_ptr(), pair.data_ptr(), token.data_ptr(), tile.data_ptr(), start.data_ptr(), *sizes) == 0
+    assert down(outs[2].data_ptr(), rows.data_ptr(), K, w.data_ptr(), pair.data_ptr(), tile.data_ptr(), start.data_ptr(), *sizes) == 0
+    at = start.tolist()
+    for e, n in enumerate(counts):
+        if n:
+            here = slice(at[e], at[e] + n)
+            want = k.gemm(rows[here].contiguous(), w[e])
+            assert torch.equal(outs[0][here], want) and torch.equal(outs[2][here], want)
+            assert torch.equal(outs[1][here], (want.float().clamp(min=0.0) ** 2).to(dtype))
+    assert all(torch.isnan(out[pair < 0]).all() for out in outs)          # nothing is stored there

@@ -625,16 +625,41 @@ static int moe_cus() {
 
 // An expert product of rows in tiles of 16: by the streaming kernel where it takes the sizes, else by the one for every K.
 extern "C++" {
+#ifdef VK_BF16
+// The (row tile, 16 features) units, of all tiles that a launch covers, from which on the streaming kernel is the faster one; 0: never.
+// Below, the other kernel's workgroups all run at once, and the streaming one's longer start (the tiles in use, a tile's expert, its
+// rows) is what a call waits for, longer still where the rows need no table (not gathered).  Measured on MI355X in recorded launches, 8
+// to 64 experts, 512 to 9,216 features, 1 to 250 tokens, the weights of two to twelve layers in turn; the other kernel against this one, us,
+// 32 experts, 4 choices, the units in brackets:
+//   one chunk: 512 x 512 weights, one token (128) 3.8, 3.2; rows as they are the same;
+//   two, rows as they are: 768 x 1,024, two tokens (384) 5.9, 6.3; 1,536 x 1,024, two (768) 10.0, 8.5;
+//   three: 512 x 1,536, five (640) 8.2, 9.7, 1,024 x 1,536, three (768) 12.7, 10.2; rows as they are, 2,048 features, two (1,024) 14.1, 14.5, 512
+//   features, 40 (1,280) 16.1, 15.5;
+//   four: 512 x 2,048, five (640) 9.8, 12.1, 1,024 x 2,048, three (768) 14.6, 12.3; rows as they are, 3,072 features, two (1,536) 24.3,
+//   28.7, 1,024 features, 24 (2,304) 33.1, 31.1;
+//   five: 1,024 x 2,560, eight (2,048) 29.6, 31.5, 512 features, 250 (2,944) 55.2, 49.1; rows as they are, 2,048 features, 24 (4,608) 75.4,
+//   80.6, 64 (5,888) 91.3, 82.8.
+// Six to eight chunks keep six to eight of the other kernel's eight waves at work in one round: three tokens of 3 choices, 6,144 x 4,096
+// weights, 90.0, 91.2.  Nine and more leave it a second round that is mostly empty: rows as they are, 512 x 4,608, three (384) 18.2, 20.8,
+// 4,096 features, one (1,024) 36.0, 35.2.
+// A reduction that ends inside a chunk costs every wave an address a slab: rows as they are, 2,048 x 768, eight (4,096) 30.2, 36.5, 40 (5,120)
+// 41.0, 40.5; 2,048 x 1,152, 40 (5,120) 48.7, 51.5; 4,096 x 1,920, eight (8,192) 85.7, 97.2; 2,048 x 2,304, 250 (11,776) 172, 191.
+static int moe_stream_units(int chunks, bool whole, bool gathered) {
+  constexpr int WHOLE[2][5] = {{1, 768, 1280, 2304, 5632}, {1, 1, 768, 768, 2560}};
+  constexpr int PARTS[2][4] = {{2304, 4608, 5632, 10240}, {768, 4096, 3072, 5632}};
+  if (!whole) return chunks <= 4 ? PARTS[gathered][chunks - 1] : 0;
+  if (chunks <= 5) return WHOLE[gathered][chunks - 1];
+  return chunks <= MOE_WAVES || chunks > MOE_STREAM_CHUNKS ? 0 : (gathered ? 1 : 768);
+}
+#endif
 template <int MODE>
 static int moe_product(elem_t* out, int64_t ldo, const elem_t* x, int64_t ldx, const elem_t* w, const int32_t* row_pair, const int32_t* row_token,
                        const int32_t* tile_expert, const int32_t* expert_start, int tiles, int E, int N, int K, hipStream_t st, const char* what) {
 #ifdef VK_BF16
-  const int chunks = (K + MOE_KC - 1) / MOE_KC;
-  // Six to eight chunks keep six to eight of the other kernel's eight waves at work in one round, and its many workgroups then bring the
-  // larger matrices in as fast (three tokens, 6,144 x 4,096 weights: 90.0 us there, 91.2 here; 4,096 x 3,072: 52.7, 54.0).
-  if (K % VK_SLAB == 0 && ldx % VK_VEC == 0 && (chunks <= 5 || (chunks > MOE_WAVES && chunks <= MOE_STREAM_CHUNKS))) {
+  const int chunks = (K + MOE_KC - 1) / MOE_KC, least = moe_stream_units(chunks, K % MOE_KC == 0, MODE != 0);
+  const int64_t units = (int64_t)tiles * ((N + 15) / 16);
+  if (K % VK_SLAB == 0 && ldx % VK_VEC == 0 && least != 0 && units >= least) {
     // As many workgroups as the device holds at once: 16 waves a compute unit (128 registers).
-    const int64_t units = (int64_t)tiles * ((N + 15) / 16);
     const int grid = (int)std::min<int64_t>(units, (int64_t)moe_cus() * (16 / chunks));
     const int vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
     const size_t smem = (size_t)2 * chunks * 64 * sizeof(f32x4);
