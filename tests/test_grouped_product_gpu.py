@@ -74,3 +74,44 @@ def test_named_rows_are_as_their_copy(N, K, lda, dtype):
         assert torch.equal(*outs)
         # More bytes than the offsets reach are refused.
         assert fn(outs[0].data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, lda, N, which.data_ptr(), N * K, None, row.data_ptr(), 1 << 30, 0, stream) != 0
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,K,activation", [(96, 1024, 1), (256, 512, 0), (1100, 512, 0), (2048, 512, 0), (4200, 512, 1), (4400, 512, 0), (4400, 192, 0)])
+def test_workgroups_of_both_widths(N, K, activation, dtype):
+    """The number of matrices, said or not, chooses between workgroups of 256 and of 128 weight rows: the same bits, rows named and copied, idle halves
+    and none.  More than 4,096 weight rows are walked in two bands of column blocks; they end inside a workgroup's tile."""
+    k = kern(dtype)
+    g = torch.Generator().manual_seed(3)
+    counts = [1, 63, 64, 65, 128, 0, 129, 200]
+    w = rand((len(counts), N, K), dtype, 5, 0.1).cuda()
+    x = rand((77, K), dtype, 6).cuda()
+    blocks, pairs = [], []
+    for e, n in enumerate(counts):
+        here = -(-n // 128)
+        blocks += [e] * here
+        pairs += list(range(n)) + [-1] * (128 * here - n)
+    blocks, pairs = blocks + [-1], pairs + [-1] * 128
+    M = len(pairs)
+    named = torch.randint(0, len(x), (M,), generator=g, dtype=torch.int32)
+    copy = x[named.long().cuda()].contiguous()
+    which, row_pair, row = (torch.as_tensor(v, dtype=torch.int32).cuda() for v in (blocks, pairs, named))
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    fn = k.lib.vk_gemm_grouped_experts
+    fn.argtypes = [p, p, p, i, i, i, l, l, p, l, i, p, p, i, i, p]
+    stream = torch.cuda.current_stream().cuda_stream
+    for matrices in (0, len(counts)):
+        for act, rows in ((copy, None), (x, row.data_ptr())):
+            for given in (None, row_pair.data_ptr()):
+                out = torch.zeros(M, N, dtype=dtype, device="cuda")
+                assert fn(out.data_ptr(), act.data_ptr(), w.data_ptr(), M, N, K, K, N, which.data_ptr(), N * K, matrices, given, rows, len(x), activation,
+                          stream) == 0
+                at = 0
+                for e, n in enumerate(counts):
+                    if n:
+                        want = k.gemm(copy[at:at + n], w[e])
+                        if activation:
+                            want = (want.float().clamp(min=0.0) ** 2).to(dtype)
+                        assert torch.equal(out[at:at + n], want)
+                    at += 128 * (-(-n // 128))
+                assert (out[M - 128:] == 0).all()          # the block that is not in use

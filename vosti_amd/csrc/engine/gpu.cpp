@@ -123,7 +123,6 @@ struct Kernels::Fn {
   int (*ssm_scan)(P, CP, int64_t, int, int, CP, int64_t, CP, CP, CP, int, P, int64_t, CP, CP, CP, int, int, int, int, int, int, hipStream_t);
   int (*ssm_gate_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, hipStream_t);
   int (*moe_max_tiles)(int, int, int, int);
-  int (*gemm_grouped)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, hipStream_t);
   int (*moe_route_plan)(P, P, P, CP, CP, CP, int, CP, int, int, int, int, int, float, int, int, int, int, float, P, P, P, P, P, int, hipStream_t);
   int (*moe_up)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_down)(P, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
@@ -158,7 +157,7 @@ struct Kernels::Fn {
   int (*attention_wide_limit)();
   int (*gemm_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_split_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
-  int (*gemm_grouped_rows)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, CP, CP, int, int, hipStream_t);
+  int (*gemm_grouped_experts)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, int, CP, CP, int, int, hipStream_t);
   int (*stream_add_norm)(P, P, CP, int, CP, int, int, int, float, hipStream_t);
   int (*embed_bigram)(P, CP, CP, CP, CP, int, int, int, int64_t, int64_t, int64_t, hipStream_t);
   int (*qkv_prepare)(CP, int64_t, P, P, P, int, CP, CP, int, int, int, float, CP, int, CP, CP, CP, int64_t, int, int, CP, int, int, int, int, int, int,
@@ -202,7 +201,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(qkv_post_angles, "vk_qkv_post_angles"); VK(embed_scaled, "vk_embed_scaled"); VK(stream_add, "vk_stream_add");
   VK(stream_pair_norm, "vk_stream_pair_norm"); VK(ssm_scan, "vk_ssm_scan"); VK(ssm_gate_norm, "vk_ssm_gate_norm");
   VK(moe_max_tiles, "vk_moe_max_tiles"); VK(moe_route_plan, "vk_moe_route_plan"); VK(moe_up, "vk_moe_up");
-  VK(moe_down, "vk_moe_down"); VK(moe_combine, "vk_moe_combine"); VK(moe_relu_square, "vk_moe_relu_square"); VK(gemm_grouped, "vk_gemm_grouped");
+  VK(moe_down, "vk_moe_down"); VK(moe_combine, "vk_moe_combine"); VK(moe_relu_square, "vk_moe_relu_square");
   VK(qkv_post_norm_angles, "vk_qkv_post_norm_angles"); VK(gate_mul, "vk_gate_mul"); VK(gla_decay, "vk_gla_decay"); VK(gla_rule, "vk_gla_rule");
   VK(gated_head_norm, "vk_gated_head_norm"); VK(moe_up_plain, "vk_moe_up_plain"); VK(moe_glu, "vk_moe_glu");
   VK(moe_combine_add, "vk_moe_combine_add"); VK(stream_norm_add_f32, "vk_stream_norm_add_f32");
@@ -213,7 +212,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(gated_row_norm, "vk_gated_row_norm"); VK(silu_columns, "vk_silu_columns");
   VK(hyper_in_place, "vk_hyper_in_place"); VK(hyper_step, "vk_hyper_step"); VK(hyper_close, "vk_hyper_close"); VK(embed_normed, "vk_embed_normed");
   VK(attention_wide, "vk_attention_wide"); VK(attention_wide_limit, "vk_attention_wide_limit");
-  VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_rows, "vk_gemm_grouped_rows");
+  VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_experts, "vk_gemm_grouped_experts");
   VK(stream_add_norm, "vk_stream_add_norm"); VK(embed_bigram, "vk_embed_bigram");
   VK(qkv_prepare, "vk_qkv_prepare"); VK(paged_attention_biased, "vk_paged_attention_biased"); VK(attn_rel_pad, "vk_attn_rel_pad");
 #undef VK
@@ -1357,8 +1356,8 @@ Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& b
   if (act_row && act.bytes() >= ((size_t)1 << 31)) return gemm_grouped(gather_rows(act, *act_row), w, block_weights, activation, row_pair);
   expect(block_weights, "the blocks' matrices", DType::I32, {rows / 128});
   Tensor out = empty({rows, w.dim(1)});
-  call(fn_->gemm_grouped_rows(out.data, act.data, w.data, (int)rows, (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), block_weights.data,
-                              w.dim(1) * w.dim(2), row_pair ? row_pair->data : nullptr, act_row ? act_row->data : nullptr, (int)act.dim(0), activation,
+  call(fn_->gemm_grouped_experts(out.data, act.data, w.data, (int)rows, (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), block_weights.data,
+                              w.dim(1) * w.dim(2), (int)w.dim(0), row_pair ? row_pair->data : nullptr, act_row ? act_row->data : nullptr, (int)act.dim(0), activation,
                               stream));
   return out;
 }

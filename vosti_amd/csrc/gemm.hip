@@ -533,7 +533,7 @@ __device__ __forceinline__ void pipe_load_to_lds16(const elem_t* src, unsigned c
 // 32-bit offset per lane.  The compiler's own form of it adds base and offset in vector registers before every
 // load (it moves what does not change along K out of the loop and is left with a vector sum); written out, the
 // advancing base costs two scalar additions per K tile for all loads together.  lds_addr: the wave's 1 KB
-// block in LDS, below 64 KB.
+// block, anywhere in LDS (the grouped product's third stage starts at 96 KB).
 __device__ __forceinline__ void pipe_load_to_lds16_sv(const unsigned char* sbase, unsigned voff, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");     // m0 is the compiler's scratch: it sets it anew before every use of its own
 }
@@ -805,10 +805,27 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
 // which move a column block from part to part, 780 to 830.
 static const int pipe_band_blocks = 64;
 
+// Whether a grouped product of 16-bit elements and K in whole chunks goes by workgroups of 256 weight rows (launch_pipe) or of 128.
+// The wide ones have one workgroup a compute unit, so that a launch of few is one round half empty where the narrow ones have two a unit or
+// the touch-ahead; and a column block that lands on another chip part with each row block (columns that are no multiple of eight, up to 16)
+// has its weights read by several.  But up to about 60 rows a matrix (M and the matrices tell: a matrix has up to 127 rows of padding)
+// half of most blocks is idle, which only the wide ones leave out.  Measured on MI355X in recorded launches with the weights of
+// several layers in turn, 947 sizes of 2 to 64 matrices, 40 to 4,096 tokens, rows named, narrow against wide, us: 32 matrices, 4 choices, 257
+// tokens 1,536 x 1,024 25.8, 22.9; 2,048 tokens 1,536 x 1,024 50.5, 57.6, 3,072 x 2,048 163, 165, 6,144 x 4,096 594, 542; 8 matrices, 2 choices,
+// 257 tokens 512 x 512 8.7, 11.7.  Rows as they lie are read by more workgroups of the narrow kernel: 2,048 tokens,
+// 768 x 1,024 42.4, 35.9.  Slower by more than 3 % than the better of the two: 82 sizes, as they
+// lie 94; the wide ones alone 415 and 353, the narrow ones 336 and 419.
+static bool grouped_wide(int M, int N, int matrices, bool named) {
+  const int64_t columns = (N + 255) / 256, groups = columns * (M / 128);
+  if (matrices > 0 && (int64_t)M + 127 <= (int64_t)matrices * (127 + 60)) return true;
+  if (columns % 8 == 0 || columns > 16) return 8 * groups >= 5 * device_cus();
+  return !named && columns <= 4 && 2 * groups >= device_cus();
+}
+
 template <int S, bool SWIGLU = false, int FNW = 4, bool GROUPED = false>
 static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                        int form, hipStream_t st, const int32_t* block_weights = nullptr, int64_t weights_stride = 0,
-                       const int32_t* row_pair = nullptr, const int32_t* act_row = nullptr) {
+                       const int32_t* row_pair = nullptr, const int32_t* act_row = nullptr, int matrices = 0) {
   constexpr int BN = SWIGLU ? 64 : 32 * FNW;                         // output columns of a workgroup
   const size_t smem = (size_t)S * (32 * FNW + 128) * T_ROWB;         // also holds the 32 KB that SWIGLU passes between waves
   static bool configured = false;
@@ -825,9 +842,9 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     // a compute unit where two workgroups of 128 with two stages have two of 32, and 16 column blocks of all row blocks before the next
     // 16 keep the blocks of an expert together in time and on their chip part.  Measured on MI355X, 32 experts, before and after with the
     // idle waves: 2,048 tokens x 3 choices, 6,144 x 4,096 weights 548 -> 484 us, 4,096 x 3,072 290 -> 241; 2,445 x 4, 6,144 x 4,096 690 ->
-    // 615; 700 x 3 394 -> 339; 1,360 x 3, 4,608 x 4,096 367 -> 327; 1,334 x 4, 2,048 x 1,536 66 -> 68.  (Touching the weights' lines two to
+    // 615; 700 x 3 394 -> 339; 1,360 x 3, 4,608 x 4,096 367 -> 327.  (Touching the weights' lines two to
     // eight tiles ahead instead: 548 -> 586 to 699.)
-    if (K % KC == 0) {
+    if (K % KC == 0 && grouped_wide(M, N, matrices, act_row != nullptr)) {
       constexpr size_t wide_smem = (size_t)3 * (256 + 128) * T_ROWB;
       static bool wide = false;
       if (!wide) {
@@ -1333,9 +1350,10 @@ static int out_form_of(const elem_t* out, int64_t ldo, int activation) {
 // (fewer than 2^31 bytes); all entries must lie in 0 .. act_rows - 1, those of rows without a pair too.
 // This spares the rows' copy in the order of the product: 32 us, of 535 with the product (2,048 tokens x 3 choices, 6,144 x 4,096 weights);
 // the product itself, which then finds a token's row in the caches for each of its experts, 505 -> 472 us.
-int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
-                         const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, const int32_t* act_row, int act_rows,
-                         int activation, hipStream_t st) {
+// matrices: how many w holds, or 0 where the caller does not say; it only helps to choose the kernel (grouped_wide).
+int vk_gemm_grouped_experts(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
+                            const int32_t* block_weights, int64_t weights_stride, int matrices, const int32_t* row_pair, const int32_t* act_row,
+                            int act_rows, int activation, hipStream_t st) {
   VK_REQUIRE(activation == 0 || activation == 1, "grouped gemm: unknown activation %d", activation);
   VK_REQUIRE(M >= 0 && N > 0 && K > 0 && M % 128 == 0, "grouped gemm: bad sizes M=%d N=%d K=%d (rows in blocks of 128)", M, N, K);
   VK_REQUIRE(K % (2 * VK_SLAB) == 0, "grouped gemm: K=%d must be a multiple of %d", K, 2 * VK_SLAB);
@@ -1345,7 +1363,14 @@ int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M,
   VK_REQUIRE(act_row == nullptr || (act_rows > 0 && (int64_t)act_rows * lda * (int64_t)sizeof(elem_t) < ((int64_t)1 << 31)),
              "grouped gemm: %d rows to choose from", act_rows);
   if (M == 0) return 0;
-  return launch_pipe<2, false, 4, true>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair, act_row);
+  return launch_pipe<2, false, 4, true>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair, act_row,
+                                         matrices);
+}
+
+int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
+                         const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, const int32_t* act_row, int act_rows,
+                         int activation, hipStream_t st) {
+  return vk_gemm_grouped_experts(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, 0, row_pair, act_row, act_rows, activation, st);
 }
 
 int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
