@@ -216,3 +216,44 @@ def test_more_channels_than_a_grid_of_groups():
             outs.append((y, state))
         assert not torch.isnan(outs[0][0]).any()
         assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K,with_bias", [(2, False), (3, True), (4, False), (4, True)])
+def test_many_channels_at_once_and_few(K, with_bias, dtype):
+    """Tokens times channels choose the kernel: all channels in one call and in pieces of 1,028 give the same bits and tails, for groups of 16 tokens within
+    a sequence, across several and at the end."""
+    k, C, piece, offset = kern(dtype), 32896, 1028, 8
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    fn = k.lib.vk_delta_conv_bias if with_bias else k.lib.vk_delta_conv
+    fn.argtypes = [p, p, l, p] + ([p] if with_bias else []) + [p, l, l, p, p, p, p, i, i, i, i, p]
+    g = torch.Generator(device="cuda").manual_seed(9)
+    new = lambda *n: torch.randn(*n, device="cuda", generator=g)
+    taps, bias = (0.4 * new(C, K)).to(dtype), (0.2 * new(C)).to(dtype)
+    for lengths in ([64], [40, 1, 17, 6], [1] * 9 + [2, 33, 21]):
+        T, S = sum(lengths), len(lengths)
+        assert T * C >= 1 << 21 > T * piece
+        x = new(T, C).to(dtype)
+        cu = [0]
+        for n in lengths:
+            cu.append(cu[-1] + n)
+        positions = [(0 if s % 2 else 3) + t for s, n in enumerate(lengths) for t in range(n)]
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+        where = [i32(v) for v in ([s for s, n in enumerate(lengths) for _ in range(n)], cu, positions, list(range(S))[::-1])]
+        tails = new(S, K - 1, C)
+        outs = []
+        for step in (C, piece):
+            y, after = torch.full((T, C), float("nan"), device="cuda"), torch.zeros_like(tails)
+            for a in range(0, C, step):
+                n = min(step, C - a)
+                part, here = torch.full((T, n), float("nan"), device="cuda"), x[:, a:a + n].contiguous()
+                state = torch.zeros(S, offset + (K - 1) * n, device="cuda")
+                state[:, offset:] = tails[:, :, a:a + n].reshape(S, -1)
+                tp, bs = taps[a:a + n].contiguous(), bias[a:a + n].contiguous()
+                args = (part.data_ptr(), here.data_ptr(), n, tp.data_ptr()) + ((bs.data_ptr(),) if with_bias else ())
+                assert fn(*args, state.data_ptr(), state.shape[1], offset, *(v.data_ptr() for v in where), T, S, n, K,
+                          torch.cuda.current_stream().cuda_stream) == 0
+                y[:, a:a + n], after[:, :, a:a + n] = part, state[:, offset:].view(S, K - 1, n)
+            outs.append((y, after))
+        assert not torch.isnan(outs[0][0]).any()
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])

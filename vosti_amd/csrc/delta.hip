@@ -770,7 +770,11 @@ static int conv_launch(float* y, const elem_t* x, int64_t ldx, const elem_t* tap
   }
   const int by = groups < 64 ? groups : 64;
   const size_t four = 4 * sizeof(elem_t);
-  if (K >= 2 && K <= 4 && groups <= 4 * 65535 && C % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % four == 0 && state_stride % 4 == 0 && tail_offset % 4 == 0 &&
+  // The walk's group of tokens is a chain of 16, and of a look back for every sequence that starts in it: a launch of few waits for that, where
+  // the kernel for every shape has a thread an output.  That one against the walk, in recorded launches with the tails' one, 4 taps, us: 25
+  // tokens of 24 sequences, 3,072 channels, 7.3, 18.6; sequences of 40, 3,072 channels: 300 tokens 10.3, 13.3, 700 16.3, 14.4, 1,500 35.6, 20.3;
+  // 12,288 channels: 100 tokens 11.8, 13.7, 200 19.6, 14.9, 400 37.9, 20.6.
+  if ((int64_t)T * C >= (1 << 21) && K >= 2 && K <= 4 && groups <= 4 * 65535 && C % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % four == 0 && state_stride % 4 == 0 && tail_offset % 4 == 0 &&
       (((uintptr_t)y | (uintptr_t)state) & 15) == 0) {
     const dim3 wgrid((T + CONV_TOKENS - 1) / CONV_TOKENS, (C / 4 + 255) / 256);
 #define CONV_WALK(K_) delta_conv_walk_kernel<K_><<<wgrid, 256, 0, st>>>(y, x, ldx, taps, state, state_stride, tail_offset, token_seq, cu_q, positions, slots, T, C, bias)
