@@ -56,3 +56,33 @@ def test_capped_rows_agree_with_prompt_rows(LENGTHS, dtype, nq, nkv, d, P, windo
                   torch.cuda.current_stream().cuda_stream) == 0
     assert not torch.isnan(out[1]).any()
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("capped", [False, True])
+@pytest.mark.parametrize("nq,nkv,d", [(16, 8, 64), (8, 8, 128), (32, 16, 48)])
+def test_many_rows_of_two_segments_and_few(nq, nkv, d, capped, dtype):
+    """More workgroups than run at once are folded by a second launch, few fold themselves: the same bits."""
+    k, R, P = kern(dtype), 70, 64
+    p, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    assert R * nkv > 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    lengths = [1 + (37 * j) % 512 for j in range(R - 1)] + [512]
+    keys, values = ([rand((n, nkv, d), dtype, s + j) for j, n in enumerate(lengths)] for s in (40, 140))
+    kc, vc, table = (x.cuda() for x in build_cache(keys, values, P, sum(-(-n // P) for n in lengths) + 3, 3, dtype, float("nan")))
+    q = rand((R, nq, d), dtype, 10).cuda()
+    cu, k_len = torch.arange(R + 1, dtype=torch.int32, device="cuda"), torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    items = torch.stack([torch.arange(R), torch.zeros(R)], 1).to(torch.int32).cuda()
+    scratch = torch.full((k.attn_scratch_floats(R, nq, d, 2),), float("nan"), device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    fn = k.lib.vk_paged_attention_capped if capped else k.lib.vk_paged_attention
+    fn.argtypes = [p] * 5 + [i, p, p, p, i, i, i, p, i, i, i, i, i, i] + ([i, f, f, p, i, p] if capped else [f, p])
+    tail = (300, 16, d ** -0.5, 20.0, None, 0, stream) if capped else (0, d ** -0.5, stream)
+    outs = []
+    for n in (R, 7):
+        out = torch.full_like(q, float("nan"))
+        for at in range(0, R, n):
+            assert fn(out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], cu.data_ptr(), k_len.data_ptr(),
+                      items[at:].data_ptr(), n, 1, 2, scratch.data_ptr(), R, nq, nkv, d, P, *tail) == 0
+        outs.append(out)
+    assert not torch.isnan(outs[0]).any()
+    assert torch.equal(*outs)

@@ -1452,6 +1452,18 @@ int vk_attn_prefill_shares_tiles(int d, int P) {
   return (d == 64 || d == 128 || d == 256) && P >= TILE_KEYS && 4 * TILE_KEYS * d * (int)sizeof(elem_t) <= 128 * 1024;
 }
 
+// Whether decoded rows of no more than two segments (512 keys) are folded by the workgroups that compute them, without the second launch:
+// while the workgroups, eight waves each, all run at once, one a compute unit, or two with rows of 128 bytes.  A recorded step's
+// launch covers 512 keys whatever it holds, so that most requests have one segment in work; with both full a compute unit brings in
+// twice the keys.  Measured on MI355X in recorded launches, two launches against one, us, 16-bit elements, 8 kv heads of 128, scores capped (plain
+// attention: about 1 less, the same ratios): 1 row of 23 keys 7.8, 5.7, of 300 11.0, 10.2, of 512 11.1, 13.2; 24 rows of 300 12.9, 10.6; 32 rows of
+// 512 18.9, 16.7; 48 rows of 300 19.1, 20.5; 128 rows of 300 34.9, 41.6; 256 rows of 23 24.1, 35.3; heads of 64: 64 rows of 23 8.0, 6.3, of 512
+// 18.4, 16.4; 96 rows of 23 8.9, 9.1.
+static bool decode_folds_itself(int nseg, int d, int64_t workgroups) {
+  const size_t row = sizeof(elem_t) * vk_dpad(d);
+  return nseg <= 2 && row <= 256 && workgroups <= (row <= 128 ? 2 : 1) * (int64_t)attn_device_cus();
+}
+
 // items: n_items pairs (sequence, first row).
 // mode 0: each item is up to vk_attn_item_rows() consecutive rows of the sequence's q_len new tokens;
 //   the kernel is chosen by shape.  mode 2: the same through the kernel that takes every shape,
@@ -1571,10 +1583,7 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
     if (exact) attn_decode_quad_kernel<DP, true, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);        \
     else attn_decode_quad_kernel<DP, false, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);             \
   } while (0)
-    // No more than two segments (512 keys): without the second launch.  A recorded step's launch covers 512 keys whatever it holds, so
-    // that most requests this is for have one segment in work: 1 token of 23 keys 8.1 -> 5.1 us, 3 of 220 keys 10.5 -> 8.3, 8 of 300
-    // 10.2 -> 9.4; with both full a compute unit brings in twice the keys (5 of 400 10.5 -> 11.3, 1 of 500 10.6 -> 12.3).
-    if (nseg <= 2 && sizeof(elem_t) * vk_dpad(d) <= 256) {
+    if (decode_folds_itself(nseg, d, grid.x * (int64_t)grid.y)) {
 #ifdef VK_BF16
       if (d > 64) DECODE_BOTH(128);
       else
@@ -1718,7 +1727,7 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     else attn_decode_quad_kernel<DP, false, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);              \
   } while (0)
 #define DECODE_BOTH_EXT(DP) do { if (rel != nullptr) DECODE_BOTH_EXT_OF(DP, true); else DECODE_BOTH_EXT_OF(DP, false); } while (0)
-    if (nseg <= 2 && sizeof(elem_t) * vk_dpad(d) <= 256) {
+    if (decode_folds_itself(nseg, d, qgrid.x * (int64_t)qgrid.y)) {
 #ifdef VK_BF16
       if (d > 64) DECODE_BOTH_EXT(128);
       else
