@@ -86,3 +86,49 @@ def test_many_rows_of_two_segments_and_few(nq, nkv, d, capped, dtype):
         outs.append(out)
     assert not torch.isnan(outs[0]).any()
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("LENGTHS", [SHORT, LENGTHS, [1, 300, 1030, 2304, 2305, 2815, 3001]], ids=["short", "long", "longer"])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,window,keep,block", [("capped", 300, 0, 0), ("capped", 257, 16, 0), ("capped", 2, 600, 0), ("blocked", 0, 0, 200),
+                                                    ("blocked", 0, 0, 1024), ("biased", 0, 0, 0), ("biased", 300, 0, 0), ("biased", 513, 70, 0)])
+@pytest.mark.parametrize("nq,nkv,d,P", [(4, 2, 64, 64), (20, 1, 112, 8), (6, 1, 208, 128)])
+def test_the_variant_s_arguments(LENGTHS, nq, nkv, d, P, kind, window, keep, block, dtype):
+    """Windows, kept keys, blocks of positions, biases by distance and a gate a head: a decoded row against the same row as a prompt portion, for requests
+    of one segment, of several and of many more than a row sees."""
+    k = kern(dtype)
+    p, i, l, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
+    head = [p] * 5 + [i, p, p, p, i, i, i, p, i, i, i, i, i]
+    S = len(LENGTHS)
+    keys, values = ([rand((n, nkv, d), dtype, s + j) for j, n in enumerate(LENGTHS)] for s in (40, 70))
+    kc, vc, table = (x.cuda() for x in build_cache(keys, values, P, sum(-(-n // P) for n in LENGTHS) + 3, 3, dtype, float("nan")))
+    q, gate = rand((S, nq, d), dtype, 10).cuda(), rand((S, nq + 3), dtype, 11).cuda()
+    cu = torch.arange(S + 1, dtype=torch.int32, device="cuda")
+    k_len = torch.tensor(LENGTHS, dtype=torch.int32, device="cuda")
+    items = torch.stack([torch.arange(S), torch.zeros(S)], 1).to(torch.int32).cuda()
+    sinks = torch.linspace(-1, 1, nq, device="cuda")
+    pad, far = k.lib.vk_attn_rel_pad(), 100
+    line = rand((nq, far + 1), torch.float32, 12)                      # the distances far .. 0
+    rel = torch.cat([line[:, :1].expand(nq, pad), line, line[:, -1:].expand(nq, pad)], 1).contiguous().cuda()
+    nseg = -(-max(LENGTHS) // 256)
+    scratch = torch.full((k.attn_scratch_floats(S, nq, d, nseg),), float("nan"), device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    out = [torch.full_like(q, float("nan")) for _ in range(2)]
+    for mode in (0, 1):
+        args = (out[mode].data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], cu.data_ptr(), k_len.data_ptr(),
+                items.data_ptr(), S, mode, nseg, scratch.data_ptr(), S, nq, nkv, d, P)
+        if kind == "capped":
+            fn = k.lib.vk_paged_attention_capped
+            fn.argtypes = head + [i, i, f, f, p, i, p]
+            rc = fn(*args, window, keep, d ** -0.5, 20.0, sinks.data_ptr(), 1, stream)
+        elif kind == "blocked":
+            fn = k.lib.vk_paged_attention_blocked
+            fn.argtypes = head + [i, f, f, p, i, p]
+            rc = fn(*args, block, d ** -0.5, 20.0, sinks.data_ptr(), 1, stream)
+        else:
+            fn = k.lib.vk_paged_attention_biased
+            fn.argtypes = head + [i, i, f, p, i, p, i, i, p, l, p]
+            rc = fn(*args, window, keep, d ** -0.5, sinks.data_ptr(), 1, rel.data_ptr(), rel.shape[1], far, gate.data_ptr(), gate.shape[1], stream)
+        assert rc == 0
+    assert not torch.isnan(out[1]).any()
+    assert torch.equal(out[0], out[1])

@@ -73,6 +73,7 @@ struct AttnArgs {
   float scale = 0.f, softcap = 0.f;   // score = softcap * tanh(q.k * scale / softcap); softcap 0: score = q.k * scale
   const void* sinks = nullptr;        // [nq] or null: exp(sinks[head]) joins the softmax's denominator, with no value
   int sinks_f32 = 0;
+  int keep_segs = 0;      // decode, a launch over some of the segments: so many first ones, then those from a row's first visible key on
   int block = 0;          // > 0 (without a window): positions are cut into blocks of this size, and a row sees the keys of its own block only
   // A bias by distance on the scores (see "A bias by distance" below) and a gate on a head's output.
   const float* rel = nullptr;         // [nq, rel_stride] or null: head h's bias for the distance n is rel[h * rel_stride + rel_zero - n]
@@ -1163,10 +1164,13 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 // (a page that turns out not to be needed is read and not used), and the four tiles' scores are computed side by side.
 // SEGS 2: a workgroup of eight waves takes both segments of a launch that has no more than two, folds them as attn_combine_kernel
 // does and writes the output: a launch less, where a launch that waits for the one before is a third of the two.
-template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1>
+// FAR: the launch covers the kept segments and those that a window or a block can touch, not all before it.  (Known when the kernel is built:
+// the page numbers then wait for the lengths, 0.4 us of a short request's 12.)
+template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1, bool FAR = false>
 __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a) {
   static_assert(SEGS == 1 || sizeof(elem_t) * DPAD <= 256, "eight waves have 256 registers each");
   static_assert(EXT || !REL, "biases by distance belong to the variant");
+  static_assert(!FAR || (EXT && SEGS == 1), "so do launches over some of a request's segments");
   constexpr int NDT = DPAD / 16, NQS = DPAD / VK_SLAB, ND = NDT / SEG_TILES;   // ND: column blocks of a wave
   constexpr int NP = EXT ? P_PARTS : 1;                                        // numbers that a weight is split into
   __shared__ frag_t probs_of[SEGS][SEG_TILES][NP][KEY_SLABS][64];
@@ -1178,10 +1182,12 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   auto& tile_sum = tile_sum_of[my_seg];
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seg = blockIdx.z * SEGS + my_seg, first_tile = seg * SEG_TILES;
   const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
   const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
   const int k_len = a.k_len[seq];
+  int seg = blockIdx.z * SEGS + my_seg;
+  if (FAR && seg >= a.keep_segs) seg = max(first_visible(a, k_len - q_len + q_off) / (TILE_KEYS * SEG_TILES), a.keep_segs) + seg - a.keep_segs;
+  const int first_tile = seg * SEG_TILES;
   const int lp = __builtin_ctz(a.P);
   int page[SEG_TILES];                  // of the segment's tiles, where a tile lies in one page
 #pragma unroll
@@ -1715,12 +1721,19 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     // a segment, 16-bit elements, head size 128, 8 kv heads: 1 token of 500 keys 24.2 against 11.9 us; 8 of 300 19.3, 11.4; 8 of
     // 2,090 27.8, 15.7; 64 of 2,060 57.4, 53.3; 32-bit: 3 tokens of 220 keys 42.6, 16.8; 64 of 2,060 182, 164.
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
-    const dim3 qgrid(n_items, nkv * ((G + 15) / 16), nseg);
-#define DECODE_QUAD_EXT_OF(DP, REL)                                                                        \
-  do {                                                                                                     \
-    if (exact) attn_decode_quad_kernel<DP, true, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);          \
-    else attn_decode_quad_kernel<DP, false, true, REL><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);               \
+    // With a window or blocks a row sees few segments of a long request: the launch covers the kept ones and as many as so many keys can touch.
+    // 64 rows of 12,000 keys, 8 kv heads, windows of 1,024, 47 segments of which six are covered, a wave a segment (four a workgroup), four waves
+    // with all 47, with six: head size 128 82.6, 88.8, 69.7 us; 64 54.2, 63.2, 45.7.
+    const int64_t span = block > 0 ? block : window, kept = (keep + TILE_KEYS * SEG_TILES - 1LL) / (TILE_KEYS * SEG_TILES);
+    const int64_t seen = span > 0 ? kept + (span + TILE_KEYS * SEG_TILES - 2) / (TILE_KEYS * SEG_TILES) + 1 : nseg;
+    a.keep_segs = (int)std::min<int64_t>(kept, nseg);
+    const dim3 qgrid(n_items, nkv * ((G + 15) / 16), (unsigned)std::min<int64_t>(seen, nseg));
+#define DECODE_QUAD_EXT_FAR(DP, REL, FAR)                                                                       \
+  do {                                                                                                          \
+    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);       \
+    else attn_decode_quad_kernel<DP, false, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);            \
   } while (0)
+#define DECODE_QUAD_EXT_OF(DP, REL) do { if (seen < nseg) DECODE_QUAD_EXT_FAR(DP, REL, true); else DECODE_QUAD_EXT_FAR(DP, REL, false); } while (0)
 #define DECODE_BOTH_EXT_OF(DP, REL)                                                                                             \
   do {                                                                                                                         \
     if (exact) attn_decode_quad_kernel<DP, true, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);         \
@@ -1745,6 +1758,7 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
 #endif
 #undef DECODE_QUAD_EXT
 #undef DECODE_QUAD_EXT_OF
+#undef DECODE_QUAD_EXT_FAR
     if (vk_check_launch("attention (decoded rows, capped scores, four waves a segment)")) return 1;
     attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
     return vk_check_launch("attention (combine)");
