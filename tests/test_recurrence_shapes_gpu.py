@@ -257,3 +257,39 @@ def test_many_channels_at_once_and_few(K, with_bias, dtype):
             outs.append((y, after))
         assert not torch.isnan(outs[0][0]).any()
         assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K", [2, 4, 6])
+@pytest.mark.parametrize("lengths", [[0, 2], [2, 0, 1], [0, 0, 3], [1, 4, 0, 0, 0]])
+def test_the_short_convolution_of_uneven_steps(lengths, K, dtype):
+    """As many tokens as sequences, but not one each: the bits and tails of a call a sequence; a sequence without tokens keeps its tail."""
+    k, C = kern(dtype), 300
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    fn = k.lib.vk_delta_conv
+    fn.argtypes = [p, p, l, p, p, l, l, p, p, p, p, i, i, i, i, p]
+    g = torch.Generator().manual_seed(11)
+    S = len(lengths)
+    T = sum(lengths)
+    x, taps = torch.randn(T, C, generator=g).to(dtype).cuda(), (0.4 * torch.randn(C, K, generator=g)).to(dtype).cuda()
+    tails = torch.randn(S, (K - 1) * C, generator=g).cuda()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+
+    def step(a, counts, slots, state):
+        """The tokens from a on, as sequences of these lengths in these slots; every second slot's sequence starts here."""
+        cu, n = [0], sum(counts)
+        for c in counts:
+            cu.append(cu[-1] + c)
+        seq = [s for s, c in enumerate(counts) for _ in range(c)]
+        positions = [(5 if slots[s] % 2 else 0) + j for s, c in enumerate(counts) for j in range(c)]
+        y, keep = torch.full((n, C), float("nan"), device="cuda"), [x[a:a + n].contiguous(), i32(seq), i32(cu), i32(positions), i32(slots)]
+        assert fn(y.data_ptr(), keep[0].data_ptr(), C, taps.data_ptr(), state.data_ptr(), state.shape[1], 0, *(v.data_ptr() for v in keep[1:]), n, len(counts),
+                  C, K, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return y
+
+    state, want = tails.clone(), tails.clone()
+    y = step(0, lengths, list(range(S)), state)
+    at = [sum(lengths[:s]) for s in range(S)]
+    rows = torch.cat([step(at[s], [n], [s], want) for s, n in enumerate(lengths) if n])
+    assert torch.equal(y, rows) and torch.equal(state, want)

@@ -123,18 +123,21 @@ __global__ __launch_bounds__(256) void delta_conv_walk_kernel(float* __restrict_
   }
 }
 
-// A step of single tokens: the convolution and the tail that it moves on in one launch, a thread a channel.
+// A step of single tokens (as many tokens as sequences): the convolution and the tail that it moves on in one launch, a thread a channel.
+// A sequence's end is read beside its start: one without a token is left as it is, and the tokens of a longer one after its first are
+// walked on the tail in memory, in a loop that costs the others nothing.
 __global__ __launch_bounds__(256) void delta_conv_token_kernel(float* __restrict__ y, const elem_t* __restrict__ x, int64_t ldx,
                                                                const elem_t* __restrict__ taps, float* state, int64_t state_stride, int64_t tail_offset,
                                                                const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions,
                                                                const int32_t* __restrict__ slots, int C, int K, const elem_t* __restrict__ bias) {
   const int s = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
-  if (c >= C) return;
-  const int64_t t = cu_q[s];
+  const int64_t t = cu_q[s], end = cu_q[s + 1];
+  if (c >= C || t >= end) return;
   const bool fresh = positions[t] == 0;
   float* tail = state + (int64_t)slots[s] * state_stride + tail_offset + c;
   const float now = to_f32(x[t * ldx + c]);
-  float acc = bias != nullptr ? to_f32(bias[c]) : 0.f;
+  const float from = bias != nullptr ? to_f32(bias[c]) : 0.f;
+  float acc = from;
   float keep[DELTA_MAX_TAPS];
 #pragma unroll
   for (int j = 0; j < DELTA_MAX_TAPS; ++j) keep[j] = j < K - 1 && !fresh ? tail[(int64_t)j * C] : 0.f;
@@ -146,6 +149,17 @@ __global__ __launch_bounds__(256) void delta_conv_token_kernel(float* __restrict
 #pragma unroll
   for (int j = 0; j < DELTA_MAX_TAPS; ++j)
     if (j < K - 1) tail[(int64_t)j * C] = j == K - 2 ? now : keep[j + 1 < DELTA_MAX_TAPS ? j + 1 : j];
+#pragma unroll 1
+  for (int64_t u = t + 1; u < end; ++u) {
+    const float in = to_f32(x[u * ldx + c]);
+    float sum = from;
+#pragma unroll 1
+    for (int j = 0; j < K - 1; ++j) {
+      sum = sum + to_f32(taps[(int64_t)c * K + j]) * tail[(int64_t)j * C];
+      tail[(int64_t)j * C] = j == K - 2 ? in : tail[(int64_t)(j + 1) * C];
+    }
+    y[u * C + c] = silu_f(sum + to_f32(taps[(int64_t)c * K + K - 1]) * in);
+  }
 }
 
 // The tail after the step: the last K - 1 inputs of the sequence, oldest first.
@@ -155,6 +169,7 @@ __global__ __launch_bounds__(256) void delta_conv_tail_kernel(const elem_t* __re
                                                               const int32_t* __restrict__ slots, int C, int K) {
   const int s = blockIdx.x;
   const int first = cu_q[s], n = cu_q[s + 1] - first;
+  if (n <= 0) return;
   const bool fresh = positions[first] == 0;
   float* tail = state + (int64_t)slots[s] * state_stride + tail_offset;
   for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < C; c += gridDim.y * blockDim.x) {
@@ -754,7 +769,7 @@ int vk_delta_lanes_per_column(int d) {
 }
 
 // y [T, C] floats from the columns x[:, 0:C] of rows of length ldx; then the tails are moved on.  bias: [C] or null, what
-// every channel's sum starts from.  T: the step's tokens, at least one a sequence.
+// every channel's sum starts from.  T: the step's tokens.
 static int conv_launch(float* y, const elem_t* x, int64_t ldx, const elem_t* taps, const elem_t* bias, float* state, int64_t state_stride,
                        int64_t tail_offset, const int32_t* token_seq, const int32_t* cu_q, const int32_t* positions, const int32_t* slots, int T,
                        int S, int C, int K, hipStream_t st) {
@@ -764,7 +779,7 @@ static int conv_launch(float* y, const elem_t* x, int64_t ldx, const elem_t* tap
   if (T == 0 || S == 0) return 0;
   // Groups of channels: more than a grid has room for are left to the kernel for every shape, whose workgroups walk them.
   const int groups = (C + 255) / 256;
-  if (T == S && groups <= 65535) {                 // every sequence brings one token
+  if (T == S && groups <= 65535) {                 // a step of single tokens
     delta_conv_token_kernel<<<dim3(S, groups), 256, 0, st>>>(y, x, ldx, taps, state, state_stride, tail_offset, cu_q, positions, slots, C, K, bias);
     return vk_check_launch("short convolution (single tokens)");
   }
