@@ -96,6 +96,17 @@ def test_the_same_bits_as_the_walk_for_every_shape(kind, d, dtype):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kind", ["delta", "gla", "linear"])
+def test_uneven_steps_of_as_many_tokens_as_sequences(kind, d, dtype):
+    """Not one token each: the bits of the walk for every shape, and the states of sequences without a token as they were."""
+    for lengths in ([0, 2], [2, 0, 1], [0, 0, 3], [0, 1, 3, 0, 1]):
+        got, want = (run(kern(dtype), kind, d, 4, lengths, False, odd, dtype) for odd in (False, True))
+        assert not torch.isnan(got[0]).any()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def run_scan(k, heads, P, lengths, fresh, odd):
     """The state-space scan with 128 state rows over sequences of these lengths; odd: rows one number longer."""
     g = torch.Generator().manual_seed(4)

@@ -626,7 +626,8 @@ __global__ __launch_bounds__(RULE_THREADS, 2) void rule_walk_kernel(float* __res
 
 // The same for a step of single tokens: no LDS, a lane holds four channels of four columns, and states, q, k and decays are asked for
 // together.  What bounds it is the states' way in and out; the walk's workgroups, with LDS for chunks of tokens, did not all fit the
-// device at once.  8 tokens x 32 heads of 128 x 128 (33.5 MB): 18.6 -> 6.2 us.
+// device at once.  8 tokens x 32 heads of 128 x 128 (33.5 MB): 18.6 -> 6.2 us.  (It is chosen by as many tokens as sequences: one without a
+// token keeps its state, one with several walks them.)
 template <int D, bool DELTA, typename IN, bool HEAD_DECAY>
 __global__ __launch_bounds__(RULE_THREADS) void rule_token_kernel(float* __restrict__ out, const IN* __restrict__ qkv, int64_t ld, int q_col, int k_col,
                                                                   int v_col, const float* __restrict__ decay, const elem_t* __restrict__ b, int64_t ldb,
@@ -638,51 +639,56 @@ __global__ __launch_bounds__(RULE_THREADS) void rule_token_kernel(float* __restr
   const int r = lane % LANES, col = blockIdx.z * CB + (wave * (64 / LANES) + lane / LANES) * CC;
   if (col >= dv) return;                            // columns are whole groups of four; no barrier follows
   const int g = h / (H / G);
-  const int64_t t = cu_q[s];
-  const bool fresh = positions[t] == 0;
+  const int64_t first = cu_q[s], end = cu_q[s + 1];
+  if (first >= end) return;
   float* S_mem = state + (int64_t)slots[s] * state_stride + ((int64_t)h * dv + col) * D + r * 4;
-  f32x4 S[CC];
+  auto token = [&](int64_t t, bool fresh) {
+    f32x4 S[CC];
 #pragma unroll
-  for (int j = 0; j < CC; ++j) S[j] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(S_mem + (int64_t)j * D);
-  const IN* row = qkv + t * ld;
-  float k4[4], q4[4], g4[4], v[CC], o[CC];
-  load_row<4>(row + k_col + (int64_t)g * D + r * 4, k4);
-  load_row<4>(row + q_col + (int64_t)g * D + r * 4, q4);
-  if (HEAD_DECAY) {
-    const float head_g = decay[h];
+    for (int j = 0; j < CC; ++j) S[j] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(S_mem + (int64_t)j * D);
+    const IN* row = qkv + t * ld;
+    float k4[4], q4[4], g4[4], v[CC], o[CC];
+    load_row<4>(row + k_col + (int64_t)g * D + r * 4, k4);
+    load_row<4>(row + q_col + (int64_t)g * D + r * 4, q4);
+    if (HEAD_DECAY) {
+      const float head_g = decay[h];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) g4[i] = head_g;
-  } else {
-    load_row<4>(decay + (t * H + h) * D + r * 4, g4);
-  }
-#pragma unroll
-  for (int j = 0; j < CC; ++j) v[j] = to_f32(row[v_col + (int64_t)h * dv + col + j]);
-  const float beta = DELTA ? sigmoid_f(to_f32(b[t * ldb + h])) : 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) q4[i] = DELTA ? q4[i] : q4[i] * q_scale;
-#pragma unroll
-  for (int j = 0; j < CC; ++j) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S[j][i] = S[j][i] * g4[i];
-    if (DELTA) {
-      float dot = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(S[j][i], k4[i], dot);
-      v[j] = beta * (v[j] - group_sum<LANES>(dot));
+      for (int i = 0; i < 4; ++i) g4[i] = head_g;
+    } else {
+      load_row<4>(decay + (t * H + h) * D + r * 4, g4);
     }
-    o[j] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      S[j][i] = __builtin_fmaf(k4[i], v[j], S[j][i]);
-      o[j] = __builtin_fmaf(S[j][i], q4[i], o[j]);
+    for (int j = 0; j < CC; ++j) v[j] = to_f32(row[v_col + (int64_t)h * dv + col + j]);
+    const float beta = DELTA ? sigmoid_f(to_f32(b[t * ldb + h])) : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q4[i] = DELTA ? q4[i] : q4[i] * q_scale;
+#pragma unroll
+    for (int j = 0; j < CC; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[j][i] = S[j][i] * g4[i];
+      if (DELTA) {
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dot = __builtin_fmaf(S[j][i], k4[i], dot);
+        v[j] = beta * (v[j] - group_sum<LANES>(dot));
+      }
+      o[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        S[j][i] = __builtin_fmaf(k4[i], v[j], S[j][i]);
+        o[j] = __builtin_fmaf(S[j][i], q4[i], o[j]);
+      }
+      *reinterpret_cast<f32x4*>(S_mem + (int64_t)j * D) = S[j];
+      o[j] = group_sum<LANES>(o[j]);
     }
-    *reinterpret_cast<f32x4*>(S_mem + (int64_t)j * D) = S[j];
-    o[j] = group_sum<LANES>(o[j]);
-  }
-  if (r == 0) {
+    if (r == 0) {
 #pragma unroll
-    for (int j = 0; j < CC; ++j) out[(t * H + h) * dv + col + j] = o[j];
-  }
+      for (int j = 0; j < CC; ++j) out[(t * H + h) * dv + col + j] = o[j];
+    }
+  };
+  token(first, positions[first] == 0);
+#pragma unroll 1
+  for (int64_t t = first + 1; t < end; ++t) token(t, false);
 }
 
 // y[t, h, :] = o / sqrt(mean(o^2) + eps) * w * sigmoid(gate[t, h, :]) (gate_kind 1: * silu(gate[t, h, :])), stored as elements in rows of length ldy; the
@@ -860,7 +866,7 @@ static int rule_cus() {
 
 // out [T, H, dv] floats.  qkv: float rows of length ld with q (G heads of d) at q_col, k at k_col, v (H heads of dv) at
 // v_col; decay [T, H, d] floats; b: elements, beta's pre-activation of head h at b[t * ldb + h].  state: per slot,
-// the H states at its start, each [dv][d].  T: the step's tokens, at least one a sequence.
+// the H states at its start, each [dv][d].  T: the step's tokens.
 extern "C++" {
 template <bool DELTA, typename IN, bool HEAD_DECAY = false>
 static int rule_launch(float* out, const IN* qkv, int64_t ld, int q_col, int k_col, int v_col, const float* decay, const elem_t* b, int64_t ldb,
