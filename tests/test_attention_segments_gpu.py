@@ -132,3 +132,37 @@ def test_the_variant_s_arguments(LENGTHS, nq, nkv, d, P, kind, window, keep, blo
         assert rc == 0
     assert not torch.isnan(out[1]).any()
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("capped", [False, True])
+@pytest.mark.parametrize("R,n", [(20, 1000), (70, 1700)])
+@pytest.mark.parametrize("nq,nkv,d", [(16, 8, 80), (8, 8, 128), (8, 8, 160), (16, 8, 256)])
+def test_many_segments_and_few(nq, nkv, d, R, n, capped, dtype):
+    """The number of segments of a launch chooses its kernel: all rows at once and few at a time give the same bits."""
+    k, P, nseg = kern(dtype), 64, -(-n // 256)
+    p, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    lengths = [1 + (337 * j) % n for j in range(R - 1)] + [n]
+    g = torch.Generator(device="cuda").manual_seed(1)
+    pages = [-(-m // P) for m in lengths]
+    kc, vc = (torch.randn(sum(pages), nkv, P, d, device="cuda", generator=g).to(dtype) for _ in range(2))
+    table = torch.zeros(R, max(pages), dtype=torch.int32, device="cuda")
+    order = torch.randperm(sum(pages), device="cuda", generator=g).to(torch.int32)
+    for r in range(R):
+        table[r, :pages[r]] = order[sum(pages[:r]):sum(pages[:r + 1])]
+    q = torch.randn(R, nq, d, device="cuda", generator=g).to(dtype)
+    cu, k_len = torch.arange(R + 1, dtype=torch.int32, device="cuda"), torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    items = torch.stack([torch.arange(R), torch.zeros(R)], 1).to(torch.int32).cuda()
+    scratch = torch.full((k.attn_scratch_floats(R, nq, d, nseg),), float("nan"), device="cuda")
+    fn = k.lib.vk_paged_attention_capped if capped else k.lib.vk_paged_attention
+    fn.argtypes = [p] * 5 + [i, p, p, p, i, i, i, p, i, i, i, i, i, i] + ([i, f, f, p, i, p] if capped else [f, p])
+    tail = (0, 0, d ** -0.5, 20.0, None, 0) if capped else (0, d ** -0.5)
+    outs = []
+    for few in (R, 3):
+        out = torch.full_like(q, float("nan"))
+        for at in range(0, R, few):
+            assert fn(out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], cu.data_ptr(), k_len.data_ptr(),
+                      items[at:].data_ptr(), min(few, R - at), 1, nseg, scratch.data_ptr(), R, nq, nkv, d, P, *tail, torch.cuda.current_stream().cuda_stream) == 0
+        outs.append(out)
+    assert not torch.isnan(outs[0]).any()
+    assert torch.equal(*outs)

@@ -1575,8 +1575,14 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   // 530, 192: 12.1, 10.4; 8 of 1,030, 320: 14.2, 12.6; 8 of 2,090, 576: 21.0, 19.3; 24 of 2,048, 1,536: 35.8, 36.3; head size 64,
   // 1,536: 16.7, 18.0; 32-bit, head size 128: 3 tokens of 220 keys 43.5, 17.2; 64 of 530, 1,536: 99.7, 78.6; 64 of 2,060, 4,608:
   // 258, 276.  (32-bit with wider heads: four tiles' fragments do not fit the registers.)
+  // With padded rows of 512 bytes a workgroup, one a compute unit, takes as long as with whole ones, and the other kernel does not: two rounds of
+  // them, or three in 32 bits with more than 80 entries (the other, four waves: 576 segments of about 256 keys and heads of 160 32.4, 40.3 us, of 192
+  // 38.9, 44.4, of 256 48.5, 41.4; 512 of 160 33.7, 30.2; 32-bit, 1,024 of 80 52.6, 65.7, of 96 59.8, 71.4; 768 of 80 46.6, 49.3, of 96 49.2, 51.2 at
+  // the most and 1.1 times the other way on the mean; 512 of 80 1.2 times the other way).
   const bool quad_fits = sizeof(elem_t) * vk_dpad(d) <= 512;
-  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = (seg_fits || sizeof(elem_t) == 2 ? 5 : 12) * (int64_t)attn_device_cus() / 2;
+  const bool padded = !seg_fits && d < vk_dpad(d);
+  const int half_rounds = padded ? (sizeof(elem_t) == 2 || d <= 80 ? 4 : 6) : (sizeof(elem_t) == 2 || seg_fits ? 5 : 12);
+  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = half_rounds * (int64_t)attn_device_cus() / 2;
   if (quad_fits && (vk_decode_variant == 4 || (vk_decode_variant == 0 && segments <= quad_most))) {
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
 #define DECODE_QUAD(DP)                                                                               \
