@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(256) void attn_prefill_ext_kernel(AttnArgs a, int h
 }
 
 // Decoded tokens: attn_decode_plain_kernel with the things above, for heads whose four tiles no workgroup's registers hold
-// (32-bit, wider than 128); attn_combine_kernel folds its segments.
+// (32-bit, wider than 128) and for many segments of those that hold them one workgroup a compute unit; attn_combine_kernel folds its segments.
 #ifndef VK_BF16
 template <int DPAD, bool V_LATE, bool REL>
 __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnArgs a) {
@@ -1721,17 +1721,24 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
   a.part_ml = scratch;
   a.part_acc = scratch + (((int64_t)n_items * nq * nseg * 2 + 3) & ~(int64_t)3);
   VK_REQUIRE(nkv * ((G + 15) / 16) <= 65535 && nq <= 65535, "attention: too many heads");
-  if (sizeof(elem_t) * vk_dpad(d) <= 512) {
-    // Four waves a segment whatever the number of segments: a tile costs the variant three products a slab and the cap's exponentials,
+  const size_t row = sizeof(elem_t) * vk_dpad(d);
+  const int64_t span = block > 0 ? block : window, kept = (keep + TILE_KEYS * SEG_TILES - 1LL) / (TILE_KEYS * SEG_TILES);
+  const int64_t seen = span > 0 ? kept + (span + TILE_KEYS * SEG_TILES - 2) / (TILE_KEYS * SEG_TILES) + 1 : nseg;
+  // 32-bit rows of 512 bytes (see below): six workgroups a compute unit, three if the rows are padded, where a launch covers every segment.
+  const bool many = sizeof(elem_t) == 4 && row == 512 && seen >= nseg &&
+                    (int64_t)n_items * (nkv * ((G + 15) / 16)) * nseg > (d == vk_dpad(d) ? 6 : 3) * (int64_t)attn_device_cus();
+  if (row <= 512 && !many) {
+    // Four waves a segment, whatever the number of segments in 16 bits: a tile costs the variant three products a slab and the cap's exponentials,
     // so that a wave a segment was a chain of arithmetic too.  Measured on MI355X with the fold, windows of 1,024, a wave against four
     // a segment, 16-bit elements, head size 128, 8 kv heads: 1 token of 500 keys 24.2 against 11.9 us; 8 of 300 19.3, 11.4; 8 of
     // 2,090 27.8, 15.7; 64 of 2,060 57.4, 53.3; 32-bit: 3 tokens of 220 keys 42.6, 16.8; 64 of 2,060 182, 164.
+    // 32-bit rows of 512 bytes leave one workgroup a compute unit, which in the long run is slower than the kernel that asks for a tile when it needs it:
+    // without a window, 1,536 segments with heads of 128 1.1 times as fast as that one, 2,048 of 8,000 keys 120 against 139 us, 6,144 322, 360; heads
+    // of 96, 768 1.2 times as fast, 1,024 59.8, 66.4, 3,072 136, 183; heads of 80 the same ratios.
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
     // With a window or blocks a row sees few segments of a long request: the launch covers the kept ones and as many as so many keys can touch.
     // 64 rows of 12,000 keys, 8 kv heads, windows of 1,024, 47 segments of which six are covered, a wave a segment (four a workgroup), four waves
     // with all 47, with six: head size 128 82.6, 88.8, 69.7 us; 64 54.2, 63.2, 45.7.
-    const int64_t span = block > 0 ? block : window, kept = (keep + TILE_KEYS * SEG_TILES - 1LL) / (TILE_KEYS * SEG_TILES);
-    const int64_t seen = span > 0 ? kept + (span + TILE_KEYS * SEG_TILES - 2) / (TILE_KEYS * SEG_TILES) + 1 : nseg;
     a.keep_segs = (int)std::min<int64_t>(kept, nseg);
     const dim3 qgrid(n_items, nkv * ((G + 15) / 16), (unsigned)std::min<int64_t>(seen, nseg));
 #define DECODE_QUAD_EXT_FAR(DP, REL, FAR)                                                                       \
@@ -1774,14 +1781,16 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
 #else
   const dim3 grid(n_items, nkv * ((G + 15) / 16), (nseg + PLAIN_WAVES - 1) / PLAIN_WAVES);
   const bool late = (int64_t)grid.x * grid.y * nseg > 1024;
-#define DECODE_EXT(REL)                                                                        \
-  do {                                                                                         \
-    if (late) attn_decode_ext_kernel<256, true, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);    \
-    else attn_decode_ext_kernel<256, false, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);        \
+#define DECODE_EXT_OF(DP, REL)                                                                \
+  do {                                                                                        \
+    if (late) attn_decode_ext_kernel<DP, true, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);    \
+    else attn_decode_ext_kernel<DP, false, REL><<<grid, 64 * PLAIN_WAVES, 0, st>>>(a);        \
   } while (0)
-  if (rel != nullptr) DECODE_EXT(true);
-  else DECODE_EXT(false);
+#define DECODE_EXT(DP) do { if (rel != nullptr) DECODE_EXT_OF(DP, true); else DECODE_EXT_OF(DP, false); } while (0)
+  if (d <= 128) DECODE_EXT(128);          // (64 and less went the way above)
+  else DECODE_EXT(256);
 #undef DECODE_EXT
+#undef DECODE_EXT_OF
   if (vk_check_launch("attention (decoded rows, capped scores)")) return 1;
   attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
   return vk_check_launch("attention (combine)");
