@@ -58,7 +58,7 @@ def test_turned_heads_of_many_tokens(d, rot_half, norm_d, neighbours, dtype):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,groups,keep,kind", [(1, 1, 1, 1, 0), (32, 4, 1, 1, 0), (32, 3, 8, 3, 1), (64, 6, 1, 1, 2), (65, 2, 1, 1, 0), (70, 5, 7, 2, 1)])
 def test_routers_of_few_and_many_tokens(E, top, groups, keep, kind, dtype):
-    """Choice and plan in one launch (up to 32 tokens) and in two, an expert a workgroup and four (from 256 tokens on); up to 64 experts
+    """Choice and plan in one launch (up to 12 or 16 tokens) and in two, an expert a workgroup and four (many tokens and experts); up to 64 experts
     and more.  Every plan is checked: each pair once, in a tile of its expert."""
     k, W = kern(dtype), 224
     h, router = rand((300, W), dtype, 1).cuda(), rand((E, W), dtype, 2, 0.1).cuda()
@@ -91,3 +91,33 @@ def test_routers_of_few_and_many_tokens(E, top, groups, keep, kind, dtype):
             padded = -(-counts // tile_rows) * tile_rows
             assert start.tolist() == [0] + padded.cumsum(0).tolist()
             assert (expert[start[-1] // tile_rows:] == -1).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E,top,kind", [(32, 4, 0), (32, 5, 1), (64, 1, 0), (64, 8, 2), (72, 4, 0)])
+def test_routers_on_both_sides_of_their_lines(E, top, kind, dtype):
+    """Choice and plan in one launch or two, one expert a workgroup or four: the choices, weights and logits of a token are the same bits beside any number of
+    others, and every plan holds each pair once, in a tile of its expert."""
+    k, W = kern(dtype), 224
+    many = 600
+    h, router = rand((many, W), dtype, 1).cuda(), rand((E, W), dtype, 2, 0.1).cuda()
+    fn, most = k.lib.vk_moe_route_plan, k.lib.vk_moe_max_tiles
+    fn.argtypes = [P, P, P, P, P, P, I, P, I, I, I, I, I, F, I, I, I, I, F, P, P, P, P, P, I, P]
+    most.argtypes = [I, I, I, I]
+    whole = None
+    for T in (many, 513, 512, 505, 257, 249, 17, 16, 13, 12, 2):
+        tiles = most(T, top, E, 16)
+        new = lambda *n: torch.full(n, -7, dtype=torch.int32, device="cuda")
+        idx, pair, token, pair_row, expert, start = new(T, top), new(tiles * 16), new(tiles * 16), new(T * top), new(tiles), new(E + 1)
+        wts, logits = torch.zeros(T, top, device="cuda"), torch.zeros(T, E, device="cuda")
+        assert fn(at(idx), at(wts), at(logits), at(h), at(router), None, 0, None, 0, T, W, E, top, 1e-6, kind, 1, 1, 0, 1.0, at(pair), at(token), at(pair_row),
+                  at(expert), at(start), 16, torch.cuda.current_stream().cuda_stream) == 0
+        if whole is None:
+            whole = idx, wts, logits
+        for part, all_of_it in zip((idx, wts, logits), whole):
+            assert torch.equal(part, all_of_it[:T])
+        idx, pair, token, pair_row, expert = (v.cpu() for v in (idx.flatten(), pair, token, pair_row, expert))
+        rows = torch.nonzero(pair >= 0).flatten()
+        assert sorted(pair[rows].tolist()) == list(range(T * top))
+        assert torch.equal(pair_row[pair[rows].long()].long(), rows) and torch.equal(token[rows], pair[rows] // top)
+        assert torch.equal(expert[rows // 16], idx[pair[rows].long()])

@@ -25,7 +25,7 @@
 // order depends on the width alone.
 // bias: one number an expert that is added to its logit (elements or floats), or null.
 // EX: experts of a workgroup, one after the other on the rows it holds: with one every expert's workgroup reads a group's rows again from
-// the second-level cache, which a prompt's 32 experts wait for (2,048 tokens of 4,096 entries: 37 us, with four 24); few tokens want the workgroups.
+// the second-level cache, which a prompt's 32 experts wait for (2,048 tokens of 4,096 entries: 37 us, with four 24); fewer tokens want the workgroups (route_launch).
 template <int EX>
 __global__ __launch_bounds__(256) void moe_logits_kernel(float* __restrict__ z, const elem_t* __restrict__ h, const elem_t* __restrict__ router,
                                                          int T, int W, int E, const void* __restrict__ bias, int bias_is_f32) {
@@ -269,16 +269,15 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(MoePlanArgs a) {
   moe_make_plan(a, plan);
 }
 
-// The choice and the plan of a few tokens in one launch, a wave a token after the other: two launches that wait for each other took 11 to
-// 15 us for some hundred numbers.
-#define MOE_FEW_TOKENS 32
+// The choice and the plan of a few tokens in one launch, a wave a token: two launches that wait for each other took 11 to 15 us for some
+// hundred numbers.  The waves share one compute unit, where a choice is a chain of searches: router and plan of 64 experts in one launch
+// against two, us: one choice, 16 tokens 8.5, 9.1; four, 12 tokens 10.1, 10.8, 16 11.0, 10.8; eight, 12 tokens 12.9, 13.0, 16 14.2, 13.0; beyond 16,
+// with a second token a wave, 24 tokens of four 12.9, 10.8, 32 of eight 21.5, 13.0.
+#define MOE_FEW_TOKENS(top) ((top) <= 4 ? 16 : 12)
 __global__ __launch_bounds__(1024) void moe_choose_plan_kernel(MoeChoice c, MoePlanArgs p) {
   extern __shared__ float scores[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int t = wave; t < c.T; t += 16) {
-    moe_choose_token(c, scores, t, wave, 16, lane);
-    wave_lds_fence();
-  }
+  if (wave < c.T) moe_choose_token(c, scores, wave, wave, 16, lane);
   __syncthreads();                // every choice is made and, through this compute unit's cache, to be read by all its waves
   moe_make_plan(p, reinterpret_cast<int32_t*>(scores));
 }
@@ -562,6 +561,17 @@ int vk_moe_max_tiles(int T, int top, int E, int tile_rows) {
   return (int)((pairs + busy * (tile_rows - 1)) / tile_rows);
 }
 
+static int moe_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    cus = n > 0 ? n : 256;
+  }
+  return cus;
+}
+
 // logits: scratch [T, E] floats.  bias [E] (elements, or floats with bias_is_f32) or null.
 static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32, int T, int W,
                         int E, int top, float weight_eps, hipStream_t st, int score_kind = 0, int groups = 1, int keep = 1, float scale = 1.f, int group_score = 0,
@@ -576,13 +586,16 @@ static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h
   // whose cache then holds its rows.
   const int groups_of_tokens = (T + MOE_ROUTE_TOKENS - 1) / MOE_ROUTE_TOKENS;
   const int grid_x = groups_of_tokens > 8 ? (groups_of_tokens + 7) / 8 * 8 : groups_of_tokens;
-  if (E % 4 == 0 && T >= 256) moe_logits_kernel<4><<<dim3(grid_x, E / 4), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
+  // Four experts a workgroup from eight workgroups a compute unit on, with one each: that is where a group's rows, read again, become the longer
+  // wait (one against four, with choice and plan: 256 tokens of 4,096 entries, 8 experts 10.7, 13.5 us; 32 experts, 255 and 256 tokens of
+  // 4,096 11.5, 13.9, 512 15.0, 14.8; 64 experts, 256 tokens of 2,048 11.7, 12.3, 2,048 of them 46, 28).
+  if (E % 4 == 0 && (int64_t)groups_of_tokens * E >= 8 * (int64_t)moe_cus()) moe_logits_kernel<4><<<dim3(grid_x, E / 4), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
   else moe_logits_kernel<1><<<dim3(grid_x, E), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
   if (vk_check_launch("router (logits)")) return 1;
   const MoeChoice c = {idx, wts, logits, T, E, top, weight_eps, score_kind, groups, keep, scale, group_score, correction, correction_is_f32};
   const size_t a_wave = ((correction != nullptr ? 2 : 1) * (size_t)E + (keep < groups ? groups : 0)) * sizeof(float);
   VK_REQUIRE(4 * a_wave <= 65536, "router: %d experts in %d groups are too many", E, groups);
-  if (plan != nullptr && T <= MOE_FEW_TOKENS && 16 * a_wave <= 65536) {
+  if (plan != nullptr && T <= MOE_FEW_TOKENS(top) && 16 * a_wave <= 65536) {
     moe_choose_plan_kernel<<<1, 1024, std::max(16 * a_wave, (size_t)2 * E * sizeof(int32_t)), st>>>(c, *plan);
     return vk_check_launch("router (choice and plan)");
   }
@@ -610,17 +623,6 @@ int vk_moe_route_plan(int32_t* idx, float* wts, float* logits, const elem_t* h, 
   const MoePlanArgs plan = {idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E, vk_moe_max_tiles(T, top, E, tile_rows), tile_rows};
   return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale, group_score, correction,
                       correction_is_f32, &plan);
-}
-
-static int moe_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
 }
 
 // An expert product of rows in tiles of 16: by the streaming kernel where it takes the sizes, else by the one for every K.
