@@ -39,8 +39,7 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(float* __restrict__ z, 
 #pragma unroll
     for (int i = 0; i < MOE_ROUTE_TOKENS; ++i) acc[x][i] = 0.f;
   const elem_t* wr = router + (int64_t)e0 * W;
-#pragma unroll EX == 1 ? 2 : 1
-  for (int c = threadIdx.x * VK_VEC; c < W; c += 256 * VK_VEC) {
+  auto step = [&](int c) {
     float wv[EX][VK_VEC];
 #pragma unroll
     for (int x = 0; x < EX; ++x) load_elems(wr + (int64_t)x * W + c, wv[x]);
@@ -53,6 +52,13 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(float* __restrict__ z, 
 #pragma unroll
         for (int j = 0; j < VK_VEC; ++j) acc[x][i] = __builtin_fmaf(hv[j], wv[x][j], acc[x][i]);
     }
+  };
+  if constexpr (EX == 1) {
+#pragma unroll 2
+    for (int c = threadIdx.x * VK_VEC; c < W; c += 256 * VK_VEC) step(c);
+  } else {
+#pragma unroll 1
+    for (int c = threadIdx.x * VK_VEC; c < W; c += 256 * VK_VEC) step(c);
   }
 #pragma unroll
   for (int x = 0; x < EX; ++x)
