@@ -228,8 +228,9 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(float* x, int64_t ld, i
                                                          float q_scale, float* __restrict__ g, const elem_t* __restrict__ a,
                                                          const void* __restrict__ dt_bias, const void* __restrict__ A_log, int w_is_f32, int T) {
   const int per = 2 * G + H, lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int t = (int)(item / per), j = (int)(item - (int64_t)t * per);
+  // (A wave's own numbers, known to be: the division and the rows' addresses are scalar.)
+  const unsigned item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = (int)(item / (unsigned)per), j = (int)(item - (unsigned)t * (unsigned)per);
   if (t >= T) return;                             // the whole wave; no barrier follows
   if (j < 2 * G) {
     const bool is_q = j < G;
@@ -697,8 +698,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(elem_t* __restrict__ y, 
                                                         const elem_t* __restrict__ gate, int64_t ldg, const void* __restrict__ w, int w_is_f32,
                                                         int H, int dv, float eps, int gate_kind, int T) {
   const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int t = (int)(item / H), h = (int)(item - (int64_t)t * H);
+  const unsigned item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (as delta_prep_kernel)
+  const int t = (int)(item / (unsigned)H), h = (int)(item - (unsigned)t * (unsigned)H);
   if (t >= T) return;                             // the whole wave; no barrier follows
   const float* row = o + ((int64_t)t * H + h) * dv;
   float part = 0.f;
