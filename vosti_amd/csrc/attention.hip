@@ -33,8 +33,8 @@
 //   attn_decode_seg    decoded tokens: a wave walks the tiles of a segment with the next tile's
 //                      fragments in flight; the segment's (M, L, ACC) goes to a scratch buffer ...
 //   attn_combine       ... which this one folds.
-//   attn_decode_quad   the same with four waves a segment, one tile's scores each: for steps with few segments, and for
-//                      every step of the variant with capped scores.
+//   attn_decode_quad   the same with four waves a segment, one tile's scores each: for steps with few segments, and for the variant
+//                      with capped scores (in 32 bits: heads of up to 64, and few segments of heads of up to 128).
 //   attn_decode_plain  the same with a tile's fragments asked for when they are needed: for head and
 //                      element sizes whose fragments of two tiles do not fit a wave's registers.
 //
@@ -1442,17 +1442,6 @@ int vk_attn_item_rows(void) { return ITEM_ROWS; }
 
 static int vk_dpad(int d) { return d <= 64 ? 64 : (d <= 128 ? 128 : 256); }
 
-static int attn_device_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus <= 0) cus = 256;
-  }
-  return cus;
-}
-
 // 1 if prompt rows of this shape go through the kernel that shares key tiles in LDS.
 int vk_attn_prefill_shares_tiles(int d, int P) {
   return (d == 64 || d == 128 || d == 256) && P >= TILE_KEYS && 4 * TILE_KEYS * d * (int)sizeof(elem_t) <= 128 * 1024;
@@ -1467,7 +1456,7 @@ int vk_attn_prefill_shares_tiles(int d, int P) {
 // 18.4, 16.4; 96 rows of 23 8.9, 9.1.
 static bool decode_folds_itself(int nseg, int d, int64_t workgroups) {
   const size_t row = sizeof(elem_t) * vk_dpad(d);
-  return nseg <= 2 && row <= 256 && workgroups <= (row <= 128 ? 2 : 1) * (int64_t)attn_device_cus();
+  return nseg <= 2 && row <= 256 && workgroups <= (row <= 128 ? 2 : 1) * (int64_t)vk_device_cus();
 }
 
 // items: n_items pairs (sequence, first row).
@@ -1531,13 +1520,13 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
     // 83 -> 74; from two workgroups per unit on eight waves win by 2 to 8 %).  Two row tiles per wave would
     // halve the LDS traffic but need more than the 256 registers that two waves per SIMD leave: with spills
     // or with one wave per SIMD they measured 40 % slower.
-    const int v = (vk_prefill_variant == 14 || (vk_prefill_variant == 0 && 2 * (int64_t)n_items * nq < 3 * (int64_t)attn_device_cus())) ? 14 : 0;
+    const int v = (vk_prefill_variant == 14 || (vk_prefill_variant == 0 && 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus())) ? 14 : 0;
     // With many workgroups (two rounds or more of the three four-wave workgroups that a compute unit holds when
     // each has one buffer of 32 KB) the occupancy is worth more than loads that overlap a workgroup's own work:
     // 12 waves a unit instead of 8 (2 prompts of 2,048 tokens: 140 -> 121 us; 8,192 tokens: 890 -> 718, with 64
     // heads 1,580 -> 1,388).  With fewer it loses to the rounds (2,048 rows after 14,336 keys: 756 -> 825).
     const bool one_buffer = vk_prefill_variant == 19 ||
-                            (vk_prefill_variant == 0 && sizeof(elem_t) == 2 && (int64_t)n_items * nq >= 3 * (int64_t)attn_device_cus());
+                            (vk_prefill_variant == 0 && sizeof(elem_t) == 2 && (int64_t)n_items * nq >= 3 * (int64_t)vk_device_cus());
     if (one_buffer) {
       if (d == 64) PREFILL_LDS1(64); else if (d == 128) PREFILL_LDS1(128); else PREFILL_LDS1(256);
       return vk_check_launch("attention (prompt rows, shared tiles, one buffer)");
@@ -1582,7 +1571,7 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   const bool quad_fits = sizeof(elem_t) * vk_dpad(d) <= 512;
   const bool padded = !seg_fits && d < vk_dpad(d);
   const int half_rounds = padded ? (sizeof(elem_t) == 2 || d <= 80 ? 4 : 6) : (sizeof(elem_t) == 2 || seg_fits ? 5 : 12);
-  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = half_rounds * (int64_t)attn_device_cus() / 2;
+  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = half_rounds * (int64_t)vk_device_cus() / 2;
   if (quad_fits && (vk_decode_variant == 4 || (vk_decode_variant == 0 && segments <= quad_most))) {
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
 #define DECODE_QUAD(DP)                                                                               \
@@ -1693,7 +1682,7 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
   } while (0)
 #define PREFILL_LDS_EXT(DP, NW) do { if (rel != nullptr) PREFILL_LDS_EXT_OF(DP, NW, true); else PREFILL_LDS_EXT_OF(DP, NW, false); } while (0)
     // (In 32-bit with the widest heads eight waves' registers do not hold the three-part products' operands.)
-    const bool four = 2 * (int64_t)n_items * nq < 3 * (int64_t)attn_device_cus() || (sizeof(elem_t) == 4 && d == 256);
+    const bool four = 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus() || (sizeof(elem_t) == 4 && d == 256);
     if (d == 64) { if (four) PREFILL_LDS_EXT(64, 4); else PREFILL_LDS_EXT(64, 8); }
     else if (d == 128) { if (four) PREFILL_LDS_EXT(128, 4); else PREFILL_LDS_EXT(128, 8); }
     else { if (four) PREFILL_LDS_EXT(256, 4); else PREFILL_LDS_EXT(256, 8); }
@@ -1726,7 +1715,7 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
   const int64_t seen = span > 0 ? kept + (span + TILE_KEYS * SEG_TILES - 2) / (TILE_KEYS * SEG_TILES) + 1 : nseg;
   // 32-bit rows of 512 bytes (see below): six workgroups a compute unit, three if the rows are padded, where a launch covers every segment.
   const bool many = sizeof(elem_t) == 4 && row == 512 && seen >= nseg &&
-                    (int64_t)n_items * (nkv * ((G + 15) / 16)) * nseg > (d == vk_dpad(d) ? 6 : 3) * (int64_t)attn_device_cus();
+                    (int64_t)n_items * (nkv * ((G + 15) / 16)) * nseg > (d == vk_dpad(d) ? 6 : 3) * (int64_t)vk_device_cus();
   if (row <= 512 && !many) {
     // Four waves a segment, whatever the number of segments in 16 bits: a tile costs the variant three products a slab and the cap's exponentials,
     // so that a wave a segment was a chain of arithmetic too.  Measured on MI355X with the fold, windows of 1,024, a wave against four
@@ -1777,7 +1766,7 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     return vk_check_launch("attention (combine)");
   }
 #ifdef VK_BF16
-  return vk_fail("attention: no kernel for decoded rows of head size %d", d);      // (none is wider than 256)
+  return 1;      // (not reached: every head took the way above)
 #else
   const dim3 grid(n_items, nkv * ((G + 15) / 16), (nseg + PLAIN_WAVES - 1) / PLAIN_WAVES);
   const bool late = (int64_t)grid.x * grid.y * nseg > 1024;

@@ -181,3 +181,15 @@ int vk_check_launch(const char* what);
   do {                                    \
     if (!(cond)) return vk_fail(__VA_ARGS__); \
   } while (0)
+
+// Compute units of the current device.
+static inline int vk_device_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    cus = n > 0 ? n : 256;
+  }
+  return cus;
+}

@@ -854,17 +854,6 @@ int vk_delta_prep(float* x, int64_t ld, int q_col, int k_col, int T, int G, int 
   return vk_check_launch("delta prep");
 }
 
-static int rule_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
-
 // out [T, H, dv] floats.  qkv: float rows of length ld with q (G heads of d) at q_col, k at k_col, v (H heads of dv) at
 // v_col; decay [T, H, d] floats; b: elements, beta's pre-activation of head h at b[t * ldb + h].  state: per slot,
 // the H states at its start, each [dv][d].  T: the step's tokens.
@@ -897,7 +886,7 @@ static int rule_launch(float* out, const IN* qkv, int64_t ld, int q_col, int k_c
   // the instructions a token and column (2,048 tokens of 32 heads, a column each against two: linear 192 and 222 us, delta 333 and 365,
   // of 8 heads 142 and 194, 272 and 350; three prompts of 1,111, 741 and 370 tokens and 32 heads: 207 and 166, 401 and 311).
   const int per = 256 / (d / 4);                      // columns of a workgroup with a column a lane
-  const int walk_cols = (int64_t)S * H * ((dv + per - 1) / per) <= 2 * (int64_t)rule_cus() ? per : 2 * per;
+  const int walk_cols = (int64_t)S * H * ((dv + per - 1) / per) <= 2 * (int64_t)vk_device_cus() ? per : 2 * per;
   if (vectors && T > S && dv % walk_cols == 0) {
     const dim3 wgrid(S, H, dv / walk_cols);
     VK_REQUIRE(wgrid.y <= 65535 && wgrid.z <= 65535, "delta rule: too many heads or columns");

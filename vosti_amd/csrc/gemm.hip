@@ -40,8 +40,6 @@
 #define KC_SLABS (KC / VK_SLAB)       // 16 (bfloat16) or 32 (float)
 #define SK_WAVES 8
 
-static int device_cus();      // compute units of the current device (defined with the host code below)
-
 // How a product's sums leave a kernel: whether rows take 16-byte (8-byte) stores, and an activation on the rounded sums.
 #define OUT_VEC 1
 #define OUT_SQUARED_RELU 2            // max(., 0)^2
@@ -818,8 +816,8 @@ static const int pipe_band_blocks = 64;
 static bool grouped_wide(int M, int N, int matrices, bool named) {
   const int64_t columns = (N + 255) / 256, groups = columns * (M / 128);
   if (matrices > 0 && (int64_t)M + 127 <= (int64_t)matrices * (127 + 60)) return true;
-  if (columns % 8 == 0 || columns > 16) return 8 * groups >= 5 * device_cus();
-  return !named && columns <= 4 && 2 * groups >= device_cus();
+  if (columns % 8 == 0 || columns > 16) return 8 * groups >= 5 * vk_device_cus();
+  return !named && columns <= 4 && 2 * groups >= vk_device_cus();
 }
 
 template <int S, bool SWIGLU = false, int FNW = 4, bool GROUPED = false>
@@ -863,7 +861,7 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     // touching the lines four tiles ahead brings them into the second-level cache in time (300 rows, 4,096 x
     // 12,288: 146 -> 112 us).  With more workgroups the touches cost more than they bring: the path from
     // that cache into LDS is as busy as the MFMA unit (2,048 rows: 1,057 -> 660 TFLOP/s).
-    if (K % KC == 0 && (int64_t)grid.x * grid.y <= device_cus()) {
+    if (K % KC == 0 && (int64_t)grid.x * grid.y <= vk_device_cus()) {
       static bool touched = false;
       if (!touched) {
         (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 4, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
@@ -1202,7 +1200,7 @@ static int launch_split(elem_t* out, const elem_t* act, const elem_t* w, int M, 
   f32x4* partial = reinterpret_cast<f32x4*>(workspace);
   // Eight waves a workgroup where that still leaves two workgroups or more per compute unit, else four
   // (64 rows, 4096 x 12288: 37.3 against 35.7 us; 6144 x 4096: 19.1 against 19.9 us; sixteen waves were slower).
-  if ((int64_t)((ntiles16 + 7) / 8) * nchunks >= 2 * device_cus())
+  if ((int64_t)((ntiles16 + 7) / 8) * nchunks >= 2 * vk_device_cus())
     gemm_split_kernel<MT, 8><<<dim3((ntiles16 + 7) / 8, nchunks), 512, 0, st>>>(partial, act, w, M, rows, K, lda, ntiles16);
   else
     gemm_split_kernel<MT, 4><<<dim3((ntiles16 + 3) / 4, nchunks), 256, 0, st>>>(partial, act, w, M, rows, K, lda, ntiles16);
@@ -1216,17 +1214,6 @@ static int launch_split(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 #endif
 
 // ==================================================================== host
-static int device_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus <= 0) cus = 256;
-  }
-  return cus;
-}
-
 // Waves a workgroup of the streaming kernels at up to 16 rows, for K of nchunks chunks.  Wave w takes the chunks
 // w, w + waves, ...: with eight waves and ten chunks two waves have a second chunk and six wait for them at every
 // tile's barrier, and with two chunks six of eight waves only take up room.  One chunk a wave where a workgroup
@@ -1281,7 +1268,7 @@ static int stream_waves(int nchunks) {
 // With a workspace the products of up to 64 rows that vk_gemm_split_preferred names go through chunk sums
 // instead (the caller's choice: vk_gemm_split).
 static int choose_gemm_kernel(int M, int N, int K) {
-  const int cus = device_cus();
+  const int cus = vk_device_cus();
   const int wg16 = (N + 15) / 16, wg32 = (N + 31) / 32, wg64 = (N + 63) / 64, wg128 = (N + 127) / 128;
   const bool whole = K % KC == 0, k_resident = K <= SK_WAVES * KC;
   const bool many16 = 2 * wg16 >= 3 * cus;
@@ -1315,7 +1302,7 @@ static int choose_gemm_kernel(int M, int N, int K) {
 // (62 -> 53 us).
 static int pipe_fragments_by_rounds(int M, int N) {
   static const double round_cost[6] = {0, 0, 0, 0.9, 1.0, 1.25};
-  const double slots = 2.0 * device_cus();
+  const double slots = 2.0 * vk_device_cus();
   const int mb = (M + 127) / 128;
   auto estimate = [&](int f) {
     const double rounds = (double)((N + 32 * f - 1) / (32 * f)) * mb / slots;
@@ -1376,11 +1363,6 @@ int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M,
 int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                         const int32_t* block_weights, int64_t weights_stride, const int32_t* row_pair, int activation, hipStream_t st) {
   return vk_gemm_grouped_rows(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, row_pair, nullptr, 0, activation, st);
-}
-
-int vk_gemm_grouped(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
-                    const int32_t* block_weights, int64_t weights_stride, hipStream_t st) {
-  return vk_gemm_grouped_act(out, act, w, M, N, K, lda, ldo, block_weights, weights_stride, nullptr, 0, st);
 }
 
 // kernel: 0 = choose by size, 1 = skinny (M <= 64), 2 = tiled (pipelined if K allows), 3 = tiled through
@@ -1452,7 +1434,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
         // A few weight tiles more than workgroups in flight (one per compute unit) would mean a second
         // pass of a few: two tiles a workgroup then finish sooner (16 rows, 5120 x 25600: 111 -> 86 us),
         // unless one chunk a wave keeps the activations in registers (6144 x 4096: 12.6 against 15.7 us).
-        const int cus = device_cus();
+        const int cus = vk_device_cus();
         const int tiles16 = (N + 15) / 16;
         // One chunk a wave, its activations in registers, wherever a workgroup can have as many waves as K has
         // chunks (stream_waves): no wave then waits at the round's barrier for one that has a second chunk.
@@ -1509,7 +1491,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     // (512 rows, 4096 x 12288: 163 -> 145 us; a workgroup alone on its compute unit is bound by what one
     // compute unit can read, whatever the number of stages).
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
-    if (kernel == 13 || (by_size && tiles <= device_cus())) return launch_pipe<2, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
+    if (kernel == 13 || (by_size && tiles <= vk_device_cus())) return launch_pipe<2, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
     const int fragments = kernel == 15 ? 3 : (kernel == 16 ? 5 : (by_size ? pipe_fragments_by_rounds(M, N) : 4));
     if (fragments == 3) return launch_pipe<2, false, 3>(out, act, w, M, N, K, lda, ldo, form, st);
     if (fragments == 5) return launch_pipe<2, false, 5>(out, act, w, M, N, K, lda, ldo, form, st);
@@ -1558,7 +1540,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
     // best, a workgroup per unit at a time; the larger one where two fill them alike.  64 rows, K = 4096:
     // 12288 gate rows (192, 256, 384 workgroups) 55.4, 49.7, 58.5 us; 8192 gate rows (128, 171, 256) 52.8, 47.0,
     // 41.6 us; 17408 gate rows at K = 5120 (272, 363, 544) 127.5, 108.4, 123.2 us.
-    const int tiles = (I + 15) / 16, cus = device_cus();
+    const int tiles = (I + 15) / 16, cus = vk_device_cus();
     int gt = 4;
     double best = 0.0;
     for (int g = 4; g >= 2; --g) {
@@ -1646,7 +1628,7 @@ int64_t vk_gemm_split_floats(int M, int rows, int K, int swiglu) {
 //     K of up to 8 chunks: never (4096 x 4096 9.1 -> 10.3 us, 2560 x 4096, fill 0.63, 8.3 -> 9.2).
 int vk_gemm_split_preferred(int M, int rows, int K, int swiglu) {
   if (swiglu || vk_gemm_split_floats(M, rows, K, swiglu) == 0) return 0;
-  const int cus = device_cus();
+  const int cus = vk_device_cus();
   const int64_t bytes = (int64_t)rows * K * (int64_t)sizeof(elem_t);
   if (bytes < (int64_t)cus * 65536 || 4 * ((rows + 127) / 128) > cus) return 0;
   if (M > 16) return 1;

@@ -567,21 +567,10 @@ int vk_moe_max_tiles(int T, int top, int E, int tile_rows) {
   return (int)((pairs + busy * (tile_rows - 1)) / tile_rows);
 }
 
-static int moe_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
-
 // logits: scratch [T, E] floats.  bias [E] (elements, or floats with bias_is_f32) or null.
 static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32, int T, int W,
-                        int E, int top, float weight_eps, hipStream_t st, int score_kind = 0, int groups = 1, int keep = 1, float scale = 1.f, int group_score = 0,
-                        const void* correction = nullptr, int correction_is_f32 = 0, const MoePlanArgs* plan = nullptr) {
+                        int E, int top, float weight_eps, hipStream_t st, int score_kind, int groups, int keep, float scale, int group_score, const void* correction,
+                        int correction_is_f32, const MoePlanArgs& plan) {
   VK_REQUIRE(T >= 0 && W > 0 && W % VK_VEC == 0 && E > 0 && top > 0 && top <= E && E <= 4096,
              "router: bad sizes T=%d W=%d E=%d top=%d (the width in whole 16-byte vectors, at most 4096 experts)", T, W, E, top);
   VK_REQUIRE(((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0, "router: operands must be 16-byte aligned");
@@ -595,20 +584,19 @@ static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h
   // Four experts a workgroup from eight workgroups a compute unit on, with one each: that is where a group's rows, read again, become the longer
   // wait (one against four, with choice and plan: 256 tokens of 4,096 entries, 8 experts 10.7, 13.5 us; 32 experts, 255 and 256 tokens of
   // 4,096 11.5, 13.9, 512 15.0, 14.8; 64 experts, 256 tokens of 2,048 11.7, 12.3, 2,048 of them 46, 28).
-  if (E % 4 == 0 && (int64_t)groups_of_tokens * E >= 8 * (int64_t)moe_cus()) moe_logits_kernel<4><<<dim3(grid_x, E / 4), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
+  if (E % 4 == 0 && (int64_t)groups_of_tokens * E >= 8 * (int64_t)vk_device_cus()) moe_logits_kernel<4><<<dim3(grid_x, E / 4), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
   else moe_logits_kernel<1><<<dim3(grid_x, E), 256, 0, st>>>(logits, h, router, T, W, E, bias, bias_is_f32);
   if (vk_check_launch("router (logits)")) return 1;
   const MoeChoice c = {idx, wts, logits, T, E, top, weight_eps, score_kind, groups, keep, scale, group_score, correction, correction_is_f32};
   const size_t a_wave = ((correction != nullptr ? 2 : 1) * (size_t)E + (keep < groups ? groups : 0)) * sizeof(float);
   VK_REQUIRE(4 * a_wave <= 65536, "router: %d experts in %d groups are too many", E, groups);
-  if (plan != nullptr && T <= MOE_FEW_TOKENS(top) && 16 * a_wave <= 65536) {
-    moe_choose_plan_kernel<<<1, 1024, std::max(16 * a_wave, (size_t)2 * E * sizeof(int32_t)), st>>>(c, *plan);
+  if (T <= MOE_FEW_TOKENS(top) && 16 * a_wave <= 65536) {
+    moe_choose_plan_kernel<<<1, 1024, std::max(16 * a_wave, (size_t)2 * E * sizeof(int32_t)), st>>>(c, plan);
     return vk_check_launch("router (choice and plan)");
   }
   moe_choose_kernel<<<(T + 3) / 4, 256, 4 * a_wave, st>>>(c);
   if (vk_check_launch("router (choice)")) return 1;
-  if (plan == nullptr) return 0;
-  moe_plan_kernel<<<1, 1024, (size_t)2 * E * sizeof(int32_t), st>>>(*plan);
+  moe_plan_kernel<<<1, 1024, (size_t)2 * E * sizeof(int32_t), st>>>(plan);
   return vk_check_launch("expert plan");
 }
 
@@ -628,7 +616,7 @@ int vk_moe_route_plan(int32_t* idx, float* wts, float* logits, const elem_t* h, 
   if (T == 0) return 0;
   const MoePlanArgs plan = {idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E, vk_moe_max_tiles(T, top, E, tile_rows), tile_rows};
   return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale, group_score, correction,
-                      correction_is_f32, &plan);
+                      correction_is_f32, plan);
 }
 
 // An expert product of rows in tiles of 16: by the streaming kernel where it takes the sizes, else by the one for every K.
@@ -668,7 +656,7 @@ static int moe_product(elem_t* out, int64_t ldo, const elem_t* x, int64_t ldx, c
   const int64_t units = (int64_t)tiles * ((N + 15) / 16);
   if (K % VK_SLAB == 0 && ldx % VK_VEC == 0 && least != 0 && units >= least) {
     // As many workgroups as the device holds at once: 16 waves a compute unit (128 registers).
-    const int grid = (int)std::min<int64_t>(units, (int64_t)moe_cus() * (16 / chunks));
+    const int grid = (int)std::min<int64_t>(units, (int64_t)vk_device_cus() * (16 / chunks));
     const int vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
     const size_t smem = (size_t)2 * chunks * 64 * sizeof(f32x4);
     if (K % MOE_KC == 0)

@@ -413,14 +413,7 @@ int vk_ssm_scan(float* y, const float* xbc, int64_t ldx, int b_col, int c_col, c
       return vk_check_launch("state-space scan (single tokens)");
     }
     if (!single_tokens && P % 16 == 0) {
-      static int cus = 0;
-      if (cus == 0) {
-        int dev = 0, n = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        cus = n > 0 ? n : 256;
-      }
-      if (P % 32 != 0 || (int64_t)S * H * (P / 16) <= 2 * (int64_t)cus) ssm_walk_kernel<1><<<dim3(S, H, P / 16), SSM_THREADS, 0, st>>>(a);
+      if (P % 32 != 0 || (int64_t)S * H * (P / 16) <= 2 * (int64_t)vk_device_cus()) ssm_walk_kernel<1><<<dim3(S, H, P / 16), SSM_THREADS, 0, st>>>(a);
       else ssm_walk_kernel<2><<<dim3(S, H, P / 32), SSM_THREADS, 0, st>>>(a);
       return vk_check_launch("state-space scan (chunks)");
     }
