@@ -29,8 +29,12 @@
 //                       workgroup, 64x64 per wave, tiles straight from global memory into LDS, two
 //                       stages; a second accumulator set holds the total.  Optionally SwiGLU in the
 //                       epilogue.
+//   gemm_alternate      256 rows or more, K a multiple of 512, 16-bit elements: 256 x 192, 160 or 128 per workgroup of eight
+//                       waves whose two halves take turns between LDS and the matrix unit.  Optionally SwiGLU in the epilogue
+//                       (alternate_fragments says when).
 //   gemm_tiled          any M and K: the same tile through registers into LDS, predicated.
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "mma.h"
@@ -876,6 +880,189 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   return vk_check_launch("gemm_pipe");
 }
 
+#ifdef VK_BF16
+// ------------------------------------------------------------- alternating
+// Tiles of 256 activation rows and 32 FNW weight rows, eight waves, a workgroup a compute unit: 16-bit elements, K in whole chunks, at least
+// a tile's rows of both.  A wave has 64 activation rows and 16 FNW weight rows, in two groups of four waves, one of each a SIMD.  The groups
+// take turns: while one multiplies a slab (4 FNW MFMAs a wave), the other fetches its next slab's fragments from LDS, and a barrier
+// swaps them, so that a SIMD's matrix unit always has a wave whose operands are in registers.  SA (SW) K tiles of two slabs of activations (weights)
+// lie in LDS or are on their way there straight from global memory, brought by group 0 (1); a tile's place is refilled as soon as both groups have
+// read it.  The last block of rows or columns starts early enough to be whole: what it shares with the one before is computed twice and stored
+// twice with the same bits.  Reduction order, operand roles and bits are those of gemm_pipe_kernel.
+//
+// What bounds it: the tile kernel asks the second-level cache for 32 KB per 2.1 MFLOP, which alone takes it 45 % of its time; 256 x 192 asks
+// for 19 KB.  (256 x 256 would need 512 KB of registers for chunk sums and totals, all that a compute unit has.)  Without loads from global
+// memory this kernel reaches 1,430 TFLOP/s, which is near what the chip sustains of these MFMAs (1,640).  Measured on MI355X with the weights
+// of several layers in turn, tile kernel against this one, us: gate/up with SwiGLU 12,288 x 4,096, 2,048 rows 404 -> 349 (1,180 TFLOP/s), 4,096
+// rows 741 -> 646 (1,280); 4,096 x 12,288, 2,048 rows 189 -> 169, 4,096 rows 364 -> 322; 6,144 x 4,096, 2,048 rows 108 -> 93; 5,120 x
+// 17,408, 3,900 rows 633 -> 540 (1,290).  Over 532 sizes of 256 to 4,096 rows 288 take it, 66.2 -> 60.2 ms in all, the worst 7 % slower
+// than before (1,024 rows, 6,144 x 2,560).
+// Tried: K tiles of one slab (rows of 64 bytes, five places: half of every line that the cache sends is not asked for, 162 -> 190 us at 4,096
+// rows, 6,144 x 4,096); a slab's activations read a phase ahead (5 to 15 % slower); a tile's loads in quarters, also between the MFMAs (4 %
+// slower than in halves).
+__device__ __forceinline__ void al_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+template <int FNW, int SA, int SW, bool SWIGLU>
+__global__ __launch_bounds__(512, 2) void gemm_alternate_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w,
+                                                                int M, int N, int K, int64_t lda, int64_t ldo, int out_form, int row_blocks) {
+  static_assert(!SWIGLU || FNW % 2 == 0, "as many gate as up fragments a wave");
+  constexpr int BM = 256, BN = 32 * FNW, COLS = SWIGLU ? BN / 2 : BN;
+  constexpr int A_BYTES = BM * T_ROWB, W_BYTES = BN * T_ROWB;
+  constexpr int LA = BM / 32, LW = BN / 32;                // loads of 8 rows a wave and K tile: group 0's, group 1's
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // [SA][256 rows], [SW][BN rows]
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int group = wave >> 2, q = wave & 3;
+  // Workgroup i runs on chip part i % 8.  A part takes consecutive tiles of an order that walks bands of eight column blocks, all row blocks of
+  // a band before the next: the 32 tiles that a part works on at a time are four row blocks by eight column blocks (the fewest distinct rows
+  // for its cache, whatever the numbers of blocks), and a band's weights come from HBM for one part or two.
+  const int lin = blockIdx.x, tiles = gridDim.x, part = lin & 7;
+  const int tile = part * (tiles >> 3) + min(part, tiles & 7) + (lin >> 3);
+  const int per_band = 8 * row_blocks, band = tile / per_band, at = tile - band * per_band;
+  const int wide = min(8, (N + COLS - 1) / COLS - band * 8);
+  const int mb = at / wide, nb = band * 8 + (at - mb * wide);
+  const int n_blk = min(nb * COLS, N - COLS), m_blk = min(mb * BM, M - BM);
+
+  // A wave-level load brings 8 rows of 128 bytes: lane i fills row i / 8, place i % 8, which holds the row's 16-byte column (i % 8) ^ (i / 8).
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  const int64_t ld = group == 0 ? lda : K;
+  const unsigned voff = (unsigned)((lr * ld + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+  // A wave's rows lie one after the other: 64 of the activations, or 8 FNW of the weights.  With SWIGLU group g's weight rows are 8 FNW of the
+  // gate and their up rows: an even wave brings gate rows, an odd one up rows.
+  const int64_t row0 = group == 0 ? m_blk + q * 64 : SWIGLU ? (int64_t)(q & 1) * N + n_blk + (q >> 1) * (8 * FNW) : n_blk + q * (8 * FNW);
+  const unsigned char* src = reinterpret_cast<const unsigned char*>((group == 0 ? act : w) + row0 * ld);
+  const int64_t step = 8 * ld * (int64_t)sizeof(elem_t);
+  const unsigned lds0 = lds_offset_of(lds) + (group == 0 ? q * LA * 8 * T_ROWB : SA * A_BYTES + q * LW * 8 * T_ROWB);
+  unsigned fill = 0;                                       // the place that the next K tile to be asked for takes
+  // The loads FROM .. TO of a tile of group G; the tile's last ones move on to the next tile.
+  auto issue = [&](auto g_, int from, int to) __attribute__((always_inline)) {
+    constexpr int G = decltype(g_)::value, L = G ? LW : LA;
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      if (j >= from && j < to) pipe_load_to_lds16_sv(src + j * step, voff, __builtin_amdgcn_readfirstlane(lds0 + fill + j * 8 * T_ROWB));
+    if (to < L) return;
+    src += T_ROWB;
+    fill = fill == (G ? (SW - 1) * W_BYTES : (SA - 1) * A_BYTES) ? 0 : fill + (G ? W_BYTES : A_BYTES);
+  };
+
+  f32x4 acc[FNW][4], total[FNW][4];
+#pragma unroll
+  for (int i = 0; i < FNW; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int frag = r16 * T_ROWB + ((kg ^ (r16 & 7)) * 16);
+  const int a_at = q * 64 * T_ROWB + frag, w_at = SA * A_BYTES + group * (16 * FNW) * T_ROWB + frag;
+  unsigned read_a = 0, read_w = 0;
+  // Slab S of a K tile of group G: the first of a chunk starts from zero; where no tile is left to ask for, all loads that still fly are waited
+  // for.  A tile is asked for in two halves where three places give the second one the time.
+  auto slab = [&](auto g_, int S, bool first, bool more) __attribute__((always_inline)) {
+    constexpr int G = decltype(g_)::value, L = G ? LW : LA, HALF = (G ? SW : SA) > 2 ? L / 2 : L;
+    // Fetch: this slab's fragments.
+    frag_t af[4], wf[FNW];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) af[j] = *reinterpret_cast<const frag_t*>(lds + (a_at ^ (S * 64)) + read_a + j * 16 * T_ROWB);
+#pragma unroll
+    for (int i = 0; i < FNW; ++i) wf[i] = *reinterpret_cast<const frag_t*>(lds + (w_at ^ (S * 64)) + read_w + i * 16 * T_ROWB);
+    if (S == 1) {
+      read_a = read_a == (SA - 1) * A_BYTES ? 0 : read_a + A_BYTES;
+      read_w = read_w == (SW - 1) * W_BYTES ? 0 : read_w + W_BYTES;
+    }
+    if (more && S == 0) issue(g_, 0, HALF);
+    if (more && S == 1 && HALF < L) issue(g_, HALF, L);
+    if (G == 1 && S == 1) {                                 // the next tile's weights are there when group 0 starts on it
+      if (more) wait_vmcnt_n<(SW - 2) * LW>(); else wait_vmcnt_n<0>();
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    al_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    // Multiply.
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = mma_slab(wf[i], af[j], first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (G == 0 && S == 1) {
+      if (more) wait_vmcnt_n<(SA - 2) * LA>(); else wait_vmcnt_n<0>();
+    }
+    al_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto chunk = [&](auto g_, bool last) __attribute__((always_inline)) {
+    constexpr int ST = decltype(g_)::value ? SW : SA;
+#pragma unroll
+    for (int t = 0; t < T_CHUNK_TILES; ++t) {
+      const bool more = !last || t + ST - 1 < T_CHUNK_TILES;
+      slab(g_, 0, t == 0, more);
+      slab(g_, 1, false, more);
+    }
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        total[i][j].x = total[i][j].x + acc[i][j].x;
+        total[i][j].y = total[i][j].y + acc[i][j].y;
+        total[i][j].z = total[i][j].z + acc[i][j].z;
+        total[i][j].w = total[i][j].w + acc[i][j].w;
+      }
+  };
+  auto walk = [&](auto g_) __attribute__((always_inline)) {
+    constexpr int G = decltype(g_)::value;
+#pragma unroll
+    for (int p = 0; p < (G ? SW : SA) - 1; ++p) issue(g_, 0, G ? LW : LA);      // K is a chunk or more: more tiles than places
+    wait_vmcnt_n<G ? (SW - 2) * LW : (SA - 2) * LA>();
+    al_barrier();
+    if (G == 1) al_barrier();
+    for (int c = 1; c < K / KC; ++c) chunk(g_, false);
+    chunk(g_, true);
+    if (G == 0) al_barrier();
+  };
+  if (group == 0) walk(std::integral_constant<int, 0>()); else walk(std::integral_constant<int, 1>());
+
+  const int m0 = m_blk + q * 64 + r16, n0 = n_blk + group * (SWIGLU ? 8 * FNW : 16 * FNW) + 4 * kg;
+  if constexpr (SWIGLU) {
+#pragma unroll
+    for (int i = 0; i < FNW / 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = round_to_elem(total[i][j][e]), u = round_to_elem(total[i + FNW / 2][j][e]);
+          y[e] = (g * (1.0f / (1.0f + expf(-g)))) * u;
+        }
+        store_out4(out, ldo, m0 + j * 16, n0 + i * 16, M, N, y, out_form);
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) store_out4(out, ldo, m0 + j * 16, n0 + i * 16, M, N, total[i][j], out_form);
+  }
+}
+
+template <int FNW, int SA, int SW, bool SWIGLU = false>
+static int launch_alternate(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, hipStream_t st) {
+  constexpr int COLS = SWIGLU ? 16 * FNW : 32 * FNW;
+  constexpr size_t smem = (size_t)(SA * 256 + SW * 32 * FNW) * T_ROWB;
+  VK_REQUIRE(M >= 256 && N >= COLS && K % KC == 0, "gemm: the alternating kernel takes 256 rows, %d columns and whole chunks or more", COLS);
+  static bool configured = false;
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_alternate_kernel<FNW, SA, SW, SWIGLU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    configured = true;
+  }
+  const int row_blocks = (M + 255) / 256;
+  const int64_t tiles = (int64_t)row_blocks * ((N + COLS - 1) / COLS);
+  VK_REQUIRE(tiles < (1 << 30), "gemm: too many rows (%d)", M);
+  gemm_alternate_kernel<FNW, SA, SW, SWIGLU><<<(unsigned)tiles, 512, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, row_blocks);
+  return vk_check_launch("gemm_alternate");
+}
+#endif
+
 // ------------------------------------------------------------------ mid
 // 17 to 64 rows.  The streaming kernels read all activations once per 16 weight rows, which at 64 rows
 // is four times the weights and binds them to the second-level cache.  Here a workgroup of eight waves
@@ -1264,7 +1451,8 @@ static int stream_waves(int nchunks) {
 //              wg64 >= 0.5 cus                                 8 up to three blocks, else 2
 //              two blocks                                      9 (wg32 <= 0.5 cus) or 8
 //              else                                            2 (k_resident and wg16 >= 1.5 cus) or 8
-//   more                                                       2   the pipelined tile kernel
+//   more                                                       2   the pipelined tile kernel, or the alternating one
+//                                                                  (alternate_fragments)
 // With a workspace the products of up to 64 rows that vk_gemm_split_preferred names go through chunk sums
 // instead (the caller's choice: vk_gemm_split).
 static int choose_gemm_kernel(int M, int N, int K) {
@@ -1300,7 +1488,7 @@ static int choose_gemm_kernel(int M, int N, int K) {
 // 5,120 weight rows at 2,048 rows are 1.25 rounds of 128 or one of 160 (5,120 x 5,120: 121 -> 93 us, 5,120 x
 // 17,408: 452 -> 337, 5,120 x 25,600: 705 -> 481), 6,144 weight rows at 1,024 rows 0.75 rounds of 128 or one of 96
 // (62 -> 53 us).
-static int pipe_fragments_by_rounds(int M, int N) {
+static int pipe_fragments_by_rounds(int M, int N, double* rounds_of_128 = nullptr) {
   static const double round_cost[6] = {0, 0, 0, 0.9, 1.0, 1.25};
   const double slots = 2.0 * vk_device_cus();
   const int mb = (M + 127) / 128;
@@ -1318,8 +1506,42 @@ static int pipe_fragments_by_rounds(int M, int N) {
       best = f;
     }
   }
+  if (rounds_of_128) *rounds_of_128 = estimate(best);
   return best;
 }
+
+#ifdef VK_BF16
+// How many weight fragments a wave of the alternating kernel takes (6, 5 or 4), or 0: the tile kernel is the faster one.  Both kernels' times go in
+// rounds of the workgroups that run at a time, one a compute unit here; with k = K / 1,024 a round was measured at 13.1 k + 7, 15.8 k + 6 and
+// 18.9 k + 8 us for 128, 160 and 192 columns, at 15 k + 4.5 for the tile kernel's round of as much as the first, and a last round at 0.64 + 0.33
+// of its filled part.
+static int alternate_fragments(int M, int N, int K, bool swiglu) {
+  if (M < 256 || K % KC != 0 || N < (swiglu ? 96 : 192)) return 0;
+  const int cus = vk_device_cus(), out_cols = swiglu ? 2 * N : N;
+  if (!swiglu && (int64_t)((N + 127) / 128) * ((M + 127) / 128) <= cus) return 0;      // workgroups of 64 weight rows
+  static const double slope[7] = {0, 0, 0, 0, 13.1, 15.8, 18.9}, start[7] = {0, 0, 0, 0, 7, 6, 8};
+  const double k = K / 1024.0;
+  double rounds = 0;
+  if (swiglu) {
+    const double r = (double)((N + 63) / 64) * ((M + 127) / 128) / (2.0 * cus), whole = std::floor(r), part = r - whole;
+    rounds = whole + (part == 0 ? 0.0 : (part <= 0.5 ? 0.72 : 1.0));
+  } else {
+    pipe_fragments_by_rounds(M, N, &rounds);
+  }
+  double least = 0.97 * rounds * (15.0 * k + 4.5);
+  int best = 0;
+  for (int f = 6; f >= 4; --f) {
+    if (swiglu && f == 5) continue;
+    const double r = (double)((out_cols + 32 * f - 1) / (32 * f)) * ((M + 255) / 256) / cus, whole = std::floor(r), part = r - whole;
+    const double e = (whole + (part == 0 ? 0.0 : 0.64 + 0.33 * part)) * (slope[f] * k + start[f]);
+    if (e < least) {
+      least = e;
+      best = f;
+    }
+  }
+  return best;
+}
+#endif
 
 extern "C" {
 
@@ -1380,11 +1602,16 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
              (long long)lda, VK_VEC);
   VK_REQUIRE(ldo >= N, "gemm: output row stride %lld is smaller than N=%d", (long long)ldo, N);
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm: operands must be 16-byte aligned");
-  VK_REQUIRE(kernel >= 0 && kernel <= 16 && kernel != 14, "gemm: unknown kernel %d", kernel);
+  VK_REQUIRE(kernel >= 0 && kernel <= 19 && kernel != 14, "gemm: unknown kernel %d", kernel);
   if (M == 0) return 0;
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
   if (kernel == 0) kernel = choose_gemm_kernel(M, N, K);
+#ifdef VK_BF16
+  if (kernel == 17) return launch_alternate<6, 2, 3>(out, act, w, M, N, K, lda, ldo, form, st);
+  if (kernel == 18) return launch_alternate<5, 3, 3>(out, act, w, M, N, K, lda, ldo, form, st);
+  if (kernel == 19) return launch_alternate<4, 3, 4>(out, act, w, M, N, K, lda, ldo, form, st);
+#endif
   if (kernel == 12) {      // 32 weight rows per workgroup, four chunks in work, blocks of 32 rows
     VK_REQUIRE(M > 16 && M <= 512 && K % KC == 0, "gemm: the mid kernel takes 17 to 512 rows and K a multiple of %d", KC);
     return launch_mid<2, 4>(out, act, w, M, N, K, lda, ldo, form, st);
@@ -1492,6 +1719,14 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     // compute unit can read, whatever the number of stages).
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
     if (kernel == 13 || (by_size && tiles <= vk_device_cus())) return launch_pipe<2, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
+#ifdef VK_BF16
+    if (by_size) {
+      const int f = alternate_fragments(M, N, K, false);
+      if (f == 6) return launch_alternate<6, 2, 3>(out, act, w, M, N, K, lda, ldo, form, st);
+      if (f == 5) return launch_alternate<5, 3, 3>(out, act, w, M, N, K, lda, ldo, form, st);
+      if (f == 4) return launch_alternate<4, 3, 4>(out, act, w, M, N, K, lda, ldo, form, st);
+    }
+#endif
     const int fragments = kernel == 15 ? 3 : (kernel == 16 ? 5 : (by_size ? pipe_fragments_by_rounds(M, N) : 4));
     if (fragments == 3) return launch_pipe<2, false, 3>(out, act, w, M, N, K, lda, ldo, form, st);
     if (fragments == 5) return launch_pipe<2, false, 5>(out, act, w, M, N, K, lda, ldo, form, st);
@@ -1532,6 +1767,13 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   VK_REQUIRE(how != 0, "gemm_swiglu: sizes M=%d I=%d K=%d are not supported", M, I, K);
   VK_REQUIRE(lda >= K && lda % VK_VEC == 0 && ldo >= I, "gemm_swiglu: bad row strides");
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm_swiglu: operands must be 16-byte aligned");
+#ifdef VK_BF16
+  if (how == 2) {
+    const int f = alternate_fragments(M, I, K, true), ok4 = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
+    if (f == 6) return launch_alternate<6, 2, 3, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
+    if (f == 4) return launch_alternate<4, 3, 4, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
+  }
+#endif
   if (how == 2)
     return launch_pipe<2, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
   if (how == 3) {
