@@ -184,6 +184,12 @@ __global__ void cast_to_f32_kernel(float* __restrict__ out, const elem_t* __rest
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = to_f32(in[i]);
 }
+// Rows that the host reads next, written straight into pinned host memory: a launch of a few us where a copy that the runtime puts on
+// another queue adds 15 to 20 us to a step.  Bound by the bus (50 GB/s): a few workgroups with whole vectors are enough.
+template <typename V>
+__global__ __launch_bounds__(256) void copy_out_kernel(V* __restrict__ out, const V* __restrict__ in, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = in[i];
+}
 __global__ void cast_from_f32_kernel(elem_t* __restrict__ out, const float* __restrict__ in, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = from_f32<elem_t>(in[i]);
@@ -361,6 +367,20 @@ int vk_cast_to_f32(float* out, const elem_t* in, int64_t n, hipStream_t st) {
   if (n <= 0) return 0;
   cast_to_f32_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(out, in, n);
   return vk_check_launch("cast_to_f32");
+}
+
+// n elements to memory that the GPU can write, on the device or the host.
+int vk_copy_out(elem_t* out, const elem_t* in, int64_t n, hipStream_t st) {
+  VK_REQUIRE(n >= 0 && n < ((int64_t)1 << 40), "copy_out: bad size %lld", (long long)n);
+  if (n == 0) return 0;
+  if (n % VK_VEC == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)in % 16 == 0) {
+    const int64_t v = n / VK_VEC, wgs = (v + 255) / 256;
+    copy_out_kernel<u32x4><<<(unsigned)(wgs < 256 ? wgs : 256), 256, 0, st>>>(reinterpret_cast<u32x4*>(out), reinterpret_cast<const u32x4*>(in), v);
+  } else {
+    const int64_t wgs = (n + 255) / 256;
+    copy_out_kernel<elem_t><<<(unsigned)(wgs < 1024 ? wgs : 1024), 256, 0, st>>>(out, in, n);
+  }
+  return vk_check_launch("copy_out");
 }
 
 int vk_cast_from_f32(elem_t* out, const float* in, int64_t n, hipStream_t st) {

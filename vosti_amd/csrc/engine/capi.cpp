@@ -166,9 +166,7 @@ int64_t ve_trace_step(void* h, int n_entries, const int64_t* ids, const int32_t*
     const int64_t rows = logits.numel() ? logits.dim(0) : 0;
     if (rows > 0) {
       if (logits.numel() > out_floats) throw EngineError("the caller's buffer is too small for the wanted logits");
-      Kernels& k = e->model().kernels();
-      const Tensor f = k.to_f32(logits);
-      hip_check(hipMemcpyAsync(out, f.data, f.bytes(), hipMemcpyDeviceToHost, k.stream), "logits readback");
+      e->read_logits(logits, out);
     }
     e->synchronize();
     return rows;

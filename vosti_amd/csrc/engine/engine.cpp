@@ -2,7 +2,10 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cstring>
 #include <numeric>
+
+#include <emmintrin.h>
 
 namespace vosti {
 
@@ -80,9 +83,60 @@ Engine::~Engine() {
   runner_.reset();
   if (sample_in_) (void)hipHostFree(sample_in_);
   if (sample_out_) (void)hipHostFree(sample_out_);
+  for (hipEvent_t e : read_done_)
+    if (e) (void)hipEventDestroy(e);
+  if (read_places_) (void)hipHostFree(read_places_);
 }
 
 void Engine::synchronize() { hip_check(hipStreamSynchronize(kernels_->stream), "waiting for the stream"); }
+
+// n elements of 16 bits as float32 (exact: the upper half of each).
+static void widen(float* out, const uint16_t* in, size_t n) {
+  const __m128i zero = _mm_setzero_si128();
+  size_t i = 0;
+  for (; i + 8 <= n; i += 8) {
+    const __m128i v = _mm_loadu_si128(reinterpret_cast<const __m128i*>(in + i));
+    _mm_storeu_si128(reinterpret_cast<__m128i*>(out + i), _mm_unpacklo_epi16(zero, v));
+    _mm_storeu_si128(reinterpret_cast<__m128i*>(out + i + 4), _mm_unpackhi_epi16(zero, v));
+  }
+  for (; i < n; ++i) {
+    const uint32_t bits = (uint32_t)in[i] << 16;
+    std::memcpy(out + i, &bits, sizeof bits);
+  }
+}
+
+// Through pinned memory that the engine keeps, as elements, piece after piece: a copy into the caller's pageable memory goes through
+// the runtime's own staging (measured on this machine: 600 KB 260 us against 19 into pinned memory and 20 from there).  The caller's memory is
+// usually fresh: its pages are touched while the GPU still works on the step (4.7 MB: 400 to 1,000 us of page faults).
+void Engine::read_logits(const Tensor& logits, float* out) {
+  const DType type = kernels_->dtype();
+  if (logits.dtype != type) throw EngineError("logits of " + logits.describe() + " cannot be read back");
+  const size_t total = (size_t)logits.numel(), size = dtype_bytes(type);
+  if (!total) return;
+  for (hipEvent_t& e : read_done_)
+    if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event creation");
+  if (!read_places_) hip_check(hipHostMalloc(reinterpret_cast<void**>(&read_places_), kReadPlaces * kReadBytes, hipHostMallocDefault), "pinned allocation");
+  // Up to 1 MB in one piece (a launch and an event a piece); more in quarters and at most as much as a place holds, so that
+  // a piece is widened while the next is on its way.
+  const size_t quarter = (total + kReadPlaces - 1) / kReadPlaces;
+  const size_t piece = std::min(kReadBytes / size, std::max<size_t>((quarter + 7) & ~(size_t)7, ((size_t)1 << 20) / size));
+  const size_t pieces = (total + piece - 1) / piece;
+  auto ask = [&](size_t i) {
+    kernels_->copy_out(read_places_ + (i % kReadPlaces) * kReadBytes, logits, (int64_t)(i * piece), (int64_t)std::min(piece, total - i * piece));
+    hip_check(hipEventRecord(read_done_[i % kReadPlaces], kernels_->stream), "event record");
+  };
+  for (size_t i = 0; i < std::min<size_t>(pieces, kReadPlaces); ++i) ask(i);
+  volatile char* page = reinterpret_cast<volatile char*>(out);
+  for (size_t b = 0; b < total * sizeof(float); b += 4096) page[b] = 0;
+  for (size_t i = 0; i < pieces; ++i) {
+    hip_check(hipEventSynchronize(read_done_[i % kReadPlaces]), "logits readback");
+    const char* from = read_places_ + (i % kReadPlaces) * kReadBytes;
+    const size_t first = i * piece, n = std::min(piece, total - first);
+    if (type == DType::F32) std::memcpy(out + first, from, n * sizeof(float));
+    else widen(out + first, reinterpret_cast<const uint16_t*>(from), n);
+    if (i + kReadPlaces < pieces) ask(i + kReadPlaces);
+  }
+}
 
 RequestId Engine::add_request(const std::vector<int32_t>& prompt, const SamplingParams& params) {
   if (params.max_tokens <= 0) throw EngineError("max_tokens must be positive");
@@ -165,10 +219,8 @@ std::vector<int32_t> Engine::forward_and_sample(const std::vector<PlanRow>& rows
   if (R == 0) return sampled;
   if (R > sample_rows_) throw EngineError("more sampled rows than the engine was made for");
   if (observer_.active()) {
-    const Tensor f = kernels_->to_f32(logits);
-    observed_.resize((size_t)f.numel());
-    hip_check(hipMemcpyAsync(observed_.data(), f.data, f.bytes(), hipMemcpyDeviceToHost, kernels_->stream), "logits readback");
-    hip_check(hipStreamSynchronize(kernels_->stream), "logits readback");
+    observed_.resize((size_t)logits.numel());
+    read_logits(logits, observed_.data());
     std::vector<int> places;
     for (size_t i = 0; i < rows.size(); ++i)
       if (rows[i].sample) places.push_back((int)i);

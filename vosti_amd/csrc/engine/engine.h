@@ -74,6 +74,8 @@ class Engine {
   std::vector<std::vector<int32_t>> generate(const std::vector<std::vector<int32_t>>& prompts, const std::vector<SamplingParams>& params,
                                              const std::vector<int>& arrival_steps = {}, std::FILE* trace = nullptr);
   void synchronize();
+  // The logits (elements, anywhere on the GPU) as float32 at `out`, once everything before them on the stream is done.
+  void read_logits(const Tensor& logits, float* out);
 
   CacheManager& cache() { return pool_->manager(); }
   Scheduler& scheduler() { return *scheduler_; }
@@ -110,6 +112,11 @@ class Engine {
   // that batch differently (python/vosti_kernels/kernels.py:1020-1033).
   LogitsObserver observer_;
   std::vector<float> observed_;
+  // The pinned places that logits pass through on their way to the host, used in turn, each with the event of its last copy.
+  static constexpr int kReadPlaces = 4;
+  static constexpr size_t kReadBytes = (size_t)2 << 20;
+  char* read_places_ = nullptr;       // pinned [kReadPlaces, kReadBytes], from the first readback on
+  hipEvent_t read_done_[kReadPlaces] = {};
   // The sampler's buffers: temperatures and uniform numbers up, token ids down.
   float* sample_in_ = nullptr;        // pinned [2, rows]
   int32_t* sample_out_ = nullptr;     // pinned [rows]

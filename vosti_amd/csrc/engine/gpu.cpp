@@ -83,6 +83,7 @@ struct Kernels::Fn {
   int (*swiglu)(P, CP, int, int, hipStream_t);
   int (*gather_rows)(P, CP, CP, int, int, hipStream_t);
   int (*cast_to_f32)(P, CP, int64_t, hipStream_t);
+  int (*copy_out)(P, CP, int64_t, hipStream_t);
   int (*rope_tables)(P, P, CP, int, int, hipStream_t);
   int (*fill_random)(P, int64_t, uint64_t, int, float, float, hipStream_t);
   int (*gemm)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
@@ -187,7 +188,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
     throw EngineError(path + " has ABI " + std::to_string(fn_->abi_version()) + ", expected " + std::to_string(KERNEL_ABI) + "; rebuild it");
   if (fn_->elem_bytes() != dtype_bytes(dtype_)) throw EngineError(path + " was built for another element type");
   VK(embedding, "vk_embedding"); VK(rmsnorm, "vk_rmsnorm"); VK(add_rmsnorm, "vk_add_rmsnorm"); VK(swiglu, "vk_swiglu");
-  VK(gather_rows, "vk_gather_rows"); VK(cast_to_f32, "vk_cast_to_f32"); VK(rope_tables, "vk_rope_tables"); VK(fill_random, "vk_fill_random");
+  VK(gather_rows, "vk_gather_rows"); VK(cast_to_f32, "vk_cast_to_f32"); VK(copy_out, "vk_copy_out"); VK(rope_tables, "vk_rope_tables"); VK(fill_random, "vk_fill_random");
   VK(gemm, "vk_gemm"); VK(gemm_swiglu, "vk_gemm_swiglu"); VK(gemm_swiglu_supported, "vk_gemm_swiglu_supported");
   VK(gemm_split, "vk_gemm_split"); VK(gemm_split_floats, "vk_gemm_split_floats"); VK(gemm_split_preferred, "vk_gemm_split_preferred");
   VK(qkv_post, "vk_qkv_post"); VK(paged_attention, "vk_paged_attention"); VK(sample, "vk_sample");
@@ -315,6 +316,11 @@ Tensor Kernels::to_f32(const Tensor& x) {
   Tensor out = empty(x.shape, DType::F32);
   call(fn_->cast_to_f32(out.data, x.data, x.numel(), stream));
   return out;
+}
+
+void Kernels::copy_out(void* out, const Tensor& x, int64_t first, int64_t count) {
+  if (x.dtype != dtype_ || first < 0 || count < 0 || first + count > x.numel()) throw EngineError("copy_out: " + std::to_string(count) + " elements of " + x.describe());
+  call(fn_->copy_out(out, static_cast<const char*>(x.data) + first * (int64_t)dtype_bytes(dtype_), count, stream));
 }
 
 Tensor Kernels::to_elements(const Tensor& x) {

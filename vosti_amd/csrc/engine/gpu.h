@@ -109,6 +109,8 @@ class Kernels {
   Tensor swiglu(const Tensor& gate_up);
   Tensor gather_rows(const Tensor& x, const Tensor& rows);
   Tensor to_f32(const Tensor& x);
+  // The elements first .. first + count of x to memory that the GPU can write (pinned host memory).
+  void copy_out(void* out, const Tensor& x, int64_t first, int64_t count);
   // A 32-bit tensor as elements (the tensor itself where the elements are 32-bit).
   Tensor to_elements(const Tensor& x);
   // Columns [first, first + count) of a [rows, width] tensor as a tensor of their own.
