@@ -104,6 +104,9 @@ struct Kernels::Fn {
   int (*stream_norm_add)(P, CP, CP, CP, int, int, int, float, float, float, hipStream_t);
   int (*stream_mix)(P, CP, int64_t, CP, int, int, int64_t, hipStream_t);
   int (*gather_rows_f32)(P, CP, CP, int, int, hipStream_t);
+  int (*stream_step_takes)(int);
+  int (*stream_norm_step)(P, CP, CP, int, CP, int, int, int, float, float, float, P, CP, int64_t, CP, int, int, P, CP, int, float, float, hipStream_t);
+  int (*stream_sum_norms)(P, CP, CP, int, int, P, CP, int, float, float, P, CP, int, float, float, hipStream_t);
   int (*softcap)(P, float, int64_t, hipStream_t);
   int (*qkv_post_bias)(CP, int64_t, P, P, P, CP, CP, int, CP, CP, int, CP, CP, int, int, int, int, int, float, CP, hipStream_t);
   int (*paged_attention_capped)(P, CP, CP, CP, CP, int, CP, CP, CP, int, int, int, P, int, int, int, int, int, int, int, float, float, CP, int,
@@ -195,7 +198,8 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(sample_scratch_words, "vk_sample_scratch_words"); VK(attn_scratch_floats, "vk_attn_scratch_floats");
   VK(attn_segment_keys, "vk_attn_segment_keys"); VK(attn_item_rows, "vk_attn_item_rows");
   VK(embed_sinusoid, "vk_embed_sinusoid"); VK(stream_norm, "vk_stream_norm"); VK(stream_norm_add, "vk_stream_norm_add");
-  VK(stream_mix, "vk_stream_mix"); VK(gather_rows_f32, "vk_gather_rows_f32"); VK(softcap, "vk_softcap");
+  VK(stream_mix, "vk_stream_mix"); VK(stream_step_takes, "vk_stream_step_takes"); VK(stream_norm_step, "vk_stream_norm_step"); VK(stream_sum_norms, "vk_stream_sum_norms");
+  VK(gather_rows_f32, "vk_gather_rows_f32"); VK(softcap, "vk_softcap");
   VK(qkv_post_bias, "vk_qkv_post_bias"); VK(paged_attention_capped, "vk_paged_attention_capped");
   VK(delta_conv, "vk_delta_conv"); VK(delta_prep, "vk_delta_prep"); VK(delta_unit, "vk_delta_unit"); VK(delta_decay, "vk_delta_decay"); VK(delta_rule, "vk_delta_rule");
   VK(delta_out, "vk_delta_out"); VK(delta_conv_bias, "vk_delta_conv_bias"); VK(paged_attention_blocked, "vk_paged_attention_blocked");
@@ -536,6 +540,45 @@ void Kernels::stream_norm_add(Tensor& out, const Tensor& base, const Tensor& y, 
     return;
   }
   call(fn_->stream_norm_add(out.data, base.data, y.data, w.data, wf, (int)y.dim(0), (int)y.dim(1), eps, offset, mult, stream));
+}
+
+bool Kernels::stream_step_takes(int64_t H, std::initializer_list<const Tensor*> rows) const {
+  for (const Tensor* t : rows)
+    if (reinterpret_cast<uintptr_t>(t->data) % 16) return false;
+  return H <= (1 << 24) && fn_->stream_step_takes((int)H) != 0;
+}
+
+Tensor Kernels::stream_norm_step(Tensor& out, const Tensor& base, const Tensor& y, const RowNorm& add, float mult, const RowNorm& next, const Tensor* states,
+                                 const Tensor* coef, int n, Tensor* mixed) {
+  if (y.dtype != DType::F32) expect(y, "norm input", dtype_);
+  if (y.shape.size() != 2) throw EngineError("norm input is " + y.describe());
+  expect(base, "stream", DType::F32, y.shape);
+  expect(out, "stream", DType::F32, y.shape);
+  const int wf = norm_weight(*add.weight, "norm weight", y.dim(1)), wf2 = norm_weight(*next.weight, "norm weight", y.dim(1));
+  int cf = 0;
+  if (mixed) {
+    expect(*states, "stream states", DType::F32);
+    expect(*mixed, "stream", DType::F32, y.shape);
+    if (n <= 0 || n > states->dim(0) || states->numel() != states->dim(0) * y.numel()) throw EngineError("stream mix: " + std::to_string(n) + " of " + states->describe());
+    cf = norm_weight(*coef, "mixing weights", n);
+  }
+  Tensor normed = empty(y.shape);
+  call(fn_->stream_norm_step(out.data, base.data, y.data, y.dtype == DType::F32 ? 1 : 0, add.weight->data, wf, (int)y.dim(0), (int)y.dim(1), add.eps, add.offset, mult,
+                             mixed ? mixed->data : nullptr, mixed ? states->data : nullptr, y.numel(), mixed ? coef->data : nullptr, cf, n, normed.data, next.weight->data,
+                             wf2, next.eps, next.offset, stream));
+  return normed;
+}
+
+std::pair<Tensor, Tensor> Kernels::stream_sum_norms(Tensor& s, const Tensor& a, const Tensor& b, const RowNorm& first, const RowNorm& second) {
+  if (s.shape.size() != 2) throw EngineError("the stream is " + s.describe());
+  expect(s, "stream", DType::F32);
+  expect(a, "a sublayer's output", DType::F32, s.shape);
+  expect(b, "a sublayer's output", DType::F32, s.shape);
+  const int wf = norm_weight(*first.weight, "norm weight", s.dim(1)), wf2 = norm_weight(*second.weight, "norm weight", s.dim(1));
+  std::pair<Tensor, Tensor> out = {empty(s.shape), empty(s.shape)};
+  call(fn_->stream_sum_norms(s.data, a.data, b.data, (int)s.dim(0), (int)s.dim(1), out.first.data, first.weight->data, wf, first.eps, first.offset, out.second.data,
+                             second.weight->data, wf2, second.eps, second.offset, stream));
+  return out;
 }
 
 Tensor Kernels::stream_mix(const Tensor& states, const Tensor& coef, int n) {

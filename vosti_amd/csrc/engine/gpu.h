@@ -10,6 +10,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstdint>
+#include <initializer_list>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -148,6 +149,18 @@ class Kernels {
   // rounded (elements of out's shape, or null): the new rows rounded to elements as well.
   void stream_norm_add(Tensor& out, const Tensor& base, const Tensor& y, const Tensor& w, float eps, float offset, float mult, Tensor* rounded = nullptr);
   // out = sum over j < n of coef[j] * states[j]; states [>= n, ...] floats.
+  // A norm over rows, y = x * rsqrt(mean(x^2) + eps) * (offset + weight); no weight: another kind of norm.
+  struct RowNorm {
+    const Tensor* weight = nullptr;
+    float eps = 0.f, offset = 0.f;
+  };
+  // Whether the two launches below take these rows of this length, by size and alignment (the others do the same one after the other, with the same bits).
+  bool stream_step_takes(int64_t H, std::initializer_list<const Tensor*> rows) const;
+  // out = base + mult * add(y); with `mixed`, mixed = sum over j < n of coef[j] * states[j], of which out is the last; returns next(mixed), or next(out).
+  Tensor stream_norm_step(Tensor& out, const Tensor& base, const Tensor& y, const RowNorm& add, float mult, const RowNorm& next, const Tensor* states = nullptr,
+                          const Tensor* coef = nullptr, int n = 0, Tensor* mixed = nullptr);
+  // s += a + b (floats); returns both norms of the new rows.
+  std::pair<Tensor, Tensor> stream_sum_norms(Tensor& s, const Tensor& a, const Tensor& b, const RowNorm& first, const RowNorm& second);
   Tensor stream_mix(const Tensor& states, const Tensor& coef, int n);
   void softcap(Tensor& x, float cap);          // x <- cap * tanh(x / cap)
   // gemm on the columns [first, first + w.dim(1)) of act.

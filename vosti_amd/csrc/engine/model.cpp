@@ -335,6 +335,8 @@ Tensor DecoderModel::forward(const Tensor& ids, StepContext& ctx, std::vector<Ca
   ctx.ids = ids;
   Tensor hidden = embedding_->forward(ids, ctx), residual;
   for (size_t i = 0; i < spec_.schedule.size(); ++i) {
+    ctx.running = layers_[spec_.schedule[i].layer].get();
+    ctx.following = i + 1 < spec_.schedule.size() ? layers_[spec_.schedule[i + 1].layer]->input_norms() : std::pair<Norm*, Norm*>(nullptr, nullptr);
     auto hr = layers_[spec_.schedule[i].layer]->forward(hidden, residual, ctx, caches[i]);
     hidden = hr.first;
     residual = hr.second;

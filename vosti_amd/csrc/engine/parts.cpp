@@ -93,6 +93,21 @@ std::pair<Tensor, Tensor> PositionEncoding::apply(const Tensor& q, const Tensor&
   return {rotate(q), k.data ? rotate(k) : Tensor()};
 }
 
+std::pair<Tensor, Tensor> Block::take_left(StepContext& ctx, const Tensor& hidden, Norm* first, Norm* second) const {
+  std::pair<Tensor, Tensor> out;
+  if (ctx.running != this) return out;
+  if (ctx.left_of.data && ctx.left_of.data == hidden.data && ctx.left_of.shape == hidden.shape && ctx.left_by == std::make_pair(first, second)) out = ctx.left_normed;
+  ctx.left_normed = {};
+  ctx.left_of = Tensor();
+  return out;
+}
+
+void Block::leave(StepContext& ctx, const Tensor& stream, std::pair<Tensor, Tensor> normed) const {
+  ctx.left_normed = std::move(normed);
+  ctx.left_of = stream;
+  ctx.left_by = ctx.following;
+}
+
 std::pair<Tensor, Tensor> Block::rows_for_the_end(const Tensor& hidden, const Tensor& residual, StepContext& ctx, const Tensor& rows) {
   (void)ctx;
   return {kernels.gather_rows(hidden, rows), residual.data ? kernels.gather_rows(residual, rows) : Tensor()};
@@ -367,6 +382,11 @@ class RMSNorm : public Norm {
   }
   const Tensor* row_scale_weight() const override { return offset_ == 0.f ? &weight_ : nullptr; }
   float eps() const override { return eps_; }
+  // (In 32-bit elements a weight without an offset goes by the elements' norm, whose order is another.)
+  Kernels::RowNorm stream_norm() const override {
+    if (offset_ == 0.f && kernels.dtype() == DType::F32) return {};
+    return {&weight_, eps_, offset_};
+  }
 
  private:
   int64_t size_;
@@ -1204,14 +1224,19 @@ class SandwichDepthBlock : public Block {
     if (hidden.dtype != DType::F32 || hidden.shape.size() != 2 || hidden.dim(1) != hidden_)
       throw EngineError("a sandwich_depth block takes the 32-bit residual stream, not " + hidden.describe());
     const int64_t T = hidden.dim(0);
+    // What a sublayer gives is normed, scaled, added to the stream (and, at the end of a deep layer, summed with the earlier states), and the next
+    // sublayer's norm follows: one launch where the norms are the stream's own, also from one layer to the next (StepContext::following).
+    Norm* input = norms_["mixer_in"].get();
+    Tensor ready = take_left(ctx, hidden, input, nullptr).first;
+    const Tensor mixed = mixer_->forward(ready.data ? ready : input->forward(hidden), ctx, cache);
     if (!deep_) {
       // The plain arrangement (kind "sandwich"): the stream itself is passed on.
       Tensor stream = hidden;
-      const Tensor mixed = mixer_->forward(norms_["mixer_in"]->forward(hidden), ctx, cache);
-      norms_["mixer_out"]->forward_scaled_add(mixed, hidden, stream, mult_);
       if (has_ffn_) {
-        const Tensor fed = ffn_->forward(norms_["ffn_in"]->forward(stream), ctx);
-        norms_["ffn_out"]->forward_scaled_add(fed, stream, stream, mult_);
+        const Tensor fed = ffn_->forward(add_and_norm("mixer_out", mixed, hidden, stream, *norms_["ffn_in"]), ctx);
+        add_and_leave(ctx, "ffn_out", fed, stream, stream);
+      } else {
+        add_and_leave(ctx, "mixer_out", mixed, hidden, stream);
       }
       return {stream, residual};
     }
@@ -1222,19 +1247,40 @@ class SandwichDepthBlock : public Block {
     }
     if (!states.data || states.dim(0) != states_ || states.dim(1) != T) throw EngineError("a sandwich_depth block found no states of this step's stream");
     Tensor result = states.rows(depth_ + 1, 1).view({T, hidden_});
-    const Tensor mixed = mixer_->forward(norms_["mixer_in"]->forward(hidden), ctx, cache);
+    const char* last = "mixer_out";
+    Tensor base = hidden, y = mixed;
     if (has_ffn_) {
-      Tensor mid = k.empty({T, hidden_}, DType::F32);
-      norms_["mixer_out"]->forward_scaled_add(mixed, hidden, mid, mult_);
-      const Tensor fed = ffn_->forward(norms_["ffn_in"]->forward(mid), ctx);
-      norms_["ffn_out"]->forward_scaled_add(fed, mid, result, mult_);
-    } else {
-      norms_["mixer_out"]->forward_scaled_add(mixed, hidden, result, mult_);
+      base = k.empty({T, hidden_}, DType::F32);
+      y = ffn_->forward(add_and_norm("mixer_out", mixed, hidden, base, *norms_["ffn_in"]), ctx);
+      last = "ffn_out";
     }
+    const Kernels::RowNorm add = norms_[last]->stream_norm(), next = following(ctx).first ? following(ctx).first->stream_norm() : Kernels::RowNorm();
+    if (add.weight && next.weight && !following(ctx).second && k.stream_step_takes(hidden_, {&result, &base, &y, &states})) {
+      Tensor sum = k.empty({T, hidden_}, DType::F32);
+      const Tensor normed = k.stream_norm_step(result, base, y, add, mult_, next, &states, &weights_, depth_ + 2, &sum);
+      leave(ctx, sum, {normed, Tensor()});
+      return {sum, residual};
+    }
+    norms_[last]->forward_scaled_add(y, base, result, mult_);
     return {k.stream_mix(states, weights_, depth_ + 2), residual};
   }
+  std::pair<Norm*, Norm*> input_norms() override { return {norms_["mixer_in"].get(), nullptr}; }
 
  private:
+  // out = base + mult * norm(y); returns next(out).
+  Tensor add_and_norm(const char* norm, const Tensor& y, const Tensor& base, Tensor& out, Norm& next) {
+    const Kernels::RowNorm add = norms_[norm]->stream_norm(), after = next.stream_norm();
+    if (add.weight && after.weight && kernels.stream_step_takes(hidden_, {&out, &base, &y})) return kernels.stream_norm_step(out, base, y, add, mult_, after);
+    norms_[norm]->forward_scaled_add(y, base, out, mult_);
+    return next.forward(out);
+  }
+  // The same at a layer's end, with the next layer's norm where it is known.
+  void add_and_leave(StepContext& ctx, const char* norm, const Tensor& y, const Tensor& base, Tensor& out) {
+    Norm* next = following(ctx).second ? nullptr : following(ctx).first;
+    if (next && norms_[norm]->stream_norm().weight && next->stream_norm().weight && kernels.stream_step_takes(hidden_, {&out, &base, &y}))
+      leave(ctx, out, {add_and_norm(norm, y, base, out, *next), Tensor()});
+    else norms_[norm]->forward_scaled_add(y, base, out, mult_);
+  }
   std::unique_ptr<Mixer> mixer_;
   std::unique_ptr<FeedForward> ffn_;
   std::map<std::string, std::unique_ptr<Norm>> norms_;
@@ -1526,14 +1572,22 @@ class ParallelSumBlock : public Block {
     return c;
   }
   Mixer& mixer() override { return *mixer_; }
+  std::pair<Norm*, Norm*> input_norms() override { return {norms_["mixer_in"].get(), has_ffn_ ? norms_["ffn_in"].get() : nullptr}; }
   std::pair<Tensor, Tensor> forward(const Tensor& hidden, Tensor residual, StepContext& ctx, CacheEntry& cache) override {
     if (hidden.dtype != DType::F32 || hidden.shape.size() != 2 || hidden.dim(1) != hidden_)
       throw EngineError("a parallel_sum block takes the 32-bit residual stream, not " + hidden.describe());
     Tensor stream = hidden;
-    const Tensor mixed = mixer_->forward(norms_["mixer_in"]->forward(hidden), ctx, cache);
+    Norm *first = norms_["mixer_in"].get(), *second = has_ffn_ ? norms_["ffn_in"].get() : nullptr;
+    const std::pair<Tensor, Tensor> ready = take_left(ctx, hidden, first, second);
+    const Tensor mixed = mixer_->forward(ready.first.data ? ready.first : first->forward(hidden), ctx, cache);
     if (has_ffn_) {
-      const Tensor fed = ffn_->forward(norms_["ffn_in"]->forward(hidden), ctx);
-      kernels.stream_add(stream, mixed, &fed);
+      const Tensor fed = ffn_->forward(ready.second.data ? ready.second : second->forward(hidden), ctx);
+      // The sum and both norms of the next layer, where it is of this kind, in one launch.
+      const std::pair<Norm*, Norm*> next = following(ctx);
+      if (next.first && next.second && next.first->stream_norm().weight && next.second->stream_norm().weight && mixed.dtype == DType::F32 &&
+          fed.dtype == DType::F32 && kernels.stream_step_takes(hidden_, {&stream, &mixed, &fed}))
+        leave(ctx, stream, kernels.stream_sum_norms(stream, mixed, fed, next.first->stream_norm(), next.second->stream_norm()));
+      else kernels.stream_add(stream, mixed, &fed);
     } else {
       kernels.stream_add(stream, mixed, nullptr);
     }

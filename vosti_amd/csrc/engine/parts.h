@@ -56,6 +56,9 @@ struct HeadColumns {
   int heads = 0, stride = 0, size = 0;
 };
 
+class Norm;
+class Block;
+
 struct StepContext {
   Kernels* kernels = nullptr;
   int num_tokens = 0, num_seqs = 0;
@@ -66,6 +69,13 @@ struct StepContext {
   std::map<std::string, Tensor> carry;               // what a part leaves for later parts of the same step (empty at its start)
   HeadColumns first_values;                          // the values that the step's first layer that mixes values projected
   std::function<Tensor(int64_t)> workspace;           // float32 scratch of at least that many elements
+  // The layer that the model runs, and the norms that the layer after it takes of the stream it is handed (null: none, or not said).  What the
+  // running layer's last launch took of the stream left_of by those norms is there for the next layer, which finds it when they are its own norms
+  // of the very stream that it is handed.  A block that another one runs inside itself (`running` is not it) neither leaves nor finds anything.
+  Block* running = nullptr;
+  std::pair<Norm*, Norm*> following, left_by;
+  std::pair<Tensor, Tensor> left_normed;
+  Tensor left_of;
 };
 
 // What a mixer keeps between steps.
@@ -123,6 +133,9 @@ class Norm : public Part {
   // A norm that is y = x * rsqrt(mean(x^2) + eps) * w says so; a mixer may then run it inside a launch of its own.
   virtual const Tensor* row_scale_weight() const { return nullptr; }
   virtual float eps() const { return 0.f; }
+  // A norm whose forward() on a 32-bit stream is y = x * rsqrt(mean(x^2) + eps) * (offset + w), in the order of the stream's kernels, says so; a block
+  // may then run it inside a launch of its own.
+  virtual Kernels::RowNorm stream_norm() const { return {}; }
   // out = base + mult * norm(y) on a residual stream that is kept in 32-bit; out may be base.  rounded (or null): elements of
   // out's shape that receive the new rows rounded, for a sublayer that reads the stream as it is.
   virtual void forward_scaled_add(const Tensor& y, const Tensor& base, Tensor& out, float mult, Tensor* rounded = nullptr);
@@ -168,11 +181,20 @@ class Block : public Part {
  public:
   using Part::Part;
   virtual Mixer& mixer() = 0;
+  // The norms that forward() takes of the stream it is handed (a second one where both sublayers read it), for the layer before
+  // (StepContext::following); by default none is named.
+  virtual std::pair<Norm*, Norm*> input_norms() { return {nullptr, nullptr}; }
   // (hidden, residual) -> (hidden, residual); `residual` has no memory before the first layer.
   virtual std::pair<Tensor, Tensor> forward(const Tensor& hidden, Tensor residual, StepContext& ctx, CacheEntry& cache) = 0;
   // The rows of (hidden, residual) that the model's end reads, asked of the last layer that ran.  An arrangement that keeps
   // the stream in another form between layers brings it into the form of the final norm here.
   virtual std::pair<Tensor, Tensor> rows_for_the_end(const Tensor& hidden, const Tensor& residual, StepContext& ctx, const Tensor& rows);
+
+ protected:
+  // What the layer before left of this stream, if these are the norms it took; empty tensors otherwise.  Nothing is left for anyone after that.
+  std::pair<Tensor, Tensor> take_left(StepContext& ctx, const Tensor& hidden, Norm* first, Norm* second) const;
+  std::pair<Norm*, Norm*> following(const StepContext& ctx) const { return ctx.running == this ? ctx.following : std::pair<Norm*, Norm*>(nullptr, nullptr); }
+  void leave(StepContext& ctx, const Tensor& stream, std::pair<Tensor, Tensor> normed) const;
 };
 
 using PartFactory = std::function<std::unique_ptr<Part>(const PartSpec&, Kernels&)>;

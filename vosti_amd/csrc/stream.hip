@@ -232,6 +232,135 @@ __global__ __launch_bounds__(STREAM_THREADS) void stream_add_norm_vec_kernel(ele
   }
 }
 
+// A row of what follows a sublayer in one launch: o = base + mult * norm(y) (out, which may be base), with MIX the weighted sum
+// m = sum over j < n of coef[j] * states[j] whose last state is o (mixed), and the next sublayer's norm of o or m as elements (normed).
+// The sums and their orders are those of stream_norm_add_vec_kernel, stream_mix_vec_kernel and stream_norm_vec_kernel, so the bits are.
+// A few rows are latency: two or three launches of 2 us become one (a decode step of the 1,024-wide Tezinex shape, two rows: 453 -> 420 us); many are
+// bytes: the row stays in registers between the norms instead of going to memory and back twice.
+template <int NV, bool MIX, typename Y>
+__global__ __launch_bounds__(STREAM_THREADS) void stream_norm_step_kernel(float* out, const float* base_rows, const Y* __restrict__ y,
+                                                                          const void* __restrict__ w, int w_is_f32, int H, float eps, float offset,
+                                                                          float mult, float* __restrict__ mixed, const float* states, int64_t stride,
+                                                                          const void* __restrict__ coef, int coef_is_f32, int n,
+                                                                          elem_t* __restrict__ normed, const void* __restrict__ w2, int w2_is_f32,
+                                                                          float eps2, float offset2) {
+  __shared__ float red[4], red2[4];
+  const int64_t base = (int64_t)blockIdx.x * H;
+  const int nvec = H / 4;
+  f32x4 v[NV], b[NV], m[NV];
+  float part = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = threadIdx.x + j * STREAM_THREADS;
+    v[j] = b[j] = m[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c < nvec) {
+      if constexpr (sizeof(Y) == 4) v[j] = *reinterpret_cast<const f32x4*>(y + base + 4 * c);
+      else v[j] = load_elems4(y + base + 4 * c);
+      b[j] = *reinterpret_cast<const f32x4*>(base_rows + base + 4 * c);
+    }
+    part = part + v[j].x * v[j].x;
+    part = part + v[j].y * v[j].y;
+    part = part + v[j].z * v[j].z;
+    part = part + v[j].w * v[j].w;
+  }
+  if (MIX) {                         // the earlier states do not wait for the norm
+    for (int i = 0; i + 1 < n; ++i) {
+      const float ci = load_weight(coef, coef_is_f32, i);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const int c = threadIdx.x + j * STREAM_THREADS;
+        if (c < nvec) {
+          const f32x4 u = *reinterpret_cast<const f32x4*>(states + i * stride + base + 4 * c);
+          m[j].x = m[j].x + ci * u.x;
+          m[j].y = m[j].y + ci * u.y;
+          m[j].z = m[j].z + ci * u.z;
+          m[j].w = m[j].w + ci * u.w;
+        }
+      }
+    }
+  }
+  const float rr = rsqrtf(stream_block_sum(part, red) / (float)H + eps);
+  const float last = MIX ? load_weight(coef, coef_is_f32, n - 1) : 0.f;
+  part = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = threadIdx.x + j * STREAM_THREADS;
+    if (c < nvec) {
+      f32x4 o;
+      o.x = b[j].x + mult * ((v[j].x * rr) * (offset + load_weight(w, w_is_f32, 4 * c)));
+      o.y = b[j].y + mult * ((v[j].y * rr) * (offset + load_weight(w, w_is_f32, 4 * c + 1)));
+      o.z = b[j].z + mult * ((v[j].z * rr) * (offset + load_weight(w, w_is_f32, 4 * c + 2)));
+      o.w = b[j].w + mult * ((v[j].w * rr) * (offset + load_weight(w, w_is_f32, 4 * c + 3)));
+      *reinterpret_cast<f32x4*>(out + base + 4 * c) = o;
+      if (MIX) {
+        m[j].x = m[j].x + last * o.x;
+        m[j].y = m[j].y + last * o.y;
+        m[j].z = m[j].z + last * o.z;
+        m[j].w = m[j].w + last * o.w;
+        *reinterpret_cast<f32x4*>(mixed + base + 4 * c) = m[j];
+      } else {
+        m[j] = o;
+      }
+    }
+    part = part + m[j].x * m[j].x;
+    part = part + m[j].y * m[j].y;
+    part = part + m[j].z * m[j].z;
+    part = part + m[j].w * m[j].w;
+  }
+  const float rr2 = rsqrtf(stream_block_sum(part, red2) / (float)H + eps2);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = threadIdx.x + j * STREAM_THREADS;
+    if (c < nvec)
+      store_elems4(normed + base + 4 * c, f32x4{(m[j].x * rr2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c)), (m[j].y * rr2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 1)),
+                                                (m[j].z * rr2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 2)), (m[j].w * rr2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 3))});
+  }
+}
+
+// x <- x + (a + b) (rows of floats) and two norms of the new row as elements, each with its own weight and eps, in one launch: stream_add_kernel's sum,
+// stream_norm_vec_kernel's norms.
+template <int NV>
+__global__ __launch_bounds__(STREAM_THREADS) void stream_sum_norms_kernel(float* __restrict__ x, const float* __restrict__ a, const float* __restrict__ b, int H,
+                                                                          elem_t* __restrict__ out1, const void* __restrict__ w1, int w1_is_f32, float eps1,
+                                                                          float offset1, elem_t* __restrict__ out2, const void* __restrict__ w2, int w2_is_f32,
+                                                                          float eps2, float offset2) {
+  __shared__ float red[4];
+  const int64_t base = (int64_t)blockIdx.x * H;
+  const int nvec = H / 4;
+  f32x4 v[NV];
+  float part = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = threadIdx.x + j * STREAM_THREADS;
+    v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c < nvec) {
+      const f32x4 p = *reinterpret_cast<const f32x4*>(a + base + 4 * c), q = *reinterpret_cast<const f32x4*>(b + base + 4 * c);
+      const f32x4 r = *reinterpret_cast<const f32x4*>(x + base + 4 * c);
+      v[j].x = r.x + (p.x + q.x);
+      v[j].y = r.y + (p.y + q.y);
+      v[j].z = r.z + (p.z + q.z);
+      v[j].w = r.w + (p.w + q.w);
+      *reinterpret_cast<f32x4*>(x + base + 4 * c) = v[j];
+    }
+    part = part + v[j].x * v[j].x;
+    part = part + v[j].y * v[j].y;
+    part = part + v[j].z * v[j].z;
+    part = part + v[j].w * v[j].w;
+  }
+  const float mean = stream_block_sum(part, red) / (float)H;
+  const float r1 = rsqrtf(mean + eps1), r2 = rsqrtf(mean + eps2);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = threadIdx.x + j * STREAM_THREADS;
+    if (c < nvec) {
+      store_elems4(out1 + base + 4 * c, f32x4{(v[j].x * r1) * (offset1 + load_weight(w1, w1_is_f32, 4 * c)), (v[j].y * r1) * (offset1 + load_weight(w1, w1_is_f32, 4 * c + 1)),
+                                              (v[j].z * r1) * (offset1 + load_weight(w1, w1_is_f32, 4 * c + 2)), (v[j].w * r1) * (offset1 + load_weight(w1, w1_is_f32, 4 * c + 3))});
+      store_elems4(out2 + base + 4 * c, f32x4{(v[j].x * r2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c)), (v[j].y * r2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 1)),
+                                              (v[j].z * r2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 2)), (v[j].w * r2) * (offset2 + load_weight(w2, w2_is_f32, 4 * c + 3))});
+    }
+  }
+}
+
 // out[e] = sum over j < n of coef[j] * states[j * stride + e], added in ascending j from zero.
 __global__ __launch_bounds__(256) void stream_mix_kernel(float* __restrict__ out, const float* __restrict__ states, int64_t stride,
                                                          const void* __restrict__ coef, int coef_is_f32, int n, int64_t numel) {
@@ -507,6 +636,58 @@ int vk_stream_mix(float* out, const float* states, int64_t stride, const void* c
   else
     stream_mix_kernel<<<(unsigned)((numel + 255) / 256), 256, 0, st>>>(out, states, stride, coef, coef_is_f32, n, numel);
   return vk_check_launch("stream mix");
+}
+
+// 1 if rows of H fit the launches below (whole vectors, in the registers of a workgroup).
+int vk_stream_step_takes(int H) { return H > 0 && H % 4 == 0 && H <= 4 * STREAM_THREADS * 8; }
+
+extern "C++" {
+template <bool MIX, typename Y>
+static int norm_step_launch(float* out, const float* base, const Y* y, const void* w, int w_is_f32, int rows, int H, float eps, float offset, float mult, float* mixed,
+                            const float* states, int64_t stride, const void* coef, int coef_is_f32, int n, elem_t* normed, const void* w2, int w2_is_f32,
+                            float eps2, float offset2, hipStream_t st) {
+  const int nv = (H / 4 + STREAM_THREADS - 1) / STREAM_THREADS;
+#define NORM_STEP(NV)                                                                                                                                     \
+  stream_norm_step_kernel<NV, MIX, Y><<<rows, STREAM_THREADS, 0, st>>>(out, base, y, w, w_is_f32, H, eps, offset, mult, mixed, states, stride, coef,   \
+                                                                       coef_is_f32, n, normed, w2, w2_is_f32, eps2, offset2)
+  if (nv <= 1) NORM_STEP(1); else if (nv <= 2) NORM_STEP(2); else if (nv <= 4) NORM_STEP(4); else NORM_STEP(8);
+#undef NORM_STEP
+  return vk_check_launch("stream norm-step");
+}
+}  // extern "C++"
+
+// out = base + mult * norm(y); mixed (or null: no sum) = sum over j < n of coef[j] * state j, states `stride` floats apart, the last of them out; normed = the
+// second norm of mixed, or of out.  y: elements, or floats with y_is_f32.
+int vk_stream_norm_step(float* out, const float* base, const void* y, int y_is_f32, const void* w, int w_is_f32, int rows, int H, float eps, float offset, float mult,
+                        float* mixed, const float* states, int64_t stride, const void* coef, int coef_is_f32, int n, elem_t* normed, const void* w2, int w2_is_f32,
+                        float eps2, float offset2, hipStream_t st) {
+  VK_REQUIRE(rows >= 0 && vk_stream_step_takes(H) && eps >= 0.f && eps2 >= 0.f, "stream norm-step: bad sizes rows=%d H=%d", rows, H);
+  VK_REQUIRE(mixed == nullptr || (n > 0 && stride >= (int64_t)rows * H && stride % 4 == 0 && states != nullptr && coef != nullptr && out == states + (n - 1) * stride),
+             "stream norm-step: the new rows must be the last of the %d states", n);
+  VK_REQUIRE((uintptr_t)out % 16 == 0 && (uintptr_t)base % 16 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)mixed % 16 == 0 && (uintptr_t)states % 16 == 0 && (uintptr_t)normed % 16 == 0,
+             "stream norm-step: rows must be 16-byte aligned");
+  if (rows == 0) return 0;
+#define STEP_OF(MIX, Y)                                                                                                                                       \
+  norm_step_launch<MIX, Y>(out, base, static_cast<const Y*>(y), w, w_is_f32, rows, H, eps, offset, mult, mixed, states, stride, coef, coef_is_f32, n, normed, w2, \
+                           w2_is_f32, eps2, offset2, st)
+  if (mixed) return y_is_f32 ? STEP_OF(true, float) : STEP_OF(true, elem_t);
+  return y_is_f32 ? STEP_OF(false, float) : STEP_OF(false, elem_t);
+#undef STEP_OF
+}
+
+// x [rows, H] floats <- x + (a + b), floats; out1 and out2 = the two norms of the new rows.
+int vk_stream_sum_norms(float* x, const float* a, const float* b, int rows, int H, elem_t* out1, const void* w1, int w1_is_f32, float eps1, float offset1, elem_t* out2,
+                        const void* w2, int w2_is_f32, float eps2, float offset2, hipStream_t st) {
+  VK_REQUIRE(rows >= 0 && vk_stream_step_takes(H) && eps1 >= 0.f && eps2 >= 0.f, "stream sum-norms: bad sizes rows=%d H=%d", rows, H);
+  VK_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)b % 16 == 0 && (uintptr_t)out1 % 16 == 0 && (uintptr_t)out2 % 16 == 0,
+             "stream sum-norms: rows must be 16-byte aligned");
+  if (rows == 0) return 0;
+  const int nv = (H / 4 + STREAM_THREADS - 1) / STREAM_THREADS;
+#define SUM_NORMS(NV) \
+  stream_sum_norms_kernel<NV><<<rows, STREAM_THREADS, 0, st>>>(x, a, b, H, out1, w1, w1_is_f32, eps1, offset1, out2, w2, w2_is_f32, eps2, offset2)
+  if (nv <= 1) SUM_NORMS(1); else if (nv <= 2) SUM_NORMS(2); else if (nv <= 4) SUM_NORMS(4); else SUM_NORMS(8);
+#undef SUM_NORMS
+  return vk_check_launch("stream sum-norms");
 }
 
 int vk_gather_rows_f32(float* out, const float* x, const int32_t* rows, int R, int H, hipStream_t st) {
