@@ -1,0 +1,32 @@
+"""Products of up to 16 rows whose activations come through LDS: the bits of the tile kernel."""
+import pytest
+import torch
+from test_kernels_gpu import DTYPES, kern, rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("chunks", [1, 2, 3, 5, 6, 8, 9, 10, 12, 13, 19])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 7, 8, 9, 15, 16])
+def test_rows_and_chunks(M, chunks, dtype):
+    """One row to 16, waves with a chunk, with several and without one, weight rows that end inside a tile, more tiles than workgroups; rows further
+    apart than they are long."""
+    k = kern(dtype)
+    K = 512 * chunks
+    x = rand((M, K + 32), dtype, 1).cuda()[:, :K]
+    for N in (9, 300, 4200 if chunks > 3 else 17000):
+        w = rand((N, K), dtype, 2, 0.1).cuda()
+        assert torch.equal(k.gemm(x, w), k.gemm(x, w, kernel=4)), N
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("chunks", [1, 2, 4, 5, 6, 8])
+@pytest.mark.parametrize("M", [1, 3, 8, 9, 16])
+def test_gate_and_up(M, chunks, dtype):
+    k = kern(dtype)
+    K = 512 * chunks
+    x = rand((M, K), dtype, 3).cuda()
+    for I in (24, 4200):
+        w = rand((2 * I, K), dtype, 4, 0.1).cuda()
+        assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4)))

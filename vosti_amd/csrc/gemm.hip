@@ -75,6 +75,51 @@ __device__ __forceinline__ void store_out4(elem_t* out, int64_t ldo, int m, int 
   }
 }
 
+// 16 bytes per lane from global memory into LDS at lds_addr + 16 * lane, the address in two parts: a base held in scalar registers, the same for every lane, and a
+// 32-bit offset per lane.  The compiler's own form of it adds base and offset in vector registers before every
+// load (it moves what does not change along K out of the loop and is left with a vector sum); written out, the
+// advancing base costs two scalar additions per K tile for all loads together.  lds_addr: the wave's 1 KB
+// block, anywhere in LDS (the grouped product's third stage starts at 96 KB).
+__device__ __forceinline__ void pipe_load_to_lds16_sv(const unsigned char* sbase, unsigned voff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");     // m0 is the compiler's scratch: it sets it anew before every use of its own
+}
+__device__ __forceinline__ unsigned lds_offset_of(const unsigned char* p) {
+  return (unsigned)(unsigned long)((__attribute__((address_space(3))) const void*)p);
+}
+
+template <int N_>
+__device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ below 64; the other counters at their maxima
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N_ & 0xF) | ((N_ >> 4) << 14));
+}
+
+
+// Up to 16 rows (HALVES: 8 or 16) of one chunk's activations as a wave's fragments, through LDS of the wave's own (HALVES * CHUNK_HALF_BYTES).
+// The fragments' own addresses put four rows side by side in four neighbouring lanes, so that a load takes the address unit 64 clocks
+// where whole lines take 16: the activations cost a launch of a few weight tiles a workgroup as much of that unit as its weights.  Here a load
+// brings eight rows of 128 bytes.  Measured on MI355X, recorded launches with the weights of several layers in turn, us: 4,096 x 4,096,
+// 1, 8 and 16 rows 8.9 -> 8.1, 9.2 -> 8.5, 10.8 -> 9.4; 6,144 x 4,096, 8 rows 14.2 -> 13.2; 2,048 x 6,144,
+// 8 rows 11.6 -> 9.6; 1,024 x 3,072, 1 row 5.7 -> 5.4; gate/up with SwiGLU 12,288 x 4,096, 8 rows 37.7 -> 37.0.  Over 228 sizes of
+// 1 to 16 rows 3,439 -> 3,296 us, the slowest 5 % over what it was (1,536 x 1,024, 1 row: 3.25 -> 3.44).  (Weights through LDS alike do not pay: they come from
+// memory, 7.1 us for 33 MB against 7.4.  Tiles of eight or four weight rows for few of them do not either: 1,024 x 2,048 4.4 -> 4.6.)
+#define CHUNK_PAIRS (KC_SLABS / 2)                                // pairs of slabs: 128 bytes of a row
+#define CHUNK_HALF_BYTES (CHUNK_PAIRS * 1024)                     // eight rows of a chunk
+template <int HALVES>
+__device__ __forceinline__ void ask_chunk_rows(const elem_t* act, int64_t lda, int M, int lane, unsigned lds_addr) {      // HALVES * CHUNK_PAIRS loads
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h) {
+    const unsigned voff = (unsigned)((min(h * 8 + lr, M - 1) * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+#pragma unroll
+    for (int i = 0; i < CHUNK_PAIRS; ++i)
+      pipe_load_to_lds16_sv(reinterpret_cast<const unsigned char*>(act) + i * 128, voff, __builtin_amdgcn_readfirstlane(lds_addr + (h * CHUNK_PAIRS + i) * 1024));
+  }
+}
+template <int HALVES>
+__device__ __forceinline__ frag_t chunk_fragment(const unsigned char* rows, int slab, int r16, int kg) {      // with 8 rows the others repeat them
+  const int r = r16 & 7, h = HALVES == 2 ? r16 >> 3 : 0;
+  return *reinterpret_cast<const frag_t*>(rows + (h * CHUNK_PAIRS + (slab >> 1)) * 1024 + r * 128 + ((((slab & 1) * 4 + kg) ^ r) * 16));
+}
+
 // ------------------------------------------------------------------ skinny
 // MT: 16-row activation tiles (M <= 16*MT).  W: slabs in flight per wave.
 template <int MT, int W>
@@ -162,7 +207,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(elem_t* __re
 // a loaded value makes the compiler wait for it at once; and with RC > 0 a wave
 // keeps the activations of its RC chunks (K <= RC * 4096) in registers for the
 // whole kernel.  One barrier per round of eight chunks.
-template <int MT, int W, int RC, int NT, int NW = SK_WAVES>
+// HALVES: 1 or 2: the resident activations (one tile) come through LDS, 8 or 16 rows; 0: straight to their registers.
+template <int MT, int W, int RC, int NT, int NW = SK_WAVES, int HALVES = 0>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict__ out,
                                                                     const elem_t* __restrict__ act,
                                                                     const elem_t* __restrict__ w, int M, int N, int K,
@@ -178,17 +224,22 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
   static_assert(NT * MT <= NW, "one wave adds up each output tile");
   __shared__ f32x4 part[2][NW][NT * MT][64];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  static_assert(HALVES == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // HALVES * CHUNK_HALF_BYTES a wave
+
+  const int lane = threadIdx.x & 63, wave = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int nchunks = K / KC;
   const int ntiles = (N + 16 * NT - 1) / (16 * NT);     // tile: NT * 16 weight rows
+  unsigned char* own_rows = rows_lds + wave * (HALVES * CHUNK_HALF_BYTES);
+  if constexpr (HALVES > 0) ask_chunk_rows<HALVES>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
 
   const elem_t* arow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) arow[mt] = act + (int64_t)min(mt * 16 + r16, M - 1) * lda + kg * VK_VEC;
 
   frag_t wbuf[W][NT], abuf[RES ? RC * KC_SLABS : W][MT];
-  if (RES) {
+  if (RES && HALVES == 0) {
 #pragma unroll
     for (int r = 0; r < RC; ++r) {
       const int c = min(r * NW + wave, nchunks - 1);     // beyond K: the last chunk again (not used)
@@ -214,6 +265,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
   if (tile < ntiles && wave < nchunks) {
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, wave, i, i);
+  }
+  if constexpr (HALVES > 0) {
+    if (wave < nchunks) {                                // a wave with a chunk has a tile: there are no more workgroups than tiles
+      __builtin_amdgcn_sched_barrier(0);                 // the weights' loads stay in front of the wait that counts them
+      wait_vmcnt_n<W * NT>();                            // the rows are there, the first weights on their way
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = chunk_fragment<HALVES>(own_rows, i, r16, kg);
+    } else {
+      wait_vmcnt_n<0>();
+    }
   }
   int parity = 0;
   for (; tile < ntiles; tile += gridDim.x) {
@@ -282,7 +345,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 // two projections rounded to the element type first, which is what the separate
 // GEMM and SwiGLU kernels compute (kernels/triton_kernels/silu_mul.py:64-87).
 // M <= 16, K <= 4096 (activations resident in registers).
-template <int W, int MT, int RC, int NW = SK_WAVES>
+template <int W, int MT, int RC, int NW = SK_WAVES, int HALVES = 0>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __restrict__ out,
                                                                            const elem_t* __restrict__ act,
                                                                            const elem_t* __restrict__ w, int M, int I,
@@ -292,15 +355,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   static_assert(MT * RC <= 2, "two chunk tiles of activations stay in registers: two tiles of a chunk or two chunks of a tile");
   __shared__ f32x4 part[2][RC][NW][2 * MT][64];      // two sets, used in turn: one barrier per tile
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  static_assert(HALVES == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // HALVES * CHUNK_HALF_BYTES a wave
+  const int lane = threadIdx.x & 63, wave = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int nchunks = K / KC;
   const int ntiles = (I + 15) / 16;
+  unsigned char* own_rows = rows_lds + wave * (HALVES * CHUNK_HALF_BYTES);
+  if constexpr (HALVES > 0) ask_chunk_rows<HALVES>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
 
   // Wave w has chunks w, w + 8, ...: RC of them (chunks beyond K are read as the last and not used).
   frag_t wg[W], wu[W], abuf[RC * KC_SLABS][MT];
 #pragma unroll
-  for (int r = 0; r < RC; ++r) {
+  for (int r = 0; r < (HALVES ? 0 : RC); ++r) {
     const int c = min(r * NW + wave, nchunks - 1);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -326,6 +393,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   if (tile < ntiles && active) {
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, i, i);
+  }
+  if constexpr (HALVES > 0) {
+    if (active) {                                        // as in the kernel above
+      __builtin_amdgcn_sched_barrier(0);
+      wait_vmcnt_n<2 * W>();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = chunk_fragment<HALVES>(own_rows, i, r16, kg);
+    } else {
+      wait_vmcnt_n<0>();
+    }
   }
   int parity = 0;
   for (; tile < ntiles; tile += gridDim.x) {
@@ -531,18 +610,6 @@ __device__ __forceinline__ void pipe_load_to_lds16(const elem_t* src, unsigned c
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-// The same load with its address in two parts: a base held in scalar registers, the same for every lane, and a
-// 32-bit offset per lane.  The compiler's own form of it adds base and offset in vector registers before every
-// load (it moves what does not change along K out of the loop and is left with a vector sum); written out, the
-// advancing base costs two scalar additions per K tile for all loads together.  lds_addr: the wave's 1 KB
-// block, anywhere in LDS (the grouped product's third stage starts at 96 KB).
-__device__ __forceinline__ void pipe_load_to_lds16_sv(const unsigned char* sbase, unsigned voff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");     // m0 is the compiler's scratch: it sets it anew before every use of its own
-}
-__device__ __forceinline__ unsigned lds_offset_of(const unsigned char* p) {
-  return (unsigned)(unsigned long)((__attribute__((address_space(3))) const void*)p);
-}
-
 // FNW: 16-row weight fragments per wave, 2 to 5: a workgroup takes 32 FNW weight rows.  4 is the square tile; 2
 // gives twice the workgroups, for grids that would leave compute units with one workgroup or none; 3 and 5 are
 // for grids whose last round of workgroups would otherwise run nearly empty (pipe_fragments_by_rounds).  Six
@@ -553,11 +620,6 @@ __device__ __forceinline__ unsigned lds_offset_of(const unsigned char* p) {
 __device__ __forceinline__ void pipe_touch_line(const unsigned char* sbase, unsigned voff, unsigned& keep) {
   asm volatile("global_load_dword %0, %1, %2 sc1" : "+v"(keep) : "v"(voff), "s"(sbase) : "memory");
 }
-template <int N_>
-__device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ below 64; the other counters at their maxima
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N_ & 0xF) | ((N_ >> 4) << 14));
-}
-
 // PFD > 0: every wave touches, PFD tiles ahead, the 64 rows of the workgroup's tiles that are its share.
 // NWN: waves along the weight rows, two of a workgroup of four waves or four of eight, which takes 64 FNW weight rows.
 // GROUPED: block_weights, row_pair and act_row count.
@@ -1420,6 +1482,15 @@ static int stream_waves(int nchunks) {
   return 8;
 }
 
+// How a streaming kernel of `waves` waves with a chunk each brings in the activations of M rows: through LDS as 8 rows (1) or 16 (2) a wave, or
+// straight to registers (0) where that does not fit beside the chunk sums (sums_bytes).  In 32-bit, 16 rows through LDS leave room
+// for fewer workgroups, which only launches of one weight tile a workgroup do not miss (151,936 x 1,024: 128 -> 165 us; 1,024 x 2,048: 11.6 -> 9.5).
+static constexpr int stream_row_halves(int M, int waves, int sums_bytes) {
+  const int halves = M > 8 ? 2 : 1;
+  return halves * waves * CHUNK_HALF_BYTES + sums_bytes <= 160 * 1024 ? halves : 0;
+}
+static bool stream_rows_pay(int M, int weight_tiles) { return M <= 8 || sizeof(elem_t) == 2 || weight_tiles <= vk_device_cus(); }
+
 // Which kernel computes a product (speed only: all give the same bits).  Every threshold is a count of
 // workgroups against the device's compute units (cus), or a count of 16-row activation tiles, or whether a
 // wave's share of K fits its registers; none is a model's size.  With the workgroups a kernel would start:
@@ -1641,20 +1712,32 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     const int mt = (M + 15) / 16;
     const unsigned grid = (unsigned)((N + 15) / 16);
     if (K % KC == 0) {
-#define STW(MT, W, RC, NT, NW)                                                                            \
+#define STH(MT, W, RC, NT, NW, HALVES)                                                                    \
   do {                                                                                                    \
+    constexpr size_t rows_bytes = (size_t)(HALVES) * NW * CHUNK_HALF_BYTES;                               \
     static int resident = 0; /* workgroups of this kernel that the device holds at once */               \
     if (resident == 0) {                                                                                  \
       int dev = 0, cus = 0, per_cu = 0;                                                                   \
       (void)hipGetDevice(&dev);                                                                           \
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);                      \
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_kernel<MT, W, RC, NT, NW>,  \
-                                                         64 * NW, 0);                                     \
+      if (rows_bytes)                                                                                     \
+        (void)hipFuncSetAttribute((const void*)gemm_stream_kernel<MT, W, RC, NT, NW, HALVES>,             \
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_bytes);           \
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_kernel<MT, W, RC, NT, NW, HALVES>, \
+                                                         64 * NW, rows_bytes);                            \
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                       \
     }                                                                                                     \
     const unsigned groups = (unsigned)((N + 16 * NT - 1) / (16 * NT));                                    \
-    gemm_stream_kernel<MT, W, RC, NT, NW><<<groups < (unsigned)resident ? groups : (unsigned)resident,    \
-                                             64 * NW, 0, st>>>(out, act, w, M, N, K, lda, ldo, form);   \
+    gemm_stream_kernel<MT, W, RC, NT, NW, HALVES><<<groups < (unsigned)resident ? groups : (unsigned)resident, \
+                                             64 * NW, rows_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form); \
+  } while (0)
+#define STW(MT, W, RC, NT, NW) STH(MT, W, RC, NT, NW, 0)
+#define STN(NW)                                                                                           \
+  do {                                                                                                    \
+    const int halves = stream_rows_pay(M, (N + 15) / 16) ? stream_row_halves(M, NW, NW * 2048) : 0;       \
+    if (halves == 2) STH(1, 8, 1, 1, NW, stream_row_halves(16, NW, NW * 2048));                           \
+    else if (halves == 1) STH(1, 8, 1, 1, NW, stream_row_halves(8, NW, NW * 2048));                       \
+    else STH(1, 8, 1, 1, NW, 0);                                                                          \
   } while (0)
 #define ST(MT, W, RC, NT) STW(MT, W, RC, NT, SK_WAVES)
       if (mt == 1) {
@@ -1666,16 +1749,17 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
         // One chunk a wave, its activations in registers, wherever a workgroup can have as many waves as K has
         // chunks (stream_waves): no wave then waits at the round's barrier for one that has a second chunk.
         const int nw = kernel == 7 ? SK_WAVES : stream_waves(K / KC);
-        if (nw == 2) STW(1, 8, 1, 1, 2);
-        else if (nw == 4) STW(1, 8, 1, 1, 4);
-        else if (nw == 5) STW(1, 8, 1, 1, 5);
-        else if (nw == 6) STW(1, 8, 1, 1, 6);
+        if (nw == 2) STN(2);
+        else if (nw == 4) STN(4);
+        else if (nw == 5) STN(5);
+        else if (nw == 6) STN(6);
 #ifdef VK_BF16
-        else if (nw == 10) STW(1, 8, 1, 1, 10);
-        else if (nw == 12) STW(1, 8, 1, 1, 12);
+        else if (nw == 10) STN(10);
+        else if (nw == 12) STN(12);
 #endif
         else
         if (kernel == 7 || (by_size && K > SK_WAVES * KC && tiles16 > cus && 2 * tiles16 <= 3 * cus)) ST(1, 8, 0, 2);
+        else if (K <= SK_WAVES * KC && kernel != 7) STN(SK_WAVES);
         else if (K <= SK_WAVES * KC) ST(1, 8, 1, 1);
 #ifdef VK_BF16
         // Two chunks a wave are 128 registers of activations (16 rows, 34816 x 5120: 118 -> 87 us);
@@ -1695,7 +1779,9 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
       else if (mt == 3) { if (kernel == 7) ST(3, 4, 0, 2); else ST(3, 4, 0, 1); }
       else { if (kernel == 7) ST(4, 4, 0, 2); else ST(4, 4, 0, 1); }
 #undef ST
+#undef STN
 #undef STW
+#undef STH
       return vk_check_launch("gemm_stream");
     }
 #define SK(MT, W) gemm_skinny_kernel<MT, W><<<grid, 64 * SK_WAVES, 0, st>>>(out, act, w, M, N, K, lda, ldo, form)
@@ -1801,29 +1887,40 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   }
   const int ntiles = (I + 15) / 16;
   const int form = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
-#define SWIGLU_STREAMW(W, MT, RC, NW)                                                                       \
+#define SWIGLU_STREAMH(W, MT, RC, NW, HALVES)                                                               \
   do {                                                                                                     \
+    constexpr size_t rows_bytes = (size_t)(HALVES) * NW * CHUNK_HALF_BYTES;                                \
     static int resident = 0;                                                                               \
     if (resident == 0) {                                                                                   \
       int dev = 0, cus = 0, per_cu = 0;                                                                    \
       (void)hipGetDevice(&dev);                                                                            \
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);                       \
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, MT, RC, NW>, \
-                                                         64 * NW, 0);                                      \
+      if (rows_bytes)                                                                                      \
+        (void)hipFuncSetAttribute((const void*)gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES>,           \
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_bytes);            \
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES>, \
+                                                         64 * NW, rows_bytes);                             \
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                        \
     }                                                                                                      \
-    gemm_stream_swiglu_kernel<W, MT, RC, NW><<<ntiles < resident ? ntiles : resident, 64 * NW, 0, st>>>(   \
+    gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
         out, act, w, M, I, K, lda, ldo, form);                                                           \
   } while (0)
-#define SWIGLU_STREAM(W, MT, RC) SWIGLU_STREAMW(W, MT, RC, SK_WAVES)
+#define SWIGLU_STREAM(W, MT, RC) SWIGLU_STREAMH(W, MT, RC, SK_WAVES, 0)
+#define SWIGLU_STREAMN(NW)                                                                                 \
+  do {                                                                                                     \
+    const int halves = stream_rows_pay(M, ntiles) ? stream_row_halves(M, NW, NW * 4096) : 0;               \
+    if (halves == 2) SWIGLU_STREAMH(8, 1, 1, NW, stream_row_halves(16, NW, NW * 4096));                    \
+    else if (halves == 1) SWIGLU_STREAMH(8, 1, 1, NW, stream_row_halves(8, NW, NW * 4096));                \
+    else SWIGLU_STREAMH(8, 1, 1, NW, 0);                                                                   \
+  } while (0)
   const int nw = M <= 16 ? stream_waves(K / KC) : SK_WAVES;       // as in vk_gemm
-  if (nw == 2) SWIGLU_STREAMW(8, 1, 1, 2);
-  else if (nw == 4) SWIGLU_STREAMW(8, 1, 1, 4);
-  else if (nw == 5) SWIGLU_STREAMW(8, 1, 1, 5);
-  else if (nw == 6) SWIGLU_STREAMW(8, 1, 1, 6);
+  if (nw == 2) SWIGLU_STREAMN(2);
+  else if (nw == 4) SWIGLU_STREAMN(4);
+  else if (nw == 5) SWIGLU_STREAMN(5);
+  else if (nw == 6) SWIGLU_STREAMN(6);
 #ifdef VK_BF16
-  else if (nw == 10) SWIGLU_STREAMW(8, 1, 1, 10);
-  else if (nw == 12) SWIGLU_STREAMW(8, 1, 1, 12);
+  else if (nw == 10) SWIGLU_STREAMH(8, 1, 1, 10, 0);       // ten waves with the rows in LDS: 17,408 x 5,120 77.5 -> 79.9 us at 8 rows
+  else if (nw == 12) SWIGLU_STREAMH(8, 1, 1, 12, 0);
 #endif
   else
 #ifdef VK_BF16
@@ -1831,9 +1928,10 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   else if (K > SK_WAVES * KC) SWIGLU_STREAM(4, 1, 2);
   else
 #endif
-    SWIGLU_STREAM(8, 1, 1);
+    SWIGLU_STREAMN(SK_WAVES);
+#undef SWIGLU_STREAMN
+#undef SWIGLU_STREAMH
 #undef SWIGLU_STREAM
-#undef SWIGLU_STREAMW
   return vk_check_launch("gemm_swiglu");
 }
 
