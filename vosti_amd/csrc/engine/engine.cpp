@@ -74,6 +74,8 @@ Engine::Engine(const EngineOptions& opt) {
   sample_rows_ = opt.max_num_seqs;
   hip_check(hipHostMalloc(reinterpret_cast<void**>(&sample_in_), 2 * sample_rows_ * sizeof(float), hipHostMallocDefault), "pinned allocation");
   hip_check(hipHostMalloc(reinterpret_cast<void**>(&sample_out_), sample_rows_ * sizeof(int32_t), hipHostMallocDefault), "pinned allocation");
+  for (hipEvent_t& e : read_done_) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event creation");
+  hip_check(hipHostMalloc(reinterpret_cast<void**>(&read_places_), kReadPlaces * kReadBytes, hipHostMallocDefault), "pinned allocation");
   // [temperatures | uniform numbers | token ids | the sampler's scratch]
   sample_dev_ = std::make_unique<DeviceBuffer>(3 * sample_stride() + (size_t)kernels_->sample_scratch_words(sample_rows_) * 4);
 }
@@ -113,13 +115,8 @@ void Engine::read_logits(const Tensor& logits, float* out) {
   if (logits.dtype != type) throw EngineError("logits of " + logits.describe() + " cannot be read back");
   const size_t total = (size_t)logits.numel(), size = dtype_bytes(type);
   if (!total) return;
-  for (hipEvent_t& e : read_done_)
-    if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event creation");
-  if (!read_places_) hip_check(hipHostMalloc(reinterpret_cast<void**>(&read_places_), kReadPlaces * kReadBytes, hipHostMallocDefault), "pinned allocation");
-  // Up to 1 MB in one piece (a launch and an event a piece); more in quarters and at most as much as a place holds, so that
-  // a piece is widened while the next is on its way.
-  const size_t quarter = (total + kReadPlaces - 1) / kReadPlaces;
-  const size_t piece = std::min(kReadBytes / size, std::max<size_t>((quarter + 7) & ~(size_t)7, ((size_t)1 << 20) / size));
+  // As much as a place holds a launch: a piece is widened while the next is on its way.
+  const size_t piece = kReadBytes / size;
   const size_t pieces = (total + piece - 1) / piece;
   auto ask = [&](size_t i) {
     kernels_->copy_out(read_places_ + (i % kReadPlaces) * kReadBytes, logits, (int64_t)(i * piece), (int64_t)std::min(piece, total - i * piece));

@@ -114,8 +114,8 @@ class Engine {
   std::vector<float> observed_;
   // The pinned places that logits pass through on their way to the host, used in turn, each with the event of its last copy.
   static constexpr int kReadPlaces = 4;
-  static constexpr size_t kReadBytes = (size_t)2 << 20;
-  char* read_places_ = nullptr;       // pinned [kReadPlaces, kReadBytes], from the first readback on
+  static constexpr size_t kReadBytes = (size_t)1 << 20;
+  char* read_places_ = nullptr;       // pinned [kReadPlaces, kReadBytes]
   hipEvent_t read_done_[kReadPlaces] = {};
   // The sampler's buffers: temperatures and uniform numbers up, token ids down.
   float* sample_in_ = nullptr;        // pinned [2, rows]
