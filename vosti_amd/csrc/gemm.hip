@@ -93,31 +93,44 @@ __device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ be
 }
 
 
-// Up to 16 rows (HALVES: 8 or 16) of one chunk's activations as a wave's fragments, through LDS of the wave's own (HALVES * CHUNK_HALF_BYTES).
+// Up to ROWS (1, 4, 8 or 16) rows of one chunk's activations as a wave's fragments, through LDS of the wave's own (CHUNK_ROWS_BYTES(ROWS)).
 // The fragments' own addresses put four rows side by side in four neighbouring lanes, so that a load takes the address unit 64 clocks
 // where whole lines take 16: the activations cost a launch of a few weight tiles a workgroup as much of that unit as its weights.  Here a load
-// brings eight rows of 128 bytes.  Measured on MI355X, recorded launches with the weights of several layers in turn, us: 4,096 x 4,096,
-// 1, 8 and 16 rows 8.9 -> 8.1, 9.2 -> 8.5, 10.8 -> 9.4; 6,144 x 4,096, 8 rows 14.2 -> 13.2; 2,048 x 6,144,
-// 8 rows 11.6 -> 9.6; 1,024 x 3,072, 1 row 5.7 -> 5.4; gate/up with SwiGLU 12,288 x 4,096, 8 rows 37.7 -> 37.0.  Over 228 sizes of
-// 1 to 16 rows 3,439 -> 3,296 us, the slowest 5 % over what it was (1,536 x 1,024, 1 row: 3.25 -> 3.44).  (Weights through LDS alike do not pay: they come from
+// brings whole lines: eight rows of 128 bytes, four of 256, or one of 1,024.  Measured on MI355X, recorded launches with the weights of several
+// layers in turn, us, against rows straight to registers: 16-bit 4,096 x 4,096, 1, 8 and 16 rows 8.9 -> 7.9, 9.3 -> 8.5, 10.8 -> 9.4; 6,144 x 4,096,
+// 8 rows 14.1 -> 12.1; 2,048 x 6,144, 8 rows 11.6 -> 9.6; 1,024 x 3,072, 1 row 5.7 -> 5.2; 4,096 x 12,288, rows a chunk ahead, 1 and 16 rows
+// 21.2 -> 19.3, 28.9 -> 23.4; gate/up with SwiGLU 12,288 x 4,096, 8 rows 37.7 -> 36.5; 32-bit 2,048 x 2,048, 1 and 16 rows 9.6 -> 6.2, 11.9 -> 7.3.  Over
+// 315 sizes of 1 to 16 rows 5,163 -> 4,777 us in 16-bit, the slowest 3 % over what it was (4,096 x 1,024, 12 rows: 4.03 -> 4.15), and 9,536 -> 8,496 in
+// 32-bit.  Part of it is the order of the weights' loads (EARLY in the kernels).  (Weights through LDS alike do not pay: they come from
 // memory, 7.1 us for 33 MB against 7.4.  Tiles of eight or four weight rows for few of them do not either: 1,024 x 2,048 4.4 -> 4.6.)
-#define CHUNK_PAIRS (KC_SLABS / 2)                                // pairs of slabs: 128 bytes of a row
-#define CHUNK_HALF_BYTES (CHUNK_PAIRS * 1024)                     // eight rows of a chunk
-template <int HALVES>
-__device__ __forceinline__ void ask_chunk_rows(const elem_t* act, int64_t lda, int M, int lane, unsigned lds_addr) {      // HALVES * CHUNK_PAIRS loads
-  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
-#pragma unroll
-  for (int h = 0; h < HALVES; ++h) {
-    const unsigned voff = (unsigned)((min(h * 8 + lr, M - 1) * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
-#pragma unroll
-    for (int i = 0; i < CHUNK_PAIRS; ++i)
-      pipe_load_to_lds16_sv(reinterpret_cast<const unsigned char*>(act) + i * 128, voff, __builtin_amdgcn_readfirstlane(lds_addr + (h * CHUNK_PAIRS + i) * 1024));
+#define CHUNK_ROWS_BYTES(ROWS) ((ROWS) * KC * (int)sizeof(elem_t))
+template <int ROWS>
+struct ChunkRows {
+  static constexpr int LOADS = CHUNK_ROWS_BYTES(ROWS) / 1024;              // of a kilobyte each
+  static constexpr int PER = ROWS < 8 ? ROWS : 8, PIECES = 64 / PER;       // rows of a load, 16-byte pieces of each
+  static constexpr int TURN = PER == 8 ? 1 : 4;                            // a row's pieces lie at piece ^ (row * TURN): no two rows on the same banks
+  static constexpr int HALF = PER * KC * (int)sizeof(elem_t);              // eight rows, or all
+  // The lane's part of a load's address, in bytes from the first row, for the rows PER h ...
+  __device__ static __forceinline__ unsigned offset(int h, int64_t lda, int M, int lane) {
+    const int row = lane / PIECES, piece = (lane % PIECES) ^ (row * TURN);
+    return (unsigned)((min(h * PER + row, M - 1) * lda + piece * VK_VEC) * (int64_t)sizeof(elem_t));
   }
-}
-template <int HALVES>
-__device__ __forceinline__ frag_t chunk_fragment(const unsigned char* rows, int slab, int r16, int kg) {      // with 8 rows the others repeat them
-  const int r = r16 & 7, h = HALVES == 2 ? r16 >> 3 : 0;
-  return *reinterpret_cast<const frag_t*>(rows + (h * CHUNK_PAIRS + (slab >> 1)) * 1024 + r * 128 + ((((slab & 1) * 4 + kg) ^ r) * 16));
+  __device__ static __forceinline__ frag_t fragment(const unsigned char* rows, int slab, int r16, int kg) {     // rows beyond ROWS repeat them
+    const int r = r16 & (PER - 1), h = ROWS == 16 ? r16 >> 3 : 0, piece = slab * 4 + kg;
+    return *reinterpret_cast<const frag_t*>(rows + h * HALF + (piece / PIECES) * 1024 + r * (1024 / PER) + ((piece % PIECES) ^ (r * TURN)) * 16);
+  }
+};
+// Asks for them: LOADS loads.
+template <int ROWS>
+__device__ __forceinline__ void ask_chunk_rows(const elem_t* act, int64_t lda, int M, int lane, unsigned lds_addr) {
+  using C = ChunkRows<ROWS>;
+#pragma unroll
+  for (int h = 0; h < (ROWS == 16 ? 2 : 1); ++h) {
+    const unsigned voff = C::offset(h, lda, M, lane);
+#pragma unroll
+    for (int i = 0; i < C::HALF / 1024; ++i)
+      pipe_load_to_lds16_sv(reinterpret_cast<const unsigned char*>(act) + i * (1024 / C::PER), voff, __builtin_amdgcn_readfirstlane(lds_addr + h * C::HALF + i * 1024));
+  }
 }
 
 // ------------------------------------------------------------------ skinny
@@ -207,8 +220,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(elem_t* __re
 // a loaded value makes the compiler wait for it at once; and with RC > 0 a wave
 // keeps the activations of its RC chunks (K <= RC * 4096) in registers for the
 // whole kernel.  One barrier per round of eight chunks.
-// HALVES: 1 or 2: the resident activations (one tile) come through LDS, 8 or 16 rows; 0: straight to their registers.
-template <int MT, int W, int RC, int NT, int NW = SK_WAVES, int HALVES = 0>
+// ROWS: 1, 4, 8 or 16: the activations (one tile) come through LDS (ChunkRows): resident ones once, others a chunk ahead; 0: straight to registers.
+template <int MT, int W, int RC, int NT, int NW = SK_WAVES, int ROWS = 0>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict__ out,
                                                                     const elem_t* __restrict__ act,
                                                                     const elem_t* __restrict__ w, int M, int N, int K,
@@ -224,22 +237,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
   static_assert(NT * MT <= NW, "one wave adds up each output tile");
   __shared__ f32x4 part[2][NW][NT * MT][64];
 
-  static_assert(HALVES == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
-  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // HALVES * CHUNK_HALF_BYTES a wave
+  static_assert(ROWS == 0 || (MT == 1 && NT == 1 && RC <= 1), "one chunk tile of activations comes through LDS");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // CHUNK_ROWS_BYTES(ROWS) a wave
 
-  const int lane = threadIdx.x & 63, wave = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = ROWS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int nchunks = K / KC;
   const int ntiles = (N + 16 * NT - 1) / (16 * NT);     // tile: NT * 16 weight rows
-  unsigned char* own_rows = rows_lds + wave * (HALVES * CHUNK_HALF_BYTES);
-  if constexpr (HALVES > 0) ask_chunk_rows<HALVES>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  // The loop over tiles written out twice (with a tile to ask for next, and without), its loads kept in the order of the slabs: a load that may or may not
+  // be asked for makes the compiler wait for all of them.  16-bit 6,144 x 2,560, 16 rows 10.3 -> 9.5 us, 32-bit 2,048 x 2,048 10.0 -> 7.3; not with more
+  // than eight waves of 32-bit values or two projections' windows, whose registers do not suffice (SwiGLU 17,408 x 5,120 75.8 -> 82 us).
+  constexpr bool EARLY = RC == 1 && MT == 1 && (NW <= 8 || sizeof(elem_t) == 2);
+  constexpr bool AHEAD = ROWS > 0 && !RES;               // a chunk's rows are asked for while the one before is computed, into registers
+  unsigned char* own_rows = rows_lds + wave * CHUNK_ROWS_BYTES(ROWS);
+  if constexpr (ROWS > 0) ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
 
   const elem_t* arow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) arow[mt] = act + (int64_t)min(mt * 16 + r16, M - 1) * lda + kg * VK_VEC;
 
-  frag_t wbuf[W][NT], abuf[RES ? RC * KC_SLABS : W][MT];
-  if (RES && HALVES == 0) {
+  frag_t wbuf[W][NT], abuf[RES ? RC * KC_SLABS : AHEAD ? 1 : W][MT];
+  if (RES && ROWS == 0) {
 #pragma unroll
     for (int r = 0; r < RC; ++r) {
       const int c = min(r * NW + wave, nchunks - 1);     // beyond K: the last chunk again (not used)
@@ -255,7 +273,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       wbuf[slot][nt] = *reinterpret_cast<const frag_t*>(w + (int64_t)min((tile * NT + nt) * 16 + r16, N - 1) * K + kg * VK_VEC + k);
-    if (!RES) {
+    if (!RES && !AHEAD) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) abuf[slot][mt] = *reinterpret_cast<const frag_t*>(arow[mt] + k);
     }
@@ -266,22 +284,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, wave, i, i);
   }
-  if constexpr (HALVES > 0) {
+  if constexpr (ROWS > 0) {
     if (wave < nchunks) {                                // a wave with a chunk has a tile: there are no more workgroups than tiles
       __builtin_amdgcn_sched_barrier(0);                 // the weights' loads stay in front of the wait that counts them
       wait_vmcnt_n<W * NT>();                            // the rows are there, the first weights on their way
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (RES) {
 #pragma unroll
-      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = chunk_fragment<HALVES>(own_rows, i, r16, kg);
+        for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
+      }
     } else {
       wait_vmcnt_n<0>();
     }
   }
+  using C = ChunkRows<AHEAD ? ROWS : 1>;
+  frag_t held[AHEAD ? C::LOADS : 1];
   int parity = 0;
-  for (; tile < ntiles; tile += gridDim.x) {
+  auto one_tile = [&](auto more_) __attribute__((always_inline)) {
     f32x4 total = {0.f, 0.f, 0.f, 0.f};
-    auto round = [&](int base, int r) {       // chunks base .. base + 7; r = base / 8 where that is a constant
+    auto round = [&](auto next_, int base, int r) __attribute__((always_inline)) {       // chunks base .. base + 7; r = base / 8 where that is a constant
+      constexpr int NEXT = decltype(next_)::value;
       const int c = base + wave;
       f32x4 acc[NT][MT];
 #pragma unroll
@@ -289,13 +312,23 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (c < nchunks) {
-        // What this wave streams next: its next chunk of this tile, else its first chunk of the next tile.
+        // What this wave streams next: its next chunk of this tile, else its first chunk of the next tile.  A load that may or may not be asked for
+        // makes the compiler wait for all of them when the chunk ends: where something always follows (NEXT) the loads are plain ones, of this
+        // chunk again for the few waves that have none; a workgroup's last tile (one chunk a wave) asks for nothing.
         int nt_ = tile, nc = c + NW;
+        bool has_next = true;
         if (nc >= nchunks) {
-          nt_ = tile + gridDim.x;
-          nc = wave;
+          has_next = tile + (int)gridDim.x < ntiles;
+          nt_ = has_next ? tile + gridDim.x : tile;
+          nc = has_next ? wave : c;
         }
-        const bool has_next = nt_ < ntiles;
+        const bool ask = NEXT == 2 ? has_next : NEXT == 1;
+        if (AHEAD && ask) {
+          const unsigned char* rows = reinterpret_cast<const unsigned char*>(act + (int64_t)nc * KC);
+#pragma unroll
+          for (int l = 0; l < C::LOADS; ++l)
+            held[l] = *reinterpret_cast<const frag_t*>(rows + C::offset(l / (C::HALF / 1024), lda, M, lane) + l % (C::HALF / 1024) * (1024 / C::PER));
+        }
 #pragma unroll
         for (int i = 0; i < KC_SLABS; ++i) {
           const int slot = i % W;
@@ -303,13 +336,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) fw[nt] = wbuf[slot][nt];
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) fa[mt] = RES ? abuf[r * KC_SLABS + i][mt] : abuf[slot][mt];
+          for (int mt = 0; mt < MT; ++mt) {
+            if constexpr (AHEAD) fa[mt] = C::fragment(own_rows, i, r16, kg);
+            else fa[mt] = RES ? abuf[r * KC_SLABS + i][mt] : abuf[slot][mt];
+          }
           if (i + W < KC_SLABS) issue(tile, c, i + W, slot);
-          else if (has_next) issue(nt_, nc, i + W - KC_SLABS, slot);
+          else if (ask) issue(nt_, nc, i + W - KC_SLABS, slot);
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = mma_slab(fw[nt], fa[mt], acc[nt][mt]);
+          if (EARLY) __builtin_amdgcn_sched_barrier(0);      // the compiler would ask for the slabs of the second half when the first is done
+        }
+        if (AHEAD && ask) {                              // this chunk's fragments have been read: its place is free
+#pragma unroll
+          for (int l = 0; l < C::LOADS; ++l) *reinterpret_cast<frag_t*>(own_rows + l * 1024 + lane * 16) = held[l];
         }
       }
 #pragma unroll
@@ -327,15 +368,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
       }
       parity ^= 1;
     };
-    if (RES) {
+    const std::integral_constant<int, 2> maybe;
+    if constexpr (RC == 1) {
+      if (0 < nchunks) round(more_, 0, 0);
+    } else if constexpr (RES) {
 #pragma unroll
-      for (int r = 0; r < (RES ? RC : 1); ++r)
-        if (r * NW < nchunks) round(r * NW, r);
+      for (int r = 0; r < RC; ++r)
+        if (r * NW < nchunks) round(maybe, r * NW, r);
     } else {
-      for (int base = 0; base < nchunks; base += NW) round(base, 0);
+      int base = 0;
+      if (sizeof(elem_t) == 2)                            // (32-bit, 5,120 x 17,408, 1 row: 102.6 -> 107.8 us)
+        for (; base + NW < nchunks; base += NW) round(std::integral_constant<int, 1>(), base, 0);
+      for (; base < nchunks; base += NW) round(maybe, base, 0);
     }
     if (wave < NT * MT)
       store_out4(out, ldo, (wave % MT) * 16 + r16, (tile * NT + wave / MT) * 16 + 4 * kg, M, N, total, out_form);
+  };
+  if constexpr (EARLY) {
+    for (; tile + (int)gridDim.x < ntiles; tile += gridDim.x) one_tile(std::integral_constant<int, 1>());
+    if (tile < ntiles) one_tile(std::integral_constant<int, 0>());
+  } else {
+    for (; tile < ntiles; tile += gridDim.x) one_tile(std::integral_constant<int, 2>());
   }
 }
 
@@ -345,7 +398,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 // two projections rounded to the element type first, which is what the separate
 // GEMM and SwiGLU kernels compute (kernels/triton_kernels/silu_mul.py:64-87).
 // M <= 16, K <= 4096 (activations resident in registers).
-template <int W, int MT, int RC, int NW = SK_WAVES, int HALVES = 0>
+template <int W, int MT, int RC, int NW = SK_WAVES, int ROWS = 0>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __restrict__ out,
                                                                            const elem_t* __restrict__ act,
                                                                            const elem_t* __restrict__ w, int M, int I,
@@ -355,19 +408,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   static_assert(MT * RC <= 2, "two chunk tiles of activations stay in registers: two tiles of a chunk or two chunks of a tile");
   __shared__ f32x4 part[2][RC][NW][2 * MT][64];      // two sets, used in turn: one barrier per tile
 
-  static_assert(HALVES == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
-  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // HALVES * CHUNK_HALF_BYTES a wave
-  const int lane = threadIdx.x & 63, wave = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+  static_assert(ROWS == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
+  constexpr bool EARLY = ROWS > 0 && NW <= 8;             // as in the kernel above; two projections' windows leave fewer registers
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // CHUNK_ROWS_BYTES(ROWS) a wave
+  const int lane = threadIdx.x & 63, wave = ROWS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int nchunks = K / KC;
   const int ntiles = (I + 15) / 16;
-  unsigned char* own_rows = rows_lds + wave * (HALVES * CHUNK_HALF_BYTES);
-  if constexpr (HALVES > 0) ask_chunk_rows<HALVES>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  unsigned char* own_rows = rows_lds + wave * CHUNK_ROWS_BYTES(ROWS);
+  if constexpr (ROWS > 0) ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
 
   // Wave w has chunks w, w + 8, ...: RC of them (chunks beyond K are read as the last and not used).
   frag_t wg[W], wu[W], abuf[RC * KC_SLABS][MT];
 #pragma unroll
-  for (int r = 0; r < (HALVES ? 0 : RC); ++r) {
+  for (int r = 0; r < (ROWS ? 0 : RC); ++r) {
     const int c = min(r * NW + wave, nchunks - 1);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -394,22 +448,23 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, i, i);
   }
-  if constexpr (HALVES > 0) {
+  if constexpr (ROWS > 0) {
     if (active) {                                        // as in the kernel above
       __builtin_amdgcn_sched_barrier(0);
       wait_vmcnt_n<2 * W>();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = chunk_fragment<HALVES>(own_rows, i, r16, kg);
+      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
     } else {
       wait_vmcnt_n<0>();
     }
   }
   int parity = 0;
-  for (; tile < ntiles; tile += gridDim.x) {
+  auto one_tile = [&](auto more_) __attribute__((always_inline)) {
+    constexpr int NEXT = decltype(more_)::value;          // as in the kernel above
     const int nt = tile + gridDim.x;
-    const bool has_next = nt < ntiles;
+    const bool ask = NEXT == 2 ? nt < ntiles : NEXT == 1;
 #pragma unroll
     for (int r = 0; r < RC; ++r) {
       f32x4 ag[MT], au[MT];
@@ -421,13 +476,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
           const int slot = i % W;
           const frag_t fg = wg[slot], fu = wu[slot];
           const int g = r * KC_SLABS + i + W;             // the slab that takes this slot
-          if (g < my_slabs) issue(tile, g, slot);
-          else if (has_next) issue(nt, g - my_slabs, slot);
+          if (EARLY ? i + W < KC_SLABS : g < my_slabs) issue(tile, g, slot);
+          else if (ask) issue(nt, g - my_slabs, slot);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
             ag[mt] = mma_slab(fg, abuf[r * KC_SLABS + i][mt], ag[mt]);
             au[mt] = mma_slab(fu, abuf[r * KC_SLABS + i][mt], au[mt]);
           }
+          if (EARLY) __builtin_amdgcn_sched_barrier(0);
         }
       }
 #pragma unroll
@@ -455,6 +511,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
       store_out4(out, ldo, wave * 16 + r16, tile * 16 + 4 * kg, M, I, y, out_form);
     }
     parity ^= 1;
+  };
+  if constexpr (EARLY) {
+    for (; tile + (int)gridDim.x < ntiles; tile += gridDim.x) one_tile(std::integral_constant<int, 1>());
+    if (tile < ntiles) one_tile(std::integral_constant<int, 0>());
+  } else {
+    for (; tile < ntiles; tile += gridDim.x) one_tile(std::integral_constant<int, 2>());
   }
 }
 
@@ -603,13 +665,6 @@ static int launch_tiled(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // gate, those with wn = 1 the up projection), and at the end the up values pass through LDS to the
 // waves that hold the gate values, which write  silu(g) * u  with g and u rounded to the element type
 // first: the bits of the plain projection followed by swiglu_kernel.
-// 16 bytes per lane from global memory into LDS at dst + 16 * lane.  In a function of its own: called
-// with template-dependent arguments from inside the kernel template, the builtin keeps the compiler
-// from emitting the kernel's host-side stub.
-__device__ __forceinline__ void pipe_load_to_lds16(const elem_t* src, unsigned char* dst) {
-  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-}
-
 // FNW: 16-row weight fragments per wave, 2 to 5: a workgroup takes 32 FNW weight rows.  4 is the square tile; 2
 // gives twice the workgroups, for grids that would leave compute units with one workgroup or none; 3 and 5 are
 // for grids whose last round of workgroups would otherwise run nearly empty (pipe_fragments_by_rounds).  Six
@@ -1482,14 +1537,17 @@ static int stream_waves(int nchunks) {
   return 8;
 }
 
-// How a streaming kernel of `waves` waves with a chunk each brings in the activations of M rows: through LDS as 8 rows (1) or 16 (2) a wave, or
-// straight to registers (0) where that does not fit beside the chunk sums (sums_bytes).  In 32-bit, 16 rows through LDS leave room
+// How many of M rows' activations a streaming kernel of `waves` waves brings in through LDS (1, 4, 8 or 16 a wave and chunk), or 0:
+// straight to registers, where that does not fit beside the chunk sums (sums_bytes).  In 32-bit, 16 rows through LDS leave room
 // for fewer workgroups, which only launches of one weight tile a workgroup do not miss (151,936 x 1,024: 128 -> 165 us; 1,024 x 2,048: 11.6 -> 9.5).
-static constexpr int stream_row_halves(int M, int waves, int sums_bytes) {
-  const int halves = M > 8 ? 2 : 1;
-  return halves * waves * CHUNK_HALF_BYTES + sums_bytes <= 160 * 1024 ? halves : 0;
+static constexpr int stream_lds_rows(int M, int waves, int sums_bytes) {
+  const int rows = M == 1 ? 1 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
+  return waves * CHUNK_ROWS_BYTES(rows) + sums_bytes <= 160 * 1024 ? rows : 0;
 }
-static bool stream_rows_pay(int M, int weight_tiles) { return M <= 8 || sizeof(elem_t) == 2 || weight_tiles <= vk_device_cus(); }
+static bool stream_rows_pay(int M, int weight_tiles, int64_t lda) {
+  if (lda > (1 << 26)) return false;        // a row's offset is of 32 bits
+  return M <= 8 || sizeof(elem_t) == 2 || weight_tiles <= vk_device_cus();
+}
 
 // Which kernel computes a product (speed only: all give the same bits).  Every threshold is a count of
 // workgroups against the device's compute units (cus), or a count of 16-row activation tiles, or whether a
@@ -1663,7 +1721,8 @@ int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // such a variant, 8, 9 and 10 = activations shared through LDS with 64, 32 and 128 weight rows per workgroup
 // (17 to 512 rows, in blocks of 64 rows), 11 = skinny with two activation tiles resident in registers (17 to
 // 32 rows of 16-bit elements, K <= 4096), 12 = as 9 in blocks of 32 rows, 13, 15 and 16 = pipelined with 64, 96
-// and 160 weight rows per workgroup (14 is the callers' name for the route through chunk sums); for measurements and tests.  The result does not depend on the choice.
+// and 160 weight rows per workgroup (14 is the callers' name for the route through chunk sums), 17, 18 and 19 = alternating
+// with 192, 160 and 128 weight rows per workgroup (256 rows or more, 16-bit elements, K a multiple of 512); for measurements and tests.  The result does not depend on the choice.
 static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                        int kernel, int activation, hipStream_t st) {
   VK_REQUIRE(activation == 0 || activation == 1, "gemm: unknown activation %d", activation);
@@ -1712,31 +1771,33 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     const int mt = (M + 15) / 16;
     const unsigned grid = (unsigned)((N + 15) / 16);
     if (K % KC == 0) {
-#define STH(MT, W, RC, NT, NW, HALVES)                                                                    \
+#define STH(MT, W, RC, NT, NW, ROWS)                                                                    \
   do {                                                                                                    \
-    constexpr size_t rows_bytes = (size_t)(HALVES) * NW * CHUNK_HALF_BYTES;                               \
+    constexpr size_t rows_bytes = (size_t)NW * CHUNK_ROWS_BYTES(ROWS);                                \
     static int resident = 0; /* workgroups of this kernel that the device holds at once */               \
     if (resident == 0) {                                                                                  \
       int dev = 0, cus = 0, per_cu = 0;                                                                   \
       (void)hipGetDevice(&dev);                                                                           \
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);                      \
       if (rows_bytes)                                                                                     \
-        (void)hipFuncSetAttribute((const void*)gemm_stream_kernel<MT, W, RC, NT, NW, HALVES>,             \
+        (void)hipFuncSetAttribute((const void*)gemm_stream_kernel<MT, W, RC, NT, NW, ROWS>,             \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_bytes);           \
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_kernel<MT, W, RC, NT, NW, HALVES>, \
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_kernel<MT, W, RC, NT, NW, ROWS>, \
                                                          64 * NW, rows_bytes);                            \
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                       \
     }                                                                                                     \
     const unsigned groups = (unsigned)((N + 16 * NT - 1) / (16 * NT));                                    \
-    gemm_stream_kernel<MT, W, RC, NT, NW, HALVES><<<groups < (unsigned)resident ? groups : (unsigned)resident, \
+    gemm_stream_kernel<MT, W, RC, NT, NW, ROWS><<<groups < (unsigned)resident ? groups : (unsigned)resident, \
                                              64 * NW, rows_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form); \
   } while (0)
 #define STW(MT, W, RC, NT, NW) STH(MT, W, RC, NT, NW, 0)
 #define STN(NW)                                                                                           \
   do {                                                                                                    \
-    const int halves = stream_rows_pay(M, (N + 15) / 16) ? stream_row_halves(M, NW, NW * 2048) : 0;       \
-    if (halves == 2) STH(1, 8, 1, 1, NW, stream_row_halves(16, NW, NW * 2048));                           \
-    else if (halves == 1) STH(1, 8, 1, 1, NW, stream_row_halves(8, NW, NW * 2048));                       \
+    const int rows = stream_rows_pay(M, (N + 15) / 16, lda) ? stream_lds_rows(M, NW, NW * 2048) : 0;           \
+    if (rows == 16) STH(1, 8, 1, 1, NW, stream_lds_rows(16, NW, NW * 2048));                              \
+    else if (rows == 8) STH(1, 8, 1, 1, NW, stream_lds_rows(8, NW, NW * 2048));                           \
+    else if (rows == 4) STH(1, 8, 1, 1, NW, 4);                                                           \
+    else if (rows == 1) STH(1, 8, 1, 1, NW, 1);                                                           \
     else STH(1, 8, 1, 1, NW, 0);                                                                          \
   } while (0)
 #define ST(MT, W, RC, NT) STW(MT, W, RC, NT, SK_WAVES)
@@ -1766,7 +1827,18 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
         // three did not fit beside the rest and were slower than none (4096 x 12288: 29 -> 36 us).
         else if (K <= 2 * SK_WAVES * KC) ST(1, 8, 2, 1);
 #endif
-        else ST(1, 8, 0, 1);
+        else {
+#ifdef VK_BF16
+          // Not in 32-bit: the rows held are twice as many registers there (4,096 x 4,608, 8 rows 22.7 -> 29.4 us; 7,168 x 5,120, 4 rows 35.7 -> 40.2).
+          const int rows = stream_rows_pay(M, tiles16, lda) ? stream_lds_rows(M, SK_WAVES, SK_WAVES * 2048) : 0;
+          if (rows == 16) STH(1, 8, 0, 1, SK_WAVES, stream_lds_rows(16, SK_WAVES, SK_WAVES * 2048));
+          else if (rows == 8) STH(1, 8, 0, 1, SK_WAVES, 8);
+          else if (rows == 4) STH(1, 8, 0, 1, SK_WAVES, 4);
+          else if (rows == 1) STH(1, 8, 0, 1, SK_WAVES, 1);
+          else
+#endif
+          ST(1, 8, 0, 1);
+        }
       }
       else if (mt == 2) {
 #ifdef VK_BF16
@@ -1887,30 +1959,32 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   }
   const int ntiles = (I + 15) / 16;
   const int form = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
-#define SWIGLU_STREAMH(W, MT, RC, NW, HALVES)                                                               \
+#define SWIGLU_STREAMH(W, MT, RC, NW, ROWS)                                                               \
   do {                                                                                                     \
-    constexpr size_t rows_bytes = (size_t)(HALVES) * NW * CHUNK_HALF_BYTES;                                \
+    constexpr size_t rows_bytes = (size_t)NW * CHUNK_ROWS_BYTES(ROWS);                                \
     static int resident = 0;                                                                               \
     if (resident == 0) {                                                                                   \
       int dev = 0, cus = 0, per_cu = 0;                                                                    \
       (void)hipGetDevice(&dev);                                                                            \
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);                       \
       if (rows_bytes)                                                                                      \
-        (void)hipFuncSetAttribute((const void*)gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES>,           \
+        (void)hipFuncSetAttribute((const void*)gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS>,           \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_bytes);            \
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES>, \
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS>, \
                                                          64 * NW, rows_bytes);                             \
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                        \
     }                                                                                                      \
-    gemm_stream_swiglu_kernel<W, MT, RC, NW, HALVES><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
+    gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
         out, act, w, M, I, K, lda, ldo, form);                                                           \
   } while (0)
 #define SWIGLU_STREAM(W, MT, RC) SWIGLU_STREAMH(W, MT, RC, SK_WAVES, 0)
 #define SWIGLU_STREAMN(NW)                                                                                 \
   do {                                                                                                     \
-    const int halves = stream_rows_pay(M, ntiles) ? stream_row_halves(M, NW, NW * 4096) : 0;               \
-    if (halves == 2) SWIGLU_STREAMH(8, 1, 1, NW, stream_row_halves(16, NW, NW * 4096));                    \
-    else if (halves == 1) SWIGLU_STREAMH(8, 1, 1, NW, stream_row_halves(8, NW, NW * 4096));                \
+    const int rows = stream_rows_pay(M, ntiles, lda) ? stream_lds_rows(M, NW, NW * 4096) : 0;                   \
+    if (rows == 16) SWIGLU_STREAMH(8, 1, 1, NW, stream_lds_rows(16, NW, NW * 4096));                       \
+    else if (rows == 8) SWIGLU_STREAMH(8, 1, 1, NW, stream_lds_rows(8, NW, NW * 4096));                    \
+    else if (rows == 4) SWIGLU_STREAMH(8, 1, 1, NW, 4);                                                    \
+    else if (rows == 1) SWIGLU_STREAMH(8, 1, 1, NW, 1);                                                    \
     else SWIGLU_STREAMH(8, 1, 1, NW, 0);                                                                   \
   } while (0)
   const int nw = M <= 16 ? stream_waves(K / KC) : SK_WAVES;       // as in vk_gemm
@@ -1919,8 +1993,8 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   else if (nw == 5) SWIGLU_STREAMN(5);
   else if (nw == 6) SWIGLU_STREAMN(6);
 #ifdef VK_BF16
-  else if (nw == 10) SWIGLU_STREAMH(8, 1, 1, 10, 0);       // ten waves with the rows in LDS: 17,408 x 5,120 77.5 -> 79.9 us at 8 rows
-  else if (nw == 12) SWIGLU_STREAMH(8, 1, 1, 12, 0);
+  else if (nw == 10) SWIGLU_STREAMN(10);
+  else if (nw == 12) SWIGLU_STREAMN(12);
 #endif
   else
 #ifdef VK_BF16
