@@ -377,7 +377,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
         if (r * NW < nchunks) round(maybe, r * NW, r);
     } else {
       int base = 0;
-      if (sizeof(elem_t) == 2)                            // (32-bit, 5,120 x 17,408, 1 row: 102.6 -> 107.8 us)
+      if (MT == 1 && sizeof(elem_t) == 2)                 // (elsewhere it does not pay: 32-bit 5,120 x 17,408, 1 row 102.6 -> 107.8 us; 4,096 x 4,608, 17 rows 12.8 -> 15.9)
         for (; base + NW < nchunks; base += NW) round(std::integral_constant<int, 1>(), base, 0);
       for (; base < nchunks; base += NW) round(maybe, base, 0);
     }
