@@ -46,6 +46,27 @@ def test_product_by_size(M, N, K):
     assert torch.equal(k.gemm(act, w), k.gemm(act, w, kernel=4))
 
 
+@pytest.mark.parametrize("M,N,K", [(256, 195, 512), (700, 1633, 1024), (2048, 4097, 512), (511, 4099, 1024), (300, 4102, 512)])
+def test_columns_that_are_no_multiple_of_four(M, N, K):
+    """Rows of the output on whole vectors, a last block of columns that does not begin on one: every store on its type's alignment, nothing beyond a row's
+    end, plain and with SwiGLU folded in."""
+    k = kern(torch.bfloat16)
+    ldo = (N + 7) // 4 * 4
+    act, w = rand((M, K), torch.bfloat16, 9).cuda(), rand((2 * N, K), torch.bfloat16, 10, 0.1).cuda()
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    k.lib.vk_gemm.argtypes = [p, p, p, i, i, i, l, l, i, p]
+    k.lib.vk_gemm_swiglu.argtypes = [p, p, p, i, i, i, l, l, p]
+    stream = torch.cuda.current_stream().cuda_stream
+    plain, gated = k.gemm(act, w[:N], kernel=4), k.swiglu(k.gemm(act, w, kernel=4))
+    for code in (0, 17, 18, 19):
+        out = torch.full((M, ldo), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert k.lib.vk_gemm(out.data_ptr(), act.data_ptr(), w.data_ptr(), M, N, K, K, ldo, code, stream) == 0
+        assert torch.equal(out[:, :N], plain) and bool((out[:, N:] == 7.0).all()), code
+    out = torch.full((M, ldo), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert k.lib.vk_gemm_swiglu(out.data_ptr(), act.data_ptr(), w.data_ptr(), M, N, K, K, ldo, stream) == 0
+    assert torch.equal(out[:, :N], gated) and bool((out[:, N:] == 7.0).all())
+
+
 def test_sizes_below_a_tile_are_refused():
     k = kern(torch.bfloat16)
     w = rand((256, 512), torch.bfloat16, 7).cuda()

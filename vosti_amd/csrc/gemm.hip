@@ -1175,6 +1175,7 @@ static int launch_alternate(elem_t* out, const elem_t* act, const elem_t* w, int
   const int row_blocks = (M + 255) / 256;
   const int64_t tiles = (int64_t)row_blocks * ((N + COLS - 1) / COLS);
   VK_REQUIRE(tiles < (1 << 30), "gemm: too many rows (%d)", M);
+  if (N % 4 != 0) form &= ~OUT_VEC;       // the last block of columns begins at N - COLS: four of its columns are then no aligned vector
   gemm_alternate_kernel<FNW, SA, SW, SWIGLU><<<(unsigned)tiles, 512, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, row_blocks);
   return vk_check_launch("gemm_alternate");
 }
