@@ -73,3 +73,12 @@ def test_sizes_below_a_tile_are_refused():
     for code, rows, M, K in ((17, 191, 256, 512), (18, 159, 256, 512), (19, 128, 255, 512), (19, 128, 256, 448)):
         with pytest.raises(Exception, match="alternating"):
             k.gemm(rand((M, K), torch.bfloat16, 8).cuda(), w.flatten()[: rows * K].view(rows, K), kernel=code)
+
+
+@pytest.mark.parametrize("code", [17, 18, 19])
+@pytest.mark.parametrize("M", [0, 256])
+def test_32_bit_elements_are_refused(M, code):
+    k = kern(torch.float32)
+    x = rand((256, 512), torch.float32, 11).cuda()
+    with pytest.raises(Exception, match="unknown kernel"):
+        k.gemm(x[:M], x, kernel=code)

@@ -1733,7 +1733,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
              (long long)lda, VK_VEC);
   VK_REQUIRE(ldo >= N, "gemm: output row stride %lld is smaller than N=%d", (long long)ldo, N);
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm: operands must be 16-byte aligned");
-  VK_REQUIRE(kernel >= 0 && kernel <= 19 && kernel != 14, "gemm: unknown kernel %d", kernel);
+  VK_REQUIRE(kernel >= 0 && kernel <= (sizeof(elem_t) == 2 ? 19 : 16) && kernel != 14, "gemm: unknown kernel %d", kernel);      // the alternating one takes 16-bit elements
   if (M == 0) return 0;
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
