@@ -1012,8 +1012,10 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
 // memory this kernel reaches 1,430 TFLOP/s, which is near what the chip sustains of these MFMAs (1,640).  Measured on MI355X with the weights
 // of several layers in turn, tile kernel against this one, us: gate/up with SwiGLU 12,288 x 4,096, 2,048 rows 404 -> 349 (1,180 TFLOP/s), 4,096
 // rows 741 -> 646 (1,280); 4,096 x 12,288, 2,048 rows 189 -> 169, 4,096 rows 364 -> 322; 6,144 x 4,096, 2,048 rows 108 -> 93; 5,120 x
-// 17,408, 3,900 rows 633 -> 540 (1,290).  Over 532 sizes of 256 to 4,096 rows 288 take it, 66.2 -> 60.2 ms in all, the worst 7 % slower
-// than before (1,024 rows, 6,144 x 2,560).
+// 17,408, 3,900 rows 633 -> 540 (1,290).  Over 920 sizes of 256 to 4,096 rows, weights from memory, 515 take it, 114.6 -> 104.0 ms in all (103.8 with
+// the better kernel at every size).  Three of them are 5 to 8 % slower than the tile kernel (850 to 1,024 rows, 6,144 x 2,560: 38 to 39 us against 41,
+// where 96 columns fill exactly one round of that), one 5 % (850 rows, 16,384 x 4,096), six 2 to 3 %; a rule that leaves these to the tile kernel
+// gives up as much at others (1,300 rows, 4,096 x 2,048: 32.5 -> 30.7).
 // Tried: K tiles of one slab (rows of 64 bytes, five places: half of every line that the cache sends is not asked for, 162 -> 190 us at 4,096
 // rows, 6,144 x 4,096); a slab's activations read a phase ahead (5 to 15 % slower); a tile's loads in quarters, also between the MFMAs (4 %
 // slower than in halves).
@@ -1648,7 +1650,9 @@ static int pipe_fragments_by_rounds(int M, int N, double* rounds_of_128 = nullpt
 static int alternate_fragments(int M, int N, int K, bool swiglu) {
   if (M < 256 || K % KC != 0 || N < (swiglu ? 96 : 192)) return 0;
   const int cus = vk_device_cus(), out_cols = swiglu ? 2 * N : N;
-  if (!swiglu && (int64_t)((N + 127) / 128) * ((M + 127) / 128) <= cus) return 0;      // workgroups of 64 weight rows
+  // At most one workgroup a compute unit of the tile kernel's: its round is shorter then than a full one's 0.72 (1,536 x 2,048 with SwiGLU, 256 to 512
+  // rows: 26 to 29 us against 30).  The plain product's caller has asked that before.
+  if (swiglu && (int64_t)((N + 63) / 64) * ((M + 127) / 128) <= cus) return 0;
   static const double slope[7] = {0, 0, 0, 0, 13.1, 15.8, 18.9}, start[7] = {0, 0, 0, 0, 7, 6, 8};
   const double k = K / 1024.0;
   double rounds = 0;
