@@ -30,3 +30,11 @@ def test_gate_and_up(M, chunks, dtype):
     for I in (24, 4200):
         w = rand((2 * I, K), dtype, 4, 0.1).cuda()
         assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4)))
+
+
+@pytest.mark.parametrize("M,I,K", [(17, 12300, 512), (24, 8201, 1024), (32, 4097, 4096), (20, 16, 2048), (31, 4096, 2560)])
+def test_gate_and_up_of_two_tiles_of_rows(M, I, K):
+    """17 to 32 rows: several weight tiles a workgroup and one, the last of them partial, waves without a chunk."""
+    k = kern(torch.bfloat16)
+    x, w = rand((M, K), torch.bfloat16, 5).cuda(), rand((2 * I, K), torch.bfloat16, 6, 0.1).cuda()
+    assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4)))

@@ -415,7 +415,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   __shared__ f32x4 part[2][RC][NW][2 * MT][64];      // two sets, used in turn: one barrier per tile
 
   static_assert(ROWS == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
-  constexpr bool EARLY = ROWS > 0 && NW <= 8;             // as in the kernel above; two projections' windows leave fewer registers
+  // As in the kernel above; two projections' windows leave fewer registers.  Two tiles of rows: the loop in one piece took 3,072 x 1,024, 24 rows 11.0 us,
+  // as a function of its own 11.4, and written out twice 10.0 (12,288 x 4,096, 20 rows 44.0, 43.6 and 41.8).
+  constexpr bool EARLY = MT == 2 || (ROWS > 0 && NW <= 8);
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // CHUNK_ROWS_BYTES(ROWS) a wave
   const int lane = threadIdx.x & 63, wave = ROWS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
