@@ -38,3 +38,13 @@ def test_gate_and_up_of_two_tiles_of_rows(M, I, K):
     k = kern(torch.bfloat16)
     x, w = rand((M, K), torch.bfloat16, 5).cuda(), rand((2 * I, K), torch.bfloat16, 6, 0.1).cuda()
     assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4)))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N", [3072, 3088, 4090, 4096, 4097])
+@pytest.mark.parametrize("M", [8, 9, 16])
+def test_two_chunks_and_about_a_weight_tile_a_compute_unit(M, N, dtype):
+    """On both sides of the line between rows through LDS and rows straight to registers."""
+    k = kern(dtype)
+    x, w = rand((M, 1024), dtype, 7).cuda(), rand((N, 1024), dtype, 8, 0.1).cuda()
+    assert torch.equal(k.gemm(x, w), k.gemm(x, w, kernel=4))

@@ -100,7 +100,7 @@ __device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ be
 // layers in turn, us, against rows straight to registers: 16-bit 4,096 x 4,096, 1, 8 and 16 rows 8.9 -> 7.9, 9.3 -> 8.5, 10.8 -> 9.4; 6,144 x 4,096,
 // 8 rows 14.1 -> 12.1; 2,048 x 6,144, 8 rows 11.6 -> 9.6; 1,024 x 3,072, 1 row 5.7 -> 5.2; 4,096 x 12,288, rows a chunk ahead, 1 and 16 rows
 // 21.2 -> 19.3, 28.9 -> 23.4; gate/up with SwiGLU 12,288 x 4,096, 8 rows 37.7 -> 36.5; 32-bit 2,048 x 2,048, 1 and 16 rows 9.6 -> 6.2, 11.9 -> 7.3.  Over
-// 315 sizes of 1 to 16 rows 5,163 -> 4,777 us in 16-bit, the slowest 3 % over what it was (4,096 x 1,024, 12 rows: 4.03 -> 4.15), and 9,536 -> 8,496 in
+// 315 sizes of 1 to 16 rows 5,163 -> 4,777 us in 16-bit, none more than 2 % over what it was, and 9,536 -> 8,496 in
 // 32-bit.  Part of it is the order of the weights' loads (EARLY in the kernels).  (Weights through LDS alike do not pay: they come from
 // memory, 7.1 us for 33 MB against 7.4.  Tiles of eight or four weight rows for few of them do not either: 1,024 x 2,048 4.4 -> 4.6.)
 #define CHUNK_ROWS_BYTES(ROWS) ((ROWS) * KC * (int)sizeof(elem_t))
@@ -1555,8 +1555,11 @@ static constexpr int stream_lds_rows(int M, int waves, int sums_bytes) {
   const int rows = M == 1 ? 1 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
   return waves * CHUNK_ROWS_BYTES(rows) + sums_bytes <= 160 * 1024 ? rows : 0;
 }
-static bool stream_rows_pay(int M, int weight_tiles, int64_t lda) {
+// Nor do 9 to 16 rows of K = 1,024 (two chunks of 16-bit elements) on about one weight tile a compute unit: 4,096 weight rows, 9 and 16 rows take 3.89 and 3.94 us
+// straight to registers, 4.14 and 4.17 through LDS; up to 3,072 and from 4,352 weight rows on the times are the same or LDS is the faster way.
+static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0) {
   if (lda > (1 << 26)) return false;        // a row's offset is of 32 bits
+  if (sizeof(elem_t) == 2 && M > 8 && chunks == 2 && weight_tiles <= vk_device_cus() && 4 * weight_tiles > 3 * vk_device_cus()) return false;
   return M <= 8 || sizeof(elem_t) == 2 || weight_tiles <= vk_device_cus();
 }
 
@@ -1806,7 +1809,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
 #define STW(MT, W, RC, NT, NW) STH(MT, W, RC, NT, NW, 0)
 #define STN(NW)                                                                                           \
   do {                                                                                                    \
-    const int rows = stream_rows_pay(M, (N + 15) / 16, lda) ? stream_lds_rows(M, NW, NW * 2048) : 0;           \
+    const int rows = stream_rows_pay(M, (N + 15) / 16, lda, K / KC) ? stream_lds_rows(M, NW, NW * 2048) : 0;   \
     if (rows == 16) STH(1, 8, 1, 1, NW, stream_lds_rows(16, NW, NW * 2048));                              \
     else if (rows == 8) STH(1, 8, 1, 1, NW, stream_lds_rows(8, NW, NW * 2048));                           \
     else if (rows == 4) STH(1, 8, 1, 1, NW, 4);                                                           \
