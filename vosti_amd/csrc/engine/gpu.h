@@ -109,7 +109,7 @@ class Kernels {
   Tensor add_rmsnorm(const Tensor& x, Tensor& residual, const Tensor& w, float eps);
   Tensor swiglu(const Tensor& gate_up);
   Tensor gather_rows(const Tensor& x, const Tensor& rows);
-  Tensor to_f32(const Tensor& x);
+  Tensor to_f32(const Tensor& x);        // for parts from outside: the engine itself reads its logits back as elements
   // The elements first .. first + count of x to memory that the GPU can write (pinned host memory).
   void copy_out(void* out, const Tensor& x, int64_t first, int64_t count);
   // A 32-bit tensor as elements (the tensor itself where the elements are 32-bit).
@@ -148,7 +148,6 @@ class Kernels {
   // out = base + mult * norm(y), floats; out may be base.
   // rounded (elements of out's shape, or null): the new rows rounded to elements as well.
   void stream_norm_add(Tensor& out, const Tensor& base, const Tensor& y, const Tensor& w, float eps, float offset, float mult, Tensor* rounded = nullptr);
-  // out = sum over j < n of coef[j] * states[j]; states [>= n, ...] floats.
   // A norm over rows, y = x * rsqrt(mean(x^2) + eps) * (offset + weight); no weight: another kind of norm.
   struct RowNorm {
     const Tensor* weight = nullptr;
@@ -161,6 +160,7 @@ class Kernels {
                           const Tensor* coef = nullptr, int n = 0, Tensor* mixed = nullptr);
   // s += a + b (floats); returns both norms of the new rows.
   std::pair<Tensor, Tensor> stream_sum_norms(Tensor& s, const Tensor& a, const Tensor& b, const RowNorm& first, const RowNorm& second);
+  // out = sum over j < n of coef[j] * states[j]; states [>= n, ...] floats.
   Tensor stream_mix(const Tensor& states, const Tensor& coef, int n);
   void softcap(Tensor& x, float cap);          // x <- cap * tanh(x / cap)
   // gemm on the columns [first, first + w.dim(1)) of act.

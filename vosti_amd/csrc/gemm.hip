@@ -1807,6 +1807,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
                                              64 * NW, rows_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form); \
   } while (0)
 #define STW(MT, W, RC, NT, NW) STH(MT, W, RC, NT, NW, 0)
+// Where as many rows do not fit beside the sums, stream_lds_rows names the kernel without them instead: nothing is compiled for a branch that is not taken.
 #define STN(NW)                                                                                           \
   do {                                                                                                    \
     const int rows = stream_rows_pay(M, (N + 15) / 16, lda, K / KC) ? stream_lds_rows(M, NW, NW * 2048) : 0;   \
@@ -1836,8 +1837,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
 #endif
         else
         if (kernel == 7 || (by_size && K > SK_WAVES * KC && tiles16 > cus && 2 * tiles16 <= 3 * cus)) ST(1, 8, 0, 2);
-        else if (K <= SK_WAVES * KC && kernel != 7) STN(SK_WAVES);
-        else if (K <= SK_WAVES * KC) ST(1, 8, 1, 1);
+        else if (K <= SK_WAVES * KC) STN(SK_WAVES);
 #ifdef VK_BF16
         // Two chunks a wave are 128 registers of activations (16 rows, 34816 x 5120: 118 -> 87 us);
         // three did not fit beside the rest and were slower than none (4096 x 12288: 29 -> 36 us).
