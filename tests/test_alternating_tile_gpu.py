@@ -67,6 +67,20 @@ def test_columns_that_are_no_multiple_of_four(M, N, K):
     assert torch.equal(out[:, :N], gated) and bool((out[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(2048, 6144, 512), (3333, 4096, 512), (2048, 6150, 512), (1500, 5123, 1024)])
+def test_squared_relu_by_size(M, N, K):
+    """The activation in the epilogue, blocks that overlap the one before among them (they are computed and stored twice)."""
+    k = kern(torch.bfloat16)
+    act, w = rand((M, K), torch.bfloat16, 12).cuda(), rand((N, K), torch.bfloat16, 13, 0.1).cuda()
+    p, i, l = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    k.lib.vk_gemm_act.argtypes = [p, p, p, i, i, i, l, l, i, p]
+    for ldo in (N, (N + 7) // 4 * 4):
+        out = torch.full((M, ldo), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert k.lib.vk_gemm_act(out.data_ptr(), act.data_ptr(), w.data_ptr(), M, N, K, K, ldo, 1, torch.cuda.current_stream().cuda_stream) == 0
+        r = k.gemm(act, w, kernel=4).float().clamp(min=0)
+        assert torch.equal(out[:, :N], (r * r).to(torch.bfloat16)) and bool((out[:, N:] == 7.0).all())
+
+
 def test_sizes_below_a_tile_are_refused():
     k = kern(torch.bfloat16)
     w = rand((256, 512), torch.bfloat16, 7).cuda()
