@@ -101,7 +101,8 @@ __device__ __forceinline__ void wait_vmcnt_n() {             // vmcnt(N_), N_ be
 // 8 rows 14.1 -> 12.1; 2,048 x 6,144, 8 rows 11.6 -> 9.6; 1,024 x 3,072, 1 row 5.7 -> 5.2; 4,096 x 12,288, rows a chunk ahead, 1 and 16 rows
 // 21.2 -> 19.3, 28.9 -> 23.4; gate/up with SwiGLU 12,288 x 4,096, 8 rows 37.7 -> 36.5; 32-bit 2,048 x 2,048, 1 and 16 rows 9.6 -> 6.2, 11.9 -> 7.3.  Over
 // 315 sizes of 1 to 16 rows 5,163 -> 4,777 us in 16-bit, none more than 2 % over what it was, and 9,536 -> 8,496 in
-// 32-bit.  Part of it is the order of the weights' loads (EARLY in the kernels).  (Weights through LDS alike do not pay: they come from
+// 32-bit.  One row as such and not as eight is 2.4 % of that (2,048 x 9,216: 13.97 -> 13.01), two to four rows as four 1.2 % (6,144 x 2,560, 2 rows 9.28 ->
+// 8.98; 32-bit 24,600 x 512 11.33 -> 10.56).  Part of it is the order of the weights' loads (EARLY in the kernels).  (Weights through LDS alike do not pay: they come from
 // memory, 7.1 us for 33 MB against 7.4.  Tiles of eight or four weight rows for few of them do not either: 1,024 x 2,048 4.4 -> 4.6.)
 #define CHUNK_ROWS_BYTES(ROWS) ((ROWS) * KC * (int)sizeof(elem_t))
 template <int ROWS>
