@@ -19,6 +19,8 @@
 //                       sums meet in LDS and are added in chunk order.  W is eight, or, up to 16 rows, the
 //                       number of chunks where that is 2, 4, 5, 6, 10 or 12 (stream_waves).
 //   gemm_stream_swiglu  the same for the gate/up projection with SwiGLU folded in (M <= 16).
+//   gemm_lines          M <= 16, K a multiple of 512 up to 6,144, 16-bit elements: weights and activations through LDS in whole lines, tiles of eight
+//                       or four weight rows, optionally SwiGLU in the epilogue (lines_rows says when).
 //   gemm_mid            17 <= M <= 64, K a multiple of 512: 64 or 32 weight rows per workgroup, weights
 //                       streamed into registers, the activations of the chunks in work shared through LDS.
 //   gemm_split          M <= 64, K a multiple of 512, 16-bit elements, with a workspace: a workgroup per
@@ -82,6 +84,10 @@ __device__ __forceinline__ void store_out4(elem_t* out, int64_t ldo, int m, int 
 // block, anywhere in LDS (the grouped product's third stage starts at 96 KB).
 __device__ __forceinline__ void pipe_load_to_lds16_sv(const unsigned char* sbase, unsigned voff, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");     // m0 is the compiler's scratch: it sets it anew before every use of its own
+}
+// The same for bytes that one workgroup reads once: they pass through the caches without taking the place of what stays.
+__device__ __forceinline__ void pipe_load_to_lds16_once(const unsigned char* sbase, unsigned voff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 __device__ __forceinline__ unsigned lds_offset_of(const unsigned char* p) {
   return (unsigned)(unsigned long)((__attribute__((address_space(3))) const void*)p);
@@ -528,6 +534,197 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
     for (; tile < ntiles; tile += gridDim.x) one_tile(std::integral_constant<int, 2>());
   }
 }
+
+// ------------------------------------------------------------------- lines
+// Up to 16 rows of 16-bit elements, K of up to twelve chunks, one a wave.  What bounds such a product is how its weights come from memory.  In the operands'
+// own order (the streaming kernels) an instruction touches 16 rows, half a cache line of each: the address unit takes 64 clocks for a kilobyte, and
+// a line must stay in the first cache until its other half is asked for, so that the loads cannot say that they are the only ones.  Here a load
+// brings one row of a chunk, a whole kilobyte, into LDS, marked as read once: plain reads of 201 MB by 256 workgroups take 35.1 us in strides, 34.0 in pieces of
+// their own and 30.3 marked so (7.0 TB/s); 64-byte pieces marked so are slower than unmarked (36.7 -> 39).  The activations come the same way, once, and stay in
+// registers.  A workgroup walks over tiles of R weight rows with a ring of slots a wave; every wave waits for its own loads only, and a barrier a
+// tile stands between the chunk sums and the wave (another one each tile) that adds them in chunk order, the order of every kernel here.  With the
+// barrier a wave that is early cannot ask for more than its ring holds; counting arrivals in LDS instead, the last wave adding, was slower (4,096 x
+// 4,096, 8 rows 8.3 -> 8.4 us, gate/up 9,728 x 2,560 18.1 -> 19.1), as were sums read four or eight at a time.
+// Measured on MI355X, recorded launches with the weights of several layers in turn, us, against the streaming kernels: 1,024 x 2,048, 1 row 4.13 -> 3.22;
+// 1,024 x 3,072, 8 rows 5.7 -> 4.5; 2,048 x 2,048, 8 rows 4.6 -> 4.1; 2,048 x 6,144, 1 row 8.6 -> 6.4; 5,120 x 5,120, 8 rows 15.3 -> 11.7; 6,144 x 4,096, 8 rows
+// 12.2 -> 11.1; gate/up with SwiGLU 1,536 x 2,048, 8 rows 6.8 -> 5.3; 9,728 x 2,560 24.1 -> 18.2; 12,288 x 4,096 36.8 -> 34.3; 17,408 x 5,120 77.5 -> 58.3 (6.1 TB/s).
+// Not in 32-bit: four to eight of a product's sixteen rows leave three quarters or half of the matrix unit unused, which a 32-bit slab cannot spare
+// (2,048 x 2,048 6.4 -> 7.1).
+#ifdef VK_BF16
+// Rows of one chunk in LDS, a kilobyte each, the 16-byte piece j of row r at piece j ^ turn(r): the fragments of no two rows lie on the same banks, and
+// a load brings one row whole.
+template <int ROWS>
+struct LineRows {
+  static constexpr int ROW_BYTES = KC * (int)sizeof(elem_t);
+  static_assert(ROW_BYTES == 1024, "a load brings a row of a chunk");
+  __device__ static __forceinline__ int turn(int r) { return ROWS == 1 ? 0 : r * (16 / ROWS); }
+  // Asks for the rows from `first` on, `stride` elements apart; beyond the first `count` the last one again.
+  template <bool ONCE>
+  __device__ static __forceinline__ void ask(const elem_t* first, int64_t stride, int count, int lane, unsigned lds_addr) {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const unsigned char* row = reinterpret_cast<const unsigned char*>(first + (int64_t)min(r, count - 1) * stride);
+      const unsigned at = __builtin_amdgcn_readfirstlane(lds_addr + r * ROW_BYTES), piece = (unsigned)((lane ^ turn(r)) * 16);
+      if (ONCE) pipe_load_to_lds16_once(row, piece, at);
+      else pipe_load_to_lds16_sv(row, piece, at);
+    }
+  }
+  __device__ static __forceinline__ frag_t fragment(const unsigned char* rows, int slab, int r16, int kg) {      // rows beyond ROWS repeat them
+    const int r = r16 & (ROWS - 1);
+    return *reinterpret_cast<const frag_t*>(rows + r * ROW_BYTES + ((slab * 4 + kg) ^ turn(r)) * 16);
+  }
+};
+
+#define LINE_SLOTS 6                    // of a wave's ring, at most
+// What a launch fixes: bytes of LDS a wave has to itself, slots in them, and how many of those lie beside the activations.
+struct LinePlan {
+  int own_bytes, slots, first_slots;
+};
+template <int R, int ROWS, int P>
+__global__ __launch_bounds__(768) void gemm_lines_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w, int M, int N,
+                                                         int K, int64_t lda, int64_t ldo, int out_form, LinePlan plan) {
+  using W = LineRows<R>;
+  using A = LineRows<ROWS>;
+  constexpr int W_BYTES = R * 1024, SLOT = P * W_BYTES, L = P * R, SUMS = R / 4 * 16;      // L: loads of a slot; SUMS: lanes with sums
+  constexpr int S_MAX = 63 / L < LINE_SLOTS ? 63 / L : LINE_SLOTS;                         // no more loads than their counter counts
+  extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int S = plan.slots, step = gridDim.x, tiles = ((N + R - 1) / R - 1 - (int)blockIdx.x) / step + 1;      // of this workgroup, at least one
+  unsigned char* own = lines_lds + wave * plan.own_bytes;
+  f32x4* part = reinterpret_cast<f32x4*>(lines_lds + waves * plan.own_bytes);            // [2][waves][P][SUMS]
+  auto slot_at = [&](int s) { return own + plan.own_bytes - (s + 1) * SLOT; };            // the first ones lie beside the activations, the others in their place
+  auto ask = [&](int k, int s) {                            // the workgroup's tile k
+    const int tile = (int)blockIdx.x + k * step;
+    const elem_t* first = w + (int64_t)tile * R * K + wave * KC;
+    const unsigned at = lds_offset_of(slot_at(s));
+    W::template ask<true>(first, K, N - tile * R, lane, at);
+    if constexpr (P == 2) W::template ask<true>(first + (int64_t)N * K, K, N - tile * R, lane, at + W_BYTES);
+  };
+  auto wait_for_all_but = [&](int slots) {                  // the loads of that many slots, asked for last, may still be on their way
+    __builtin_amdgcn_sched_barrier(0);
+    if (S_MAX >= 6 && slots >= 6) wait_vmcnt_n<(S_MAX >= 6 ? 6 : 0) * L>();
+    else if (S_MAX >= 5 && slots == 5) wait_vmcnt_n<(S_MAX >= 5 ? 5 : 0) * L>();
+    else if (S_MAX >= 4 && slots == 4) wait_vmcnt_n<(S_MAX >= 4 ? 4 : 0) * L>();
+    else if (S_MAX >= 3 && slots == 3) wait_vmcnt_n<(S_MAX >= 3 ? 3 : 0) * L>();
+    else if (S_MAX >= 2 && slots == 2) wait_vmcnt_n<(S_MAX >= 2 ? 2 : 0) * L>();
+    else if (slots == 1) wait_vmcnt_n<L>();
+    else wait_vmcnt_n<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto lds_done = [&]() {                                   // this wave's accesses to LDS: what it has read may be overwritten, what it wrote is there
+    __builtin_amdgcn_s_waitcnt(0xC07F);                    // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int before = min(plan.first_slots, tiles);
+  A::template ask<false>(act + wave * KC, lda, M, lane, lds_offset_of(own));
+#pragma unroll
+  for (int s = 0; s < S_MAX; ++s)
+    if (s < before) ask(s, s);
+  wait_for_all_but(before);
+  frag_t rows[KC_SLABS];
+#pragma unroll
+  for (int i = 0; i < KC_SLABS; ++i) rows[i] = A::fragment(own, i, r16, kg);
+  lds_done();
+#pragma unroll
+  for (int s = 0; s < S_MAX; ++s)
+    if (s >= before && s < S && s < tiles) ask(s, s);
+  int s = 0;
+  for (int k = 0; k < tiles; ++k) {
+    wait_for_all_but(min(S, tiles - k) - 1);
+    const unsigned char* at = slot_at(s);
+    f32x4 acc[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < KC_SLABS; ++i)
+#pragma unroll
+      for (int p = 0; p < P; ++p) acc[p] = mma_slab(W::fragment(at + p * W_BYTES, i, r16, kg), rows[i], acc[p]);
+    f32x4* sums = part + (k & 1) * waves * P * SUMS;
+    if (lane < SUMS) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) sums[(wave * P + p) * SUMS + lane] = acc[p];
+    }
+    lds_done();
+    if (k + S < tiles) ask(k + S, s);
+    s = s + 1 == S ? 0 : s + 1;
+    __builtin_amdgcn_s_barrier();                           // (the loads that are on their way need no wait here)
+    asm volatile("" ::: "memory");
+    if (wave == k % waves && lane < SUMS) {                 // in chunk order; these sums' place is written again two barriers on
+      const int n0 = ((int)blockIdx.x + k * step) * R;
+      f32x4 total[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) total[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < waves; ++c) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const f32x4 v = sums[(c * P + p) * SUMS + lane];
+          total[p].x = total[p].x + v.x; total[p].y = total[p].y + v.y; total[p].z = total[p].z + v.z; total[p].w = total[p].w + v.w;
+        }
+      }
+      if constexpr (P == 2) {
+        const float g[4] = {round_to_elem(total[0].x), round_to_elem(total[0].y), round_to_elem(total[0].z), round_to_elem(total[0].w)};
+        const float u[4] = {round_to_elem(total[1].x), round_to_elem(total[1].y), round_to_elem(total[1].z), round_to_elem(total[1].w)};
+        total[0].x = (g[0] * (1.0f / (1.0f + expf(-g[0])))) * u[0];
+        total[0].y = (g[1] * (1.0f / (1.0f + expf(-g[1])))) * u[1];
+        total[0].z = (g[2] * (1.0f / (1.0f + expf(-g[2])))) * u[2];
+        total[0].w = (g[3] * (1.0f / (1.0f + expf(-g[3])))) * u[3];
+      }
+      store_out4(out, ldo, r16, n0 + 4 * kg, M, min(N, n0 + R), total[0], out_form);
+    }
+  }
+}
+
+// How gemm_lines_kernel's LDS is laid out for M rows of K and tiles of R weight rows of each projection; false: it does not take them.
+static bool line_plan(int M, int K, int R, int projections, LinePlan* plan, int* lds_bytes) {
+  const int waves = K / KC, rows = M == 1 ? 1 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
+  if (M < 1 || M > 16 || K % KC != 0 || waves < 1 || waves > 12) return false;
+  const int slot = projections * R * 1024, sums = 2 * waves * projections * R / 4 * 256;
+  const int most = 63 / (projections * R) < LINE_SLOTS ? 63 / (projections * R) : LINE_SLOTS;
+  for (int groups = 16 / waves > 1 ? 16 / waves : 1; groups >= 1; --groups) {               // a compute unit's LDS among about 16 waves
+    int own = ((160 * 1024 / groups - sums) / waves) & ~1023;
+    if (own < slot || own < rows * 1024 || (groups > 1 && own < slot + rows * 1024)) continue;
+    plan->slots = own / slot < most ? own / slot : most;
+    if (plan->slots * slot + rows * 1024 < own) own = plan->slots * slot + rows * 1024;
+    plan->own_bytes = own;
+    plan->first_slots = (own - rows * 1024) / slot < plan->slots ? (own - rows * 1024) / slot : plan->slots;
+    *lds_bytes = waves * own + sums;
+    return true;
+  }
+  return false;
+}
+template <int R, int ROWS, int P>
+static int launch_lines_of(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, const LinePlan& plan, int lds_bytes,
+                           hipStream_t st) {
+  static bool configured = false;
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_lines_kernel<R, ROWS, P>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    configured = true;
+  }
+  const int waves = K / KC;
+  static int per_cu[16] = {};                               // workgroups that a compute unit holds, by waves (which fix the LDS)
+  if (per_cu[waves] == 0) {
+    int held = 0;
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&held, gemm_lines_kernel<R, ROWS, P>, 64 * waves, lds_bytes);
+    per_cu[waves] = held > 0 ? held : 1;
+  }
+  const int tiles = (N + R - 1) / R, resident = per_cu[waves] * vk_device_cus();
+  gemm_lines_kernel<R, ROWS, P><<<tiles < resident ? tiles : resident, 64 * waves, lds_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form, plan);
+  return vk_check_launch("gemm_lines");
+}
+template <int R, int P>
+static int launch_lines(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, hipStream_t st) {
+  LinePlan plan;
+  int lds = 0;
+  VK_REQUIRE(line_plan(M, K, R, P, &plan, &lds), "gemm: %d rows of K=%d do not fit a workgroup of %d weight rows", M, K, R);
+  if (M == 1) return launch_lines_of<R, 1, P>(out, act, w, M, N, K, lda, ldo, form, plan, lds, st);
+  if (M <= 4) return launch_lines_of<R, 4, P>(out, act, w, M, N, K, lda, ldo, form, plan, lds, st);
+  if (M <= 8) return launch_lines_of<R, 8, P>(out, act, w, M, N, K, lda, ldo, form, plan, lds, st);
+  return launch_lines_of<R, 16, P>(out, act, w, M, N, K, lda, ldo, form, plan, lds, st);
+}
+#endif
 
 // ------------------------------------------------------------------- tiled
 // Workgroup of four waves (2 x 2); a wave owns FN x FM tiles of 16 x 16, so the
@@ -1572,6 +1769,7 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //   k_resident             K <= 8 chunks: each of a workgroup's 8 waves has one chunk, whose activations stay in registers
 //
 //   rows     condition                                         kernel
+//   1..16    where lines_rows says so                           20, 21  whole lines
 //   1..16                                                      1   streaming
 //   17..32   16-bit, K whole chunks, k_resident,               11  streaming, both activation tiles of a wave's chunk in
 //            wg16 >= 1.5 cus                                       registers (32 rows, 24576 x 4096: 53 -> 44 us)
@@ -1622,6 +1820,38 @@ static int choose_gemm_kernel(int M, int N, int K) {
     return (k_resident && many16) ? 2 : 8;
   }
   return 2;
+}
+
+// How many weight rows a tile of gemm_lines_kernel has for a product of these sizes (8 or 4), or 0: a streaming kernel is the faster one.
+// Measured over 2,233 sizes (N of 256 to 32,768, K of 512 to 6,144, 1 to 16 rows, with and without SwiGLU): 30.9 ms with the streaming kernels, 27.4 with the
+// better one everywhere.  With tiles of 16 weight rows for the streaming kernel's workgroups:
+//   at most one for two compute units     whole lines from two chunks on (1.0 to 2.4 times; nine rows and more of two chunks without SwiGLU 0.94 to 1.04: from three)
+//   up to one a compute unit             the streaming kernel asks for all it needs at once and has no second tile: 0.85 to 1.03 below eight chunks (five
+//                                         with SwiGLU, up to seven), 0.99 to 1.11 from there on
+//   more                                 the streaming kernel's last round is partly empty: 1.0 to 1.45 from four chunks on (with SwiGLU from two, up to eight
+//                                         rows); only where two rounds are just filled and nine rows and more 0.94 to 0.98 below eight chunks
+// Tiles of eight rows, or of four where those of eight leave more than half of the units without one, or do not fit.
+static int lines_rows(int M, int N, int K, int projections) {
+#ifdef VK_BF16
+  if (M > 16 || K % KC != 0) return 0;
+  const int cus = vk_device_cus(), chunks = K / KC, tiles16 = (N + 15) / 16;
+  const bool swiglu = projections == 2;
+  if (2 * tiles16 <= cus) {
+    if (chunks < 2 || (!swiglu && chunks == 2 && M > 8)) return 0;
+  } else if (tiles16 <= cus) {
+    if (swiglu ? chunks < 5 || chunks > 7 : chunks < 8) return 0;
+  } else {
+    if (chunks < (swiglu && M <= 8 ? 2 : 4)) return 0;
+    if (!swiglu && M > 8 && chunks < 8 && tiles16 <= 2 * cus && 16 * tiles16 > 30 * cus) return 0;
+  }
+  LinePlan plan;
+  int lds = 0;
+  if (N > 2 * cus && line_plan(M, K, 8, projections, &plan, &lds)) return 8;
+  return line_plan(M, K, 4, projections, &plan, &lds) ? 4 : 0;
+#else
+  (void)M; (void)N; (void)K; (void)projections;
+  return 0;
+#endif
 }
 
 // How many 16-row weight fragments a wave of the tile kernel takes (a workgroup: 32 of them in weight rows).  The
@@ -1739,7 +1969,8 @@ int vk_gemm_grouped_act(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // (17 to 512 rows, in blocks of 64 rows), 11 = skinny with two activation tiles resident in registers (17 to
 // 32 rows of 16-bit elements, K <= 4096), 12 = as 9 in blocks of 32 rows, 13, 15 and 16 = pipelined with 64, 96
 // and 160 weight rows per workgroup (14 is the callers' name for the route through chunk sums), 17, 18 and 19 = alternating
-// with 192, 160 and 128 weight rows per workgroup (256 rows or more, 16-bit elements, K a multiple of 512); for measurements and tests.  The result does not depend on the choice.
+// with 192, 160 and 128 weight rows per workgroup (256 rows or more, 16-bit elements, K a multiple of 512), 20 and 21 = whole lines in
+// tiles of 4 and 8 weight rows (1 to 16 rows, 16-bit elements, K a multiple of 512 up to 6,144 and as many rows as fit the LDS); for measurements and tests.  The result does not depend on the choice.
 static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
                        int kernel, int activation, hipStream_t st) {
   VK_REQUIRE(activation == 0 || activation == 1, "gemm: unknown activation %d", activation);
@@ -1749,15 +1980,22 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
              (long long)lda, VK_VEC);
   VK_REQUIRE(ldo >= N, "gemm: output row stride %lld is smaller than N=%d", (long long)ldo, N);
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm: operands must be 16-byte aligned");
-  VK_REQUIRE(kernel >= 0 && kernel <= (sizeof(elem_t) == 2 ? 19 : 16) && kernel != 14, "gemm: unknown kernel %d", kernel);      // the alternating one takes 16-bit elements
+  VK_REQUIRE(kernel >= 0 && kernel <= (sizeof(elem_t) == 2 ? 21 : 16) && kernel != 14, "gemm: unknown kernel %d", kernel);      // the alternating one takes 16-bit elements
   if (M == 0) return 0;
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
-  if (kernel == 0) kernel = choose_gemm_kernel(M, N, K);
+  if (kernel == 0) {
+    const int rows = lines_rows(M, N, K, 1);
+    kernel = rows ? (rows == 4 ? 20 : 21) : choose_gemm_kernel(M, N, K);
+  }
 #ifdef VK_BF16
   if (kernel == 17) return launch_alternate<6, 2, 3>(out, act, w, M, N, K, lda, ldo, form, st);
   if (kernel == 18) return launch_alternate<5, 3, 3>(out, act, w, M, N, K, lda, ldo, form, st);
   if (kernel == 19) return launch_alternate<4, 3, 4>(out, act, w, M, N, K, lda, ldo, form, st);
+#endif
+#ifdef VK_BF16
+  if (kernel == 20) return launch_lines<4, 1>(out, act, w, M, N, K, lda, ldo, form, st);
+  if (kernel == 21) return launch_lines<8, 1>(out, act, w, M, N, K, lda, ldo, form, st);
 #endif
   if (kernel == 12) {      // 32 weight rows per workgroup, four chunks in work, blocks of 32 rows
     VK_REQUIRE(M > 16 && M <= 512 && K % KC == 0, "gemm: the mid kernel takes 17 to 512 rows and K a multiple of %d", KC);
@@ -1833,8 +2071,8 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
         else if (nw == 5) STN(5);
         else if (nw == 6) STN(6);
 #ifdef VK_BF16
-        else if (nw == 10) STN(10);
-        else if (nw == 12) STN(12);
+        else if (nw == 10) STW(1, 8, 1, 1, 10);         // nine rows and more (lines_rows takes the others), which do not fit the LDS
+        else if (nw == 12) STW(1, 8, 1, 1, 12);
 #endif
         else
         if (kernel == 7 || (by_size && K > SK_WAVES * KC && tiles16 > cus && 2 * tiles16 <= 3 * cus)) ST(1, 8, 0, 2);
@@ -1976,6 +2214,11 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   }
   const int ntiles = (I + 15) / 16;
   const int form = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
+#ifdef VK_BF16
+  const int lines = lines_rows(M, I, K, 2);
+  if (lines == 4) return launch_lines<4, 2>(out, act, w, M, I, K, lda, ldo, form, st);
+  if (lines == 8) return launch_lines<8, 2>(out, act, w, M, I, K, lda, ldo, form, st);
+#endif
 #define SWIGLU_STREAMH(W, MT, RC, NW, ROWS)                                                               \
   do {                                                                                                     \
     constexpr size_t rows_bytes = (size_t)NW * CHUNK_ROWS_BYTES(ROWS);                                \
@@ -2052,10 +2295,11 @@ int64_t vk_gemm_split_floats(int M, int rows, int K, int swiglu) {
 //   Up to 16 rows the streaming kernel is the other choice.  With `fill` the share of the compute units that
 //   its last round of one workgroup per 16 weight rows keeps busy:
 //     K of more than 16 chunks (its waves read their activations again for every chunk): when fill < 0.9
-//       (8 rows: 5120 x 17408 56.8 -> 41.7 us, 5120 x 25600 80.8 -> 57.8, 2560 x 9728 19.7 -> 15.3) or from 8 rows on
-//       (4096 x 12288, fill 1: 1 row 23.0 -> 24.5 us, 4 rows 24.7 -> 24.5, 8 rows 27.2 -> 23.9, 16 rows 29.3 -> 24.0);
-//     K of 9 to 16 chunks: when fill < 0.7 (8 rows: 5120 x 5120 18.5 -> 16.6 us, 5120 x 8192 25.9 -> 24.0, 2048 x
-//       6144 11.2 -> 9.6; but 7168 x 5120, fill 0.88, 19.1 -> 21.2);
+//       (8 rows: 5120 x 17408 52.8 -> 40.3 us, 2560 x 9728 16.2 -> 14.9) or from 13 rows on
+//       (4096 x 12288, fill 1: 1 row 19.4 -> 23.5 us, 8 rows 20.9 -> 23.7, 12 rows 22.6 -> 23.7, 16 rows 23.4 -> 23.7; 8192 x 12288: 8 rows 38.2 -> 42.7, 12 rows
+//       42.6 -> 42.4, 16 rows 44.5 -> 42.4);
+//     K of 9 to 16 chunks, where lines_rows does not take it: when fill < 0.7 (2048 x 8192, 8 rows 16.1 -> 11.4 us, 5120 x 5120, 16 rows 17.9 -> 16.7; but
+//       7168 x 5120, fill 0.88, 16 rows 19.2 -> 21.0);
 //     K of up to 8 chunks: never (4096 x 4096 9.1 -> 10.3 us, 2560 x 4096, fill 0.63, 8.3 -> 9.2).
 int vk_gemm_split_preferred(int M, int rows, int K, int swiglu) {
   if (swiglu || vk_gemm_split_floats(M, rows, K, swiglu) == 0) return 0;
@@ -2063,10 +2307,11 @@ int vk_gemm_split_preferred(int M, int rows, int K, int swiglu) {
   const int64_t bytes = (int64_t)rows * K * (int64_t)sizeof(elem_t);
   if (bytes < (int64_t)cus * 65536 || 4 * ((rows + 127) / 128) > cus) return 0;
   if (M > 16) return 1;
+  if (lines_rows(M, rows, K, 1)) return 0;
   const int nchunks = K / KC, tiles16 = (rows + 15) / 16;
   const int rounds = (tiles16 + cus - 1) / cus;
   const bool fill_below_09 = 10 * tiles16 < 9 * rounds * cus, fill_below_07 = 10 * tiles16 < 7 * rounds * cus;
-  if (nchunks > 2 * SK_WAVES) return fill_below_09 || M >= 8;
+  if (nchunks > 2 * SK_WAVES) return fill_below_09 || M > 12;
   return nchunks > SK_WAVES && fill_below_07;
 }
 
