@@ -47,3 +47,11 @@ def test_sizes_that_do_not_fit():
             k.gemm(rand((rows, 512 * chunks), B, 6).cuda(), w[:, :512 * chunks].contiguous(), kernel=21)
     with pytest.raises(KernelError):
         kern(torch.float32).gemm(torch.zeros(1, 512, device="cuda"), torch.zeros(8, 512, device="cuda"), kernel=20)
+
+
+@pytest.mark.parametrize("N,K", [(1449, 800), (1702, 1024), (1393, 1184), (1301, 1536), (1500, 2048), (1100, 2336), (700, 3072), (699, 3104), (700, 4096), (64, 8192)])
+def test_experts(N, K):
+    """Experts' products from the line on at which their weights come in whole lines, for every number of chunks, whole and not; features that end inside a
+    group of eight."""
+    from test_expert_tiles_gpu import test_tiles_get_the_plain_product
+    test_tiles_get_the_plain_product(N, K, B)
