@@ -89,6 +89,8 @@ struct Kernels::Fn {
   int (*gemm)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_swiglu)(P, CP, CP, int, int, int, int64_t, int64_t, hipStream_t);
   int (*gemm_swiglu_supported)(int, int, int);
+  int (*gemm_normed_takes)(int, int, int, int);
+  int (*gemm_normed)(P, P, CP, CP, CP, float, CP, int, int, int, int64_t, int, hipStream_t);
   int (*gemm_split)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
   int64_t (*gemm_split_floats)(int, int, int, int);
   int (*gemm_split_preferred)(int, int, int, int);
@@ -193,6 +195,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(embedding, "vk_embedding"); VK(rmsnorm, "vk_rmsnorm"); VK(add_rmsnorm, "vk_add_rmsnorm"); VK(swiglu, "vk_swiglu");
   VK(gather_rows, "vk_gather_rows"); VK(cast_to_f32, "vk_cast_to_f32"); VK(copy_out, "vk_copy_out"); VK(rope_tables, "vk_rope_tables"); VK(fill_random, "vk_fill_random");
   VK(gemm, "vk_gemm"); VK(gemm_swiglu, "vk_gemm_swiglu"); VK(gemm_swiglu_supported, "vk_gemm_swiglu_supported");
+  VK(gemm_normed_takes, "vk_gemm_normed_takes"); VK(gemm_normed, "vk_gemm_normed");
   VK(gemm_split, "vk_gemm_split"); VK(gemm_split_floats, "vk_gemm_split_floats"); VK(gemm_split_preferred, "vk_gemm_split_preferred");
   VK(qkv_post, "vk_qkv_post"); VK(paged_attention, "vk_paged_attention"); VK(sample, "vk_sample");
   VK(sample_scratch_words, "vk_sample_scratch_words"); VK(attn_scratch_floats, "vk_attn_scratch_floats");
@@ -416,6 +419,24 @@ Tensor Kernels::gemm_swiglu(const Tensor& act, const Tensor& w, const Tensor* wo
   Tensor out = empty({M, I});
   if (split(out, act, w, true, workspace)) return out;
   call(fn_->gemm_swiglu(out.data, act.data, w.data, (int)M, (int)I, (int)K, K, I, stream));
+  return out;
+}
+
+bool Kernels::added_takes(const AddedRows& in, int64_t N, bool swiglu) const {
+  const Tensor &x = in.x, &r = in.residual;
+  if (!in.weight || in.weight->dtype != dtype_ || x.dtype != dtype_ || r.dtype != dtype_ || x.shape.size() != 2 || r.shape != x.shape) return false;
+  if (in.weight->numel() != x.dim(1) || (swiglu && N % 2) || x.dim(0) > 8) return false;
+  return fn_->gemm_normed_takes((int)x.dim(0), (int)(swiglu ? N / 2 : N), (int)x.dim(1), swiglu ? 2 : 1) != 0;
+}
+
+Tensor Kernels::gemm_added(const AddedRows& in, const Tensor& w, bool swiglu, Tensor& sum) {
+  expect(w, "weight", dtype_);
+  if (w.shape.size() != 2 || !added_takes(in, w.dim(0), swiglu) || w.dim(1) != in.x.dim(1))
+    throw EngineError("gemm_added: rows " + in.x.describe() + " and " + in.residual.describe() + " with weight " + w.describe());
+  const int64_t M = in.x.dim(0), N = swiglu ? w.dim(0) / 2 : w.dim(0);
+  sum = empty(in.x.shape);
+  Tensor out = empty({M, N});
+  call(fn_->gemm_normed(out.data, sum.data, in.x.data, in.residual.data, in.weight->data, in.eps, w.data, (int)M, (int)N, (int)in.x.dim(1), N, swiglu ? 2 : 1, stream));
   return out;
 }
 

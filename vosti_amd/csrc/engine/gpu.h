@@ -126,6 +126,16 @@ class Kernels {
   // take a faster route to the same bits.  activation 1: the square of max(., 0) on the rounded outputs, in the same launch.
   Tensor gemm(const Tensor& act, const Tensor& w, const Tensor* workspace = nullptr, int activation = 0);
   Tensor gemm_swiglu(const Tensor& act, const Tensor& w_gate_up, const Tensor* workspace = nullptr);
+  // Rows x + residual, not yet added and normed: what a product may do itself (gemm_added).
+  struct AddedRows {
+    Tensor x, residual;
+    const Tensor* weight = nullptr;
+    float eps = 0.f;
+  };
+  // Whether gemm_added takes so many rows of K and this weight [N, K] (with swiglu: gate and up rows, N in all), where that is the faster way.
+  bool added_takes(const AddedRows& in, int64_t N, bool swiglu) const;
+  // gemm or gemm_swiglu of the norm of x + residual; sum receives the sum's rows, which add_rmsnorm leaves in the residual.  One launch, the same bits.
+  Tensor gemm_added(const AddedRows& in, const Tensor& w, bool swiglu, Tensor& sum);
   // float32 elements of workspace with which gemm / gemm_swiglu take the route through chunk sums for these
   // sizes, or 0 where that route does not exist or is the slower one.
   int64_t gemm_workspace_floats(int64_t M, int64_t rows, int64_t K, bool swiglu = false) const;

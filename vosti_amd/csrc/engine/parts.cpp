@@ -113,6 +113,15 @@ std::pair<Tensor, Tensor> Block::rows_for_the_end(const Tensor& hidden, const Te
   return {kernels.gather_rows(hidden, rows), residual.data ? kernels.gather_rows(residual, rows) : Tensor()};
 }
 
+Tensor Mixer::forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx, CacheEntry& cache) {
+  (void)in; (void)sum; (void)ctx; (void)cache;
+  throw EngineError("this mixer kind does not norm its rows itself");
+}
+Tensor FeedForward::forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx) {
+  (void)in; (void)sum; (void)ctx;
+  throw EngineError("this feed-forward kind does not norm its rows itself");
+}
+
 void Norm::forward_scaled_add(const Tensor& y, const Tensor& base, Tensor& out, float mult, Tensor* rounded) {
   (void)y; (void)base; (void)out; (void)mult; (void)rounded;
   throw EngineError("this norm kind cannot add its scaled output to a 32-bit residual stream");
@@ -685,10 +694,18 @@ class Attention : public Mixer {
     return need;
   }
 
-  Tensor forward(const Tensor& x, StepContext& ctx, CacheEntry& cache) override {
+  // Rows of the stacked weight that an execution on this cache projects: all, or (another's keys and values) q's, the first.
+  int64_t projected(const CacheEntry& cache) const { return cache.writable || !own_kv_ || gate_ ? w_qkv_.dim(0) : (int64_t)nq_ * d_; }
+  bool takes_added(const Kernels::AddedRows& in, const CacheEntry& cache) const override { return kernels.added_takes(in, projected(cache), false); }
+  Tensor forward(const Tensor& x, StepContext& ctx, CacheEntry& cache) override { return run(&x, nullptr, nullptr, ctx, cache); }
+  Tensor forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx, CacheEntry& cache) override { return run(nullptr, &in, &sum, ctx, cache); }
+
+ private:
+  // On x, or on added rows that the first product norms.
+  Tensor run(const Tensor* x, const Kernels::AddedRows* added, Tensor* sum, StepContext& ctx, CacheEntry& cache) {
     if (cache.kind != CacheNeed::Pages) throw EngineError("attention was handed a cache entry without pages");
     Kernels& k = kernels;
-    const int64_t T = x.dim(0);
+    const int64_t T = x ? x->dim(0) : added->x.dim(0);
     GroupTables& tables = ctx.groups.at(cache.group);
     // Without a cache of its own the keys and values are an earlier execution's: only q is projected.
     // The projections, the attention of decoded tokens and the next projection use the step's workspace one
@@ -701,10 +718,10 @@ class Attention : public Mixer {
     // Rows of the stacked weight: q, then k and v (where the layer has them), then the output gate.  An execution that
     // reads another's cache projects q and the gate alone; without a gate, q's rows are the first of the weight.
     const int64_t heads_w = (int64_t)(nq_ + (cache.writable ? 2 * nkv_ : 0)) * d_;
-    Tensor qkv_all;
-    if (cache.writable || !own_kv_) qkv_all = k.gemm(x, w_qkv_, ws);
-    else if (!gate_) qkv_all = k.gemm(x, w_qkv_.rows(0, (int64_t)nq_ * d_), ws);
-    else throw EngineError("an attention layer with an output gate and projections of its own cannot read another execution's cache");
+    if (!cache.writable && own_kv_ && gate_)
+      throw EngineError("an attention layer with an output gate and projections of its own cannot read another execution's cache");
+    const Tensor w = projected(cache) == w_qkv_.dim(0) ? w_qkv_ : w_qkv_.rows(0, projected(cache));
+    const Tensor qkv_all = x ? k.gemm(*x, w, ws) : k.gemm_added(*added, w, false, *sum);
     const bool padded_norm = d_ != dk_ && (q_norm_ || k_norm_);
     const bool norm_angles = position_ && position_->angle_frequencies() && (q_norm_ || k_norm_) && fused();
     if (padded_norm && !norm_angles && !prepared()) throw ConfigError("attention: head norms on padded head sizes are built for rotations by computed angles only");
@@ -770,7 +787,6 @@ class Attention : public Mixer {
     return k.gemm(heads, w_o_, ws);
   }
 
- private:
   // Norms, rotation, the values' blend and the store in one launch (qkv_prepare).
   Tensor prepare(const Tensor& qkv, StepContext& ctx, CacheEntry& cache, GroupTables& tables) {
     if (!cache.writable) throw EngineError("attention: unit or whole norms and mixed values need a cache of the layer's own");
@@ -892,14 +908,19 @@ class SwiGLU : public FeedForward {
     for (int q : step.q_lens) T += q;
     return gemm_floats(T);
   }
-  Tensor forward(const Tensor& x, StepContext& ctx) override {
-    const int64_t n = gemm_floats(x.dim(0));
-    Tensor ws;
-    if (n) ws = ctx.workspace(n);
-    return kernels.gemm(kernels.gemm_swiglu(x, w_gate_up_, n ? &ws : nullptr), w_down_, n ? &ws : nullptr);
-  }
+  bool takes_added(const Kernels::AddedRows& in) const override { return kernels.added_takes(in, w_gate_up_.dim(0), true); }
+  Tensor forward(const Tensor& x, StepContext& ctx) override { return run(&x, nullptr, nullptr, ctx); }
+  Tensor forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx) override { return run(nullptr, &in, &sum, ctx); }
 
  private:
+  Tensor run(const Tensor* x, const Kernels::AddedRows* added, Tensor* sum, StepContext& ctx) {
+    const int64_t n = gemm_floats(x ? x->dim(0) : added->x.dim(0));
+    Tensor ws;
+    if (n) ws = ctx.workspace(n);
+    const Tensor inner = x ? kernels.gemm_swiglu(*x, w_gate_up_, n ? &ws : nullptr) : kernels.gemm_added(*added, w_gate_up_, true, *sum);
+    return kernels.gemm(inner, w_down_, n ? &ws : nullptr);
+  }
+
   int64_t hidden_, inter_, inter_run_ = 0;   // inter_run_: the intermediate size as the kernels see it
   Tensor w_gate_up_, w_down_;
 };
@@ -957,22 +978,30 @@ class PreNormBlock : public Block {
   }
   Mixer& mixer() override { return *mixer_; }
   std::pair<Tensor, Tensor> forward(const Tensor& hidden, Tensor residual, StepContext& ctx, CacheEntry& cache) override {
-    Tensor normed;
+    // Few rows: a sublayer whose first product adds and norms them itself saves a launch.
+    Tensor mixed, sum;
     if (residual.data == nullptr) {
       residual = hidden;
-      normed = norms_["input"]->forward(hidden);
+      mixed = mixer_->forward(norms_["input"]->forward(hidden), ctx, cache);
+    } else if (const Kernels::AddedRows in = added(*norms_["input"], hidden, residual); mixer_->takes_added(in, cache)) {
+      mixed = mixer_->forward_added(in, sum, ctx, cache);
+      residual = sum;
     } else {
-      normed = norms_["input"]->forward_add(hidden, residual);
+      mixed = mixer_->forward(norms_["input"]->forward_add(hidden, residual), ctx, cache);
     }
-    const Tensor mixed = mixer_->forward(normed, ctx, cache);
     if (!has_ffn_) return {mixed, residual};
-    normed = norms_["post_mixer"]->forward_add(mixed, residual);
+    if (const Kernels::AddedRows in = added(*norms_["post_mixer"], mixed, residual); ffn_->takes_added(in)) {
+      const Tensor out = ffn_->forward_added(in, sum, ctx);
+      return {out, sum};
+    }
+    const Tensor normed = norms_["post_mixer"]->forward_add(mixed, residual);
     return {ffn_->forward(normed, ctx), residual};
   }
 
  private:
   std::unique_ptr<Mixer> mixer_;
   std::unique_ptr<FeedForward> ffn_;
+  static Kernels::AddedRows added(const Norm& norm, const Tensor& x, const Tensor& residual) { return {x, residual, norm.row_scale_weight(), norm.eps()}; }
   std::map<std::string, std::unique_ptr<Norm>> norms_;
   bool has_ffn_ = true;
 };

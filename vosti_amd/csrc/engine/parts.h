@@ -163,12 +163,17 @@ class Mixer : public Part {
   using Part::Part;
   virtual CacheNeed cache_need() const = 0;
   virtual Tensor forward(const Tensor& x, StepContext& ctx, CacheEntry& cache) = 0;
+  // Whether the mixer runs on rows that it adds and norms itself (Kernels::gemm_added); forward_added is forward() on their norm and gives their sum.
+  virtual bool takes_added(const Kernels::AddedRows& in, const CacheEntry& cache) const { (void)in; (void)cache; return false; }
+  virtual Tensor forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx, CacheEntry& cache);
 };
 
 class FeedForward : public Part {
  public:
   using Part::Part;
   virtual Tensor forward(const Tensor& x, StepContext& ctx) = 0;
+  virtual bool takes_added(const Kernels::AddedRows& in) const { (void)in; return false; }        // as a mixer's
+  virtual Tensor forward_added(const Kernels::AddedRows& in, Tensor& sum, StepContext& ctx);
 };
 
 class Head : public Part {

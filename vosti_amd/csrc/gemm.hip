@@ -35,6 +35,7 @@
 //                       waves whose two halves take turns between LDS and the matrix unit.  Optionally SwiGLU in the epilogue
 //                       (alternate_fragments says when).
 //   gemm_tiled          any M and K: the same tile through registers into LDS, predicated.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -104,6 +105,9 @@ struct ChunkRows {
     const int r = r16 & (PER - 1), h = ROWS == 16 ? r16 >> 3 : 0, piece = slab * 4 + kg;
     return *reinterpret_cast<const frag_t*>(rows + h * HALF + (piece / PIECES) * 1024 + r * (1024 / PER) + ((piece % PIECES) ^ (r * TURN)) * 16);
   }
+  __device__ static __forceinline__ unsigned char* place(unsigned char* rows, int row, int piece) {      // of one of the first eight rows
+    return rows + (piece / PIECES) * 1024 + row * (1024 / PER) + ((piece % PIECES) ^ (row * TURN)) * 16;
+  }
 };
 // Asks for them: LOADS loads.
 template <int ROWS>
@@ -117,6 +121,106 @@ __device__ __forceinline__ void ask_chunk_rows(const elem_t* act, int64_t lda, i
       pipe_load_to_lds16_sv(reinterpret_cast<const unsigned char*>(act) + i * (1024 / C::PER), voff, __builtin_amdgcn_readfirstlane(lds_addr + h * C::HALF + i * 1024));
   }
 }
+
+// The activations of a product that norms them itself: row m is (x + residual) * rsqrt(mean(.^2) + eps) * weight, the sum in 32-bit, and the sum's rounded rows
+// go to `sum` (the first workgroup writes them): what vk_add_rmsnorm computes, bit for bit, its order of additions included.
+struct NormArgs {
+  const elem_t* residual;    // [M, K]
+  elem_t* sum;               // [M, K]
+  const elem_t* weight;      // [K]
+  float eps;
+};
+// Up to ROWS rows of NW chunks by NW waves.  vk_add_rmsnorm's workgroup of four waves takes the kilobytes (groups) of a row in turn, wave q those with g % 4 ==
+// q, and adds its own partial sums first: here a (row, q) pair is one wave's, all pairs in turn, a lane holding what that kernel's lane holds.
+// load() reads the rows and waits for them (a weight asked for before them would have to arrive first: loads are counted in order); the weights
+// are asked for next, and finish() sums, norms and puts the rows into LDS meanwhile.  A norm of its own is a launch of 3.6 us of eight rows of 4,096 and 2.6 of one
+// of 1,024 between two products (normed_product has the pairs measured).
+template <int ROWS, int NW>
+struct NormRows {
+  static constexpr int GROUPS = NW * KC * (int)sizeof(elem_t) / 1024, Q = GROUPS < 4 ? GROUPS : 4, J = (GROUPS + 3) / 4, PAIRS = (ROWS * Q + NW - 1) / NW;
+  float a[PAIRS][J][VK_VEC];
+  frag_t w[PAIRS][J];
+  __device__ __forceinline__ void load(const NormArgs& n, const elem_t* x, int64_t ldx, int M, int wave, int lane) {
+    constexpr int K = NW * KC;
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i) {
+      const int p = wave + i * NW, row = p / Q;
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int g = p % Q + 4 * j;
+        if (row < M && g < GROUPS) {
+          w[i][j] = *reinterpret_cast<const frag_t*>(n.weight + (g * 64 + lane) * VK_VEC);
+          float b[VK_VEC];
+          load_elems(x + row * ldx + (g * 64 + lane) * VK_VEC, a[i][j]);
+          load_elems(n.residual + (int64_t)row * K + (g * 64 + lane) * VK_VEC, b);
+#pragma unroll
+          for (int e = 0; e < VK_VEC; ++e) a[i][j][e] = a[i][j][e] + b[e];
+        }
+      }
+    }
+    if (blockIdx.x == 0) {
+#pragma unroll
+      for (int i = 0; i < PAIRS; ++i) {
+        const int p = wave + i * NW, row = p / Q;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int g = p % Q + 4 * j;
+          if (row < M && g < GROUPS) store_elems(n.sum + (int64_t)row * K + (g * 64 + lane) * VK_VEC, a[i][j]);
+        }
+      }
+    }
+  }
+  // A barrier that waits for what went to LDS, and not for the loads on their way.
+  __device__ static __forceinline__ void meet() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  // red: [ROWS][4] floats of LDS; place(row, g): where the lane's 16 bytes of a row's group go.
+  template <typename PLACE>
+  __device__ __forceinline__ void finish(const NormArgs& n, int M, int wave, int lane, float* red, PLACE place) {
+    constexpr int K = NW * KC;
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i) {
+      const int p = wave + i * NW, row = p / Q;
+      if (row < M) {
+        float part = 0.f;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          if (p % Q + 4 * j < GROUPS) {
+#pragma unroll
+            for (int e = 0; e < VK_VEC; ++e) part = part + a[i][j][e] * a[i][j][e];
+          }
+        }
+        part = wave_sum_xor(part);
+        if (lane == 0) red[row * 4 + p % Q] = part;
+      }
+    }
+    meet();
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i) {
+      const int p = wave + i * NW, row = p / Q;
+      if (row < M) {
+        float total = red[row * 4];
+#pragma unroll
+        for (int q = 1; q < Q; ++q) total = total + red[row * 4 + q];
+        const float rr = rsqrtf(total / (float)K + n.eps);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int g = p % Q + 4 * j;
+          if (g < GROUPS) {
+            float y[VK_VEC];
+#pragma unroll
+            for (int e = 0; e < VK_VEC; ++e) y[e] = (a[i][j][e] * rr) * to_f32(w[i][j][e]);
+            store_elems(reinterpret_cast<elem_t*>(place(row, g)), y);
+          }
+        }
+      }
+    }
+    meet();
+  }
+};
 
 // ------------------------------------------------------------------ skinny
 // MT: 16-row activation tiles (M <= 16*MT).  W: slabs in flight per wave.
@@ -206,11 +310,12 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(elem_t* __re
 // keeps the activations of its RC chunks (K <= RC * 4096) in registers for the
 // whole kernel.  One barrier per round of eight chunks.
 // ROWS: 1, 4, 8 or 16: the activations (one tile) come through LDS (ChunkRows): resident ones once, others a chunk ahead; 0: straight to registers.
-template <int MT, int W, int RC, int NT, int NW = SK_WAVES, int ROWS = 0>
+// NORM: the rows are normed first (NormRows), K is NW chunks.
+template <int MT, int W, int RC, int NT, int NW = SK_WAVES, int ROWS = 0, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict__ out,
                                                                     const elem_t* __restrict__ act,
                                                                     const elem_t* __restrict__ w, int M, int N, int K,
-                                                                    int64_t lda, int64_t ldo, int out_form) {
+                                                                    int64_t lda, int64_t ldo, int out_form, NormArgs norm) {
   // NT: 16-row weight tiles per workgroup.  With several activation tiles every workgroup reads all
   // activations once, M * K elements beside its 16 * NT * K weights: more weight rows per workgroup
   // keep that traffic, which comes from the second-level cache, in proportion.
@@ -235,7 +340,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
   constexpr bool EARLY = RC == 1 && MT == 1 && (NW <= 8 || sizeof(elem_t) == 2);
   constexpr bool AHEAD = ROWS > 0 && !RES;               // a chunk's rows are asked for while the one before is computed, into registers
   unsigned char* own_rows = rows_lds + wave * CHUNK_ROWS_BYTES(ROWS);
-  if constexpr (ROWS > 0) ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  static_assert(!NORM || (RES && ROWS > 0 && ROWS <= 8), "rows are normed on their way through LDS");
+  NormRows<NORM ? ROWS : 1, NORM ? NW : 2> normed;
+  if constexpr (NORM) {
+    normed.load(norm, act, lda, M, wave, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  } else if constexpr (ROWS > 0) {
+    ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  }
 
   const elem_t* arow[MT];
 #pragma unroll
@@ -269,7 +381,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, wave, i, i);
   }
-  if constexpr (ROWS > 0) {
+  if constexpr (NORM) {
+    __builtin_amdgcn_sched_barrier(0);
+    normed.finish(norm, M, wave, lane, reinterpret_cast<float*>(part), [&](int row, int g) {
+      constexpr int PER_CHUNK = KC * (int)sizeof(elem_t) / 1024;
+      return ChunkRows<ROWS>::place(rows_lds + g / PER_CHUNK * CHUNK_ROWS_BYTES(ROWS), row, g % PER_CHUNK * 64 + lane);
+    });
+#pragma unroll
+    for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
+  } else if constexpr (ROWS > 0) {
     if (wave < nchunks) {                                // a wave with a chunk has a tile: there are no more workgroups than tiles
       __builtin_amdgcn_sched_barrier(0);                 // the weights' loads stay in front of the wait that counts them
       wait_vmcnt_n<W * NT>();                            // the rows are there, the first weights on their way
@@ -389,12 +509,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 // two projections rounded to the element type first, which is what the separate
 // GEMM and SwiGLU kernels compute (kernels/triton_kernels/silu_mul.py:64-87).
 // M <= 16, K <= 4096 (activations resident in registers).
-template <int W, int MT, int RC, int NW = SK_WAVES, int ROWS = 0>
+template <int W, int MT, int RC, int NW = SK_WAVES, int ROWS = 0, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __restrict__ out,
                                                                            const elem_t* __restrict__ act,
                                                                            const elem_t* __restrict__ w, int M, int I,
                                                                            int K, int64_t lda, int64_t ldo,
-                                                                           int out_form) {
+                                                                           int out_form, NormArgs norm) {
   static_assert(KC_SLABS % W == 0, "the window must divide a chunk");
   static_assert(MT * RC <= 2, "two chunk tiles of activations stay in registers: two tiles of a chunk or two chunks of a tile");
   __shared__ f32x4 part[2][RC][NW][2 * MT][64];      // two sets, used in turn: one barrier per tile
@@ -409,7 +529,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   const int nchunks = K / KC;
   const int ntiles = (I + 15) / 16;
   unsigned char* own_rows = rows_lds + wave * CHUNK_ROWS_BYTES(ROWS);
-  if constexpr (ROWS > 0) ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  static_assert(!NORM || (ROWS > 0 && ROWS <= 8), "rows are normed on their way through LDS");
+  NormRows<NORM ? ROWS : 1, NORM ? NW : 2> normed;
+  if constexpr (NORM) {
+    normed.load(norm, act, lda, M, wave, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  } else if constexpr (ROWS > 0) {
+    ask_chunk_rows<ROWS>(act + (int64_t)min(wave, nchunks - 1) * KC, lda, M, lane, lds_offset_of(own_rows));
+  }
 
   // Wave w has chunks w, w + 8, ...: RC of them (chunks beyond K are read as the last and not used).
   frag_t wg[W], wu[W], abuf[RC * KC_SLABS][MT];
@@ -441,7 +568,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
 #pragma unroll
     for (int i = 0; i < W; ++i) issue(tile, i, i);
   }
-  if constexpr (ROWS > 0) {
+  if constexpr (NORM) {
+    __builtin_amdgcn_sched_barrier(0);
+    normed.finish(norm, M, wave, lane, reinterpret_cast<float*>(part), [&](int row, int g) {
+      constexpr int PER_CHUNK = KC * (int)sizeof(elem_t) / 1024;
+      return ChunkRows<ROWS>::place(rows_lds + g / PER_CHUNK * CHUNK_ROWS_BYTES(ROWS), row, g % PER_CHUNK * 64 + lane);
+    });
+#pragma unroll
+    for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
+  } else if constexpr (ROWS > 0) {
     if (active) {                                        // as in the kernel above
       __builtin_amdgcn_sched_barrier(0);
       wait_vmcnt_n<2 * W>();
@@ -533,15 +668,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
 struct LinePlan {
   int own_bytes, slots, first_slots;
 };
-template <int R, int ROWS, int P>
-__global__ __launch_bounds__(768) void gemm_lines_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w, int M, int N,
-                                                         int K, int64_t lda, int64_t ldo, int out_form, LinePlan plan) {
+// NORM: 0, or K's chunks: the rows are normed first (NormRows).
+template <int R, int ROWS, int P, int NORM = 0>
+__global__ __launch_bounds__(NORM ? 64 * NORM : 768) void gemm_lines_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w,
+                                                                            int M, int N, int K, int64_t lda, int64_t ldo, int out_form, LinePlan plan,
+                                                                            NormArgs norm) {
   using W = LineRows<R>;
   using A = LineRows<ROWS>;
   constexpr int W_BYTES = R * 1024, SLOT = P * W_BYTES, L = P * R, SUMS = R / 4 * 16;      // L: loads of a slot; SUMS: lanes with sums
   constexpr int S_MAX = 63 / L < LINE_SLOTS ? 63 / L : LINE_SLOTS;                         // no more loads than their counter counts
   extern __shared__ __attribute__((aligned(16))) unsigned char lines_lds[];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = NORM ? NORM : blockDim.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int S = plan.slots, step = gridDim.x, tiles = ((N + R - 1) / R - 1 - (int)blockIdx.x) / step + 1;      // of this workgroup, at least one
   unsigned char* own = lines_lds + wave * plan.own_bytes;
@@ -572,11 +709,23 @@ __global__ __launch_bounds__(768) void gemm_lines_kernel(elem_t* __restrict__ ou
     __builtin_amdgcn_sched_barrier(0);
   };
   const int before = min(plan.first_slots, tiles);
-  A::template ask<false>(act + wave * KC, lda, M, lane, lds_offset_of(own));
+  static_assert(ROWS <= 8 || !NORM, "up to eight rows are normed");
+  NormRows<NORM ? ROWS : 1, NORM ? NORM : 2> normed;
+  if constexpr (NORM != 0) {
+    normed.load(norm, act, lda, M, wave, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt_n<0>();                                     // (a workgroup's part of the sums as well)
+  } else {
+    A::template ask<false>(act + wave * KC, lda, M, lane, lds_offset_of(own));
+  }
 #pragma unroll
   for (int s = 0; s < S_MAX; ++s)
     if (s < before) ask(s, s);
-  wait_for_all_but(before);
+  if constexpr (NORM != 0) {
+    normed.finish(norm, M, wave, lane, reinterpret_cast<float*>(part), [&](int row, int g) { return lines_lds + g * plan.own_bytes + row * 1024 + ((lane ^ A::turn(row)) * 16); });
+  } else {
+    wait_for_all_but(before);
+  }
   frag_t rows[KC_SLABS];
 #pragma unroll
   for (int i = 0; i < KC_SLABS; ++i) rows[i] = A::fragment(own, i, r16, kg);
@@ -664,7 +813,7 @@ static int launch_lines_of(elem_t* out, const elem_t* act, const elem_t* w, int 
     per_cu[waves] = held > 0 ? held : 1;
   }
   const int tiles = (N + R - 1) / R, resident = per_cu[waves] * vk_device_cus();
-  gemm_lines_kernel<R, ROWS, P><<<tiles < resident ? tiles : resident, 64 * waves, lds_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form, plan);
+  gemm_lines_kernel<R, ROWS, P><<<tiles < resident ? tiles : resident, 64 * waves, lds_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form, plan, NormArgs{});
   return vk_check_launch("gemm_lines");
 }
 template <int R, int P>
@@ -1996,7 +2145,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
     }                                                                                                     \
     const unsigned groups = (unsigned)((N + 16 * NT - 1) / (16 * NT));                                    \
     gemm_stream_kernel<MT, W, RC, NT, NW, ROWS><<<groups < (unsigned)resident ? groups : (unsigned)resident, \
-                                             64 * NW, rows_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form); \
+                                             64 * NW, rows_bytes, st>>>(out, act, w, M, N, K, lda, ldo, form, NormArgs{}); \
   } while (0)
 #define STW(MT, W, RC, NT, NW) STH(MT, W, RC, NT, NW, 0)
 // Where as many rows do not fit beside the sums, stream_lds_rows names the kernel without them instead: nothing is compiled for a branch that is not taken.
@@ -2188,7 +2337,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                        \
     }                                                                                                      \
     gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
-        out, act, w, M, I, K, lda, ldo, form);                                                           \
+        out, act, w, M, I, K, lda, ldo, form, NormArgs{});                                                \
   } while (0)
 #define SWIGLU_STREAM(W, MT, RC) SWIGLU_STREAMH(W, MT, RC, SK_WAVES, 0)
 #define SWIGLU_STREAMN(NW)                                                                                 \
@@ -2222,6 +2371,107 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   return vk_check_launch("gemm_swiglu");
 }
 
+
+// ---- products that norm their rows themselves (NormRows)
+extern "C++" {
+template <typename KERNEL>
+static int workgroups_at_once(KERNEL kernel, int threads, int lds_bytes) {
+  int n = 0;
+  if (lds_bytes > 0) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds_bytes);
+  return (n > 0 ? n : 1) * vk_device_cus();
+}
+template <int ROWS, int P, int NW>
+static int launch_stream_normed(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int64_t ldx, int64_t ldo, int form, const NormArgs& norm, hipStream_t st) {
+  constexpr int LDS = NW * CHUNK_ROWS_BYTES(ROWS);
+  const int tiles = (N + 15) / 16;
+  if constexpr (P == 2) {
+    static const int at_once = workgroups_at_once(gemm_stream_swiglu_kernel<8, 1, 1, NW, ROWS, true>, 64 * NW, LDS);
+    gemm_stream_swiglu_kernel<8, 1, 1, NW, ROWS, true><<<std::min(tiles, at_once), 64 * NW, LDS, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, norm);
+  } else {
+    static const int at_once = workgroups_at_once(gemm_stream_kernel<1, 8, 1, 1, NW, ROWS, true>, 64 * NW, LDS);
+    gemm_stream_kernel<1, 8, 1, 1, NW, ROWS, true><<<std::min(tiles, at_once), 64 * NW, LDS, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, norm);
+  }
+  return vk_check_launch("gemm_stream (normed rows)");
+}
+#ifdef VK_BF16
+template <int R, int ROWS, int P, int NW>
+static int launch_lines_normed(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int64_t ldx, int64_t ldo, int form, const NormArgs& norm, hipStream_t st) {
+  LinePlan plan;
+  int lds = 0;
+  VK_REQUIRE(line_plan(M, NW * KC, R, P, &plan, &lds), "gemm: %d normed rows of K=%d do not fit", M, NW * KC);
+  static const int at_once = workgroups_at_once(gemm_lines_kernel<R, ROWS, P, NW>, 64 * NW, lds);      // (ROWS and NW fix the LDS)
+  gemm_lines_kernel<R, ROWS, P, NW><<<std::min((N + R - 1) / R, at_once), 64 * NW, lds, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, plan, norm);
+  return vk_check_launch("gemm_lines (normed rows)");
+}
+#endif
+// The launch for these sizes, or (out null) whether there is one: 1, 0.  The norm is done again by every workgroup, a row's kilobytes a wave, so that it pays
+// for few rows: the add and norm and the product by themselves against both in one, us, 1, 4 and 8 rows, 16-bit: 4,096 x 1,024 6.5, 6.7, 6.9 against 4.9, 5.7, 7.1; gate/up 3,072 x
+// 1,024 7.7, 7.9, 8.1, 6.4, 7.1, 8.5; 9,728 x 2,560 20.4, 20.7, 20.8, 18.0, 19.6, 21.6; 6,144 x 4,096 12.7, 13.4, 13.8, 10.4, 11.0, 12.5; gate/up 12,288 x 4,096 36.3,
+// 36.8, 37.2, 33.1, 35.0, 37.1; 32-bit, 1, 2 and 4 rows: 4,096 x 1,024 8.3, 8.3, 8.4, 6.8, 7.9, 9.3; 4,096 x 2,048 11.0, 11.1, 11.2, 9.5, 9.8, 10.7; 6,144 x 2,560 18.6, 18.7, 19.0,
+// 16.9, 17.9, 19.6; gate/up 12,288 x 4,096 81.4, 81.8, 82.1, 72.6, 72.3, 73.6, 8 rows 81.5, 77.1.
+template <int ROWS, int P>
+static int normed_product(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int K, int64_t ldx, int64_t ldo, const NormArgs& norm, hipStream_t st) {
+  const int chunks = K / KC, form = out == nullptr ? 0 : (ldo % 4 == 0 && (uintptr_t)out % 16 == 0);
+#define STREAMED(NW) return out == nullptr ? 1 : launch_stream_normed<ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
+#ifdef VK_BF16
+#define LINED(R, NW) return out == nullptr ? 1 : launch_lines_normed<R, ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
+  const int rows = lines_rows(M, N, K, P);
+  if (rows == 8 && chunks == 8) LINED(8, 8);
+  if constexpr (ROWS <= 4) {
+    if (rows == 8 && P == 2 && chunks == 2) LINED(8, 2);
+    if (rows == 8 && chunks == 4) LINED(8, 4);
+    if (rows == 8 && chunks == 5) LINED(8, 5);
+    if constexpr (P == 1) {
+      if (rows == 8 && chunks == 10) LINED(8, 10);
+    } else {
+      if (rows == 4 && chunks == 10) LINED(4, 10);
+    }
+    if (rows == 0 && chunks == 2) STREAMED(2);
+    if (rows == 0 && chunks == 4) STREAMED(4);
+  }
+#undef LINED
+#else
+  if (chunks == 8) STREAMED(8);
+  if constexpr (ROWS <= 4) {
+    if (chunks == 2 && M <= 2) STREAMED(2);
+    if (chunks == 4) STREAMED(4);
+    if (chunks == 5 && M <= 2) STREAMED(5);
+  }
+#endif
+#undef STREAMED
+  (void)form; (void)x; (void)w; (void)ldx; (void)norm; (void)st;
+  return 0;
+}
+template <int P>
+static int normed_product(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int K, int64_t ldx, int64_t ldo, const NormArgs& norm, hipStream_t st) {
+  if (M < 1 || M > 8 || N < 1 || K < KC || K % KC != 0) return 0;
+  if (M == 1) return normed_product<1, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
+  if (M <= 4) return normed_product<4, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
+  return normed_product<8, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
+}
+}  // extern "C++"
+
+// 1 if vk_gemm_normed takes these sizes (projections 1, or 2 with N gate rows) and is the faster way (normed_product).
+int vk_gemm_normed_takes(int M, int N, int K, int projections) {
+  return projections == 2 ? normed_product<2>(nullptr, nullptr, nullptr, M, N, K, K, N, NormArgs{}, nullptr)
+                          : normed_product<1>(nullptr, nullptr, nullptr, M, N, K, K, N, NormArgs{}, nullptr);
+}
+
+// out = norm(x + residual) w^T, or with two projections silu(gate) * up: vk_add_rmsnorm (sum, [M, K], takes the place of its new residual and is
+// another buffer than either input) and vk_gemm or vk_gemm_swiglu in one launch, the same bits.  x, residual and sum [M, K], norm_weight [K] elements.
+int vk_gemm_normed(elem_t* out, elem_t* sum, const elem_t* x, const elem_t* residual, const elem_t* norm_weight, float eps, const elem_t* w, int M, int N, int K,
+                   int64_t ldo, int projections, hipStream_t st) {
+  VK_REQUIRE(projections == 1 || projections == 2, "gemm_normed: one projection or two, not %d", projections);
+  VK_REQUIRE(M >= 0, "gemm_normed: bad sizes M=%d N=%d K=%d", M, N, K);
+  if (M == 0) return 0;
+  VK_REQUIRE(vk_gemm_normed_takes(M, N, K, projections), "gemm_normed: sizes M=%d N=%d K=%d are not supported", M, N, K);
+  VK_REQUIRE(out != nullptr && ldo >= N, "gemm_normed: output row stride %lld is smaller than N=%d", (long long)ldo, N);
+  VK_REQUIRE((((uintptr_t)x | (uintptr_t)residual | (uintptr_t)sum | (uintptr_t)norm_weight | (uintptr_t)w) % 16) == 0, "gemm_normed: operands must be 16-byte aligned");
+  VK_REQUIRE(sum != x && sum != residual && x != nullptr && residual != nullptr && sum != nullptr && norm_weight != nullptr, "gemm_normed: the sum needs a buffer of its own");
+  const NormArgs norm = {residual, sum, norm_weight, eps};
+  return projections == 2 ? normed_product<2>(out, x, w, M, N, K, K, ldo, norm, st) : normed_product<1>(out, x, w, M, N, K, K, ldo, norm, st);
+}
 
 // float32 elements of workspace that vk_gemm_split needs for these sizes, or 0 if it does not take them:
 // up to 64 rows of 16-bit elements, K in whole chunks; rows: weight rows (with swiglu: gate and up rows
