@@ -82,6 +82,22 @@ struct AttnArgs {
   int64_t gate_stride = 0;
 };
 
+// Decoded rows as the projections leave them: what vk_qkv_post does to them (head norm, rotation by tables, the store of key and value) happens in the
+// attention's own launch.
+struct RowArgs {
+  const elem_t* qkv;      // [T, row_stride]: nq q heads, nkv k heads, nkv v heads
+  int64_t row_stride;
+  elem_t* kc;             // the caches, written
+  elem_t* vc;
+  const elem_t* q_w;      // [d] or null
+  const elem_t* k_w;
+  const elem_t* cos_t;    // [positions, d / 2] or null
+  const elem_t* sin_t;
+  const int32_t* positions;
+  const int32_t* slots;
+  float eps;
+};
+
 // What a distance table has to hold beyond its distances 0 .. rel_far, on either side: a tile that is not wholly beyond rel_far
 // is read for all its keys and for all 16 rows of a wave.
 #define REL_PAD 96
@@ -1155,6 +1171,69 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 }
 #endif
 
+// A head's row as an operand of the matrix unit: lane (r16, g) holds the elements s * VK_SLAB + g * VK_VEC ... of its row, its norm and its rotation by
+// qkv_post_vec_kernel's operations in that kernel's order (there a lane holds 16 bytes and the sums go over neighbouring lanes; here the four lanes g
+// of a row come first and a lane's slabs after them: the same tree).
+template <int NQS>
+struct HeadRow {
+  frag_t x[NQS], w[NQS];
+  struct Angles {
+    frag_t cs[NQS / 2], sn[NQS / 2];
+    __device__ __forceinline__ void load(const elem_t* cosines, const elem_t* sines, int g) {
+#pragma unroll
+      for (int s = 0; s < NQS / 2; ++s) {
+        cs[s] = *reinterpret_cast<const frag_t*>(cosines + s * VK_SLAB + g * VK_VEC);
+        sn[s] = *reinterpret_cast<const frag_t*>(sines + s * VK_SLAB + g * VK_VEC);
+      }
+    }
+  };
+  __device__ __forceinline__ void load(const elem_t* row, const elem_t* weight, int g) {
+#pragma unroll
+    for (int s = 0; s < NQS; ++s) {
+      x[s] = *reinterpret_cast<const frag_t*>(row + s * VK_SLAB + g * VK_VEC);
+      if (weight != nullptr) w[s] = *reinterpret_cast<const frag_t*>(weight + s * VK_SLAB + g * VK_VEC);
+    }
+  }
+  __device__ __forceinline__ void finish(bool norm, bool turn, const Angles& angles, float eps, frag_t (&out)[NQS]) const {
+    float v[NQS][VK_VEC];
+#pragma unroll
+    for (int s = 0; s < NQS; ++s)
+#pragma unroll
+      for (int e = 0; e < VK_VEC; ++e) v[s][e] = to_f32(x[s][e]);
+    if (norm) {
+      float quad[NQS];
+#pragma unroll
+      for (int s = 0; s < NQS; ++s) {
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < VK_VEC; ++e) part = part + v[s][e] * v[s][e];
+        part = part + lane_xor16(part);
+        quad[s] = part + lane_xor32(part);
+      }
+#pragma unroll
+      for (int step = 1; step < NQS; step *= 2)
+#pragma unroll
+        for (int s = 0; s < NQS; s += 2 * step) quad[s] = quad[s] + quad[s + step];
+      const float rr = rsqrtf(quad[0] / (float)(NQS * VK_SLAB) + eps);
+#pragma unroll
+      for (int s = 0; s < NQS; ++s)
+#pragma unroll
+        for (int e = 0; e < VK_VEC; ++e) v[s][e] = round_to_elem((v[s][e] * rr) * to_f32(w[s][e]));
+    }
+#pragma unroll
+    for (int s = 0; s < NQS; ++s)
+#pragma unroll
+      for (int e = 0; e < VK_VEC; ++e) {
+        float y = v[s][e];
+        if (turn) {
+          const float other = v[s ^ (NQS / 2)][e], c = to_f32(angles.cs[s % (NQS / 2)][e]), n = to_f32(angles.sn[s % (NQS / 2)][e]);
+          y = s < NQS / 2 ? y * c - other * n : y * c + other * n;
+        }
+        out[s][e] = from_f32<elem_t>(y);
+      }
+  }
+};
+
 // Decoded tokens, four waves a segment, for the plain attention and (EXT) the variant.  Wave j computes the scores of the
 // segment's tile j; the tiles' maxima pass through LDS, so that every wave knows how the rows' reference maximum moves from tile to
 // tile; wave j turns its scores into weights, which pass through LDS too; then every wave adds up a quarter of the output columns over
@@ -1164,10 +1243,14 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 // (a page that turns out not to be needed is read and not used), and the four tiles' scores are computed side by side.
 // SEGS 2: a workgroup of eight waves takes both segments of a launch that has no more than two, folds them as attn_combine_kernel
 // does and writes the output: a launch less, where a launch that waits for the one before is a third of the two.
+// ROWS (the plain attention, EXACT): the step's rows come as the projections leave them (RowArgs).  Every wave with a tile norms and turns its heads' rows; the
+// segment that holds a row's own key puts that key and value among its tile's, and the first of a kv head's workgroups stores them.  A launch of its
+// own for that, between the projection and the attention, took 3.8 us of one row of 32 heads and 5.1 of eight of 48.
 // FAR: the launch covers the kept segments and those that a window or a block can touch, not all before it.  (Known when the kernel is built:
 // the page numbers then wait for the lengths, 0.4 us of a short request's 12.)
-template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1, bool FAR = false>
-__global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a) {
+template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1, bool FAR = false, bool ROWS = false>
+__global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256 ? 2 : 1) void attn_decode_quad_kernel(AttnArgs a, RowArgs rows) {
+  static_assert(!ROWS || (EXACT && !EXT), "rows as the projections leave them: plain attention, whole heads, a tile in one page");
   static_assert(SEGS == 1 || sizeof(elem_t) * DPAD <= 256, "eight waves have 256 registers each");
   static_assert(EXT || !REL, "biases by distance belong to the variant");
   static_assert(!FAR || (EXT && SEGS == 1), "so do launches over some of a request's segments");
@@ -1221,12 +1304,45 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   const bool mine = (wanted >> wave) & 1u;
   frag_t qf[NQS];
   frag_t kf[KSUB][NQS];
+  const int own_tile = pos / TILE_KEYS - first_tile;          // the segment's tile with the row's own key, where that is 0 .. SEG_TILES - 1
+  int slot = -1;
+  HeadRow<NQS> q_row, k_row;
+  typename HeadRow<NQS>::Angles angles;
+  elem_t own_value[ND];
+  if constexpr (ROWS) {
+    // These loads first: loads arrive in the order in which they are asked for.
+    slot = rows.slots[tok];
+    const elem_t* row = rows.qkv + (int64_t)tok * rows.row_stride;
+    if (mine) {
+      q_row.load(row + (int64_t)(c.row_ok ? head : kvh * G) * DPAD, rows.q_w, c.g);
+      if (wave == own_tile) k_row.load(row + (int64_t)(a.nq + kvh) * DPAD, rows.k_w, c.g);
+      if (rows.cos_t != nullptr) {
+        const int64_t at = (int64_t)rows.positions[tok] * (DPAD / 2);
+        angles.load(rows.cos_t + at, rows.sin_t + at, c.g);
+      }
+    }
+    if (own_tile >= 0 && own_tile < SEG_TILES) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) own_value[dt] = row[(int64_t)(a.nq + a.nkv + kvh) * DPAD + (wave * ND + dt) * 16 + c.r16];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if (mine) {
-    load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
+    if constexpr (!ROWS) load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
     int my_page = page[0];
 #pragma unroll
     for (int j = 1; j < SEG_TILES; ++j) my_page = wave == j ? page[j] : my_page;
     load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf, my_page);
+  }
+  frag_t own_key[ROWS ? NQS : 1];
+  if constexpr (ROWS) {
+    // Between the keys' loads and the values': the registers of both, of two rows and of their arithmetic are too many at once.
+    __builtin_amdgcn_sched_barrier(0);
+    if (mine) {
+      q_row.finish(rows.q_w != nullptr, rows.cos_t != nullptr, angles, rows.eps, qf);
+      if (wave == own_tile) k_row.finish(rows.k_w != nullptr, rows.cos_t != nullptr, angles, rows.eps, own_key);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   // This wave's columns of every tile's values: a context whose head starts at them.
   RowCtx cv = c;
@@ -1237,6 +1353,49 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   for (int j = 0; j < SEG_TILES; ++j)
     if ((wanted >> j) & 1u) load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
   __builtin_amdgcn_sched_barrier(0);
+
+  if constexpr (ROWS) {
+    const int own_page = slot >> lp, own_off = slot & (a.P - 1);
+    const bool stores = ht == 0 && slot >= 0;
+    if (mine && wave == own_tile && slot >= 0) {
+      if (stores && c.r16 == 0) {
+        elem_t* o = rows.kc + (((int64_t)own_page * a.nkv + kvh) * a.P + own_off) * DPAD + c.g * VK_VEC;
+#pragma unroll
+        for (int s = 0; s < NQS; ++s) *reinterpret_cast<frag_t*>(o + s * VK_SLAB) = own_key[s];
+      }
+      const int at = pos % TILE_KEYS;
+#pragma unroll
+      for (int sub = 0; sub < KSUB; ++sub) {
+#ifdef VK_BF16
+        const bool here = at == (sub >> 1) * VK_SLAB + 8 * (c.r16 >> 2) + 4 * (sub & 1) + (c.r16 & 3);
+#else
+        const bool here = at == sub * VK_SLAB + c.r16;
+#endif
+#pragma unroll
+        for (int s = 0; s < NQS; ++s) kf[sub][s] = here ? own_key[s] : kf[sub][s];
+      }
+    }
+    if (own_tile >= 0 && own_tile < SEG_TILES && slot >= 0) {
+      if (stores && c.g == 0) {
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+          rows.vc[(((int64_t)own_page * a.nkv + kvh) * DPAD + (wave * ND + dt) * 16 + c.r16) * a.P + own_off] = own_value[dt];
+      }
+      const int at = pos % TILE_KEYS;
+#pragma unroll
+      for (int j = 0; j < SEG_TILES; ++j) {
+        if (j == own_tile) {
+#pragma unroll
+          for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+            for (int ks = 0; ks < KEY_SLABS; ++ks)
+#pragma unroll
+              for (int e = 0; e < VK_VEC; ++e)
+                if (at == ks * VK_SLAB + c.g * VK_VEC + e) vf[j][dt][ks][e] = own_value[dt];
+        }
+      }
+    }
+  }
 
   // ---- the scores of this wave's tile and their maximum a row ----
   const float unit = EXT ? LOG2E : a.scale_log2;             // what takes a score to powers of two
@@ -1459,6 +1618,13 @@ static bool decode_folds_itself(int nseg, int d, int64_t workgroups) {
   return nseg <= 2 && row <= 256 && workgroups <= (row <= 128 ? 2 : 1) * (int64_t)vk_device_cus();
 }
 
+// How many segments go with four waves each (the reasons stand at the launch).
+static int64_t quad_segments(int d) {
+  const bool seg_fits = sizeof(elem_t) * vk_dpad(d) <= 256, padded = !seg_fits && d < vk_dpad(d);
+  const int half_rounds = padded ? (sizeof(elem_t) == 2 || d <= 80 ? 4 : 6) : (sizeof(elem_t) == 2 || seg_fits ? 5 : 12);
+  return half_rounds * (int64_t)vk_device_cus() / 2;
+}
+
 // items: n_items pairs (sequence, first row).
 // mode 0: each item is up to vk_attn_item_rows() consecutive rows of the sequence's q_len new tokens;
 //   the kernel is chosen by shape.  mode 2: the same through the kernel that takes every shape,
@@ -1569,20 +1735,18 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   // 38.9, 44.4, of 256 48.5, 41.4; 512 of 160 33.7, 30.2; 32-bit, 1,024 of 80 52.6, 65.7, of 96 59.8, 71.4; 768 of 80 46.6, 49.3, of 96 49.2, 51.2 at
   // the most and 1.1 times the other way on the mean; 512 of 80 1.2 times the other way).
   const bool quad_fits = sizeof(elem_t) * vk_dpad(d) <= 512;
-  const bool padded = !seg_fits && d < vk_dpad(d);
-  const int half_rounds = padded ? (sizeof(elem_t) == 2 || d <= 80 ? 4 : 6) : (sizeof(elem_t) == 2 || seg_fits ? 5 : 12);
-  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = half_rounds * (int64_t)vk_device_cus() / 2;
+  const int64_t segments = (int64_t)grid.x * grid.y * grid.z, quad_most = quad_segments(d);
   if (quad_fits && (vk_decode_variant == 4 || (vk_decode_variant == 0 && segments <= quad_most))) {
     const bool exact = P >= TILE_KEYS && d == vk_dpad(d);
 #define DECODE_QUAD(DP)                                                                               \
   do {                                                                                                \
-    if (exact) attn_decode_quad_kernel<DP, true, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);   \
-    else attn_decode_quad_kernel<DP, false, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a);        \
+    if (exact) attn_decode_quad_kernel<DP, true, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a, RowArgs{});   \
+    else attn_decode_quad_kernel<DP, false, false, false><<<grid, 64 * SEG_TILES, 0, st>>>(a, RowArgs{});        \
   } while (0)
 #define DECODE_BOTH(DP)                                                                                                        \
   do {                                                                                                                         \
-    if (exact) attn_decode_quad_kernel<DP, true, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);        \
-    else attn_decode_quad_kernel<DP, false, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a);             \
+    if (exact) attn_decode_quad_kernel<DP, true, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a, RowArgs{});        \
+    else attn_decode_quad_kernel<DP, false, false, false, 2><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a, RowArgs{});             \
   } while (0)
     if (decode_folds_itself(nseg, d, grid.x * (int64_t)grid.y)) {
 #ifdef VK_BF16
@@ -1633,6 +1797,50 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   else DECODE_PLAIN(256);
 #undef DECODE_PLAIN
   if (vk_check_launch("attention (decoded rows)")) return 1;
+  attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
+  return vk_check_launch("attention (combine)");
+}
+
+// 1 if vk_paged_attention_rows takes so many decoded rows: heads of 64 or 128, pages of a tile or more, and segments few enough for four waves each.
+int vk_paged_attention_rows_takes(int n_items, int nseg, int nq, int nkv, int d, int P) {
+  if (n_items <= 0 || nseg <= 0 || nkv <= 0 || nq <= 0 || nq % nkv != 0 || (d != 64 && d != 128) || P < TILE_KEYS || (P & (P - 1)) != 0) return 0;
+  return (int64_t)n_items * (nkv * ((nq / nkv + 15) / 16)) * nseg <= quad_segments(d);
+}
+
+// vk_qkv_post (heads of d with a rotation of the whole head or none, weights of elements or none, every row stored where its slot says) and
+// vk_paged_attention (mode 1, every row of the step one item) in one launch for the two, the same bits.  qkv [T, row_stride].
+int vk_paged_attention_rows(elem_t* out, const elem_t* qkv, int64_t row_stride, elem_t* kc, elem_t* vc, const elem_t* q_w, const elem_t* k_w, float eps,
+                            const elem_t* cos_t, const elem_t* sin_t, const int32_t* positions, const int32_t* slots, const int32_t* block_table, int bt_stride,
+                            const int32_t* cu_q, const int32_t* k_len, const int32_t* items, int n_items, int nseg, float* scratch, int nq, int nkv, int d, int P,
+                            int window, float scale, hipStream_t st) {
+  if (n_items <= 0) return 0;
+  VK_REQUIRE(vk_paged_attention_rows_takes(n_items, nseg, nq, nkv, d, P), "attention: %d rows of %d segments with %d / %d heads of %d and pages of %d are not taken as they are",
+             n_items, nseg, nq, nkv, d, P);
+  VK_REQUIRE(window >= 0 && scale > 0.f && nseg <= 65535 && scratch != nullptr, "attention: bad window, scale or segments");
+  VK_REQUIRE(row_stride >= (int64_t)(nq + 2 * nkv) * d && row_stride % VK_VEC == 0, "attention: row stride %lld too small or uneven", (long long)row_stride);
+  VK_REQUIRE((((uintptr_t)qkv | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)q_w | (uintptr_t)k_w | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16) == 0,
+             "attention: operands must be 16-byte aligned");
+  VK_REQUIRE((cos_t == nullptr) == (sin_t == nullptr) && (cos_t == nullptr || positions != nullptr) && slots != nullptr, "attention: a rotation needs tables and positions, a store slots");
+  AttnArgs a;
+  a.q = nullptr; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
+  a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
+  a.nseg = nseg; a.scale_log2 = scale * 1.4426950408889634f;
+  a.part_ml = scratch;
+  a.part_acc = scratch + (((int64_t)n_items * nq * nseg * 2 + 3) & ~(int64_t)3);
+  const RowArgs rows = {qkv, row_stride, kc, vc, q_w, k_w, cos_t, sin_t, positions, slots, eps};
+  const dim3 grid(n_items, nkv * ((nq / nkv + 15) / 16), nseg);
+  VK_REQUIRE(grid.y <= 65535 && nq <= 65535, "attention: too many heads");
+  if (decode_folds_itself(nseg, d, grid.x * (int64_t)grid.y)) {
+#ifdef VK_BF16
+    if (d == 128) attn_decode_quad_kernel<128, true, false, false, 2, false, true><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a, rows);
+    else
+#endif
+      attn_decode_quad_kernel<64, true, false, false, 2, false, true><<<dim3(grid.x, grid.y), 128 * SEG_TILES, 0, st>>>(a, rows);
+    return vk_check_launch("attention (projected rows, both segments)");
+  }
+  if (d == 128) attn_decode_quad_kernel<128, true, false, false, 1, false, true><<<grid, 64 * SEG_TILES, 0, st>>>(a, rows);
+  else attn_decode_quad_kernel<64, true, false, false, 1, false, true><<<grid, 64 * SEG_TILES, 0, st>>>(a, rows);
+  if (vk_check_launch("attention (projected rows, four waves a segment)")) return 1;
   attn_combine_kernel<<<dim3(n_items, nq), 64, 0, st>>>(a);
   return vk_check_launch("attention (combine)");
 }
@@ -1732,14 +1940,14 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     const dim3 qgrid(n_items, nkv * ((G + 15) / 16), (unsigned)std::min<int64_t>(seen, nseg));
 #define DECODE_QUAD_EXT_FAR(DP, REL, FAR)                                                                       \
   do {                                                                                                          \
-    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);       \
-    else attn_decode_quad_kernel<DP, false, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a);            \
+    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a, RowArgs{});       \
+    else attn_decode_quad_kernel<DP, false, true, REL, 1, FAR><<<qgrid, 64 * SEG_TILES, 0, st>>>(a, RowArgs{});            \
   } while (0)
 #define DECODE_QUAD_EXT_OF(DP, REL) do { if (seen < nseg) DECODE_QUAD_EXT_FAR(DP, REL, true); else DECODE_QUAD_EXT_FAR(DP, REL, false); } while (0)
 #define DECODE_BOTH_EXT_OF(DP, REL)                                                                                             \
   do {                                                                                                                         \
-    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);         \
-    else attn_decode_quad_kernel<DP, false, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a);              \
+    if (exact) attn_decode_quad_kernel<DP, true, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a, RowArgs{});         \
+    else attn_decode_quad_kernel<DP, false, true, REL, 2><<<dim3(qgrid.x, qgrid.y), 128 * SEG_TILES, 0, st>>>(a, RowArgs{});              \
   } while (0)
 #define DECODE_BOTH_EXT(DP) do { if (rel != nullptr) DECODE_BOTH_EXT_OF(DP, true); else DECODE_BOTH_EXT_OF(DP, false); } while (0)
     if (decode_folds_itself(nseg, d, qgrid.x * (int64_t)qgrid.y)) {

@@ -96,6 +96,8 @@ struct Kernels::Fn {
   int (*gemm_split_preferred)(int, int, int, int);
   int (*qkv_post)(CP, int64_t, P, P, P, CP, CP, int, CP, CP, int, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*paged_attention)(P, CP, CP, CP, CP, int, CP, CP, CP, int, int, int, P, int, int, int, int, int, int, float, hipStream_t);
+  int (*paged_attention_rows_takes)(int, int, int, int, int, int);
+  int (*paged_attention_rows)(P, CP, int64_t, P, P, CP, CP, float, CP, CP, CP, CP, CP, int, CP, CP, CP, int, int, P, int, int, int, int, int, float, hipStream_t);
   int (*sample)(P, CP, CP, CP, P, int, int, int64_t, hipStream_t);
   int (*sample_scratch_words)(int);
   int64_t (*attn_scratch_floats)(int, int, int, int);
@@ -197,7 +199,8 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(gemm, "vk_gemm"); VK(gemm_swiglu, "vk_gemm_swiglu"); VK(gemm_swiglu_supported, "vk_gemm_swiglu_supported");
   VK(gemm_normed_takes, "vk_gemm_normed_takes"); VK(gemm_normed, "vk_gemm_normed");
   VK(gemm_split, "vk_gemm_split"); VK(gemm_split_floats, "vk_gemm_split_floats"); VK(gemm_split_preferred, "vk_gemm_split_preferred");
-  VK(qkv_post, "vk_qkv_post"); VK(paged_attention, "vk_paged_attention"); VK(sample, "vk_sample");
+  VK(qkv_post, "vk_qkv_post"); VK(paged_attention, "vk_paged_attention");
+  VK(paged_attention_rows_takes, "vk_paged_attention_rows_takes"); VK(paged_attention_rows, "vk_paged_attention_rows"); VK(sample, "vk_sample");
   VK(sample_scratch_words, "vk_sample_scratch_words"); VK(attn_scratch_floats, "vk_attn_scratch_floats");
   VK(attn_segment_keys, "vk_attn_segment_keys"); VK(attn_item_rows, "vk_attn_item_rows");
   VK(embed_sinusoid, "vk_embed_sinusoid"); VK(stream_norm, "vk_stream_norm"); VK(stream_norm_add, "vk_stream_norm_add");
@@ -483,6 +486,42 @@ Tensor Kernels::qkv_post(const Tensor& qkv, int nq, int nkv, int d, const Tensor
 
 int64_t Kernels::attn_scratch_floats(int items, int nq, int d, int nseg) const {
   return fn_->attn_scratch_floats(items, nq, d, nseg);
+}
+
+bool Kernels::attention_takes_rows(int64_t items, int nseg, int nq, int nkv, int d, int page_size, const Tensor* q_w, const Tensor* k_w, const Tensor* cos) const {
+  if ((q_w && q_w->dtype != dtype_) || (k_w && k_w->dtype != dtype_) || (cos && 2 * cos->dim(1) != d) || items > INT32_MAX) return false;
+  return fn_->paged_attention_rows_takes((int)items, nseg, nq, nkv, d, page_size) != 0;
+}
+
+void Kernels::paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int nkv, int d, const Tensor& k_cache, const Tensor& v_cache, int page_size, const Tensor* q_w,
+                                   const Tensor* k_w, float eps, const Tensor* cos, const Tensor* sin, const Tensor& positions, const Tensor& slots,
+                                   const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items, float scale, int window, int max_k_len, int nseg,
+                                   const Tensor& scratch) {
+  const int64_t T = qkv.dim(0), W = (int64_t)(nq + 2 * nkv) * d, pages = k_cache.dim(0), S = k_len.dim(0);
+  expect(qkv, "qkv", dtype_, {T, W});
+  expect(k_cache, "k cache", dtype_, {pages, nkv, page_size, d});
+  expect(v_cache, "v cache", dtype_, {pages, nkv, d, page_size});
+  if (q_w) expect(*q_w, "q norm weight", dtype_, {d});
+  if (k_w) expect(*k_w, "k norm weight", dtype_, {d});
+  if (cos) {
+    if (!sin) throw EngineError("attention: a rotation needs cosines and sines");
+    expect(*cos, "cosine table", dtype_, {cos->dim(0), d / 2});
+    expect(*sin, "sine table", dtype_, cos->shape);
+  }
+  expect(positions, "positions", DType::I32, {T});
+  expect(slots, "slots", DType::I32, {T});
+  expect(block_table, "block table", DType::I32, {S, block_table.dim(1)});
+  expect(cu_q, "cu_q", DType::I32, {S + 1});
+  expect(k_len, "k_len", DType::I32, {S});
+  expect(items, "items", DType::I32, {T, 2});          // every row is an item
+  expect(out, "attention output", dtype_, {T, nq, d});
+  if (block_table.dim(1) * page_size < max_k_len || nseg < (max_k_len + segment_keys_ - 1) / segment_keys_)
+    throw EngineError("attention: a block table of " + block_table.describe() + " and " + std::to_string(nseg) + " segments do not cover " + std::to_string(max_k_len) + " keys");
+  const int64_t need = attn_scratch_floats((int)T, nq, d, nseg);
+  if (scratch.dtype != DType::F32 || scratch.numel() < need) throw EngineError("attention: scratch of " + std::to_string(need) + " floats needed");
+  call(fn_->paged_attention_rows(out.data, qkv.data, W, k_cache.data, v_cache.data, q_w ? q_w->data : nullptr, k_w ? k_w->data : nullptr, eps, cos ? cos->data : nullptr,
+                                 cos ? sin->data : nullptr, positions.data, slots.data, block_table.data, (int)block_table.dim(1), cu_q.data, k_len.data, items.data, (int)T,
+                                 nseg, scratch.data, nq, nkv, d, page_size, window, scale, stream));
 }
 
 void Kernels::paged_attention(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,

@@ -727,6 +727,23 @@ class Attention : public Mixer {
     if (padded_norm && !norm_angles && !prepared()) throw ConfigError("attention: head norms on padded head sizes are built for rotations by computed angles only");
     // The kernels between the projections take rows of exactly the heads' width, except the one that says otherwise.
     const Tensor qkv = (qkv_all.dim(1) == heads_w || norm_angles || prepared()) ? qkv_all : k.columns(qkv_all, 0, heads_w);
+    AttentionItems& m = items(*ctx.host);
+    const Tensor& prefill_items = ctx.inputs.at("attention.prefill_items");
+    const Tensor& decode_items = ctx.inputs.at("attention.decode_items");
+    // A step of decoded rows alone: plain attention takes the projections' rows as they are, where it has such a launch.
+    const bool plain = !prepared() && !bias_ && !biased() && !capped() && !gate_ && d_ == dk_ && fused() && !(position_ && position_->angle_frequencies());
+    if (plain && cache.writable && !prefill_items.dim(0) && decode_items.dim(0) == T) {
+      const Tensor *q_w = q_norm_ ? q_norm_->row_scale_weight() : nullptr, *k_w = k_norm_ ? k_norm_->row_scale_weight() : nullptr;
+      const Tensor *cos = position_ ? position_->cos_table() : nullptr, *sin = position_ ? position_->sin_table() : nullptr;
+      if (k.attention_takes_rows(T, m.nseg, nq_, nkv_, d_, cache.page_size, q_w, k_w, cos)) {
+        const Norm* en = q_norm_ ? q_norm_.get() : k_norm_.get();
+        const Tensor scratch = ctx.workspace(k.attn_scratch_floats((int)T, nq_, d_, m.nseg));
+        Tensor heads = k.empty({T, (int64_t)nq_, (int64_t)d_});
+        k.paged_attention_rows(heads, qkv_all, nq_, nkv_, d_, cache.k, cache.v, cache.page_size, q_w, k_w, en ? en->eps() : 0.f, cos, sin, ctx.positions, tables.slots,
+                               tables.block_table, ctx.cu_q, ctx.k_len, decode_items, scale_, window_, m.decode_bound, m.nseg, scratch);
+        return k.gemm(heads.view({T, (int64_t)nq_ * d_}), w_o_, ws);
+      }
+    }
     Tensor q;
     if (prepared()) {
       q = prepare(qkv, ctx, cache, tables);
@@ -754,9 +771,6 @@ class Attention : public Mixer {
       q = unfused(qkv, ctx, cache, tables);
     }
     Tensor out = k.empty(q.shape);
-    AttentionItems& m = items(*ctx.host);
-    const Tensor& prefill_items = ctx.inputs.at("attention.prefill_items");
-    const Tensor& decode_items = ctx.inputs.at("attention.decode_items");
     const Tensor* sinks = sink_ ? &sinks_ : nullptr;
     const Tensor *rel = bias_by_distance_ ? &rel_ : nullptr, *head_gate = head_gate_ ? &qkv_all : nullptr;
     if (prefill_items.dim(0)) {
