@@ -1,0 +1,32 @@
+"""Tile products whose workgroups are at most as many as the compute units: the bits of the two-stage square tiles on both sides of each line."""
+import pytest
+import torch
+from test_kernels_gpu import DTYPES, kern, rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K", [64, 128, 192, 512, 576, 1024, 1536, 2112])
+@pytest.mark.parametrize("M", [65, 128, 129, 257, 641])
+def test_widths_of_one_round(M, K, dtype):
+    """The widest product that fits with 64, 96 and 128 weight rows a workgroup, one more weight row than that, and one that ends inside the first
+    workgroup; fewer tiles of K than stages, and K in whole chunks and not.  Rows further apart than they are long."""
+    k = kern(dtype)
+    cus, blocks = torch.cuda.get_device_properties(0).multi_processor_count, -(-M // 128)
+    x = rand((M, K + 32), dtype, 1).cuda()[:, :K]
+    for N in [7, 200] + [width * (cus // blocks) + more for width in (64, 96, 128) for more in (0, 1)]:
+        w = rand((N, K), dtype, 2, 0.1).cuda()
+        assert torch.equal(k.gemm(x, w), k.gemm(x, w, kernel=4)), N
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("K", [64, 128, 576, 1024])
+@pytest.mark.parametrize("M", [65, 128, 300, 641])
+def test_gate_and_up(M, K, dtype):
+    k = kern(dtype)
+    cus, blocks = torch.cuda.get_device_properties(0).multi_processor_count, -(-M // 128)
+    x = rand((M, K), dtype, 3).cuda()
+    for I in (7, 200, 64 * (cus // blocks), 64 * (cus // blocks) + 1):
+        w = rand((2 * I, K), dtype, 4, 0.1).cuda()
+        assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4))), I

@@ -977,24 +977,16 @@ static int launch_tiled(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // gives twice the workgroups, for grids that would leave compute units with one workgroup or none; 3 and 5 are
 // for grids whose last round of workgroups would otherwise run nearly empty (pipe_fragments_by_rounds).  Six
 // would need more than the 256 registers of a wave.
-// One 4-byte load per lane whose value nobody reads: it brings the lane's 128-byte line into the second-level
-// cache ahead of the LDS-direct load that will want it.  `keep` is one register that every such load writes
-// (in order, so they may overlap) and that stays allocated to the end of the kernel.
-__device__ __forceinline__ void pipe_touch_line(const unsigned char* sbase, unsigned voff, unsigned& keep) {
-  asm volatile("global_load_dword %0, %1, %2 sc1" : "+v"(keep) : "v"(voff), "s"(sbase) : "memory");
-}
-// PFD > 0: every wave touches, PFD tiles ahead, the 64 rows of the workgroup's tiles that are its share.
 // NWN: waves along the weight rows, two of a workgroup of four waves or four of eight, which takes 64 FNW weight rows.
 // GROUPED: block_weights, row_pair and act_row count.
-template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int PFD = 0, int NWN = 2, bool GROUPED = false>
+template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int NWN = 2, bool GROUPED = false>
 __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act,
                                                         const elem_t* __restrict__ w, int M, int N, int K,
                                                         int64_t lda, int64_t ldo, int out_form, int band_w,
                                                         const int32_t* __restrict__ block_weights, int64_t weights_stride,
                                                         const int32_t* __restrict__ row_pair, const int32_t* __restrict__ act_row) {
   static_assert(FNW >= 2 && FNW <= 5 && (FNW == 4 || !SWIGLU), "two to five weight fragments per wave; four with SwiGLU");
-  static_assert(PFD == 0 || FNW == 2 || FNW == 4, "the touch-ahead wants a wave's 64 rows to be of one kind");
-  static_assert(NWN == 2 || (NWN == 4 && !SWIGLU && PFD == 0), "two waves or four along the weight rows");
+  static_assert(NWN == 2 || (NWN == 4 && !SWIGLU), "two waves or four along the weight rows");
   constexpr int BN = 16 * FNW * NWN;                    // weight rows of the workgroup
   constexpr int NA = 8 / NWN, PER_TILE = FNW + NA;      // loads of activation rows, and all loads, per K tile and wave
   constexpr int W_BYTES = BN * T_ROWB, STAGE_BYTES = W_BYTES + 128 * T_ROWB;
@@ -1070,24 +1062,6 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
     for (int j = 0; j < NA; ++j) pipe_load_to_lds16_sv(abase + kb, offa[j], base + W_BYTES + (wave * NA + j) * 8 * T_ROWB);
   };
 
-  // The lines a wave touches ahead: row wave * 64 + lane of the workgroup's weight rows followed by its
-  // activation rows (a wave's 64 rows are all weights, all up rows, or all activations).
-  static_assert(PFD == 0 || S == 2, "the touch-ahead counts its loads for two stages");
-  unsigned pf_off = 0, pf_keep = 0;
-  const unsigned char* pf_base = wbase;
-  if (PFD > 0) {
-    const int r = wave * 64 + lane;
-    if (wave * 64 < BN) {
-      const bool up = SWIGLU && wave * 64 >= 64;
-      const int local = up ? r - 64 : r;
-      pf_base = up ? ubase : wbase;
-      pf_off = (unsigned)((int64_t)(min(n_blk + local, N - 1) - min(n_blk, N - 1)) * K * (int64_t)sizeof(elem_t));
-    } else {
-      pf_base = abase;
-      pf_off = act_off(min(r - BN, 127), 0);
-    }
-  }
-
   f32x4 acc[FNW][4], total[FNW][4];
 #pragma unroll
   for (int i = 0; i < FNW; ++i)
@@ -1113,18 +1087,12 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
 
   auto step = [&](int kt) {
     // Tile kt has landed once at most the loads of the tiles after it are outstanding (PER_TILE per tile and wave).
-    if (PFD > 0) {
-      if (kt == 0) wait_vmcnt_n<0>(); else wait_vmcnt_n<1>();      // the one touch that was issued behind tile kt's loads may still fly
-    } else {
-      const int later = min(S - 2, ntiles - 1 - kt);
-      if (later == 0) wait_vmcnt_n<0>();
-      else if (later == 1) wait_vmcnt_n<PER_TILE>();
-      else wait_vmcnt_n<2 * PER_TILE>();
-    }
+    const int later = min(S - 2, ntiles - 1 - kt);
+    if (later == 0) wait_vmcnt_n<0>();
+    else if (later == 1) wait_vmcnt_n<PER_TILE>();
+    else wait_vmcnt_n<2 * PER_TILE>();
     __syncthreads();       // every wave's part of tile kt is there; everyone is done with tile kt-1's buffer
     if (kt + S - 1 < ntiles) issue(kt + S - 1);
-    if (PFD > 0)           // always one, so that the count above holds: beyond the end the last tile again
-      pipe_touch_line(pf_base + (int64_t)min(kt + PFD, ntiles - 1) * 2 * VK_SLAB * (int64_t)sizeof(elem_t), pf_off, pf_keep);
     const unsigned char* base = lds + (kt % S) * STAGE_BYTES;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -1179,10 +1147,6 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
     }
   }
 
-  if (PFD > 0) {
-    wait_vmcnt_n<0>();                                        // the last touches
-    asm volatile("" : : "v"(pf_keep));                        // the register was theirs until here
-  }
   if constexpr (SWIGLU) {
     // The two waves of a row block split the 64 output columns: the gate wave keeps columns 0..31 and
     // gets their up values, the up wave keeps columns 32..63 and gets their gate values.
@@ -1233,8 +1197,9 @@ __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(
 static const int pipe_band_blocks = 64;
 
 // Whether a grouped product of 16-bit elements and K in whole chunks goes by workgroups of 256 weight rows (launch_pipe) or of 128.
-// The wide ones have one workgroup a compute unit, so that a launch of few is one round half empty where the narrow ones have two a unit or
-// the touch-ahead; and a column block that lands on another chip part with each row block (columns that are no multiple of eight, up to 16)
+// The wide ones have one workgroup a compute unit, so that a launch of few is one round half empty where the narrow ones have two a unit,
+// or one with four stages (at most one a unit: 896 sizes of 4 to 64 matrices of 20 to 200 rows, most of them wide before, 26.5 -> 23.0 ms, 22.7 with the better of
+// the two everywhere); and a column block that lands on another chip part with each row block (columns that are no multiple of eight, up to 16)
 // has its weights read by several.  But up to about 60 rows a matrix (M and the matrices tell: a matrix has up to 127 rows of padding)
 // half of most blocks is idle, which only the wide ones leave out.  Measured on MI355X in recorded launches with the weights of
 // several layers in turn, 947 sizes of 2 to 64 matrices, 40 to 4,096 tokens, rows named, narrow against wide, us: 32 matrices, 4 choices, 257
@@ -1244,6 +1209,7 @@ static const int pipe_band_blocks = 64;
 // lie 94; the wide ones alone 415 and 353, the narrow ones 336 and 419.
 static bool grouped_wide(int M, int N, int matrices, bool named) {
   const int64_t columns = (N + 255) / 256, groups = columns * (M / 128);
+  if ((N + 127) / 128 * (int64_t)(M / 128) <= vk_device_cus()) return false;
   if (matrices > 0 && (int64_t)M + 127 <= (int64_t)matrices * (127 + 60)) return true;
   if (columns % 8 == 0 || columns > 16) return 8 * groups >= 5 * vk_device_cus();
   return !named && columns <= 4 && 2 * groups >= vk_device_cus();
@@ -1254,11 +1220,12 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
                        int form, hipStream_t st, const int32_t* block_weights = nullptr, int64_t weights_stride = 0,
                        const int32_t* row_pair = nullptr, const int32_t* act_row = nullptr, int matrices = 0) {
   constexpr int BN = SWIGLU ? 64 : 32 * FNW;                         // output columns of a workgroup
+  static_assert(S >= 2 && S <= 4, "the waits count up to two tiles behind the next");
   const size_t smem = (size_t)S * (32 * FNW + 128) * T_ROWB;         // also holds the 32 KB that SWIGLU passes between waves
   static bool configured = false;
   if (!configured) {
-    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 0, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, false, SWIGLU, FNW, 0, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, false, SWIGLU, FNW, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     configured = true;
   }
   dim3 grid((N + BN - 1) / BN, (M + 127) / 128);
@@ -1275,33 +1242,23 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
       constexpr size_t wide_smem = (size_t)3 * (256 + 128) * T_ROWB;
       static bool wide = false;
       if (!wide) {
-        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<3, true, false, 4, 0, 4, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_smem);
+        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<3, true, false, 4, 4, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_smem);
         wide = true;
       }
       const dim3 wgrid((N + 255) / 256, grid.y);
-      gemm_pipe_kernel<3, true, false, 4, 0, 4, true><<<wgrid, 512, wide_smem, st>>>(out, act, w, M, N, K, lda, ldo, form, wgrid.x > 16 ? 16 : (int)wgrid.x, block_weights,
+      gemm_pipe_kernel<3, true, false, 4, 4, true><<<wgrid, 512, wide_smem, st>>>(out, act, w, M, N, K, lda, ldo, form, wgrid.x > 16 ? 16 : (int)wgrid.x, block_weights,
                                                                               weights_stride, row_pair, act_row);
       return vk_check_launch("gemm_pipe (grouped)");
     }
   }
-  const int band_w = (pipe_band_blocks > 0 && grid.y > 1 && (int)grid.x > pipe_band_blocks) ? pipe_band_blocks : (int)grid.x;
-  if constexpr (S == 2 && (FNW == 2 || FNW == 4)) {
-    // No more workgroups than compute units: each waits for its own loads with nothing to run meanwhile, and
-    // touching the lines four tiles ahead brings them into the second-level cache in time (300 rows, 4,096 x
-    // 12,288: 146 -> 112 us).  With more workgroups the touches cost more than they bring: the path from
-    // that cache into LDS is as busy as the MFMA unit (2,048 rows: 1,057 -> 660 TFLOP/s).
-    if (K % KC == 0 && (int64_t)grid.x * grid.y <= vk_device_cus()) {
-      static bool touched = false;
-      if (!touched) {
-        (void)hipFuncSetAttribute((const void*)gemm_pipe_kernel<S, true, SWIGLU, FNW, 4, 2, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        touched = true;
-      }
-      gemm_pipe_kernel<S, true, SWIGLU, FNW, 4, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
-      return vk_check_launch("gemm_pipe");
-    }
+  // No more workgroups than compute units: four stages (pipe_fragments_in_one_round says why).
+  if constexpr (S == 2 && (SWIGLU || GROUPED)) {
+    if ((int64_t)grid.x * grid.y <= vk_device_cus())
+      return launch_pipe<4, SWIGLU, FNW, GROUPED>(out, act, w, M, N, K, lda, ldo, form, st, block_weights, weights_stride, row_pair, act_row, matrices);
   }
-  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW, 0, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
-  else gemm_pipe_kernel<S, false, SWIGLU, FNW, 0, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
+  const int band_w = (pipe_band_blocks > 0 && grid.y > 1 && (int)grid.x > pipe_band_blocks) ? pipe_band_blocks : (int)grid.x;
+  if (K % KC == 0) gemm_pipe_kernel<S, true, SWIGLU, FNW, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
+  else gemm_pipe_kernel<S, false, SWIGLU, FNW, 2, GROUPED><<<grid, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, band_w, block_weights, weights_stride, row_pair, act_row);
   return vk_check_launch("gemm_pipe");
 }
 
@@ -1888,14 +1845,17 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //              else                                            9   the streaming kernel would need a second pass for a few tiles
 //                                                                  (32 rows, 5120 x 17408: 111 -> 65 us)
 //   17..64   K not in whole chunks                             2 (rows > 32 and wg128 >= 0.5 cus), else 7 / 1 as above
-//   65..256  K whole chunks, wg128 < 0.5 cus:                      the tile kernel would have a workgroup or less per unit, each
-//                                                                  walking all of K alone (4096 x 12288: 170 us at any of these
-//                                                                  rows); the LDS-sharing kernel in blocks of 64 rows fills the
-//                                                                  chip (100 rows: 51 us, 200 rows: 82 us)
-//              wg64 >= 0.5 cus                                 8 up to three blocks, else 2
-//              two blocks                                      9 (wg32 <= 0.5 cus) or 8
-//              else                                            2 (k_resident and wg16 >= 1.5 cus) or 8
-//   more                                                       2   the pipelined tile kernel, or the alternating one
+//   65..256  K whole chunks, wg128 < 0.5 cus:                      the kernel that shares activations through LDS, in blocks of 64 rows
+//              16-bit, two blocks, K > 2 chunks,               9   so few weight rows that the tile kernel's workgroups of 64 leave three
+//                wg32 <= 0.5 cus                                     quarters of the units idle (128 rows, 4096 x 12288: 81 us against
+//                                                                  54; 1024 x 2048: 13.7 against 11.6)
+//              16-bit                                          2   the tile kernel in one round (pipe_fragments_in_one_round; 200 rows,
+//                                                                  6144 x 4096: 40 -> 27 us)
+//              32-bit, wg64 >= 0.5 cus                         8 up to three blocks, else 2
+//              32-bit, two blocks                              9 (wg32 <= 0.5 cus) or 8
+//              32-bit, else                                    2 (k_resident and wg16 >= 1.5 cus) or 8
+//   more                                                       2   the pipelined tile kernel, in one round where it can be
+//                                                                  (pipe_fragments_in_one_round), or the alternating one
 //                                                                  (alternate_fragments)
 // With a workspace the products of up to 64 rows that vk_gemm_split_preferred names go through chunk sums
 // instead (the caller's choice: vk_gemm_split).
@@ -1917,6 +1877,7 @@ static int choose_gemm_kernel(int M, int N, int K) {
   if (M <= 64) return (2 * wg128 >= cus && M > 32) ? 2 : (many16 ? 7 : 1);
   if (M <= 256 && whole && 2 * wg128 < cus) {
     const int blocks = (M + 63) / 64;
+    if (sizeof(elem_t) == 2) return blocks == 2 && 2 * wg32 <= cus && K > 2 * KC ? 9 : 2;
     if (2 * wg64 >= cus) return blocks <= 3 ? 8 : 2;
     if (blocks == 2) return 2 * wg32 <= cus ? 9 : 8;
     return (k_resident && many16) ? 2 : 8;
@@ -1986,6 +1947,25 @@ static int pipe_fragments_by_rounds(int M, int N, double* rounds_of_128 = nullpt
   return best;
 }
 
+// How many weight fragments a wave of the tile kernel takes where that leaves no compute unit with more than one workgroup (2, 3 or 4), or 0.
+// A workgroup that is alone on its unit has only its own stages to cover the way from memory, and two tiles of 32 KB do not: four stages (96 to 128
+// KB of LDS, which it has to itself) keep three on their way, and of the tiles that give one round the narrowest puts most units to work.  Measured
+// on MI355X in recorded launches with the weights of several layers in turn, against 64 weight rows with two stages that touch their lines four
+// tiles ahead (below 257 rows: the kernels that share activations through LDS), us: 4,096 x 12,288, 130 rows 74 -> 68, 512 rows 126 -> 81, 1,000 rows
+// (96 weight rows) 145 -> 114; 6,144 x 4,096, 300 rows 51 -> 33; 2,048 x 6,144, 651 rows 53 -> 36; 1,024 x 1,024, 65 to 1,024 rows 9.7 to 10.7 -> 8.6;
+// with SwiGLU 9,728 x 2,560, 100 rows 47 -> 34; grouped, 2,048 x 2,048, 16 blocks 37 -> 27.  556 plain sizes of 65 to 2,048 rows (N of 1,024 to
+// 16,384, K of 1,024 to 12,288) 25.8 -> 19.6 ms (three of them 3 to 5 % slower: 128 rows, 5,120 to 8,192 x 6,144), 102 with SwiGLU 3.21 -> 2.73.
+// Three stages are 5 % slower with 64 weight rows and as fast with 96 and 128, five and six are slower.  32-bit elements are bound by the matrix unit:
+// 96 weight rows 4.02 -> 3.29 ms over 27 sizes, the others within 2 %.
+static int pipe_fragments_in_one_round(int M, int N, int K) {
+  const int64_t mb = (M + 127) / 128;
+  if ((N + 63) / 64 * mb <= vk_device_cus()) return 2;
+  if ((N + 95) / 96 * mb <= vk_device_cus()) return 3;
+  // 32-bit elements, K of up to two chunks, and K not in whole chunks are as fast with two workgroups of 64 rows a unit (two stages).
+  if (sizeof(elem_t) == 2 && K % KC == 0 && K > 2 * KC && (N + 127) / 128 * mb <= vk_device_cus()) return 4;
+  return 0;
+}
+
 #ifdef VK_BF16
 // How many weight fragments a wave of the alternating kernel takes (6, 5 or 4), or 0: the tile kernel is the faster one.  Both kernels' times go in
 // rounds of the workgroups that run at a time, one a compute unit here; with k = K / 1,024 a round was measured at 13.1 k + 7, 15.8 k + 6 and
@@ -1994,8 +1974,8 @@ static int pipe_fragments_by_rounds(int M, int N, double* rounds_of_128 = nullpt
 static int alternate_fragments(int M, int N, int K, bool swiglu) {
   if (M < 256 || K % KC != 0 || N < (swiglu ? 96 : 192)) return 0;
   const int cus = vk_device_cus(), out_cols = swiglu ? 2 * N : N;
-  // At most one workgroup a compute unit of the tile kernel's: its round is shorter then than a full one's 0.72 (1,536 x 2,048 with SwiGLU, 256 to 512
-  // rows: 26 to 29 us against 30).  The plain product's caller has asked that before.
+  // At most one workgroup a compute unit of the tile kernel's: its round is shorter then than a full one's 0.72, and has four stages (1,536 x 2,048 with SwiGLU, 256 to 512
+  // rows: 22 to 23 us against 30).  The plain product's caller has asked that before.
   if (swiglu && (int64_t)((N + 63) / 64) * ((M + 127) / 128) <= cus) return 0;
   static const double slope[7] = {0, 0, 0, 0, 13.1, 15.8, 18.9}, start[7] = {0, 0, 0, 0, 7, 6, 8};
   const double k = K / 1024.0;
@@ -2229,9 +2209,13 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   if (kernel == 6 && k_whole) return launch_pipe<4>(out, act, w, M, N, K, lda, ldo, form, st);
   // Two stages of 32 KB leave room for two workgroups per compute unit, which hides more latency than a third stage.
   if (k_whole) {
-    // No more 128 x 128 tiles than compute units: 64 weight rows a workgroup, twice as many of them
-    // (512 rows, 4096 x 12288: 163 -> 145 us; a workgroup alone on its compute unit is bound by what one
-    // compute unit can read, whatever the number of stages).
+    if (by_size) {
+      const int f = pipe_fragments_in_one_round(M, N, K);
+      if (f == 2) return launch_pipe<4, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
+      if (f == 3) return launch_pipe<4, false, 3>(out, act, w, M, N, K, lda, ldo, form, st);
+      if (f == 4) return launch_pipe<4>(out, act, w, M, N, K, lda, ldo, form, st);
+    }
+    // No more 128 x 128 tiles than compute units: 64 weight rows a workgroup, twice as many of them.
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
     if (kernel == 13 || (by_size && tiles <= vk_device_cus())) return launch_pipe<2, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
 #ifdef VK_BF16
