@@ -1448,6 +1448,185 @@ static int launch_alternate(elem_t* out, const elem_t* act, const elem_t* w, int
 }
 #endif
 
+#ifdef VK_BF16
+// ---------------------------------------------------------------- few rows
+// 17 to 64 rows of 16-bit elements, K in whole chunks.  The streaming kernels and the one that shares activations through LDS bring weights into
+// registers in the order of the matrix unit's operands: an instruction touches 16 rows, half a cache line of each, which holds them to about 4 TB/s.  Here tiles of
+// TS slabs of a row, one or two whole lines, go from memory straight into LDS, weights (read by this workgroup alone: past the caches) and activations
+// alike, S of them in a ring, one barrier a tile.  A workgroup has NW waves and walks all of K; a wave has FNW x 16 weight rows, or with
+// SwiGLU 16 gate rows and the 16 up rows that go with them, and all 16 FA activation rows.  Operand roles, reduction order and bits are those of
+// gemm_pipe_kernel.  A row's 16-byte piece j lies at piece j ^ (row mod pieces), so that 16 rows' fragments lie on different banks.  Rows beyond N or
+// M are the last one again (their results are dropped).
+//
+// What bounds it: memory where enough bytes are on their way (151,936 x 4,096, 17 rows: 5.9 TB/s), below that a workgroup's chain of a wait, a barrier, the
+// fragments' way from LDS and the MFMAs for each tile; several workgroups a compute unit cover each other, so stages are kept to what lets three (up to 32 rows) or two
+// fit a unit: six or twelve stages with fewer of them are 2 to 15 % slower.  Measured on MI355X in recorded launches with the weights
+// of several layers in turn, before and after, us, 17 and 64 rows: with SwiGLU 17,408 x 5,120 89 -> 72, 101 -> 93; 9,728 x 2,560 30.6 -> 22.3, 32.9 -> 26.8; 6,144 x 2,048
+// 18.1 -> 12.4, 20.8 -> 14.2; plain 7,168 x 5,120 23.2 -> 15.7, 29.9 -> 23.8; 12,288 x 4,096 24.5 -> 20.7, 33.2 -> 24.1; 32,768 x 2,048 34.6 -> 27.2, 36.6 -> 28.1.
+template <int NW, int FNW, int FA, int TS, int S, bool SWIGLU>
+__global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w,
+                                                           int M, int N, int K, int64_t lda, int64_t ldo, int out_form) {
+  static_assert(!SWIGLU || FNW == 2, "a wave has its gate rows and the up rows that go with them");
+  constexpr int ROWB = TS * VK_SLAB * (int)sizeof(elem_t), LOAD_ROWS = 1024 / ROWB, PIECES = ROWB / 16;
+  constexpr int BN = 16 * FNW * NW, BM = 16 * FA;
+  constexpr int LW = 16 * FNW / LOAD_ROWS, LA = BM / LOAD_ROWS / NW, PER_TILE = LW + LA;      // loads a tile and wave
+  constexpr int STAGE = (BN + BM) * ROWB, CHUNK_TILES = KC / (TS * VK_SLAB);
+  static_assert(LA * NW * LOAD_ROWS == BM, "the waves bring as many activation rows each");
+  static_assert((S - 2) * PER_TILE < 64, "loads in flight are counted by six bits");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int n0 = (blockIdx.x * NW + wave) * 16 * (SWIGLU ? 1 : FNW);
+  const int first = min(n0, N - 1), ntiles = K / (TS * VK_SLAB);
+  // Load j of a wave's weights or activations brings LOAD_ROWS rows, a kilobyte; lane i fills piece i % PIECES of row i / PIECES.
+  const int lr = lane / PIECES, lp = lane % PIECES;
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (int64_t)first * K);
+  const unsigned char* ubase = reinterpret_cast<const unsigned char*>(w + (int64_t)(N + first) * K);
+  const unsigned char* abase = reinterpret_cast<const unsigned char*>(act);
+  unsigned offw[LW], offa[LA];
+#pragma unroll
+  for (int j = 0; j < LW; ++j) {
+    const int row = j * LOAD_ROWS + lr, local = SWIGLU ? row & 15 : row;
+    offw[j] = (unsigned)(((int64_t)(min(n0 + local, N - 1) - first) * K + ((lp ^ (row & (PIECES - 1))) * VK_VEC)) * (int64_t)sizeof(elem_t));
+  }
+#pragma unroll
+  for (int j = 0; j < LA; ++j) {
+    const int row = (wave * LA + j) * LOAD_ROWS + lr;
+    offa[j] = (unsigned)(((int64_t)min(row, M - 1) * lda + ((lp ^ (row & (PIECES - 1))) * VK_VEC)) * (int64_t)sizeof(elem_t));
+  }
+  const unsigned lds0 = lds_offset_of(lds);
+  auto issue = [&](int kt, int slot) {
+    const unsigned base = lds0 + slot * STAGE;
+    const int64_t kb = (int64_t)kt * ROWB;
+#pragma unroll
+    for (int j = 0; j < LW; ++j) {
+      const bool up = SWIGLU && j * LOAD_ROWS >= 16;
+      pipe_load_to_lds16_once((up ? ubase : wbase) + kb, offw[j], base + (wave * LW + j) * 1024);
+    }
+#pragma unroll
+    for (int j = 0; j < LA; ++j) pipe_load_to_lds16_sv(abase + kb, offa[j], base + BN * ROWB + (wave * LA + j) * 1024);
+  };
+  f32x4 acc[FNW][FA], total[FNW][FA];
+#pragma unroll
+  for (int i = 0; i < FNW; ++i)
+#pragma unroll
+    for (int j = 0; j < FA; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < S - 1; ++p)
+    if (p < ntiles) issue(p, p);
+  int slot = 0, ahead = S - 1;
+  for (int c = 0; c < ntiles; c += CHUNK_TILES) {
+#pragma unroll
+    for (int u = 0; u < CHUNK_TILES; ++u) {
+      const int kt = c + u;
+      // Tile kt has landed once at most the S - 2 tiles behind it are outstanding; near the end, where there are fewer, once none is.
+      if (kt + S - 2 < ntiles) wait_vmcnt_n<(S - 2) * PER_TILE>();
+      else wait_vmcnt_n<0>();
+      __syncthreads();       // every wave's part of tile kt is there; everyone is done with tile kt - 1's place
+      if (kt + S - 1 < ntiles) issue(kt + S - 1, ahead);
+      const unsigned char* base = lds + slot * STAGE;
+      frag_t wf[TS][FNW], af[TS][FA];
+#pragma unroll
+      for (int s = 0; s < TS; ++s) {
+        const int col = ((s * 4 + kg) ^ (r16 & (PIECES - 1))) * 16;
+#pragma unroll
+        for (int i = 0; i < FNW; ++i) wf[s][i] = *reinterpret_cast<const frag_t*>(base + ((wave * FNW + i) * 16 + r16) * ROWB + col);
+#pragma unroll
+        for (int j = 0; j < FA; ++j) af[s][j] = *reinterpret_cast<const frag_t*>(base + (BN + j * 16 + r16) * ROWB + col);
+      }
+#pragma unroll
+      for (int s = 0; s < TS; ++s)
+#pragma unroll
+        for (int i = 0; i < FNW; ++i)
+#pragma unroll
+          for (int j = 0; j < FA; ++j) acc[i][j] = mma_slab(wf[s][i], af[s][j], acc[i][j]);
+      slot = slot + 1 == S ? 0 : slot + 1;
+      ahead = ahead + 1 == S ? 0 : ahead + 1;
+    }
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < FA; ++j) {
+        total[i][j].x = total[i][j].x + acc[i][j].x;
+        total[i][j].y = total[i][j].y + acc[i][j].y;
+        total[i][j].z = total[i][j].z + acc[i][j].z;
+        total[i][j].w = total[i][j].w + acc[i][j].w;
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  if constexpr (SWIGLU) {
+#pragma unroll
+    for (int j = 0; j < FA; ++j) {
+      f32x4 g = total[0][j], u = total[1][j], y;
+      g.x = round_to_elem(g.x); g.y = round_to_elem(g.y); g.z = round_to_elem(g.z); g.w = round_to_elem(g.w);
+      u.x = round_to_elem(u.x); u.y = round_to_elem(u.y); u.z = round_to_elem(u.z); u.w = round_to_elem(u.w);
+      y.x = (g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x;
+      y.y = (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y;
+      y.z = (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z;
+      y.w = (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w;
+      store_out4(out, ldo, j * 16 + r16, n0 + 4 * kg, M, N, y, out_form);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < FA; ++j) store_out4(out, ldo, j * 16 + r16, n0 + i * 16 + 4 * kg, M, N, total[i][j], out_form);
+  }
+}
+
+template <int NW, int FNW, int FA, int TS, int S, bool SWIGLU = false>
+static int launch_rows(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, hipStream_t st) {
+  constexpr int smem = S * (16 * FNW * NW + 16 * FA) * TS * VK_SLAB * (int)sizeof(elem_t);
+  static_assert(smem <= 160 * 1024, "LDS");
+  static bool configured = false;
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_rows_kernel<NW, FNW, FA, TS, S, SWIGLU>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    configured = true;
+  }
+  constexpr int cols = 16 * NW * (SWIGLU ? 1 : FNW);
+  gemm_rows_kernel<NW, FNW, FA, TS, S, SWIGLU><<<(unsigned)((N + cols - 1) / cols), 64 * NW, smem, st>>>(out, act, w, M, N, K, lda, ldo, form);
+  return vk_check_launch("gemm_rows");
+}
+
+// How a product of 17 to 64 rows is cut for gemm_rows_kernel: the weight rows (with SwiGLU: gate rows) of a workgroup, or 0 where the other kernels are
+// the faster ones.  The narrowest workgroups that still have enough to do are the fastest up to one or two a compute unit; then wider ones, whose
+// activations serve more weights.  Measured over 240 plain sizes (N of 3,072 to 32,768, K of 1,024 to 8,192) and 176 with SwiGLU (1,024 to 25,600 x 1,024 to
+// 5,120); before / after by the number of workgroups of 32, g, against the compute units:
+//   plain   g <= 1/2             the other kernels (which split K over waves or workgroups) 1.02 to 1.8 times as fast, but for K of two chunks
+//           up to 1              32 weight rows (0.98 to 1.55); not for 33 rows and more where g < 3/4 and K is more than 4 chunks (0.91 to 1.02).
+//                                K of 5 to 8 chunks, up to 32 rows, g > 7/8: 64 weight rows (1.03; 32: 0.94)
+//           more                 64 weight rows (1.04 to 2.4)
+//   SwiGLU  g <= 1/2             16 gate rows (1.03 to 2.2; 32: 0.87 to 1.8)
+//           up to 1              32 (1.1 to 2.0); K of 5 to 8 chunks, g > 7/8: 64 (1.01 to 1.28; 32: 0.87 to 1.15)
+//           up to 2, above 3     64 (1.02 to 1.8; 32: 0.97 to 1.8)
+//           above 2, up to 3     32, of which a compute unit holds three (1.03 to 1.6; 64, a nearly empty second round: 0.88 to 1.3)
+static int rows_width(int M, int N, int K, int64_t lda, bool swiglu) {
+  if (M <= 16 || M > 64 || K % KC != 0 || lda > (1 << 25)) return 0;       // a row's offset is of 32 bits
+  const int cus = vk_device_cus(), chunks = K / KC, g = (N + 31) / 32;
+  const bool middle = chunks > 4 && chunks <= 8 && 8 * g > 7 * cus && g <= cus;
+  if (swiglu) {
+    if (2 * g <= cus) return 16;
+    if (g <= cus) return middle ? 64 : 32;
+    return g <= 2 * cus || g > 3 * cus ? 64 : 32;
+  }
+  if (2 * g <= cus || (M > 32 && chunks > 4 && 4 * g < 3 * cus)) return 0;
+  return g > cus || (middle && M <= 32) ? 64 : 32;
+}
+static int gemm_rows(int width, bool swiglu, elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, hipStream_t st) {
+#define ROWS(NW, FNW, TS, S, SWIGLU)                                                                                      \
+  return M <= 32 ? launch_rows<NW, FNW, 2, TS, S, SWIGLU>(out, act, w, M, N, K, lda, ldo, form, st)                       \
+                 : launch_rows<NW, FNW, 4, TS, S, SWIGLU>(out, act, w, M, N, K, lda, ldo, form, st)
+  if (swiglu) {
+    if (width == 16) ROWS(1, 2, 4, 4, true);
+    if (width == 32) ROWS(2, 2, 2, 4, true);
+    ROWS(4, 2, 4, 3, true);
+  }
+  if (width == 32) ROWS(2, 1, 4, 4, false);
+  ROWS(4, 1, 2, 4, false);
+#undef ROWS
+}
+#endif
+
 // ------------------------------------------------------------------ mid
 // 17 to 64 rows.  The streaming kernels read all activations once per 16 weight rows, which at 64 rows
 // is four times the weights and binds them to the second-level cache.  Here a workgroup of eight waves
@@ -1830,8 +2009,7 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //   rows     condition                                         kernel
 //   1..16    where lines_rows says so                           20, 21  whole lines
 //   1..16                                                      1   streaming
-//   17..32   16-bit, K whole chunks, k_resident,               11  streaming, both activation tiles of a wave's chunk in
-//            wg16 >= 1.5 cus                                       registers (32 rows, 24576 x 4096: 53 -> 44 us)
+//   17..64   16-bit, where rows_width says so                   -   gemm_rows_kernel; the rest of this table is then for the others
 //   17..64   K whole chunks:
 //              wg128 >= 0.75 cus                               10  128 weight rows a workgroup: the activations that every
 //                                                                  workgroup reads are half the weight bytes (64 rows, 51200 x
@@ -1865,7 +2043,6 @@ static int choose_gemm_kernel(int M, int N, int K) {
   const bool whole = K % KC == 0, k_resident = K <= SK_WAVES * KC;
   const bool many16 = 2 * wg16 >= 3 * cus;
   if (M <= 16) return 1;
-  if (M <= 32 && whole && k_resident && many16 && sizeof(elem_t) == 2) return 11;
   if (M <= 64 && whole) {
     if (4 * wg128 >= 3 * cus) return 10;
     if (2 * wg64 >= cus) return 8;
@@ -2067,6 +2244,10 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
   if (kernel == 0) {
+#ifdef VK_BF16
+    const int width = rows_width(M, N, K, lda, false);
+    if (width) return gemm_rows(width, false, out, act, w, M, N, K, lda, ldo, form, st);
+#endif
     const int rows = lines_rows(M, N, K, 1);
     kernel = rows ? (rows == 4 ? 20 : 21) : choose_gemm_kernel(M, N, K);
   }
@@ -2246,12 +2427,11 @@ int vk_gemm_act(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, i
 }
 
 // 1 if vk_gemm_swiglu takes these sizes (the caller otherwise runs vk_gemm and vk_swiglu, with the same result).
-// 1: the streaming kernel (few rows), 2: the pipelined tile kernel (many rows), 3: the kernel for 17 to 64
-// rows that shares activations through LDS, 0: none.
+// 1: the streaming kernels (few rows), 2: the pipelined tile kernel (many rows), 3: the kernels for 17 to 64
+// rows, 0: none.
 int vk_gemm_swiglu_supported(int M, int I, int K) {
   if (M >= 1 && M <= 16 && I > 0 && K % KC == 0 && K <= SK_WAVES * KC) return 1;
 #ifdef VK_BF16
-  if (M > 16 && M <= 32 && I > 0 && K % KC == 0 && K <= SK_WAVES * KC) return 1;    // two activation tiles in registers
   if (M >= 1 && M <= 16 && I > 0 && K % KC == 0 && K <= 2 * SK_WAVES * KC) return 1;   // two chunks a wave
 #endif
   if (M > 64 && I > 0 && K % (2 * VK_SLAB) == 0) return 2;
@@ -2275,6 +2455,10 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
 #endif
   if (how == 2)
     return launch_pipe<2, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+#ifdef VK_BF16
+  if (const int width = how == 3 ? rows_width(M, I, K, lda, true) : 0)
+    return gemm_rows(width, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+#endif
   if (how == 3) {
     const int ok4 = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
     // Gate tiles per workgroup: of four, three and two, the number whose workgroups fill the compute units
@@ -2333,7 +2517,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
     else if (rows == 1) SWIGLU_STREAMH(8, 1, 1, NW, 1);                                                    \
     else SWIGLU_STREAMH(8, 1, 1, NW, 0);                                                                   \
   } while (0)
-  const int nw = M <= 16 ? stream_waves(K / KC) : SK_WAVES;       // as in vk_gemm
+  const int nw = stream_waves(K / KC);       // as in vk_gemm
   if (nw == 2) SWIGLU_STREAMN(2);
   else if (nw == 4) SWIGLU_STREAMN(4);
   else if (nw == 5) SWIGLU_STREAMN(5);
@@ -2344,8 +2528,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
 #endif
   else
 #ifdef VK_BF16
-  if (M > 16) SWIGLU_STREAM(4, 2, 1);
-  else if (K > SK_WAVES * KC) SWIGLU_STREAM(4, 1, 2);
+  if (K > SK_WAVES * KC) SWIGLU_STREAM(4, 1, 2);
   else
 #endif
     SWIGLU_STREAMN(SK_WAVES);
@@ -2477,8 +2660,8 @@ int64_t vk_gemm_split_floats(int M, int rows, int K, int swiglu) {
 // unit (1000 x 1024 at 32 rows: 4.8 -> 6.5 us), and not where workgroups of 128 weight rows are a quarter of the
 // compute units or more: the other kernels then have workgroups enough, and the chunk sums would be a large
 // share of the traffic.
-//   17 to 64 rows: always then (64 rows: 4096 x 12288 45 -> 32 us, 6144 x 4096 20.6 -> 18.2, 4096 x 4096 16.0 -> 13.8;
-//     32 rows: 41 -> 27, 17.8 -> 14.7, 13.4 -> 11.7 us).
+//   17 to 64 rows: always then (64 rows: 4096 x 12288 45 -> 32 us, 4096 x 4096 16.0 -> 13.8; 32 rows: 41 -> 27, 13.4 -> 11.7 us).  Where rows_width
+//     takes such sizes, which is faster still, vk_gemm_split does so too and leaves the workspace alone.
 //   Up to 16 rows the streaming kernel is the other choice.  With `fill` the share of the compute units that
 //   its last round of one workgroup per 16 weight rows keeps busy:
 //     K of more than 16 chunks (its waves read their activations again for every chunk): when fill < 0.9
@@ -2517,6 +2700,8 @@ static int gemm_split_launch(elem_t* out, const elem_t* act, const elem_t* w, in
 #ifdef VK_BF16
   const int form = out_form_of(out, ldo, activation);
   const int mt = (M + 15) / 16;
+  const int width = vk_gemm_split_preferred(M, rows, K, swiglu) ? rows_width(M, rows, K, lda, false) : 0;
+  if (width) return gemm_rows(width, false, out, act, w, M, rows, K, lda, ldo, form, st);
   if (mt == 1) return launch_split<1>(out, act, w, M, rows, K, lda, ldo, swiglu, workspace, form, st);
   if (mt == 2) return launch_split<2>(out, act, w, M, rows, K, lda, ldo, swiglu, workspace, form, st);
   if (mt == 3) return launch_split<3>(out, act, w, M, rows, K, lda, ldo, swiglu, workspace, form, st);
