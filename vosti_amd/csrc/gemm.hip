@@ -21,7 +21,9 @@
 //   gemm_stream_swiglu  the same for the gate/up projection with SwiGLU folded in (M <= 16).
 //   gemm_lines          M <= 16, K a multiple of 512 up to 6,144, 16-bit elements: weights and activations through LDS in whole lines, tiles of eight
 //                       or four weight rows, optionally SwiGLU in the epilogue (lines_rows says when).
-//   gemm_mid            17 <= M <= 64, K a multiple of 512: 64 or 32 weight rows per workgroup, weights
+//   gemm_rows           17 <= M <= 64, K a multiple of 512, 16-bit elements: weights and activations through LDS in whole lines, a workgroup walks all
+//                       of K, optionally SwiGLU in the epilogue (rows_width says when).
+//   gemm_mid            17 <= M <= 64 (more in blocks), K a multiple of 512: 64 or 32 weight rows per workgroup, weights
 //                       streamed into registers, the activations of the chunks in work shared through LDS.
 //   gemm_split          M <= 64, K a multiple of 512, 16-bit elements, with a workspace: a workgroup per
 //                       (128 weight rows, chunk) leaves its chunk sums in the workspace, a second kernel
@@ -29,7 +31,8 @@
 //   gemm_skinny         M <= 64, any K: the same decomposition with predicated loads.
 //   gemm_pipe           any M, K a multiple of two slabs (128 bytes of a row): 128x128 output tile per
 //                       workgroup, 64x64 per wave, tiles straight from global memory into LDS, two
-//                       stages; a second accumulator set holds the total.  Optionally SwiGLU in the
+//                       stages, or four and 64 or 96 weight rows where no compute unit has more than one
+//                       workgroup (pipe_fragments_in_one_round); a second accumulator set holds the total.  Optionally SwiGLU in the
 //                       epilogue.
 //   gemm_alternate      256 rows or more, K a multiple of 512, 16-bit elements: 256 x 192, 160 or 128 per workgroup of eight
 //                       waves whose two halves take turns between LDS and the matrix unit.  Optionally SwiGLU in the epilogue
@@ -1628,7 +1631,8 @@ static int gemm_rows(int width, bool swiglu, elem_t* out, const elem_t* act, con
 #endif
 
 // ------------------------------------------------------------------ mid
-// 17 to 64 rows.  The streaming kernels read all activations once per 16 weight rows, which at 64 rows
+// 17 to 64 rows, of 16-bit elements those that rows_width leaves (at most 4,096 weight rows, mostly) and up to 128 in blocks.  The streaming kernels
+// read all activations once per 16 weight rows, which at 64 rows
 // is four times the weights and binds them to the second-level cache.  Here a workgroup of eight waves
 // takes 64 weight rows: wave (nt, kh) streams weight tile nt (16 rows) for the chunks kh, kh + 2, ...
 // into registers with a rolling window, as the streaming kernels do, and the activations of the two
@@ -2461,7 +2465,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
 #endif
   if (how == 3) {
     const int ok4 = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
-    // Gate tiles per workgroup: of four, three and two, the number whose workgroups fill the compute units
+    // (32-bit elements, and rows too far apart for gemm_rows_kernel; the figures are 16-bit.)  Gate tiles per workgroup: of four, three and two, the number whose workgroups fill the compute units
     // best, a workgroup per unit at a time; the larger one where two fill them alike.  64 rows, K = 4096:
     // 12288 gate rows (192, 256, 384 workgroups) 55.4, 49.7, 58.5 us; 8192 gate rows (128, 171, 256) 52.8, 47.0,
     // 41.6 us; 17408 gate rows at K = 5120 (272, 363, 544) 127.5, 108.4, 123.2 us.
