@@ -512,20 +512,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(elem_t* __restrict
 // two projections rounded to the element type first, which is what the separate
 // GEMM and SwiGLU kernels compute (kernels/triton_kernels/silu_mul.py:64-87).
 // M <= 16, K <= 4096 (activations resident in registers).
-template <int W, int MT, int RC, int NW = SK_WAVES, int ROWS = 0, bool NORM = false>
+template <int W, int RC, int NW = SK_WAVES, int ROWS = 0, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __restrict__ out,
                                                                            const elem_t* __restrict__ act,
                                                                            const elem_t* __restrict__ w, int M, int I,
                                                                            int K, int64_t lda, int64_t ldo,
                                                                            int out_form, NormArgs norm) {
   static_assert(KC_SLABS % W == 0, "the window must divide a chunk");
-  static_assert(MT * RC <= 2, "two chunk tiles of activations stay in registers: two tiles of a chunk or two chunks of a tile");
-  __shared__ f32x4 part[2][RC][NW][2 * MT][64];      // two sets, used in turn: one barrier per tile
+  static_assert(RC <= 2, "two chunks of activations stay in registers");
+  __shared__ f32x4 part[2][RC][NW][2][64];      // two sets, used in turn: one barrier per tile
 
-  static_assert(ROWS == 0 || (MT == 1 && RC == 1), "one chunk tile of activations comes through LDS");
-  // As in the kernel above; two projections' windows leave fewer registers.  Two tiles of rows: the loop in one piece took 3,072 x 1,024, 24 rows 11.0 us,
-  // as a function of its own 11.4, and written out twice 10.0 (12,288 x 4,096, 20 rows 44.0, 43.6 and 41.8).
-  constexpr bool EARLY = MT == 2 || (ROWS > 0 && NW <= 8);
+  static_assert(ROWS == 0 || RC == 1, "one chunk tile of activations comes through LDS");
+  // As in the kernel above; two projections' windows leave fewer registers.
+  constexpr bool EARLY = ROWS > 0 && NW <= 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];      // CHUNK_ROWS_BYTES(ROWS) a wave
   const int lane = threadIdx.x & 63, wave = ROWS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
@@ -542,17 +541,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
   }
 
   // Wave w has chunks w, w + 8, ...: RC of them (chunks beyond K are read as the last and not used).
-  frag_t wg[W], wu[W], abuf[RC * KC_SLABS][MT];
+  frag_t wg[W], wu[W], abuf[RC * KC_SLABS];
 #pragma unroll
   for (int r = 0; r < (ROWS ? 0 : RC); ++r) {
     const int c = min(r * NW + wave, nchunks - 1);
+    const elem_t* arow = act + (int64_t)min(r16, M - 1) * lda + kg * VK_VEC;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const elem_t* arow = act + (int64_t)min(mt * 16 + r16, M - 1) * lda + kg * VK_VEC;
-#pragma unroll
-      for (int s = 0; s < KC_SLABS; ++s)
-        abuf[r * KC_SLABS + s][mt] = *reinterpret_cast<const frag_t*>(arow + c * KC + s * VK_SLAB);
-    }
+    for (int s = 0; s < KC_SLABS; ++s) abuf[r * KC_SLABS + s] = *reinterpret_cast<const frag_t*>(arow + c * KC + s * VK_SLAB);
   }
   // Slab g of this wave's stream over a tile: chunk (g / 16) * 8 + wave, slab g % 16 of it.
   const int my_chunks = wave < nchunks ? (nchunks - wave + NW - 1) / NW : 0;     // <= RC
@@ -578,7 +573,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
       return ChunkRows<ROWS>::place(rows_lds + g / PER_CHUNK * CHUNK_ROWS_BYTES(ROWS), row, g % PER_CHUNK * 64 + lane);
     });
 #pragma unroll
-    for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
+    for (int i = 0; i < KC_SLABS; ++i) abuf[i] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
   } else if constexpr (ROWS > 0) {
     if (active) {                                        // as in the kernel above
       __builtin_amdgcn_sched_barrier(0);
@@ -586,7 +581,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < KC_SLABS; ++i) abuf[i][0] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
+      for (int i = 0; i < KC_SLABS; ++i) abuf[i] = ChunkRows<ROWS>::fragment(own_rows, i, r16, kg);
     } else {
       wait_vmcnt_n<0>();
     }
@@ -598,9 +593,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
     const bool ask = NEXT == 2 ? nt < ntiles : NEXT == 1;
 #pragma unroll
     for (int r = 0; r < RC; ++r) {
-      f32x4 ag[MT], au[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) ag[mt] = au[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
       if (r < my_chunks) {
 #pragma unroll
         for (int i = 0; i < KC_SLABS; ++i) {
@@ -609,26 +602,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
           const int g = r * KC_SLABS + i + W;             // the slab that takes this slot
           if (EARLY ? i + W < KC_SLABS : g < my_slabs) issue(tile, g, slot);
           else if (ask) issue(nt, g - my_slabs, slot);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            ag[mt] = mma_slab(fg, abuf[r * KC_SLABS + i][mt], ag[mt]);
-            au[mt] = mma_slab(fu, abuf[r * KC_SLABS + i][mt], au[mt]);
-          }
+          ag = mma_slab(fg, abuf[r * KC_SLABS + i], ag);
+          au = mma_slab(fu, abuf[r * KC_SLABS + i], au);
           if (EARLY) __builtin_amdgcn_sched_barrier(0);
         }
       }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        part[parity][r][wave][2 * mt][lane] = ag[mt];
-        part[parity][r][wave][2 * mt + 1][lane] = au[mt];
-      }
+      part[parity][r][wave][0][lane] = ag;
+      part[parity][r][wave][1][lane] = au;
     }
     __syncthreads();
-    if (wave < MT) {       // wave mt adds up, in chunk order, and finishes the rows of activation tile mt
+    if (wave == 0) {       // adds up, in chunk order, and finishes the rows
       f32x4 tg = {0.f, 0.f, 0.f, 0.f}, tu = {0.f, 0.f, 0.f, 0.f};
       for (int c = 0; c < nchunks; ++c) {
-        const f32x4 pg = part[parity][c / NW][c % NW][2 * wave][lane];
-        const f32x4 pu = part[parity][c / NW][c % NW][2 * wave + 1][lane];
+        const f32x4 pg = part[parity][c / NW][c % NW][0][lane];
+        const f32x4 pu = part[parity][c / NW][c % NW][1][lane];
         tg.x = tg.x + pg.x; tg.y = tg.y + pg.y; tg.z = tg.z + pg.z; tg.w = tg.w + pg.w;
         tu.x = tu.x + pu.x; tu.y = tu.y + pu.y; tu.z = tu.z + pu.z; tu.w = tu.w + pu.w;
       }
@@ -639,7 +626,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
       y.y = (g[1] * (1.0f / (1.0f + expf(-g[1])))) * u[1];
       y.z = (g[2] * (1.0f / (1.0f + expf(-g[2])))) * u[2];
       y.w = (g[3] * (1.0f / (1.0f + expf(-g[3])))) * u[3];
-      store_out4(out, ldo, wave * 16 + r16, tile * 16 + 4 * kg, M, I, y, out_form);
+      store_out4(out, ldo, r16, tile * 16 + 4 * kg, M, I, y, out_form);
     }
     parity ^= 1;
   };
@@ -2493,7 +2480,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   if (lines == 4) return launch_lines<4, 2>(out, act, w, M, I, K, lda, ldo, form, st);
   if (lines == 8) return launch_lines<8, 2>(out, act, w, M, I, K, lda, ldo, form, st);
 #endif
-#define SWIGLU_STREAMH(W, MT, RC, NW, ROWS)                                                               \
+#define SWIGLU_STREAMH(W, RC, NW, ROWS)                                                                   \
   do {                                                                                                     \
     constexpr size_t rows_bytes = (size_t)NW * CHUNK_ROWS_BYTES(ROWS);                                \
     static int resident = 0;                                                                               \
@@ -2502,24 +2489,24 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
       (void)hipGetDevice(&dev);                                                                            \
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);                       \
       if (rows_bytes)                                                                                      \
-        (void)hipFuncSetAttribute((const void*)gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS>,           \
+        (void)hipFuncSetAttribute((const void*)gemm_stream_swiglu_kernel<W, RC, NW, ROWS>,           \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_bytes);            \
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS>, \
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gemm_stream_swiglu_kernel<W, RC, NW, ROWS>, \
                                                          64 * NW, rows_bytes);                             \
       resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);                                        \
     }                                                                                                      \
-    gemm_stream_swiglu_kernel<W, MT, RC, NW, ROWS><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
+    gemm_stream_swiglu_kernel<W, RC, NW, ROWS><<<ntiles < resident ? ntiles : resident, 64 * NW, rows_bytes, st>>>( \
         out, act, w, M, I, K, lda, ldo, form, NormArgs{});                                                \
   } while (0)
-#define SWIGLU_STREAM(W, MT, RC) SWIGLU_STREAMH(W, MT, RC, SK_WAVES, 0)
+#define SWIGLU_STREAM(W, RC) SWIGLU_STREAMH(W, RC, SK_WAVES, 0)
 #define SWIGLU_STREAMN(NW)                                                                                 \
   do {                                                                                                     \
     const int rows = stream_rows_pay(M, ntiles, lda) ? stream_lds_rows(M, NW, NW * 4096) : 0;                   \
-    if (rows == 16) SWIGLU_STREAMH(8, 1, 1, NW, stream_lds_rows(16, NW, NW * 4096));                       \
-    else if (rows == 8) SWIGLU_STREAMH(8, 1, 1, NW, stream_lds_rows(8, NW, NW * 4096));                    \
-    else if (rows == 4) SWIGLU_STREAMH(8, 1, 1, NW, 4);                                                    \
-    else if (rows == 1) SWIGLU_STREAMH(8, 1, 1, NW, 1);                                                    \
-    else SWIGLU_STREAMH(8, 1, 1, NW, 0);                                                                   \
+    if (rows == 16) SWIGLU_STREAMH(8, 1, NW, stream_lds_rows(16, NW, NW * 4096));                       \
+    else if (rows == 8) SWIGLU_STREAMH(8, 1, NW, stream_lds_rows(8, NW, NW * 4096));                    \
+    else if (rows == 4) SWIGLU_STREAMH(8, 1, NW, 4);                                                    \
+    else if (rows == 1) SWIGLU_STREAMH(8, 1, NW, 1);                                                    \
+    else SWIGLU_STREAMH(8, 1, NW, 0);                                                                   \
   } while (0)
   const int nw = stream_waves(K / KC);       // as in vk_gemm
   if (nw == 2) SWIGLU_STREAMN(2);
@@ -2532,7 +2519,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
 #endif
   else
 #ifdef VK_BF16
-  if (K > SK_WAVES * KC) SWIGLU_STREAM(4, 1, 2);
+  if (K > SK_WAVES * KC) SWIGLU_STREAM(4, 2);
   else
 #endif
     SWIGLU_STREAMN(SK_WAVES);
@@ -2557,8 +2544,8 @@ static int launch_stream_normed(elem_t* out, const elem_t* x, const elem_t* w, i
   constexpr int LDS = NW * CHUNK_ROWS_BYTES(ROWS);
   const int tiles = (N + 15) / 16;
   if constexpr (P == 2) {
-    static const int at_once = workgroups_at_once(gemm_stream_swiglu_kernel<8, 1, 1, NW, ROWS, true>, 64 * NW, LDS);
-    gemm_stream_swiglu_kernel<8, 1, 1, NW, ROWS, true><<<std::min(tiles, at_once), 64 * NW, LDS, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, norm);
+    static const int at_once = workgroups_at_once(gemm_stream_swiglu_kernel<8, 1, NW, ROWS, true>, 64 * NW, LDS);
+    gemm_stream_swiglu_kernel<8, 1, NW, ROWS, true><<<std::min(tiles, at_once), 64 * NW, LDS, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, norm);
   } else {
     static const int at_once = workgroups_at_once(gemm_stream_kernel<1, 8, 1, 1, NW, ROWS, true>, 64 * NW, LDS);
     gemm_stream_kernel<1, 8, 1, 1, NW, ROWS, true><<<std::min(tiles, at_once), 64 * NW, LDS, st>>>(out, x, w, M, N, NW * KC, ldx, ldo, form, norm);
