@@ -59,3 +59,16 @@ def test_rows_apart_from_magnitude():
     y = k.add_rmsnorm(x, residual, weight, 1e-6)
     assert torch.equal(out.view(torch.int16), k.gemm(y, w, kernel=4).view(torch.int16)) or torch.equal(out.isnan(), k.gemm(y, w, kernel=4).isnan())
     assert torch.equal(out[[0, 1, 3]], k.gemm(y, w, kernel=4)[[0, 1, 3]]) and torch.equal(total.view(torch.int16), residual.view(torch.int16))
+
+
+def test_a_negative_eps_is_refused():
+    """As the norm by itself refuses it: a NaN in a row whose mean square is smaller would be the only sign of it."""
+    k = kern(torch.bfloat16)
+    x, residual, weight, w = (rand(s, torch.bfloat16, 9).cuda() for s in ((2, 2048), (2, 2048), (2048,), (4096, 2048)))
+    run = k.lib.vk_gemm_normed
+    run.argtypes = [P, P, P, P, P, ctypes.c_float, P, I, I, I, ctypes.c_int64, I, P]
+    out, total = torch.zeros((2, 4096), dtype=x.dtype, device="cuda"), torch.zeros_like(x)
+    rc = run(out.data_ptr(), total.data_ptr(), x.data_ptr(), residual.data_ptr(), weight.data_ptr(), -1e-6, w.data_ptr(), 2, 4096, 2048, 4096, 1,
+             torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc != 0 and b"eps" in k.lib.vk_last_error() and not out.any() and not total.any()

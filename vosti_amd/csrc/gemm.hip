@@ -2622,6 +2622,7 @@ int vk_gemm_normed(elem_t* out, elem_t* sum, const elem_t* x, const elem_t* resi
                    int64_t ldo, int projections, hipStream_t st) {
   VK_REQUIRE(projections == 1 || projections == 2, "gemm_normed: one projection or two, not %d", projections);
   VK_REQUIRE(M >= 0, "gemm_normed: bad sizes M=%d N=%d K=%d", M, N, K);
+  VK_REQUIRE(eps >= 0.f, "gemm_normed: eps must not be negative");
   if (M == 0) return 0;
   VK_REQUIRE(vk_gemm_normed_takes(M, N, K, projections), "gemm_normed: sizes M=%d N=%d K=%d are not supported", M, N, K);
   VK_REQUIRE(out != nullptr && ldo >= N, "gemm_normed: output row stride %lld is smaller than N=%d", (long long)ldo, N);
