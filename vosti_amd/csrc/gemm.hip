@@ -137,7 +137,7 @@ struct NormArgs {
 // q, and adds its own partial sums first: here a (row, q) pair is one wave's, all pairs in turn, a lane holding what that kernel's lane holds.
 // load() reads the rows and waits for them (a weight asked for before them would have to arrive first: loads are counted in order); the weights
 // are asked for next, and finish() sums, norms and puts the rows into LDS meanwhile.  A norm of its own is a launch of 3.6 us of eight rows of 4,096 and 2.6 of one
-// of 1,024 between two products (normed_product has the pairs measured).
+// of 1,024 between two products (normed_rows has the pairs measured).
 template <int ROWS, int NW>
 struct NormRows {
   static constexpr int GROUPS = NW * KC * (int)sizeof(elem_t) / 1024, Q = GROUPS < 4 ? GROUPS : 4, J = (GROUPS + 3) / 4, PAIRS = (ROWS * Q + NW - 1) / NW;
@@ -2563,57 +2563,62 @@ static int launch_lines_normed(elem_t* out, const elem_t* x, const elem_t* w, in
   return vk_check_launch("gemm_lines (normed rows)");
 }
 #endif
-// The launch for these sizes, or (out null) whether there is one: 1, 0.  The norm is done again by every workgroup, a row's kilobytes a wave, so that it pays
-// for few rows: the add and norm and the product by themselves against both in one, us, 1, 4 and 8 rows, 16-bit: 4,096 x 1,024 6.5, 6.7, 6.9 against 4.9, 5.7, 7.1; gate/up 3,072 x
-// 1,024 7.7, 7.9, 8.1, 6.4, 7.1, 8.5; 9,728 x 2,560 20.4, 20.7, 20.8, 18.0, 19.6, 21.6; 6,144 x 4,096 12.7, 13.4, 13.8, 10.4, 11.0, 12.5; gate/up 12,288 x 4,096 36.3,
-// 36.8, 37.2, 33.1, 35.0, 37.1; 32-bit, 1, 2 and 4 rows: 4,096 x 1,024 8.3, 8.3, 8.4, 6.8, 7.9, 9.3; 4,096 x 2,048 11.0, 11.1, 11.2, 9.5, 9.8, 10.7; 6,144 x 2,560 18.6, 18.7, 19.0,
-// 16.9, 17.9, 19.6; gate/up 12,288 x 4,096 81.4, 81.8, 82.1, 72.6, 72.3, 73.6, 8 rows 81.5, 77.1.
+// How many rows, at most, are normed on their way into a product of so many chunks (0: none).  The norm is done again by every workgroup, (row, quarter) pairs a wave, so
+// that it pays for few rows.  Measured as the add and norm and the product by themselves over both in one, N of 256 to 16,384, one projection and two:
+//   16-bit  1 to 4 rows, K of 1 to 12 chunks        1.04 to 1.6 (a row 1.04 to 1.6, four rows 1.04 to 1.36)
+//           5 and 6 rows, from 8 chunks on          0.99 to 1.24 from 1,000 weight rows on; below eight chunks 0.91 to 1.3, eight rows there 0.81 to 1.2
+//           7 and 8 rows, 8 chunks (four pairs a    1.00 to 1.16; of 9 to 12 chunks 0.90 to 1.2
+//             wave)
+//   32-bit  1 and 2 rows                            1.00 to 1.27
+//           3 and 4 rows, 4, 6 and 8 chunks         0.99 to 1.16; of 2 chunks (eight pairs a wave) 0.88 to 1.06, of 5 (four of three kilobytes) 0.93 to 1.06
+//           5 and 6 rows, 8 chunks                  1.01 to 1.07
+//           7 and 8 rows, 8 chunks                  with SwiGLU 0.99 to 1.07, else from a weight tile a compute unit on 1.00 to 1.02 (below 0.94 to 0.99)
+// A launch is of as many waves as K has chunks, so that 32-bit products of 1, 3 and 7 chunks, which the streaming kernels take with waves to spare, have none.
+static int normed_rows(int N, int chunks, int projections) {
+#ifdef VK_BF16
+  if (chunks < 1 || chunks > 12) return 0;
+  return chunks < 8 || N <= 2 * vk_device_cus() ? 4 : chunks == 8 ? 8 : 6;
+#else
+  if (chunks == 2 || chunks == 5) return 2;
+  if (chunks == 4 || chunks == 6) return 4;
+  return chunks != 8 ? 0 : projections == 2 || (N + 15) / 16 >= vk_device_cus() ? 8 : 6;
+#endif
+}
+// The launch.  16-bit: whole lines in tiles of eight weight rows, or of four where those do not fit the LDS (up to 512 weight rows four are as fast or, of gate and up,
+// 4 to 10 % faster; otherwise up to 25 % slower), also where the streaming kernel is the faster one of a product by itself: one barrier a tile, and the norm's, cost it
+// more than the lines'.  But three and four rows of two chunks and one projection are faster with it by the mean of 7 % (0.93 to 1.10 times as fast).
+// Before and after, us, 1, 4 and (from eight chunks on) 8 rows, 16-bit: 4,096 x 1,024 5.8, 6.3 -> 4.0, 5.2; gate/up 3,072 x 1,024 7.8, 7.8 -> 5.2, 7.0; 4,096 x 1,536 7.0, 7.2 -> 4.5, 6.2;
+// 6,144 x 3,072 10.8, 11.8 -> 8.2, 9.8; gate/up 10,240 x 2,560 21.3, 21.6 -> 18.8, 20.6; 6,144 x 4,096 12.7, 13.7, 14.5 -> 10.4, 11.3, 12.6; gate/up 10,240 x 4,096 31.8, 32.9,
+// 33.3 -> 28.4, 30.7, 32.6; gate/up 10,240 x 6,144 44.2, 45.2 -> 40.9, 42.6; 32-bit, 1, 2 and 4 rows: 4,096 x 1,024 8.0, 8.1 -> 6.6, 7.7; 4,096 x 2,048 11.2, 11.2, 11.4 -> 9.7, 9.9, 10.8;
+// 6,144 x 2,560 18.6, 19.0 -> 17.1, 18.3; 6,144 x 3,072 20.8, 20.9, 21.4 -> 19.1, 19.5, 20.4; gate/up 10,240 x 4,096 75.1, 75.3, 75.8 -> 68.9, 69.1, 70.2.
 template <int ROWS, int P>
 static int normed_product(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int K, int64_t ldx, int64_t ldo, const NormArgs& norm, hipStream_t st) {
-  const int chunks = K / KC, form = out == nullptr ? 0 : (ldo % 4 == 0 && (uintptr_t)out % 16 == 0);
-#define STREAMED(NW) return out == nullptr ? 1 : launch_stream_normed<ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
+  const int chunks = K / KC, form = ldo % 4 == 0 && (uintptr_t)out % 16 == 0;
+#define STREAMED(NW) if (chunks == NW) return launch_stream_normed<ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
 #ifdef VK_BF16
-#define LINED(R, NW) return out == nullptr ? 1 : launch_lines_normed<R, ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
-  const int rows = lines_rows(M, N, K, P);
-  if (rows == 8 && chunks == 8) LINED(8, 8);
-  if constexpr (ROWS <= 4) {
-    if (rows == 8 && P == 2 && chunks == 2) LINED(8, 2);
-    if (rows == 8 && chunks == 4) LINED(8, 4);
-    if (rows == 8 && chunks == 5) LINED(8, 5);
-    if constexpr (P == 1) {
-      if (rows == 8 && chunks == 10) LINED(8, 10);
-    } else {
-      if (rows == 4 && chunks == 10) LINED(4, 10);
-    }
-    if (rows == 0 && chunks == 2) STREAMED(2);
-    if (rows == 0 && chunks == 4) STREAMED(4);
+  if constexpr (ROWS == 4 && P == 1) {
+    if (M > 2) STREAMED(2);
   }
+#define LINED(NW) if (chunks == NW) return launch_lines_normed<P == 1 || NW <= 8 ? 8 : 4, ROWS, P, NW>(out, x, w, M, N, ldx, ldo, form, norm, st)
+  if constexpr (ROWS <= 4) {
+    LINED(1); LINED(2); LINED(3); LINED(4); LINED(5); LINED(6); LINED(7);
+  }
+  LINED(8); LINED(9); LINED(10); LINED(11); LINED(12);
 #undef LINED
 #else
-  if (chunks == 8) STREAMED(8);
   if constexpr (ROWS <= 4) {
-    if (chunks == 2 && M <= 2) STREAMED(2);
-    if (chunks == 4) STREAMED(4);
-    if (chunks == 5 && M <= 2) STREAMED(5);
+    STREAMED(2); STREAMED(4); STREAMED(5); STREAMED(6);
   }
+  STREAMED(8);
 #endif
 #undef STREAMED
-  (void)form; (void)x; (void)w; (void)ldx; (void)norm; (void)st;
-  return 0;
-}
-template <int P>
-static int normed_product(elem_t* out, const elem_t* x, const elem_t* w, int M, int N, int K, int64_t ldx, int64_t ldo, const NormArgs& norm, hipStream_t st) {
-  if (M < 1 || M > 8 || N < 1 || K < KC || K % KC != 0) return 0;
-  if (M == 1) return normed_product<1, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
-  if (M <= 4) return normed_product<4, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
-  return normed_product<8, P>(out, x, w, M, N, K, ldx, ldo, norm, st);
+  return vk_fail("gemm_normed: no launch for %d rows of K=%d", M, K);
 }
 }  // extern "C++"
 
-// 1 if vk_gemm_normed takes these sizes (projections 1, or 2 with N gate rows) and is the faster way (normed_product).
+// 1 if vk_gemm_normed takes these sizes (projections 1, or 2 with N gate rows) and is the faster way (normed_rows).
 int vk_gemm_normed_takes(int M, int N, int K, int projections) {
-  return projections == 2 ? normed_product<2>(nullptr, nullptr, nullptr, M, N, K, K, N, NormArgs{}, nullptr)
-                          : normed_product<1>(nullptr, nullptr, nullptr, M, N, K, K, N, NormArgs{}, nullptr);
+  return M >= 1 && N >= 1 && K >= KC && K % KC == 0 && M <= normed_rows(N, K / KC, projections);
 }
 
 // out = norm(x + residual) w^T, or with two projections silu(gate) * up: vk_add_rmsnorm (sum, [M, K], takes the place of its new residual and is
@@ -2629,7 +2634,11 @@ int vk_gemm_normed(elem_t* out, elem_t* sum, const elem_t* x, const elem_t* resi
   VK_REQUIRE((((uintptr_t)x | (uintptr_t)residual | (uintptr_t)sum | (uintptr_t)norm_weight | (uintptr_t)w) % 16) == 0, "gemm_normed: operands must be 16-byte aligned");
   VK_REQUIRE(sum != x && sum != residual && x != nullptr && residual != nullptr && sum != nullptr && norm_weight != nullptr, "gemm_normed: the sum needs a buffer of its own");
   const NormArgs norm = {residual, sum, norm_weight, eps};
-  return projections == 2 ? normed_product<2>(out, x, w, M, N, K, K, ldo, norm, st) : normed_product<1>(out, x, w, M, N, K, K, ldo, norm, st);
+#define NORMED(ROWS) return projections == 2 ? normed_product<ROWS, 2>(out, x, w, M, N, K, K, ldo, norm, st) : normed_product<ROWS, 1>(out, x, w, M, N, K, K, ldo, norm, st)
+  if (M == 1) NORMED(1);
+  if (M <= 4) NORMED(4);
+  NORMED(8);
+#undef NORMED
 }
 
 // float32 elements of workspace that vk_gemm_split needs for these sizes, or 0 if it does not take them:
