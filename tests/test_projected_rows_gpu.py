@@ -78,3 +78,21 @@ def test_what_is_not_taken():
     assert both(torch.bfloat16, [40], 8, 4, 96, 64, 0, True, True) is None
     assert both(torch.bfloat16, [40], 8, 4, 128, 32, 0, True, True) is None
     assert both(torch.bfloat16, [40] * 90, 8, 8, 128, 64, 0, True, True) is None
+
+
+def test_where_it_is_the_faster_way():
+    """One segment a row and several, on both sides of one and two segments a compute unit; never where it is not taken."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for dtype in DTYPES:
+        takes, pays = (getattr(kern(dtype).lib, "vk_paged_attention_rows_" + n) for n in ("takes", "preferred"))
+        takes.argtypes = pays.argtypes = [I] * 6
+        bf16 = dtype == torch.bfloat16
+        for nseg in (1, 2, 4):
+            for segments in (2 * nseg, cus, cus + 2 * nseg, 2 * cus, 2 * cus + 2 * nseg, 3 * cus):
+                rows = segments // (2 * nseg)                # two kv heads
+                n = 2 * nseg * rows
+                can = [bool(takes(rows, nseg, 4, 2, d, 64)) for d in (64, 128)]
+                want = [bf16 or n <= 2 * cus, n <= 2 * cus or nseg > 1 if bf16 else nseg > 1 and n <= cus]
+                assert can == [n <= 5 * cus // 2, n <= (5 if bf16 else 12) * cus // 2]
+                assert [bool(pays(rows, nseg, 4, 2, d, 64)) for d in (64, 128)] == [a and b for a, b in zip(can, want)], (dtype, nseg, segments)
+        assert not pays(4, 2, 4, 2, 96, 64) and not pays(4, 2, 4, 2, 64, 32) and not pays(0, 1, 4, 2, 64, 64)

@@ -1807,6 +1807,22 @@ int vk_paged_attention_rows_takes(int n_items, int nseg, int nq, int nkv, int d,
   return (int64_t)n_items * (nkv * ((nq / nkv + 15) / 16)) * nseg <= quad_segments(d);
 }
 
+// 1 if it is also the faster way.  A row's norm and turn stand in front of its attention, in registers that leave room for two workgroups a compute unit (heads of
+// 256 bytes) or one (512); a launch of its own does them for all rows at once.  vk_qkv_post and vk_paged_attention over the one launch, 8, 16, 32 and 40 heads on 8 and
+// 32 on 2, 1 to 80 rows of 30 to 4,000 keys, by segments of the launch against the compute units, cus:
+//   heads of 128 bytes   0.95 to 1.17 wherever four waves go to a segment (one size below 0.98)
+//   of 256, 16-bit       1.01 to 1.23 (one row of 200 keys, 16 on 8: 11.1 -> 9.4 us; of 500 15.6 -> 13.5); one segment a row and more than 2 cus: 0.77 to 1.03
+//   of 256, 32-bit       up to 2 cus 0.97 to 1.12, more 0.76 to 0.93 (80 rows of 30 keys, 16 on 8: 14.1 -> 18.0 us)
+//   of 512               never folded.  Two segments a row and more, up to cus: 1.00 to 1.16 (two rows of 500 keys, 16 on 8: 23.1 -> 19.9 us); up to 2 cus 0.97 to 1.07, more 0.95
+//                        to 0.98; one segment: 0.78 to 0.94 with 30 keys, 0.95 to 1.10 with 200
+int vk_paged_attention_rows_preferred(int n_items, int nseg, int nq, int nkv, int d, int P) {
+  if (!vk_paged_attention_rows_takes(n_items, nseg, nq, nkv, d, P)) return 0;
+  const int64_t segments = (int64_t)n_items * (nkv * ((nq / nkv + 15) / 16)) * nseg, cus = vk_device_cus();
+  const int row = (int)sizeof(elem_t) * d;
+  if (row > 256) return nseg > 1 && segments <= cus;
+  return row < 256 || segments <= 2 * cus || (sizeof(elem_t) == 2 && nseg > 1);
+}
+
 // vk_qkv_post (heads of d with a rotation of the whole head or none, weights of elements or none, every row stored where its slot says) and
 // vk_paged_attention (mode 1, every row of the step one item) in one launch for the two, the same bits.  qkv [T, row_stride].
 int vk_paged_attention_rows(elem_t* out, const elem_t* qkv, int64_t row_stride, elem_t* kc, elem_t* vc, const elem_t* q_w, const elem_t* k_w, float eps,

@@ -96,7 +96,7 @@ struct Kernels::Fn {
   int (*gemm_split_preferred)(int, int, int, int);
   int (*qkv_post)(CP, int64_t, P, P, P, CP, CP, int, CP, CP, int, CP, CP, int, int, int, int, int, float, hipStream_t);
   int (*paged_attention)(P, CP, CP, CP, CP, int, CP, CP, CP, int, int, int, P, int, int, int, int, int, int, float, hipStream_t);
-  int (*paged_attention_rows_takes)(int, int, int, int, int, int);
+  int (*paged_attention_rows_preferred)(int, int, int, int, int, int);
   int (*paged_attention_rows)(P, CP, int64_t, P, P, CP, CP, float, CP, CP, CP, CP, CP, int, CP, CP, CP, int, int, P, int, int, int, int, int, float, hipStream_t);
   int (*sample)(P, CP, CP, CP, P, int, int, int64_t, hipStream_t);
   int (*sample_scratch_words)(int);
@@ -200,7 +200,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(gemm_normed_takes, "vk_gemm_normed_takes"); VK(gemm_normed, "vk_gemm_normed");
   VK(gemm_split, "vk_gemm_split"); VK(gemm_split_floats, "vk_gemm_split_floats"); VK(gemm_split_preferred, "vk_gemm_split_preferred");
   VK(qkv_post, "vk_qkv_post"); VK(paged_attention, "vk_paged_attention");
-  VK(paged_attention_rows_takes, "vk_paged_attention_rows_takes"); VK(paged_attention_rows, "vk_paged_attention_rows"); VK(sample, "vk_sample");
+  VK(paged_attention_rows_preferred, "vk_paged_attention_rows_preferred"); VK(paged_attention_rows, "vk_paged_attention_rows"); VK(sample, "vk_sample");
   VK(sample_scratch_words, "vk_sample_scratch_words"); VK(attn_scratch_floats, "vk_attn_scratch_floats");
   VK(attn_segment_keys, "vk_attn_segment_keys"); VK(attn_item_rows, "vk_attn_item_rows");
   VK(embed_sinusoid, "vk_embed_sinusoid"); VK(stream_norm, "vk_stream_norm"); VK(stream_norm_add, "vk_stream_norm_add");
@@ -490,7 +490,7 @@ int64_t Kernels::attn_scratch_floats(int items, int nq, int d, int nseg) const {
 
 bool Kernels::attention_takes_rows(int64_t items, int nseg, int nq, int nkv, int d, int page_size, const Tensor* q_w, const Tensor* k_w, const Tensor* cos) const {
   if ((q_w && q_w->dtype != dtype_) || (k_w && k_w->dtype != dtype_) || (cos && 2 * cos->dim(1) != d) || items > INT32_MAX) return false;
-  return fn_->paged_attention_rows_takes((int)items, nseg, nq, nkv, d, page_size) != 0;
+  return fn_->paged_attention_rows_preferred((int)items, nseg, nq, nkv, d, page_size) != 0;
 }
 
 void Kernels::paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int nkv, int d, const Tensor& k_cache, const Tensor& v_cache, int page_size, const Tensor* q_w,

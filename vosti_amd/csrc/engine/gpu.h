@@ -148,7 +148,7 @@ class Kernels {
                        const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode,
                        float scale, int window, int max_k_len, int nseg, const Tensor* scratch);
   // qkv_post and paged_attention of decoded rows alone (every row of qkv [T, (nq + 2 nkv) d] is an item of its own) in one launch, where
-  // attention_takes_rows says that there is one: the same bits.
+  // attention_takes_rows says that there is one and that it is the faster way: the same bits.
   bool attention_takes_rows(int64_t items, int nseg, int nq, int nkv, int d, int page_size, const Tensor* q_w, const Tensor* k_w, const Tensor* cos) const;
   void paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int nkv, int d, const Tensor& k_cache, const Tensor& v_cache, int page_size, const Tensor* q_w,
                             const Tensor* k_w, float eps, const Tensor* cos, const Tensor* sin, const Tensor& positions, const Tensor& slots,
