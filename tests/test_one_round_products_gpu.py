@@ -30,3 +30,17 @@ def test_gate_and_up(M, K, dtype):
     for I in (7, 200, 64 * (cus // blocks), 64 * (cus // blocks) + 1):
         w = rand((2 * I, K), dtype, 4, 0.1).cuda()
         assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4))), I
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_far_apart(dtype):
+    """Rows whose distance from the first of their block is no longer a number of 32 bits in bytes: 127 of them are more than 4 GiB, by 23 MB."""
+    k = kern(dtype)
+    M, K, apart = 128, 512, 17_000_000 if dtype == torch.bfloat16 else 8_500_000
+    rows = rand((M, K), dtype, 5).cuda()
+    x = torch.empty(((M - 1) * apart + K,), dtype=dtype, device="cuda").as_strided((M, K), (apart, 1))
+    x.copy_(rows)
+    w = rand((512, K), dtype, 6, 0.1).cuda()
+    expected = k.gemm(rows, w, kernel=3)
+    assert torch.equal(k.gemm(x, w), expected) and torch.equal(k.gemm(x, w, kernel=2), expected)
+    assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(expected))

@@ -968,6 +968,7 @@ static int launch_tiled(elem_t* out, const elem_t* act, const elem_t* w, int M, 
 // for grids whose last round of workgroups would otherwise run nearly empty (pipe_fragments_by_rounds).  Six
 // would need more than the 256 registers of a wave.
 // NWN: waves along the weight rows, two of a workgroup of four waves or four of eight, which takes 64 FNW weight rows.
+// A lane's offset from its block's first row is of 32 bits: rows_far says which rows are too far apart for that.
 // GROUPED: block_weights, row_pair and act_row count.
 template <int S, bool WHOLE, bool SWIGLU, int FNW = 4, int NWN = 2, bool GROUPED = false>
 __global__ __launch_bounds__(128 * NWN, NWN == 2 ? 2 : 1) void gemm_pipe_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act,
@@ -1204,6 +1205,8 @@ static bool grouped_wide(int M, int N, int matrices, bool named) {
   if (columns % 8 == 0 || columns > 16) return 8 * groups >= 5 * vk_device_cus();
   return !named && columns <= 4 && 2 * groups >= vk_device_cus();
 }
+
+static bool rows_far(int64_t lda) { return (127 * lda + 2 * VK_SLAB) * (int64_t)sizeof(elem_t) > (int64_t)UINT32_MAX; }
 
 template <int S, bool SWIGLU = false, int FNW = 4, bool GROUPED = false>
 static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
@@ -2374,7 +2377,7 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
 #undef SK
     return vk_check_launch("gemm_skinny");
   }
-  const bool k_whole = K % (2 * VK_SLAB) == 0;
+  const bool k_whole = K % (2 * VK_SLAB) == 0 && !rows_far(lda);
   if (kernel == 3) return launch_tiled<4, 4>(out, act, w, M, N, K, lda, ldo, form, st);
   if (kernel == 4 && k_whole) return launch_pipe<2>(out, act, w, M, N, K, lda, ldo, form, st);
   if (kernel == 5 && k_whole) return launch_pipe<3>(out, act, w, M, N, K, lda, ldo, form, st);
@@ -2444,6 +2447,10 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
     if (f == 4) return launch_alternate<4, 3, 4, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
   }
 #endif
+  if (how == 2 && rows_far(lda)) {
+    VK_REQUIRE(K % KC == 0, "gemm_swiglu: rows %lld elements apart need K in whole chunks of %d", (long long)lda, KC);
+    return launch_mid<4, 1, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+  }
   if (how == 2)
     return launch_pipe<2, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
 #ifdef VK_BF16
