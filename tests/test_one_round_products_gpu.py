@@ -32,6 +32,18 @@ def test_gate_and_up(M, K, dtype):
         assert torch.equal(k.gemm_swiglu(x, w), k.swiglu(k.gemm(x, w, kernel=4))), I
 
 
+@pytest.mark.parametrize("M", [112, 113, 128, 129])
+@pytest.mark.parametrize("K", [4608, 5120])
+def test_a_second_block_of_rows(M, K):
+    """Both sides of the lines in rows, chunks and weight rows at which 16-bit products of two blocks of 64 rows share activations through LDS instead."""
+    k = kern(torch.bfloat16)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    x = rand((M, K), torch.bfloat16, 7).cuda()
+    for N in (16 * cus, 16 * cus + 1, 32 * cus, 32 * cus + 1):
+        w = (torch.randn((N, K), generator=torch.Generator("cuda").manual_seed(8), device="cuda") * 0.1).to(torch.bfloat16)
+        assert torch.equal(k.gemm(x, w), k.gemm(x, w, kernel=4)), N
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_rows_far_apart(dtype):
     """Rows whose distance from the first of their block is no longer a number of 32 bits in bytes: 127 of them are more than 4 GiB, by 23 MB."""

@@ -2021,6 +2021,9 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //              16-bit, two blocks, K > 2 chunks,               9   so few weight rows that the tile kernel's workgroups of 64 leave three
 //                wg32 <= 0.5 cus                                     quarters of the units idle (128 rows, 4096 x 12288: 81 us against
 //                                                                  54; 1024 x 2048: 13.7 against 11.6)
+//              16-bit, rows > 112, two blocks, K >= 10        8   with all of a block's rows in use and long chains the tile kernel in one round is the slower one (128 rows,
+//                chunks, wg64 <= 0.5 cus                             5,120 x 5,120: 41.4 against 37.4 us; 8,192 x 6,144: 48.8, 45.4; 7 and 8 K a few sizes 1 to 4 % the other
+//                                                                  way; up to 112 rows and nine chunks 0.92 to 1.33 times, 1.09 on the mean)
 //              16-bit                                          2   the tile kernel in one round (pipe_fragments_in_one_round; 200 rows,
 //                                                                  6144 x 4096: 40 -> 27 us)
 //              32-bit, wg64 >= 0.5 cus                         8 up to three blocks, else 2
@@ -2048,7 +2051,10 @@ static int choose_gemm_kernel(int M, int N, int K) {
   if (M <= 64) return (2 * wg128 >= cus && M > 32) ? 2 : (many16 ? 7 : 1);
   if (M <= 256 && whole && 2 * wg128 < cus) {
     const int blocks = (M + 63) / 64;
-    if (sizeof(elem_t) == 2) return blocks == 2 && 2 * wg32 <= cus && K > 2 * KC ? 9 : 2;
+    if (sizeof(elem_t) == 2) {
+      if (blocks == 2 && 2 * wg32 <= cus && K > 2 * KC) return 9;
+      return blocks == 2 && M > 112 && K >= 10 * KC && 2 * wg64 <= cus ? 8 : 2;
+    }
     if (2 * wg64 >= cus) return blocks <= 3 ? 8 : 2;
     if (blocks == 2) return 2 * wg32 <= cus ? 9 : 8;
     return (k_resident && many16) ? 2 : 8;
