@@ -381,9 +381,9 @@ __global__ __launch_bounds__(64 * MOE_WAVES) void moe_gemm_kernel(elem_t* __rest
 // is bound by its workgroups' starts: 64 to 128 KB of weights each behind three dependent loads, and idle waves where K has fewer than
 // eight chunks.  Workgroups of a wave a chunk stay for the whole launch and take equal, contiguous shares of the (row tile, MOE_LINE_ROWS
 // features) units of all tiles in use, tile by tile; a wave keeps its chunk of the tile's rows in registers; the weights come as in
-// gemm_lines_kernel, a row of a chunk a load, marked as read once, into a ring of slots a wave that runs on across units and tiles; one
-// barrier a unit, and the waves take turns at adding up a unit's chunk sums.  Rows without a pair are not read and not stored, features beyond
-// N are clamped.
+// gemm_lines_kernel, a row of a chunk a load, marked as read once, into a slot a wave, or two of seven to nine chunks: what LDS has for about twelve waves a
+// compute unit, which cover each other's way to memory (slots of four rows, two or three a wave, were 4 to 12 % slower); one barrier a unit, and the waves take
+// turns at adding up a unit's chunk sums.  Rows without a pair are not read and not stored, features beyond N are clamped.
 // What bounds it: a launch's start (expert_start, a tile's expert, its rows) where units are few, else how fast memory gives lines: 6.2 to 6.6 TB/s.
 // Measured on MI355X, 32 experts, eight tokens of 4 choices, against the same stream in the operands' order straight to registers: 1,536 x
 // 2,048 weights, 21 experts 28.1 -> 24.8 us, 2,048 x 1,536 31.6 -> 27.1, 3,072 x 2,048, 18 experts 48.1 -> 39.2; five chunks and more: 4,096 x 4,608, 21
@@ -442,9 +442,7 @@ __global__ __launch_bounds__(64 * MOE_LINE_CHUNKS) void moe_lines_kernel(elem_t*
     // All but the slots asked for after this one's (and a store or a tile's rows, which are waited for by count as well: never too short a wait).
     const int later = ask_u - u - 1;
     __builtin_amdgcn_sched_barrier(0);
-    if (later >= 3) wait_vmcnt_n<3 * R>();
-    else if (later == 2) wait_vmcnt_n<2 * R>();
-    else if (later == 1) wait_vmcnt_n<R>();
+    if (later > 0) wait_vmcnt_n<R>();               // a ring has two slots at most
     else wait_vmcnt_n<0>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -491,6 +489,60 @@ __global__ __launch_bounds__(64 * MOE_LINE_CHUNKS) void moe_lines_kernel(elem_t*
       ++tile;
       if (u + 1 < hi) bring(tile);
     }
+  }
+}
+// The same for one and two whole chunks and few units, a unit of 16 features a workgroup, a wave a chunk, all of it asked for at once in the operands' order
+// straight to registers.  What bounds it is the way to its first bytes, which here is a tile's expert and the weights behind it, with no way through LDS; and units
+// of 16 features read the tile's rows half as often as those of eight.  No load is predicated.
+// moe_product_kernel has both sides measured.
+template <int MODE, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void moe_unit_kernel(elem_t* __restrict__ out, int64_t ldo, const elem_t* __restrict__ x, int64_t ldx,
+                                                              const elem_t* __restrict__ w, int64_t expert_stride, const int32_t* __restrict__ row_pair,
+                                                              const int32_t* __restrict__ row_token, const int32_t* __restrict__ tile_expert, int N, int K, int vec) {
+  __shared__ f32x4 part[WAVES][64];
+  const int tile = blockIdx.y, e = tile_expert[tile];
+  if (e < 0) return;                              // the whole workgroup
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int row = tile * MOE_TILE + r16, first = blockIdx.x * 16 + kq * 4;
+  const bool live = row_pair[row] >= 0;           // the lane's row has a pair
+  const int64_t k0 = (int64_t)wave * MOE_KC + kq * VK_VEC;
+  const elem_t* wr = w + (int64_t)e * expert_stride + (int64_t)min((int)blockIdx.x * 16 + r16, N - 1) * K + k0;
+  frag_t weights[MOE_KC_SLABS], rows[MOE_KC_SLABS];
+#pragma unroll
+  for (int i = 0; i < MOE_KC_SLABS; ++i) weights[i] = *reinterpret_cast<const frag_t*>(wr + i * VK_SLAB);
+  // As in the kernel above: instead of rows without a pair the last one with one, or, gathered, the token that the plan names there.
+  const int from = MODE != 0 ? row_token[row] : tile * MOE_TILE + min(r16, max(__popcll(__ballot(live) & 0xFFFFu) - 1, 0));
+  const elem_t* xr = x + (int64_t)from * ldx + k0;
+#pragma unroll
+  for (int i = 0; i < MOE_KC_SLABS; ++i) rows[i] = *reinterpret_cast<const frag_t*>(xr + i * VK_SLAB);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, total = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < MOE_KC_SLABS; ++i) acc = mma_slab(weights[i], rows[i], acc);
+  if constexpr (WAVES > 1) {
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+  }
+#pragma unroll
+  for (int c = 0; c < WAVES; ++c) {
+    const f32x4 p = WAVES > 1 ? part[c][lane] : acc;
+    total.x = total.x + p.x; total.y = total.y + p.y; total.z = total.z + p.z; total.w = total.w + p.w;
+  }
+  if (MODE == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float rl = fmaxf(round_to_elem(total[i]), 0.f);
+      total[i] = rl * rl;
+    }
+  }
+  if (!live) return;
+  elem_t* o = out + (int64_t)row * ldo + first;
+  if (vec && first + 3 < N) {
+    store_elems4(o, total);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (first + i < N) o[i] = from_f32<elem_t>(total[i]);
   }
 }
 #endif
@@ -647,35 +699,50 @@ int vk_moe_route_plan(int32_t* idx, float* wts, float* logits, const elem_t* h, 
                       correction_is_f32, plan);
 }
 
-// An expert product of rows in tiles of 16: by the streaming kernel where it takes the sizes, else by the one for every K.
+// An expert product of rows in tiles of 16: by the kernels for whole slabs where they take the sizes, else by the one for every K.
 extern "C++" {
 #ifdef VK_BF16
-// The (row tile, 16 features) units, of all tiles that a launch covers, from which on the kernel of whole lines is the faster one.
-// Below, the other kernel's workgroups all run at once, and this one's longer start (the tiles in use, a tile's expert, its rows, a barrier a
-// unit) is what a call waits for.  Measured on MI355X in recorded launches, 32 experts, 3 and 4 choices, 1 to 24 tokens, weights of two to twelve layers in turn; the
-// other kernel against this one, us, the units in brackets:
-//   two chunks, rows as they are: 1,152 x 1,024 weights, two tokens (576) 6.8, 7.6; 1,536 x 1,024, two (768) 10.4, 7.9; gathered always: 768 x 1,024, one
-//   (192) 5.4, 5.0, 1,536 x 1,024, three (864) 11.5, 8.9;
-//   three: 512 x 1,536, five (640) 8.6, 8.7; 2,048 x 1,536, two (768) 14.0, 11.1;
-//   four: 1,536 x 2,048, two (576) 9.7, 10.7, 512 x 2,048, eight (768) 9.5, 11.7, 3,072 x 2,048, three (2,304) 35.3, 28.5;
-//   six to eight: 1,024 x 4,096, one (256) 9.8, 10.1; 3,072 x 4,096, eight 83.9, 72.6, 24 150, 122; 6,144 x 4,096, 24 292, 239;
-//   a reduction that ends inside a chunk: 1,024 x 768, two (512) 6.0, 6.6, 4,096 x 768, eight 110, 55; 1,024 x 1,152, three (768) 10.0, 10.3, eight
-//   28.9, 19.8; 2,048 x 2,304, one (512) 10.8, 10.9, eight 73, 53.
-// Over 654 sizes 31.9 ms with the other kernel, 24.4 with this one, 30.1 with a stream of 16-row tiles straight to registers in its place.
-static int moe_lines_units(int chunks, bool whole, bool gathered) {
-  if (chunks > MOE_LINE_CHUNKS) return 0;
-  if (!whole) return chunks == 1 ? (gathered ? 768 : 2304) : (chunks == 3 || chunks == 4 ? 780 : 540);
-  constexpr int UNITS[9] = {0, 1, 600, 660, 780, 1, 260, 260, 260};
-  return chunks > 8 || (chunks == 2 && gathered) ? 1 : UNITS[chunks];
+// Which kernel is the fastest one, by the (row tile, 16 features) units of all tiles that a launch covers.  The kernel of whole lines has a long start (the
+// tiles in use, a tile's expert, its rows, a barrier a unit) and reads a tile's rows twice as often; the one for every K has eight waves whatever K.
+// Measured on MI355X in recorded launches, 8 to 64 experts, 2 to 6 choices, 1 to 64 tokens, weights of two to twelve layers in turn.
+// One and two whole chunks, 588 sizes: 5,966 us by whole lines, 9,773 by the kernel for every K, 5,599 by a unit a workgroup, 6,740 by a stream of such units that stays (which
+// these three replace).  A unit a workgroup against whole lines, by units: one chunk, up to 1,000 0.69 to 1.04 (512 x 512, 32 experts, three tokens 4.4 -> 3.9 us), up to
+// 4,096 0.69 to 0.99, up to 6,000 0.87 to 1.14, more 0.88 to 1.18; two chunks, up to 1,400 0.63 to 1.05 (1,024 x 1,024, eight experts, eleven tokens 7.1 -> 5.6), up to 2,048 0.81 to 1.02, up to
+// 4,200 0.86 to 1.17 (the mean 0.99), more 0.88 to 1.29.
+// More chunks, the kernel for every K against whole lines, us, the units in brackets: where units are at most half of the compute units the latter are ahead (512 x 1,536, one
+// token (64) 5.3, 4.4; 512 x 2,048 (128) 5.9, 5.1; 512 x 2,560 (128) 6.2, 5.5; 256 x 3,584 (64) 7.0, 5.4; 512 x 4,096 (128) 7.5, 6.7); then
+//   three: 512 x 1,536 (320) 5.9, 7.7, (640) 10.7, 10.5, 768 x 1,536 (720) 11.2, 13.5; 2,048 x 1,536 (768) 7.8, 8.6, (1,024) 12.1, 11.1;
+//   four: 512 x 2,048 (640) 8.6, 10.1, (736) 11.7, 12.0, (1,024) 15.8, 12.4; 1,536 x 2,048 (768) 15.9, 12.2;
+//   five: 512 x 2,560 (256) 6.6, 7.5, (480) 12.6, 14.0, (640) 14.4, 12.9; 256 x 2,560 (512) 12.2, 11.2;
+//   six: 384 x 3,072 (336) 8.8, 11.3; 512 x 3,072 (384) 10.9, 11.2; 256 x 3,072 (512) 12.5, 11.6; 1,024 x 3,072 (576) 14.3, 12.6;
+//   seven: 512 x 3,584 (288) 9.9, 10.0, (384) 12.1, 11.6; 1,024 x 3,584 (512) 12.3, 13.6, (576) 16.2, 14.4, (768) 17.4, 17.8;
+//   eight: 512 x 4,096 (256) 8.3, 10.1, (320) 11.8, 11.1; 384 x 4,096 (288) 8.5, 10.7; 3,072 x 4,096, eight tokens 83.9, 72.6, 24 150, 122;
+//   nine and more: the other kernel needs a second round: 512 x 4,608 (128) 9.7, 7.2, (576) 20.8, 16.8; at 192 to 256 units as fast, within 10 % either way;
+//   a reduction that ends inside a chunk: 1,024 x 768 (576) 6.0, 7.6, (768) 8.5, 7.8, 4,096 x 768, eight tokens 110, 55; 1,024 x 1,152 (768) 9.3, 10.4, (2,048) 18.4, 13.8; 1,024 x 2,304 (576) 10.9,
+//   11.3, (768) 13.8, 13.0.
+enum { MOE_TILES, MOE_LINES, MOE_UNITS };
+static int moe_product_kernel(int chunks, bool whole, bool gathered, int64_t units) {
+  if (chunks > MOE_LINE_CHUNKS) return MOE_TILES;
+  if (!whole) return units >= (chunks == 1 ? (gathered ? 768 : 2304) : (chunks == 3 || chunks == 4 ? 780 : 600)) ? MOE_LINES : MOE_TILES;
+  if (chunks <= 2) return units < (chunks == 1 ? 4096 : 2048) ? MOE_UNITS : MOE_LINES;
+  constexpr int LINES_FROM[9] = {0, 0, 0, 780, 750, 500, 500, 260, 300};
+  return chunks > 8 || units >= LINES_FROM[chunks] || 2 * units <= vk_device_cus() ? MOE_LINES : MOE_TILES;
 }
 #endif
 template <int MODE>
 static int moe_product(elem_t* out, int64_t ldo, const elem_t* x, int64_t ldx, const elem_t* w, const int32_t* row_pair, const int32_t* row_token,
                        const int32_t* tile_expert, const int32_t* expert_start, int tiles, int E, int N, int K, hipStream_t st, const char* what) {
 #ifdef VK_BF16
-  const int chunks = (K + MOE_KC - 1) / MOE_KC, least = moe_lines_units(chunks, K % MOE_KC == 0, MODE != 0);
+  const int chunks = (K + MOE_KC - 1) / MOE_KC, vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
   const int64_t units = (int64_t)tiles * ((N + 15) / 16);
-  if (K % VK_SLAB == 0 && ldx % VK_VEC == 0 && least != 0 && units >= least) {
+  const int kernel = K % VK_SLAB == 0 && ldx % VK_VEC == 0 ? moe_product_kernel(chunks, K % MOE_KC == 0, MODE != 0, units) : MOE_TILES;
+  if (kernel == MOE_UNITS) {
+    const dim3 grid((N + 15) / 16, tiles);
+    if (chunks == 1) moe_unit_kernel<MODE, 1><<<grid, 64, 0, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, N, K, vec);
+    else moe_unit_kernel<MODE, 2><<<grid, 128, 0, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, N, K, vec);
+    return vk_check_launch(what);
+  }
+  if (kernel == MOE_LINES) {
     // About twelve waves a compute unit, which share its LDS (measured over 544 sizes, the streams of 8, 12 and 16 waves 23.2, 22.7 and 23.0 ms, the one before them 28.8).
     static bool configured = false;
     if (!configured) {
@@ -684,9 +751,8 @@ static int moe_product(elem_t* out, int64_t ldo, const elem_t* x, int64_t ldx, c
       configured = true;
     }
     const int groups = std::max(1, 12 / chunks), sums = chunks * MOE_LINE_ROWS / 4 * 16 * 2 * (int)sizeof(f32x4);
-    const int slots = std::min((160 * 1024 / groups - sums) / (chunks * MOE_LINE_ROWS * 1024), 4);
+    const int slots = std::min((160 * 1024 / groups - sums) / (chunks * MOE_LINE_ROWS * 1024), 2);
     const int grid = (int)std::min<int64_t>((int64_t)tiles * ((N + MOE_LINE_ROWS - 1) / MOE_LINE_ROWS), (int64_t)vk_device_cus() * groups);
-    const int vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
     const size_t smem = (size_t)chunks * slots * MOE_LINE_ROWS * 1024 + sums;
     if (K % MOE_KC == 0)
       moe_lines_kernel<MODE, true><<<grid, 64 * chunks, smem, st>>>(out, ldo, x, ldx, w, (int64_t)N * K, row_pair, row_token, tile_expert, expert_start, E, N, K, vec, slots);
