@@ -643,7 +643,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_swiglu_kernel(elem_t* __r
 // own order (the streaming kernels) an instruction touches 16 rows, half a cache line of each: the address unit takes 64 clocks for a kilobyte, and
 // a line must stay in the first cache until its other half is asked for, so that the loads cannot say that they are the only ones.  Here a load
 // brings one row of a chunk, a whole kilobyte, into LDS, marked as read once: plain reads of 201 MB by 256 workgroups take 35.1 us in strides, 34.0 in pieces of
-// their own and 30.3 marked so (7.0 TB/s); 64-byte pieces marked so are slower than unmarked (36.7 -> 39).  The activations come the same way, once, and stay in
+// their own and 30.3 marked so (6.6 TB/s); 64-byte pieces marked so are slower than unmarked (36.7 -> 39).  The activations come the same way, once, and stay in
 // registers.  A workgroup walks over tiles of R weight rows with a ring of slots a wave; every wave waits for its own loads only, and a barrier a
 // tile stands between the chunk sums and the wave (another one each tile) that adds them in chunk order, the order of every kernel here.  With the
 // barrier a wave that is early cannot ask for more than its ring holds; counting arrivals in LDS instead, the last wave adding, was slower (4,096 x
@@ -2003,7 +2003,9 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //   rows     condition                                         kernel
 //   1..16    where lines_rows says so                           20, 21  whole lines
 //   1..16                                                      1   streaming
-//   17..64   16-bit, where rows_width says so                   -   gemm_rows_kernel; the rest of this table is then for the others
+//   17..64   16-bit, where rows_width says so                   -   gemm_rows_kernel.  It leaves up to 4,096 weight rows (up to 6,112 of 33 rows and more of K
+//                                                                  above four chunks) and rows further apart than it counts: below, 16-bit sizes reach
+//                                                                  12, 9 and 1, and 10, 8 and 7 of 17 to 64 rows are for 32 bits (figures: 16-bit, from before it)
 //   17..64   K whole chunks:
 //              wg128 >= 0.75 cus                               10  128 weight rows a workgroup: the activations that every
 //                                                                  workgroup reads are half the weight bytes (64 rows, 51200 x
@@ -2465,8 +2467,12 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
 #endif
   if (how == 3) {
     const int ok4 = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
-    // (32-bit elements, and rows too far apart for gemm_rows_kernel; the figures are 16-bit.)  Gate tiles per workgroup: of four, three and two, the number whose workgroups fill the compute units
-    // best, a workgroup per unit at a time; the larger one where two fill them alike.  64 rows, K = 4096:
+#ifdef VK_BF16
+    // Rows too far apart for gemm_rows_kernel.
+    return M <= 32 ? launch_mid<2, 1, true>(out, act, w, M, I, K, lda, ldo, ok4, st) : launch_mid<4, 1, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
+#else
+    // Gate tiles per workgroup: of four, three and two, the number whose workgroups fill the compute units
+    // best, a workgroup per unit at a time; the larger one where two fill them alike.  (Measured in 16-bit, before gemm_rows_kernel.)  64 rows, K = 4096:
     // 12288 gate rows (192, 256, 384 workgroups) 55.4, 49.7, 58.5 us; 8192 gate rows (128, 171, 256) 52.8, 47.0,
     // 41.6 us; 17408 gate rows at K = 5120 (272, 363, 544) 127.5, 108.4, 123.2 us.
     const int tiles = (I + 15) / 16, cus = vk_device_cus();
@@ -2485,6 +2491,7 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
     if (gt == 3) return launch_mid<4, 1, true, 3>(out, act, w, M, I, K, lda, ldo, ok4, st);
     if (gt == 2) return launch_mid<4, 1, true, 2>(out, act, w, M, I, K, lda, ldo, ok4, st);
     return launch_mid<4, 1, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
+#endif
   }
   const int ntiles = (I + 15) / 16;
   const int form = (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0);
@@ -2524,11 +2531,12 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   const int nw = stream_waves(K / KC);       // as in vk_gemm
   if (nw == 2) SWIGLU_STREAMN(2);
   else if (nw == 4) SWIGLU_STREAMN(4);
-  else if (nw == 5) SWIGLU_STREAMN(5);
-  else if (nw == 6) SWIGLU_STREAMN(6);
 #ifdef VK_BF16
   else if (nw == 10) SWIGLU_STREAMN(10);
   else if (nw == 12) SWIGLU_STREAMN(12);
+#else
+  else if (nw == 5) SWIGLU_STREAMN(5);       // 16-bit: whole lines, all of them (lines_rows)
+  else if (nw == 6) SWIGLU_STREAMN(6);
 #endif
   else
 #ifdef VK_BF16
