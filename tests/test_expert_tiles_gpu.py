@@ -54,7 +54,7 @@ def test_tiles_get_the_plain_product(N, K, dtype):
     for e, n in enumerate(counts):
         if n:
             at = slice(start[e], start[e] + n)
-            want = k.gemm(x[token[at].long()].contiguous(), w[e])
+            want = k.gemm(x[token[at].long()].contiguous(), w[e], kernel=3)      # the tile kernel through registers: by size it may be one that brings lines as the experts' does
             assert torch.equal(outs[0][at], want) and torch.equal(outs[2][at], want)
             assert torch.equal(outs[1][at], (want.float().clamp(min=0.0) ** 2).to(dtype))
     assert torch.isnan(outs[0][pair < 0]).all()           # nothing is stored there
@@ -147,7 +147,7 @@ def test_workgroups_that_stay_for_several_units(N, K, dtype):
     for e, n in enumerate(counts):
         if n:
             here = slice(at[e], at[e] + n)
-            want = k.gemm(rows[here].contiguous(), w[e])
+            want = k.gemm(rows[here].contiguous(), w[e], kernel=3)
             assert torch.equal(outs[0][here], want) and torch.equal(outs[2][here], want)
             assert torch.equal(outs[1][here], (want.float().clamp(min=0.0) ** 2).to(dtype))
     assert all(torch.isnan(out[pair < 0]).all() for out in outs)          # nothing is stored there
