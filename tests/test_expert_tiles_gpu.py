@@ -60,10 +60,11 @@ def test_tiles_get_the_plain_product(N, K, dtype):
     assert torch.isnan(outs[0][pair < 0]).all()           # nothing is stored there
 
 
-@pytest.mark.parametrize("N,K", [(6544, 512), (6545, 512), (3264, 1024), (3265, 1024), (192, 2048), (193, 2048), (192, 4096), (193, 4096), (7, 512), (9, 1024)])
+@pytest.mark.parametrize("N,K", [(400, 512), (401, 512), (6544, 512), (6545, 512), (400, 1024), (401, 1024), (3264, 1024), (3265, 1024), (192, 2048), (193, 2048), (192, 4096), (193, 4096),
+                                 (7, 512), (9, 1024)])
 def test_both_sides_of_the_lines(N, K):
-    """Ten tiles and 409 and 410, 204 and 205 groups of 16 features: where one and two chunks go from a unit a workgroup to whole lines, and, 12 and 13 groups,
-    where units are more than half of the compute units; features that end inside the first group."""
+    """Ten tiles and 25 and 26, 409 and 410, 204 and 205 groups of 16 features: between which one and two chunks go by a unit a workgroup; 12 and 13 groups, where units are
+    more than half of the compute units; features that end inside the first group."""
     test_tiles_get_the_plain_product(N, K, torch.bfloat16)
 
 

@@ -491,7 +491,7 @@ __global__ __launch_bounds__(64 * MOE_LINE_CHUNKS) void moe_lines_kernel(elem_t*
     }
   }
 }
-// The same for one and two whole chunks and few units, a unit of 16 features a workgroup, a wave a chunk, all of it asked for at once in the operands' order
+// The same for one and two whole chunks and units between few and many, a unit of 16 features a workgroup, a wave a chunk, all of it asked for at once in the operands' order
 // straight to registers.  What bounds it is the way to its first bytes, which here is a tile's expert and the weights behind it, with no way through LDS; and units
 // of 16 features read the tile's rows half as often as those of eight.  No load is predicated.
 // moe_product_kernel has both sides measured.
@@ -704,28 +704,26 @@ extern "C++" {
 #ifdef VK_BF16
 // Which kernel is the fastest one, by the (row tile, 16 features) units of all tiles that a launch covers.  The kernel of whole lines has a long start (the
 // tiles in use, a tile's expert, its rows, a barrier a unit) and reads a tile's rows twice as often; the one for every K has eight waves whatever K.
-// Measured on MI355X in recorded launches, 8 to 64 experts, 2 to 6 choices, 1 to 64 tokens, weights of two to twelve layers in turn.
-// One and two whole chunks, 588 sizes: 5,966 us by whole lines, 9,773 by the kernel for every K, 5,599 by a unit a workgroup, 6,740 by a stream of such units that stays (which
-// these three replace).  A unit a workgroup against whole lines, by units: one chunk, up to 1,000 0.69 to 1.04 (512 x 512, 32 experts, three tokens 4.4 -> 3.9 us), up to
-// 4,096 0.69 to 0.99, up to 6,000 0.87 to 1.14, more 0.88 to 1.18; two chunks, up to 1,400 0.63 to 1.05 (1,024 x 1,024, eight experts, eleven tokens 7.1 -> 5.6), up to 2,048 0.81 to 1.02, up to
-// 4,200 0.86 to 1.17 (the mean 0.99), more 0.88 to 1.29.
-// More chunks, the kernel for every K against whole lines, us, the units in brackets: where units are at most half of the compute units the latter are ahead (512 x 1,536, one
+// Measured on MI355X in recorded launches, 8 to 64 experts, 2 to 6 choices, 1 to 64 tokens; the lines lie where weights come from memory (512 MB of layers in turn).
+// One and two whole chunks, a unit a workgroup over whole lines, by units: up to the compute units 0.94 to 1.18 (512 x 1,024, one token 4.7, 4.0 us), from there to 600 0.88 to 1.05, up to 1,400
+// 0.74 to 0.99, then one chunk up to 4,096 0.81 to 1.02 and two up to 2,048 0.94 to 1.05, more 0.98 to 1.28.  Where the weights are in the caches (twelve layers of few experts) a unit a
+// workgroup is ahead by 10 % more; the stream of such units that stayed was behind the better one by 5 to 30 % from 600 units on.
+// More chunks, the kernel for every K against whole lines, us, the units in brackets.  Where units are at most half of the compute units the latter are ahead (512 x 1,536, one
 // token (64) 5.3, 4.4; 512 x 2,048 (128) 5.9, 5.1; 512 x 2,560 (128) 6.2, 5.5; 256 x 3,584 (64) 7.0, 5.4; 512 x 4,096 (128) 7.5, 6.7); then
-//   three: 512 x 1,536 (320) 5.9, 7.7, (640) 10.7, 10.5, 768 x 1,536 (720) 11.2, 13.5; 2,048 x 1,536 (768) 7.8, 8.6, (1,024) 12.1, 11.1;
-//   four: 512 x 2,048 (640) 8.6, 10.1, (736) 11.7, 12.0, (1,024) 15.8, 12.4; 1,536 x 2,048 (768) 15.9, 12.2;
-//   five: 512 x 2,560 (256) 6.6, 7.5, (480) 12.6, 14.0, (640) 14.4, 12.9; 256 x 2,560 (512) 12.2, 11.2;
-//   six: 384 x 3,072 (336) 8.8, 11.3; 512 x 3,072 (384) 10.9, 11.2; 256 x 3,072 (512) 12.5, 11.6; 1,024 x 3,072 (576) 14.3, 12.6;
-//   seven: 512 x 3,584 (288) 9.9, 10.0, (384) 12.1, 11.6; 1,024 x 3,584 (512) 12.3, 13.6, (576) 16.2, 14.4, (768) 17.4, 17.8;
-//   eight: 512 x 4,096 (256) 8.3, 10.1, (320) 11.8, 11.1; 384 x 4,096 (288) 8.5, 10.7; 3,072 x 4,096, eight tokens 83.9, 72.6, 24 150, 122;
+//   three: 512 x 1,536 (640) 10.7, 10.5; 1,024 x 1,536 (768) 13.5, 11.1; 2,048 x 1,536, two tokens (768) 14.0, 11.1;
+//   four: 1,536 x 2,048, two tokens (576) 9.7, 10.7; 512 x 2,048 (640) 8.6, 10.1; 1,536 x 2,048 (768) 15.9, 12.2, 3,072 x 2,048, three tokens (2,304) 35.3, 28.5;
+//   five: always (1,000 x 2,560 (189) 7.4, 7.2; 512 x 2,560 (480) 11.5, 10.9; 1,536 x 2,560 (576) 17.2, 13.1; in the caches 10 to 18 % the other way from 192 to 480 units);
+//   six: 768 x 3,072 (288) 12.0, 11.0, 1,536 x 3,072 (384) 12.0, 11.0; seven: 1,024 x 3,584 (576) 16.2, 14.4;
+//   eight: 256 x 4,096 (288) 9.9, 10.5, 384 x 4,096 (408) 16.8, 14.3; 3,072 x 4,096, eight tokens 83.9, 72.6, 24 150, 122; 6,144 x 4,096, 24 292, 239;
 //   nine and more: the other kernel needs a second round: 512 x 4,608 (128) 9.7, 7.2, (576) 20.8, 16.8; at 192 to 256 units as fast, within 10 % either way;
-//   a reduction that ends inside a chunk: 1,024 x 768 (576) 6.0, 7.6, (768) 8.5, 7.8, 4,096 x 768, eight tokens 110, 55; 1,024 x 1,152 (768) 9.3, 10.4, (2,048) 18.4, 13.8; 1,024 x 2,304 (576) 10.9,
-//   11.3, (768) 13.8, 13.0.
+//   a reduction that ends inside a chunk: 1,024 x 768, two (512) 6.0, 6.6, 4,096 x 768, eight 110, 55; 1,024 x 1,152, three (768) 10.0, 10.3, eight
+//   28.9, 19.8; 2,048 x 2,304, one (512) 10.8, 10.9, eight 73, 53.
 enum { MOE_TILES, MOE_LINES, MOE_UNITS };
 static int moe_product_kernel(int chunks, bool whole, bool gathered, int64_t units) {
   if (chunks > MOE_LINE_CHUNKS) return MOE_TILES;
-  if (!whole) return units >= (chunks == 1 ? (gathered ? 768 : 2304) : (chunks == 3 || chunks == 4 ? 780 : 600)) ? MOE_LINES : MOE_TILES;
-  if (chunks <= 2) return units < (chunks == 1 ? 4096 : 2048) ? MOE_UNITS : MOE_LINES;
-  constexpr int LINES_FROM[9] = {0, 0, 0, 780, 750, 500, 500, 260, 300};
+  if (!whole) return units >= (chunks == 1 ? (gathered ? 768 : 2304) : (chunks == 3 || chunks == 4 ? 780 : 540)) ? MOE_LINES : MOE_TILES;
+  if (chunks <= 2) return units > vk_device_cus() && units < (chunks == 1 ? 4096 : 2048) ? MOE_UNITS : MOE_LINES;
+  constexpr int LINES_FROM[9] = {0, 0, 0, 660, 750, 1, 260, 260, 300};
   return chunks > 8 || units >= LINES_FROM[chunks] || 2 * units <= vk_device_cus() ? MOE_LINES : MOE_TILES;
 }
 #endif
