@@ -27,6 +27,7 @@ typedef __bf16 elem_t;
 #endif
 
 #define VK_WAVE 64
+#define EXPERT_PART_ROWS 192   // the most rows of one expert that a workgroup of the experts' product takes (gemm_experts_kernel)
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;

@@ -131,7 +131,7 @@ struct Kernels::Fn {
   int (*ssm_scan)(P, CP, int64_t, int, int, CP, int64_t, CP, CP, CP, int, P, int64_t, CP, CP, CP, int, int, int, int, int, int, hipStream_t);
   int (*ssm_gate_norm)(P, int64_t, CP, CP, int64_t, CP, int, int, int, int, float, hipStream_t);
   int (*moe_max_tiles)(int, int, int, int);
-  int (*moe_route_plan)(P, P, P, CP, CP, CP, int, CP, int, int, int, int, int, float, int, int, int, int, float, P, P, P, P, P, int, hipStream_t);
+  int (*moe_route_plan_ordered)(P, P, P, CP, CP, CP, int, CP, int, int, int, int, int, float, int, int, int, int, float, P, P, P, P, P, int, P, hipStream_t);
   int (*moe_up)(P, int64_t, CP, int64_t, CP, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_down)(P, CP, int64_t, CP, CP, CP, CP, int, int, int, int, int, hipStream_t);
   int (*moe_combine)(P, CP, CP, CP, int, int, int, hipStream_t);
@@ -165,6 +165,9 @@ struct Kernels::Fn {
   int (*attention_wide_limit)();
   int (*gemm_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, hipStream_t);
   int (*gemm_split_act)(P, CP, CP, int, int, int, int64_t, int64_t, int, P, int64_t, hipStream_t);
+  int (*gemm_experts_takes)(int, int, int, int64_t, int, int);
+  int (*gemm_experts)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int, int64_t, CP, int, int, hipStream_t);
+  int (*gemm_experts_glu)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int, int64_t, CP, int, float, float, float, CP, CP, hipStream_t);
   int (*gemm_grouped_experts)(P, CP, CP, int, int, int, int64_t, int64_t, CP, int64_t, int, CP, CP, int, int, hipStream_t);
   int (*stream_add_norm)(P, P, CP, int, CP, int, int, int, float, hipStream_t);
   int (*embed_bigram)(P, CP, CP, CP, CP, int, int, int, int64_t, int64_t, int64_t, hipStream_t);
@@ -211,7 +214,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(delta_out, "vk_delta_out"); VK(delta_conv_bias, "vk_delta_conv_bias"); VK(paged_attention_blocked, "vk_paged_attention_blocked");
   VK(qkv_post_angles, "vk_qkv_post_angles"); VK(embed_scaled, "vk_embed_scaled"); VK(stream_add, "vk_stream_add");
   VK(stream_pair_norm, "vk_stream_pair_norm"); VK(ssm_scan, "vk_ssm_scan"); VK(ssm_gate_norm, "vk_ssm_gate_norm");
-  VK(moe_max_tiles, "vk_moe_max_tiles"); VK(moe_route_plan, "vk_moe_route_plan"); VK(moe_up, "vk_moe_up");
+  VK(moe_max_tiles, "vk_moe_max_tiles"); VK(moe_route_plan_ordered, "vk_moe_route_plan_ordered"); VK(moe_up, "vk_moe_up");
   VK(moe_down, "vk_moe_down"); VK(moe_combine, "vk_moe_combine"); VK(moe_relu_square, "vk_moe_relu_square");
   VK(qkv_post_norm_angles, "vk_qkv_post_norm_angles"); VK(gate_mul, "vk_gate_mul"); VK(gla_decay, "vk_gla_decay"); VK(gla_rule, "vk_gla_rule");
   VK(gated_head_norm, "vk_gated_head_norm"); VK(moe_up_plain, "vk_moe_up_plain"); VK(moe_glu, "vk_moe_glu");
@@ -224,6 +227,7 @@ Kernels::Kernels(const std::string& lib_dir, const std::string& name) : name_(na
   VK(hyper_in_place, "vk_hyper_in_place"); VK(hyper_step, "vk_hyper_step"); VK(hyper_close, "vk_hyper_close"); VK(embed_normed, "vk_embed_normed");
   VK(attention_wide, "vk_attention_wide"); VK(attention_wide_limit, "vk_attention_wide_limit");
   VK(gemm_act, "vk_gemm_act"); VK(gemm_split_act, "vk_gemm_split_act"); VK(gemm_grouped_experts, "vk_gemm_grouped_experts");
+  VK(gemm_experts_takes, "vk_gemm_experts_takes"); VK(gemm_experts, "vk_gemm_experts"); VK(gemm_experts_glu, "vk_gemm_experts_glu");
   VK(stream_add_norm, "vk_stream_add_norm"); VK(embed_bigram, "vk_embed_bigram");
   VK(qkv_prepare, "vk_qkv_prepare"); VK(paged_attention_biased, "vk_paged_attention_biased"); VK(attn_rel_pad, "vk_attn_rel_pad");
 #undef VK
@@ -1039,6 +1043,7 @@ Kernels::MoePlan Kernels::empty_plan(const Tensor& h, const Tensor& router, int 
   p.pair_row = empty({T * top}, DType::I32);
   p.tile_expert = empty({tiles}, DType::I32);
   p.expert_start = empty({E + 1}, DType::I32);
+  if (tile_rows == 128) p.order = empty({E, 4}, DType::I32);
   return p;
 }
 
@@ -1048,9 +1053,9 @@ void Kernels::route_and_plan(MoePlan& p, const Tensor& h, const Tensor& router, 
   const int64_t T = h.dim(0), E = router.dim(0);
   const int bf = bias ? norm_weight(*bias, "router bias", E) : 0, cf = correction ? norm_weight(*correction, "router correction", E) : 0;
   Tensor logits = empty({T, E}, DType::F32);
-  call(fn_->moe_route_plan(p.idx.data, p.wts.data, logits.data, h.data, router.data, bias ? bias->data : nullptr, bf, correction ? correction->data : nullptr, cf,
+  call(fn_->moe_route_plan_ordered(p.idx.data, p.wts.data, logits.data, h.data, router.data, bias ? bias->data : nullptr, bf, correction ? correction->data : nullptr, cf,
                            (int)T, (int)h.dim(1), (int)E, p.top, weight_eps, score_kind, groups, keep, group_score, scale, p.row_pair.data, p.row_token.data,
-                           p.pair_row.data, p.tile_expert.data, p.expert_start.data, p.tile_rows, stream));
+                           p.pair_row.data, p.tile_expert.data, p.expert_start.data, p.tile_rows, p.order.data, stream));
 }
 
 Kernels::MoePlan Kernels::moe_route_corrected(const Tensor& h, const Tensor& router, const Tensor& correction, int top, int tile_rows, int groups, int keep,
@@ -1469,6 +1474,35 @@ Tensor Kernels::gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& b
                               w.dim(1) * w.dim(2), (int)w.dim(0), row_pair ? row_pair->data : nullptr, act_row ? act_row->data : nullptr, (int)act.dim(0), activation,
                               stream));
   return out;
+}
+
+Tensor Kernels::experts_product(const Tensor& act, const Tensor& w, const MoePlan& plan, int activation, bool named) {
+  const int64_t rows = plan.row_token.numel();
+  if (act.shape.size() == 2 && w.shape.size() == 3 && act.dim(1) == w.dim(2) && w.dim(0) == plan.experts && plan.tile_rows == 128 && (named || act.dim(0) == rows) &&
+      !(named && act.bytes() >= ((size_t)1 << 31)) && fn_->gemm_experts_takes((int)rows, (int)w.dim(1), (int)w.dim(2), act.dim(1), plan.experts, 0)) {
+    expect(act, "activation", dtype_);
+    expect(w, "weights", dtype_);
+    Tensor out = empty({rows, w.dim(1)});
+    call(fn_->gemm_experts(out.data, act.data, w.data, (int)rows, (int)w.dim(1), (int)w.dim(2), act.dim(1), w.dim(1), plan.order.data, plan.experts,
+                           w.dim(1) * w.dim(2), named ? plan.row_token.data : nullptr, (int)act.dim(0), activation, stream));
+    return out;
+  }
+  return gemm_grouped(act, w, plan.tile_expert, activation, &plan.row_pair, named ? &plan.row_token : nullptr);
+}
+
+Tensor Kernels::experts_gated(const Tensor& x, const Tensor& w, const MoePlan& plan, float limit, float slope, float shift, bool weighed) {
+  const int64_t rows = plan.row_token.numel(), F = w.shape.size() == 3 ? w.dim(1) / 2 : 0;
+  if (x.shape.size() == 2 && F > 0 && w.dim(1) == 2 * F && x.dim(1) == w.dim(2) && w.dim(0) == plan.experts && plan.tile_rows == 128 && x.bytes() < ((size_t)1 << 31) &&
+      fn_->gemm_experts_takes((int)rows, (int)F, (int)w.dim(2), x.dim(1), plan.experts, 1)) {
+    expect(x, "activation", dtype_);
+    expect(w, "weights", dtype_);
+    Tensor out = empty({rows, F});
+    call(fn_->gemm_experts_glu(out.data, x.data, w.data, (int)rows, (int)F, (int)w.dim(2), x.dim(1), F, plan.order.data, plan.experts, w.dim(1) * w.dim(2),
+                               plan.row_token.data, (int)x.dim(0), limit, slope, shift, weighed ? plan.row_pair.data : nullptr, weighed ? plan.wts.data : nullptr, stream));
+    return out;
+  }
+  const Tensor both = experts_product(x, w, plan, 0, true);
+  return weighed ? moe_glu_weighed(both, limit, slope, shift, plan) : moe_glu(both, limit, slope, shift);
 }
 
 int Kernels::sample_scratch_words(int rows) const { return fn_->sample_scratch_words(rows); }

@@ -244,6 +244,7 @@ class Kernels {
     Tensor idx, wts;                            // [T, top]
     Tensor row_pair, row_token, pair_row, tile_expert;
     Tensor expert_start;                        // [experts + 1] on the GPU: every expert's first row, and the rows in use
+    Tensor order;                               // [experts, 4], with tiles of 128 rows: vk_gemm_experts' order
     int top = 0, experts = 0, tile_rows = 16;   // an expert's rows are padded to whole tiles of this many
   };
   // tile_rows 16: for moe_up / moe_down; 128: for gemm_grouped, whose blocks are the plan's tiles.
@@ -266,6 +267,11 @@ class Kernels {
   Tensor gemm_grouped(const Tensor& act, const Tensor& w, const Tensor& block_weights, int activation = 0, const Tensor* row_pair = nullptr,
                       const Tensor* act_row = nullptr);
   bool gemm_grouped_takes(int64_t K) const;
+  // The experts' product over a plan with tiles of 128 rows: gemm_grouped's bits in the rows that have a pair, by the kernel that is the faster one.
+  // named: act's rows are the tokens; else they lie in the plan's order.
+  Tensor experts_product(const Tensor& act, const Tensor& w, const MoePlan& plan, int activation, bool named);
+  // The tokens' product with [gate: F | up: F] matrices, then moe_glu or (weighed) moe_glu_weighed: [rows, F], in one launch where the kernel takes it.
+  Tensor experts_gated(const Tensor& x, const Tensor& w, const MoePlan& plan, float limit, float slope, float shift, bool weighed);
   // moe_route with a choice of score: 0 as moe_route; 1: a chosen expert's weight is the logistic function of its logit.
   // 2: the softmax over all experts as it is.  groups, keep: only experts of the `keep` best of that many equal groups can be
   // chosen; scale: on every weight.

@@ -1567,10 +1567,9 @@ class RoutedExperts : public FeedForward {
       return k.moe_sum(k.moe_down(act, w_down_, plan), plan, extra);
     }
     const Kernels::MoePlan plan = route(x, 128, bias);
-    Tensor act = k.gemm_grouped(x, w_up_, plan.tile_expert, gated_ ? 0 : 1, &plan.row_pair, &plan.row_token);
-    if (weigh_input_) return k.moe_sum_unweighed(k.gemm_grouped(k.moe_glu_weighed(act, limit_, slope_, shift_, plan), w_down_, plan.tile_expert, 0, &plan.row_pair), plan);
-    if (gated_) act = k.moe_glu(act, limit_, slope_, shift_);
-    return k.moe_sum(k.gemm_grouped(act, w_down_, plan.tile_expert, 0, &plan.row_pair), plan, extra);
+    const Tensor act = gated_ ? k.experts_gated(x, w_up_, plan, limit_, slope_, shift_, weigh_input_) : k.experts_product(x, w_up_, plan, 1, true);
+    const Tensor y = k.experts_product(act, w_down_, plan, 0, false);
+    return weigh_input_ ? k.moe_sum_unweighed(y, plan) : k.moe_sum(y, plan, extra);
   }
   static constexpr int kRowsAnExpertForTiles = 32;
 

@@ -1206,7 +1206,7 @@ static bool grouped_wide(int M, int N, int matrices, bool named) {
   return !named && columns <= 4 && 2 * groups >= vk_device_cus();
 }
 
-static bool rows_far(int64_t lda) { return (127 * lda + 2 * VK_SLAB) * (int64_t)sizeof(elem_t) > (int64_t)UINT32_MAX; }
+static bool rows_far(int64_t lda, int rows = 128) { return ((rows - 1) * lda + 2 * VK_SLAB) * (int64_t)sizeof(elem_t) > (int64_t)UINT32_MAX; }
 
 template <int S, bool SWIGLU = false, int FNW = 4, bool GROUPED = false>
 static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
@@ -1438,6 +1438,248 @@ static int launch_alternate(elem_t* out, const elem_t* act, const elem_t* w, int
   if (N % 4 != 0) form &= ~OUT_VEC;       // the last block of columns begins at N - COLS: four of its columns are then no aligned vector
   gemm_alternate_kernel<FNW, SA, SW, SWIGLU><<<(unsigned)tiles, 512, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, row_blocks);
   return vk_check_launch("gemm_alternate");
+}
+#endif
+
+#ifdef VK_BF16
+// ------------------------------------------------------------ grouped, alternating
+// The experts' product by a plan's order: 16-bit elements, K in whole chunks.  A workgroup takes one part of a matrix's rows, up to 192 as they are, in
+// steps of 32 (FA: 16-row fragments of a wave, one to six), and 256 weight rows (GLU: 128 of the gate and their up rows), by two groups of four waves that take
+// turns as in gemm_alternate_kernel: group 0 has the first half of the rows and brings the activations, group 1 the second half and brings the weights; wave q
+// of either has weight rows 64 q .. 64 q + 63.  Reduction order, operand roles and bits are those of gemm_pipe_kernel.
+//
+// What bounds it: an expert's matrix serves one or two parts, so that weights come from memory at 4 to 5.7 TB/s, and a part's height decides how long the
+// matrix unit and LDS (4 + FA fragments for 4 FA products) are busy beside that.  Blocks of 128 rows, which this replaces, multiplied up to 64 rows
+// of padding a block, brought a matrix in once a block and took LDS 8 fragments for 16 products.  Parts are levelled (193 rows: 128 and 65 at
+// most, not 192 and 1), up to four rows of fragments leave LDS for a fourth tile of weights, and a matrix that serves one part passes the caches by (nt: 4,608 x 4,096, 1,360 tokens x 3
+// choices of 32 268 -> 242 us; with two parts a matrix 2 to 8 % slower).  The order has the tallest parts first, as the launch's last workgroups else run alone
+// (309 -> 266 us there).  Parts of a matrix lie next to each other for eight column blocks at a time: workgroup i runs on chip part i % 8, whose cache
+// then has a column block's weights for all parts.  (All tiles of a matrix on one chip part instead: no gain.)
+// Measured on MI355X, 32 experts, random choices, gemm_pipe_kernel's blocks against this, us: 2,048 tokens x 3, 6,144 x 4,096 465 -> 400 (with the gated activation,
+// a pass of its own before, 516 -> 402), 4,096 x 3,072 277 -> 206; 2,445 x 4, 6,144 x 4,096 610 -> 533, 4,096 x 3,072 334 -> 302; 2,400 x 4, 3,072 x 2,048 194 ->
+// 165; 1,334 x 4, 1,536 x 2,048 86 -> 57; 700 x 3, 6,144 x 4,096 331 -> 283 (5.7 TB/s); 8 experts, 2,048 x 2, 4,096 x 3,072 154 -> 117.
+struct GluArgs {
+  float limit, slope, shift;
+  const int32_t* row_pair;           // both or neither
+  const float* wts;
+};
+template <bool GLU, int FA>
+__device__ __forceinline__ void experts_tile(unsigned char* lds, elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w, int M, int N, int K,
+                                             int64_t lda, int64_t ldo, int out_form, int m_blk, int n_blk, bool once, const int32_t* __restrict__ act_row,
+                                             const GluArgs& glu) {
+  constexpr int FNW = 4, SA = FA <= 2 || FA == 5 ? 3 : 2, SW = FA <= 4 ? 4 : 3, BN = 256;
+  constexpr int A_BYTES = 32 * FA * T_ROWB, W_BYTES = BN * T_ROWB;
+  constexpr int LA = FA, LW = 8;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int group = wave >> 2, q = wave & 3;
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  const unsigned lds0 = lds_offset_of(lds) + (group == 0 ? q * LA * 8 * T_ROWB : SA * A_BYTES + q * LW * 8 * T_ROWB);
+  f32x4 total[FNW][FA];
+#pragma unroll
+  for (int i = 0; i < FNW; ++i)
+#pragma unroll
+    for (int j = 0; j < FA; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int frag = r16 * T_ROWB + ((kg ^ (r16 & 7)) * 16);
+  const int a_at = group * FA * 16 * T_ROWB + frag, w_at = SA * A_BYTES + q * 64 * T_ROWB + frag;
+
+  auto walk = [&](auto g_, auto once_) __attribute__((always_inline)) {
+    constexpr bool ONCE = decltype(once_)::value;
+    constexpr int G = decltype(g_)::value, L = G ? LW : LA, ST = G ? SW : SA, BYTES = G ? W_BYTES : A_BYTES, HALF = ST > 2 ? (L + 1) / 2 : L;
+    unsigned voff[G ? 1 : FA];
+    const unsigned char* src;
+    int64_t step = 0, up = 0;
+    if constexpr (G == 1) {
+      src = reinterpret_cast<const unsigned char*>(w + (int64_t)(n_blk + q * (GLU ? 32 : 64)) * K);
+      step = 8 * (int64_t)K * (int64_t)sizeof(elem_t);
+      up = GLU ? (int64_t)(N - 32) * K * (int64_t)sizeof(elem_t) : 0;
+      voff[0] = (unsigned)((lr * (int64_t)K + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+    } else {
+      src = reinterpret_cast<const unsigned char*>(act + (act_row != nullptr ? 0 : (int64_t)m_blk * lda));
+#pragma unroll
+      for (int j = 0; j < FA; ++j) {
+        const int row = min(m_blk + (q * FA + j) * 8 + lr, M - 1);
+        voff[j] = (unsigned)(((int64_t)(act_row != nullptr ? act_row[row] : row - m_blk) * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+      }
+    }
+    unsigned fill = 0, read_a = 0, read_w = 0;
+    auto issue = [&](int from, int to) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < L; ++j)
+        if (j >= from && j < to) {
+          const unsigned at = __builtin_amdgcn_readfirstlane(lds0 + fill + j * 8 * T_ROWB);
+          if constexpr (G == 1 && ONCE) pipe_load_to_lds16_once(src + j * step + (j >= 4 ? up : 0), voff[0], at);
+          else if constexpr (G == 1) pipe_load_to_lds16_sv(src + j * step + (j >= 4 ? up : 0), voff[0], at);
+          else pipe_load_to_lds16_sv(src, voff[j], at);
+        }
+      if (to < L) return;
+      src += T_ROWB;
+      fill = fill == (ST - 1) * BYTES ? 0 : fill + BYTES;
+    };
+    f32x4 acc[FNW][FA];
+    auto slab = [&](int S, bool first, bool more) __attribute__((always_inline)) {
+      frag_t af[FA], wf[FNW];
+#pragma unroll
+      for (int j = 0; j < FA; ++j) af[j] = *reinterpret_cast<const frag_t*>(lds + (a_at ^ (S * 64)) + read_a + j * 16 * T_ROWB);
+#pragma unroll
+      for (int i = 0; i < FNW; ++i) wf[i] = *reinterpret_cast<const frag_t*>(lds + (w_at ^ (S * 64)) + read_w + i * 16 * T_ROWB);
+      if (S == 1) {
+        read_a = read_a == (SA - 1) * A_BYTES ? 0 : read_a + A_BYTES;
+        read_w = read_w == (SW - 1) * W_BYTES ? 0 : read_w + W_BYTES;
+      }
+      if (more && S == 0) issue(0, HALF);
+      if (more && S == 1 && HALF < L) issue(HALF, L);
+      if (G == 1 && S == 1) {
+        if (more) wait_vmcnt_n<(SW - 2) * LW>(); else wait_vmcnt_n<0>();
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      al_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < FNW; ++i)
+#pragma unroll
+        for (int j = 0; j < FA; ++j) acc[i][j] = mma_slab(wf[i], af[j], first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (G == 0 && S == 1) {
+        if (more) wait_vmcnt_n<(SA - 2) * LA>(); else wait_vmcnt_n<0>();
+      }
+      al_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto chunk = [&](bool last) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < T_CHUNK_TILES; ++t) {
+        const bool more = !last || t + ST - 1 < T_CHUNK_TILES;
+        slab(0, t == 0, more);
+        slab(1, false, more);
+      }
+#pragma unroll
+      for (int i = 0; i < FNW; ++i)
+#pragma unroll
+        for (int j = 0; j < FA; ++j) {
+          total[i][j].x = total[i][j].x + acc[i][j].x;
+          total[i][j].y = total[i][j].y + acc[i][j].y;
+          total[i][j].z = total[i][j].z + acc[i][j].z;
+          total[i][j].w = total[i][j].w + acc[i][j].w;
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < ST - 1; ++p) issue(0, L);
+    wait_vmcnt_n<(ST - 2) * L>();
+    al_barrier();
+    if (G == 1) al_barrier();
+    for (int c = 1; c < K / KC; ++c) chunk(false);
+    chunk(true);
+    if (G == 0) al_barrier();
+  };
+  if (group == 0) walk(std::integral_constant<int, 0>(), std::false_type());
+  else if (once) walk(std::integral_constant<int, 1>(), std::true_type());
+  else walk(std::integral_constant<int, 1>(), std::false_type());
+
+  const int m0 = m_blk + group * FA * 16 + r16, n0 = n_blk + q * (GLU ? 32 : 64) + 4 * kg;
+  if constexpr (GLU) {
+#pragma unroll
+    for (int j = 0; j < FA; ++j) {
+      const int m = m0 + j * 16;
+      float rw = 1.f;
+      bool none = false;
+      if (glu.wts != nullptr && m < M) {
+        const int pair = glu.row_pair[m];
+        none = pair < 0;
+        rw = glu.wts[max(pair, 0)];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = fminf(round_to_elem(total[i][j][e]) * rw, glu.limit), u = fminf(fmaxf(round_to_elem(total[i + 2][j][e]) * rw, -glu.limit), glu.limit);
+          y[e] = none ? 0.f : (g / (1.f + expf(-glu.slope * g))) * (u + glu.shift);
+        }
+        store_out4(out, ldo, m, n0 + i * 16, M, N, y, out_form);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FNW; ++i)
+#pragma unroll
+      for (int j = 0; j < FA; ++j) store_out4(out, ldo, m0 + j * 16, n0 + i * 16, M, N, total[i][j], out_form);
+  }
+}
+
+template <bool GLU>
+__global__ __launch_bounds__(512, 2) void gemm_experts_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w, int N, int K,
+                                                              int64_t lda, int64_t ldo, int out_form, const int4* __restrict__ order, int matrices,
+                                                              int64_t weights_stride, const int32_t* __restrict__ act_row, GluArgs glu) {
+  constexpr int COLS = GLU ? 128 : 256;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int lane = threadIdx.x & 63, cols = (N + COLS - 1) / COLS, lin = blockIdx.x;
+  int before = 0, first = 0, rows = 0, which = 0;
+  for (int e0 = 0; e0 < matrices; e0 += 64) {
+    const int4 entry = order[min(e0 + lane, matrices - 1)];
+    const uint64_t begun = __ballot(e0 + lane < matrices && entry.z > 0 && entry.x * cols <= lin);
+    if (begun == 0) break;
+    const int from = 63 - __builtin_clzll(begun);
+    before = __builtin_amdgcn_readlane(entry.x, from);
+    first = __builtin_amdgcn_readlane(entry.y, from);
+    rows = __builtin_amdgcn_readlane(entry.z, from);
+    which = __builtin_amdgcn_readlane(entry.w, from);
+    if (begun != ~0ull) break;
+  }
+  const int parts = (rows + EXPERT_PART_ROWS - 1) / EXPERT_PART_ROWS, o = lin - before * cols;
+  if (o >= parts * cols) return;
+  const int cg = o / (8 * parts), rem = o - cg * 8 * parts, wide = min(8, cols - cg * 8);
+  const int r = rem / wide, nb = cg * 8 + (rem - r * wide);
+  const int per = ((rows + parts - 1) / parts + 31) & ~31;
+  const int count = min(per, rows - r * per);
+  const int m_blk = __builtin_amdgcn_readfirstlane(first + r * per), n_blk = __builtin_amdgcn_readfirstlane(min(nb * COLS, N - COLS));
+  const int M = __builtin_amdgcn_readfirstlane(m_blk + count), fa = __builtin_amdgcn_readfirstlane((count + 31) / 32);
+  const elem_t* wm = w + (int64_t)which * weights_stride;
+  switch (fa) {
+    case 1: experts_tile<GLU, 1>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+    case 2: experts_tile<GLU, 2>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+    case 3: experts_tile<GLU, 3>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+    case 4: experts_tile<GLU, 4>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+    case 5: experts_tile<GLU, 5>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+    default: experts_tile<GLU, 6>(lds, out, act, wm, M, N, K, lda, ldo, out_form, m_blk, n_blk, parts == 1, act_row, glu); break;
+  }
+}
+
+static_assert(EXPERT_PART_ROWS == 32 * 6, "six heights");
+// Whether a product goes this way or by blocks of 128 rows (launch_pipe), by the workgroups that it can be expected to have: a matrix's rows, as M and the
+// matrices tell them, are a part or somewhat more than their share of one.  A workgroup is alone on its compute unit and as long as all
+// of K, so that few of them, or a few more than one round, lose to the smaller tiles of the other kernel; the fewer rows a matrix has, the more
+// its weights' way from memory decides, which this kernel is better at.  Measured on MI355X in recorded launches with the weights of several layers in turn, 346
+// sizes of 8 to 128 matrices, 32 to 1,024 rows a matrix, 256 x 1,024 to 6,144 x 4,096 weights: blocks alone 36.7 ms, parts alone 31.8, by
+// this rule 31.3, with the better one everywhere 31.2; 8 matrices, 777 tokens x 2, 1,024 x 1,024 (about 45 workgroups) 14.6, 24.7 us; 16 matrices of 512 rows, 1,536 x 1,024 (312)
+// 46.9, 56.7; 16 of 97, 4,096 x 3,072 (256) 117, 76; 64 of 127, 1,536 x 1,024 (402) 87, 58; one chunk, 64 of 384, 512 x 512 31.0, 33.8.  Slower by
+// more than 3 % than the better one: 27 sizes, the worst 8 of 194, 4,096 x 3,072 64.9, 72.7.
+static bool experts_takes(int M, int N, int K, int64_t lda, int matrices, bool gated) {
+  const int columns = gated ? 128 : 256;
+  if (K % KC != 0 || K == KC || N < columns || matrices < 1 || rows_far(lda, EXPERT_PART_ROWS)) return false;
+  const double rows = std::max(M - 127.0 * matrices, 1.0) / matrices, units = vk_device_cus();
+  const double groups = matrices * std::max(1.0, rows / EXPERT_PART_ROWS + 0.35) * ((N + columns - 1) / columns);
+  if (rows < 48) return groups >= 0.4 * units;
+  if (rows < 100) return groups >= 0.5 * units;
+  return groups >= 0.66 * units && (groups <= units || groups >= 1.33 * units || K >= 4 * KC);
+}
+template <bool GLU>
+static int launch_experts(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, const int32_t* order, int matrices,
+                          int64_t weights_stride, const int32_t* act_row, const GluArgs& glu, hipStream_t st) {
+  constexpr int COLS = GLU ? 128 : 256;
+  constexpr int smem = (2 * 128 + 4 * 256) * T_ROWB;      // the most of the heights: two tiles of 128 rows beside four of weights
+  static bool configured = false;
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_experts_kernel<GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    configured = true;
+  }
+  if (N % 4 != 0) form &= ~OUT_VEC;
+  const int64_t tiles = (int64_t)(M / 128) * ((N + COLS - 1) / COLS);
+  gemm_experts_kernel<GLU><<<(unsigned)tiles, 512, smem, st>>>(out, act, w, N, K, lda, ldo, form, (const int4*)order, matrices, weights_stride, act_row, glu);
+  return vk_check_launch("gemm (experts)");
 }
 #endif
 
@@ -2189,6 +2431,18 @@ static int out_form_of(const elem_t* out, int64_t ldo, int activation) {
   return ((ldo % 4 == 0) && ((uintptr_t)out % 16 == 0) ? OUT_VEC : 0) | (activation == 1 ? OUT_SQUARED_RELU : 0);
 }
 
+static int experts_refuse(const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, const int32_t* order, int matrices, int64_t weights_stride,
+                          const int32_t* act_row, int act_rows, bool gated) {
+  VK_REQUIRE(sizeof(elem_t) == 2, "experts' product: 16-bit elements");
+  VK_REQUIRE(M >= 0 && M % 128 == 0 && N >= (gated ? 128 : 256) && K > 0 && K % KC == 0, "experts' product: bad sizes M=%d N=%d K=%d", M, N, K);
+  VK_REQUIRE(lda >= K && lda % VK_VEC == 0 && ldo >= N, "experts' product: bad row strides");
+  VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0 && weights_stride % VK_VEC == 0, "experts' product: operands must be 16-byte aligned");
+  VK_REQUIRE(order != nullptr && (uintptr_t)order % 16 == 0 && matrices > 0, "experts' product: a plan's order is needed");
+  VK_REQUIRE(act_row != nullptr ? act_rows > 0 && (int64_t)act_rows * lda * (int64_t)sizeof(elem_t) < ((int64_t)1 << 31) : !rows_far(lda, EXPERT_PART_ROWS),
+             "experts' product: rows too far apart");
+  return 0;
+}
+
 // A grouped product through the tile kernel: rows in blocks of 128, block b multiplied by the weight matrix
 // block_weights[b] of several [N, K] matrices that lie weights_stride elements apart (negative: the block is skipped and
 // its output rows are left as they are).  K in whole pairs of slabs (128 bytes of a row).  The same bits as vk_gemm gives
@@ -2212,6 +2466,44 @@ int vk_gemm_grouped_experts(elem_t* out, const elem_t* act, const elem_t* w, int
   if (M == 0) return 0;
   return launch_pipe<2, false, 4, true>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), st, block_weights, weights_stride, row_pair, act_row,
                                          matrices);
+}
+
+// Whether vk_gemm_experts (gated: vk_gemm_experts_glu) takes a product of this size: rows as vk_gemm_grouped_experts counts them.
+int vk_gemm_experts_takes(int M, int N, int K, int64_t lda, int matrices, int gated) {
+#ifdef VK_BF16
+  return experts_takes(M, N, K, lda, matrices, gated != 0);
+#else
+  return 0;
+#endif
+}
+
+// The experts' product by a plan's order (vk_moe_route_plan_ordered) instead of its blocks: act, w, act_row and activation as in
+// vk_gemm_grouped_experts, whose bits it gives.  Rows of out that no pair has are left as they are.
+int vk_gemm_experts(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, const int32_t* order, int matrices,
+                    int64_t weights_stride, const int32_t* act_row, int act_rows, int activation, hipStream_t st) {
+  VK_REQUIRE(activation == 0 || activation == 1, "experts' product: unknown activation %d", activation);
+  if (experts_refuse(act, w, M, N, K, lda, ldo, order, matrices, weights_stride, act_row, act_rows, false)) return 1;
+  if (M == 0) return 0;
+#ifdef VK_BF16
+  return launch_experts<false>(out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, activation), order, matrices, weights_stride, act_row, GluArgs{}, st);
+#else
+  return 1;
+#endif
+}
+
+// The same for matrices of F gate rows and then F up rows, out [., F]: the gated activation (moe_glu_kernel) of the product's elements.
+// wts, row_pair (both or neither): as in vk_moe_glu_weighed.
+int vk_gemm_experts_glu(elem_t* out, const elem_t* act, const elem_t* w, int M, int F, int K, int64_t lda, int64_t ldo, const int32_t* order, int matrices,
+                        int64_t weights_stride, const int32_t* act_row, int act_rows, float limit, float slope, float shift, const int32_t* row_pair,
+                        const float* wts, hipStream_t st) {
+  VK_REQUIRE(limit > 0.f && (row_pair == nullptr) == (wts == nullptr), "experts' product: a positive limit, rows' pairs and weights or neither");
+  if (experts_refuse(act, w, M, F, K, lda, ldo, order, matrices, weights_stride, act_row, act_rows, true)) return 1;
+  if (M == 0) return 0;
+#ifdef VK_BF16
+  return launch_experts<true>(out, act, w, M, F, K, lda, ldo, out_form_of(out, ldo, 0), order, matrices, weights_stride, act_row, {limit, slope, shift, row_pair, wts}, st);
+#else
+  return 1;
+#endif
 }
 
 int vk_gemm_grouped_rows(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,

@@ -215,10 +215,13 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(MoeChoice a) {
 // its place).  row_pair [max_rows]: the pair (token * top + choice) of a row, or -1; row_token [max_rows]: the row's
 // token (0 for a row without a pair); pair_row [pairs]; tile_expert [max_tiles]: the expert of a tile, or -1 beyond the
 // last; expert_start [E + 1]: the first row of every expert, and the rows in use.
+// order [E] or null (vk_gemm_experts): {parts before, first row, rows, expert}, an expert's rows in ceil(rows / EXPERT_PART_ROWS) parts; experts without
+// rows come last.  Up to 64 experts: the ones of taller parts first, so that a launch's last workgroups are its shortest.
 struct MoePlanArgs {
   const int32_t* idx;
   int32_t *row_pair, *row_token, *pair_row, *tile_expert, *expert_start;
   int pairs, top, E, max_tiles, tile_rows;
+  int4* order;
 };
 // By all threads of a workgroup of 1,024; plan: LDS, [E] counts, then [E] cursors.
 __device__ __forceinline__ void moe_make_plan(const MoePlanArgs& a, int32_t* plan) {
@@ -251,16 +254,34 @@ __device__ __forceinline__ void moe_make_plan(const MoePlanArgs& a, int32_t* pla
         for (int j = 0; j < n; ++j) a.tile_expert[tile + j] = e;
         if (e == a.E - 1) a.expert_start[a.E] = upto * a.tile_rows;
       }
+      if (a.order != nullptr) {
+        const int rows = e < a.E ? count[e] : 0, parts = (rows + EXPERT_PART_ROWS - 1) / EXPERT_PART_ROWS;
+        const int key = (rows > 0 ? (rows + parts - 1) / parts : 0) * 64 + 63 - e;       // different for every lane
+        int rank = 0, before = 0;
+#pragma unroll
+        for (int i = 0; i < 64; ++i) {
+          const bool ahead = __builtin_amdgcn_readlane(key, i) > key;
+          rank += ahead ? 1 : 0;
+          before += ahead ? __builtin_amdgcn_readlane(parts, i) : 0;
+        }
+        if (rank < a.E) a.order[rank] = int4{before, tile * a.tile_rows, rows, e < a.E ? e : 0};
+      }
     }
   } else if (threadIdx.x == 0) {
-    int tile = 0;
+    int tile = 0, parts = 0, busy = 0;
     for (int e = 0; e < a.E; ++e) {
       const int n = (count[e] + a.tile_rows - 1) / a.tile_rows;
       cursor[e] = tile * a.tile_rows;
       a.expert_start[e] = tile * a.tile_rows;
       for (int j = 0; j < n; ++j) a.tile_expert[tile + j] = e;
+      if (a.order != nullptr && n > 0) {
+        a.order[busy++] = int4{parts, tile * a.tile_rows, count[e], e};
+        parts += (count[e] + EXPERT_PART_ROWS - 1) / EXPERT_PART_ROWS;
+      }
       tile += n;
     }
+    if (a.order != nullptr)
+      for (; busy < a.E; ++busy) a.order[busy] = int4{parts, 0, 0, 0};
     a.expert_start[a.E] = tile * a.tile_rows;
   }
   __syncthreads();
@@ -685,18 +706,27 @@ static int route_launch(int32_t* idx, float* wts, float* logits, const elem_t* h
 // chosen logits alone, whatever the others are); 1: the logistic function of a chosen logit as it is; 2: the softmax over all experts as it
 // is.  groups, keep: only experts of the `keep` best of that many equal groups can be chosen (1, 1: all); group_score 0: a group is worth
 // its largest score, 1: the sum of its two largest.  correction (score 1, no bias; [E] elements or floats): joins the scores for the choice
-// of groups and experts and not for the weights.  scale: on every weight.  tile_rows: rows of a tile of the plan (moe_plan_kernel).
+// of groups and experts and not for the weights.  scale: on every weight.  tile_rows: rows of a tile of the plan (moe_plan_kernel).  order: [E][4], 16-byte aligned, or null.
+int vk_moe_route_plan_ordered(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32,
+                              const void* correction, int correction_is_f32, int T, int W, int E, int top, float weight_eps, int score_kind, int groups, int keep,
+                              int group_score, float scale, int32_t* row_pair, int32_t* row_token, int32_t* pair_row, int32_t* tile_expert, int32_t* expert_start,
+                              int tile_rows, int32_t* order, hipStream_t st) {
+  VK_REQUIRE(score_kind >= 0 && score_kind <= 2 && (group_score == 0 || group_score == 1), "router: score kind %d, group score %d", score_kind, group_score);
+  VK_REQUIRE(correction == nullptr || (bias == nullptr && score_kind == 1), "router: a correction goes with logistic scores and without a bias");
+  VK_REQUIRE(T >= 0 && top > 0 && E > 0 && E <= 4096 && tile_rows > 0, "expert plan: bad sizes T=%d top=%d E=%d", T, top, E);
+  VK_REQUIRE((uintptr_t)order % 16 == 0, "expert plan: the order must be 16-byte aligned");
+  if (T == 0) return 0;
+  const MoePlanArgs plan = {idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E, vk_moe_max_tiles(T, top, E, tile_rows), tile_rows, (int4*)order};
+  return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale, group_score, correction,
+                      correction_is_f32, plan);
+}
+
 int vk_moe_route_plan(int32_t* idx, float* wts, float* logits, const elem_t* h, const elem_t* router, const void* bias, int bias_is_f32,
                       const void* correction, int correction_is_f32, int T, int W, int E, int top, float weight_eps, int score_kind, int groups, int keep,
                       int group_score, float scale, int32_t* row_pair, int32_t* row_token, int32_t* pair_row, int32_t* tile_expert, int32_t* expert_start,
                       int tile_rows, hipStream_t st) {
-  VK_REQUIRE(score_kind >= 0 && score_kind <= 2 && (group_score == 0 || group_score == 1), "router: score kind %d, group score %d", score_kind, group_score);
-  VK_REQUIRE(correction == nullptr || (bias == nullptr && score_kind == 1), "router: a correction goes with logistic scores and without a bias");
-  VK_REQUIRE(T >= 0 && top > 0 && E > 0 && E <= 4096 && tile_rows > 0, "expert plan: bad sizes T=%d top=%d E=%d", T, top, E);
-  if (T == 0) return 0;
-  const MoePlanArgs plan = {idx, row_pair, row_token, pair_row, tile_expert, expert_start, T * top, top, E, vk_moe_max_tiles(T, top, E, tile_rows), tile_rows};
-  return route_launch(idx, wts, logits, h, router, bias, bias_is_f32, T, W, E, top, weight_eps, st, score_kind, groups, keep, scale, group_score, correction,
-                      correction_is_f32, plan);
+  return vk_moe_route_plan_ordered(idx, wts, logits, h, router, bias, bias_is_f32, correction, correction_is_f32, T, W, E, top, weight_eps, score_kind, groups, keep,
+                                   group_score, scale, row_pair, row_token, pair_row, tile_expert, expert_start, tile_rows, nullptr, st);
 }
 
 // An expert product of rows in tiles of 16: by the kernels for whole slabs where they take the sizes, else by the one for every K.
