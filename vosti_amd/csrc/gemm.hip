@@ -37,6 +37,8 @@
 //   gemm_alternate      256 rows or more, K a multiple of 512, 16-bit elements: 256 x 192, 160 or 128 per workgroup of eight
 //                       waves whose two halves take turns between LDS and the matrix unit.  Optionally SwiGLU in the epilogue
 //                       (alternate_fragments says when).
+//   gemm_fine           32-bit elements, more than 64 rows (32 where K is short or with SwiGLU), K as gemm_pipe: tiles of 32 x 32 to 96 x 64 or 64 x 128, the one
+//                       whose launch ends first (fine_takes, fine_tile).  Optionally SwiGLU in the epilogue.
 //   gemm_tiled          any M and K: the same tile through registers into LDS, predicated.
 #include <algorithm>
 #include <cmath>
@@ -1255,6 +1257,185 @@ static int launch_pipe(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   return vk_check_launch("gemm_pipe");
 }
 
+#ifdef VK_F32
+// ------------------------------------------------------------ 32-bit tiles
+// The tile kernel of 32-bit elements: K in whole pairs of slabs, 32 FM activation rows and 32 FN weight rows a workgroup of four waves (SWIGLU: 16 FN gate rows and
+// their up rows, which the same wave multiplies), S stages.  Operand roles, reduction order and bits are those of gemm_tiled_kernel.
+//
+// What bounds it: the 32-bit matrix instruction takes 32 clocks for 2 KB of operands, so that LDS and caches are idle most of the time even with tiles of 32 x 64,
+// and what a launch loses are rows of padding and the compute units that wait for the ones with a tile more.  Tiles of 128 x 128 (gemm_pipe_kernel, before) at 651 rows are 6 x 96 for
+// gate/up of 6,144 x 2,048: 15 % of the rows are padding, and 576 tiles are three for some of 256 units.  Here the tile is chosen for the launch (fine_tile).  Measured on
+// MI355X in recorded launches with the weights of several layers in turn, before and after, us: 651 rows, gate/up with SwiGLU 6,144 x 2,048 366 -> 260 (126 TFLOP/s), 2,048 x 6,144
+// 220 -> 157, 4,096 x 2,048 126 -> 96, 2,048 x 2,048 78 -> 57; 217 rows, 3,072 x 1,024 with SwiGLU 72 -> 31, 1,024 x 3,072 69 -> 30; 434 rows, 1,024 x 1,024 40 -> 15; 2,048 rows,
+// 6,144 x 2,048 721 -> 714.  The four instructions of a slab go round the tile's fragments, so that none waits for the one before it.
+template <int FM, int FN, int S, bool SWIGLU, bool WHOLE>
+__global__ __launch_bounds__(256) void gemm_fine_kernel(elem_t* __restrict__ out, const elem_t* __restrict__ act, const elem_t* __restrict__ w, int M, int N, int K,
+                                                        int64_t lda, int64_t ldo, int out_form, int row_blocks) {
+  static_assert(!SWIGLU || FN % 2 == 0, "as many gate as up fragments a wave");
+  constexpr int BM = 32 * FM, BN = 32 * FN, COLS = SWIGLU ? BN / 2 : BN;
+  constexpr int W_BYTES = BN * T_ROWB, STAGE_BYTES = W_BYTES + BM * T_ROWB;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // [S][weights, activations]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kg = lane >> 4, wn = wave & 1, wm = wave >> 1;
+  const int lin = blockIdx.x, tiles = gridDim.x, part = lin & 7;
+  const int tile = part * (tiles >> 3) + min(part, tiles & 7) + (lin >> 3);
+  const int per_band = 8 * row_blocks, band = tile / per_band, at = tile - band * per_band;
+  const int wide = min(8, (N + COLS - 1) / COLS - band * 8);
+  const int mb = at / wide, nb = band * 8 + (at - mb * wide);
+  const int n_blk = nb * COLS, m_blk = mb * BM, ntiles = K / (2 * VK_SLAB);
+
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  const unsigned char* wbase = reinterpret_cast<const unsigned char*>(w + (int64_t)n_blk * K);
+  const unsigned char* ubase = reinterpret_cast<const unsigned char*>(w + (int64_t)(N + n_blk) * K);
+  const unsigned char* abase = reinterpret_cast<const unsigned char*>(act + (int64_t)m_blk * lda);
+  unsigned offw[FN], offa[FM];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int row = (wave * FN + j) * 8 + lr;                              // of the workgroup's weight rows; a wave along them has 16 FN
+    const int of_wave = row / (16 * FN), in = row - of_wave * 16 * FN;
+    const int local = SWIGLU ? of_wave * 8 * FN + in % (8 * FN) : row;     // gate rows first, then their up rows
+    offw[j] = (unsigned)(((int64_t)(min(n_blk + local, N - 1) - n_blk) * K + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+  }
+#pragma unroll
+  for (int j = 0; j < FM; ++j)
+    offa[j] = (unsigned)(((int64_t)(min(m_blk + (wave * FM + j) * 8 + lr, M - 1) - m_blk) * lda + lc * VK_VEC) * (int64_t)sizeof(elem_t));
+  const unsigned lds0 = lds_offset_of(lds);
+  auto issue = [&](int kt) {
+    const unsigned base = lds0 + (kt % S) * STAGE_BYTES;
+    const int64_t kb = (int64_t)kt * T_ROWB;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const bool up = SWIGLU && ((wave * FN + j) * 8) % (16 * FN) >= 8 * FN;
+      pipe_load_to_lds16_sv((up ? ubase : wbase) + kb, offw[j], base + (wave * FN + j) * 8 * T_ROWB);
+    }
+#pragma unroll
+    for (int j = 0; j < FM; ++j) pipe_load_to_lds16_sv(abase + kb, offa[j], base + W_BYTES + (wave * FM + j) * 8 * T_ROWB);
+  };
+  f32x4 acc[FN][FM], total[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < S - 1; ++p)
+    if (p < ntiles) issue(p);
+  auto step = [&](int kt) {
+    // Tile kt has landed once at most the loads of the tiles after it are outstanding.
+    const int later = min(S - 2, ntiles - 1 - kt);
+    if (later <= 0) wait_vmcnt_n<0>();
+    else if (later == 1) wait_vmcnt_n<FM + FN>();
+    else wait_vmcnt_n<2 * (FM + FN)>();
+    __syncthreads();
+    if (kt + S - 1 < ntiles) issue(kt + S - 1);
+    const unsigned char* base = lds + (kt % S) * STAGE_BYTES;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      frag_t wf[FN], af[FM];
+      const int col = ((s * 4 + kg) ^ (r16 & 7)) * 16;
+#pragma unroll
+      for (int i = 0; i < FN; ++i) wf[i] = *reinterpret_cast<const frag_t*>(base + (wn * 16 * FN + i * 16 + r16) * T_ROWB + col);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const frag_t*>(base + W_BYTES + (wm * 16 * FM + i * 16 + r16) * T_ROWB + col);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+          for (int j = 0; j < FM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
+    }
+  };
+  auto close_chunk = [&]() {
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j) {
+        total[i][j].x = total[i][j].x + acc[i][j].x;
+        total[i][j].y = total[i][j].y + acc[i][j].y;
+        total[i][j].z = total[i][j].z + acc[i][j].z;
+        total[i][j].w = total[i][j].w + acc[i][j].w;
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  if (WHOLE) {
+    for (int kt0 = 0; kt0 < ntiles; kt0 += T_CHUNK_TILES) {
+#pragma unroll 2
+      for (int u = 0; u < T_CHUNK_TILES; ++u) step(kt0 + u);
+      close_chunk();
+    }
+  } else {
+    for (int kt = 0; kt < ntiles; ++kt) {
+      step(kt);
+      if ((kt + 1) % T_CHUNK_TILES == 0 || kt + 1 == ntiles) close_chunk();
+    }
+  }
+  const int m0 = m_blk + wm * 16 * FM + r16, n0 = n_blk + wn * (SWIGLU ? 8 : 16) * FN + 4 * kg;
+#pragma unroll
+  for (int i = 0; i < (SWIGLU ? FN / 2 : FN); ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      f32x4 y = total[i][j];
+      if constexpr (SWIGLU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = (y[e] * (1.0f / (1.0f + expf(-y[e])))) * total[i + FN / 2][j][e];
+      }
+      store_out4(out, ldo, m0 + j * 16, n0 + i * 16, M, N, y, out_form);
+    }
+}
+
+template <int FM, int FN, int S, bool SWIGLU>
+static int launch_fine(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form, hipStream_t st) {
+  constexpr int COLS = SWIGLU ? 16 * FN : 32 * FN;
+  constexpr size_t smem = (size_t)S * 32 * (FM + FN) * T_ROWB;
+  static_assert(S >= 2 && S <= 4, "the waits count up to two tiles behind the next");
+  static bool configured = false;
+  if (!configured) {
+    (void)hipFuncSetAttribute((const void*)gemm_fine_kernel<FM, FN, S, SWIGLU, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    (void)hipFuncSetAttribute((const void*)gemm_fine_kernel<FM, FN, S, SWIGLU, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    configured = true;
+  }
+  const int row_blocks = (M + 32 * FM - 1) / (32 * FM);
+  const int64_t tiles = (int64_t)row_blocks * ((N + COLS - 1) / COLS);
+  VK_REQUIRE(tiles < (1 << 30), "gemm: too many rows (%d)", M);
+  if (K % KC == 0) gemm_fine_kernel<FM, FN, S, SWIGLU, true><<<(unsigned)tiles, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, row_blocks);
+  else gemm_fine_kernel<FM, FN, S, SWIGLU, false><<<(unsigned)tiles, 256, smem, st>>>(out, act, w, M, N, K, lda, ldo, form, row_blocks);
+  return vk_check_launch("gemm_fine");
+}
+static int gemm_fine(int fm, int fn, bool swiglu, elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int form,
+                     hipStream_t st) {
+#define FINE(FM, FN) if (fm == FM && fn == FN) return swiglu ? launch_fine<FM, FN, 2, true>(out, act, w, M, N, K, lda, ldo, form, st) : launch_fine<FM, FN, 2, false>(out, act, w, M, N, K, lda, ldo, form, st)
+  if (fm == 1 && fn == 1 && !swiglu) return launch_fine<1, 1, 3, false>(out, act, w, M, N, K, lda, ldo, form, st);
+  FINE(1, 2);
+  FINE(2, 2);
+  FINE(3, 2);
+  FINE(1, 4);
+  FINE(2, 4);
+#undef FINE
+  return vk_fail("gemm: no tile of %d by %d fragments", fm, fn);
+}
+
+// Which products go by these tiles.  Up to 64 rows the kernels that share activations through LDS are ahead where K is long: 64 rows, 1,024 x 1,024 17.4, 11.5 us,
+// 3,072 x 1,536 19.1, 16.5, 2,048 x 2,048 18.3, 20.2, 4,096 x 12,288 100, 128; with SwiGLU 6,144 x 2,048 64, 52, 12,288 x 4,096 175, 130; up to 32 rows
+// always (20 rows, 4,096 x 1,024 11.0, 11.2, 2,048 x 6,144 36.6, 59.3).
+static bool fine_takes(int M, int K, int64_t lda, bool swiglu) {
+  return K % (2 * VK_SLAB) == 0 && !rows_far(lda) && (M > 64 || (M > 32 && (swiglu ? K % KC == 0 : K <= 3 * KC)));
+}
+// The tile whose launch ends first: a unit's share is ceil(tiles / units) tiles, a tile's time is its products' (FM x FN fragments), and below a share that depends
+// on the tile a K tile's wait for memory.  ns for 32 elements of K and a product of fragments, fitted to 84 products of 70 to 2,048 rows, 256 x 1,024 to
+// 12,288 x 2,048: {at least, in front, a tile}.  The tile so chosen against the best of the six: 1 % slower on the mean, 12 % at most.
+static void fine_tile(int M, int N, bool swiglu, int& fm, int& fn) {
+  static const struct { int fm, fn; double least, front, each; } kinds[6] = {{2, 4, 140, 10, 121}, {3, 2, 147, 15, 121}, {2, 2, 160, 20, 124},
+                                                                               {1, 4, 175, 20, 129}, {1, 2, 250, 50, 134}, {1, 1, 320, 180, 142}};
+  double best = 0.0;
+  for (const auto& k : kinds) {
+    if (swiglu && k.fn == 1) continue;
+    const int columns = (swiglu ? 16 : 32) * k.fn;
+    const int64_t tiles = (int64_t)((M + 32 * k.fm - 1) / (32 * k.fm)) * ((N + columns - 1) / columns);
+    const double time = k.fm * k.fn * std::max(k.least, k.front + k.each * (double)((tiles + vk_device_cus() - 1) / vk_device_cus()));
+    if (best == 0.0 || time < best) { best = time; fm = k.fm; fn = k.fn; }
+  }
+}
+#endif
+
 #ifdef VK_BF16
 // ------------------------------------------------------------- alternating
 // Tiles of 256 activation rows and 32 FNW weight rows, eight waves, a workgroup a compute unit: 16-bit elements, K in whole chunks, at least
@@ -2261,7 +2442,7 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //              else                                            9   the streaming kernel would need a second pass for a few tiles
 //                                                                  (32 rows, 5120 x 17408: 111 -> 65 us)
 //   17..64   K not in whole chunks                             2 (rows > 32 and wg128 >= 0.5 cus), else 7 / 1 as above
-//   65..256  K whole chunks, wg128 < 0.5 cus:                      the kernel that shares activations through LDS, in blocks of 64 rows
+//   65..256  K whole chunks, wg128 < 0.5 cus, 16-bit:              the kernel that shares activations through LDS, in blocks of 64 rows
 //              16-bit, two blocks, K > 2 chunks,               9   so few weight rows that the tile kernel's workgroups of 64 leave three
 //                wg32 <= 0.5 cus                                     quarters of the units idle (128 rows, 4096 x 12288: 81 us against
 //                                                                  54; 1024 x 2048: 13.7 against 11.6)
@@ -2270,9 +2451,6 @@ static bool stream_rows_pay(int M, int weight_tiles, int64_t lda, int chunks = 0
 //                                                                  way; up to 112 rows and nine chunks 0.92 to 1.33 times, 1.09 on the mean)
 //              16-bit                                          2   the tile kernel in one round (pipe_fragments_in_one_round; 200 rows,
 //                                                                  6144 x 4096: 40 -> 27 us)
-//              32-bit, wg64 >= 0.5 cus                         8 up to three blocks, else 2
-//              32-bit, two blocks                              9 (wg32 <= 0.5 cus) or 8
-//              32-bit, else                                    2 (k_resident and wg16 >= 1.5 cus) or 8
 //   more                                                       2   the pipelined tile kernel, in one round where it can be
 //                                                                  (pipe_fragments_in_one_round), or the alternating one
 //                                                                  (alternate_fragments)
@@ -2293,15 +2471,9 @@ static int choose_gemm_kernel(int M, int N, int K) {
     return 9;
   }
   if (M <= 64) return (2 * wg128 >= cus && M > 32) ? 2 : (many16 ? 7 : 1);
-  if (M <= 256 && whole && 2 * wg128 < cus) {
-    const int blocks = (M + 63) / 64;
-    if (sizeof(elem_t) == 2) {
-      if (blocks == 2 && 2 * wg32 <= cus && K > 2 * KC) return 9;
-      return blocks == 2 && M > 112 && K >= 10 * KC && 2 * wg64 <= cus ? 8 : 2;
-    }
-    if (2 * wg64 >= cus) return blocks <= 3 ? 8 : 2;
-    if (blocks == 2) return 2 * wg32 <= cus ? 9 : 8;
-    return (k_resident && many16) ? 2 : 8;
+  if (sizeof(elem_t) == 2 && M <= 128 && whole && 2 * wg128 < cus) {
+    if (2 * wg32 <= cus && K > 2 * KC) return 9;
+    return M > 112 && K >= 10 * KC && 2 * wg64 <= cus ? 8 : 2;
   }
   return 2;
 }
@@ -2376,15 +2548,13 @@ static int pipe_fragments_by_rounds(int M, int N, double* rounds_of_128 = nullpt
 // (96 weight rows) 145 -> 114; 6,144 x 4,096, 300 rows 51 -> 33; 2,048 x 6,144, 651 rows 53 -> 36; 1,024 x 1,024, 65 to 1,024 rows 9.7 to 10.7 -> 8.6;
 // with SwiGLU 9,728 x 2,560, 100 rows 47 -> 34; grouped, 2,048 x 2,048, 16 blocks 37 -> 27.  556 plain sizes of 65 to 2,048 rows (N of 1,024 to
 // 16,384, K of 1,024 to 12,288) 25.8 -> 19.6 ms (three of them 3 to 5 % slower: 128 rows, 5,120 to 8,192 x 6,144), 102 with SwiGLU 3.21 -> 2.73.
-// Three stages are 5 % slower with 64 weight rows and as fast with 96 and 128, five and six are slower.  32-bit elements are bound by the matrix unit:
-// 96 weight rows 4.02 -> 3.29 ms over 27 sizes, the others within 2 %.
+// Three stages are 5 % slower with 64 weight rows and as fast with 96 and 128, five and six are slower.
 static int pipe_fragments_in_one_round(int M, int N, int K) {
   const int64_t mb = (M + 127) / 128;
-  // 32-bit elements and K not in whole chunks: two stages are 5 % faster (96 rows, 5,840 x 1,280 49.3 -> 46.9 us; 72 of 72 sizes of 65 to 300 rows).
-  if ((N + 63) / 64 * mb <= vk_device_cus()) return sizeof(elem_t) == 4 && K % KC != 0 ? 0 : 2;
+  if ((N + 63) / 64 * mb <= vk_device_cus()) return 2;
   if ((N + 95) / 96 * mb <= vk_device_cus()) return 3;
-  // 32-bit elements, K of up to two chunks, and K not in whole chunks are as fast with two workgroups of 64 rows a unit (two stages).
-  if (sizeof(elem_t) == 2 && K % KC == 0 && K > 2 * KC && (N + 127) / 128 * mb <= vk_device_cus()) return 4;
+  // K of up to two chunks and K not in whole chunks are as fast with two workgroups of 64 rows a unit (two stages).
+  if (K % KC == 0 && K > 2 * KC && (N + 127) / 128 * mb <= vk_device_cus()) return 4;
   return 0;
 }
 
@@ -2538,6 +2708,13 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   if (M == 0) return 0;
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
+#ifdef VK_F32
+  if (kernel == 0 && fine_takes(M, K, lda, false)) {
+    int fm = 0, fn = 0;
+    fine_tile(M, N, false, fm, fn);
+    return gemm_fine(fm, fn, false, out, act, w, M, N, K, lda, ldo, form, st);
+  }
+#endif
   if (kernel == 0) {
 #ifdef VK_BF16
     const int width = rows_width(M, N, K, lda, false);
@@ -2710,6 +2887,19 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   return launch_tiled<4, 4>(out, act, w, M, N, K, lda, ldo, form, st);
 }
 
+// A product of 32-bit elements by tiles of 32 fm x 32 fn (0, 0: the ones chosen by size), for measurements and tests.
+int vk_gemm_fine(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo, int fm, int fn, int swiglu, hipStream_t st) {
+  VK_REQUIRE(sizeof(elem_t) == 4 && M > 0 && N > 0 && K > 0 && K % (2 * VK_SLAB) == 0 && lda >= K && lda % VK_VEC == 0 && !rows_far(lda) && ldo >= N,
+             "gemm: bad sizes M=%d N=%d K=%d for tiles of 32-bit elements", M, N, K);
+  VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm: operands must be 16-byte aligned");
+#ifdef VK_F32
+  if (fm == 0) fine_tile(M, N, swiglu != 0, fm, fn);
+  return gemm_fine(fm, fn, swiglu != 0, out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, 0), st);
+#else
+  return 1;
+#endif
+}
+
 int vk_gemm(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, int K, int64_t lda, int64_t ldo,
             int kernel, hipStream_t st) {
   return gemm_launch(out, act, w, M, N, K, lda, ldo, kernel, 0, st);
@@ -2748,13 +2938,20 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
     if (f == 4) return launch_alternate<4, 3, 4, true>(out, act, w, M, I, K, lda, ldo, ok4, st);
   }
 #endif
+#ifdef VK_F32
+  if (fine_takes(M, K, lda, true)) {
+    int fm = 0, fn = 0;
+    fine_tile(M, I, true, fm, fn);
+    return gemm_fine(fm, fn, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+  }
+#endif
   if (how == 2 && rows_far(lda)) {
     VK_REQUIRE(K % KC == 0, "gemm_swiglu: rows %lld elements apart need K in whole chunks of %d", (long long)lda, KC);
     return launch_mid<4, 1, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
   }
+#ifdef VK_BF16
   if (how == 2)
     return launch_pipe<2, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
-#ifdef VK_BF16
   if (const int width = how == 3 ? rows_width(M, I, K, lda, true) : 0)
     return gemm_rows(width, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
 #endif
