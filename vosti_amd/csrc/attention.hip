@@ -109,6 +109,23 @@ __device__ __forceinline__ int first_visible(const AttnArgs& a, int pos) {
   return a.window > 0 ? max(0, pos - a.window + 1) : 0;
 }
 
+// Over the lanes l, l ^ 16, l ^ 32 and l ^ 48, which hold a row's numbers: (v + v of l ^ 16), and that + the same of l ^ 32, in every lane.
+__device__ __forceinline__ float row_sum(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  v = pair_sum(__builtin_amdgcn_permlane16_swap(u, u, false, false));
+  const unsigned w = __builtin_bit_cast(unsigned, v);
+  return pair_sum(__builtin_amdgcn_permlane32_swap(w, w, false, false));
+}
+__device__ __forceinline__ float row_max(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned a = r[0], b = r[1];
+  const unsigned w = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)));
+  const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  const unsigned c = q[0], e = q[1];
+  return fmaxf(__builtin_bit_cast(float, c), __builtin_bit_cast(float, e));
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // What a wave needs to know about its 16 rows and its sequence's pages.
@@ -147,8 +164,7 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
     float tmax = sc[0];
 #pragma unroll
     for (int i = 1; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
-    tmax = fmaxf(tmax, lane_xor16(tmax));
-    tmax = fmaxf(tmax, lane_xor32(tmax));
+    tmax = row_max(tmax);
     const float m = tmax * scale_log2;
     Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
     ca = fast_exp2(M - Mn);                 // 1 where the maximum stands, 0 for a row whose state was empty
@@ -163,11 +179,10 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
       const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
-      vis[i] = row_ok && key >= lo && key <= pos;
+      vis[i] = (int)row_ok & (int)(key >= lo) & (int)(key <= pos);
       tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
     }
-    tmax = fmaxf(tmax, lane_xor16(tmax));
-    tmax = fmaxf(tmax, lane_xor32(tmax));
+    tmax = row_max(tmax);
     const float m = tmax * scale_log2;      // -inf: the row sees no key of the tile
     Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
     ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
@@ -177,8 +192,7 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
       psum = psum + pr[i];
     }
   }
-  psum = psum + lane_xor16(psum);
-  psum = psum + lane_xor32(psum);
+  psum = row_sum(psum);
   L = __builtin_fmaf(L, ca, psum);
   M = Mn;
 #pragma unroll
@@ -456,30 +470,39 @@ __device__ __forceinline__ void natural_scores(float (&sc)[S_PER_LANE], float sc
 }
 
 // tile_probs for scores in natural units (already scaled and capped), with kept first keys and unrounded weights.
-__device__ __forceinline__ void tile_probs_ext(float (&sc)[S_PER_LANE], int kb, int g, bool row_ok, int lo, int pos, int keep,
+__device__ __forceinline__ void tile_probs_ext(float (&sc)[S_PER_LANE], int kb, int g, bool row_ok, int lo, int pos, int keep, bool full,
                                                float& M, float& L, float& ca, frag_t (&pf)[P_PARTS][KEY_SLABS]) {
   float pr[S_PER_LANE];
   float psum = 0.f;
-  bool vis[S_PER_LANE];
+  // The numbers of a lane's visible keys, a bit each; all of them where every row of the wave sees every key.  (Masks written as
+  // conditions become branches, seven hundred instructions of a tile's thousand.)
+  unsigned vis = ~0u;
+  if (!full) {
+    vis = 0;
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) {
+      const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
+      vis |= (unsigned)((int)row_ok & (int)(key <= pos) & ((int)(key >= lo) | (int)(key < keep))) << i;
+    }
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) sc[i] = vis >> i & 1u ? sc[i] : -INFINITY;
+  }
   float tmax = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < S_PER_LANE; ++i) {
-    const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
-    vis[i] = row_ok && key <= pos && (key >= lo || key < keep);
-    tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
-  }
-  tmax = fmaxf(tmax, lane_xor16(tmax));
-  tmax = fmaxf(tmax, lane_xor32(tmax));
+  for (int i = 0; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
+  tmax = row_max(tmax);
   const float m = tmax * LOG2E;             // -inf: the row sees no key of the tile
   const float Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
   ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
 #pragma unroll
-  for (int i = 0; i < S_PER_LANE; ++i) {
-    pr[i] = vis[i] ? fast_exp2(__builtin_fmaf(sc[i], LOG2E, -Mn)) : 0.f;
-    psum = psum + pr[i];
+  for (int i = 0; i < S_PER_LANE; ++i) pr[i] = fast_exp2(__builtin_fmaf(sc[i], LOG2E, -Mn));
+  if (!full) {
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) pr[i] = vis >> i & 1u ? pr[i] : 0.f;
   }
-  psum = psum + lane_xor16(psum);
-  psum = psum + lane_xor32(psum);
+#pragma unroll
+  for (int i = 0; i < S_PER_LANE; ++i) psum = psum + pr[i];
+  psum = row_sum(psum);
   L = __builtin_fmaf(L, ca, psum);
   M = Mn;
 #pragma unroll
@@ -513,7 +536,7 @@ __device__ __forceinline__ void tile_softmax_pv_ext(const RowCtx& c, float scale
   frag_t pf[P_PARTS][KEY_SLABS];
   float ca;
   const bool fresh = !(M > -INFINITY);
-  tile_probs_ext(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.keep, M, L, ca, pf);
+  tile_probs_ext(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.keep, false, M, L, ca, pf);
   scale_state<NDT>(ACC, ca, fresh);
   if (kb + TILE_KEYS > c.k_len || kb < c.wave_lo) {
 #pragma unroll
@@ -611,6 +634,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a, int heads
 // of the two waves of a SIMD the one that feeds the matrix unit goes first and the
 // other's vector instructions fill in.  The arithmetic per row is tile_step's and
 // fold's, operation for operation.
+//
+// What bounds it: eight waves share a tile of 32 KB (heads of 128) and a barrier, two a SIMD, so that each wait of a step is seen by all.  The page of the next tile was read
+// in front of its loads, and the variant's masks were branches, in every tile: measured on MI355X in recorded launches, before and after a page read a tile ahead, masks as numbers, none
+// where a wave sees a whole tile, and lanes' sums and maxima without selects, us: 32 heads of 128 on 8, one prompt of 2,048 tokens 70.1 -> 66.2; with a window of
+// 1,024 and sinks 140 -> 87, scores capped 151 -> 100; 3 prompts of 1,111 to 520, capped 115 -> 86; 32 heads on one of 256 144 -> 113; heads of 64, 2 x 1,024, capped 42 -> 29.
+// (The variant with four waves and one buffer, three workgroups a unit: 8 % faster at one prompt of 2,048, 10 to 15 % slower at 8 of 256 and 24 of 100.)
 //
 // LDS holds the key tile as [64 keys][d] and the value tile as [d][64 keys],
 // in 16-byte columns that are XOR-swizzled by row so that the 16 lanes of a
@@ -724,10 +753,13 @@ __global__ __launch_bounds__(64 * NW, EXT ? 1 : 2) void attn_prefill_lds_kernel(
     const int vcol = (lane % CV) ^ val_swz(vrow);
     voff[j] = vrow * a.P + vcol * VK_VEC;
   }
+  // The page of the tile that is asked for next: it is read a tile ahead, beside that tile's keys and values, so that no step waits for it.
+  int next_page = 0;
+  auto ask_page = [&](int i) { next_page = bt[tile_of(min(i, n_tiles - 1)) * TILE_KEYS >> lp]; };
   auto issue = [&](int t, int stage) {
     const int kb = t * TILE_KEYS;
     // The page number is the same for the wave: as a scalar, its arithmetic stays off the vector unit.
-    const int64_t page = (int64_t)__builtin_amdgcn_readfirstlane(bt[kb >> lp]) * page_stride;
+    const int64_t page = (int64_t)__builtin_amdgcn_readfirstlane(next_page) * page_stride;
     const int in_page = kb & (a.P - 1);
     const elem_t* kt = kbase + page + (int64_t)in_page * DPAD;
     const elem_t* vt = vbase + page + in_page;
@@ -744,7 +776,9 @@ __global__ __launch_bounds__(64 * NW, EXT ? 1 : 2) void attn_prefill_lds_kernel(
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) ACC[dt] = As[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  ask_page(0);
   issue(tile_of(0), 0);
+  ask_page(1);
   // The buffer a tile lies in is a constant in the code of its step (the loop below takes two steps a turn), so that
   // the LDS addresses of the fragments are computed once for the kernel and not added to a buffer's base in every tile.
   auto step = [&](int i, auto stage_c) {
@@ -753,7 +787,10 @@ __global__ __launch_bounds__(64 * NW, EXT ? 1 : 2) void attn_prefill_lds_kernel(
     const bool last = i + 1 == n_tiles;
     wait_vm_loads();
     __syncthreads();      // tile t is in LDS; every wave is done with the other buffer
-    if (NST == 2 && !last) issue(tile_of(i + 1), stage ^ 1);
+    if (NST == 2 && !last) {
+      issue(tile_of(i + 1), stage ^ 1);
+      ask_page(i + 2);
+    }
     if (t * TILE_KEYS + TILE_KEYS > k_len || (t * TILE_KEYS < item_lo && t * TILE_KEYS + TILE_KEYS > keep)) {
       // Keys outside [item_lo, k_len) may lie in pages this sequence does not own: their values are replaced by
       // zero in LDS, so that stale NaN or Inf cannot reach a sum (their probabilities are zero).  The first and
@@ -798,13 +835,13 @@ __global__ __launch_bounds__(64 * NW, EXT ? 1 : 2) void attn_prefill_lds_kernel(
       __builtin_amdgcn_sched_barrier(0);
       // ---- the row's new maximum, its probabilities, its sums so far under the new maximum ----
       const bool full = rows_wave >= 16 && kb + TILE_KEYS - 1 <= pos_wave &&
-                        kb >= (first_visible(a, pos_wave + 15));
+                        (kb >= first_visible(a, pos_wave + 15) || (EXT && kb + TILE_KEYS <= keep));
       frag_t pf[EXT ? P_PARTS : 1][KEY_SLABS];
       float ca;
       const bool fresh = !(Ms > -INFINITY);
       if constexpr (EXT) {
         natural_scores<REL>(sc, a.scale, a.softcap, rb);
-        tile_probs_ext(sc, kb, g, row_ok, lo, pos, keep, Ms, Ls, ca, pf);
+        tile_probs_ext(sc, kb, g, row_ok, lo, pos, keep, full, Ms, Ls, ca, pf);
       } else {
         tile_probs(sc, kb, g, row_ok, lo, pos, a.scale_log2, full, Ms, Ls, ca, pf[0]);
       }
@@ -853,6 +890,7 @@ __global__ __launch_bounds__(64 * NW, EXT ? 1 : 2) void attn_prefill_lds_kernel(
     if (NST == 1 && !last) {                               // one buffer: the next tile may come when every wave has read this one
       __syncthreads();
       issue(tile_of(i + 1), 0);
+      ask_page(i + 2);
     }
     if (last || tile_of(i + 1) / SEG_TILES != t / SEG_TILES) {   // the segment is complete
       fold<NDT>(M, L, ACC, Ms, Ls, As);
@@ -1207,8 +1245,7 @@ struct HeadRow {
         float part = 0.f;
 #pragma unroll
         for (int e = 0; e < VK_VEC; ++e) part = part + v[s][e] * v[s][e];
-        part = part + lane_xor16(part);
-        quad[s] = part + lane_xor32(part);
+        quad[s] = row_sum(part);
       }
 #pragma unroll
       for (int step = 1; step < NQS; step *= 2)
@@ -1411,11 +1448,10 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
       const int key = kb + (i / VK_VEC) * VK_SLAB + c.g * VK_VEC + (i % VK_VEC);
-      vis[i] = c.row_ok && key <= pos && (key >= lo || key < keep);
+      vis[i] = (int)c.row_ok & (int)(key <= pos) & ((int)(key >= lo) | (int)(key < keep));      // (as conditions they become branches)
       tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
     }
-    tmax = fmaxf(tmax, lane_xor16(tmax));
-    tmax = fmaxf(tmax, lane_xor32(tmax));
+    tmax = row_max(tmax);
   }
   if (c.g == 0) tile_max[wave][c.r16] = tmax;
   __syncthreads();
@@ -1446,8 +1482,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
         pf[2][i / VK_VEC][i % VK_VEC] = (elem_t)(r1 - (float)mid);
       }
     }
-    psum = psum + lane_xor16(psum);
-    psum = psum + lane_xor32(psum);
+    psum = row_sum(psum);
     if (c.g == 0) tile_sum[wave][c.r16] = psum;
 #pragma unroll
     for (int part = 0; part < NP; ++part)
@@ -1686,7 +1721,9 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
     // 83 -> 74; from two workgroups per unit on eight waves win by 2 to 8 %).  Two row tiles per wave would
     // halve the LDS traffic but need more than the 256 registers that two waves per SIMD leave: with spills
     // or with one wave per SIMD they measured 40 % slower.
-    const int v = (vk_prefill_variant == 14 || (vk_prefill_variant == 0 && 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus())) ? 14 : 0;
+    // Heads of 256 in 16-bit, whose tiles of 64 KB are a wave's longest wait, always eight (150 rows 16.3 -> 14.3 us, 1,024 61 -> 52).
+    const bool few = 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus() && (d < 256 || sizeof(elem_t) == 4);
+    const int v = (vk_prefill_variant == 14 || (vk_prefill_variant == 0 && few)) ? 14 : 0;
     // With many workgroups (two rounds or more of the three four-wave workgroups that a compute unit holds when
     // each has one buffer of 32 KB) the occupancy is worth more than loads that overlap a workgroup's own work:
     // 12 waves a unit instead of 8 (2 prompts of 2,048 tokens: 140 -> 121 us; 8,192 tokens: 890 -> 718, with 64
@@ -1905,8 +1942,9 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
     attn_prefill_lds_kernel<DP, NW, 2, true, REL><<<n_items * (ITEM_ROWS / (16 * NW)) * nq, 64 * NW, smem, st>>>(a, n_items); \
   } while (0)
 #define PREFILL_LDS_EXT(DP, NW) do { if (rel != nullptr) PREFILL_LDS_EXT_OF(DP, NW, true); else PREFILL_LDS_EXT_OF(DP, NW, false); } while (0)
-    // (In 32-bit with the widest heads eight waves' registers do not hold the three-part products' operands.)
-    const bool four = 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus() || (sizeof(elem_t) == 4 && d == 256);
+    // Not with heads of 256, whose tiles of 64 KB are a wave's longest wait (eight waves against four, us, 32 heads on one kv head: 1 prompt of 150 tokens 19.6 -> 17.0,
+    // 1,024 75.6 -> 51.6 with a window of 512 and 75.4 -> 74.3 without, 4 of 150 31.8 -> 17.7); but in 32-bit eight waves' registers do not hold their operands.
+    const bool four = d == 256 ? sizeof(elem_t) == 4 : 2 * (int64_t)n_items * nq < 3 * (int64_t)vk_device_cus();
     if (d == 64) { if (four) PREFILL_LDS_EXT(64, 4); else PREFILL_LDS_EXT(64, 8); }
     else if (d == 128) { if (four) PREFILL_LDS_EXT(128, 4); else PREFILL_LDS_EXT(128, 8); }
     else { if (four) PREFILL_LDS_EXT(256, 4); else PREFILL_LDS_EXT(256, 8); }
