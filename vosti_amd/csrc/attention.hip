@@ -78,9 +78,23 @@ struct AttnArgs {
   // A bias by distance on the scores (see "A bias by distance" below) and a gate on a head's output.
   const float* rel = nullptr;         // [nq, rel_stride] or null: head h's bias for the distance n is rel[h * rel_stride + rel_zero - n]
   int rel_stride = 0, rel_zero = 0, rel_far = 0;   // from the distance rel_far on it is what it is at rel_far
+  int group = 0, head_tiles = 0;      // decode: nq / nkv, and tiles of 16 of them (a division in the kernel stands in front of its first loads)
   const elem_t* gate = nullptr;       // [T, gate_stride] or null: head h's output is multiplied by the logistic function of gate[token, h]
   int64_t gate_stride = 0;
 };
+
+// Row and sequence of a decoded item; the row stands `back` places before the sequence's end.  Without items (a.items null) row i is all that sequence
+// i brings: nothing has to be read for it, where an item's numbers and those of its sequence are two reads that everything after them waits for (0.4 us each
+// of a launch of five to nine).
+__device__ __forceinline__ void decoded_row(const AttnArgs& a, int item, int& seq, int& tok, int& back) {
+  seq = tok = item;
+  back = 1;
+  if (a.items != nullptr) {
+    seq = a.items[2 * item];
+    tok = a.cu_q[seq] + a.items[2 * item + 1];
+    back = a.cu_q[seq + 1] - tok;
+  }
+}
 
 // Decoded rows as the projections leave them: what vk_qkv_post does to them (head norm, rotation by tables, the store of key and value) happens in the
 // attention's own launch.
@@ -224,15 +238,40 @@ __device__ __forceinline__ void scale_state(f32x4 (&ACC)[NDT], float ca, bool fr
 // Keys outside [first, k_len) may lie in pages this sequence does not own
 // (never written, or given back once the window passed them): their values
 // are replaced by zero so that stale NaN or Inf cannot reach the sum.
-__device__ __forceinline__ void zero_unowned(frag_t (&vf)[KEY_SLABS], int kb, int g, int first, int k_len, int keep = 0) {
+// The keys of a lane's vectors as masks of bits, made once for all column blocks: a compare and a select an element, and putting 16-bit
+// elements back together, took hundreds of instructions a tile in decoded attention's longest wave, four to five cycles each.
+constexpr int VEC_DWORDS = 4;
+struct OwnedMask {
+  u32x4 bits[KEY_SLABS];
+  // All ones in a vector's elements in front of `end`, counted from its first.  (Compares would become one chain of scalar operations an element.)
+  __device__ static __forceinline__ u32x4 before(int end) {
+    constexpr int PER = VK_VEC / VEC_DWORDS;                 // elements of a dword
+    u32x4 m;
 #pragma unroll
-  for (int ks = 0; ks < KEY_SLABS; ++ks) {
-    const int k0 = kb + ks * VK_SLAB + g * VK_VEC;
-#pragma unroll
-    for (int j = 0; j < VK_VEC; ++j)
-      if (k0 + j >= k_len || (k0 + j < first && k0 + j >= keep)) vf[ks][j] = (elem_t)0.f;
+    for (int i = 0; i < VEC_DWORDS; ++i) {
+      const int out = (16 / PER) * (PER - min(max(end - i * PER, 0), PER));        // half the bits that are not in front
+      m[i] = (~0u >> out) >> out;
+    }
+    return m;
   }
-}
+  __device__ __forceinline__ OwnedMask(int kb, int g, int first, int k_len, int keep) {
+#pragma unroll
+    for (int ks = 0; ks < KEY_SLABS; ++ks) {
+      const int k0 = kb + ks * VK_SLAB + g * VK_VEC;
+      bits[ks] = before(k_len - k0);
+      if (kb < first) bits[ks] &= ~before(first - k0) | before(keep - k0);
+    }
+  }
+  template <int NDT>
+  __device__ __forceinline__ void apply(frag_t (&vf)[NDT][KEY_SLABS], int blocks = NDT) const {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+      if (dt < blocks) {
+#pragma unroll
+        for (int ks = 0; ks < KEY_SLABS; ++ks) vf[dt][ks] = __builtin_bit_cast(frag_t, __builtin_bit_cast(u32x4, vf[dt][ks]) & bits[ks]);
+      }
+  }
+};
 
 // The pieces of a tile's work, for the kernels that read fragments straight from global memory.
 // No load is predicated on data: addresses of keys beyond k_len are clamped to a key of this
@@ -243,15 +282,16 @@ constexpr int KSUB = S_PER_LANE / 4;    // 16-key MFMA sub-tiles per tile
 // Key fragments of the whole tile, all in flight together.
 // EXACT (here and below): the head size is the padded one and a page holds a tile or more, known
 // at compile time, so that no branch on either is left in the code.
-// page: the tile's page where the caller has read it from the table already, else -1.
-template <int NQS, bool EXACT>
-__device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[KSUB][NQS], int page = -1) {
+// PAGE: the caller has read the tile's page from the table already (a tile in one page).  (A page that says by its sign whether it was read leaves a
+// second read in the code, and in front of every tile's loads a wait for the ones before.)
+template <int NQS, bool EXACT, bool PAGE = false>
+__device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[KSUB][NQS], int page = 0) {
   const int d = EXACT ? NQS * VK_SLAB : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const bool dfull = EXACT || d % VK_SLAB == 0;    // else the last slab along d is partly outside the head
   const int last_key = c.k_len - 1;
   // With pages of at least a tile, the tile lies in one page: one table lookup for the wave.
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* kpage = c.kbase + (one_page ? (int64_t)(page >= 0 ? page : c.bt[kb >> lp]) * c.page_stride : 0);
+  const elem_t* kpage = c.kbase + (one_page ? (int64_t)(PAGE ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int sub = 0; sub < KSUB; ++sub) {
 #ifdef VK_BF16
@@ -273,12 +313,12 @@ __device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[
   }
 }
 
-template <int NDT, bool EXACT>
-__device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf)[NDT][KEY_SLABS], int page = -1) {
+template <int NDT, bool EXACT, bool PAGE = false>
+__device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf)[NDT][KEY_SLABS], int page = 0) {
   const int d = EXACT ? NDT * 16 : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const int last_key = c.k_len - 1;
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* vpage = c.vbase + (one_page ? (int64_t)(page >= 0 ? page : c.bt[kb >> lp]) * c.page_stride : 0);
+  const elem_t* vpage = c.vbase + (one_page ? (int64_t)(PAGE ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
     if (dt * 16 < d) {
@@ -299,16 +339,21 @@ template <int NQS, bool EXACT>
 __device__ __forceinline__ void tile_scores(const RowCtx& c, const frag_t (&kf)[KSUB][NQS], const frag_t (&qf)[NQS],
                                             float (&sc)[S_PER_LANE]) {
   const int d = EXACT ? NQS * VK_SLAB : c.d;
+  f32x4 s4[KSUB];
+#pragma unroll
+  for (int sub = 0; sub < KSUB; ++sub) s4[sub] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < NQS; ++s)             // the sub-tiles side by side: no product waits for the one before it
+    if (s * VK_SLAB < d) {
+#pragma unroll
+      for (int sub = 0; sub < KSUB; ++sub) s4[sub] = mma_slab(kf[sub][s], qf[s], s4[sub]);
+    }
 #pragma unroll
   for (int sub = 0; sub < KSUB; ++sub) {
-    f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < NQS; ++s)
-      if (s * VK_SLAB < d) s4 = mma_slab(kf[sub][s], qf[s], s4);
-    sc[4 * sub + 0] = s4.x;
-    sc[4 * sub + 1] = s4.y;
-    sc[4 * sub + 2] = s4.z;
-    sc[4 * sub + 3] = s4.w;
+    sc[4 * sub + 0] = s4[sub].x;
+    sc[4 * sub + 1] = s4[sub].y;
+    sc[4 * sub + 2] = s4[sub].z;
+    sc[4 * sub + 3] = s4[sub].w;
   }
 }
 
@@ -318,9 +363,7 @@ __device__ __forceinline__ void tile_pv(const RowCtx& c, int kb, frag_t (&vf)[ND
                                         f32x4 (&ACC)[NDT]) {
   const int d = EXACT ? NDT * 16 : c.d;
   if (kb + TILE_KEYS > c.k_len || kb < c.wave_lo) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      if (dt * 16 < d) zero_unowned(vf[dt], kb, c.g, c.wave_lo, c.k_len);
+    OwnedMask(kb, c.g, c.wave_lo, c.k_len, 0).apply(vf, (d + 15) / 16);
   }
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
@@ -539,9 +582,7 @@ __device__ __forceinline__ void tile_softmax_pv_ext(const RowCtx& c, float scale
   tile_probs_ext(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.keep, false, M, L, ca, pf);
   scale_state<NDT>(ACC, ca, fresh);
   if (kb + TILE_KEYS > c.k_len || kb < c.wave_lo) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      if (dt * 16 < c.d) zero_unowned(vf[dt], kb, c.g, c.wave_lo, c.k_len, c.keep);
+    OwnedMask(kb, c.g, c.wave_lo, c.k_len, c.keep).apply(vf, (c.d + 15) / 16);
   }
   // A sum takes its products in the order (key slab, part).  (Walking several column blocks side by side, so that no MFMA
   // follows one it depends on, costs the decode kernels more registers than a wave has: they spill.)
@@ -931,11 +972,9 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_plain_kernel(Att
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
   const int seg = blockIdx.z * PLAIN_WAVES + wave;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
+  int seq, tok, back;
+  decoded_row(a, blockIdx.x, seq, tok, back);
+  const int k_len = a.k_len[seq], pos = k_len - back;
   const int lo = first_visible(a, pos);
   const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
   if (t0 > t1) return;   // whole wave; no barrier follows
@@ -983,11 +1022,9 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
   const int seg = blockIdx.z * SEG_WAVES + wave;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
+  int seq, tok, back;
+  decoded_row(a, blockIdx.x, seq, tok, back);
+  const int k_len = a.k_len[seq], pos = k_len - back;
   const int lo = first_visible(a, pos);
   const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
   if (t0 > t1) return;   // whole wave; no barrier follows
@@ -1165,11 +1202,9 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
   const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
   const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
   const int seg = blockIdx.z * PLAIN_WAVES + wave;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
+  int seq, tok, back;
+  decoded_row(a, blockIdx.x, seq, tok, back);
+  const int k_len = a.k_len[seq], pos = k_len - back;
   const int lo = first_visible(a, pos);
   const int keep = a.window > 0 ? a.keep : 0;
   const int keep_tiles = (keep + TILE_KEYS - 1) / TILE_KEYS, tile_lo = lo / TILE_KEYS;
@@ -1209,67 +1244,67 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 }
 #endif
 
-// A head's row as an operand of the matrix unit: lane (r16, g) holds the elements s * VK_SLAB + g * VK_VEC ... of its row, its norm and its rotation by
-// qkv_post_vec_kernel's operations in that kernel's order (there a lane holds 16 bytes and the sums go over neighbouring lanes; here the four lanes g
-// of a row come first and a lane's slabs after them: the same tree).
-template <int NQS>
-struct HeadRow {
-  frag_t x[NQS], w[NQS];
-  struct Angles {
-    frag_t cs[NQS / 2], sn[NQS / 2];
-    __device__ __forceinline__ void load(const elem_t* cosines, const elem_t* sines, int g) {
-#pragma unroll
-      for (int s = 0; s < NQS / 2; ++s) {
-        cs[s] = *reinterpret_cast<const frag_t*>(cosines + s * VK_SLAB + g * VK_VEC);
-        sn[s] = *reinterpret_cast<const frag_t*>(sines + s * VK_SLAB + g * VK_VEC);
-      }
-    }
-  };
-  __device__ __forceinline__ void load(const elem_t* row, const elem_t* weight, int g) {
-#pragma unroll
-    for (int s = 0; s < NQS; ++s) {
-      x[s] = *reinterpret_cast<const frag_t*>(row + s * VK_SLAB + g * VK_VEC);
-      if (weight != nullptr) w[s] = *reinterpret_cast<const frag_t*>(weight + s * VK_SLAB + g * VK_VEC);
-    }
+// A lane's piece of a projected row, VK_VEC elements; the lanes of a row sit side by side as in qkv_post_vec_kernel, whose operations, in that
+// kernel's order, norm and turn it.
+template <int DPAD>
+struct RowPiece {
+  static constexpr int LANES = DPAD / VK_VEC;                // of a row
+  frag_t x, w;
+  __device__ __forceinline__ void load(const elem_t* row, uint64_t weight, int j) {
+    x = *reinterpret_cast<const frag_t*>(row + j * VK_VEC);
+    if (weight != 0) w = *((const __attribute__((address_space(1))) frag_t*)weight + j);
   }
-  __device__ __forceinline__ void finish(bool norm, bool turn, const Angles& angles, float eps, frag_t (&out)[NQS]) const {
-    float v[NQS][VK_VEC];
+  __device__ __forceinline__ frag_t finish(bool any_norm, bool norm, bool turn, const frag_t& cosines, const frag_t& sines, float eps, int j) const {
+    float v[VK_VEC];
 #pragma unroll
-    for (int s = 0; s < NQS; ++s)
+    for (int e = 0; e < VK_VEC; ++e) v[e] = to_f32(x[e]);
+    if (any_norm) {
+      float part = 0.f;
 #pragma unroll
-      for (int e = 0; e < VK_VEC; ++e) v[s][e] = to_f32(x[s][e]);
-    if (norm) {
-      float quad[NQS];
+      for (int e = 0; e < VK_VEC; ++e) part = part + v[e] * v[e];
+      part = group_sum<LANES>(part);
+      const float rr = rsqrtf(part / (float)DPAD + eps);
 #pragma unroll
-      for (int s = 0; s < NQS; ++s) {
-        float part = 0.f;
-#pragma unroll
-        for (int e = 0; e < VK_VEC; ++e) part = part + v[s][e] * v[s][e];
-        quad[s] = row_sum(part);
-      }
-#pragma unroll
-      for (int step = 1; step < NQS; step *= 2)
-#pragma unroll
-        for (int s = 0; s < NQS; s += 2 * step) quad[s] = quad[s] + quad[s + step];
-      const float rr = rsqrtf(quad[0] / (float)(NQS * VK_SLAB) + eps);
-#pragma unroll
-      for (int s = 0; s < NQS; ++s)
-#pragma unroll
-        for (int e = 0; e < VK_VEC; ++e) v[s][e] = round_to_elem((v[s][e] * rr) * to_f32(w[s][e]));
+      for (int e = 0; e < VK_VEC; ++e) v[e] = norm ? round_to_elem((v[e] * rr) * to_f32(w[e])) : v[e];
     }
+    frag_t out;
+    if (turn) {
+      // The partner's elements are of the element type: whole dwords change places.
+      frag_t mine;
 #pragma unroll
-    for (int s = 0; s < NQS; ++s)
+      for (int e = 0; e < VK_VEC; ++e) mine[e] = from_f32<elem_t>(v[e]);
+      const u32x4 bits = __builtin_bit_cast(u32x4, mine);
+      u32x4 theirs;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned u = bits[i];
+        theirs[i] = LANES == 16 ? (unsigned)__builtin_amdgcn_mov_dpp((int)u, 0x128, 0xF, 0xF, true)      // row_ror:8
+                                : (unsigned)__shfl_xor((int)u, LANES / 2, VK_WAVE);
+      }
+      const frag_t other = __builtin_bit_cast(frag_t, theirs);
+      const unsigned flip = j < LANES / 2 ? 0x80000000u : 0u;                                            // the first half subtracts
 #pragma unroll
       for (int e = 0; e < VK_VEC; ++e) {
-        float y = v[s][e];
-        if (turn) {
-          const float other = v[s ^ (NQS / 2)][e], c = to_f32(angles.cs[s % (NQS / 2)][e]), n = to_f32(angles.sn[s % (NQS / 2)][e]);
-          y = s < NQS / 2 ? y * c - other * n : y * c + other * n;
-        }
-        out[s][e] = from_f32<elem_t>(y);
+        const float t = to_f32(other[e]) * to_f32(sines[e]);
+        v[e] = v[e] * to_f32(cosines[e]) + __builtin_bit_cast(float, __builtin_bit_cast(unsigned, t) ^ flip);
       }
+    }
+#pragma unroll
+    for (int e = 0; e < VK_VEC; ++e) out[e] = from_f32<elem_t>(v[e]);
+    return out;
   }
 };
+
+// The bits of a lane's scores (score i is key (i / VK_VEC) * VK_SLAB + i % VK_VEC from its first) whose keys lie in front of `end`, counted from its first key.
+__device__ __forceinline__ unsigned keys_before(int end) {
+  unsigned bits = 0;
+#pragma unroll
+  for (int ks = 0; ks < KEY_SLABS; ++ks) {
+    const int n = min(max(end - ks * VK_SLAB, 0), VK_VEC);
+    bits |= ((1u << n) - 1u) << (ks * VK_VEC);
+  }
+  return bits;
+}
 
 // Decoded tokens, four waves a segment, for the plain attention and (EXT) the variant.  Wave j computes the scores of the
 // segment's tile j; the tiles' maxima pass through LDS, so that every wave knows how the rows' reference maximum moves from tile to
@@ -1280,9 +1315,12 @@ struct HeadRow {
 // (a page that turns out not to be needed is read and not used), and the four tiles' scores are computed side by side.
 // SEGS 2: a workgroup of eight waves takes both segments of a launch that has no more than two, folds them as attn_combine_kernel
 // does and writes the output: a launch less, where a launch that waits for the one before is a third of the two.
-// ROWS (the plain attention, EXACT): the step's rows come as the projections leave them (RowArgs).  Every wave with a tile norms and turns its heads' rows; the
-// segment that holds a row's own key puts that key and value among its tile's, and the first of a kv head's workgroups stores them.  A launch of its
-// own for that, between the projection and the attention, took 3.8 us of one row of 32 heads and 5.1 of eight of 48.
+// ROWS (the plain attention, EXACT): the step's rows come as the projections leave them (RowArgs).  The workgroup's waves norm and turn its heads' rows and the key's,
+// a lane VK_VEC elements, and pass them through LDS; the segment that holds a row's own key puts that key and value among its tile's, and the first of a kv
+// head's workgroups stores them.  A launch of its own for that, between the projection and the attention, took 3.8 us of one row of 32 heads and 5.1 of eight
+// of 48.  With every wave norming and turning all its heads' rows for itself one
+// row of 30 keys, 16 heads on 8, took 7.9 us beside its neighbours and takes 5.8 with what stands at decoded_row and OwnedMask; of 300 11.1 -> 9.9, 40 of 300, 32 on 8, 23.1 -> 21.3;
+// but 8 of 530, three segments of full tiles, 11.2 -> 11.7, which wait for the slowest wave's rows.
 // FAR: the launch covers the kept segments and those that a window or a block can touch, not all before it.  (Known when the kernel is built:
 // the page numbers then wait for the lengths, 0.4 us of a short request's 12.)
 template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1, bool FAR = false, bool ROWS = false>
@@ -1295,26 +1333,58 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   constexpr int NP = EXT ? P_PARTS : 1;                                        // numbers that a weight is split into
   __shared__ frag_t probs_of[SEGS][SEG_TILES][NP][KEY_SLABS][64];
   __shared__ float tile_max_of[SEGS][SEG_TILES][16], tile_sum_of[SEGS][SEG_TILES][16];
+  constexpr int ROW_PITCH = DPAD + VK_VEC;                                     // rows of LDS lie a vector further apart: 16 of them are read side by side
+  __shared__ __attribute__((aligned(16))) elem_t turned[ROWS ? 17 : 1][ROWS ? ROW_PITCH : VK_VEC];       // the q heads' rows, then the key's
   const int lane = threadIdx.x & 63;
   const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave8 % SEG_TILES, my_seg = wave8 / SEG_TILES;
   auto& probs = probs_of[my_seg];
   auto& tile_max = tile_max_of[my_seg];
   auto& tile_sum = tile_sum_of[my_seg];
-  const int G = a.nq / a.nkv, HT = (G + 15) >> 4;
-  const int kvh = blockIdx.y / HT, ht = blockIdx.y - kvh * HT;
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  int seg = blockIdx.z * SEGS + my_seg;
-  if (FAR && seg >= a.keep_segs) seg = max(first_visible(a, k_len - q_len + q_off) / (TILE_KEYS * SEG_TILES), a.keep_segs) + seg - a.keep_segs;
-  const int first_tile = seg * SEG_TILES;
+  // What needs nothing but the arguments first, together: a step of few keys is a chain of reads of 0.3 to 0.5 us each.
+  const int G = a.group, HT = a.head_tiles;
+  const int kvh = HT > 1 ? blockIdx.y / HT : blockIdx.y, ht = blockIdx.y - kvh * HT;
+  int seq, tok, back;
+  decoded_row(a, blockIdx.x, seq, tok, back);
   const int lp = __builtin_ctz(a.P);
   int page[SEG_TILES];                  // of the segment's tiles, where a tile lies in one page
+  auto read_pages = [&](int first_tile) {
 #pragma unroll
-  for (int j = 0; j < SEG_TILES; ++j)
-    page[j] = EXACT || a.P >= TILE_KEYS ? a.block_table[(int64_t)seq * a.bt_stride + min((first_tile + j) * TILE_KEYS >> lp, a.bt_stride - 1)] : -1;
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
+    for (int j = 0; j < SEG_TILES; ++j)
+      page[j] = EXACT || a.P >= TILE_KEYS ? a.block_table[(int64_t)seq * a.bt_stride + min((first_tile + j) * TILE_KEYS >> lp, a.bt_stride - 1)] : 0;
+  };
+  int seg = blockIdx.z * SEGS + my_seg;
+  const int k_len = a.k_len[seq];
+  if constexpr (!FAR) read_pages(seg * SEG_TILES);
+  // A pass of the workgroup's waves over the rows: this lane's, its piece of it, and what it is turned by.
+  constexpr int ROW_LANES = RowPiece<DPAD>::LANES, ROWS_A_WAVE = 64 / ROW_LANES;
+  const int q_rows = min(16, G - ht * 16), piece_at = lane % ROW_LANES;
+  int slot = -1, turn_at = 0;
+  RowPiece<DPAD> piece;
+  elem_t own_value[ND];
+  // Rows go round the waves, and rows beyond the key's are the key's once more: every wave asks for rows and angles in front of its keys.  (Waves without rows
+  // would fill the queue with keys in front of the others' angles, which all wait for.)
+  const int my_row = wave8 + SEGS * SEG_TILES * (lane / ROW_LANES);
+  // (The weights' addresses as numbers that the compiler does not look into: it would choose between the arguments' places and read one of them a lane.)
+  uint64_t q_weight = reinterpret_cast<uint64_t>(rows.q_w), k_weight = reinterpret_cast<uint64_t>(rows.k_w);
+  if constexpr (ROWS) asm("" : "+s"(q_weight), "+s"(k_weight));
+  [[maybe_unused]] auto load_piece = [&](int first) {
+    const int r = min(first + my_row, q_rows);
+    const int64_t at = (int64_t)(r < q_rows ? kvh * G + ht * 16 + r : a.nq + kvh) * DPAD;
+    piece.load(rows.qkv + (int64_t)tok * rows.row_stride + at, r < q_rows ? q_weight : k_weight, piece_at);
+  };
+  if constexpr (ROWS) {
+    slot = rows.slots[tok];
+    if (rows.cos_t != nullptr) turn_at = rows.positions[tok];
+    load_piece(0);
+    const elem_t* value = rows.qkv + (int64_t)tok * rows.row_stride + (int64_t)(a.nq + a.nkv + kvh) * DPAD + wave * ND * 16 + (lane & 15);
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) own_value[dt] = value[dt * 16];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const int pos = k_len - back;
+  if (FAR && seg >= a.keep_segs) seg = max(first_visible(a, pos) / (TILE_KEYS * SEG_TILES), a.keep_segs) + seg - a.keep_segs;
+  const int first_tile = seg * SEG_TILES;
+  if constexpr (FAR) read_pages(first_tile);
   const int lo = first_visible(a, pos);
   const int keep = EXT && a.window > 0 ? a.keep : 0;
   const int keep_tiles = (keep + TILE_KEYS - 1) / TILE_KEYS, tile_lo = lo / TILE_KEYS;
@@ -1342,25 +1412,13 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   frag_t qf[NQS];
   frag_t kf[KSUB][NQS];
   const int own_tile = pos / TILE_KEYS - first_tile;          // the segment's tile with the row's own key, where that is 0 .. SEG_TILES - 1
-  int slot = -1;
-  HeadRow<NQS> q_row, k_row;
-  typename HeadRow<NQS>::Angles angles;
-  elem_t own_value[ND];
+  frag_t cosines, sines;
   if constexpr (ROWS) {
-    // These loads first: loads arrive in the order in which they are asked for.
-    slot = rows.slots[tok];
-    const elem_t* row = rows.qkv + (int64_t)tok * rows.row_stride;
-    if (mine) {
-      q_row.load(row + (int64_t)(c.row_ok ? head : kvh * G) * DPAD, rows.q_w, c.g);
-      if (wave == own_tile) k_row.load(row + (int64_t)(a.nq + kvh) * DPAD, rows.k_w, c.g);
-      if (rows.cos_t != nullptr) {
-        const int64_t at = (int64_t)rows.positions[tok] * (DPAD / 2);
-        angles.load(rows.cos_t + at, rows.sin_t + at, c.g);
-      }
-    }
-    if (own_tile >= 0 && own_tile < SEG_TILES) {
-#pragma unroll
-      for (int dt = 0; dt < ND; ++dt) own_value[dt] = row[(int64_t)(a.nq + a.nkv + kvh) * DPAD + (wave * ND + dt) * 16 + c.r16];
+    // In front of the keys: loads arrive in the order in which they are asked for.
+    if (rows.cos_t != nullptr) {
+      const int64_t at = (int64_t)turn_at * (DPAD / 2) + piece_at % (ROW_LANES / 2) * VK_VEC;
+      cosines = *reinterpret_cast<const frag_t*>(rows.cos_t + at);
+      sines = *reinterpret_cast<const frag_t*>(rows.sin_t + at);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1369,17 +1427,29 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     int my_page = page[0];
 #pragma unroll
     for (int j = 1; j < SEG_TILES; ++j) my_page = wave == j ? page[j] : my_page;
-    load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf, my_page);
+    if (EXACT || a.P >= TILE_KEYS) load_keys<NQS, EXACT, true>(c, (first_tile + wave) * TILE_KEYS, kf, my_page);
+    else load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf);
   }
-  frag_t own_key[ROWS ? NQS : 1];
+  __builtin_amdgcn_sched_barrier(0);
+  const int own_page = slot >> lp, own_off = slot & (a.P - 1);
   if constexpr (ROWS) {
-    // Between the keys' loads and the values': the registers of both, of two rows and of their arithmetic are too many at once.
-    __builtin_amdgcn_sched_barrier(0);
-    if (mine) {
-      q_row.finish(rows.q_w != nullptr, rows.cos_t != nullptr, angles, rows.eps, qf);
-      if (wave == own_tile) k_row.finish(rows.k_w != nullptr, rows.cos_t != nullptr, angles, rows.eps, own_key);
+    // The workgroup that holds the row's own key, in either segment, stores it.
+    const int own_of_all = pos / TILE_KEYS - (int)blockIdx.z * SEGS * SEG_TILES;
+    const bool stores = ht == 0 && slot >= 0 && own_of_all >= 0 && own_of_all < SEGS * SEG_TILES;
+    for (int first = 0; first <= q_rows; first += SEGS * SEG_TILES * ROWS_A_WAVE) {
+      if (first > 0) load_piece(first);
+      const int r = first + my_row;
+      const frag_t x = piece.finish((q_weight | k_weight) != 0, (r < q_rows ? q_weight : k_weight) != 0, rows.cos_t != nullptr, cosines, sines,
+                                    rows.eps, piece_at);
+      if (r <= q_rows) *reinterpret_cast<frag_t*>(&turned[r][piece_at * VK_VEC]) = x;
+      if (r == q_rows && stores)
+        *reinterpret_cast<frag_t*>(rows.kc + (((int64_t)own_page * a.nkv + kvh) * a.P + own_off) * DPAD + piece_at * VK_VEC) = x;
     }
-    __builtin_amdgcn_sched_barrier(0);
+    if (own_tile >= 0 && own_tile < SEG_TILES && stores && c.g == 0) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+        rows.vc[(((int64_t)own_page * a.nkv + kvh) * DPAD + (wave * ND + dt) * 16 + c.r16) * a.P + own_off] = own_value[dt];
+    }
   }
   // This wave's columns of every tile's values: a context whose head starts at them.
   RowCtx cv = c;
@@ -1388,47 +1458,34 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   frag_t vf[SEG_TILES][ND][KEY_SLABS];
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j)
-    if ((wanted >> j) & 1u) load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
+    if ((wanted >> j) & 1u) {
+      if (EXACT || a.P >= TILE_KEYS) load_values<ND, EXACT, true>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
+      else load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j]);
+    }
   __builtin_amdgcn_sched_barrier(0);
 
   if constexpr (ROWS) {
-    const int own_page = slot >> lp, own_off = slot & (a.P - 1);
-    const bool stores = ht == 0 && slot >= 0;
-    if (mine && wave == own_tile && slot >= 0) {
-      if (stores && c.r16 == 0) {
-        elem_t* o = rows.kc + (((int64_t)own_page * a.nkv + kvh) * a.P + own_off) * DPAD + c.g * VK_VEC;
+    __syncthreads();
+    if (mine) {
 #pragma unroll
-        for (int s = 0; s < NQS; ++s) *reinterpret_cast<frag_t*>(o + s * VK_SLAB) = own_key[s];
-      }
-      const int at = pos % TILE_KEYS;
+      for (int s = 0; s < NQS; ++s) qf[s] = *reinterpret_cast<const frag_t*>(&turned[c.row_ok ? c.r16 : 0][s * VK_SLAB + c.g * VK_VEC]);
+      if (wave == own_tile && slot >= 0) {
+        frag_t own_key[NQS];
 #pragma unroll
-      for (int sub = 0; sub < KSUB; ++sub) {
+        for (int s = 0; s < NQS; ++s) own_key[s] = *reinterpret_cast<const frag_t*>(&turned[q_rows][s * VK_SLAB + c.g * VK_VEC]);
+        // (load_keys says which key a lane holds in which sub-tile)
+        const int at = pos % TILE_KEYS;
 #ifdef VK_BF16
-        const bool here = at == (sub >> 1) * VK_SLAB + 8 * (c.r16 >> 2) + 4 * (sub & 1) + (c.r16 & 3);
+        const int own_sub = (at / VK_SLAB) * 2 + ((at >> 2) & 1), own_r16 = ((at % VK_SLAB) >> 3) * 4 + (at & 3);
 #else
-        const bool here = at == sub * VK_SLAB + c.r16;
+        const int own_sub = at / VK_SLAB, own_r16 = at % VK_SLAB;
 #endif
 #pragma unroll
-        for (int s = 0; s < NQS; ++s) kf[sub][s] = here ? own_key[s] : kf[sub][s];
-      }
-    }
-    if (own_tile >= 0 && own_tile < SEG_TILES && slot >= 0) {
-      if (stores && c.g == 0) {
+        for (int sub = 0; sub < KSUB; ++sub) {
+          if (sub == own_sub) {
 #pragma unroll
-        for (int dt = 0; dt < ND; ++dt)
-          rows.vc[(((int64_t)own_page * a.nkv + kvh) * DPAD + (wave * ND + dt) * 16 + c.r16) * a.P + own_off] = own_value[dt];
-      }
-      const int at = pos % TILE_KEYS;
-#pragma unroll
-      for (int j = 0; j < SEG_TILES; ++j) {
-        if (j == own_tile) {
-#pragma unroll
-          for (int dt = 0; dt < ND; ++dt)
-#pragma unroll
-            for (int ks = 0; ks < KEY_SLABS; ++ks)
-#pragma unroll
-              for (int e = 0; e < VK_VEC; ++e)
-                if (at == ks * VK_SLAB + c.g * VK_VEC + e) vf[j][dt][ks][e] = own_value[dt];
+            for (int s = 0; s < NQS; ++s) kf[sub][s] = c.r16 == own_r16 ? own_key[s] : kf[sub][s];
+          }
         }
       }
     }
@@ -1437,7 +1494,6 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   // ---- the scores of this wave's tile and their maximum a row ----
   const float unit = EXT ? LOG2E : a.scale_log2;             // what takes a score to powers of two
   float sc[S_PER_LANE];
-  bool vis[S_PER_LANE];
   const int kb = (first_tile + wave) * TILE_KEYS;
   float tmax = -INFINITY;
   if (mine) {
@@ -1445,12 +1501,15 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     if constexpr (REL) tile_bias<REL>(c, kb, rb);
     tile_scores<NQS, EXACT>(c, kf, qf, sc);
     if constexpr (EXT) natural_scores<REL>(sc, a.scale, a.softcap, rb);
+    if (kb + TILE_KEYS - 1 > pos || kb < lo) {               // else every key is seen
+      const int at = kb + c.g * VK_VEC;
+      unsigned vis = keys_before(pos + 1 - at);
+      if (kb < lo) vis &= ~keys_before(lo - at) | keys_before(keep - at);
 #pragma unroll
-    for (int i = 0; i < S_PER_LANE; ++i) {
-      const int key = kb + (i / VK_VEC) * VK_SLAB + c.g * VK_VEC + (i % VK_VEC);
-      vis[i] = (int)c.row_ok & (int)(key <= pos) & ((int)(key >= lo) | (int)(key < keep));      // (as conditions they become branches)
-      tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
+      for (int i = 0; i < S_PER_LANE; ++i) sc[i] = vis >> i & 1u ? sc[i] : -INFINITY;
     }
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
     tmax = row_max(tmax);
   }
   if (c.g == 0) tile_max[wave][c.r16] = tmax;
@@ -1471,7 +1530,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     frag_t pf[NP][KEY_SLABS];
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
-      const float p = vis[i] ? fast_exp2(__builtin_fmaf(sc[i], unit, -my_max)) : 0.f;
+      const float p = fast_exp2(__builtin_fmaf(sc[i], unit, -my_max));       // 0 for a key that is not seen (a tile that is computed has one that is)
       psum = psum + p;
       const elem_t hi = (elem_t)p;
       pf[0][i / VK_VEC][i % VK_VEC] = hi;
@@ -1502,10 +1561,33 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
       const int kj = (first_tile + j) * TILE_KEYS;
       L = __builtin_fmaf(L, ca[j], tile_sum[j][c.r16]);
       scale_state<ND>(ACC, ca[j], false);
-      if (kj + TILE_KEYS > k_len || kj < lo) {
+      if constexpr (ROWS) {
+        if (j == own_tile && slot >= 0) {                    // the row's own value among them, as a mask of its place
+          const int at = pos % TILE_KEYS, e = at % VK_VEC;
+          constexpr int PER = VK_VEC / VEC_DWORDS;
+          const unsigned half = PER == 1 ? ~0u : (e & 1 ? 0xFFFF0000u : 0xFFFFu);
+          const unsigned here = c.g == (at % VK_SLAB) / VK_VEC ? half : 0u;
 #pragma unroll
-        for (int dt = 0; dt < ND; ++dt) zero_unowned(vf[j][dt], kj, c.g, lo, k_len, keep);
+          for (int ks = 0; ks < KEY_SLABS; ++ks) {
+            if (ks == at / VK_SLAB) {
+#pragma unroll
+              for (int dt = 0; dt < ND; ++dt) {
+                unsigned both;
+                if constexpr (PER == 1) both = __builtin_bit_cast(unsigned, (float)own_value[dt]);
+                else both = __builtin_bit_cast(unsigned, (float)own_value[dt]) | __builtin_bit_cast(unsigned, (float)own_value[dt]) >> 16;
+                u32x4 v = __builtin_bit_cast(u32x4, vf[j][dt][ks]);
+#pragma unroll
+                for (int i = 0; i < VEC_DWORDS; ++i) {
+                  const unsigned m = e / PER == i ? here : 0u;
+                  v[i] = (v[i] & ~m) | (both & m);
+                }
+                vf[j][dt][ks] = __builtin_bit_cast(frag_t, v);
+              }
+            }
+          }
+        }
       }
+      if (kj + TILE_KEYS > k_len || kj < lo) OwnedMask(kj, c.g, lo, k_len, keep).apply(vf[j]);
       frag_t pf[NP][KEY_SLABS];
 #pragma unroll
       for (int part = 0; part < NP; ++part)
@@ -1522,26 +1604,29 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   }
   if constexpr (SEGS == 2) {
     // The second segment's state to the first one's waves, lane by lane: the same lanes hold the same rows and columns.
-    __syncthreads();                      // the weights have been read
+    const bool second = pos >= SEG_TILES * TILE_KEYS;        // the same for the workgroup: else that segment has no keys and its state is empty
+    if (second) __syncthreads();          // the weights have been read
     f32x4* hand = reinterpret_cast<f32x4*>(&probs_of[0][0][0][0][0]);
     static_assert((size_t)SEG_TILES * (ND + 1) * 64 * sizeof(f32x4) <= sizeof(probs_of), "the hand-over fits the weights' place");
-    if (my_seg == 1) {
+    if (second && my_seg == 1) {
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt) hand[(wave * (ND + 1) + dt) * 64 + lane] = ACC[dt];
       hand[(wave * (ND + 1) + ND) * 64 + lane] = f32x4{M, L, 0.f, 0.f};
     }
-    __syncthreads();
+    if (second) __syncthreads();
     if (my_seg == 1 || !c.row_ok) return;
     float Mt = -INFINITY, Lt = 0.f;
     f32x4 out[ND];
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) out[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     fold<ND>(Mt, Lt, out, M, L, ACC);
-    const f32x4 other = hand[(wave * (ND + 1) + ND) * 64 + lane];
-    f32x4 theirs[ND];
+    if (second) {
+      const f32x4 other = hand[(wave * (ND + 1) + ND) * 64 + lane];
+      f32x4 theirs[ND];
 #pragma unroll
-    for (int dt = 0; dt < ND; ++dt) theirs[dt] = hand[(wave * (ND + 1) + dt) * 64 + lane];
-    fold<ND>(Mt, Lt, out, other.x, other.y, theirs);
+      for (int dt = 0; dt < ND; ++dt) theirs[dt] = hand[(wave * (ND + 1) + dt) * 64 + lane];
+      fold<ND>(Mt, Lt, out, other.x, other.y, theirs);
+    }
     if (a.sinks != nullptr && Mt > -INFINITY) Lt = Lt + sink_term(a, head, Mt);
     const float inv = (Lt > 0.f ? 1.0f / Lt : 0.f) * out_gate(a, tok, head);
     elem_t* orow = a.out + ((int64_t)tok * a.nq + head) * a.d + wave * ND * 16 + 4 * c.g;
@@ -1566,42 +1651,48 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
 // Folds the segment results of one (token, head) in ascending segment order.
 // One wave per row; lane j owns output columns j, j+64, ...
 __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a) {
-  const int seq = a.items[2 * blockIdx.x], q_off = a.items[2 * blockIdx.x + 1];
+  int seq, tok, back;
+  decoded_row(a, blockIdx.x, seq, tok, back);
   const int head = blockIdx.y;
-  const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
-  const int k_len = a.k_len[seq];
-  const int tok = q_begin + q_off;
-  const int pos = k_len - q_len + q_off;
-  const int lo = first_visible(a, pos);
-  // Segments that hold kept first keys come before the window's; those in between were not computed.
-  const int keep_tiles = a.window > 0 ? (a.keep + TILE_KEYS - 1) / TILE_KEYS : 0, tile_lo = lo / TILE_KEYS;
-  const int seg_begin = keep_tiles > 0 ? 0 : lo / (TILE_KEYS * SEG_TILES), seg_end = pos / (TILE_KEYS * SEG_TILES) + 1;
   const int d = a.d;
   float M = -INFINITY, L = 0.f;
   float ACC[4] = {0.f, 0.f, 0.f, 0.f};   // d <= 256
   const int64_t row0 = ((int64_t)blockIdx.x * a.nq + head) * a.nseg;
-  // Four segments are fetched together, then folded one after the other.
-  for (int seg0 = seg_begin; seg0 < seg_end; seg0 += 4) {
-    float m[4], l[4], v[4][4];
+  // Four segments are fetched together, then folded one after the other.  Sums are asked for beside the maxima that say whether there are any (what an
+  // empty segment's place holds is not used); a launch of at most four segments asks for all of them before the sequence's length is there.
+  // Reads one after the other, the length's and the item's among them, are most of the launch.
+  float m[4], l[4], v[4][4];
+  auto fetch = [&](int first, int last) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bool in = seg0 + j < seg_end && ((seg0 + j) * SEG_TILES < keep_tiles || (seg0 + j) * SEG_TILES + SEG_TILES > tile_lo);
-      const int64_t r = row0 + (in ? seg0 + j : seg_begin);
-      m[j] = in ? a.part_ml[2 * r] : -INFINITY;
+      const int64_t r = row0 + min(first + j, last);
+      m[j] = a.part_ml[2 * r];
       l[j] = a.part_ml[2 * r + 1];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t r = row0 + (m[j] > -INFINITY ? seg0 + j : seg_begin);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int col = threadIdx.x + 64 * i;
-        v[j][i] = (col < d && m[j] > -INFINITY) ? a.part_acc[r * d + col] : 0.f;
+        v[j][i] = col < d ? a.part_acc[r * d + col] : 0.f;
       }
     }
+  };
+  const bool few = a.nseg <= 4;
+  int seg0 = 0;
+  if (few) fetch(0, a.nseg - 1);
+  const int pos = a.k_len[seq] - back;
+  const int lo = first_visible(a, pos);
+  // Segments that hold kept first keys come before the window's; those in between were not computed.
+  const int keep_tiles = a.window > 0 ? (a.keep + TILE_KEYS - 1) / TILE_KEYS : 0, tile_lo = lo / TILE_KEYS;
+  const int seg_begin = keep_tiles > 0 ? 0 : lo / (TILE_KEYS * SEG_TILES), seg_end = pos / (TILE_KEYS * SEG_TILES) + 1;
+  if (!few) {
+    seg0 = seg_begin;
+    fetch(seg0, seg_end - 1);
+  }
+  for (;;) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (m[j] > -INFINITY) {
+      const int seg = seg0 + j;
+      const bool in = seg >= seg_begin && seg < seg_end && (seg * SEG_TILES < keep_tiles || seg * SEG_TILES + SEG_TILES > tile_lo);
+      if (in && m[j] > -INFINITY) {
         float Mn, ca, cb;
         fold_scales(M, m[j], Mn, ca, cb);
 #pragma unroll
@@ -1610,6 +1701,9 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a) {
         M = Mn;
       }
     }
+    seg0 += 4;
+    if (seg0 >= seg_end || few) break;
+    fetch(seg0, seg_end - 1);
   }
   if (a.sinks != nullptr && M > -INFINITY) L = L + sink_term(a, head, M);
   const float inv = (L > 0.f ? 1.0f / L : 0.f) * out_gate(a, tok, head);
@@ -1665,7 +1759,7 @@ static int64_t quad_segments(int d) {
 //   the kernel is chosen by shape.  mode 2: the same through the kernel that takes every shape,
 //   modes 6, 8 and 9: through the one that shares tiles in LDS with four waves, with eight, and with four and
 //   one buffer instead of two, whatever the shape (tests and measurements; the result is the same bits).
-// mode 1: each item is one token; the keys are split by segment over nseg workgroups (nseg must cover
+// mode 1: each item is one token (items and cu_q null: item i is the one row of sequence i, and its token is row i); the keys are split by segment over nseg workgroups (nseg must cover
 //   the longest sequence; scratch must hold vk_attn_scratch_floats(n_items, ...)) and folded by a
 //   second kernel; the kernel is chosen by shape.  modes 3, 4, 5, 7: the same through a named kernel
 //   (3 and 4: a wave per segment that asks for a tile's fragments when it needs them, the kernel for every
@@ -1686,9 +1780,11 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   if (mode == 6 || mode == 8 || mode == 9) mode = 0;
   if (mode >= 3) mode = 1;
   if (n_items <= 0) return 0;
+  VK_REQUIRE(mode == 1 || items != nullptr, "attention: prompt rows need items");
   AttnArgs a;
   a.q = q; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
   a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
+  a.group = nq / nkv; a.head_tiles = (nq / nkv + 15) / 16;
   a.nseg = nseg; a.scale_log2 = scale * 1.4426950408889634f;
   a.part_ml = nullptr; a.part_acc = nullptr;
   const int G = nq / nkv;
@@ -1877,6 +1973,7 @@ int vk_paged_attention_rows(elem_t* out, const elem_t* qkv, int64_t row_stride, 
   AttnArgs a;
   a.q = nullptr; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
   a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
+  a.group = nq / nkv; a.head_tiles = (nq / nkv + 15) / 16;
   a.nseg = nseg; a.scale_log2 = scale * 1.4426950408889634f;
   a.part_ml = scratch;
   a.part_acc = scratch + (((int64_t)n_items * nq * nseg * 2 + 3) & ~(int64_t)3);
@@ -1919,9 +2016,11 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
              "attention: a bias by distance excludes a cap, and its rows hold %d entries more than its distances", 2 * REL_PAD);
   VK_REQUIRE(gate == nullptr || gate_stride >= nq, "attention: a gate a head needs rows of at least %d", nq);
   if (n_items <= 0) return 0;
+  VK_REQUIRE(mode == 1 || items != nullptr, "attention: prompt rows need items");
   AttnArgs a;
   a.q = q; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
   a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
+  a.group = nq / nkv; a.head_tiles = (nq / nkv + 15) / 16;
   a.nseg = nseg; a.scale_log2 = scale * LOG2E;
   a.part_ml = nullptr; a.part_acc = nullptr;
   a.keep = keep; a.scale = scale; a.softcap = softcap; a.sinks = sinks; a.sinks_f32 = sinks_f32; a.block = block;

@@ -488,6 +488,13 @@ Tensor Kernels::qkv_post(const Tensor& qkv, int nq, int nkv, int d, const Tensor
   return q_out;
 }
 
+// The list of decoded items that a launch is handed: none where every sequence of the step brings one row (the kernels then read none).
+static const void* decode_list(const Tensor& items, int64_t sequences, int64_t rows, bool alone) {
+  if (!alone) return items.data;
+  if (items.dim(0) != rows || sequences != rows) throw EngineError("attention: " + std::to_string(rows) + " rows are not one a sequence");
+  return nullptr;
+}
+
 int64_t Kernels::attn_scratch_floats(int items, int nq, int d, int nseg) const {
   return fn_->attn_scratch_floats(items, nq, d, nseg);
 }
@@ -500,7 +507,7 @@ bool Kernels::attention_takes_rows(int64_t items, int nseg, int nq, int nkv, int
 void Kernels::paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int nkv, int d, const Tensor& k_cache, const Tensor& v_cache, int page_size, const Tensor* q_w,
                                    const Tensor* k_w, float eps, const Tensor* cos, const Tensor* sin, const Tensor& positions, const Tensor& slots,
                                    const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items, float scale, int window, int max_k_len, int nseg,
-                                   const Tensor& scratch) {
+                                   const Tensor& scratch, bool alone) {
   const int64_t T = qkv.dim(0), W = (int64_t)(nq + 2 * nkv) * d, pages = k_cache.dim(0), S = k_len.dim(0);
   expect(qkv, "qkv", dtype_, {T, W});
   expect(k_cache, "k cache", dtype_, {pages, nkv, page_size, d});
@@ -524,13 +531,13 @@ void Kernels::paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int n
   const int64_t need = attn_scratch_floats((int)T, nq, d, nseg);
   if (scratch.dtype != DType::F32 || scratch.numel() < need) throw EngineError("attention: scratch of " + std::to_string(need) + " floats needed");
   call(fn_->paged_attention_rows(out.data, qkv.data, W, k_cache.data, v_cache.data, q_w ? q_w->data : nullptr, k_w ? k_w->data : nullptr, eps, cos ? cos->data : nullptr,
-                                 cos ? sin->data : nullptr, positions.data, slots.data, block_table.data, (int)block_table.dim(1), cu_q.data, k_len.data, items.data, (int)T,
+                                 cos ? sin->data : nullptr, positions.data, slots.data, block_table.data, (int)block_table.dim(1), cu_q.data, k_len.data, decode_list(items, S, T, alone), (int)T,
                                  nseg, scratch.data, nq, nkv, d, page_size, window, scale, stream));
 }
 
 void Kernels::paged_attention(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
                               const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items,
-                              int mode, float scale, int window, int max_k_len, int nseg, const Tensor* scratch) {
+                              int mode, float scale, int window, int max_k_len, int nseg, const Tensor* scratch, bool alone) {
   expect(q, "q", dtype_);
   expect(k_cache, "k cache", dtype_);
   expect(block_table, "block table", DType::I32);
@@ -559,7 +566,7 @@ void Kernels::paged_attention(Tensor& out, const Tensor& q, const Tensor& k_cach
     sp = scratch->data;
   }
   call(fn_->paged_attention(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data,
-                            items.data, (int)n_items, mode, nseg, sp, (int)T, (int)nq, (int)nkv, (int)d, (int)P, window, scale,
+                            decode_list(items, S, T, alone && mode == 1), (int)n_items, mode, nseg, sp, (int)T, (int)nq, (int)nkv, (int)d, (int)P, window, scale,
                             stream));
 }
 
@@ -699,7 +706,7 @@ Tensor Kernels::qkv_post_bias(const Tensor& qkv, int nq, int nkv, int d, const T
 
 void Kernels::paged_attention_capped(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
                                      const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode, float scale, int window, int keep,
-                                     float softcap, const Tensor* sinks, int max_k_len, int nseg, const Tensor* scratch, int block) {
+                                     float softcap, const Tensor* sinks, int max_k_len, int nseg, const Tensor* scratch, int block, bool alone) {
   expect(q, "q", dtype_);
   expect(block_table, "block table", DType::I32);
   if (block < 0 || (block > 0 && (window != 0 || keep != 0))) throw EngineError("attention: blocks of positions exclude a window");
@@ -736,13 +743,14 @@ void Kernels::paged_attention_capped(Tensor& out, const Tensor& q, const Tensor&
       throw EngineError("attention: scratch of " + std::to_string(need) + " floats needed");
     sp = scratch->data;
   }
+  const void* list = decode_list(items, S, T, alone && mode == 1);
   if (block > 0) {
-    call(fn_->paged_attention_blocked(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, items.data,
+    call(fn_->paged_attention_blocked(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, list,
                                       (int)n_items, mode, nseg, sp, (int)T, (int)nq, (int)nkv, (int)d, (int)P, block, scale, softcap,
                                       sinks ? sinks->data : nullptr, sf, stream));
     return;
   }
-  call(fn_->paged_attention_capped(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, items.data,
+  call(fn_->paged_attention_capped(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, list,
                                    (int)n_items, mode, nseg, sp, (int)T, (int)nq, (int)nkv, (int)d, (int)P, window, keep, scale, softcap,
                                    sinks ? sinks->data : nullptr, sf, stream));
 }
@@ -1311,7 +1319,7 @@ Tensor Kernels::qkv_prepare(const Tensor& qkv, int nq, int nkv, int d, int size,
 
 void Kernels::paged_attention_biased(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
                                      const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode, float scale, int window, const Tensor* rel,
-                                     int far, const Tensor* gate, int64_t gate_col, int max_k_len, int nseg, const Tensor* scratch) {
+                                     int far, const Tensor* gate, int64_t gate_col, int max_k_len, int nseg, const Tensor* scratch, bool alone) {
   expect(q, "q", dtype_);
   expect(block_table, "block table", DType::I32);
   if (q.shape.size() != 3 || k_cache.shape.size() != 4 || block_table.shape.size() != 2)
@@ -1344,7 +1352,7 @@ void Kernels::paged_attention_biased(Tensor& out, const Tensor& q, const Tensor&
       throw EngineError("attention: scratch of " + std::to_string(need) + " floats needed");
     sp = scratch->data;
   }
-  call(fn_->paged_attention_biased(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, items.data,
+  call(fn_->paged_attention_biased(out.data, q.data, k_cache.data, v_cache.data, block_table.data, (int)W, cu_q.data, k_len.data, decode_list(items, S, T, alone && mode == 1),
                                    (int)n_items, mode, nseg, sp, (int)T, (int)nq, (int)nkv, (int)d, (int)P, window, 0, scale, nullptr, 0,
                                    rel ? rel->data : nullptr, rel ? (int)rel->dim(1) : 0, far,
                                    gate ? static_cast<const char*>(gate->data) + (size_t)gate_col * dtype_bytes(dtype_) : nullptr, gate ? gate->dim(1) : 0,

@@ -144,16 +144,17 @@ class Kernels {
                   const Tensor* q_w, const Tensor* k_w, float eps, const Tensor* cos, const Tensor* sin,
                   const Tensor* positions, const Tensor* slots);
   int64_t attn_scratch_floats(int items, int nq, int d, int nseg) const;
+  // alone (here and in the others): every sequence of the step brings one row and items lists them all, in order.
   void paged_attention(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
                        const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode,
-                       float scale, int window, int max_k_len, int nseg, const Tensor* scratch);
+                       float scale, int window, int max_k_len, int nseg, const Tensor* scratch, bool alone = false);
   // qkv_post and paged_attention of decoded rows alone (every row of qkv [T, (nq + 2 nkv) d] is an item of its own) in one launch, where
   // attention_takes_rows says that there is one and that it is the faster way: the same bits.
   bool attention_takes_rows(int64_t items, int nseg, int nq, int nkv, int d, int page_size, const Tensor* q_w, const Tensor* k_w, const Tensor* cos) const;
   void paged_attention_rows(Tensor& out, const Tensor& qkv, int nq, int nkv, int d, const Tensor& k_cache, const Tensor& v_cache, int page_size, const Tensor* q_w,
                             const Tensor* k_w, float eps, const Tensor* cos, const Tensor* sin, const Tensor& positions, const Tensor& slots,
                             const Tensor& block_table, const Tensor& cu_q, const Tensor& k_len, const Tensor& items, float scale, int window, int max_k_len, int nseg,
-                            const Tensor& scratch);
+                            const Tensor& scratch, bool alone = false);
   // Token ids per row: the largest logit, or a draw at temps[r] > 0 with the uniform number unis[r].
   void sample(Tensor& out, const Tensor& logits, const Tensor* temps, const Tensor* unis, Tensor& scratch);
   int sample_scratch_words(int rows) const;
@@ -189,7 +190,7 @@ class Kernels {
   // (without a window): positions are cut into blocks of that many, and a row sees the keys of its own block only.
   void paged_attention_capped(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
                               const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode, float scale, int window, int keep,
-                              float softcap, const Tensor* sinks, int max_k_len, int nseg, const Tensor* scratch, int block = 0);
+                              float softcap, const Tensor* sinks, int max_k_len, int nseg, const Tensor* scratch, int block = 0, bool alone = false);
   // ---- the gated delta rule with a decay per key channel (delta.hip)
   // silu(short causal convolution) of the first taps.dim(0) columns of x, floats [T, C]; the state's tails move on.
   // first_col: where the convolution's channels start in x's rows; bias: [channels] or null.
@@ -344,7 +345,7 @@ class Kernels {
   // or null) and a gate a head (the columns [gate_col, gate_col + nq) of gate, or null).
   void paged_attention_biased(Tensor& out, const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_table,
                               const Tensor& cu_q, const Tensor& k_len, const Tensor& items, int mode, float scale, int window, const Tensor* rel,
-                              int far, const Tensor* gate, int64_t gate_col, int max_k_len, int nseg, const Tensor* scratch);
+                              int far, const Tensor* gate, int64_t gate_col, int max_k_len, int nseg, const Tensor* scratch, bool alone = false);
   int distance_pad() const;                      // entries a row of rel holds beyond its distances, at either end
   // The widest cached row that attention takes; rows of more than 256 entries go through vector arithmetic.
   int attention_limit() const;

@@ -499,6 +499,7 @@ class RotaryStretched : public PositionEncoding {
 struct AttentionItems {
   HostArray prefill, decode;
   int decode_bound = 0, nseg = 0;
+  bool alone = false;      // every sequence of the step brings one row: the decoded items are the rows, in order
 };
 
 // The items of a step, derived once a step and shared by every mixer that runs the paged attention kernels.
@@ -522,6 +523,7 @@ AttentionItems& attention_items(Kernels& kernels, HostStep& step) {
   }
   m->prefill.shape = {(int64_t)m->prefill.data.size() / 2, 2};
   m->decode.shape = {(int64_t)m->decode.data.size() / 2, 2};
+  m->alone = (size_t)m->decode.shape[0] == step.q_lens.size();
   // Recorded launches must cover every length that the tables can hold.
   m->decode_bound = step.frozen ? step.k_len_bound : decode_keys;
   m->nseg = (m->decode_bound + kernels.segment_keys() - 1) / kernels.segment_keys();
@@ -740,7 +742,7 @@ class Attention : public Mixer {
         const Tensor scratch = ctx.workspace(k.attn_scratch_floats((int)T, nq_, d_, m.nseg));
         Tensor heads = k.empty({T, (int64_t)nq_, (int64_t)d_});
         k.paged_attention_rows(heads, qkv_all, nq_, nkv_, d_, cache.k, cache.v, cache.page_size, q_w, k_w, en ? en->eps() : 0.f, cos, sin, ctx.positions, tables.slots,
-                               tables.block_table, ctx.cu_q, ctx.k_len, decode_items, scale_, window_, m.decode_bound, m.nseg, scratch);
+                               tables.block_table, ctx.cu_q, ctx.k_len, decode_items, scale_, window_, m.decode_bound, m.nseg, scratch, m.alone);
         return k.gemm(heads.view({T, (int64_t)nq_ * d_}), w_o_, ws);
       }
     }
@@ -788,13 +790,13 @@ class Attention : public Mixer {
       const Tensor scratch = ctx.workspace(k.attn_scratch_floats((int)decode_items.dim(0), nq_, d_, m.nseg));
       if (biased())
         k.paged_attention_biased(out, q, cache.k, cache.v, tables.block_table, ctx.cu_q, ctx.k_len, decode_items, 1, scale_, window_, rel, far_,
-                                 head_gate, heads_w, m.decode_bound, m.nseg, &scratch);
+                                 head_gate, heads_w, m.decode_bound, m.nseg, &scratch, m.alone);
       else if (capped())
         k.paged_attention_capped(out, q, cache.k, cache.v, tables.block_table, ctx.cu_q, ctx.k_len, decode_items, 1, scale_, window_, keep_,
-                                 softcap_, sinks, m.decode_bound, m.nseg, &scratch, block_);
+                                 softcap_, sinks, m.decode_bound, m.nseg, &scratch, block_, m.alone);
       else
         k.paged_attention(out, q, cache.k, cache.v, tables.block_table, ctx.cu_q, ctx.k_len, decode_items, 1, scale_, window_,
-                          m.decode_bound, m.nseg, &scratch);
+                          m.decode_bound, m.nseg, &scratch, m.alone);
     }
     Tensor heads = out.view({T, (int64_t)nq_ * d_});
     if (gate_) k.gate_mul(heads, qkv_all, heads_w, 0);
@@ -1806,7 +1808,7 @@ class LatentAttention : public Mixer {
     if (decode_items.dim(0)) {
       const Tensor scratch = ctx.workspace(k.attn_scratch_floats((int)decode_items.dim(0), H_, D_, m.nseg));
       k.paged_attention_capped(out, q_abs, cache.k, cache.v, tables.block_table, ctx.cu_q, ctx.k_len, decode_items, 1, scale_, window_, 0, 0.f, sinks,
-                               m.decode_bound, m.nseg, &scratch, 0);
+                               m.decode_bound, m.nseg, &scratch, 0, m.alone);
     }
     Tensor heads = k.empty({T, (int64_t)H_ * dvp_});
     k.gemm_heads(heads, dvp_, out.view({T, (int64_t)H_ * D_}), 0, D_, w_expand_);
