@@ -38,7 +38,7 @@
 //                       waves whose two halves take turns between LDS and the matrix unit.  Optionally SwiGLU in the epilogue
 //                       (alternate_fragments says when).
 //   gemm_fine           32-bit elements, more than 64 rows (32 where K is short or with SwiGLU), K as gemm_pipe: tiles of 32 x 32 to 96 x 64 or 64 x 128, the one
-//                       whose launch ends first (fine_takes, fine_tile).  Optionally SwiGLU in the epilogue.
+//                       whose launch ends first, unless larger ones of gemm_pipe fill the units (fine_takes, fine_tile).  Optionally SwiGLU in the epilogue.
 //   gemm_tiled          any M and K: the same tile through registers into LDS, predicated.
 #include <algorithm>
 #include <cmath>
@@ -1356,16 +1356,19 @@ __global__ __launch_bounds__(256) void gemm_fine_kernel(elem_t* __restrict__ out
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
   };
-  if (WHOLE) {
-    for (int kt0 = 0; kt0 < ntiles; kt0 += T_CHUNK_TILES) {
+  // K not in whole chunks: whole ones first and what is left after them.  (Asking every tile whether it ends a chunk takes 3 to 12 % longer, 2,048 rows, 2,048 x 2,080 145 -> 130 us;
+  // but with the two products of 1 x 2 fragments 2 to 7 % less.)
+  constexpr bool ASK = !WHOLE && FM * FN == 2;
+  const int whole = WHOLE ? ntiles : ASK ? 0 : ntiles - ntiles % T_CHUNK_TILES;
+  for (int kt0 = 0; kt0 < whole; kt0 += T_CHUNK_TILES) {
 #pragma unroll 2
-      for (int u = 0; u < T_CHUNK_TILES; ++u) step(kt0 + u);
-      close_chunk();
-    }
-  } else {
-    for (int kt = 0; kt < ntiles; ++kt) {
+    for (int u = 0; u < T_CHUNK_TILES; ++u) step(kt0 + u);
+    close_chunk();
+  }
+  if (!WHOLE) {
+    for (int kt = whole; kt < ntiles; ++kt) {
       step(kt);
-      if ((kt + 1) % T_CHUNK_TILES == 0 || kt + 1 == ntiles) close_chunk();
+      if ((ASK && (kt + 1) % T_CHUNK_TILES == 0) || kt + 1 == ntiles) close_chunk();
     }
   }
   const int m0 = m_blk + wm * 16 * FM + r16, n0 = n_blk + wn * (SWIGLU ? 8 : 16) * FN + 4 * kg;
@@ -1411,28 +1414,6 @@ static int gemm_fine(int fm, int fn, bool swiglu, elem_t* out, const elem_t* act
   FINE(2, 4);
 #undef FINE
   return vk_fail("gemm: no tile of %d by %d fragments", fm, fn);
-}
-
-// Which products go by these tiles.  Up to 64 rows the kernels that share activations through LDS are ahead where K is long: 64 rows, 1,024 x 1,024 17.4, 11.5 us,
-// 3,072 x 1,536 19.1, 16.5, 2,048 x 2,048 18.3, 20.2, 4,096 x 12,288 100, 128; with SwiGLU 6,144 x 2,048 64, 52, 12,288 x 4,096 175, 130; up to 32 rows
-// always (20 rows, 4,096 x 1,024 11.0, 11.2, 2,048 x 6,144 36.6, 59.3).
-static bool fine_takes(int M, int K, int64_t lda, bool swiglu) {
-  return K % (2 * VK_SLAB) == 0 && !rows_far(lda) && (M > 64 || (M > 32 && (swiglu ? K % KC == 0 : K <= 3 * KC)));
-}
-// The tile whose launch ends first: a unit's share is ceil(tiles / units) tiles, a tile's time is its products' (FM x FN fragments), and below a share that depends
-// on the tile a K tile's wait for memory.  ns for 32 elements of K and a product of fragments, fitted to 84 products of 70 to 2,048 rows, 256 x 1,024 to
-// 12,288 x 2,048: {at least, in front, a tile}.  The tile so chosen against the best of the six: 1 % slower on the mean, 12 % at most.
-static void fine_tile(int M, int N, bool swiglu, int& fm, int& fn) {
-  static const struct { int fm, fn; double least, front, each; } kinds[6] = {{2, 4, 140, 10, 121}, {3, 2, 147, 15, 121}, {2, 2, 160, 20, 124},
-                                                                               {1, 4, 175, 20, 129}, {1, 2, 250, 50, 134}, {1, 1, 320, 180, 142}};
-  double best = 0.0;
-  for (const auto& k : kinds) {
-    if (swiglu && k.fn == 1) continue;
-    const int columns = (swiglu ? 16 : 32) * k.fn;
-    const int64_t tiles = (int64_t)((M + 32 * k.fm - 1) / (32 * k.fm)) * ((N + columns - 1) / columns);
-    const double time = k.fm * k.fn * std::max(k.least, k.front + k.each * (double)((tiles + vk_device_cus() - 1) / vk_device_cus()));
-    if (best == 0.0 || time < best) { best = time; fm = k.fm; fn = k.fn; }
-  }
 }
 #endif
 
@@ -2553,10 +2534,67 @@ static int pipe_fragments_in_one_round(int M, int N, int K) {
   const int64_t mb = (M + 127) / 128;
   if ((N + 63) / 64 * mb <= vk_device_cus()) return 2;
   if ((N + 95) / 96 * mb <= vk_device_cus()) return 3;
-  // K of up to two chunks and K not in whole chunks are as fast with two workgroups of 64 rows a unit (two stages).
-  if (K % KC == 0 && K > 2 * KC && (N + 127) / 128 * mb <= vk_device_cus()) return 4;
+  // 32-bit elements (which the smaller tiles of gemm_fine_kernel leave with more workgroups than that only), K of up to two chunks and K not in whole chunks are as fast with two
+  // workgroups of 64 rows a unit (two stages).
+  if (sizeof(elem_t) == 2 && K % KC == 0 && K > 2 * KC && (N + 127) / 128 * mb <= vk_device_cus()) return 4;
   return 0;
 }
+
+#ifdef VK_F32
+// Which products go by gemm_fine_kernel's tiles or by those of 128 rows (fine_tile says which).  Whole chunks: up to 64 rows the kernels that share activations through LDS are
+// ahead where K is long (those kernels against these tiles, us: 64 rows, 1,024 x 1,024 17.4, 11.5, 3,072 x 1,536 19.1, 16.5, 2,048 x 2,048 18.3, 20.2, 4,096 x 12,288 100, 128; with SwiGLU 6,144 x 2,048 64, 52,
+// 12,288 x 4,096 175, 130), up to 32 rows always (20 rows, 4,096 x 1,024 11.0, 11.2, 2,048 x 6,144 36.6, 59.3); from 65 rows on they are nowhere by more than 2 % (350 sizes of 65
+// to 256 rows, 256 x 1,024 to 12,288 x 12,288: 1.45 times as fast on the mean; 65 rows, 4,096 x 12,288 147, 136, 128 rows, 8,192 x 8,192 181, 184).  K not in whole chunks, 33 to 64
+// rows: the streaming kernels share K among eight waves, which few weight rows need (48 rows and fewer, K of two to three chunks: 33 rows, 1,024 x 1,504 14.1, 17.3, 4,096 x 1,504 16.4,
+// 18.6, 5,840 x 1,280 29.4, 20.1; 64 rows, 2,048 x 1,280 18, 15.3), and K above three chunks up to as many as tiles of 128 fill half of the units; there it was tiles of 128
+// x 64 (64 rows, 16,384 x 2,080 76.9, 48.6, 6,176 220, 138).
+static bool fine_takes(int M, int N, int K, int64_t lda, bool swiglu) {
+  if (K % (2 * VK_SLAB) != 0 || rows_far(lda) || M <= 32) return false;
+  if (M > 64) return true;
+  const int cus = vk_device_cus();
+  if (K % KC == 0) return swiglu || K <= 3 * KC;
+  if (K > 3 * KC) return 2 * ((N + 127) / 128) >= cus;
+  return K <= 2 * KC || M > 48 || (N + 15) / 16 > cus;
+}
+// The tile whose launch ends first: a unit's share is ceil(tiles / units) tiles, a tile's time is its products' (FM x FN fragments), and below a share that depends
+// on the tile a K tile's wait for memory.  ns for 32 elements of K and a product of fragments, fitted to 84 products of 70 to 2,048 rows, 256 x 1,024 to
+// 12,288 x 2,048: {at least, in front, a tile}.  The tile so chosen against the best of the six: 2 % slower on the mean, 20 % at most (645 products of up to 20,480 x 4,096).
+// false: a tile of 128 rows by gemm_pipe_kernel is the faster one (M above 64, and not where those leave units with one workgroup).  Larger tiles are ahead where they fill
+// the units' rounds: 512 rows, 10,240 x 2,080, 256 tiles of 128 x 160 172 us, small ones 189; 2,048 rows, 4,096 x 544, 1,024 of 128 x 128 72.2, 86.2; with SwiGLU 512 rows,
+// 8,192 x 544 73.3, 85.3.  Their time, good to 2 %: two workgroups a unit (three with 64 weight rows) at a time, a round's fixed cost, and
+// {in front, a tile} as above.  The small tiles' is good to 10 %, hence the factors, by which 15 of 2,619 products (33 to 2,048 rows) take 3 to 8 % longer
+// than without small tiles, all but three of them of K up to 544; with small ones alone 42 of 900 take 3 to 16 % longer.
+static bool fine_tile(int M, int N, int K, bool swiglu, int& fm, int& fn) {
+  static const struct { int fm, fn; double least, front, each; } kinds[6] = {{2, 4, 140, 10, 121}, {3, 2, 147, 15, 121}, {2, 2, 160, 20, 124},
+                                                                               {1, 4, 175, 20, 129}, {1, 2, 250, 50, 134}, {1, 1, 320, 180, 142}};
+  auto share = [](int64_t tiles) { return (tiles + vk_device_cus() - 1) / vk_device_cus(); };
+  double best = 0.0;
+  for (const auto& k : kinds) {
+    if (swiglu && k.fn == 1) continue;
+    const int columns = (swiglu ? 16 : 32) * k.fn;
+    const int64_t tiles = (int64_t)((M + 32 * k.fm - 1) / (32 * k.fm)) * ((N + columns - 1) / columns);
+    const double time = k.fm * k.fn * std::max(k.least, k.front + k.each * (double)share(tiles));
+    if (best == 0.0 || time < best) { best = time; fm = k.fm; fn = k.fn; }
+  }
+  if (M <= 64) return true;
+  best *= K / 32 * 1e-3;                                             // us
+  const int64_t row_blocks = (M + 127) / 128;
+  auto tall = [&](int products, int64_t tiles, int resident, double front, double each, double round) {
+    const int64_t rounds = share(tiles) / resident, rest = share(tiles) % resident;
+    return products * (K / 32) * 1e-3 * ((double)rounds * (front + each * resident) + (rest ? std::max(120.0, front + each * (double)rest) : 0.0)) +
+           round * (double)(rounds + (rest > 0));
+  };
+  if (swiglu) {
+    const int64_t tiles = row_blocks * ((N + 63) / 64);
+    return tall(16, tiles, 2, 17, 109, 5.3) >= (share(tiles) == 2 ? 1.05 : 1.0) * best;
+  }
+  if (pipe_fragments_in_one_round(M, N, K) != 0) return true;
+  if ((N + 127) / 128 * row_blocks <= vk_device_cus()) return tall(8, row_blocks * ((N + 63) / 64), 3, 3, 119, 4.3) >= 1.06 * best;
+  const int f = pipe_fragments_by_rounds(M, N);
+  const int64_t tiles = row_blocks * ((N + 32 * f - 1) / (32 * f));
+  return tall(4 * f, tiles, 2, 17, 109, 5.3) >= (100 * tiles >= 95 * share(tiles) * vk_device_cus() ? 1.14 : 1.06) * best;
+}
+#endif
 
 #ifdef VK_BF16
 // How many weight fragments a wave of the alternating kernel takes (6, 5 or 4), or 0: the tile kernel is the faster one.  Both kernels' times go in
@@ -2709,10 +2747,9 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   const int form = out_form_of(out, ldo, activation);
   const bool by_size = kernel == 0;
 #ifdef VK_F32
-  if (kernel == 0 && fine_takes(M, K, lda, false)) {
+  if (kernel == 0 && fine_takes(M, N, K, lda, false)) {
     int fm = 0, fn = 0;
-    fine_tile(M, N, false, fm, fn);
-    return gemm_fine(fm, fn, false, out, act, w, M, N, K, lda, ldo, form, st);
+    if (fine_tile(M, N, K, false, fm, fn)) return gemm_fine(fm, fn, false, out, act, w, M, N, K, lda, ldo, form, st);
   }
 #endif
   if (kernel == 0) {
@@ -2862,12 +2899,14 @@ static int gemm_launch(elem_t* out, const elem_t* act, const elem_t* w, int M, i
   if (kernel == 6 && k_whole) return launch_pipe<4>(out, act, w, M, N, K, lda, ldo, form, st);
   // Two stages of 32 KB leave room for two workgroups per compute unit, which hides more latency than a third stage.
   if (k_whole) {
+#ifdef VK_BF16
     if (by_size) {
       const int f = pipe_fragments_in_one_round(M, N, K);
       if (f == 2) return launch_pipe<4, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
       if (f == 3) return launch_pipe<4, false, 3>(out, act, w, M, N, K, lda, ldo, form, st);
       if (f == 4) return launch_pipe<4>(out, act, w, M, N, K, lda, ldo, form, st);
     }
+#endif
     // No more 128 x 128 tiles than compute units: 64 weight rows a workgroup, twice as many of them.
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
     if (kernel == 13 || (by_size && tiles <= vk_device_cus())) return launch_pipe<2, false, 2>(out, act, w, M, N, K, lda, ldo, form, st);
@@ -2893,10 +2932,20 @@ int vk_gemm_fine(elem_t* out, const elem_t* act, const elem_t* w, int M, int N, 
              "gemm: bad sizes M=%d N=%d K=%d for tiles of 32-bit elements", M, N, K);
   VK_REQUIRE(((uintptr_t)act % 16) == 0 && ((uintptr_t)w % 16) == 0, "gemm: operands must be 16-byte aligned");
 #ifdef VK_F32
-  if (fm == 0) fine_tile(M, N, swiglu != 0, fm, fn);
+  if (fm == 0) (void)fine_tile(M, N, K, swiglu != 0, fm, fn);
   return gemm_fine(fm, fn, swiglu != 0, out, act, w, M, N, K, lda, ldo, out_form_of(out, ldo, 0), st);
 #else
   return 1;
+#endif
+}
+
+// 1 if a product chosen by size goes by those tiles.
+int vk_gemm_fine_takes(int M, int N, int K, int64_t lda, int swiglu) {
+#ifdef VK_F32
+  int fm = 0, fn = 0;
+  return M > 0 && N > 0 && K > 0 && fine_takes(M, N, K, lda, swiglu != 0) && fine_tile(M, N, K, swiglu != 0, fm, fn);
+#else
+  return 0;
 #endif
 }
 
@@ -2939,19 +2988,19 @@ int vk_gemm_swiglu(elem_t* out, const elem_t* act, const elem_t* w, int M, int I
   }
 #endif
 #ifdef VK_F32
-  if (fine_takes(M, K, lda, true)) {
+  if (fine_takes(M, I, K, lda, true)) {
     int fm = 0, fn = 0;
-    fine_tile(M, I, true, fm, fn);
-    return gemm_fine(fm, fn, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+    if (fine_tile(M, I, K, true, fm, fn))
+      return gemm_fine(fm, fn, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
   }
 #endif
   if (how == 2 && rows_far(lda)) {
     VK_REQUIRE(K % KC == 0, "gemm_swiglu: rows %lld elements apart need K in whole chunks of %d", (long long)lda, KC);
     return launch_mid<4, 1, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
   }
-#ifdef VK_BF16
   if (how == 2)
     return launch_pipe<2, true>(out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
+#ifdef VK_BF16
   if (const int width = how == 3 ? rows_width(M, I, K, lda, true) : 0)
     return gemm_rows(width, true, out, act, w, M, I, K, lda, ldo, (ldo % 4 == 0) && ((uintptr_t)out % 16 == 0), st);
 #endif
