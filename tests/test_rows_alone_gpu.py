@@ -72,3 +72,32 @@ def test_projected_rows_without_a_list(nq, nkv, d, dtype):
                        items.data_ptr() if listed else None, S, nseg, scratch.data_ptr(), nq, nkv, d, P, 0, d ** -0.5, stream) == 0
             got.append((out, kc1, vc1))
         assert not torch.isnan(got[0][0]).any() and all(torch.equal(a, b) for a, b in zip(*got)), n
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [[0, 5, 300], [130, 0, 700], [64, 0, 2100, 0]], ids=["two", "three", "nine"])
+@pytest.mark.parametrize("nq,nkv,d,P,window,keep", [(8, 2, 128, 64, 0, 0), (4, 4, 48, 16, 64, 7), (6, 1, 256, 64, 300, 70)])
+def test_a_sequence_without_keys(nq, nkv, d, P, window, keep, n, dtype):
+    """Its row is zeros, whatever its pages hold, and the other rows are what they are beside sequences with a key."""
+    k, S = kern(dtype), len(n)
+    lib, stream, nseg = k.lib, torch.cuda.current_stream().cuda_stream, -(-max(n) // 256)
+    keys, values = ([rand((m, nkv, d), dtype, s + j) for j, m in enumerate(n)] for s in (40, 140))
+    kc, vc, table = (x.cuda() for x in build_cache(keys, values, P, sum(-(-m // P) for m in n) + 3, 3, dtype, float("nan")))
+    q = torch.cat([rand((1, nq, d), dtype, 10 + j) for j in range(S)]).cuda()
+    cu, items = torch.arange(S + 1, dtype=torch.int32, device="cuda"), torch.stack([torch.arange(S), torch.zeros(S)], 1).to(torch.int32).cuda()
+    sinks, empty = torch.linspace(-1, 1, nq, device="cuda"), torch.tensor([m == 0 for m in n], device="cuda")
+    plain, capped = lib.vk_paged_attention, lib.vk_paged_attention_capped
+    plain.argtypes, capped.argtypes = [P_] * 5 + [I, *LISTS, I, F, P_], [P_] * 5 + [I, *LISTS, I, I, F, F, P_, I, P_]
+
+    def run(fn, lengths, listed, mode, *rest):
+        out, scratch = torch.full_like(q, float("nan")), torch.full((k.attn_scratch_floats(S, nq, d, nseg),), float("nan"), device="cuda")
+        k_len = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+        assert fn(out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), table.shape[1], cu.data_ptr() if listed else None, k_len.data_ptr(),
+                  items.data_ptr() if listed else None, S, mode, nseg, scratch.data_ptr(), S, nq, nkv, d, P, *rest, stream) == 0
+        return out
+
+    calls = [(plain, mode, window, d ** -0.5) for mode in (1, 3, 4, 5, 7)] + [(capped, 1, window, keep, d ** -0.5, 5.0, sinks.data_ptr(), 1)]
+    for fn, *rest in calls:
+        for listed in (True, False):
+            out, beside = run(fn, n, listed, *rest), run(fn, [max(m, 1) for m in n], listed, *rest)
+            assert not out[empty].any() and torch.equal(out[~empty], beside[~empty]) and not torch.isnan(out[~empty]).any(), rest

@@ -49,6 +49,7 @@
 #include "vec.h"
 
 #define TILE_KEYS 64
+#define TILE_SHIFT 6                      // log2 of it
 #define SEG_TILES 4
 #define KEY_SLABS (TILE_KEYS / VK_SLAB)   // key slabs per tile: 2 (bfloat16) or 4 (float)
 #define S_PER_LANE 16                     // scores per lane per tile
@@ -95,6 +96,10 @@ __device__ __forceinline__ void decoded_row(const AttnArgs& a, int item, int& se
     back = a.cu_q[seq + 1] - tok;
   }
 }
+
+// The tile of the key at `pos`; -1 for the row of a sequence without keys, which stands at -1 and sees none (a division would round that up to tile 0).
+__device__ __forceinline__ int tile_of_key(int pos) { return pos >> TILE_SHIFT; }
+static_assert(TILE_KEYS == 1 << TILE_SHIFT, "keys of a tile");
 
 // Decoded rows as the projections leave them: what vk_qkv_post does to them (head norm, rotation by tables, the store of key and value) happens in the
 // attention's own launch.
@@ -976,7 +981,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_plain_kernel(Att
   decoded_row(a, blockIdx.x, seq, tok, back);
   const int k_len = a.k_len[seq], pos = k_len - back;
   const int lo = first_visible(a, pos);
-  const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
+  const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(tile_of_key(pos), seg * SEG_TILES + SEG_TILES - 1);
   if (t0 > t1) return;   // whole wave; no barrier follows
 
   RowCtx c;
@@ -1026,7 +1031,7 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
   decoded_row(a, blockIdx.x, seq, tok, back);
   const int k_len = a.k_len[seq], pos = k_len - back;
   const int lo = first_visible(a, pos);
-  const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
+  const int t0 = max(lo / TILE_KEYS, seg * SEG_TILES), t1 = min(tile_of_key(pos), seg * SEG_TILES + SEG_TILES - 1);
   if (t0 > t1) return;   // whole wave; no barrier follows
 
   RowCtx c;
@@ -1208,7 +1213,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
   const int lo = first_visible(a, pos);
   const int keep = a.window > 0 ? a.keep : 0;
   const int keep_tiles = (keep + TILE_KEYS - 1) / TILE_KEYS, tile_lo = lo / TILE_KEYS;
-  const int t0 = seg * SEG_TILES, t1 = min(pos / TILE_KEYS, seg * SEG_TILES + SEG_TILES - 1);
+  const int t0 = seg * SEG_TILES, t1 = min(tile_of_key(pos), seg * SEG_TILES + SEG_TILES - 1);
   if (t0 > t1 || (t0 >= keep_tiles && t1 < tile_lo)) return;   // whole wave; no barrier follows
 
   RowCtx c;
@@ -1392,7 +1397,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j) {
     const int t = first_tile + j;
-    if (t <= pos / TILE_KEYS && (t < keep_tiles || t >= tile_lo)) wanted |= 1u << j;
+    if (t <= tile_of_key(pos) && (t < keep_tiles || t >= tile_lo)) wanted |= 1u << j;
   }
   wanted = __builtin_amdgcn_readfirstlane(wanted);
   if (SEGS == 1 && wanted == 0) return;   // the whole workgroup
@@ -1411,7 +1416,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   const bool mine = (wanted >> wave) & 1u;
   frag_t qf[NQS];
   frag_t kf[KSUB][NQS];
-  const int own_tile = pos / TILE_KEYS - first_tile;          // the segment's tile with the row's own key, where that is 0 .. SEG_TILES - 1
+  const int own_tile = tile_of_key(pos) - first_tile;          // the segment's tile with the row's own key, where that is 0 .. SEG_TILES - 1
   frag_t cosines, sines;
   if constexpr (ROWS) {
     // In front of the keys: loads arrive in the order in which they are asked for.
@@ -1434,7 +1439,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   const int own_page = slot >> lp, own_off = slot & (a.P - 1);
   if constexpr (ROWS) {
     // The workgroup that holds the row's own key, in either segment, stores it.
-    const int own_of_all = pos / TILE_KEYS - (int)blockIdx.z * SEGS * SEG_TILES;
+    const int own_of_all = tile_of_key(pos) - (int)blockIdx.z * SEGS * SEG_TILES;
     const bool stores = ht == 0 && slot >= 0 && own_of_all >= 0 && own_of_all < SEGS * SEG_TILES;
     for (int first = 0; first <= q_rows; first += SEGS * SEG_TILES * ROWS_A_WAVE) {
       if (first > 0) load_piece(first);
@@ -1682,10 +1687,10 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a) {
   const int lo = first_visible(a, pos);
   // Segments that hold kept first keys come before the window's; those in between were not computed.
   const int keep_tiles = a.window > 0 ? (a.keep + TILE_KEYS - 1) / TILE_KEYS : 0, tile_lo = lo / TILE_KEYS;
-  const int seg_begin = keep_tiles > 0 ? 0 : lo / (TILE_KEYS * SEG_TILES), seg_end = pos / (TILE_KEYS * SEG_TILES) + 1;
+  const int seg_begin = keep_tiles > 0 ? 0 : lo / (TILE_KEYS * SEG_TILES), seg_end = pos < 0 ? 0 : pos / (TILE_KEYS * SEG_TILES) + 1;
   if (!few) {
     seg0 = seg_begin;
-    fetch(seg0, seg_end - 1);
+    fetch(seg0, max(seg_end - 1, 0));
   }
   for (;;) {
 #pragma unroll
@@ -1759,7 +1764,7 @@ static int64_t quad_segments(int d) {
 //   the kernel is chosen by shape.  mode 2: the same through the kernel that takes every shape,
 //   modes 6, 8 and 9: through the one that shares tiles in LDS with four waves, with eight, and with four and
 //   one buffer instead of two, whatever the shape (tests and measurements; the result is the same bits).
-// mode 1: each item is one token (items and cu_q null: item i is the one row of sequence i, and its token is row i); the keys are split by segment over nseg workgroups (nseg must cover
+// mode 1: each item is one token (items and cu_q null: item i is the one row of sequence i, and its token is row i), zeros where its sequence has no keys; the keys are split by segment over nseg workgroups (nseg must cover
 //   the longest sequence; scratch must hold vk_attn_scratch_floats(n_items, ...)) and folded by a
 //   second kernel; the kernel is chosen by shape.  modes 3, 4, 5, 7: the same through a named kernel
 //   (3 and 4: a wave per segment that asks for a tile's fragments when it needs them, the kernel for every
