@@ -101,3 +101,21 @@ def test_a_sequence_without_keys(nq, nkv, d, P, window, keep, n, dtype):
         for listed in (True, False):
             out, beside = run(fn, n, listed, *rest), run(fn, [max(m, 1) for m in n], listed, *rest)
             assert not out[empty].any() and torch.equal(out[~empty], beside[~empty]) and not torch.isnan(out[~empty]).any(), rest
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_lists_that_are_refused(dtype):
+    """Prompt rows without items, rows without items that are not all of them, items without their sequences' first rows."""
+    k, P, d = kern(dtype), 64, 64
+    lib, stream = k.lib, torch.cuda.current_stream().cuda_stream
+    cache, q, scratch = torch.zeros(2, 1, P, d, dtype=dtype, device="cuda"), torch.zeros(2, 3, d, dtype=dtype, device="cuda"), torch.zeros(4096, device="cuda")
+    ints = torch.ones(2, 2, dtype=torch.int32, device="cuda")
+    plain, capped, rows = lib.vk_paged_attention, lib.vk_paged_attention_capped, lib.vk_paged_attention_rows
+    plain.argtypes, capped.argtypes = [P_] * 5 + [I, *LISTS, I, F, P_], [P_] * 5 + [I, *LISTS, I, I, F, F, P_, I, P_]
+    for fn, rest in ((plain, (0, 1.0)), (capped, (0, 0, 1.0, 0.0, None, 0))):
+        for listed, cu, n_items, mode in ((False, True, 2, 0), (False, False, 1, 1), (False, False, 3, 1), (True, False, 2, 1), (True, False, 2, 0)):
+            assert fn(q.data_ptr(), q.data_ptr(), cache.data_ptr(), cache.data_ptr(), ints.data_ptr(), 2, ints.data_ptr() if cu else None, ints.data_ptr(),
+                      ints.data_ptr() if listed else None, n_items, mode, 1, scratch.data_ptr(), 2, 3, 1, d, P, *rest, stream) != 0, (listed, cu, n_items, mode)
+    rows.argtypes = [P_, P_, ctypes.c_int64, P_, P_, P_, P_, F, P_, P_, P_, P_, P_, I, P_, P_, P_, I, I, P_, I, I, I, I, I, F, P_]
+    assert rows(q.data_ptr(), q.data_ptr(), 5 * d, cache.data_ptr(), cache.data_ptr(), None, None, 1e-6, None, None, ints.data_ptr(), ints.data_ptr(), ints.data_ptr(), 2,
+                None, ints.data_ptr(), ints.data_ptr(), 1, 1, scratch.data_ptr(), 3, 1, d, P, 0, 1.0, stream) != 0

@@ -1786,6 +1786,8 @@ int vk_paged_attention(elem_t* out, const elem_t* q, const elem_t* kc, const ele
   if (mode >= 3) mode = 1;
   if (n_items <= 0) return 0;
   VK_REQUIRE(mode == 1 || items != nullptr, "attention: prompt rows need items");
+  VK_REQUIRE(items != nullptr ? cu_q != nullptr : n_items == total_tokens, "attention: items need their sequences' first rows; without items every one of the %d rows is one, not %d",
+             total_tokens, n_items);
   AttnArgs a;
   a.q = q; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
   a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
@@ -1974,6 +1976,7 @@ int vk_paged_attention_rows(elem_t* out, const elem_t* qkv, int64_t row_stride, 
   VK_REQUIRE(row_stride >= (int64_t)(nq + 2 * nkv) * d && row_stride % VK_VEC == 0, "attention: row stride %lld too small or uneven", (long long)row_stride);
   VK_REQUIRE((((uintptr_t)qkv | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)q_w | (uintptr_t)k_w | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16) == 0,
              "attention: operands must be 16-byte aligned");
+  VK_REQUIRE(items == nullptr || cu_q != nullptr, "attention: items need their sequences' first rows");
   VK_REQUIRE((cos_t == nullptr) == (sin_t == nullptr) && (cos_t == nullptr || positions != nullptr) && slots != nullptr, "attention: a rotation needs tables and positions, a store slots");
   AttnArgs a;
   a.q = nullptr; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
@@ -2008,7 +2011,6 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
                                    int nseg, float* scratch, int total_tokens, int nq, int nkv, int d, int P, int window, int keep, int block,
                                    float scale, float softcap, const void* sinks, int sinks_f32, hipStream_t st, const float* rel = nullptr,
                                    int rel_stride = 0, int rel_far = 0, const elem_t* gate = nullptr, int64_t gate_stride = 0) {
-  (void)total_tokens;
   VK_REQUIRE(block >= 0 && (block == 0 || window == 0), "attention: blocks of positions (%d) and a window (%d) exclude each other", block, window);
   VK_REQUIRE(nq > 0 && nkv > 0 && nq % nkv == 0, "attention: %d q heads are not a multiple of %d kv heads", nq, nkv);
   VK_REQUIRE(d >= 16 && d <= 256 && d % 16 == 0, "attention: head size %d must be a multiple of 16 in 16..256", d);
@@ -2022,6 +2024,8 @@ static int attention_capped_launch(elem_t* out, const elem_t* q, const elem_t* k
   VK_REQUIRE(gate == nullptr || gate_stride >= nq, "attention: a gate a head needs rows of at least %d", nq);
   if (n_items <= 0) return 0;
   VK_REQUIRE(mode == 1 || items != nullptr, "attention: prompt rows need items");
+  VK_REQUIRE(items != nullptr ? cu_q != nullptr : n_items == total_tokens, "attention: items need their sequences' first rows; without items every one of the %d rows is one, not %d",
+             total_tokens, n_items);
   AttnArgs a;
   a.q = q; a.out = out; a.kc = kc; a.vc = vc; a.block_table = block_table; a.cu_q = cu_q; a.k_len = k_len;
   a.items = items; a.bt_stride = bt_stride; a.nq = nq; a.nkv = nkv; a.d = d; a.P = P; a.window = window;
