@@ -73,6 +73,14 @@ def test_rows_without_a_slot_and_a_launch_for_longer_requests(dtype):
     assert both(dtype, [40, 65, 120], 8, 4, 128, 64, 0, True, True, table_pages=13) == (True, True, True)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq,nkv,d,norms", [(8, 2, 128, True), (16, 1, 128, True), (17, 1, 64, False), (6, 2, 64, True)])
+@pytest.mark.parametrize("window", [0, 40, 70, 300])
+def test_waves_without_a_tile(nq, nkv, d, norms, window, dtype):
+    """A workgroup a segment in which one to three of the four waves have none: behind the row's own key, and in front of its window."""
+    assert both(dtype, [1, 40, 65, 130, 190, 257, 330, 700], nq, nkv, d, 64, window, norms, True, table_pages=13) == (True, True, True)
+
+
 def test_what_is_not_taken():
     """Heads of other sizes, pages smaller than a tile and more segments than go with four waves each are refused."""
     assert both(torch.bfloat16, [40], 8, 4, 96, 64, 0, True, True) is None

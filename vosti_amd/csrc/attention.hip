@@ -1324,8 +1324,9 @@ __device__ __forceinline__ unsigned keys_before(int end) {
 // a lane VK_VEC elements, and pass them through LDS; the segment that holds a row's own key puts that key and value among its tile's, and the first of a kv
 // head's workgroups stores them.  A launch of its own for that, between the projection and the attention, took 3.8 us of one row of 32 heads and 5.1 of eight
 // of 48.  With every wave norming and turning all its heads' rows for itself one
-// row of 30 keys, 16 heads on 8, took 7.9 us beside its neighbours and takes 5.8 with what stands at decoded_row and OwnedMask; of 300 11.1 -> 9.9, 40 of 300, 32 on 8, 23.1 -> 21.3;
-// but 8 of 530, three segments of full tiles, 11.2 -> 11.7, which wait for the slowest wave's rows.
+// row of 30 keys, 16 heads on 8, took 8.3 us beside its neighbours and takes 5.8 with what stands at decoded_row and OwnedMask; of 300 11.0 -> 9.3, 8 of 530, 32 on 8, 12.8 -> 12.3,
+// of 700 14.5 -> 12.8, 40 of 300 23.1 -> 21.2; 32-bit, 3 of 700 20.2 -> 18.1.  (As long as waves without a tile asked for no keys, the rows waited for all keys: 8 of 530 13.3, of
+// 700 14.4, 32-bit 3 of 700 19.1; only 40 of 300, whose second segments have one tile of four, 20.7.)
 // FAR: the launch covers the kept segments and those that a window or a block can touch, not all before it.  (Known when the kernel is built:
 // the page numbers then wait for the lengths, 0.4 us of a short request's 12.)
 template <int DPAD, bool EXACT, bool EXT, bool REL, int SEGS = 1, bool FAR = false, bool ROWS = false>
@@ -1427,13 +1428,20 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (mine) {
+  // Rows: a wave without a tile asks for one key of the first tile that is wanted, over and over, so that it is known how many reads stand behind the rows'.  (A wait for an
+  // unknown number is one for all of them, and the barrier behind the rows then makes every wave wait for everybody's keys.  With both segments in one workgroup the second
+  // may have no tile at all, and its waves' reads cost more than they save.)
+  constexpr bool ALWAYS = ROWS && SEGS == 1;
+  if (ALWAYS || mine) {
     if constexpr (!ROWS) load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
+    const int of = ALWAYS && !mine ? __builtin_ctz(wanted) : wave, first_key = (first_tile + of) * TILE_KEYS;
     int my_page = page[0];
 #pragma unroll
-    for (int j = 1; j < SEG_TILES; ++j) my_page = wave == j ? page[j] : my_page;
-    if (EXACT || a.P >= TILE_KEYS) load_keys<NQS, EXACT, true>(c, (first_tile + wave) * TILE_KEYS, kf, my_page);
-    else load_keys<NQS, EXACT>(c, (first_tile + wave) * TILE_KEYS, kf);
+    for (int j = 1; j < SEG_TILES; ++j) my_page = of == j ? page[j] : my_page;
+    RowCtx ck = c;
+    if (ALWAYS && !mine) ck.k_len = first_key + 1;
+    if (EXACT || a.P >= TILE_KEYS) load_keys<NQS, EXACT, true>(ck, first_key, kf, my_page);
+    else load_keys<NQS, EXACT>(ck, first_key, kf);
   }
   __builtin_amdgcn_sched_barrier(0);
   const int own_page = slot >> lp, own_off = slot & (a.P - 1);
@@ -1441,14 +1449,19 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     // The workgroup that holds the row's own key, in either segment, stores it.
     const int own_of_all = tile_of_key(pos) - (int)blockIdx.z * SEGS * SEG_TILES;
     const bool stores = ht == 0 && slot >= 0 && own_of_all >= 0 && own_of_all < SEGS * SEG_TILES;
-    for (int first = 0; first <= q_rows; first += SEGS * SEG_TILES * ROWS_A_WAVE) {
-      if (first > 0) load_piece(first);
+    auto turn_rows = [&](int first) {
       const int r = first + my_row;
       const frag_t x = piece.finish((q_weight | k_weight) != 0, (r < q_rows ? q_weight : k_weight) != 0, rows.cos_t != nullptr, cosines, sines,
                                     rows.eps, piece_at);
       if (r <= q_rows) *reinterpret_cast<frag_t*>(&turned[r][piece_at * VK_VEC]) = x;
       if (r == q_rows && stores)
         *reinterpret_cast<frag_t*>(rows.kc + (((int64_t)own_page * a.nkv + kvh) * a.P + own_off) * DPAD + piece_at * VK_VEC) = x;
+    };
+    turn_rows(0);                       // (apart from the others, which are read behind the keys)
+    constexpr int A_PASS = SEGS * SEG_TILES * ROWS_A_WAVE;
+    for (int first = A_PASS; A_PASS <= 16 && first <= q_rows; first += A_PASS) {
+      load_piece(first);
+      turn_rows(first);
     }
     if (own_tile >= 0 && own_tile < SEG_TILES && stores && c.g == 0) {
 #pragma unroll
@@ -1947,14 +1960,15 @@ int vk_paged_attention_rows_takes(int n_items, int nseg, int nq, int nkv, int d,
   return (int64_t)n_items * (nkv * ((nq / nkv + 15) / 16)) * nseg <= quad_segments(d);
 }
 
-// 1 if it is also the faster way.  A row's norm and turn stand in front of its attention, in registers that leave room for two workgroups a compute unit (heads of
+// 1 if it is also the faster way.  A row's norm and turn stand in front of its attention, once a workgroup, of which a compute unit holds up to three (heads of
 // 256 bytes) or one (512); a launch of its own does them for all rows at once.  vk_qkv_post and vk_paged_attention over the one launch, 8, 16, 32 and 40 heads on 8 and
 // 32 on 2, 1 to 80 rows of 30 to 4,000 keys, by segments of the launch against the compute units, cus:
-//   heads of 128 bytes   0.95 to 1.17 wherever four waves go to a segment (one size below 0.98)
-//   of 256, 16-bit       1.01 to 1.23 (one row of 200 keys, 16 on 8: 11.1 -> 9.4 us; of 500 15.6 -> 13.5); one segment a row and more than 2 cus: 0.77 to 1.03
-//   of 256, 32-bit       up to 2 cus 0.97 to 1.12, more 0.76 to 0.93 (80 rows of 30 keys, 16 on 8: 14.1 -> 18.0 us)
-//   of 512               never folded.  Two segments a row and more, up to cus: 1.00 to 1.16 (two rows of 500 keys, 16 on 8: 23.1 -> 19.9 us); up to 2 cus 0.97 to 1.07, more 0.95
-//                        to 0.98; one segment: 0.78 to 0.94 with 30 keys, 0.95 to 1.10 with 200
+//   heads of 128 bytes   1.15 to 1.39 wherever four waves go to a segment
+//   of 256, 16-bit       1.10 to 1.39 (one row of 200 keys, 16 on 8, 10.5 -> 8.6 us), the less the more segments; one segment a row and more than 2 cus, left out: 1.14 to 1.21
+//   of 256, 32-bit       up to 2 cus 1.02 to 1.23, more, left out, 1.02 to 1.10
+//   of 512               never folded.  Two segments a row and more, up to cus: 0.99 to 1.20; more, left out, 0.92 to 1.11; one segment, left out: up to cus 0.97 (30 keys, 32 on 2)
+//                        to 1.09, more 0.93 to 1.00
+// What is left out was 0.76 to 1.03 while every wave normed and turned all its heads' rows for itself.
 int vk_paged_attention_rows_preferred(int n_items, int nseg, int nq, int nkv, int d, int P) {
   if (!vk_paged_attention_rows_takes(n_items, nseg, nq, nkv, d, P)) return 0;
   const int64_t segments = (int64_t)n_items * (nkv * ((nq / nkv + 15) / 16)) * nseg, cus = vk_device_cus();
