@@ -1680,10 +1680,10 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a) {
   // empty segment's place holds is not used); a launch of at most four segments asks for all of them before the sequence's length is there.
   // Reads one after the other, the length's and the item's among them, are most of the launch.
   float m[4], l[4], v[4][4];
-  auto fetch = [&](int first, int last) {
+  auto fetch = [&](auto place) {              // place(j): the segment of place j
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int64_t r = row0 + min(first + j, last);
+      const int64_t r = row0 + place(j);
       m[j] = a.part_ml[2 * r];
       l[j] = a.part_ml[2 * r + 1];
 #pragma unroll
@@ -1693,35 +1693,38 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnArgs a) {
       }
     }
   };
+  auto take = [&](int j) {
+    if (!(m[j] > -INFINITY)) return;
+    float Mn, ca, cb;
+    fold_scales(M, m[j], Mn, ca, cb);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ACC[i] = fold1(ACC[i], v[j][i], ca, cb);
+    L = fold1(L, l[j], ca, cb);
+    M = Mn;
+  };
   const bool few = a.nseg <= 4;
-  int seg0 = 0;
-  if (few) fetch(0, a.nseg - 1);
+  if (few) fetch([&](int j) { return min(j, a.nseg - 1); });
   const int pos = a.k_len[seq] - back;
   const int lo = first_visible(a, pos);
-  // Segments that hold kept first keys come before the window's; those in between were not computed.
-  const int keep_tiles = a.window > 0 ? (a.keep + TILE_KEYS - 1) / TILE_KEYS : 0, tile_lo = lo / TILE_KEYS;
-  const int seg_begin = keep_tiles > 0 ? 0 : lo / (TILE_KEYS * SEG_TILES), seg_end = pos < 0 ? 0 : pos / (TILE_KEYS * SEG_TILES) + 1;
-  if (!few) {
-    seg0 = seg_begin;
-    fetch(seg0, max(seg_end - 1, 0));
-  }
-  for (;;) {
+  // The segments that were computed: those that hold kept first keys, then the window's (or all); those in between are not visited.
+  const int keep_tiles = a.window > 0 ? (a.keep + TILE_KEYS - 1) / TILE_KEYS : 0;
+  const int from = lo / (TILE_KEYS * SEG_TILES), to = pos < 0 ? 0 : pos / (TILE_KEYS * SEG_TILES) + 1;
+  const int kept = min((keep_tiles + SEG_TILES - 1) / SEG_TILES, from);
+  if (few) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int seg = seg0 + j;
-      const bool in = seg >= seg_begin && seg < seg_end && (seg * SEG_TILES < keep_tiles || seg * SEG_TILES + SEG_TILES > tile_lo);
-      if (in && m[j] > -INFINITY) {
-        float Mn, ca, cb;
-        fold_scales(M, m[j], Mn, ca, cb);
+    for (int j = 0; j < 4; ++j)
+      if (j < kept || (j >= from && j < to)) take(j);
+  } else {
+    const int count = kept + to - from;
+    for (int at = 0; at < count; at += 4) {
+      fetch([&](int j) {
+        const int i = min(at + j, count - 1);
+        return i < kept ? i : i - kept + from;
+      });
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ACC[i] = fold1(ACC[i], v[j][i], ca, cb);
-        L = fold1(L, l[j], ca, cb);
-        M = Mn;
-      }
+      for (int j = 0; j < 4; ++j)
+        if (at + j < count) take(j);
     }
-    seg0 += 4;
-    if (seg0 >= seg_end || few) break;
-    fetch(seg0, seg_end - 1);
   }
   if (a.sinks != nullptr && M > -INFINITY) L = L + sink_term(a, head, M);
   const float inv = (L > 0.f ? 1.0f / L : 0.f) * out_gate(a, tok, head);
