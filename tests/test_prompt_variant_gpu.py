@@ -31,7 +31,7 @@ def wanted(q, keys, values, window, keep, cap, sinks):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shapes", [FEW, MANY], ids=["few", "many"])
 @pytest.mark.parametrize("window,keep,cap", [(0, 0, 5.0), (70, 0, 0.0), (64, 64, 0.0), (100, 7, 20.0), (130, 200, 5.0), (1, 1, 0.0), (300, 65, 0.0)])
-@pytest.mark.parametrize("nq,nkv,d", [(4, 2, 64), (6, 1, 128), (32, 1, 256)])
+@pytest.mark.parametrize("nq,nkv,d", [(4, 2, 64), (6, 1, 128), (8, 2, 192), (32, 1, 256)])
 def test_shared_tiles_the_general_kernel_and_64_bits(nq, nkv, d, window, keep, cap, shapes, dtype):
     """Kept keys that end at a tile's edge, inside it and in the window; tiles seen whole among them; heads of 256 in a few items and in many."""
     k, total = kern(dtype), sum(r for r, _ in shapes)

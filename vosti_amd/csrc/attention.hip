@@ -129,13 +129,24 @@ __device__ __forceinline__ int first_visible(const AttnArgs& a, int pos) {
 }
 
 // Over the lanes l, l ^ 16, l ^ 32 and l ^ 48, which hold a row's numbers: (v + v of l ^ 16), and that + the same of l ^ 32, in every lane.
+// (LEAN, here and below: see lean_waves.)
+template <bool LEAN = false>
 __device__ __forceinline__ float row_sum(float v) {
+  if constexpr (LEAN) {
+    v = v + lane_xor16(v);
+    return v + lane_xor32(v);
+  }
   const unsigned u = __builtin_bit_cast(unsigned, v);
   v = pair_sum(__builtin_amdgcn_permlane16_swap(u, u, false, false));
   const unsigned w = __builtin_bit_cast(unsigned, v);
   return pair_sum(__builtin_amdgcn_permlane32_swap(w, w, false, false));
 }
+template <bool LEAN = false>
 __device__ __forceinline__ float row_max(float v) {
+  if constexpr (LEAN) {
+    v = fmaxf(v, lane_xor16(v));
+    return fmaxf(v, lane_xor32(v));
+  }
   const unsigned u = __builtin_bit_cast(unsigned, v);
   const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
   const unsigned a = r[0], b = r[1];
@@ -146,6 +157,14 @@ __device__ __forceinline__ float row_max(float v) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Heads of more than 128 entries in the kernels that read fragments straight from global memory: a tile's fragments alone fill a wave's registers, and what is made
+// ahead of its use is spilled.  There masks of values are made an element where they are used, and 32-bit waves, but for the variant's prompt rows, walk the
+// sub-tiles one after the other and have masks as conditions.  With masks ahead and sub-tiles side by side, us, then with this: 16-bit heads of 192, seven launches
+// of 30 to 4,000 prompt rows 903 -> 811, with capped scores 1,956 -> 1,158; 32-bit 3,563 -> 3,076 and 3,633 -> 3,285; 32-bit heads of 256 on pages of 16, capped, 23 launches
+// of 1 to 64 decoded rows of 30 to 6,000 keys 5,209 -> 4,799.  (16-bit decoded rows and heads of up to 128 are as fast or faster with masks ahead.)
+constexpr bool wide_heads(int dpad) { return dpad > 128; }
+constexpr bool lean_waves(int dpad) { return wide_heads(dpad) && sizeof(elem_t) == 4; }
 
 // What a wave needs to know about its 16 rows and its sequence's pages.
 struct RowCtx {
@@ -173,6 +192,7 @@ struct RowCtx {
 // multiply-add).  `full` (the same for the whole wave) says that every row of the wave sees every key of the
 // tile: then the masks are left out, which changes no bit.  A row that sees no key of the tile keeps its state
 // (ca = 1, probabilities 0).
+template <bool LEAN = false>
 __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int g, bool row_ok, int lo, int pos,
                                            float scale_log2, bool full, float& M, float& L, float& ca,
                                            frag_t (&pf)[KEY_SLABS]) {
@@ -183,7 +203,7 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
     float tmax = sc[0];
 #pragma unroll
     for (int i = 1; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
-    tmax = row_max(tmax);
+    tmax = row_max<LEAN>(tmax);
     const float m = tmax * scale_log2;
     Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
     ca = fast_exp2(M - Mn);                 // 1 where the maximum stands, 0 for a row whose state was empty
@@ -198,10 +218,11 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
       const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
-      vis[i] = (int)row_ok & (int)(key >= lo) & (int)(key <= pos);
+      if constexpr (LEAN) vis[i] = row_ok && key >= lo && key <= pos;
+      else vis[i] = (int)row_ok & (int)(key >= lo) & (int)(key <= pos);
       tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
     }
-    tmax = row_max(tmax);
+    tmax = row_max<LEAN>(tmax);
     const float m = tmax * scale_log2;      // -inf: the row sees no key of the tile
     Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
     ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
@@ -211,7 +232,7 @@ __device__ __forceinline__ void tile_probs(float (&sc)[S_PER_LANE], int kb, int 
       psum = psum + pr[i];
     }
   }
-  psum = row_sum(psum);
+  psum = row_sum<LEAN>(psum);
   L = __builtin_fmaf(L, ca, psum);
   M = Mn;
 #pragma unroll
@@ -278,6 +299,17 @@ struct OwnedMask {
   }
 };
 
+// The same of one column block, an element at a time.
+__device__ __forceinline__ void zero_unowned(frag_t (&vf)[KEY_SLABS], int kb, int g, int first, int k_len, int keep = 0) {
+#pragma unroll
+  for (int ks = 0; ks < KEY_SLABS; ++ks) {
+    const int k0 = kb + ks * VK_SLAB + g * VK_VEC;
+#pragma unroll
+    for (int j = 0; j < VK_VEC; ++j)
+      if (k0 + j >= k_len || (k0 + j < first && k0 + j >= keep)) vf[ks][j] = (elem_t)0.f;
+  }
+}
+
 // The pieces of a tile's work, for the kernels that read fragments straight from global memory.
 // No load is predicated on data: addresses of keys beyond k_len are clamped to a key of this
 // sequence (valid memory) and what they bring is masked or zeroed later.  A select on a loaded
@@ -340,10 +372,24 @@ __device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf
 }
 
 // Scores S^T[key, row] = K Q^T.
-template <int NQS, bool EXACT>
+template <int NQS, bool EXACT, bool LEAN = false>
 __device__ __forceinline__ void tile_scores(const RowCtx& c, const frag_t (&kf)[KSUB][NQS], const frag_t (&qf)[NQS],
                                             float (&sc)[S_PER_LANE]) {
   const int d = EXACT ? NQS * VK_SLAB : c.d;
+  if constexpr (LEAN) {
+#pragma unroll
+    for (int sub = 0; sub < KSUB; ++sub) {
+      f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < NQS; ++s)
+        if (s * VK_SLAB < d) s4 = mma_slab(kf[sub][s], qf[s], s4);
+      sc[4 * sub + 0] = s4.x;
+      sc[4 * sub + 1] = s4.y;
+      sc[4 * sub + 2] = s4.z;
+      sc[4 * sub + 3] = s4.w;
+    }
+    return;
+  }
   f32x4 s4[KSUB];
 #pragma unroll
   for (int sub = 0; sub < KSUB; ++sub) s4[sub] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -368,7 +414,13 @@ __device__ __forceinline__ void tile_pv(const RowCtx& c, int kb, frag_t (&vf)[ND
                                         f32x4 (&ACC)[NDT]) {
   const int d = EXACT ? NDT * 16 : c.d;
   if (kb + TILE_KEYS > c.k_len || kb < c.wave_lo) {
-    OwnedMask(kb, c.g, c.wave_lo, c.k_len, 0).apply(vf, (d + 15) / 16);
+    if constexpr (wide_heads(16 * NDT)) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+        if (dt * 16 < d) zero_unowned(vf[dt], kb, c.g, c.wave_lo, c.k_len);
+    } else {
+      OwnedMask(kb, c.g, c.wave_lo, c.k_len, 0).apply(vf, (d + 15) / 16);
+    }
   }
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
@@ -389,7 +441,7 @@ __device__ __forceinline__ void tile_step(const RowCtx& c, const frag_t (&qf)[NQ
   // A wave that has the SIMD nearly to itself (few decoded tokens) asks for everything at once.
   if (!V_LATE) load_values<NDT, EXACT>(c, kb, vf);
   float sc[S_PER_LANE];
-  tile_scores<NQS, EXACT>(c, kf, qf, sc);
+  tile_scores<NQS, EXACT, lean_waves(16 * NDT)>(c, kf, qf, sc);
   if (V_LATE) {
     // Requested once the key fragments' registers are free again, so that more waves fit a SIMD;
     // the latency passes behind the softmax arithmetic and the other waves.
@@ -399,7 +451,7 @@ __device__ __forceinline__ void tile_step(const RowCtx& c, const frag_t (&qf)[NQ
   frag_t pf[KEY_SLABS];
   float ca;
   const bool fresh = !(M > -INFINITY);
-  tile_probs(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.scale_log2, false, M, L, ca, pf);
+  tile_probs<lean_waves(16 * NDT)>(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.scale_log2, false, M, L, ca, pf);
   scale_state<NDT>(ACC, ca, fresh);
   tile_pv<NDT, EXACT>(c, kb, vf, pf, ACC);
 }
@@ -518,39 +570,61 @@ __device__ __forceinline__ void natural_scores(float (&sc)[S_PER_LANE], float sc
 }
 
 // tile_probs for scores in natural units (already scaled and capped), with kept first keys and unrounded weights.
+template <bool LEAN = false>
 __device__ __forceinline__ void tile_probs_ext(float (&sc)[S_PER_LANE], int kb, int g, bool row_ok, int lo, int pos, int keep, bool full,
                                                float& M, float& L, float& ca, frag_t (&pf)[P_PARTS][KEY_SLABS]) {
   float pr[S_PER_LANE];
   float psum = 0.f;
-  // The numbers of a lane's visible keys, a bit each; all of them where every row of the wave sees every key.  (Masks written as
-  // conditions become branches, seven hundred instructions of a tile's thousand.)
-  unsigned vis = ~0u;
-  if (!full) {
-    vis = 0;
+  float Mn;
+  if constexpr (LEAN) {
+    bool vis[S_PER_LANE];
+    float tmax = -INFINITY;
 #pragma unroll
     for (int i = 0; i < S_PER_LANE; ++i) {
       const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
-      vis |= (unsigned)((int)row_ok & (int)(key <= pos) & ((int)(key >= lo) | (int)(key < keep))) << i;
+      vis[i] = row_ok && key <= pos && (key >= lo || key < keep);
+      tmax = fmaxf(tmax, vis[i] ? sc[i] : -INFINITY);
+    }
+    tmax = row_max<true>(tmax);
+    const float m = tmax * LOG2E;
+    Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
+    ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) {
+      pr[i] = vis[i] ? fast_exp2(__builtin_fmaf(sc[i], LOG2E, -Mn)) : 0.f;
+      psum = psum + pr[i];
+    }
+  } else {
+    // The numbers of a lane's visible keys, a bit each; all of them where every row of the wave sees every key.  (Masks written as
+    // conditions become branches, seven hundred instructions of a tile's thousand.)
+    unsigned vis = ~0u;
+    if (!full) {
+      vis = 0;
+#pragma unroll
+      for (int i = 0; i < S_PER_LANE; ++i) {
+        const int key = kb + (i / VK_VEC) * VK_SLAB + g * VK_VEC + (i % VK_VEC);
+        vis |= (unsigned)((int)row_ok & (int)(key <= pos) & ((int)(key >= lo) | (int)(key < keep))) << i;
+      }
+#pragma unroll
+      for (int i = 0; i < S_PER_LANE; ++i) sc[i] = vis >> i & 1u ? sc[i] : -INFINITY;
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
+    tmax = row_max(tmax);
+    const float m = tmax * LOG2E;             // -inf: the row sees no key of the tile
+    Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
+    ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
+#pragma unroll
+    for (int i = 0; i < S_PER_LANE; ++i) pr[i] = fast_exp2(__builtin_fmaf(sc[i], LOG2E, -Mn));
+    if (!full) {
+#pragma unroll
+      for (int i = 0; i < S_PER_LANE; ++i) pr[i] = vis >> i & 1u ? pr[i] : 0.f;
     }
 #pragma unroll
-    for (int i = 0; i < S_PER_LANE; ++i) sc[i] = vis >> i & 1u ? sc[i] : -INFINITY;
+    for (int i = 0; i < S_PER_LANE; ++i) psum = psum + pr[i];
   }
-  float tmax = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < S_PER_LANE; ++i) tmax = fmaxf(tmax, sc[i]);
-  tmax = row_max(tmax);
-  const float m = tmax * LOG2E;             // -inf: the row sees no key of the tile
-  const float Mn = (!(M > -INFINITY) || m > M + MAX_STEP) ? m : M;
-  ca = Mn > -INFINITY ? fast_exp2(M - Mn) : 1.f;
-#pragma unroll
-  for (int i = 0; i < S_PER_LANE; ++i) pr[i] = fast_exp2(__builtin_fmaf(sc[i], LOG2E, -Mn));
-  if (!full) {
-#pragma unroll
-    for (int i = 0; i < S_PER_LANE; ++i) pr[i] = vis >> i & 1u ? pr[i] : 0.f;
-  }
-#pragma unroll
-  for (int i = 0; i < S_PER_LANE; ++i) psum = psum + pr[i];
-  psum = row_sum(psum);
+  psum = row_sum<LEAN>(psum);
   L = __builtin_fmaf(L, ca, psum);
   M = Mn;
 #pragma unroll
@@ -575,7 +649,7 @@ __device__ __forceinline__ void tile_probs_ext(float (&sc)[S_PER_LANE], int kb, 
 
 // The second half of a tile's work for the variant with capped scores: the cap, the probabilities onto the row's state,
 // and P V with the unrounded weights.  vf: the tile's value fragments (from global memory; cleaned here).
-template <int NDT, bool REL>
+template <int NDT, bool REL, bool LEAN>
 __device__ __forceinline__ void tile_softmax_pv_ext(const RowCtx& c, float scale, float softcap, float (&sc)[S_PER_LANE], int kb,
                                                     frag_t (&vf)[NDT][KEY_SLABS], float& M, float& L, f32x4 (&ACC)[NDT]) {
   float rb[REL ? S_PER_LANE : 1];
@@ -584,10 +658,16 @@ __device__ __forceinline__ void tile_softmax_pv_ext(const RowCtx& c, float scale
   frag_t pf[P_PARTS][KEY_SLABS];
   float ca;
   const bool fresh = !(M > -INFINITY);
-  tile_probs_ext(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.keep, false, M, L, ca, pf);
+  tile_probs_ext<LEAN>(sc, kb, c.g, c.row_ok, c.lo, c.pos, c.keep, false, M, L, ca, pf);
   scale_state<NDT>(ACC, ca, fresh);
   if (kb + TILE_KEYS > c.k_len || kb < c.wave_lo) {
-    OwnedMask(kb, c.g, c.wave_lo, c.k_len, c.keep).apply(vf, (c.d + 15) / 16);
+    if constexpr (wide_heads(16 * NDT)) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+        if (dt * 16 < c.d) zero_unowned(vf[dt], kb, c.g, c.wave_lo, c.k_len, c.keep);
+    } else {
+      OwnedMask(kb, c.g, c.wave_lo, c.k_len, c.keep).apply(vf, (c.d + 15) / 16);
+    }
   }
   // A sum takes its products in the order (key slab, part).  (Walking several column blocks side by side, so that no MFMA
   // follows one it depends on, costs the decode kernels more registers than a wave has: they spill.)
@@ -1056,7 +1136,7 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
   auto tile = [&](int t, bool more) {
     const int kb = t * TILE_KEYS;
     float sc[S_PER_LANE];
-    tile_scores<NQS, EXACT>(c, kf, qf, sc);
+    tile_scores<NQS, EXACT, lean_waves(16 * NDT)>(c, kf, qf, sc);
     __builtin_amdgcn_sched_barrier(0);
     if (more) load_keys<NQS, EXACT>(c, kb + TILE_KEYS, kf);
     __builtin_amdgcn_sched_barrier(0);
@@ -1066,7 +1146,7 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
     frag_t pf[KEY_SLABS];
     float ca;
     const bool fresh = !(M > -INFINITY);
-    tile_probs(sc, kb, c.g, c.row_ok, lo, pos, c.scale_log2, full, M, L, ca, pf);
+    tile_probs<lean_waves(16 * NDT)>(sc, kb, c.g, c.row_ok, lo, pos, c.scale_log2, full, M, L, ca, pf);
     scale_state<NDT>(ACC, ca, fresh);
     tile_pv<NDT, EXACT>(c, kb, vf, pf, ACC);
     __builtin_amdgcn_sched_barrier(0);
@@ -1113,7 +1193,7 @@ __global__ __launch_bounds__(64 * SEG_WAVES, 2) void attn_decode_seg_kernel(Attn
 // all rows of the wave takes the last entry and reads nothing.
 //
 // A gate.  A head's output may be multiplied by the logistic function of one number a token and head, before it is rounded.
-template <int NDT, int NQS, bool V_LATE, bool REL>
+template <int NDT, int NQS, bool V_LATE, bool REL, bool LEAN>
 __device__ __forceinline__ void tile_step_ext(const RowCtx& c, float scale, float softcap, const frag_t (&qf)[NQS], int kb, float& M,
                                               float& L, f32x4 (&ACC)[NDT]) {
   frag_t kf[KSUB][NQS];
@@ -1121,12 +1201,12 @@ __device__ __forceinline__ void tile_step_ext(const RowCtx& c, float scale, floa
   load_keys<NQS, false>(c, kb, kf);
   if (!V_LATE) load_values<NDT, false>(c, kb, vf);
   float sc[S_PER_LANE];
-  tile_scores<NQS, false>(c, kf, qf, sc);
+  tile_scores<NQS, false, LEAN>(c, kf, qf, sc);
   if (V_LATE) {
     __builtin_amdgcn_sched_barrier(0);
     load_values<NDT, false>(c, kb, vf);
   }
-  tile_softmax_pv_ext<NDT, REL>(c, scale, softcap, sc, kb, vf, M, L, ACC);
+  tile_softmax_pv_ext<NDT, REL, LEAN>(c, scale, softcap, sc, kb, vf, M, L, ACC);
 }
 
 // Prompt rows: attn_prefill_kernel with the things above.
@@ -1177,7 +1257,7 @@ __global__ __launch_bounds__(256) void attn_prefill_ext_kernel(AttnArgs a, int h
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) As[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int t = t_begin; t <= t_end; ++t)
-      if (t < keep_tiles || t >= tile_lo) tile_step_ext<NDT, NQS, true, REL>(c, a.scale, a.softcap, qf, t * TILE_KEYS, Ms, Ls, As);
+      if (t < keep_tiles || t >= tile_lo) tile_step_ext<NDT, NQS, true, REL, false>(c, a.scale, a.softcap, qf, t * TILE_KEYS, Ms, Ls, As);
     fold<NDT>(M, L, ACC, Ms, Ls, As);
   }
   if (c.row_ok) {
@@ -1234,7 +1314,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_decode_ext_kernel(AttnA
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) ACC[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int t = t0; t <= t1; ++t)
-    if (t < keep_tiles || t >= tile_lo) tile_step_ext<NDT, NQS, V_LATE, REL>(c, a.scale, a.softcap, qf, t * TILE_KEYS, M, L, ACC);
+    if (t < keep_tiles || t >= tile_lo) tile_step_ext<NDT, NQS, V_LATE, REL, lean_waves(DPAD)>(c, a.scale, a.softcap, qf, t * TILE_KEYS, M, L, ACC);
   if (!c.row_ok) return;
   const int64_t prow = ((int64_t)blockIdx.x * a.nq + head) * a.nseg + seg;
   if (c.g == 0) {
