@@ -319,16 +319,16 @@ constexpr int KSUB = S_PER_LANE / 4;    // 16-key MFMA sub-tiles per tile
 // Key fragments of the whole tile, all in flight together.
 // EXACT (here and below): the head size is the padded one and a page holds a tile or more, known
 // at compile time, so that no branch on either is left in the code.
-// PAGE: the caller has read the tile's page from the table already (a tile in one page).  (A page that says by its sign whether it was read leaves a
-// second read in the code, and in front of every tile's loads a wait for the ones before.)
-template <int NQS, bool EXACT, bool PAGE = false>
+// PAGE_READ: the caller has read the tile's page from the table; PAGE_MAYBE: it has where the tile lies in one page, else the number is negative.
+enum { PAGE_UNREAD, PAGE_READ, PAGE_MAYBE };
+template <int NQS, bool EXACT, int PAGE = PAGE_UNREAD>
 __device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[KSUB][NQS], int page = 0) {
   const int d = EXACT ? NQS * VK_SLAB : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const bool dfull = EXACT || d % VK_SLAB == 0;    // else the last slab along d is partly outside the head
   const int last_key = c.k_len - 1;
   // With pages of at least a tile, the tile lies in one page: one table lookup for the wave.
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* kpage = c.kbase + (one_page ? (int64_t)(PAGE ? page : c.bt[kb >> lp]) * c.page_stride : 0);
+  const elem_t* kpage = c.kbase + (one_page ? (int64_t)(PAGE == PAGE_READ || (PAGE == PAGE_MAYBE && page >= 0) ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int sub = 0; sub < KSUB; ++sub) {
 #ifdef VK_BF16
@@ -350,12 +350,12 @@ __device__ __forceinline__ void load_keys(const RowCtx& c, int kb, frag_t (&kf)[
   }
 }
 
-template <int NDT, bool EXACT, bool PAGE = false>
+template <int NDT, bool EXACT, int PAGE = PAGE_UNREAD>
 __device__ __forceinline__ void load_values(const RowCtx& c, int kb, frag_t (&vf)[NDT][KEY_SLABS], int page = 0) {
   const int d = EXACT ? NDT * 16 : c.d, P = c.P, lp = c.lp, r16 = c.r16, g = c.g;
   const int last_key = c.k_len - 1;
   const bool one_page = EXACT || P >= TILE_KEYS;
-  const elem_t* vpage = c.vbase + (one_page ? (int64_t)(PAGE ? page : c.bt[kb >> lp]) * c.page_stride : 0);
+  const elem_t* vpage = c.vbase + (one_page ? (int64_t)(PAGE == PAGE_READ || (PAGE == PAGE_MAYBE && page >= 0) ? page : c.bt[kb >> lp]) * c.page_stride : 0);
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
     if (dt * 16 < d) {
@@ -1436,7 +1436,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   auto read_pages = [&](int first_tile) {
 #pragma unroll
     for (int j = 0; j < SEG_TILES; ++j)
-      page[j] = EXACT || a.P >= TILE_KEYS ? a.block_table[(int64_t)seq * a.bt_stride + min((first_tile + j) * TILE_KEYS >> lp, a.bt_stride - 1)] : 0;
+      page[j] = EXACT || a.P >= TILE_KEYS ? a.block_table[(int64_t)seq * a.bt_stride + min((first_tile + j) * TILE_KEYS >> lp, a.bt_stride - 1)] : -1;
   };
   int seg = blockIdx.z * SEGS + my_seg;
   const int k_len = a.k_len[seq];
@@ -1512,6 +1512,11 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
   // unknown number is one for all of them, and the barrier behind the rows then makes every wave wait for everybody's keys.  With both segments in one workgroup the second
   // may have no tile at all, and its waves' reads cost more than they save.)
   constexpr bool ALWAYS = ROWS && SEGS == 1;
+  // Heads of a padded size: one copy of the loads for pages of every size, but for the variant with heads of more than 128 entries two, one for pages of a tile and more.
+  // (16-bit, decoded rows on pages of a tile, us, two copies and one: 56 launches of 16 heads of 192 on 2 1,391, 1,300, 64 rows of 800 keys 38.1, 32.5; 24 launches of the variant, 16 heads
+  // of 96 on 2 281, 267, of 192 511, 604.  Pages of 16: 56 launches of heads of 192 2,026, 2,110.)
+  constexpr bool TWICE = !EXACT && EXT && DPAD > 128;
+  constexpr int HOW = EXACT || TWICE ? PAGE_READ : PAGE_MAYBE;
   if (ALWAYS || mine) {
     if constexpr (!ROWS) load_q<NQS>(a, tok, head, c.row_ok, c.g, qf);
     const int of = ALWAYS && !mine ? __builtin_ctz(wanted) : wave, first_key = (first_tile + of) * TILE_KEYS;
@@ -1520,7 +1525,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
     for (int j = 1; j < SEG_TILES; ++j) my_page = of == j ? page[j] : my_page;
     RowCtx ck = c;
     if (ALWAYS && !mine) ck.k_len = first_key + 1;
-    if (EXACT || a.P >= TILE_KEYS) load_keys<NQS, EXACT, true>(ck, first_key, kf, my_page);
+    if (!TWICE || a.P >= TILE_KEYS) load_keys<NQS, EXACT, HOW>(ck, first_key, kf, my_page);
     else load_keys<NQS, EXACT>(ck, first_key, kf);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -1557,7 +1562,7 @@ __global__ __launch_bounds__(64 * SEG_TILES * SEGS, sizeof(elem_t) * DPAD <= 256
 #pragma unroll
   for (int j = 0; j < SEG_TILES; ++j)
     if ((wanted >> j) & 1u) {
-      if (EXACT || a.P >= TILE_KEYS) load_values<ND, EXACT, true>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
+      if (!TWICE || a.P >= TILE_KEYS) load_values<ND, EXACT, HOW>(cv, (first_tile + j) * TILE_KEYS, vf[j], page[j]);
       else load_values<ND, EXACT>(cv, (first_tile + j) * TILE_KEYS, vf[j]);
     }
   __builtin_amdgcn_sched_barrier(0);
